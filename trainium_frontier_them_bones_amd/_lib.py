@@ -140,26 +140,76 @@ def lib():
     return _LIB
 
 
-# name -> list: when an entry point is listed here every call is bracketed by events on torch's current stream
-# (the stream the kernels are launched on) and (start, end, name, args) appended; the key "*" takes every entry point
-# not listed by name. Used by the benchmark only.
-TIMED = {}
+class _Timed(dict):
+    """name -> list: when an entry point is listed here every call is bracketed by events on torch's current stream (the
+    stream the kernels are launched on) and (start, end, name, args) appended; the key "*" takes every entry point not
+    listed by name. Used by the benchmark only. The native layer is told whether the table is empty."""
+
+    def __setitem__(self, name, rec):
+        super().__setitem__(name, rec)
+        native.set_timed(True)
+
+    def __delitem__(self, name):
+        super().__delitem__(name)
+        native.set_timed(bool(self))
+
+
+TIMED = _Timed()
+
+
+def _timed_begin(name):
+    """(record list, start event) for a timed entry point, else None."""
+    rec = TIMED.get(name)
+    if rec is None:
+        rec = TIMED.get("*")
+    if rec is None:
+        return None
+    import torch
+    s = torch.cuda.Event(enable_timing=True)
+    s.record()
+    return rec, s
+
+
+def _timed_end(handle, name, args):
+    import torch
+    rec, s = handle
+    e = torch.cuda.Event(enable_timing=True)
+    e.record()
+    rec.append((s, e, name, args))
 
 
 def call(name, *args):
-    rec = None
-    if TIMED:
-        rec = TIMED.get(name)
-        if rec is None:
-            rec = TIMED.get("*")
-    if rec is None:
-        st = getattr(lib(), name)(*args)
-    else:
-        import torch
-        s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        s.record()
-        st = getattr(lib(), name)(*args)
-        e.record()
-        rec.append((s, e, name, args))
+    h = _timed_begin(name) if TIMED else None
+    st = getattr(lib(), name)(*args)
+    if h is not None:
+        _timed_end(h, name, args)
     if st != 0:
         raise TfbError(name, st)
+
+
+# ---- the native host layer (csrc/host): the ops on tensors and the autograd nodes ------------------------------------
+HOST_PATH = os.path.join(HERE, "_tfb_host.so")
+
+
+class _Native:
+    """The extension module, loaded on first use (the package imports without a built library)."""
+
+    def __getattr__(self, name):
+        lib()      # first: the extension binds to the library loaded from LIB_PATH
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError("host extension %s is not built; run `python -m trainium_frontier_them_bones_amd.build`" % HOST_PATH)
+        import importlib.machinery
+        import importlib.util
+
+        import torch  # noqa: F401  (its libraries hold the symbols the extension links against)
+        loader = importlib.machinery.ExtensionFileLoader("_tfb_host", HOST_PATH)
+        mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_tfb_host", loader))
+        loader.exec_module(mod)
+        self.__dict__.update((k, v) for k, v in vars(mod).items() if not k.startswith("__"))
+        try:
+            return self.__dict__[name]
+        except KeyError:
+            raise AttributeError(name) from None
+
+
+native = _Native()

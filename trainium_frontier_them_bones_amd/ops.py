@@ -6,6 +6,7 @@ library. torch supplies device memory and the stream; all arithmetic is in the H
 import torch
 
 from . import _lib
+from ._lib import native
 
 bf16 = torch.bfloat16
 
@@ -15,7 +16,7 @@ def _p(t):
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _chk(t, dtype=bf16):
@@ -30,101 +31,38 @@ def _chk(t, dtype=bf16):
 
 
 # ------------------------------------------------------------------------------------------ GEMM
-_WS = {}
-
-
-def _workspace(device, nbytes=256 << 20):
-    """One fp32 split-K workspace per (device, stream), allocated on first use: launches on different streams would
-    otherwise race on the same partial sums."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
-    ws = _WS.get(key)
-    if ws is None or ws.numel() * 4 < nbytes:
-        ws = torch.empty(nbytes // 4, dtype=torch.float32, device=device)
-        _WS[key] = ws
-    return ws
-
-
 def matmul(a, b, trans_a=False, trans_b=False, out=None, accumulate=False, out_dtype=bf16, alpha=None):
     """op(a) @ op(b) with fp32 accumulation. a is [M,K] (or [K,M] with trans_a), b is [K,N] (or [N,K] with
     trans_b). `out` (bf16 or fp32) may be given; accumulate=True adds into it (one rounding). alpha: a 1-element fp32
     device tensor the product is multiplied by before that rounding (no host read-back)."""
-    _chk(a), _chk(b), _chk(alpha, torch.float32)
-    if alpha is not None and alpha.numel() != 1:
-        raise ValueError("alpha is one fp32 element")
-    M, K = (a.shape[1], a.shape[0]) if trans_a else (a.shape[0], a.shape[1])
-    Kb, N = (b.shape[1], b.shape[0]) if trans_b else (b.shape[0], b.shape[1])
-    if K != Kb:
-        raise ValueError("inner dimensions differ: %d vs %d" % (K, Kb))
-    if out is None:
-        if accumulate:
-            raise ValueError("accumulate needs out")
-        out = torch.empty(M, N, dtype=out_dtype, device=a.device)
-    else:
-        _chk(out, out.dtype)
-        if out.dtype not in (bf16, torch.float32) or tuple(out.shape) != (M, N):
-            raise ValueError("bad out")
-    ws = _workspace(a.device)
     if alpha is None:
-        _lib.call("tfb_gemm_bf16", _p(a), _p(b), _p(out), M, N, K, int(trans_a), int(trans_b),
-                  int(out.dtype == torch.float32), int(accumulate), _p(ws), ws.numel() * 4, _stream())
-    else:
-        _lib.call("tfb_gemm_bf16_scaled", _p(a), _p(b), _p(out), M, N, K, int(trans_a), int(trans_b),
-                  int(out.dtype == torch.float32), int(accumulate), _p(ws), ws.numel() * 4, _p(alpha), _stream())
-    return out
+        return native.tfb_gemm_bf16(a, b, trans_a, trans_b, out, accumulate, out_dtype == torch.float32)
+    return native.tfb_gemm_bf16_scaled(a, b, trans_a, trans_b, out, accumulate, out_dtype == torch.float32, alpha)
 
 
 def matmul_res(a, b, res, trans_b=False):
     """bf16(res + bf16(a @ op(b))): a projection with the residual add that follows it made in the GEMM's store (equal to
     matmul followed by a bf16 add, bit for bit). a [M,K]; b [K,N] or, with trans_b, [N,K]; res [M,N]."""
-    _chk(a), _chk(b), _chk(res)
-    M, K = a.shape
-    Kb, N = (b.shape[1], b.shape[0]) if trans_b else (b.shape[0], b.shape[1])
-    if K != Kb or tuple(res.shape) != (M, N):
-        raise ValueError("shapes differ")
-    out = torch.empty(M, N, dtype=bf16, device=a.device)
-    _lib.call("tfb_gemm_bf16_res", _p(a), _p(b), _p(res), _p(out), M, N, K, int(trans_b), _stream())
-    return out
+    return native.tfb_gemm_bf16_res(a, b, res, trans_b)
 
 
 def qkv_rope(x2, w, cos, sin, T, rot_cols):
     """rope(x2 @ w^T): the fused attention projection [M, N] with the rotary embedding of its first rot_cols columns
     (heads of 64) applied in the GEMM epilogue; row m is token m % T."""
-    _chk(x2), _chk(w), _chk(cos), _chk(sin)
-    M, K = x2.shape
-    N = w.shape[0]
-    out = torch.empty(M, N, dtype=bf16, device=x2.device)
-    _lib.call("tfb_qkv_rope_fwd", _p(x2), _p(w), _p(cos), _p(sin), _p(out), M, N, K, T, rot_cols, _stream())
-    return out
+    return native.tfb_qkv_rope_fwd(x2, w, cos, sin, T, rot_cols)
 
 
 # ------------------------------------------------------------------------------------------ norms
 def rmsnorm_fwd(x, weight=None, eps=2.0 ** -23, res=None):
     """y = RMSNorm(s) * weight with s = x (res None) or bf16(x + res). Returns (s, y, inv[rows] fp32)."""
-    _chk(x), _chk(res), _chk(weight)
-    C = x.shape[-1]
-    rows = x.numel() // C
-    y = torch.empty_like(x)
-    s = torch.empty_like(x) if res is not None else x
-    inv = torch.empty(rows, dtype=torch.float32, device=x.device)
-    _lib.call("tfb_rmsnorm_fwd", _p(x), _p(res), _p(weight), _p(s) if res is not None else None, _p(y), _p(inv),
-              rows, C, float(eps), _stream())
-    return s, y, inv
+    return native.tfb_rmsnorm_fwd(x, weight, eps, res)
 
 
 def rmsnorm_fwd_q(x, weight=None, eps=2.0 ** -23, res=None, y8_scale=4.0, want_y=True):
     """rmsnorm_fwd that also returns y8 = e4m3(bf16(y) * y8_scale) bytes, the operand cast of the fp8 GEMM that consumes y
     (equal to quant_fp8(y, y8_scale), bit for bit). Returns (s, y, inv, y8); want_y False: the bf16 rows are not written and
     y is None (for a consumer that reads only the bytes)."""
-    _chk(x), _chk(res), _chk(weight)
-    C = x.shape[-1]
-    rows = x.numel() // C
-    y = torch.empty_like(x) if want_y else None
-    s = torch.empty_like(x) if res is not None else x
-    inv = torch.empty(rows, dtype=torch.float32, device=x.device)
-    y8 = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    _lib.call("tfb_rmsnorm_fwd_q", _p(x), _p(res), _p(weight), _p(s) if res is not None else None, _p(y), _p(inv), _p(y8),
-              float(y8_scale), rows, C, float(eps), _stream())
-    return s, y, inv, y8
+    return native.tfb_rmsnorm_fwd_q(x, weight, eps, res, y8_scale, want_y)
 
 
 def rmsnorm_bwd(gy, s, inv, weight=None, gs=None, dw=None, accumulate=False, part=None, want_amax=False):
@@ -132,35 +70,9 @@ def rmsnorm_bwd(gy, s, inv, weight=None, gs=None, dw=None, accumulate=False, par
     added into with accumulate=True. With `part` (fp32 [tfb_norm_bwd_blocks(rows), C]) the weight gradient is left there
     as partial sums for norm_dw_finish and None is returned for it. want_amax: a third value, fp32 [tfb_norm_bwd_blocks(rows)]
     whose maximum is amax(dx) (per-workgroup partials, for mlp8_backward_scales(..., amax_part=))."""
-    _chk(gy), _chk(s), _chk(weight), _chk(gs), _chk(inv, torch.float32)
-    C = s.shape[-1]
-    rows = s.numel() // C
-    dx = torch.empty_like(s)
-    acc = 0
-    am = torch.empty(_lib.lib().tfb_norm_bwd_blocks(rows), dtype=torch.float32, device=s.device) if want_amax else None
-
-    def call(part_, dw_, acc_):
-        if want_amax:
-            _lib.call("tfb_rmsnorm_bwd_amax", _p(gy), _p(gs), _p(s), _p(weight), _p(inv), _p(dx), _p(part_), _p(dw_), acc_, _p(am),
-                      rows, C, _stream())
-        else:
-            _lib.call("tfb_rmsnorm_bwd", _p(gy), _p(gs), _p(s), _p(weight), _p(inv), _p(dx), _p(part_), _p(dw_), acc_, rows, C,
-                      _stream())
-
-    if weight is not None and part is not None:
-        _chk(part, torch.float32)
-        call(part, None, 0)
-        return (dx, None, am) if want_amax else (dx, None)
-    if weight is not None:
-        nb = _lib.lib().tfb_norm_bwd_blocks(rows)
-        part = torch.empty(nb, C, dtype=torch.float32, device=s.device)
-        if dw is None:
-            dw = torch.empty(C, dtype=torch.float32, device=s.device)
-        else:
-            _chk(dw, torch.float32)
-            acc = int(accumulate)
-    call(part, dw, acc)
-    return (dx, dw, am) if want_amax else (dx, dw)
+    if want_amax:
+        return native.tfb_rmsnorm_bwd_amax(gy, s, inv, weight, gs, dw, accumulate, part, True)
+    return native.tfb_rmsnorm_bwd(gy, s, inv, weight, gs, dw, accumulate, part, False)
 
 
 def norm_bwd_blocks(rows):
@@ -180,31 +92,12 @@ def norm_dw_finish(parts, dw, rows, accumulate=False):
 
 def block_head_fwd(x, x0, gains, skip=None, eps=2.0 ** -23):
     """x_new = l1*x + l2*x0 (+ l3*skip), x_norm = RMSNorm(x_new). gains: fp32 device tensor [3]."""
-    _chk(x), _chk(x0), _chk(skip), _chk(gains, torch.float32)
-    C = x.shape[-1]
-    rows = x.numel() // C
-    x_new = torch.empty_like(x)
-    x_norm = torch.empty_like(x)
-    inv = torch.empty(rows, dtype=torch.float32, device=x.device)
-    _lib.call("tfb_block_head_fwd", _p(x), _p(x0), _p(skip), _p(gains), _p(x_new), _p(x_norm), _p(inv), rows, C,
-              float(eps), _stream())
-    return x_new, x_norm, inv
+    return native.tfb_block_head_fwd(x, x0, gains, skip, eps)
 
 
 def block_head_bwd(g_new, g_norm, x, x0, x_new, inv, gains, skip=None):
     """Returns (dx, dx0, dskip or None, dgains fp32 [4] = sum G.x, G.x0, G.skip, 0)."""
-    _chk(g_new), _chk(g_norm), _chk(x), _chk(x0), _chk(skip), _chk(x_new)
-    C = x.shape[-1]
-    rows = x.numel() // C
-    dx = torch.empty_like(x)
-    dx0 = torch.empty_like(x)
-    dskip = torch.empty_like(x) if skip is not None else None
-    nb = _lib.lib().tfb_norm_bwd_blocks(rows)
-    part = torch.empty(nb, 4, dtype=torch.float32, device=x.device)
-    dg = torch.empty(4, dtype=torch.float32, device=x.device)
-    _lib.call("tfb_block_head_bwd", _p(g_new), _p(g_norm), _p(x), _p(x0), _p(skip), _p(x_new), _p(inv), _p(gains),
-              _p(dx), _p(dx0), _p(dskip), _p(part), _p(dg), rows, C, _stream())
-    return dx, dx0, dskip, dg
+    return native.tfb_block_head_bwd(g_new, g_norm, x, x0, x_new, inv, gains, skip)
 
 
 # ------------------------------------------------------------------------------------------ fp8 MLP
@@ -264,36 +157,19 @@ def mlp8_refresh_layers(w_fc0, w_proj0, layer_stride, layers, e4m3_limit=240.0, 
 def mlp8_backward_scales(dy2, row, amax_part=None):
     """The backward call's scale row from amax(dy2), or from amax_part (fp32 partials whose maximum is that amax, as
     rmsnorm_bwd(want_amax=True) leaves them for the dx it wrote) without reading dy2."""
-    _chk(dy2), _chk(row, torch.float32), _chk(amax_part, torch.float32)
-    M, d = dy2.shape
-    out = torch.empty(NSC, dtype=torch.float32, device=dy2.device)
     if amax_part is not None:
-        _lib.call("tfb_mlp8_backward_scales_part", _p(amax_part), amax_part.numel(), _p(row), _p(out), d, _stream())
-        return out
-    scr = _scratch(dy2.device, 4096)
-    _lib.call("tfb_mlp8_backward_scales", _p(dy2), _p(row), _p(out), _p(scr), M, d, _stream())
-    return out
+        return native.tfb_mlp8_backward_scales_part(dy2, row, amax_part)
+    return native.tfb_mlp8_backward_scales(dy2, row)
 
 
 def amax_scale(x, limit, e_lo, e_hi):
     """fp32 [3] = (s, 1/s, amax): s the largest power of two in [2^e_lo, 2^e_hi] with amax(x) * s <= limit."""
-    _chk(x)
-    out = torch.empty(3, dtype=torch.float32, device=x.device)
-    scr = _scratch(x.device, 4096)
-    _lib.call("tfb_amax_scale", _p(x), x.numel(), float(limit), int(e_lo), int(e_hi), _p(out), _p(scr), _stream())
-    return out
+    return native.tfb_amax_scale(x, limit, e_lo, e_hi)
 
 
 def quant_fp8(x, scale, fmt=FMT_E4M3):
     """uint8-carried fp8 of x * scale; scale a python float or a 1-element fp32 device tensor (no host sync)."""
-    _chk(x)
-    out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    if isinstance(scale, torch.Tensor):
-        _chk(scale, torch.float32)
-        _lib.call("tfb_quant_fp8", _p(x), _p(scale), 0.0, fmt, _p(out), x.numel(), _stream())
-    else:
-        _lib.call("tfb_quant_fp8", _p(x), None, float(scale), fmt, _p(out), x.numel(), _stream())
-    return out
+    return native.tfb_quant_fp8(x, scale, fmt)
 
 
 def precast8(w, scale):
@@ -309,50 +185,20 @@ def precast8(w, scale):
 def gemm_fp8(a8, b8, fmt_a=FMT_E4M3, dq_a=None, dq_b=None, dq=1.0):
     """bf16 [M,N] = (a8 [M,K] @ b8 [N,K]^T) * dq * dq_a * dq_b; a8 e4m3 or e5m2 bytes, b8 e4m3 bytes; dq_a, dq_b
     1-element fp32 device tensors (or None)."""
-    _chk(a8, torch.uint8), _chk(b8, torch.uint8), _chk(dq_a, torch.float32), _chk(dq_b, torch.float32)
-    M, K = a8.shape
-    N = b8.shape[0]
-    if b8.shape[1] != K:
-        raise ValueError("inner dimensions differ")
-    out = torch.empty(M, N, dtype=bf16, device=a8.device)
-    _lib.call("tfb_gemm_fp8", _p(a8), int(fmt_a), _p(b8), _p(dq_a), _p(dq_b), float(dq), _p(out), M, N, K, _stream())
-    return out
+    return native.tfb_gemm_fp8(a8, b8, fmt_a, dq_a, dq_b, dq)
 
 
 def gemm_fp8_res(a8, b8, res, dq_a=None, dq_b=None, dq=1.0):
     """bf16(res + bf16((a8 [M,K] @ b8 [N,K]^T) * dq * dq_a * dq_b)): gemm_fp8 (e4m3 activations) with the residual add
     in the store, equal to gemm_fp8 followed by a bf16 add bit for bit."""
-    _chk(a8, torch.uint8), _chk(b8, torch.uint8), _chk(dq_a, torch.float32), _chk(dq_b, torch.float32), _chk(res)
-    M, K = a8.shape
-    N = b8.shape[0]
-    if b8.shape[1] != K or tuple(res.shape) != (M, N):
-        raise ValueError("shapes differ")
-    out = torch.empty(M, N, dtype=bf16, device=a8.device)
-    _lib.call("tfb_gemm_fp8_res", _p(a8), _p(b8), _p(dq_a), _p(dq_b), float(dq), _p(res), _p(out), M, N, K, _stream())
-    return out
+    return native.tfb_gemm_fp8_res(a8, b8, FMT_E4M3, dq_a, dq_b, dq, res)
 
 
 def gemm_fp8_tn(g8, a8, fmt_g=FMT_E5M2, fmt_a=FMT_E4M3, s_g=None, s_a=None, imm=1.0, out=None, accumulate=False,
                 out_dtype=bf16):
     """[O,D] (+)= (g8 [M,O]^T @ a8 [M,D]) * imm / (s_g s_a): a weight gradient in fp8 (dw8_grad,
     round2/source/train.py:8185). s_g, s_a: 1-element fp32 device tensors (the scales the bytes were cast at) or None."""
-    _chk(g8, torch.uint8), _chk(a8, torch.uint8), _chk(s_g, torch.float32), _chk(s_a, torch.float32)
-    M, O = g8.shape
-    D = a8.shape[1]
-    if a8.shape[0] != M:
-        raise ValueError("token counts differ")
-    if out is None:
-        if accumulate:
-            raise ValueError("accumulate needs out")
-        out = torch.empty(O, D, dtype=out_dtype, device=g8.device)
-    else:
-        _chk(out, out.dtype)
-        if out.dtype not in (bf16, torch.float32) or tuple(out.shape) != (O, D):
-            raise ValueError("bad out")
-    ws = _workspace(g8.device)
-    _lib.call("tfb_gemm_fp8_tn", _p(g8), int(fmt_g), _p(a8), int(fmt_a), _p(s_g), _p(s_a), float(imm), _p(out), M, O, D,
-              int(out.dtype == torch.float32), int(accumulate), _p(ws), ws.numel() * 4, _stream())
-    return out
+    return native.tfb_gemm_fp8_tn(g8, a8, fmt_g, fmt_a, s_g, s_a, imm, out, accumulate, out_dtype == torch.float32)
 
 
 def mlp8_precast(w_fc, w_proj, row):
@@ -369,99 +215,34 @@ def mlp8_fwd(x2, w8, row, F, x_scale=4.0, want_x8=False, x8=None, res=None):
     want_x8 also returns x8 = e4m3(x x_scale) [M,d] bytes (the fp8 weight gradient's operand). A given x8 (from
     rmsnorm_fwd_q) is used instead of casting x2; with res [M,d], y = bf16(res + bf16(MLP(x))) (the block's residual add
     made in the second GEMM's store)."""
-    _chk(x2), _chk(w8, torch.uint8), _chk(row, torch.float32), _chk(x8, torch.uint8), _chk(res)
-    if x2 is None and x8 is None:
-        raise ValueError("give x2 or its bytes x8")
-    M, d = x2.shape if x2 is not None else x8.shape      # x2 may be left out when its bytes are given
-    dev = w8.device
-    if x8 is None:
-        x8 = quant_fp8(x2, x_scale, FMT_E4M3)
-    elif tuple(x8.shape) != (M, d):
-        raise ValueError("x8 shape")
-    y = torch.empty(M, d, dtype=bf16, device=dev)
-    r = torch.empty(M, F, dtype=bf16, device=dev)
-    h8 = torch.empty(M, F, dtype=torch.uint8, device=dev)
     if res is None:
-        _lib.call("tfb_mlp8_fwd", _p(x8), _p(w8), _p(row), _p(y), _p(r), _p(h8), M, d, F, _stream())
+        y, r, x8 = native.tfb_mlp8_fwd(x2, w8, row, F, x_scale, x8)
     else:
-        if tuple(res.shape) != (M, d):
-            raise ValueError("res shape")
-        _lib.call("tfb_mlp8_fwd_res", _p(x8), _p(w8), _p(row), _p(res), _p(y), _p(r), _p(h8), M, d, F, _stream())
+        y, r, x8 = native.tfb_mlp8_fwd_res(x2, w8, row, F, x_scale, x8, res)
     return (y, r, x8) if want_x8 else (y, r)
 
 
 def mlp8_bwd(dy2, r, w8, row, want_h=True):
     """dx [M,d], h [M,F] (or None), dpre [M,F]: the fp8 backward; row = this call's backward row."""
-    _chk(dy2), _chk(r), _chk(w8, torch.uint8), _chk(row, torch.float32)
-    M, d = dy2.shape
-    F = r.shape[1]
-    dy8 = quant_fp8(dy2, row[5:6], FMT_E5M2)
-    dx = torch.empty(M, d, dtype=bf16, device=dy2.device)
-    dpre = torch.empty(M, F, dtype=bf16, device=dy2.device)
-    h = torch.empty(M, F, dtype=bf16, device=dy2.device) if want_h else None
-    dp8 = torch.empty(M, F, dtype=torch.uint8, device=dy2.device)
-    _lib.call("tfb_mlp8_bwd", _p(dy8), _p(r), _p(w8), _p(row), _p(dx), _p(h), _p(dpre), _p(dp8), M, d, F, _stream())
-    return dx, h, dpre
+    return native.tfb_mlp8_bwd(dy2, r, w8, row, want_h)
 
 
 def mlp8_bwd_q(dy2, r, w8, row, e4m3_limit=240.0, want_dpre=True):
     """The fp8 backward keeping the byte tensors of the fp8 weight gradients: (dx [M,d], dpre [M,F] (None without
     want_dpre: the fp8 weight gradients read only its bytes), dp8 [M,F] e5m2 bytes, hq8 [M,F] = e4m3(min(bf16(r^2) s_h,
     e4m3_limit)) bytes, dy8 [M,d] e5m2 bytes)."""
-    _chk(dy2), _chk(r), _chk(w8, torch.uint8), _chk(row, torch.float32)
-    M, d = dy2.shape
-    F = r.shape[1]
-    dy8 = quant_fp8(dy2, row[5:6], FMT_E5M2)
-    dx = torch.empty(M, d, dtype=bf16, device=dy2.device)
-    dpre = torch.empty(M, F, dtype=bf16, device=dy2.device) if want_dpre else None
-    dp8 = torch.empty(M, F, dtype=torch.uint8, device=dy2.device)
-    hq8 = torch.empty(M, F, dtype=torch.uint8, device=dy2.device)
-    _lib.call("tfb_mlp8_bwd_q", _p(dy8), _p(r), _p(w8), _p(row), _p(dx), None, _p(dpre), _p(dp8), _p(hq8), float(e4m3_limit),
-              M, d, F, _stream())
-    return dx, dpre, dp8, hq8, dy8
+    return native.tfb_mlp8_bwd_q(dy2, r, w8, row, e4m3_limit, want_dpre)
 
 
 def mlp8_dw8(x8, dp8, hq8, dy8, row, x_scale=4.0, dw_fc=None, dw_proj=None, accumulate=False, out_dtype=bf16):
     """(dw_fc [F,d], dw_proj [d,F]) (+)= the fp8 weight gradients from the forward's x8 and the backward's dp8, hq8, dy8
     (mlp8_weight_grads under the fp8 weight-gradient switch, round2/source/train.py:8209)."""
-    for t in (x8, dp8, hq8, dy8):
-        _chk(t, torch.uint8)
-    _chk(row, torch.float32)
-    M, d = x8.shape
-    F = dp8.shape[1]
-    if tuple(hq8.shape) != (M, F) or tuple(dy8.shape) != (M, d):
-        raise ValueError("operand shapes")
-    if (dw_fc is None) != (dw_proj is None):
-        raise ValueError("give both outputs or neither")
-    if dw_fc is None:
-        if accumulate:
-            raise ValueError("accumulate needs the outputs")
-        dw_fc = torch.empty(F, d, dtype=out_dtype, device=x8.device)
-        dw_proj = torch.empty(d, F, dtype=out_dtype, device=x8.device)
-    else:
-        _chk(dw_fc, dw_fc.dtype), _chk(dw_proj, dw_proj.dtype)
-        if dw_fc.dtype != dw_proj.dtype or dw_fc.dtype not in (bf16, torch.float32):
-            raise ValueError("bad outputs")
-        if tuple(dw_fc.shape) != (F, d) or tuple(dw_proj.shape) != (d, F):
-            raise ValueError("bad output shapes")
-    ws = _workspace(x8.device)
-    xf, xd = _scale_arg(x_scale)
-    _lib.call("tfb_mlp8_dw8", _p(x8), _p(dp8), _p(hq8), _p(dy8), _p(row), xf, _p(dw_fc), _p(dw_proj), M, d, F,
-              int(dw_fc.dtype == torch.float32), int(accumulate), _p(ws), ws.numel() * 4, xd, _stream())
-    return dw_fc, dw_proj
+    return native.tfb_mlp8_dw8(x8, dp8, hq8, dy8, row, x_scale, dw_fc, dw_proj, accumulate, out_dtype == torch.float32)
 
 
 def mlp_dw_proj(dy2, r, out=None, accumulate=False, out_dtype=bf16):
     """dw_proj [d,F] (+)= dy^T @ bf16(r^2) without materialising h."""
-    _chk(dy2), _chk(r)
-    M, d = dy2.shape
-    F = r.shape[1]
-    if out is None:
-        out = torch.empty(d, F, dtype=out_dtype, device=dy2.device)
-    ws = _workspace(dy2.device)
-    _lib.call("tfb_mlp_dw_proj", _p(dy2), _p(r), _p(out), M, d, F, int(out.dtype == torch.float32), int(accumulate), _p(ws),
-              ws.numel() * 4, _stream())
-    return out
+    return native.tfb_mlp_dw_proj(dy2, r, out, accumulate, out_dtype == torch.float32)
 
 
 # ------------------------------------------------------------------------------------------ attention
@@ -580,24 +361,15 @@ def attn_bwd_static(q, k, v, o, do, lse, scale, dq, dk, dv, layout="bhtd", out_l
 
 # ------------------------------------------------------------------------------------------ elementwise
 def relu2(x):
-    _chk(x)
-    out = torch.empty_like(x)
-    _lib.call("tfb_relu2", _p(x), None, _p(out), x.numel(), 0, _stream())
-    return out
+    return native.tfb_relu2(x, None, 0)
 
 
 def relu2_bwd(x, gy):
-    _chk(x), _chk(gy)
-    out = torch.empty_like(x)
-    _lib.call("tfb_relu2", _p(x), _p(gy), _p(out), x.numel(), 1, _stream())
-    return out
+    return native.tfb_relu2(x, gy, 1)
 
 
 def relu2_bwd_from_h(h, dh):
-    _chk(h), _chk(dh)
-    out = torch.empty_like(h)
-    _lib.call("tfb_relu2", _p(h), _p(dh), _p(out), h.numel(), 2, _stream())
-    return out
+    return native.tfb_relu2(h, dh, 2)
 
 
 def rope_(x, cos, sin, T, nheads, D, inverse=False, out=None):
@@ -659,15 +431,7 @@ def resmix_bwd(g, x, x0, ab):
 
 def embedding_fwd(idx, weight):
     """weight rows gathered by idx; an id outside [0, V) gives a zero row (and receives no gradient in embedding_bwd)."""
-    _chk(weight)
-    if idx.dtype not in (torch.int64, torch.int32) or not idx.is_cuda:
-        raise TypeError("idx must be an int32/int64 device tensor")
-    idx = idx.contiguous()
-    C = weight.shape[1]
-    out = torch.empty(*idx.shape, C, dtype=bf16, device=weight.device)
-    _lib.call("tfb_embedding_fwd", _p(idx), int(idx.dtype == torch.int64), _p(weight), _p(out), idx.numel(), C,
-              weight.shape[0], _stream())
-    return out
+    return native.tfb_embedding_fwd(idx, weight)
 
 
 def embedding_bwd(idx, dy, dw, grouped=True):
@@ -687,20 +451,13 @@ def embedding_bwd(idx, dy, dw, grouped=True):
 
 
 def fill_f32_(t, val=0.0):
-    _chk(t, torch.float32)
-    _lib.call("tfb_fill_f32", _p(t), float(val), t.numel(), _stream())
+    native.tfb_fill_f32(t, val)
     return t
 
 
 def adamw_(p, g, m, v, step, lr, beta1, beta2, eps, weight_decay, p_bf16=None):
     """One in-place AdamW update of the fp32 master p (and its optional bf16 copy) from g (fp32 or bf16)."""
-    _chk(p, torch.float32), _chk(m, torch.float32), _chk(v, torch.float32), _chk(g, g.dtype), _chk(p_bf16)
-    if g.dtype not in (torch.float32, bf16):
-        raise TypeError("grad must be fp32 or bf16")
-    bias1 = 1.0 - beta1 ** step
-    bias2 = 1.0 - beta2 ** step
-    _lib.call("tfb_adamw", _p(p), _p(g), int(g.dtype == torch.float32), _p(m), _p(v), _p(p_bf16), p.numel(), float(lr),
-              float(weight_decay), float(1.0 - beta1), float(1.0 - beta2), float(eps), float(bias1), float(bias2), _stream())
+    native.tfb_adamw(p, g, m, v, step, lr, beta1, beta2, eps, weight_decay, p_bf16)
 
 
 # ------------------------------------------------------------------------------------------ loss head
@@ -712,35 +469,18 @@ def _tg(targets):
 
 def loss_fwd(logits2, targets, softcap=15.0, row_w=None):
     """Row losses (already multiplied by row_w) and lse, from bf16 logits [N, V]; targets < 0 are ignored."""
-    _chk(logits2), _chk(row_w, torch.float32)
-    tg = _tg(targets)
-    N, V = logits2.shape
-    loss = torch.empty(N, dtype=torch.float32, device=logits2.device)
-    lse = torch.empty(N, dtype=torch.float32, device=logits2.device)
-    _lib.call("tfb_loss_fwd", _p(logits2), _p(tg), int(tg.dtype == torch.int64), _p(row_w), _p(loss), _p(lse), N, V,
-              float(softcap or 0.0), _stream())
-    return loss, lse
+    return native.tfb_loss_fwd(logits2, targets, row_w, softcap)
 
 
 def loss_bwd(logits2, targets, lse, grow, softcap=15.0, inplace=False):
     """dlogits bf16 [N, V]; grow fp32 [N] = d(total)/d(row loss) * row weight."""
-    _chk(logits2), _chk(lse, torch.float32), _chk(grow, torch.float32)
-    tg = _tg(targets)
-    N, V = logits2.shape
-    out = logits2 if inplace else torch.empty_like(logits2)
-    _lib.call("tfb_loss_bwd", _p(logits2), _p(tg), int(tg.dtype == torch.int64), _p(lse), _p(grow), _p(out), N, V,
-              float(softcap or 0.0), _stream())
-    return out
+    return native.tfb_loss_bwd(logits2, targets, lse, grow, softcap, inplace)
 
 
 def loss_row_weights(targets, reduction="mean", V=None):
     """fp32 [N] weights of the row losses in the reduced loss: valid / max(1, count of valid) for "mean", valid for "sum";
     a row is valid when 0 <= t < V (the rows the loss kernels give a loss to; V None: when t >= 0)."""
-    tg = _tg(targets)
-    w = torch.empty(tg.numel(), dtype=torch.float32, device=tg.device)
-    _lib.call("tfb_loss_row_weights", _p(tg), int(tg.dtype == torch.int64), _p(w), tg.numel(), int(reduction == "mean"),
-              int(V or 0), _stream())
-    return w
+    return native.tfb_loss_row_weights(targets, reduction == "mean", V)
 
 
 LOSS_FWD_BWD_MAX_V = 65536
@@ -749,14 +489,11 @@ LOSS_FWD_BWD_MAX_V = 65536
 def loss_fwd_bwd(logits2, targets, row_w=None, softcap=15.0):
     """(loss rows fp32 [N], lse fp32 [N]) as loss_fwd gives them, and logits2 OVERWRITTEN by the gradient of sum(rows):
     row_w (softmax - onehot) (1 - tanh^2), what loss_bwd gives for grow = row_w. One pass over the logits; V <= 65536."""
-    _chk(logits2), _chk(row_w, torch.float32)
-    tg = _tg(targets)
-    N, V = logits2.shape
-    loss = torch.empty(N, dtype=torch.float32, device=logits2.device)
-    lse = torch.empty(N, dtype=torch.float32, device=logits2.device)
-    _lib.call("tfb_loss_fwd_bwd", _p(logits2), _p(tg), int(tg.dtype == torch.int64), _p(row_w), _p(loss), _p(lse), N, V,
-              float(softcap or 0.0), _stream())
-    return loss, lse
+    return native.tfb_loss_fwd_bwd(logits2, targets, row_w, softcap)
+
+
+# The functions a program may wrap by assigning to this module's name: the native nodes call what stands there.
+_WRAPPABLE = {"mlp8_backward_scales": mlp8_backward_scales, "loss_fwd_bwd": loss_fwd_bwd}
 
 
 def loss_multi_fwd(logits2, targets, row_w, softcap=15.0, eps=0.0):
@@ -790,17 +527,7 @@ def loss_multi_bwd(logits2, targets, row_w, lse, g, softcap=15.0, eps=0.0, inpla
 def lmhead_fwd(x2, W, targets, softcap=None, row_w=None):
     """logits = x2 @ W^T (W [V, d]) with the row log-sum-exp fused into the GEMM epilogue.
     Returns (logits bf16 [N, V], loss rows fp32 [N], lse fp32 [N])."""
-    _chk(x2), _chk(W), _chk(row_w, torch.float32)
-    tg = _tg(targets)
-    N, d = x2.shape
-    V = W.shape[0]
-    logits = torch.empty(N, V, dtype=bf16, device=x2.device)
-    part = torch.empty(N, V // 64, 2, dtype=torch.float32, device=x2.device)
-    loss = torch.empty(N, dtype=torch.float32, device=x2.device)
-    lse = torch.empty(N, dtype=torch.float32, device=x2.device)
-    _lib.call("tfb_lmhead_fwd", _p(x2), _p(W), _p(tg), int(tg.dtype == torch.int64), _p(row_w), _p(logits), _p(part), _p(loss),
-              _p(lse), N, d, V, float(softcap or 0.0), _stream())
-    return logits, loss, lse
+    return native.tfb_lmhead_fwd(x2, W, targets, softcap, row_w)
 
 
 # ------------------------------------------------------------------------------------------ mixture of experts
@@ -1108,31 +835,13 @@ def ns5(g, d, coeffs=NS_COEFFS):
 def mlp_fwd(x2, w_fc, w_proj):
     """(y [M,d], r [M,F]) bf16: y = bf16(bf16(r r) @ w_proj^T), r = bf16(relu(x2 @ w_fc^T)); w_fc [F,d], w_proj [d,F]
     (K/nki_mlp_fused.py:242). r is token-major (the reference's rT is r.t())."""
-    _chk(x2), _chk(w_fc), _chk(w_proj)
-    M, d = x2.shape
-    F = w_fc.shape[0]
-    if tuple(w_fc.shape) != (F, d) or tuple(w_proj.shape) != (d, F):
-        raise ValueError("w_fc is [F, d], w_proj is [d, F]")
-    y = torch.empty(M, d, dtype=bf16, device=x2.device)
-    r = torch.empty(M, F, dtype=bf16, device=x2.device)
-    h = torch.empty(M, F, dtype=bf16, device=x2.device)
-    _lib.call("tfb_mlp_fwd", _p(x2), _p(w_fc), _p(w_proj), _p(y), _p(r), _p(h), M, d, F, _stream())
-    return y, r
+    return native.tfb_mlp_fwd(x2, w_fc, w_proj)
 
 
 def mlp_bwd(dy2, r, w_fc, w_proj, want_h=True):
     """(dx [M,d], h [M,F] or None, dpre [M,F]) bf16: dpre = bf16(((dy2 @ w_proj) 2) r), h = bf16(r r), dx = bf16(dpre @ w_fc)
     (K/nki_mlp_fused.py:290 with dw_mode 0)."""
-    _chk(dy2), _chk(r), _chk(w_fc), _chk(w_proj)
-    M, d = dy2.shape
-    F = w_fc.shape[0]
-    if tuple(r.shape) != (M, F) or tuple(w_fc.shape) != (F, d) or tuple(w_proj.shape) != (d, F):
-        raise ValueError("shapes differ")
-    dx = torch.empty(M, d, dtype=bf16, device=dy2.device)
-    dpre = torch.empty(M, F, dtype=bf16, device=dy2.device)
-    h = torch.empty(M, F, dtype=bf16, device=dy2.device) if want_h else None
-    _lib.call("tfb_mlp_bwd", _p(dy2), _p(r), _p(w_fc), _p(w_proj), _p(dx), _p(h), _p(dpre), M, d, F, _stream())
-    return dx, h, dpre
+    return native.tfb_mlp_bwd(dy2, r, w_fc, w_proj, want_h)
 
 
 # ------------------------------------------------------------------------------------------ gradient norm
@@ -1154,23 +863,9 @@ def gradnorm(g_bf16=None, g_f32=None, clip=0.0):
 def mix_tail_fwd(x2, lam, T, eps=2.0 ** -23):
     """(s1, xn2, inv): s1 = bf16(x2 + bf16(lam shift1(x2))) with shift1 inside sequences of T rows, xn2 = RMSNorm(s1);
     lam a 1-element fp32 device tensor (R1:7097)."""
-    _chk(x2), _chk(lam, torch.float32)
-    rows, C = x2.shape
-    s1, xn2 = torch.empty_like(x2), torch.empty_like(x2)
-    inv = torch.empty(rows, dtype=torch.float32, device=x2.device)
-    _lib.call("tfb_mix_tail_fwd", _p(x2), _p(lam), _p(s1), _p(xn2), _p(inv), rows, C, int(T), float(eps), _stream())
-    return s1, xn2, inv
+    return native.tfb_mix_tail_fwd(x2, lam, T, eps)
 
 
 def mix_tail_bwd(s1, inv, x2, lam, T, gy=None, ge=None):
     """(gx bf16 [rows,C], dlam fp32 [1]) from the gradients gy of xn2 and ge of s1 (either may be None) (R1:7145)."""
-    _chk(s1), _chk(x2), _chk(gy), _chk(ge), _chk(inv, torch.float32), _chk(lam, torch.float32)
-    if gy is None and ge is None:
-        raise ValueError("give gy or ge")
-    rows, C = s1.shape
-    gx = torch.empty_like(s1)
-    part = _scratch(s1.device, int(_lib.lib().tfb_norm_bwd_blocks(rows)))
-    dlam = torch.empty(1, dtype=torch.float32, device=s1.device)
-    _lib.call("tfb_mix_tail_bwd", _p(s1), _p(gy), _p(ge), _p(inv), _p(x2), _p(lam), _p(gx), _p(part), _p(dlam), rows, C, int(T),
-              _stream())
-    return gx, dlam
+    return native.tfb_mix_tail_bwd(s1, inv, x2, lam, T, gy, ge)

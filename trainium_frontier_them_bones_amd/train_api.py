@@ -74,24 +74,18 @@ def nki_rope_attention(qkv, cos, sin, n_head, scale=None, nw=None):
     sc = float(scale) if scale is not None else 1.0 / math.sqrt(D)
     c, s = _tables_2d(cos, sin, T, D // 2)
     y = _none_if_shape(A.RopeNormAttentionFn.apply, qkv, c, s, n_head, sc, RMS_EPS, int(nw) if nw else 0)
-    return None if y is None else y.view(B, T, n_head, D)
+    return y
 
 
 # ------------------------------------------------------------------------------------------ loss head (R1:4691, 4908; R2:6364)
 def fused_loss(logits, targets, reduction="mean", softcap=LOGIT_SOFTCAP):
     """The static cross-entropy chain on the raw lm_head output (R1:4691): softcap * tanh(logits / softcap), log-softmax,
     ignore_index -1; reduction "mean" (over the targets not ignored), "sum" or "none" (rows in targets' shape)."""
-    V = logits.shape[-1]
-    x2 = logits.reshape(-1, V).contiguous()
-    t = targets.reshape(-1)
-    rows = A.FusedLossFn.apply(x2, t, softcap)
     if reduction == "none":
-        return rows.view(targets.shape)
-    if reduction == "sum":
-        return rows.sum()
-    if reduction != "mean":
+        return A.LossRowsFn.apply(logits.contiguous(), targets, softcap).view(targets.shape)
+    if reduction not in ("mean", "sum"):
         raise ValueError("reduction must be 'mean', 'sum' or 'none'")
-    return rows.sum() / ((t >= 0) & (t < V)).sum().clamp_min(1).to(rows.dtype)   # the rows the kernel gives a loss to
+    return A.FusedLossFn.apply(logits, targets, reduction == "mean", softcap)   # (the rows the kernel gives a loss to)
 
 
 def fused_loss_multi(logits, tg, rw, softcap=LOGIT_SOFTCAP, ref=None):
@@ -130,9 +124,7 @@ def _gain(l, like):
 
 def block_head(x, x0, l1, l2):
     """(l1*x + l2*x0, norm(l1*x + l2*x0)) (R1:5578); l1, l2 one-element tensors (the model's learnable gains)."""
-    C = x.shape[-1]
-    x_new, x_norm = A.BlockHeadFn.apply(x.reshape(-1, C), x0.reshape(-1, C), _gain(l1, x), _gain(l2, x), None, None, RMS_EPS)
-    return x_new.view(x.shape), x_norm.view(x.shape)
+    return A.BlockHeadFn.apply(x, x0, _gain(l1, x), _gain(l2, x), None, None, RMS_EPS)
 
 
 def head_skip(x, x0, skip, l1, l2, l3):
@@ -140,10 +132,7 @@ def head_skip(x, x0, skip, l1, l2, l3):
     eager form 5644-5647). skip None = the plain block head."""
     if skip is None:
         return block_head(x, x0, l1, l2)
-    C = x.shape[-1]
-    x_new, x_norm = A.BlockHeadFn.apply(x.reshape(-1, C), x0.reshape(-1, C), _gain(l1, x), _gain(l2, x),
-                                        skip.reshape(-1, C), _gain(l3, x), RMS_EPS)
-    return x_new.view(x.shape), x_norm.view(x.shape)
+    return A.BlockHeadFn.apply(x, x0, _gain(l1, x), _gain(l2, x), skip, _gain(l3, x), RMS_EPS)
 
 
 SELF_SKIP = object()   # head2's marker: the skip is the block's own (materialised) input (R1: mblk_SELF_SKIP)
@@ -162,22 +151,17 @@ def head2(x, x0, skip, l1, l2, l3, emit=False, key=None):
 
 def rmsnorm_fast(x):
     """F.rms_norm(x, (C,)) (R1:5594)."""
-    C = x.shape[-1]
-    return A.RMSNormFn.apply(x.reshape(-1, C), None, RMS_EPS).view(x.shape)
+    return A.RMSNormFn.apply(x, None, RMS_EPS)
 
 
 def tail_norm2(x_new, attn_out):
     """(x_new + attn_out, norm(x_new + attn_out)) (R1:6117)."""
-    C = x_new.shape[-1]
-    s1, y = A.AddRMSNormFn.apply(x_new.reshape(-1, C), attn_out.reshape(-1, C), None, RMS_EPS)
-    return s1.view(x_new.shape), y.view(x_new.shape)
+    return A.AddRMSNormFn.apply(x_new, attn_out, None, RMS_EPS)
 
 
 def final_norm(s1, mo):
     """norm(s1 + mo): the last block's residual add and the final RMSNorm (R1:6826)."""
-    C = s1.shape[-1]
-    _, y = A.AddRMSNormFn.apply(s1.reshape(-1, C), mo.reshape(-1, C), None, RMS_EPS)
-    return y.view(s1.shape)
+    return A.AddRMSNormFn.apply(s1, mo, None, RMS_EPS)[1]
 
 
 def relu_squared(x):
@@ -280,17 +264,13 @@ def mlp_fused8(mlp, x):
     if getattr(mlp, "tfb_mlp8", None) is None or mlp.tfb_mlp8.row is None:
         fp8_refresh_weights([mlp])
     b, t, c = x.shape
-    x2 = x.reshape(b * t, c)
-    m = x2.shape[0]
+    m = b * t
     pad = (-m) % 128
-    if pad:
-        x2 = torch.nn.functional.pad(x2, (0, 0, 0, pad))
+    x2 = torch.nn.functional.pad(x.reshape(m, c), (0, 0, 0, pad)) if pad else x
     w_fc = mlp.c_fc.weight if mlp.c_fc.weight.dtype == bf16 else mlp.c_fc.weight.to(bf16)
     w_proj = mlp.c_proj.weight if mlp.c_proj.weight.dtype == bf16 else mlp.c_proj.weight.to(bf16)
     y = A.Mlp8Fn.apply(x2, w_fc, w_proj, mlp.tfb_mlp8)
-    if pad:
-        y = y[:m]
-    return y.reshape(b, t, c)
+    return y[:m].reshape(b, t, c) if pad else y
 
 
 def moe_refresh_weights(moe, *, e4m3_limit=240.0, x_scale=4.0):
@@ -348,19 +328,15 @@ def nr_mlp(mlp, x1):
     if getattr(mlp, "tfb_mlp8", None) is None or mlp.tfb_mlp8.row is None:
         fp8_refresh_weights([mlp])
     b, t, c = x1.shape
-    x2 = x1.reshape(b * t, c)
-    if x2.dtype != bf16:
-        raise RuntimeError("the folded MLP takes bf16 rows, not %s" % x2.dtype)
-    m = x2.shape[0]
+    if x1.dtype != bf16:
+        raise RuntimeError("the folded MLP takes bf16 rows, not %s" % x1.dtype)
+    m = b * t
     pad = (-m) % 128
-    if pad:
-        x2 = torch.nn.functional.pad(x2, (0, 0, 0, pad))
+    x2 = torch.nn.functional.pad(x1.reshape(m, c), (0, 0, 0, pad)) if pad else x1
     w_fc = mlp.c_fc.weight if mlp.c_fc.weight.dtype == bf16 else mlp.c_fc.weight.to(bf16)
     w_proj = mlp.c_proj.weight if mlp.c_proj.weight.dtype == bf16 else mlp.c_proj.weight.to(bf16)
     xo = A.NrMlpFn.apply(x2, w_fc, w_proj, mlp.tfb_mlp8)
-    if pad:
-        xo = xo[:m]
-    return xo.reshape(b, t, c)
+    return xo[:m].reshape(b, t, c) if pad else xo
 
 
 def proj_residual(x, w, res):
@@ -501,11 +477,7 @@ def mlp_bwd_kernel(dy2, rT, w_fc, w_proj, tb=None, dw_mode=0):
 def mlp_fused(mlp, x):
     """MLP.forward on [b, t, n_embd] through the dense bf16 fused kernels (R2:6782): `mlp` has c_fc.weight [F, d] and
     c_proj.weight [d, F]. Raises TfbError for a shape the kernels do not take (the round-2 policy)."""
-    b, t, c = x.shape
-    x2 = x.reshape(b * t, c).contiguous()
-    w_fc = mlp.c_fc.weight.to(dtype=x.dtype)
-    w_proj = mlp.c_proj.weight.to(dtype=x.dtype)
-    return A.MlpFusedFn.apply(x2, w_fc, w_proj).view(b, t, c)
+    return A.MlpFusedFn.apply(x, mlp.c_fc.weight.to(dtype=x.dtype), mlp.c_proj.weight.to(dtype=x.dtype))
 
 
 # ------------------------------------------------------------------------------------------ gradient norm (R1:1480, 1634)
@@ -526,6 +498,4 @@ def shift1(x):
 def mix_tail(x, xn_dead, lam):
     """(s1, xn2) = (x + lam * shift1(x), RMSNorm(s1)) for a [B, T, C] stream in one launch each way (R1:7308). xn_dead (the
     head's unused x_norm) is accepted for the reference's signature and not read."""
-    B, T, C = x.shape
-    s1, y = A.MixTailFn.apply(x.reshape(B * T, C), lam, T)
-    return s1.view(B, T, C), y.view(B, T, C)
+    return A.MixTailFn.apply(x, lam, x.shape[1])
