@@ -613,6 +613,87 @@ def test_mlp8_weight_stationary_kernel_equals_the_tiled_kernel(ops, dev, M, Ms, 
     assert torch.equal(dp8[:Ms], dp8s) and torch.equal(hq8[:Ms], hq8s) and torch.equal(dxq[:Ms], dxqs) and torch.equal(dxq, dx)
 
 
+@pytest.mark.parametrize("M,Ms,F", [(10752, 10624, 3072), (16384, 16256, 2304)])
+def test_mlp8_weight_stationary_kernel_at_the_smallest_batches_it_takes(ops, dev, M, Ms, F):
+    """The weight-stationary kernel runs from eight token tiles per CU on: the shared rows of a batch it takes and of one of
+    M - 128 tokens (tiled kernel) are equal bit for bit, forward and backward."""
+    d = 768
+    g = _g(77 + F)
+    x = torch.randn(M, d, generator=g).bfloat16().to(dev)
+    wf = (0.02 * torch.randn(F, d, generator=g)).bfloat16().to(dev)
+    wp = (0.02 * torch.randn(d, F, generator=g)).bfloat16().to(dev)
+    dy = torch.randn(M, d, generator=g).bfloat16().to(dev)
+    row = ops.mlp8_forward_scales(wf, wp, 448.0)
+    w8 = ops.mlp8_precast(wf, wp, row)
+    y, r = ops.mlp8_fwd(x, w8, row, F)
+    ys, rs = ops.mlp8_fwd(x[:Ms].contiguous(), w8, row, F)
+    assert torch.equal(r[:Ms], rs) and torch.equal(y[:Ms], ys)
+    rowb = ops.mlp8_backward_scales(dy, row)
+    dx, _, dp8, hq8, _ = ops.mlp8_bwd_q(dy, r, w8, rowb, 448.0, want_dpre=False)
+    dxs, _, dp8s, hq8s, _ = ops.mlp8_bwd_q(dy[:Ms].contiguous(), rs, w8, rowb, 448.0, want_dpre=False)
+    assert torch.equal(dp8[:Ms], dp8s) and torch.equal(hq8[:Ms], hq8s) and torch.equal(dx[:Ms], dxs)
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 128, 64), (128, 256, 128), (128, 384, 192), (256, 128, 256), (256, 768, 320), (1024, 1024, 448),
+                                   (1152, 1024, 768), (2048, 1024, 768), (2176, 1024, 832), (128, 1024, 4096), (256, 512, 6144), (128, 128, 8192)])
+def test_small_output_gemms_in_every_operand_layout(ops, dev, M, N, K):
+    """Launches of few tiles run the ring kernel (64 x 64 tiles up to one per CU, then 128 x 64, contractions of 1 to 96 k-tiles of 64,
+    cut into k ranges when a quarter of the CUs or less have a tile): all four operand layouts against the fp32 product, a scaled
+    and an accumulating fp32 store, and the residual store; without a k-split the rows equal those of a large launch bit for bit."""
+    g = _g(M + N + K)
+    a = torch.randn(M, K, generator=g).bfloat16().to(dev)
+    b = (K ** -0.5 * torch.randn(N, K, generator=g)).bfloat16().to(dev)
+    want = a.float() @ b.float().t()
+    al = torch.tensor([0.37], device=dev)
+    base = torch.randn(M, N, generator=g).to(dev)
+    outs = []
+    for ta in (False, True):
+        for tb in (True, False):
+            x, w = (a.t().contiguous() if ta else a), (b if tb else b.t().contiguous())
+            y = ops.matmul(x, w, trans_a=ta, trans_b=tb)
+            assert rel_l2(y, want) < 3e-3, (ta, tb)
+            outs.append(y)
+            acc = ops.matmul(x, w, trans_a=ta, trans_b=tb, out=base.clone(), accumulate=True, alpha=al)
+            assert rel_l2(acc, base + 0.37 * want) < 1e-4, (ta, tb)
+            if not ta:
+                res = base.bfloat16()
+                z = ops.matmul_res(x, w, res, trans_b=tb)
+                assert rel_l2(z, res.float() + want) < 4e-3
+    assert all(torch.equal(o, outs[0]) for o in outs)
+    if K < 2048:
+        big = ops.matmul(a.repeat(-(-32768 // M), 1), b, trans_b=True)
+        assert torch.equal(big[:M], outs[0])
+
+
+@pytest.mark.parametrize("M,d,F", [(128, 256, 256), (256, 256, 1024), (384, 768, 3072), (1920, 1024, 2048), (2432, 768, 3072)])
+def test_small_fp8_mlps_equal_the_rows_of_a_large_one(ops, dev, M, d, F):
+    """The fp8 MLP of a small batch (ring kernel in all six GEMMs) against the same rows of a batch that takes the large kernels,
+    bit for bit in the activations; its weight gradients, whose contraction is the batch, against the fp32 product of the bytes."""
+    g = _g(M + d + F)
+    big = -(-16384 // M) * M
+    x = torch.randn(big, d, generator=g).bfloat16().to(dev)
+    wf = (0.02 * torch.randn(F, d, generator=g)).bfloat16().to(dev)
+    wp = (0.02 * torch.randn(d, F, generator=g)).bfloat16().to(dev)
+    dy = torch.randn(big, d, generator=g).bfloat16().to(dev)
+    row = ops.mlp8_forward_scales(wf, wp)
+    w8 = ops.mlp8_precast(wf, wp, row)
+    rowb = ops.mlp8_backward_scales(dy, row)
+    out = []
+    for n in (M, big):
+        y, r, x8 = ops.mlp8_fwd(x[:n].contiguous(), w8, row, F, want_x8=True)
+        yr, _ = ops.mlp8_fwd(x[:n].contiguous(), w8, row, F, res=x[:n].contiguous())
+        dx, _, dp8, hq8, dy8 = ops.mlp8_bwd_q(dy[:n].contiguous(), r, w8, rowb, want_dpre=False)
+        out.append((y, r, x8, yr, dx, dp8, hq8, dy8))
+    for s, b in zip(*out):
+        assert torch.equal(s, b[:M])
+    _, _, x8, _, _, dp8, hq8, dy8 = out[0]
+    dwf, dwp = ops.mlp8_dw8(x8, dp8, hq8, dy8, rowb)
+    e4, e5 = torch.float8_e4m3fn, torch.float8_e5m2
+    rb = rowb.cpu()
+    assert rel_l2(dwf, dp8.view(e5).float().t() @ x8.view(e4).float() / (rb[7] * 4.0).item()) < BF16_TOL
+    assert rel_l2(dwp, dy8.view(e5).float().t() @ hq8.view(e4).float() / (rb[5] * rb[13]).item()) < BF16_TOL
+
+
 @pytest.mark.parametrize("fmt", [0, 1])
 def test_fp8_projection_weight_stationary_kernel_equals_the_tiled_kernel(ops, dev, fmt):
     """tfb_gemm_fp8 / tfb_gemm_fp8_res with a contraction of 768 bytes: a batch of a multiple of 512 tokens runs the

@@ -4,6 +4,7 @@
 // Replaces the reference's nki_matmul(a, b, trans_a, trans_b) (round1/source/train.py:1137)
 // and the torch matmuls its Linear glue issues (round1/source/train.py:8419-8711).
 #include "gemm_pp.hpp"
+#include "gemm_ring.hpp"
 
 namespace {
 
@@ -49,6 +50,20 @@ int run(GemmOperand P, GemmOperand Q, int N, int M, int K, void* C, int out_f32,
   }
   const long tiles = (long)(N / 128) * (M / 128);
   const int splits = ws ? choose_splits(tiles, K / 64, (long)M * N, ws_bytes) : 1;
+  // few output tiles: the ring kernel, its k ranges inside the workgroups, or in workgroups of their own where a quarter of the CUs
+  // or less have a tile (256 x 1024 x 4096: 13.7 -> 11.6 us)
+  if (const int pick = gemm_ring_pick(N, M, K / 64, LAYP == TFB_K_STRIDED && LAYQ == TFB_K_STRIDED)) {
+    GemmArgs a = {};
+    a.P = P;
+    a.Q = Q;
+    a.np = N;
+    a.nq = M;
+    a.nkt = K / 64;
+    if (splits == 1 || 4 * (long)(N / 64) * (M / 64) > tfb_resident_slots(1))
+      return gemm_ring_launch<EpiStore, 2, LAYP, LAYQ, 0, 0>(pick, a, 1, 1, EpiStore{C, (long)N, out_f32, accumulate, alpha}, stream, splits);
+    const int st = gemm_ring_launch<EpiSplit, 2, LAYP, LAYQ, 0, 0>(pick, a, 1, splits, EpiSplit{ws, (long)N, (long)M * N}, stream);
+    return st != TFB_OK ? st : splitk_reduce(ws, C, (long)M * N, splits, out_f32, accumulate, stream, nullptr, nullptr, 1.0f, alpha);
+  }
   if (splits == 1) {
     EpiStore e{C, (long)N, out_f32, accumulate, alpha};
     // large outputs: the persistent 256 x 256 kernel (same sums in the same order), in any operand layout (the input
@@ -160,6 +175,10 @@ extern "C" int tfb_gemm_bf16_res(const void* A, const void* B, const void* res, 
   if (M <= 0 || N <= 0 || K <= 0 || M % 128 || N % 128 || K % 64) return TFB_ERR_SHAPE;
   GemmOperand P{(const uint8_t*)B, trans_b ? (long)K * 2 : (long)N * 2}, Q{(const uint8_t*)A, (long)K * 2};
   EpiStoreRes e{(bf16_t*)C, (const bf16_t*)res, (long)N};
+  int st;
+  if (trans_b ? gemm_ring_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream, st)
+              : gemm_ring_try<2, TFB_K_STRIDED, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream, st))
+    return st;
   if (trans_b && gemm_pp_applies(N, M, (long)K * 2)) return gemm_pp_launch<2, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream);
   if (trans_b)
     return gemm_launch<GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>>(P, Q, N, M, (long)K * 2, 1, LoadIdentity{},
@@ -179,6 +198,8 @@ extern "C" int tfb_qkv_rope_fwd(const void* x, const void* w, const void* cos_t,
   using Cfg = GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>;
   GemmOperand P{(const uint8_t*)w, (long)K * 2}, Q{(const uint8_t*)x, (long)K * 2};
   EpiStoreRope e{(bf16_t*)out, (long)N, (const bf16_t*)cos_t, (const bf16_t*)sin_t, T, rot_cols};
+  int st;
+  if (gemm_ring_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream, st)) return st;
   if (gemm_pp_applies(N, M, (long)K * 2)) return gemm_pp_launch<2, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream);
   return gemm_launch<Cfg>(P, Q, N, M, (long)K * 2, 1, LoadIdentity{}, LoadIdentity{}, e, (hipStream_t)stream);
 }

@@ -80,6 +80,8 @@ struct GemmArgs {
   int rows;     // block traversal: rows of tiles of the other operand in one XCD's run (0: plain traversal)
   int blk;      // gblock * rows
   FastDiv d_ntiles, d_per, d_nfast, d_blk, d_gblock, d_splits, d_split8;  // d_split8: by splits / 8
+  int ranges;   // ring kernel: k ranges summed separately inside one workgroup, then added in order (see there)
+  FastDiv d_ranges;
 };
 
 // Operand pre-operation, applied to a fragment (8 bf16 along k of one row) on its way into the MFMA.
@@ -153,15 +155,23 @@ struct TileDma<ROWS, NW, TFB_K_CONTIG, ES> {
   }
 };
 
+// slot swizzle of the K_STRIDED layout (chunk c of k-row k at slot c ^ tfb_ks_swz(k)): the transposing reads of 32 lanes (4 k-rows
+// x 64 bytes in bf16, 8 x 32 in fp8) then cover all 64 banks once
+template <int ROWS, int ES>
+__device__ __forceinline__ int tfb_ks_swz(int k) {
+  if (ES == 2) return ROWS == 64 ? 4 * ((k >> 1) & 1) : 4 * (k & 3);
+  return ROWS == 64 ? 2 * ((k >> 2) & 1) : 2 * ((k >> 1) & 3);
+}
+
 template <int ROWS, int NW, int ES>
 struct TileDma<ROWS, NW, TFB_K_STRIDED, ES> {
   static constexpr int LPR = ROWS * ES / 16;   // lanes (16-byte chunks) per k-row
   static constexpr int RPI = 64 / LPR;         // k-rows per instruction
   static constexpr int KROWS = 128 / ES;       // k-rows per tile
   static constexpr int NI = KROWS / RPI / NW;  // = ROWS / 8 / NW
-  // the swizzle term (k & 3 for bf16, (k >> 1) & 3 for fp8) must not depend on the instruction index
+  // the swizzle term must not depend on the instruction index
   static_assert((NW * RPI) % (ES == 2 ? 4 : 8) == 0, "swizzle phase vs instruction index");
-  static_assert(ES == 2 || ROWS == 128, "fp8 K_STRIDED tiles are 128 rows");
+  static_assert(ES == 2 || ROWS == 128 || ROWS == 64, "fp8 K_STRIDED tiles are 64 or 128 rows");
   const uint8_t* base;
   long step, tstep;
   uint32_t voff;
@@ -172,7 +182,7 @@ struct TileDma<ROWS, NW, TFB_K_STRIDED, ES> {
     step = (long)NW * RPI * o.ld;
     tstep = (long)KROWS * o.ld;
     const int k = wave * RPI + kl;  // the swizzle phase of the k-row this lane fills, the same for every instruction
-    const int sw = ES == 2 ? 4 * (k & 3) : 2 * ((k >> 1) & 3);
+    const int sw = tfb_ks_swz<ROWS, ES>(k);
     voff = (uint32_t)(kl * o.ld + ((slot ^ sw) * 16));
   }
   __device__ __forceinline__ void issue(uint8_t* lds, int t, int wave) const {
@@ -344,6 +354,48 @@ struct prefetch_type { typedef int type; };
 template <class T>
 struct prefetch_type<T, true> { typedef typename T::pre_t type; };
 
+__device__ __forceinline__ void gemm_tile_of(const GemmArgs& a, int L, int& lid, int& split, int& tile_p, int& tile_q) {
+  // Workgroup -> (output tile, k-split). Consecutive workgroup ids sit on consecutive XCDs. With a multiple of 8 splits a
+  // split stays on ONE XCD: the k-range of both operands it contracts over is then fetched into that XCD's L2 once and
+  // shared by all its output tiles, instead of every XCD streaming most of both operands. Without splits, ids are
+  // re-dealt so that one XCD gets a contiguous run of tiles. (Everything up to the first operand load below is serial
+  // scalar work in front of every tile: the divisions are multiplications prepared by the host.)
+  auto xcd_run = [&](int pid) { return a.per ? (pid & 7) * a.per + (pid >> 3) : pid; };
+  {
+    if (a.splits == 1) {
+      split = 0;
+      lid = xcd_run(L);
+    } else if ((a.splits & 7) == 0) {
+      const int j = L >> 3;
+      lid = fastdiv(j, a.d_split8);
+      split = (L & 7) + 8 * (j - lid * (a.splits >> 3));
+    } else {
+      split = fastdiv(L, a.d_ntiles);
+      lid = xcd_run(L - split * a.ntiles);
+    }
+  }
+  // An XCD's run of tiles walks the smaller operand's tiles fastest: the run then shares few rows of the larger
+  // operand (which is thereby partitioned over the XCDs' L2s) and re-reads the smaller one. When the smaller operand
+  // does not fit the L2 beside the streaming larger one (a 3.5 MB weight against a 4 MB L2), the run is walked in
+  // blocks of `gblock` of its tiles: block 0 against all of the run's rows of the larger operand, then block 1, ...
+  // so the smaller operand is fetched once per XCD instead of once per row of tiles.
+  {
+    int fast, slow;
+    if (a.rows > 0) {
+      const int xcd = fastdiv(lid, a.d_per), idx = lid - xcd * a.per;
+      const int b = fastdiv(idx, a.d_blk), rem = idx - b * a.blk;
+      const int rg = fastdiv(rem, a.d_gblock);
+      fast = b * a.gblock + rem - rg * a.gblock;
+      slow = xcd * a.rows + rg;
+    } else {
+      slow = fastdiv(lid, a.d_nfast);
+      fast = lid - slow * a.nfast;
+    }
+    tile_p = a.p_fast ? fast : slow;
+    tile_q = a.p_fast ? slow : fast;
+  }
+}
+
 // Epi: either  __device__ void operator()(int p, int q, const float (&v)[8], int split)  with v = D[p..p+7][q], p % 8 == 0,
 // or (with a static member kTileEpilogue)  __device__ void tile(acc, pw, qw, lr, lh, tile_id, split).
 template <class Cfg, class PreP, class PreQ, class Epi>
@@ -373,48 +425,8 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::OCC) void gemm_kernel(GemmArgs a, Pre
   const int wp = wave % Cfg::WP, wq = wave / Cfg::WP;
   const int lr = lane & 31, lh = lane >> 5;
 
-  // Workgroup -> (output tile, k-split). Consecutive workgroup ids sit on consecutive XCDs. With a multiple of 8 splits a
-  // split stays on ONE XCD: the k-range of both operands it contracts over is then fetched into that XCD's L2 once and
-  // shared by all its output tiles, instead of every XCD streaming most of both operands. Without splits, ids are
-  // re-dealt so that one XCD gets a contiguous run of tiles. (Everything up to the first operand load below is serial
-  // scalar work in front of every tile: the divisions are multiplications prepared by the host.)
-  auto xcd_run = [&](int pid) { return a.per ? (pid & 7) * a.per + (pid >> 3) : pid; };
-  int lid, split;
-  {
-    const int L = blockIdx.x;
-    if (a.splits == 1) {
-      split = 0;
-      lid = xcd_run(L);
-    } else if ((a.splits & 7) == 0) {
-      const int j = L >> 3;
-      lid = fastdiv(j, a.d_split8);
-      split = (L & 7) + 8 * (j - lid * (a.splits >> 3));
-    } else {
-      split = fastdiv(L, a.d_ntiles);
-      lid = xcd_run(L - split * a.ntiles);
-    }
-  }
-  // An XCD's run of tiles walks the smaller operand's tiles fastest: the run then shares few rows of the larger
-  // operand (which is thereby partitioned over the XCDs' L2s) and re-reads the smaller one. When the smaller operand
-  // does not fit the L2 beside the streaming larger one (a 3.5 MB weight against a 4 MB L2), the run is walked in
-  // blocks of `gblock` of its tiles: block 0 against all of the run's rows of the larger operand, then block 1, ...
-  // so the smaller operand is fetched once per XCD instead of once per row of tiles.
-  int tile_p, tile_q;
-  {
-    int fast, slow;
-    if (a.rows > 0) {
-      const int xcd = fastdiv(lid, a.d_per), idx = lid - xcd * a.per;
-      const int b = fastdiv(idx, a.d_blk), rem = idx - b * a.blk;
-      const int rg = fastdiv(rem, a.d_gblock);
-      fast = b * a.gblock + rem - rg * a.gblock;
-      slow = xcd * a.rows + rg;
-    } else {
-      slow = fastdiv(lid, a.d_nfast);
-      fast = lid - slow * a.nfast;
-    }
-    tile_p = a.p_fast ? fast : slow;
-    tile_q = a.p_fast ? slow : fast;
-  }
+  int lid, split, tile_p, tile_q;
+  gemm_tile_of(a, blockIdx.x, lid, split, tile_p, tile_q);
   const long p0 = (long)tile_p * BP, q0 = (long)tile_q * BQ;
   int kt0 = 0;
   if (a.splits > 1) {
@@ -608,9 +620,9 @@ static int gemm_launch(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes
   return gemm_launch_args<Cfg>(a, 1, splits, prep, preq, epi, stream);
 }
 
-// Launch with prepared arguments; groups_y > 1 only with a.k_seg.
-template <class Cfg, class PreP, class PreQ, class Epi>
-static int gemm_launch_args(GemmArgs a, int groups_y, int splits, PreP prep, PreQ preq, Epi epi, hipStream_t stream) {
+// The launch's tile map, with its divisions prepared; a.np, nq, nkt, ntp and the optional grouping fields are given.
+template <class Cfg>
+static int gemm_map_args(GemmArgs& a, int splits) {
   // the per-lane part of a load address is a 32-bit offset: 8 rows (K_CONTIG) or 8 k-rows (K_STRIDED) of the operand
   if (a.P.ld <= 0 || a.Q.ld <= 0 || a.P.ld > (1L << 28) || a.Q.ld > (1L << 28)) return TFB_ERR_SHAPE;
   if (((uintptr_t)a.P.base | (uintptr_t)a.Q.base | (uintptr_t)a.P.ld | (uintptr_t)a.Q.ld) & 15) return TFB_ERR_ARG;
@@ -619,12 +631,6 @@ static int gemm_launch_args(GemmArgs a, int groups_y, int splits, PreP prep, Pre
   const int ntq = a.nq / Cfg::BQ;
   if ((long)a.ntp * ntq * splits >= (1L << 31)) return TFB_ERR_SHAPE;
   a.ntiles = a.ntp * ntq;
-  // the stagger of the first round: only where there is a second round to overlap with and no k-split
-  a.slots = tfb_resident_slots(2);
-  if (!((splits == 1 || TFB_STAGGER_SPLITK) && (long)a.ntiles * splits >= 2L * a.slots)) a.slots = 0;
-  // a launch of few rounds has less to gain from the offset and pays the same for it (measured on the 1536-tile GEMMs of
-  // the step, three rounds: 0.730 / 0.755 ms per step with one / two units; on the 4608- and 6144-tile ones two is better)
-  a.sleeps = a.slots > 0 && (long)a.ntiles * splits <= TFB_STAGGER_SHORT_ROUNDS * (long)a.slots ? 1 : stagger_sleeps<Epi>::value;
   a.per = (a.ntiles & 7) == 0 ? a.ntiles >> 3 : 0;
   a.p_fast = a.np <= a.nq || a.q_group;
   a.nfast = a.p_fast ? a.ntp : ntq;
@@ -648,6 +654,20 @@ static int gemm_launch_args(GemmArgs a, int groups_y, int splits, PreP prep, Pre
   a.d_gblock = fastdiv_make(a.gblock);
   a.d_splits = fastdiv_make(splits);
   a.d_split8 = fastdiv_make(splits >> 3);
+  return TFB_OK;
+}
+
+// Launch with prepared arguments; groups_y > 1 only with a.k_seg.
+template <class Cfg, class PreP, class PreQ, class Epi>
+static int gemm_launch_args(GemmArgs a, int groups_y, int splits, PreP prep, PreQ preq, Epi epi, hipStream_t stream) {
+  const int st = gemm_map_args<Cfg>(a, splits);
+  if (st != TFB_OK) return st;
+  // the stagger of the first round: only where there is a second round to overlap with and no k-split
+  a.slots = tfb_resident_slots(2);
+  if (!((splits == 1 || TFB_STAGGER_SPLITK) && (long)a.ntiles * splits >= 2L * a.slots)) a.slots = 0;
+  // a launch of few rounds has less to gain from the offset and pays the same for it (measured on the 1536-tile GEMMs of
+  // the step, three rounds: 0.730 / 0.755 ms per step with one / two units; on the 4608- and 6144-tile ones two is better)
+  a.sleeps = a.slots > 0 && (long)a.ntiles * splits <= TFB_STAGGER_SHORT_ROUNDS * (long)a.slots ? 1 : stagger_sleeps<Epi>::value;
   dim3 grid(a.ntp * (a.nq / Cfg::BQ) * splits, groups_y, 1);
   hipLaunchKernelGGL((gemm_kernel<Cfg, PreP, PreQ, Epi>), grid, dim3(Cfg::NT), 0, stream, a, prep, preq, epi);
   TFB_LAUNCH_CHECK();
@@ -685,6 +705,7 @@ struct EpiStoreRes {
 
 // out (bf16 or fp32) [nq][ld] (+)= D
 struct EpiStore {
+  static constexpr bool kRanges = true;
   void* out;
   long ld;  // elements
   int f32;

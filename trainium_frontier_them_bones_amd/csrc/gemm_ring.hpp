@@ -1,0 +1,442 @@
+// Small-output MFMA GEMM for gfx950: D[p][q] = sum_k P[p][k] * Q[q][k], the arithmetic, operand layouts and epilogues of the
+// 128 x 128 core (gemm_core.hpp) for launches that do not fill the chip with large tiles.
+//
+// What bounds such a launch is latency: with fewer workgroups than CUs nothing hides a k-tile's trip from L2 or HBM into LDS,
+// and the core's two-stage loop pays that trip (about a microsecond) once per k-tile. Here the operand tiles go through a RING of
+// NS stages with NS - 1 k-tiles in flight, waited for one by one (s_waitcnt vmcnt(n)), and the tile is as small as it takes to
+// give every CU work (64 x 64, 128 x 64 or 128 x 128). The fragments of a k-tile are read in one go while the MFMAs of the k-tile
+// before run (two register sets), so a step costs one barrier and no exposed LDS latency.
+//
+// A contraction that the other kernels cut into k-splits (fp32 partials through memory, a reduction launch) is summed here in the
+// same ranges inside the workgroup - partial sums into one set of accumulators, folded into a second at a range's end - so that the
+// result is theirs bit for bit and does not depend on which kernel a batch size selects.
+//
+// Reads from LDS are inline assembly with explicit waits: left to the compiler, each would wait for every load in flight into LDS.
+#pragma once
+#include "gemm_core.hpp"
+
+#define TFB_MAX_RING 8
+
+// Epilogues of contractions that may be cut into k ranges declare  static constexpr bool kRanges
+template <class T, class = void>
+struct has_ranges : std::false_type {};
+template <class T>
+struct has_ranges<T, std::void_t<decltype(T::kRanges)>> : std::true_type {};
+
+template <int BP_, int BQ_, int WP_, int WQ_, int ES_, int LAYP_, int LAYQ_, int FMTP_, int FMTQ_, int NS_>
+struct RingCfg {
+  static constexpr int BP = BP_, BQ = BQ_, WP = WP_, WQ = WQ_, ES = ES_, NS = NS_;
+  static constexpr int LAYP = LAYP_, LAYQ = LAYQ_, FMTP = FMTP_, FMTQ = FMTQ_;
+  static constexpr int NW = WP * WQ, NT = NW * 64;
+  static constexpr int TP = BP / WP / 32, TQ = BQ / WQ / 32;
+  static constexpr int KS = ES == 2 ? 4 : 2;           // MFMA k-steps per k-tile of 128 bytes
+  static constexpr int STAGE_BYTES = (BP + BQ) * 128;
+  static constexpr int STAGE_LD = TP * 32 + 4;         // epilogue staging: a wavefront's slice is 32 rows of this many floats
+  static constexpr int EPI_BYTES = NW * 32 * STAGE_LD * 4;
+  static constexpr int LDS_BYTES = NS * STAGE_BYTES > EPI_BYTES ? NS * STAGE_BYTES : EPI_BYTES;
+  static_assert(NW == 4 && NS >= 3 && NS <= TFB_MAX_RING && LDS_BYTES <= 160 * 1024, "ring");
+};
+
+template <int OFF>
+__device__ __forceinline__ i32x4 ring_read128(uint32_t addr) {
+  i32x4 v;
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+  return v;
+}
+template <int OFF, int ES>
+__device__ __forceinline__ u32x2 ring_read_tr64(uint32_t addr) {
+  u32x2 v;
+  if (ES == 2) asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+  else asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+  return v;
+}
+
+// One operand's fragments of a k-tile: request() reads all of them into this object's registers, landed() ties those registers
+// to the wait that precedes it, get<i, s>() is the fragment of MFMA tile i, k-step s. The layouts are FragReader's.
+template <int ROWS, int NTILE, int ES, int LAY>
+struct RingFrags;
+
+template <int ROWS, int NTILE>
+struct RingAddr {   // per-lane byte offsets inside a stage's operand tile
+  uint32_t off[4];
+};
+
+template <int ROWS, int NTILE, int ES>
+struct RingFrags<ROWS, NTILE, ES, TFB_K_CONTIG> {
+  static constexpr int KS = ES == 2 ? 4 : 2, PER = ES == 2 ? 1 : 2;   // 128-bit reads per fragment
+  i32x4 v[NTILE][KS][PER];
+  static __device__ __forceinline__ RingAddr<ROWS, NTILE> addr(int wave_row0, int lane) {
+    const int row = wave_row0 + (lane & 31), lh = lane >> 5, f = tfb_kc_swz(row);
+    RingAddr<ROWS, NTILE> a;
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {   // n = k-step (bf16), or 2 k-step + half (fp8)
+      const int chunk = ES == 2 ? 2 * n + lh : 4 * (n >> 1) + 2 * lh + (n & 1);
+      a.off[n] = row * 128 + (((chunk ^ f) & 7) << 4);
+    }
+    return a;
+  }
+  __device__ __forceinline__ void request(const RingAddr<ROWS, NTILE>& a, uint32_t base) {
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      v[0][n / PER][n % PER] = ring_read128<0>(base + a.off[n]);
+      if constexpr (NTILE == 2) v[1][n / PER][n % PER] = ring_read128<4096>(base + a.off[n]);
+    }
+  }
+  __device__ __forceinline__ void landed() {
+#pragma unroll
+    for (int i = 0; i < NTILE; ++i)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) asm volatile("" : "+v"(v[i][n / PER][n % PER]));
+  }
+  template <int i, int s>
+  __device__ __forceinline__ auto get() const {
+    if constexpr (ES == 2) {
+      return __builtin_bit_cast(bf16x8, v[i][s][0]);
+    } else {
+      const i32x4 a = v[i][s][0], b = v[i][s][1];
+      return i32x8{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    }
+  }
+};
+
+template <int ROWS, int NTILE, int ES>
+struct RingFrags<ROWS, NTILE, ES, TFB_K_STRIDED> {
+  static constexpr int KS = ES == 2 ? 4 : 2, PER = ES == 2 ? 2 : 4;   // 64-bit transposing reads per fragment
+  static constexpr int PITCH = ROWS * ES, KSTEP = (ES == 2 ? 16 : 64) * PITCH, KQ = (ES == 2 ? 4 : 8) * PITCH;
+  u32x2 v[NTILE][KS][PER];
+  static __device__ __forceinline__ RingAddr<ROWS, NTILE> addr(int wave_row0, int lane) {
+    const int g4 = lane >> 4, j = lane & 15;
+    RingAddr<ROWS, NTILE> a;
+#pragma unroll
+    for (int i = 0; i < NTILE; ++i) {
+      if (ES == 2) {
+        const int p = wave_row0 + 32 * i + 16 * (g4 & 1) + 4 * (j & 3), k = 8 * (g4 >> 1) + (j >> 2);
+        a.off[i] = k * PITCH + ((((p >> 3) ^ tfb_ks_swz<ROWS, ES>(k)) << 4) | ((p & 4) << 1));
+      } else {
+        const int p = wave_row0 + 32 * i + 16 * (g4 & 1) + 8 * (j & 1), k = 32 * (g4 >> 1) + (j >> 1);
+        a.off[i] = k * PITCH + ((((p >> 4) ^ tfb_ks_swz<ROWS, ES>(k)) << 4) | (p & 8));
+      }
+    }
+    return a;
+  }
+  template <int i, int n>
+  __device__ __forceinline__ void req(const RingAddr<ROWS, NTILE>& a, uint32_t base) {
+    v[i][n / PER][n % PER] = ring_read_tr64<(n / PER) * KSTEP + (n % PER) * KQ, ES>(base + a.off[i]);
+    if constexpr (n + 1 < KS * PER) req<i, n + 1>(a, base);
+  }
+  __device__ __forceinline__ void request(const RingAddr<ROWS, NTILE>& a, uint32_t base) {
+    req<0, 0>(a, base);
+    if constexpr (NTILE == 2) req<1, 0>(a, base);
+  }
+  __device__ __forceinline__ void landed() {
+#pragma unroll
+    for (int i = 0; i < NTILE; ++i)
+#pragma unroll
+      for (int n = 0; n < KS * PER; ++n) asm volatile("" : "+v"(v[i][n / PER][n % PER]));
+  }
+  template <int i, int s>
+  __device__ __forceinline__ auto get() const {
+    if constexpr (ES == 2) {
+      const u32x4 w = {v[i][s][0].x, v[i][s][0].y, v[i][s][1].x, v[i][s][1].y};
+      return __builtin_bit_cast(bf16x8, w);
+    } else {
+      i32x8 w;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        w[2 * q] = (int)v[i][s][q].x;
+        w[2 * q + 1] = (int)v[i][s][q].y;
+      }
+      return w;
+    }
+  }
+};
+
+// The MFMAs that made x stay in front of this point (they have no side effects, and would otherwise sink across barriers).
+__device__ __forceinline__ void ring_pin(f32x16& x) { asm volatile("" : "+v"(x)); }
+
+// s_waitcnt vmcnt(tiles * PER): all but the newest `tiles` k-tiles of loads have landed (tiles is wavefront-uniform)
+template <int PER>
+__device__ __forceinline__ void ring_wait(int tiles) {
+#define TFB_RING_WAIT(n) case n: asm volatile("s_waitcnt vmcnt(%0)" ::"n"((n) * PER) : "memory"); break;
+  switch (tiles) {
+    TFB_RING_WAIT(1) TFB_RING_WAIT(2) TFB_RING_WAIT(3) TFB_RING_WAIT(4) TFB_RING_WAIT(5) TFB_RING_WAIT(6)
+    default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  }
+#undef TFB_RING_WAIT
+}
+
+template <class Cfg, bool RANGES, class Epi>
+__global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi epi_in) {
+  constexpr int BP = Cfg::BP, BQ = Cfg::BQ, NW = Cfg::NW, TP = Cfg::TP, TQ = Cfg::TQ, ES = Cfg::ES, NS = Cfg::NS;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[Cfg::LDS_BYTES];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wp = wave % Cfg::WP, wq = wave / Cfg::WP;
+  const int lr = lane & 31, lh = lane >> 5;
+  int lid, split, tile_p, tile_q;
+  gemm_tile_of(a, blockIdx.x, lid, split, tile_p, tile_q);
+  const long p0 = (long)tile_p * BP, q0 = (long)tile_q * BQ;
+  int kt0 = 0;
+  if (a.splits > 1) {
+    kt0 = fastdiv(split * a.nkt, a.d_splits);
+    a.nkt = fastdiv((split + 1) * a.nkt, a.d_splits) - kt0;
+  }
+  int group = 0;
+  if (a.q_group) {   // (named per 128 rows of q)
+    group = a.q_group[q0 >> 7];
+    if (group < 0) return;  // the whole workgroup leaves before any barrier
+    a.P.base += (long)group * a.p_group_stride;
+  }
+  if (a.k_seg) {
+    group = blockIdx.y;
+    const int k0 = a.k_seg[group], k1 = a.k_seg[group + 1];
+    kt0 = k0 * ES / 128;
+    a.nkt = (k1 - k0) * ES / 128;  // may be 0: the accumulators stay zero and are still written
+  }
+  const int nkt = a.nkt;
+
+  typedef TileDma<BP, NW, Cfg::LAYP, ES> DP;
+  typedef TileDma<BQ, NW, Cfg::LAYQ, ES> DQ;
+  constexpr int NI = DP::NI + DQ::NI;   // load instructions per wavefront and k-tile
+  static_assert((NS - 1) * NI < 63, "vmcnt counts to 63");
+  DP dp;
+  DQ dq;
+  dp.init(a.P, p0, (long)kt0 * 128, wave, lane);
+  dq.init(a.Q, q0, (long)kt0 * 128, wave, lane);
+  auto issue = [&](int stage, int t) {
+    dp.issue(lds + stage * Cfg::STAGE_BYTES, t, wave);
+    dq.issue(lds + stage * Cfg::STAGE_BYTES + BP * 128, t, wave);
+  };
+#pragma unroll
+  for (int t = 0; t < NS; ++t)
+    if (t < nkt) issue(t, t);
+
+  const Epi epi = epi_prepare(epi_for_group(epi_in, group));
+  typedef RingFrags<BP, TP, ES, Cfg::LAYP> FP;
+  typedef RingFrags<BQ, TQ, ES, Cfg::LAYQ> FQ;
+  const auto ap = FP::addr(wp * (TP * 32), lane);
+  const auto aq = FQ::addr(wq * (TQ * 32), lane);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(tfb_lds_void_t*)lds;
+  FP fp[2];
+  FQ fq[2];
+  auto request = [&](int set, int stage) {
+    const uint32_t b = lds0 + stage * Cfg::STAGE_BYTES;
+    fp[set].request(ap, b);
+    fq[set].request(aq, b + BP * 128);
+  };
+
+  f32x16 acc[TP][TQ];
+#pragma unroll
+  for (int i = 0; i < TP; ++i)
+#pragma unroll
+    for (int j = 0; j < TQ; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  // a.ranges k ranges [z nkt / Z, (z + 1) nkt / Z), as a k-split cuts them: total = range 0 + range 1 + ...
+  [[maybe_unused]] f32x16 total[RANGES ? TP : 1][RANGES ? TQ : 1];
+  [[maybe_unused]] int range = 1, range_end = RANGES ? fastdiv(nkt, a.d_ranges) : 0;
+  auto fold = [&]() {
+#pragma unroll
+    for (int i = 0; i < TP; ++i)
+#pragma unroll
+      for (int j = 0; j < TQ; ++j) {
+        total[i][j] = range == 1 ? acc[i][j] : total[i][j] + acc[i][j];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      }
+    ++range;
+    range_end = fastdiv(range * nkt, a.d_ranges);
+  };
+
+  // the staged epilogue's chunk of pass k: row and first column inside the wavefront's 32-row slice
+  constexpr bool kPrefetch = has_prefetch<Epi>::value && !has_tile_epilogue<Epi>::value;
+  constexpr int CPR = TP * 4, NK = 32 * CPR / 64;
+  auto chunk_row = [&](int k) { return 2 * (((lane >> 3) + k * 8) / (CPR / 4)) + ((lane >> 2) & 1); };
+  auto chunk_col = [&](int k) { return (4 * (((lane >> 3) + k * 8) % (CPR / 4)) + (lane & 3)) * 8; };
+  const int pw = wp * (TP * 32), qw = wq * (TQ * 32);  // wavefront's origin inside the tile
+  [[maybe_unused]] typename prefetch_type<Epi>::type pre[TQ][NK];
+
+  // k-step s of a set: every operand pair's MFMA
+  auto mfmas = [&](int set, auto s_) {
+    constexpr int s = decltype(s_)::value;
+    auto one = [&](auto i_, auto j_) {
+      constexpr int i = decltype(i_)::value, j = decltype(j_)::value;
+      acc[i][j] = mfma32<ES, Cfg::FMTP, Cfg::FMTQ>(fp[set].template get<i, s>(), fq[set].template get<j, s>(), acc[i][j]);
+    };
+    using N0 = std::integral_constant<int, 0>;
+    using N1 = std::integral_constant<int, 1>;
+    one(N0{}, N0{});
+    if constexpr (TQ == 2) one(N0{}, N1{});
+    if constexpr (TP == 2) one(N1{}, N0{});
+    if constexpr (TP == 2 && TQ == 2) one(N1{}, N1{});
+  };
+
+  int stage = 0;   // of the k-tile whose fragments were requested last
+  // k-tile t, whose fragments were requested into `set`: the next k-tile's are requested, its own multiplied. full_: there
+  // is a k-tile t + NS to load (the loop's body then has no branches)
+  auto step = [&](int set, int t, auto full_) {
+    constexpr bool full = decltype(full_)::value;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    fp[set].landed();
+    fq[set].landed();
+    if (full || t + 1 < nkt) {
+      const int left = nkt - 2 - t;
+      ring_wait<NI>(full || left > NS - 2 ? NS - 2 : left);
+      // behind this barrier every wavefront has k-tile t in registers (its stage is free) and its share of t + 1 in LDS
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("s_barrier" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (full || t + NS < nkt) issue(stage, t + NS);
+      stage = stage + 1 == NS ? 0 : stage + 1;
+      request(set ^ 1, stage);
+    }
+    if constexpr (RANGES)
+      if (t == range_end) fold();
+    mfmas(set, std::integral_constant<int, 0>{});
+    mfmas(set, std::integral_constant<int, 1>{});
+    if constexpr (Cfg::KS == 4) {
+      mfmas(set, std::integral_constant<int, 2>{});
+      mfmas(set, std::integral_constant<int, 3>{});
+    }
+#pragma unroll
+    for (int i = 0; i < TP; ++i)
+#pragma unroll
+      for (int j = 0; j < TQ; ++j) ring_pin(acc[i][j]);
+  };
+
+  if (nkt > 0) {
+    ring_wait<NI>(nkt - 1 < NS - 1 ? nkt - 1 : NS - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    request(0, 0);
+  }
+  if constexpr (kPrefetch) {   // the epilogue's own operands fly under the k-loop
+#pragma unroll
+    for (int j = 0; j < TQ; ++j)
+#pragma unroll
+      for (int k = 0; k < NK; ++k) pre[j][k] = epi.prefetch((int)p0 + pw + chunk_col(k), (int)q0 + qw + j * 32 + chunk_row(k));
+  }
+  int t = 0;
+  for (; t + 1 + NS < nkt; t += 2) {
+    step(0, t, std::true_type{});
+    step(1, t + 1, std::true_type{});
+  }
+  for (; t < nkt; t += 2) {
+    step(0, t, std::false_type{});
+    if (t + 1 < nkt) step(1, t + 1, std::false_type{});
+  }
+  if constexpr (RANGES) {
+#pragma unroll
+    for (int i = 0; i < TP; ++i)
+#pragma unroll
+      for (int j = 0; j < TQ; ++j) acc[i][j] = total[i][j] + acc[i][j];
+  }
+  __syncthreads();
+
+  if constexpr (has_tile_epilogue<Epi>::value) {
+    epi.tile(acc, (int)p0 + pw, (int)q0 + qw, lr, lh, lid, split);
+  } else {
+    // 32 output rows at a time through the wavefront's own LDS slice, then 8-element chunks, a row's on consecutive lanes
+    constexpr int SLD = Cfg::STAGE_LD;
+    float* stg = (float*)lds + wave * (32 * SLD);
+#pragma unroll
+    for (int j = 0; j < TQ; ++j) {
+#pragma unroll
+      for (int i = 0; i < TP; ++i)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+          const f32x4 v = {acc[i][j][jj * 4 + 0], acc[i][j][jj * 4 + 1], acc[i][j][jj * 4 + 2], acc[i][j][jj * 4 + 3]};
+          *(f32x4*)(stg + lr * SLD + i * 32 + jj * 8 + lh * 4) = v;
+        }
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int k = 0; k < NK; ++k) {
+        const int row = chunk_row(k), pc = chunk_col(k);
+        const int p = (int)p0 + pw + pc, q = (int)q0 + qw + j * 32 + row;
+        const f32x4 lo = *(const f32x4*)(stg + row * SLD + pc), hi = *(const f32x4*)(stg + row * SLD + pc + 4);
+        const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        if constexpr (has_partner32<Epi>::value) {
+          static_assert(TP == 2, "partner epilogue: 64 staged columns per wavefront");
+          const f32x4 plo = *(const f32x4*)(stg + row * SLD + (pc ^ 32)), phi = *(const f32x4*)(stg + row * SLD + (pc ^ 32) + 4);
+          const float vp[8] = {plo[0], plo[1], plo[2], plo[3], phi[0], phi[1], phi[2], phi[3]};
+          if constexpr (kPrefetch) epi(p, q, v, vp, pre[j][k], split);
+          else epi(p, q, v, vp, split);
+        } else if constexpr (kPrefetch) {
+          epi(p, q, v, pre[j][k], split);
+        } else {
+          epi(p, q, v, split);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+}
+
+// ranges > 1: the k ranges summed inside the workgroup (at most nkt of them; not with a k_seg)
+template <class Cfg, class Epi>
+static int gemm_ring_launch_args(GemmArgs a, int groups_y, int splits, int ranges, Epi epi, hipStream_t stream) {
+  const int st = gemm_map_args<Cfg>(a, splits);
+  if (st != TFB_OK) return st;
+  a.slots = 0;
+  a.sleeps = 0;
+  if (ranges > 1 && (splits > 1 || ranges > a.nkt)) return TFB_ERR_SHAPE;
+  a.ranges = ranges;
+  a.d_ranges = fastdiv_make(ranges);
+  const dim3 grid(a.ntiles * splits, groups_y, 1);
+  if constexpr (has_ranges<Epi>::value) {
+    if (ranges > 1) {
+      hipLaunchKernelGGL((gemm_ring_kernel<Cfg, true, Epi>), grid, dim3(Cfg::NT), 0, stream, a, epi);
+      TFB_LAUNCH_CHECK();
+      return TFB_OK;
+    }
+  }
+  if (ranges > 1) return TFB_ERR_ARG;
+  hipLaunchKernelGGL((gemm_ring_kernel<Cfg, false, Epi>), grid, dim3(Cfg::NT), 0, stream, a, epi);
+  TFB_LAUNCH_CHECK();
+  return TFB_OK;
+}
+
+// Which ring tile a launch of np x nq outputs (times `groups` equal ones) and nkt k-tiles takes: 1 = 64 x 64, 2 = 128 (p) x 64 (q),
+// 0 = none (the 128 x 128 core or the persistent kernel). A CU moves some 30 bytes per clock into LDS whatever the tile, so the
+// time is the bytes of the CU with the most tiles: 64 x 64 while every tile has a CU of its own, then 128 x 64 (3/4 of the bytes per
+// output) while no CU has more than two (k-strided operands, which cost the core more: two and a quarter); beyond, the core's two
+// workgroups per CU hide as much. Measured standalone, core -> ring (us): bf16 256 x 768 x 768 10.6 -> 4.9, 2048 x 768 x 768
+// 11.0 -> 6.7, 2048 x 768 x 2304 20.9 -> 13.3, 4096 x 768 x 768 11.4 -> 10.4, 2048 x 2304 x 768 14.5 -> 15.0 (576 tiles of
+// 128 x 64: beyond the line); fp8 1024 x 768 x 3072 18.7 -> 7.2, 2048 x 768 x 3072 18.8 -> 10.0, 4096 x 1024 x 4096 25.7 -> 20.4;
+// token contractions 2304 x 768 over 2048 24.2 -> 12.5, 768 x 768 over 1024 16.0 -> 6.2, fp8 3072 x 768 over 2048 14.7 -> 11.9.
+// From 96 k-tiles on the k-split forms of the other kernels are as good or better.
+static inline int gemm_ring_pick(long np, long nq, long nkt, bool strided, long groups = 1) {
+  if (nkt <= 0 || nkt > 96) return 0;
+  const long cus = tfb_resident_slots(1), t64 = (np / 64) * (nq / 64) * groups;
+  if (t64 <= cus) return 1;
+  return 2 * t64 <= (strided ? 9 : 8) * cus ? 2 : 0;
+}
+
+template <class Epi, int ES, int LAYP, int LAYQ, int FMTP, int FMTQ>
+static int gemm_ring_launch(int pick, GemmArgs a, int groups_y, int splits, Epi e, hipStream_t s, int ranges = 1) {
+  if constexpr (!has_partner32<Epi>::value && !has_tile_epilogue<Epi>::value) {   // (those take 64 columns of p per wavefront)
+    if (pick == 1) {
+      a.ntp = a.np / 64;
+      return gemm_ring_launch_args<RingCfg<64, 64, 2, 2, ES, LAYP, LAYQ, FMTP, FMTQ, 4>>(a, groups_y, splits, ranges, e, s);
+    }
+  }
+  a.ntp = a.np / 128;
+  return gemm_ring_launch_args<RingCfg<128, 64, 2, 2, ES, LAYP, LAYQ, FMTP, FMTQ, 3>>(a, groups_y, splits, ranges, e, s);
+}
+
+// A dense launch through the ring where gemm_ring_pick takes it: true, with its status in st.
+template <int ES, int LAYP, int LAYQ, int FMTP, int FMTQ, class Epi>
+static bool gemm_ring_try(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Epi e, hipStream_t s, int& st, int ranges = 1) {
+  const int pick = gemm_ring_pick(np, nq, kbytes / 128, LAYP == TFB_K_STRIDED && LAYQ == TFB_K_STRIDED);
+  if (!pick || np % 128 || nq % 128 || kbytes % 128) return false;
+  GemmArgs a = {};
+  a.P = P;
+  a.Q = Q;
+  a.np = np;
+  a.nq = nq;
+  a.nkt = (int)(kbytes / 128);
+  st = gemm_ring_launch<Epi, ES, LAYP, LAYQ, FMTP, FMTQ>(pick, a, 1, 1, e, s, ranges);
+  return true;
+}

@@ -261,11 +261,13 @@ __global__ __launch_bounds__(512, 2) void gemm_ws8_kernel(Ws8Args a, Epi epi_in)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-// np % 256 == 0, nq % 512 == 0 (64-token tiles dealt to the 8 XCDs), kbytes == 768, rows 16-byte aligned; at least one
-// step for every CU
+// np % 256 == 0, nq % 512 == 0 (64-token tiles dealt to the 8 XCDs), kbytes == 768, rows 16-byte aligned; at least eight
+// steps for every CU: a workgroup loads its weight panel and fills its pipeline once per run, and a shorter run does not pay for
+// that against the tiled kernels (up-projection / dH of a 768 x 3072 MLP, us, this kernel against them: 2048 tokens 14.5 / 18.0
+// against 10.6 / 13.9, 8192 tokens 32.4 / 42.6 against 29.5 / 40.0, 12288 tokens 41.6 / 52.9 against 43.9 / 57.2)
 static inline bool gemm_ws8_applies(long np, long nq, long kbytes) {
   return TFB_WS8 && kbytes == 768 && np > 0 && nq > 0 && np % 256 == 0 && nq % 512 == 0 &&
-         (np / 256) * (nq / 64) >= tfb_resident_slots(1);
+         (np / 256) * (nq / 64) >= 8L * tfb_resident_slots(1);
 }
 
 template <int FMTP, int FMTQ, class Epi>

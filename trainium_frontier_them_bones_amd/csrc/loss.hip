@@ -15,7 +15,7 @@
 // (in registers: a lane owns 32 of them, its partner lane the rest) into a [rows][V/64] table of
 // (max, sum) pairs; a finishing kernel merges a row's pairs, reads the target logit and writes lse and
 // the row loss. The logits make one trip to HBM (written once, read once by the backward).
-#include "gemm_core.hpp"
+#include "gemm_ring.hpp"
 
 namespace {
 
@@ -620,7 +620,9 @@ extern "C" int tfb_lmhead_fwd(const void* x, const void* W, const void* targets,
   using Cfg = GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>;
   GemmOperand P{(const uint8_t*)W, (long)d * 2}, Q{(const uint8_t*)x, (long)d * 2};
   EpiLmHead e{(bf16_t*)logits, (float*)part, (long)V, rows, V / 64, softcap};
-  int st = gemm_launch<Cfg>(P, Q, V, (int)rows, (long)d * 2, 1, LoadIdentity{}, LoadIdentity{}, e, s);
+  int st;
+  if (!gemm_ring_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, V, (int)rows, (long)d * 2, e, s, st))
+    st = gemm_launch<Cfg>(P, Q, V, (int)rows, (long)d * 2, 1, LoadIdentity{}, LoadIdentity{}, e, s);
   if (st != TFB_OK) return st;
   unsigned nb = (unsigned)((rows + 63) / 64);
   if (idx64)

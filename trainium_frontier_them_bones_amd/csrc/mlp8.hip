@@ -14,6 +14,7 @@
 //   x8 = e4m3(x * s_x); r = bf16(max(acc * dq_fc, 0)); rc = bf16(min(r * c_h, 15.375));
 //   h8 = e4m3(rc^2); y = bf16(acc * dq_proj); dy8 = e5m2(dy * s_dy);
 //   dpre = bf16((acc * dq_dh2) * r); dp8 = e5m2(dpre * s_dp); dx = bf16(acc * dq_dx).
+#include "gemm_ring.hpp"
 #include "gemm_ws8.hpp"
 
 // scale-row columns (nki_mlp_fused8.py:111-114)
@@ -815,6 +816,30 @@ extern "C" int tfb_precast8(const void* w, const void* scale_ptr, void* out8, vo
   return TFB_OK;
 }
 
+// out (+)= acc imm / (*s_g *s_a), rounded once (absent factors are 1): what splitk_reduce makes of one partial
+struct EpiDescaleStore {
+  static constexpr bool kRanges = true;
+  EpiStore base;
+  const float* s_g;
+  const float* s_a;
+  float imm;
+  float mul = 1.f;
+  __device__ __forceinline__ EpiDescaleStore prepare() const {
+    EpiDescaleStore e = *this;
+    float d = 1.0f;
+    if (s_g) d *= *s_g;
+    if (s_a) d *= *s_a;
+    e.mul = imm / d;
+    return e;
+  }
+  __device__ __forceinline__ void operator()(int p, int q, const float (&v)[8], int s) const {
+    float w[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = v[i] * mul;
+    base(p, q, w, s);
+  }
+};
+
 using Cfg8 = GemmCfg<128, 128, 2, 2, 1, TFB_K_CONTIG, TFB_K_CONTIG, TFB_FMT_E4M3, TFB_FMT_E4M3>;
 using Cfg8g = GemmCfg<128, 128, 2, 2, 1, TFB_K_CONTIG, TFB_K_CONTIG, TFB_FMT_E4M3, TFB_FMT_E5M2>;
 
@@ -824,6 +849,8 @@ template <class Cfg, class Epi>
 static int launch8(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Epi e, hipStream_t s) {
   // a contraction of 768 bytes (the fp8 attention projections of a 768-wide model): the weight-stationary kernel
   if (gemm_ws8_applies(np, nq, kbytes)) return gemm_ws8_launch<Cfg::FMTP, Cfg::FMTQ>(P, Q, np, nq, kbytes, e, s);
+  int st;
+  if (gemm_ring_try<1, TFB_K_CONTIG, TFB_K_CONTIG, Cfg::FMTP, Cfg::FMTQ>(P, Q, np, nq, kbytes, e, s, st)) return st;
   if (gemm_pp_applies(np, nq, kbytes)) return gemm_pp_launch<1, Cfg::FMTP, Cfg::FMTQ>(P, Q, np, nq, kbytes, e, s);
   return gemm_launch<Cfg>(P, Q, np, nq, kbytes, 1, LoadIdentity{}, LoadIdentity{}, e, s);
 }
@@ -834,6 +861,8 @@ static int launch8(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Ep
 template <class Cfg, class Epi>
 static int launch_k768(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Epi e, hipStream_t s) {
   if (gemm_ws8_applies(np, nq, kbytes)) return gemm_ws8_launch<Cfg::FMTP, Cfg::FMTQ>(P, Q, np, nq, kbytes, e, s);
+  int st;
+  if (gemm_ring_try<1, TFB_K_CONTIG, TFB_K_CONTIG, Cfg::FMTP, Cfg::FMTQ>(P, Q, np, nq, kbytes, e, s, st)) return st;
   return gemm_launch<Cfg>(P, Q, np, nq, kbytes, 1, LoadIdentity{}, LoadIdentity{}, e, s);
 }
 
@@ -895,11 +924,18 @@ extern "C" int tfb_gemm_fp8_tn(const void* g8, int fmt_g, const void* a8, int fm
       return splitk_reduce((const float*)workspace, out, n, sp, out_f32, accumulate, s, (const float*)s_g, (const float*)s_a, imm);
     }
   }
-  const int splits = choose_splits(n / (128 * 128), (int)(M / 128), n, workspace_bytes);
-  if ((long)splits * n * 4 > workspace_bytes) return TFB_ERR_SHAPE;
-  float* ws = (float*)workspace;
   // D[p = dd][q = o] = sum_m a8[m][dd] g8[m][o] -> out[o][dd]
   GemmOperand P{(const uint8_t*)a8, (long)D}, Q{(const uint8_t*)g8, (long)O};
+  const int splits = choose_splits(n / (128 * 128), (int)(M / 128), n, workspace_bytes);
+  {
+    EpiDescaleStore e{EpiStore{out, (long)D, out_f32, accumulate}, (const float*)s_g, (const float*)s_a, imm};
+    int st;
+    if (ga ? gemm_ring_try<1, TFB_K_STRIDED, TFB_K_STRIDED, TFB_FMT_E4M3, TFB_FMT_E5M2>(P, Q, D, O, M, e, s, st, splits)
+           : gemm_ring_try<1, TFB_K_STRIDED, TFB_K_STRIDED, TFB_FMT_E5M2, TFB_FMT_E4M3>(P, Q, D, O, M, e, s, st, splits))
+      return st;
+  }
+  if ((long)splits * n * 4 > workspace_bytes) return TFB_ERR_SHAPE;
+  float* ws = (float*)workspace;
   EpiSplit e{ws, (long)D, n};
   int st = ga ? gemm_launch<GemmCfg<128, 128, 2, 2, 1, TFB_K_STRIDED, TFB_K_STRIDED, TFB_FMT_E4M3, TFB_FMT_E5M2>>(
                     P, Q, D, O, M, splits, LoadIdentity{}, LoadIdentity{}, e, s)
@@ -1032,6 +1068,8 @@ int grouped_launch(const uint8_t* wbase, long wld, long wgroup_stride, const uin
   a.q_group = tile_expert;
   a.p_group_stride = wgroup_stride;
   a.k_seg = nullptr;
+  if (const int pick = gemm_ring_pick(np, rmax, a.nkt, false))
+    return gemm_ring_launch<Epi, Cfg::ES, Cfg::LAYP, Cfg::LAYQ, Cfg::FMTP, Cfg::FMTQ>(pick, a, 1, 1, e, s);
   return gemm_launch_args<Cfg>(a, 1, 1, LoadIdentity{}, LoadIdentity{}, e, s);
 }
 }  // namespace
@@ -1294,6 +1332,19 @@ struct EpiDpre1 {  // dpre = bf16((acc 2) r); optionally h = bf16(r r)
 };
 }  // namespace
 
+namespace {
+// A dense bf16 GEMM with Cfg's operand layouts: the ring kernel for few tiles, the persistent kernel for a plain store over a long
+// contraction, else the 128 x 128 core.
+template <class Cfg, class Epi>
+int launch16(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Epi e, hipStream_t s) {
+  int st;
+  if (gemm_ring_try<2, Cfg::LAYP, Cfg::LAYQ, 0, 0>(P, Q, np, nq, kbytes, e, s, st)) return st;
+  if constexpr (std::is_same<Epi, EpiStore>::value)
+    if (gemm_pp_applies(np, nq, kbytes)) return gemm_pp_launch_lay<2, 0, 0, Cfg::LAYP, Cfg::LAYQ>(P, Q, np, nq, kbytes, 1, e, s);
+  return gemm_launch<Cfg>(P, Q, np, nq, kbytes, 1, LoadIdentity{}, LoadIdentity{}, e, s);
+}
+}  // namespace
+
 // x bf16 [M][d], w_fc bf16 [F][d], w_proj bf16 [d][F] -> y bf16 [M][d], r bf16 [M][F] (saved for the backward), h bf16
 // [M][F] (the second GEMM's operand; scratch for the caller). M, d, F multiples of 128.
 extern "C" int tfb_mlp_fwd(const void* x, const void* w_fc, const void* w_proj, void* y, void* r, void* h, long M, int d, int F,
@@ -1303,11 +1354,11 @@ extern "C" int tfb_mlp_fwd(const void* x, const void* w_fc, const void* w_proj, 
   hipStream_t s = (hipStream_t)stream;
   GemmOperand Pw{(const uint8_t*)w_fc, d * 2L}, Qx{(const uint8_t*)x, d * 2L};
   EpiRelu2 e1{(bf16_t*)r, (bf16_t*)h, (long)F};
-  int st = gemm_launch<CfgNT>(Pw, Qx, F, (int)M, d * 2L, 1, LoadIdentity{}, LoadIdentity{}, e1, s);
+  int st = launch16<CfgNT>(Pw, Qx, F, (int)M, d * 2L, e1, s);
   if (st != TFB_OK) return st;
   GemmOperand Pp{(const uint8_t*)w_proj, F * 2L}, Qh{(const uint8_t*)h, F * 2L};
   EpiStore e2{y, (long)d, 0, 0};
-  return gemm_launch<CfgNT>(Pp, Qh, d, (int)M, F * 2L, 1, LoadIdentity{}, LoadIdentity{}, e2, s);
+  return launch16<CfgNT>(Pp, Qh, d, (int)M, F * 2L, e2, s);
 }
 
 // dy bf16 [M][d], r as the forward left it -> dx bf16 [M][d], dpre bf16 [M][F], h bf16 [M][F] (optional, may be NULL):
@@ -1320,10 +1371,10 @@ extern "C" int tfb_mlp_bwd(const void* dy, const void* r, const void* w_fc, cons
   // dh[m][f] = sum_j dy[m][j] w_proj[j][f]: the weight is the k-strided operand (k = j, contiguous in f)
   GemmOperand Pp{(const uint8_t*)w_proj, F * 2L}, Qg{(const uint8_t*)dy, d * 2L};
   EpiDpre1 e1{(const bf16_t*)r, (bf16_t*)dpre, (bf16_t*)h, (long)F};
-  int st = gemm_launch<CfgNN>(Pp, Qg, F, (int)M, d * 2L, 1, LoadIdentity{}, LoadIdentity{}, e1, s);
+  int st = launch16<CfgNN>(Pp, Qg, F, (int)M, d * 2L, e1, s);
   if (st != TFB_OK) return st;
   // dx[m][j] = sum_f dpre[m][f] w_fc[f][j]
   GemmOperand Pf{(const uint8_t*)w_fc, d * 2L}, Qd{(const uint8_t*)dpre, F * 2L};
   EpiStore e2{dx, (long)d, 0, 0};
-  return gemm_launch<CfgNN>(Pf, Qd, d, (int)M, F * 2L, 1, LoadIdentity{}, LoadIdentity{}, e2, s);
+  return launch16<CfgNN>(Pf, Qd, d, (int)M, F * 2L, e2, s);
 }

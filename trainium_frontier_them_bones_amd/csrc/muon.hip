@@ -14,7 +14,7 @@
 // operand pick it by the row tile's matrix (q_group). G and G G are symmetric bit for bit (the same products summed in
 // the same order on either side of the diagonal), so B^T = B and both products run in the k-contiguous "x @ w^T" form
 // with the [N][N] matrix as the weight; the reference's mirror fill of the lower blocks is therefore not needed.
-#include "gemm_core.hpp"
+#include "gemm_ring.hpp"
 
 namespace {
 
@@ -101,6 +101,14 @@ __global__ __launch_bounds__(256) void ns_transpose_out_kernel(const bf16_t* __r
   for (int j = 0; j < 32; j += 8) y[mat + (long)(n0 + ty + j) * M + m0 + tx] = t[tx][ty + j];
 }
 
+// A grouped launch of `nkt` k-tiles a matrix: the ring kernel for a small stack, else the 128 x 128 core.
+template <class Cfg, class Epi>
+int launch(const GemmArgs& a, int groups_y, int nkt, Epi e, hipStream_t s) {
+  if (const int pick = gemm_ring_pick(a.np, a.nq, nkt, Cfg::LAYP == TFB_K_STRIDED, groups_y))
+    return gemm_ring_launch<Epi, 2, Cfg::LAYP, Cfg::LAYQ, 0, 0>(pick, a, groups_y, 1, e, s);
+  return gemm_launch_args<Cfg>(a, groups_y, 1, LoadIdentity{}, LoadIdentity{}, e, s);
+}
+
 inline long align256(long b) { return (b + 255) & ~255L; }
 
 }  // namespace
@@ -162,7 +170,7 @@ extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, vo
     ga.p_group_stride = 0;
     ga.k_seg = k_seg;
     EpiStoreGrouped eg{EpiStore{G, (long)N, 0, 0}, (long)N * N};
-    int st = gemm_launch_args<CfgT>(ga, K, 1, LoadIdentity{}, LoadIdentity{}, eg, s);
+    int st = launch<CfgT>(ga, K, M / 64, eg, s);
     if (st != TFB_OK) return st;
     // B = c G G + b G on the stacked G: rows of G[k] against G[k] as the weight (G G^T = G G)
     GemmArgs gb2;
@@ -176,7 +184,7 @@ extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, vo
     gb2.p_group_stride = (long)N * N * 2;
     gb2.k_seg = nullptr;
     EpiAxpby eb{Bm, G, (long)N, c, b};
-    st = gemm_launch_args<CfgN>(gb2, 1, 1, LoadIdentity{}, LoadIdentity{}, eb, s);
+    st = launch<CfgN>(gb2, 1, gb2.nkt, eb, s);
     if (st != TFB_OK) return st;
     // X' = X B + a X on the stacked X: rows of X[k] against B[k] as the weight (X B^T = X B)
     GemmArgs gx;
@@ -190,7 +198,7 @@ extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, vo
     gx.p_group_stride = (long)N * N * 2;
     gx.k_seg = nullptr;
     EpiAxpby ex{xout, xin, (long)N, 1.0f, a};
-    st = gemm_launch_args<CfgN>(gx, 1, 1, LoadIdentity{}, LoadIdentity{}, ex, s);
+    st = launch<CfgN>(gx, 1, gx.nkt, ex, s);
     if (st != TFB_OK) return st;
     cur ^= 1;
   }
