@@ -665,6 +665,21 @@ def test_small_output_gemms_in_every_operand_layout(ops, dev, M, N, K):
         assert torch.equal(big[:M], outs[0])
 
 
+@pytest.mark.parametrize("M,N,K", [(8320, 4096, 256), (4224, 16384, 128), (9600, 2048, 1024)])
+def test_gemms_whose_rows_end_in_half_a_tile(ops, dev, M, N, K):
+    """From a round of 256 x 256 tiles on, 128 rows beyond the last whole tile go through the ring kernel (64 x 64 tiles, or
+    128 x 64 past N = 8192): the plain and the residual store equal those of the two parts on their own, bit for bit."""
+    g = _g(M + N + K)
+    x = torch.randn(M, K, generator=g).bfloat16().to(dev)
+    w = (K ** -0.5 * torch.randn(N, K, generator=g)).bfloat16().to(dev)
+    res = torch.randn(M, N, generator=g).bfloat16().to(dev)
+    y, z = ops.matmul(x, w, trans_b=True), ops.matmul_res(x, w, res, trans_b=True)
+    c = M - 128
+    assert torch.equal(y, torch.cat([ops.matmul(x[:c], w, trans_b=True), ops.matmul(x[c:].contiguous(), w, trans_b=True)]))
+    assert torch.equal(z[c:], ops.matmul_res(x[c:].contiguous(), w, res[c:].contiguous(), trans_b=True))
+    assert rel_l2(y, x.float() @ w.float().t()) < 3e-3 and rel_l2(z, res.float() + x.float() @ w.float().t()) < 4e-3
+
+
 @pytest.mark.parametrize("M,d,F", [(128, 256, 256), (256, 256, 1024), (384, 768, 3072), (1920, 1024, 2048), (2432, 768, 3072)])
 def test_small_fp8_mlps_equal_the_rows_of_a_large_one(ops, dev, M, d, F):
     """The fp8 MLP of a small batch (ring kernel in all six GEMMs) against the same rows of a batch that takes the large kernels,

@@ -68,8 +68,8 @@ int run(GemmOperand P, GemmOperand Q, int N, int M, int K, void* C, int out_f32,
     EpiStore e{C, (long)N, out_f32, accumulate, alpha};
     // large outputs: the persistent 256 x 256 kernel (same sums in the same order), in any operand layout (the input
     // gradient of the QKV projection, whose weight is read k-strided: 123.6 -> 117.7 us inside the step)
-    if (!out_f32 && !accumulate && gemm_pp_applies(N, M, (long)K * 2))
-      return gemm_pp_launch_lay<2, 0, 0, LAYP, LAYQ>(P, Q, N, M, (long)K * 2, 1, e, stream);
+    int st;
+    if (!out_f32 && !accumulate && gemm_pp_try<2, LAYP, LAYQ, 0, 0>(P, Q, N, M, (long)K * 2, false, e, stream, st)) return st;
     return gemm_launch<Cfg>(P, Q, N, M, (long)K * 2, 1, LoadIdentity{}, LoadIdentity{}, e, stream);
   }
   EpiSplit e{ws, (long)N, (long)M * N};
@@ -179,7 +179,7 @@ extern "C" int tfb_gemm_bf16_res(const void* A, const void* B, const void* res, 
   if (trans_b ? gemm_ring_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream, st)
               : gemm_ring_try<2, TFB_K_STRIDED, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream, st))
     return st;
-  if (trans_b && gemm_pp_applies(N, M, (long)K * 2)) return gemm_pp_launch<2, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream);
+  if (trans_b && gemm_pp_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, true, e, (hipStream_t)stream, st)) return st;
   if (trans_b)
     return gemm_launch<GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>>(P, Q, N, M, (long)K * 2, 1, LoadIdentity{},
                                                                                LoadIdentity{}, e, (hipStream_t)stream);
@@ -200,6 +200,6 @@ extern "C" int tfb_qkv_rope_fwd(const void* x, const void* w, const void* cos_t,
   EpiStoreRope e{(bf16_t*)out, (long)N, (const bf16_t*)cos_t, (const bf16_t*)sin_t, T, rot_cols};
   int st;
   if (gemm_ring_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream, st)) return st;
-  if (gemm_pp_applies(N, M, (long)K * 2)) return gemm_pp_launch<2, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream);
+  if (gemm_pp_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, true, e, (hipStream_t)stream, st)) return st;
   return gemm_launch<Cfg>(P, Q, N, M, (long)K * 2, 1, LoadIdentity{}, LoadIdentity{}, e, (hipStream_t)stream);
 }

@@ -80,6 +80,7 @@ struct GemmArgs {
   int rows;     // block traversal: rows of tiles of the other operand in one XCD's run (0: plain traversal)
   int blk;      // gblock * rows
   FastDiv d_ntiles, d_per, d_nfast, d_blk, d_gblock, d_splits, d_split8;  // d_split8: by splits / 8
+  int q_off;    // ring kernel: what the epilogue adds to its row numbers (a launch over the last rows of a larger one)
   int ranges;   // ring kernel: k ranges summed separately inside one workgroup, then added in order (see there)
   FastDiv d_ranges;
 };

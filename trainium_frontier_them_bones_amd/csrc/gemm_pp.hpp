@@ -605,19 +605,25 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stream's last (unused) loads must have landed before LDS is released
 }
 
-// Shapes this kernel takes (both operands k-contiguous): np, nq multiples of 256, at least two k-tiles of 128 bytes.
-// Shapes it is USED for: contractions of at least 16 k-tiles, or outputs of at least 4096 tiles. Measured inside the training
-// step against the 128 x 128 kernel (two workgroups per CU, one's epilogue under the other's k-loop): the 32768 x 32768 x 768
-// LM-head product 1728 -> 1532 us, the fp8 GEMMs with 24 k-tiles 82.5 -> 74.7 and 84.8 -> 83.2 us; but with 6 to 12 k-tiles and
-// a heavy epilogue per tile (rotary embedding, residual add, the MLP's activation) 141 -> 148, 55 -> 60, 112 -> 111 us: those stay.
+// Shapes this kernel takes: np, nq multiples of 256, at least two k-tiles of 128 bytes.
+// Shapes it is USED for: its tiles have to fill their rounds of the CUs, to 60 % where there is one round and to 70 % otherwise,
+// because a CU works on one tile at a time; then the half operand traffic per output wins against the 128 x 128 kernel at every
+// contraction length (standalone, us, that kernel -> this one): bf16 2048 x 32768 x 768 (4.0 rounds) 140 -> 105, 8192 x 4096 x 768
+// (2.0) 69 -> 51, 10240 x 1024 x 768 (0.62) 27.8 -> 23.8, 16384 x 768 x 2304 (0.75) 78 -> 58; fp8 16384 x 3072 x 1024 (3.0) 69 -> 50;
+// at the line 8192 x 3072 x 768 (1.5) 46.4 -> 47.2, and below it 8192 x 2304 x 768 (1.12) 37.6 -> 41.8, 8192 x 1024 x 768 (0.5)
+// 18.5 -> 23.7. A heavy epilogue per tile (rotary embedding, residual add, the MLP's activation) is serial with the k-loop here and runs
+// under another workgroup's MFMAs there: those need 16 k-tiles or 4096 tiles as well (in the training step, 6 to 12 k-tiles:
+// 141 -> 148, 55 -> 60, 112 -> 111 us).
 #ifndef TFB_PP
 #define TFB_PP 1  // 0: every GEMM on the 128 x 128 kernel; 2: every shape the kernel takes (for comparisons)
 #endif
-static inline bool gemm_pp_applies(long np, long nq, long kbytes) {
+static inline bool gemm_pp_applies(long np, long nq, long kbytes, bool heavy_epilogue = false) {
   if (!TFB_PP || np <= 0 || nq <= 0 || np % 256 || nq % 256 || kbytes < 256 || kbytes % 128) return false;
-  const long tiles = (np / 256) * (nq / 256);
+  const long tiles = (np / 256) * (nq / 256), cus = tfb_resident_slots(1), rounds = (tiles + cus - 1) / cus;
   if (tiles < 8) return false;
-  return TFB_PP == 2 || kbytes / 128 >= 16 || tiles >= 4096;
+  if (TFB_PP == 2) return true;
+  if (10 * tiles < (rounds == 1 ? 6 : 7) * rounds * cus) return false;
+  return !heavy_epilogue || kbytes / 128 >= 16 || tiles >= 4096;
 }
 
 // np, nq multiples of 256; kbytes = the contraction in bytes of a k-contiguous row (elements * ES), a multiple of 128
@@ -681,11 +687,4 @@ static inline int gemm_pp_fewtile_splits(long t256, long nkt, long out_elems, lo
   int c = t256 * 8 <= cus ? 8 * (int)(cus / 8 / t256) : (int)(cus / t256);
   while (c > 1 && (nkt / c < 16 || (long)c * out_elems * 4 > ws_bytes)) --c;
   return (c > 1 && (double)(t256 * c) >= 0.8 * (double)cus) ? c : 0;
-}
-
-// both operands k-contiguous, no k-split
-template <int ES, int FMTP, int FMTQ, class Epi>
-static int gemm_pp_launch(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Epi epi, hipStream_t stream) {
-  if (kbytes < 256) return TFB_ERR_SHAPE;
-  return gemm_pp_launch_lay<ES, FMTP, FMTQ, TFB_K_CONTIG, TFB_K_CONTIG>(P, Q, np, nq, kbytes, 1, epi, stream);
 }

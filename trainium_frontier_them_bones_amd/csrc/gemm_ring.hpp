@@ -13,7 +13,7 @@
 //
 // Reads from LDS are inline assembly with explicit waits: left to the compiler, each would wait for every load in flight into LDS.
 #pragma once
-#include "gemm_core.hpp"
+#include "gemm_pp.hpp"
 
 #define TFB_MAX_RING 8
 
@@ -316,7 +316,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
 #pragma unroll
     for (int j = 0; j < TQ; ++j)
 #pragma unroll
-      for (int k = 0; k < NK; ++k) pre[j][k] = epi.prefetch((int)p0 + pw + chunk_col(k), (int)q0 + qw + j * 32 + chunk_row(k));
+      for (int k = 0; k < NK; ++k) pre[j][k] = epi.prefetch((int)p0 + pw + chunk_col(k), a.q_off + (int)q0 + qw + j * 32 + chunk_row(k));
   }
   int t = 0;
   for (; t + 1 + NS < nkt; t += 2) {
@@ -336,7 +336,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
   __syncthreads();
 
   if constexpr (has_tile_epilogue<Epi>::value) {
-    epi.tile(acc, (int)p0 + pw, (int)q0 + qw, lr, lh, lid, split);
+    epi.tile(acc, (int)p0 + pw, a.q_off + (int)q0 + qw, lr, lh, lid, split);
   } else {
     // 32 output rows at a time through the wavefront's own LDS slice, then 8-element chunks, a row's on consecutive lanes
     constexpr int SLD = Cfg::STAGE_LD;
@@ -354,7 +354,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
 #pragma unroll
       for (int k = 0; k < NK; ++k) {
         const int row = chunk_row(k), pc = chunk_col(k);
-        const int p = (int)p0 + pw + pc, q = (int)q0 + qw + j * 32 + row;
+        const int p = (int)p0 + pw + pc, q = a.q_off + (int)q0 + qw + j * 32 + row;
         const f32x4 lo = *(const f32x4*)(stg + row * SLD + pc), hi = *(const f32x4*)(stg + row * SLD + pc + 4);
         const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         if constexpr (has_partner32<Epi>::value) {
@@ -415,7 +415,8 @@ static inline int gemm_ring_pick(long np, long nq, long nkt, bool strided, long 
 }
 
 template <class Epi, int ES, int LAYP, int LAYQ, int FMTP, int FMTQ>
-static int gemm_ring_launch(int pick, GemmArgs a, int groups_y, int splits, Epi e, hipStream_t s, int ranges = 1) {
+static int gemm_ring_launch(int pick, GemmArgs a, int groups_y, int splits, Epi e, hipStream_t s, int ranges = 1, int q_off = 0) {
+  a.q_off = q_off;
   if constexpr (!has_partner32<Epi>::value && !has_tile_epilogue<Epi>::value) {   // (those take 64 columns of p per wavefront)
     if (pick == 1) {
       a.ntp = a.np / 64;
@@ -438,5 +439,24 @@ static bool gemm_ring_try(GemmOperand P, GemmOperand Q, int np, int nq, long kby
   a.nq = nq;
   a.nkt = (int)(kbytes / 128);
   st = gemm_ring_launch<Epi, ES, LAYP, LAYQ, FMTP, FMTQ>(pick, a, 1, 1, e, s, ranges);
+  return true;
+}
+
+// A dense launch through the persistent kernel where gemm_pp_applies takes it, or takes all but the last 128 rows of q (which then go
+// through the ring: 9600 x 3072 x 1024 in bf16 79 -> 62 us): true, with its status in st. heavy: the epilogue is heavy there.
+template <int ES, int LAYP, int LAYQ, int FMTP, int FMTQ, class Epi>
+static bool gemm_pp_try(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, bool heavy, Epi e, hipStream_t s, int& st) {
+  const int rest = nq % 256, main = nq - rest;
+  if (!gemm_pp_applies(np, main, kbytes, heavy)) return false;
+  if (rest && (rest != 128 || (long)(np / 256) * (main / 256) < tfb_resident_slots(1))) return false;
+  st = gemm_pp_launch_lay<ES, FMTP, FMTQ, LAYP, LAYQ>(P, Q, np, main, kbytes, 1, e, s);
+  if (st != TFB_OK || !rest) return true;
+  GemmArgs a = {};
+  a.P = P;
+  a.Q = GemmOperand{Q.base + (LAYQ == TFB_K_CONTIG ? main * Q.ld : (long)main * ES), Q.ld};
+  a.np = np;
+  a.nq = rest;
+  a.nkt = (int)(kbytes / 128);
+  st = gemm_ring_launch<Epi, ES, LAYP, LAYQ, FMTP, FMTQ>(128L * np <= 4096L * tfb_resident_slots(1) ? 1 : 2, a, 1, 1, e, s, 1, main);
   return true;
 }

@@ -851,7 +851,7 @@ static int launch8(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Ep
   if (gemm_ws8_applies(np, nq, kbytes)) return gemm_ws8_launch<Cfg::FMTP, Cfg::FMTQ>(P, Q, np, nq, kbytes, e, s);
   int st;
   if (gemm_ring_try<1, TFB_K_CONTIG, TFB_K_CONTIG, Cfg::FMTP, Cfg::FMTQ>(P, Q, np, nq, kbytes, e, s, st)) return st;
-  if (gemm_pp_applies(np, nq, kbytes)) return gemm_pp_launch<1, Cfg::FMTP, Cfg::FMTQ>(P, Q, np, nq, kbytes, e, s);
+  if (gemm_pp_try<1, TFB_K_CONTIG, TFB_K_CONTIG, Cfg::FMTP, Cfg::FMTQ>(P, Q, np, nq, kbytes, has_prefetch<Epi>::value, e, s, st)) return st;
   return gemm_launch<Cfg>(P, Q, np, nq, kbytes, 1, LoadIdentity{}, LoadIdentity{}, e, s);
 }
 
@@ -1340,7 +1340,7 @@ int launch16(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Epi e, h
   int st;
   if (gemm_ring_try<2, Cfg::LAYP, Cfg::LAYQ, 0, 0>(P, Q, np, nq, kbytes, e, s, st)) return st;
   if constexpr (std::is_same<Epi, EpiStore>::value)
-    if (gemm_pp_applies(np, nq, kbytes)) return gemm_pp_launch_lay<2, 0, 0, Cfg::LAYP, Cfg::LAYQ>(P, Q, np, nq, kbytes, 1, e, s);
+    if (gemm_pp_try<2, Cfg::LAYP, Cfg::LAYQ, 0, 0>(P, Q, np, nq, kbytes, false, e, s, st)) return st;
   return gemm_launch<Cfg>(P, Q, np, nq, kbytes, 1, LoadIdentity{}, LoadIdentity{}, e, s);
 }
 }  // namespace
