@@ -14,7 +14,7 @@
 // stores it, and reduces exp(s - shift) over the 64 vocabulary columns a wavefront holds for each row
 // (in registers: a lane owns 32 of them, its partner lane the rest) into a [rows][V/64] table of
 // (max, sum) pairs; a finishing kernel merges a row's pairs, reads the target logit and writes lse and
-// the row loss. The logits make one trip to HBM (written once, read once by the backward).
+// the row loss. Launches large enough for the persistent 256 x 256 kernel take that instead, and a pass over the logits it wrote.
 #include "gemm_ring.hpp"
 
 namespace {
@@ -404,6 +404,13 @@ __global__ __launch_bounds__(256) void loss_multi_bwd_kernel(const bf16_t* __res
 }
 
 // ------------------------------------------------------------------------------------ LM head GEMM + lse partials
+// exp(cap tanh(x / cap) - cap) = exp(-2 cap / (exp(2 x / cap) + 1)): two exponentials and a reciprocal, half the instructions
+// of the tanh, its division and the exponential after it.
+__device__ __forceinline__ float capped_exp(float x, float icap, float cap) {
+  const float e = __builtin_amdgcn_exp2f(x * (2.8853900817779268f * icap));
+  return __builtin_amdgcn_exp2f(-2.8853900817779268f * cap * __builtin_amdgcn_rcpf(e + 1.0f));
+}
+
 struct EpiLmHead {
   static constexpr bool kTileEpilogue = true;
   bf16_t* logits;  // [rows][V]
@@ -438,7 +445,7 @@ struct EpiLmHead {
         a.m = cap;
         a.s = 0.f;
 #pragma unroll
-        for (int k = 0; k < TP * 16; ++k) a.s += fexp(cap * tanh_fast(v[k] * icap) - cap);
+        for (int k = 0; k < TP * 16; ++k) a.s += capped_exp(v[k], icap, cap);
         a.s += __shfl_xor(a.s, 32, 64);
       } else {
         float mx = v[0];
@@ -456,6 +463,64 @@ struct EpiLmHead {
     }
   }
 };
+
+// lse and loss of one row of the logits per workgroup, for the launches whose GEMM leaves them to a pass of their own: four
+// 16-byte loads a lane in flight, one running maximum for the 32 values they bring (none with a softcap, where cap bounds them).
+template <typename IDX>
+__global__ __launch_bounds__(256) void lmhead_rows_kernel(const bf16_t* __restrict__ x, const IDX* __restrict__ tg,
+                                                         const float* __restrict__ row_w, float* __restrict__ loss,
+                                                         float* __restrict__ lse, int V, float cap) {
+  __shared__ float rm[4], rs[4];
+  const long row = blockIdx.x;
+  const bf16_t* xr = x + row * V;
+  const float icap = cap > 0.f ? 1.0f / cap : 0.f;
+  MS a{cap > 0.f ? cap : -1e30f, 0.f};
+  for (int i0 = threadIdx.x * 8; i0 < V; i0 += 4 * 2048) {
+    u32x4 u[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      u[c] = i0 + 2048 * c < V ? *(const u32x4*)(xr + i0 + 2048 * c) : u32x4{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+    if (cap > 0.f) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (i0 + 2048 * c < V) {
+#pragma unroll
+          for (int k = 0; k < 4; ++k) a.s += capped_exp(bflo(u[c][k]), icap, cap) + capped_exp(bfhi(u[c][k]), icap, cap);
+        }
+    } else {
+      float mx = a.m, t = 0.f;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) mx = fmaxf(fmaxf(mx, bflo(u[c][k])), bfhi(u[c][k]));
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t += fexp(bflo(u[c][k]) - mx) + fexp(bfhi(u[c][k]) - mx);
+      a.s = a.s * fexp(a.m - mx) + t;
+      a.m = mx;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) a = ms_merge(a, MS{__shfl_xor(a.m, o, 64), __shfl_xor(a.s, o, 64)});
+  if ((threadIdx.x & 63) == 0) {
+    rm[threadIdx.x >> 6] = a.m;
+    rs[threadIdx.x >> 6] = a.s;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < 4; ++i) a = ms_merge(a, MS{rm[i], rs[i]});
+    const float l = a.m + logf(a.s);
+    lse[row] = l;
+    const long tt = (long)tg[row];
+    float out = 0.f;
+    if ((unsigned long)tt < (unsigned long)V) {  // a target outside [0, V) is an ignored row, never an address
+      const float xt = bf2f(xr[tt]);
+      out = (l - (cap > 0.f ? cap * tanh_fast(xt * icap) : xt)) * (row_w ? row_w[row] : 1.0f);
+    }
+    loss[row] = out;
+  }
+}
 
 // A workgroup per 64 rows, a lane per row: each wavefront merges a quarter of the row's slab pairs (eight coalesced 512-byte
 // loads in flight), the four quarters meet in LDS, then the target logit is read and lse and the row loss are written.
@@ -619,8 +684,22 @@ extern "C" int tfb_lmhead_fwd(const void* x, const void* W, const void* targets,
   // workgroup and nothing to hide its epilogue behind); a wavefront spans 64 vocabulary columns.
   using Cfg = GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>;
   GemmOperand P{(const uint8_t*)W, (long)d * 2}, Q{(const uint8_t*)x, (long)d * 2};
-  EpiLmHead e{(bf16_t*)logits, (float*)part, (long)V, rows, V / 64, softcap};
   int st;
+  // Where the persistent 256 x 256 kernel takes the shape, its plain store and a pass over the logits are cheaper than the
+  // exponentials in an epilogue that nothing overlaps (the call, without / with a softcap: 9600 x 8192 x 1024 261 -> 193 us /
+  // 264 -> 210, 2048 x 32768 x 768 150 -> 118 / 161 -> 121, 32768 x 32768 x 768 2166 -> 2096 / 2292 -> 2047).
+  if (gemm_pp_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, V, (int)rows, (long)d * 2, false, EpiStore{logits, (long)V, 0, 0}, s, st)) {
+    if (st != TFB_OK) return st;
+    if (idx64)
+      hipLaunchKernelGGL(lmhead_rows_kernel<long>, dim3((unsigned)rows), dim3(256), 0, s, (const bf16_t*)logits, (const long*)targets,
+                         (const float*)row_w, (float*)loss, (float*)lse, V, softcap);
+    else
+      hipLaunchKernelGGL(lmhead_rows_kernel<int>, dim3((unsigned)rows), dim3(256), 0, s, (const bf16_t*)logits, (const int*)targets,
+                         (const float*)row_w, (float*)loss, (float*)lse, V, softcap);
+    TFB_LAUNCH_CHECK();
+    return TFB_OK;
+  }
+  EpiLmHead e{(bf16_t*)logits, (float*)part, (long)V, rows, V / 64, softcap};
   if (!gemm_ring_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, V, (int)rows, (long)d * 2, e, s, st))
     st = gemm_launch<Cfg>(P, Q, V, (int)rows, (long)d * 2, 1, LoadIdentity{}, LoadIdentity{}, e, s);
   if (st != TFB_OK) return st;
