@@ -1003,6 +1003,28 @@ def test_attention_head_dim_128_at_the_reference_lengths(ops, dev, T, nw):
         assert rel_l2(dq[sl], dqo) < BF16_TOL and rel_l2(dk[sl], dko) < BF16_TOL and rel_l2(dv[sl], dvo) < BF16_TOL
 
 
+@pytest.mark.parametrize("B,H,T,nw", [(1, 1, 128, 0), (1, 2, 256, 0), (1, 3, 384, 0), (2, 4, 640, 1), (1, 8, 640, 2), (8, 16, 512, 0)])
+def test_attention_head_dim_128_pipelined_over_few_tiles(ops, dev, B, H, T, nw):
+    """The software-pipelined tile loops at their shortest: a single query block (no full tile, no half tile before the diagonal),
+    two and three, bands of one and two tiles, paired and unpaired grids; keys grow along the sequence, so that the running maximum
+    and with it the reference point of the exponentials moves from tile to tile."""
+    from oracle import attention as O
+    D, band, scale = 128, nw or None, 1.0 / math.sqrt(128)
+    g = _g(B + H + T + nw)
+    q, k, v = (torch.randn(B, H, T, D, generator=g) for _ in range(3))
+    q, k, v = q.bfloat16(), (k * torch.linspace(0.5, 6, T)[:, None]).bfloat16(), v.bfloat16()
+    do = torch.randn(B, T, H, D, generator=g).bfloat16()
+    kw = {"band": nw} if nw else {}
+    o, lse = ops.attn_fwd(q.to(dev), k.to(dev), v.to(dev), scale, **kw)
+    dq, dk, dv = ops.attn_bwd(q.to(dev), k.to(dev), v.to(dev), o, do.to(dev), lse, scale, **kw)
+    b, h = B - 1, H - 1
+    sl = (slice(b, b + 1), slice(h, h + 1))
+    oo, lo = O.forward(q[sl], k[sl], v[sl], scale, band_tiles=band)
+    assert rel_l2(o[b:b + 1, :, h:h + 1], oo) < BF16_TOL and rel_l2(lse[sl], lo) < 1e-4
+    want = O.backward(q[sl], k[sl], v[sl], o[b:b + 1, :, h:h + 1].cpu(), do[b:b + 1, :, h:h + 1], lse[sl].cpu(), scale, band_tiles=band)
+    for got, w in zip((dq, dk, dv), want):
+        assert rel_l2(got[sl], w) < BF16_TOL
+
 
 # ------------------------------------------------------------------------------------------ loss head
 @pytest.mark.parametrize("cap", [15.0, None])

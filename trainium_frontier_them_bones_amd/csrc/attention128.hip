@@ -6,7 +6,7 @@
 //     which ONE copy of a tile serves both MFMA operand forms without bank conflicts: token-major fragments (ds_read_b128:
 //     16 consecutive tokens of one chunk on 16 different 16-byte bank groups) and transposed fragments
 //     (ds_read_b64_tr_b16: the four tokens of a 32-lane access on four different 64-byte bank quarters);
-//   * two LDS stages (separate __shared__ objects), one barrier per stage;
+//   * two to four LDS stages, one barrier per stage, the next stages' loads in flight behind it;
 //   * workgroups re-dealt so that all sequence blocks of a (batch, head) pair run on one XCD (its L2 then serves the K/V or
 //     Q/dO tiles those blocks stream repeatedly), and a workgroup does block i and then block nx - 1 - i (equal causal work
 //     per workgroup);
@@ -14,19 +14,15 @@
 //     scalars and the packed score registers are directly the B operand of the second product;
 //   * the backward accumulators start from the rows' -lse / scale and -delta, which the dQ kernel makes from the dO
 //     fragments it holds anyway and leaves for dK/dV.
-// The tile loops are plain (not software-pipelined): at D = 128 a second set of scores does not fit the registers of two
-// wavefronts per SIMD. Forward and dQ run two wavefronts per SIMD (221 / 256 registers); dK/dV holds K, V fragments and
-// both gradients' accumulators (192 registers before any score) and runs one (at two it spills 100 registers and takes
-// 0.52 instead of 0.38 ms at B16 H6 T2048).
+// The tile loops are software-pipelined by hand, slot by slot: an MFMA, the LDS read of a fragment that a later slot uses, and a
+// share of the elementwise work of the neighbouring tile. What bounds them: two wavefronts per SIMD (forward, dQ: all 256 registers)
+// share the matrix pipe, which an MFMA holds for 32 cycles and a dot product (the rounded row sum) for about 16; one wavefront alone
+// on its SIMD (dK/dV with K, V and both gradients in 340 registers, and every kernel when the grid leaves CUs half empty) issues an
+// instruction every five cycles, so there the count of instructions per MFMA is the time.
+// Before, with plain loops whose LDS reads stood right in front of their MFMAs -> now: B3 H8 T1664 forward 52 -> 35 us, backward
+// 164 -> 118; B1 H8 T2048 56 -> 35, 177 -> 122; B16 H6 T2048 155 -> 120, 600 -> 475.
 #include <type_traits>
 #include "common.hpp"
-
-#ifndef TFB_DKDV128_R
-#define TFB_DKDV128_R 64  // queries per LDS stage of the dK/dV kernel (128: 0.39 vs 0.38 ms at B16 H6 T2048)
-#endif
-#ifndef TFB_DKDV128_WPE
-#define TFB_DKDV128_WPE 1  // wavefronts per SIMD the dK/dV kernel is compiled for
-#endif
 
 namespace {
 
@@ -37,9 +33,7 @@ struct AttnT {
 
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef const __attribute__((address_space(1))) void glb_void_t;
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4_t;
+typedef __attribute__((address_space(1))) uint8_t glb_u8_t;
 
 constexpr float LOG2E = 1.4426950408889634f;
 constexpr float LN2 = 0.6931471805599453f;
@@ -52,7 +46,6 @@ __device__ __forceinline__ bf16x8 frag_from(uint32_t a, uint32_t b, uint32_t c, 
   u32x4 v = {a, b, c, d};
   return __builtin_bit_cast(bf16x8, v);
 }
-__device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // s_waitcnt vmcnt(0)
 
 template <int D>
 struct Geo {
@@ -117,38 +110,23 @@ struct TileLoad {
     const int lrow = lane / G::LPT;
     // token = TPI g + lrow with g = wave + 4 i: the swizzle depends on g only through bits that 4 i does not touch
     const int chunk = (lane % G::LPT) ^ G::swz(G::TPI * wave + lrow);
-    voff = (uint32_t)(lrow * stride + chunk * 16);
+    voff = (uint32_t)((G::TPI * wave + lrow) * stride + chunk * 16);
+  }
+  __device__ __forceinline__ void issue_one(int i, const uint8_t* rows, long stride, uint8_t* lds) const {
+    const glb_u8_t* r = (const glb_u8_t*)rows;
+    uint32_t o = voff;
+    asm volatile("" : "+v"(o));   // (its widening stays in this block, where the load takes it as a 32-bit offset)
+    __builtin_amdgcn_global_load_lds((glb_void_t*)(r + i * (4 * G::TPI) * stride + o), (lds_void_t*)(lds + (wave + 4 * i) * 1024), 16, 0, 0);
   }
   __device__ __forceinline__ void issue(const uint8_t* rows, long stride, uint8_t* lds) const {
+    const glb_u8_t* r = (const glb_u8_t*)rows;   // (uniform base + 32-bit lane offset: no 64-bit address per lane)
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const int g = wave + 4 * i;
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(rows + (long)G::TPI * g * stride + (size_t)voff),
-                                       (lds_void_t*)(lds + g * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((glb_void_t*)(r + voff), (lds_void_t*)(lds + (wave + 4 * i) * 1024), 16, 0, 0);
+      r += 4 * G::TPI * stride;
     }
   }
 };
-
-// token-major fragment: token = 32 half + (lane & 31), elements 16 s + 8 (lane >> 5) .. + 7
-template <int D>
-__device__ __forceinline__ bf16x8 frag_rows(const uint8_t* tile, int half, int s, int lr, int lh) {
-  const int t = 32 * half + lr;
-  return *(const bf16x8*)(tile + t * Geo<D>::ROWB + (((2 * s + lh) ^ Geo<D>::swz(t)) << 4));
-}
-// transposed fragment: element (MFMA row) 32 dt + (lane & 31); tokens tok0 + 4 lh + {0..3} and tok0 + 8 + 4 lh + {0..3}
-template <int D>
-__device__ __forceinline__ bf16x8 frag_cols(const uint8_t* tile, int dt, int tok0, int lane) {
-  typedef Geo<D> G;
-  const int g4 = lane >> 4, j = lane & 15;
-  const int d = 32 * dt + 16 * (g4 & 1) + 4 * (j & 3);
-  const int t = tok0 + 4 * (g4 >> 1) + (j >> 2);
-  const int off0 = t * G::ROWB + (((d >> 3) ^ G::swz(t)) << 4) + ((d & 4) << 1);
-  const int off1 = (t + 8) * G::ROWB + (((d >> 3) ^ G::swz(t + 8)) << 4) + ((d & 4) << 1);
-  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(tile + off0));
-  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t*)(tile + off1));
-  const s16x8 v = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-  return __builtin_bit_cast(bf16x8, v);
-}
 
 // One token's gradient row from the NDT accumulators a lane holds (elements 32 dt + 8 j + 4 lh + i), scaled and rounded
 // once to bf16.
@@ -164,14 +142,94 @@ __device__ __forceinline__ void store_grad_row(const f32x16 (&acc)[Geo<D>::NDT],
     }
 }
 
+// ------------------------------------------------------------------------------------ pipelined fragment reads
+// The tile loops below are written slot by slot: one MFMA, the LDS read of the fragment that a later slot needs, and this slot's
+// share of the elementwise work, kept in that order by sched_barrier(0). Fragments are read by inline assembly and tied to an
+// explicit s_waitcnt lgkmcnt(n) right before their MFMA: left to the compiler, each read sits in front of its MFMA and every one
+// pays the LDS latency.
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+
+template <int I, int N, class F>
+__device__ __forceinline__ void slots(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    slots<I + 1, N>(f);
+  }
+}
+__device__ __forceinline__ void slot_end() { __builtin_amdgcn_sched_barrier(0); }
+
+// values made in this slot (they would otherwise sink to the block that uses them)
+__device__ __forceinline__ void pin(float& a, float& b) { asm volatile("" : "+v"(a), "+v"(b)); }
+template <class T>
+__device__ __forceinline__ void pin(T& a) { asm volatile("" : "+v"(a)); }
+__device__ __forceinline__ int opaque(int x) {  // (comparisons against it stay where they are used, not in registers across the loop)
+  asm volatile("" : "+v"(x));
+  return x;
+}
+struct RowFrag {  // a token-major fragment on its way: one 16-byte read
+  i32x4_t v;
+  template <int OFF>
+  __device__ __forceinline__ void request(uint32_t addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+  }
+  __device__ __forceinline__ bf16x8 get() const { return __builtin_bit_cast(bf16x8, v); }
+};
+struct ColFrag {  // a transposed fragment: two 8-byte reads
+  u32x2 a, b;
+  template <int OFF>
+  __device__ __forceinline__ void request(uint32_t lo, uint32_t hi) {
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(a) : "v"(lo), "n"(OFF));
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(b) : "v"(hi), "n"(OFF));
+  }
+  __device__ __forceinline__ bf16x8 get() const { return frag_from(a.x, a.y, b.x, b.y); }
+};
+// Two fragments are waited for together: one wavefront alone on its SIMD issues an instruction every five cycles, seven under an MFMA.
+// AFTER: LDS instructions issued since the second's.
+template <int AFTER>
+__device__ __forceinline__ void landed(RowFrag& x, RowFrag& y) {
+  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(x.v), "+v"(y.v) : "n"(AFTER));
+}
+template <int AFTER>
+__device__ __forceinline__ void landed(ColFrag& x, ColFrag& y) {
+  asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(x.a), "+v"(x.b), "+v"(y.a), "+v"(y.b) : "n"(AFTER));
+}
+// Per-lane addresses of the fragments of a tile at `base`. Token-major, rows[s]: token lane & 31, elements 16 s + 8 (lane >> 5) .. + 7.
+// Transposed, lo[dt] and hi[dt]: element (MFMA row) 32 dt + (lane & 31), tokens 4 lh + {0..3} and 8 + 4 lh + {0..3}. A tile's place,
+// the 32-token half and the 16-token step are added, as the instruction's offset where they are constants.
+template <int D>
+struct FragAddr {
+  uint32_t rows[Geo<D>::NKS], lo[Geo<D>::NDT], hi[Geo<D>::NDT];
+  __device__ __forceinline__ void init(uint32_t base, int lane) {
+    typedef Geo<D> G;
+    const int lr = lane & 31, lh = lane >> 5, g4 = lane >> 4, j = lane & 15;
+#pragma unroll
+    for (int s = 0; s < G::NKS; ++s) rows[s] = base + lr * G::ROWB + (((2 * s + lh) ^ G::swz(lr)) << 4);
+    const int t = 4 * (g4 >> 1) + (j >> 2);
+#pragma unroll
+    for (int dt = 0; dt < G::NDT; ++dt) {
+      const int d = 32 * dt + 16 * (g4 & 1) + 4 * (j & 3);
+      lo[dt] = base + t * G::ROWB + (((d >> 3) ^ G::swz(t)) << 4) + ((d & 4) << 1);
+      hi[dt] = base + (t + 8) * G::ROWB + (((d >> 3) ^ G::swz(t + 8)) << 4) + ((d & 4) << 1);
+    }
+  }
+};
+// all of this wavefront's loads into LDS have landed, and every wavefront is here
+__device__ __forceinline__ void tile_barrier() { asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ float max_halves(float x) {  // the larger of the two lanes' that share a query
+  float y = x;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y));
+  return fmaxf(x, y);
+}
+
 // =========================================================================================== forward
 template <int D>
 __global__ __launch_bounds__(256, 2) void attnD_fwd_kernel(AttnT q, AttnT k, AttnT v, AttnT o, float* __restrict__ lse, int T,
                                                            int H, float sl2, int nw) {
   typedef Geo<D> G;
-  constexpr int TILE = G::TILE, NKS = G::NKS, NDT = G::NDT;
-  __shared__ __attribute__((aligned(1024))) uint8_t st0[2 * TILE];
-  __shared__ __attribute__((aligned(1024))) uint8_t st1[2 * TILE];
+  constexpr int TILE = G::TILE, NKS = G::NKS, NDT = G::NDT, NA = 2 * NKS, NB = 4 * NDT;
+  constexpr int AH = 4;  // fragments asked for ahead of their MFMA (6: no register left, 1 % slower)
+  static_assert(NA == 16 && NB == 16, "a slot for each packed pair of scores");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * TILE];  // K even, K odd, V even, V odd tile
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int bx, bh;
@@ -186,90 +244,231 @@ __global__ __launch_bounds__(256, 2) void attnD_fwd_kernel(AttnT q, AttnT k, Att
   TileLoad<D, 16 / G::TPI> lk, lv;
   lk.init(kst, wave, lane);
   lv.init(vst, wave, lane);
-  auto issue = [&](uint8_t* st, int tile) {
-    lk.issue(kp + (long)tile * 64 * kst, kst, st);
-    lv.issue(vp + (long)tile * 64 * vst, vst, st + TILE);
-  };
+  auto issue_k = [&](int tile) { lk.issue(kp + (long)tile * 64 * kst, kst, lds + (tile & 1) * TILE); };
+  auto issue_v = [&](int tile) { lv.issue(vp + (long)tile * 64 * vst, vst, lds + (2 + (tile & 1)) * TILE); };
+  FragAddr<D> fa;
+  fa.init((uint32_t)(uintptr_t)(lds_void_t*)lds, lane);
+
   for (int pass = 0; pass < npass; ++pass) {
     const int qb = paired_block(nx, bx, pass, true);
     const int q0 = qb * 128, qw0 = q0 + wave * 32;
     bf16x8 qf[NKS];
 #pragma unroll
     for (int s = 0; s < NKS; ++s) qf[s] = *(const bf16x8*)(qp + (long)(qw0 + lr) * q.st + 16 * s + 8 * lh);
+    const int n = (q0 + 128) / 64;               // even; tiles n - 2 and n - 1 cover the workgroup's own 128 tokens
+    const int t0 = band_first_tile(qb, nw);      // even
+    const int last = n - 2 + (wave >> 1);        // the wavefront's diagonal tile; tiles beyond are in its future
+    issue_k(t0);
+    issue_v(t0);
+    issue_k(t0 + 1);
+
     f32x16 oacc[NDT];
     float m = -1e30f, l = 0.f;  // running maximum of the raw scores, running sum
 #pragma unroll
     for (int i = 0; i < NDT; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) oacc[i][e] = 0.f;
+    f32x16 scA[2], scB[2];  // raw scores S = K Q^T of an even and an odd tile (key = MFMA row: a lane holds 32 keys of one query)
+    uint32_t pA[16], pB[16];
+    RowFrag kf[NA];
+    ColFrag vf[NB];
+    float mx = 0.f, mx1 = 0.f;  // (two chains)
 
-    // one 64-key tile against the wavefront's 32 queries
-    auto tile_step = [&](const uint8_t* st, int tile) {
-      const int k0 = tile * 64;
-      if (k0 > qw0 + 31) return;  // every key in this wavefront's future
-      f32x16 sc[2];
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) sc[kt][e] = 0.f;
-#pragma unroll
-        for (int s = 0; s < NKS; ++s) sc[kt] = mfma_bf16(frag_rows<D>(st, kt, s, lr, lh), qf[s], sc[kt]);
+    auto request = [&](auto par, auto slot) {  // slots 0 .. NA - 1: K of the next tile, then V of this one; par: this tile's parity
+      constexpr int i = decltype(slot)::value, P = decltype(par)::value;
+      if constexpr (i < NA) kf[i].template request<(P ^ 1) * TILE + (i / NKS) * 32 * G::ROWB>(fa.rows[i % NKS]);
+      else if constexpr (i < NA + NB)
+        vf[i - NA].template request<(2 + P) * TILE + ((i - NA) / NDT) * 16 * G::ROWB>(fa.lo[(i - NA) % NDT], fa.hi[(i - NA) % NDT]);
+    };
+    auto score_slot = [&](auto slot, f32x16 (&sn)[2]) {
+      constexpr int i = decltype(slot)::value, kt = i / NKS, s = i % NKS;
+      constexpr int after = i + AH <= NA ? AH - 2 : (NA - 2 - i) + 2 * (i + AH - NA);
+      if constexpr (i % 2 == 0) landed<after>(kf[i], kf[i + 1]);
+      const bf16x8 f = kf[i].get();
+      if constexpr (s == 0) sn[kt] = mfma_bf16(f, qf[s], f32x16{});
+      else sn[kt] = mfma_bf16(f, qf[s], sn[kt]);
+    };
+    auto out_slot = [&](auto slot, const uint32_t (&pw)[16]) {
+      constexpr int i = decltype(slot)::value;
+      constexpr int after = 2 * (i + AH <= NB ? AH - 2 : NB - 2 - i);
+      if constexpr (i % 2 == 0) landed<after>(vf[i], vf[i + 1]);
+      const bf16x8 f = vf[i].get();
+      constexpr int g = i / NDT;
+      oacc[i % NDT] = mfma_bf16(f, frag_from(pw[4 * g], pw[4 * g + 1], pw[4 * g + 2], pw[4 * g + 3]), oacc[i % NDT]);
+    };
+    // P = exp2(sl2 (S - m)) rounded to bf16, word by word (two scores), a word's steps in different slots so that none waits for the
+    // one before; the row sum runs over the rounded values
+    float f0, f1;
+    auto step_f = [&](auto word, const f32x16 (&sc)[2], float negm) {
+      constexpr int i = decltype(word)::value, kt = i >> 3, e = 2 * (i & 7);
+      f0 = fmaf(sc[kt][e], sl2, negm);
+      f1 = fmaf(sc[kt][e + 1], sl2, negm);
+      pin(f0, f1);
+    };
+    auto step_x = [&]() {
+      f0 = fast_exp2(f0);
+      f1 = fast_exp2(f1);
+      pin(f0, f1);
+    };
+    auto step_c = [&](auto word, uint32_t (&pw)[16]) {
+      pw[decltype(word)::value] = pack2bf(f0, f1);
+      pin(pw[decltype(word)::value]);
+    };
+    auto step_d = [&](auto word, const uint32_t (&pw)[16]) {
+      l = sum2bf(pw[decltype(word)::value], l);
+      pin(l);
+    };
+    auto exp_word = [&](auto word, const f32x16 (&sc)[2], float negm, uint32_t (&pw)[16]) {
+      step_f(word, sc, negm);
+      step_x();
+      step_c(word, pw);
+    };
+    // slot r of a run of words from w0 on, two slots a word
+    auto run_slot = [&](auto r, auto w0, const f32x16 (&sc)[2], float negm, uint32_t (&pw)[16]) {
+      constexpr int R = decltype(r)::value, W = decltype(w0)::value + R / 2;
+      if constexpr (R % 2 == 0) {
+        step_x();
+      } else {
+        step_c(std::integral_constant<int, W>{}, pw);
+        if constexpr (W < 15) step_f(std::integral_constant<int, W + 1>{}, sc, negm);
       }
-      if (k0 + 63 > qw0) {  // wavefront-uniform; the per-element masking is branch-free selects
-        const int kbase = k0 + lh * 4 - (qw0 + lr);  // key - q for element (kt, e) is kbase + kt*32 + (e>>2)*8 + (e&3)
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) sc[kt][e] = (kbase + kt * 32 + (e >> 2) * 8 + (e & 3) > 0) ? -INFINITY : sc[kt][e];
-      }
-      float mx = m;
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int e = 0; e < 16; e += 2) mx = fmaxf(fmaxf(mx, sc[kt][e]), sc[kt][e + 1]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      // the reference point of the exponentials follows the running maximum only when some row's maximum has grown by more
-      // than 2^8: O and lse do not depend on it
-      if (__builtin_amdgcn_ballot_w64((mx - m) * sl2 > 8.0f)) {
-        const float alpha = fast_exp2((m - mx) * sl2);
+    };
+    auto max_pair = [&](auto pair, const f32x16 (&sc)[2]) {
+      constexpr int i = decltype(pair)::value, kt = i >> 3, e = 2 * (i & 7);
+      if constexpr (i % 2 == 0) mx = fmaxf(fmaxf(mx, sc[kt][e]), sc[kt][e + 1]);
+      else mx1 = fmaxf(fmaxf(mx1, sc[kt][e]), sc[kt][e + 1]);
+    };
+    // the reference point of the exponentials follows the running maximum only when some row's maximum has grown by more
+    // than 2^8: O and lse do not depend on it. O is scaled after the product that is under way.
+    float alpha = 1.f;
+    auto follow_max = [&]() -> bool {
+      mx = max_halves(fmaxf(mx, mx1));
+      const bool grow = __builtin_amdgcn_ballot_w64((mx - m) * sl2 > 8.0f) != 0;
+      if (grow) {
+        alpha = fast_exp2((m - mx) * sl2);
         m = mx;
         l *= alpha;
-#pragma unroll
-        for (int i = 0; i < NDT; ++i)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) oacc[i][e] *= alpha;
       }
-      const float negm = -m * sl2;
+      return grow;
+    };
+    auto rescale = [&]() {
+#pragma unroll
+      for (int i = 0; i < NDT; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) oacc[i][e] *= alpha;
+    };
+    auto mask = [&](int tile, f32x16 (&sc)[2]) {
+      const int kbase = opaque(tile * 64 + lh * 4 - (qw0 + lr));  // key - q for element (kt, e) is kbase + kt*32 + (e>>2)*8 + (e&3)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-          uint32_t pw[4];
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const int e = 8 * hf + 2 * x;
-            const float p0 = fast_exp2(fmaf(sc[kt][e], sl2, negm)), p1 = fast_exp2(fmaf(sc[kt][e + 1], sl2, negm));
-            pw[x] = pack2bf(p0, p1);
-            l = sum2bf(pw[x], l);
-          }
-          const bf16x8 bb = frag_from(pw[0], pw[1], pw[2], pw[3]);
-#pragma unroll
-          for (int dt = 0; dt < NDT; ++dt) oacc[dt] = mfma_bf16(frag_cols<D>(st + TILE, dt, kt * 32 + 16 * hf, lane), bb, oacc[dt]);
-        }
+        for (int e = 0; e < 16; ++e) sc[kt][e] = (kbase + kt * 32 + (e >> 2) * 8 + (e & 3) > 0) ? -INFINITY : sc[kt][e];
+    };
+    // Tile t (parity par): its words 4 .. 11 run under the next tile's scores, words 12 .. 15, the next tile's row maximum and its
+    // words 0 .. 3 under O += P V. The dot products of the row sum need the matrix pipe and go together where it is free.
+    // One barrier per tile: past it tile t + 1's K and tile t's V are in LDS and the buffers of K t and V t - 1 are free.
+    constexpr std::integral_constant<int, 0> c0{};
+    constexpr std::integral_constant<int, 4> c4{};
+    auto full_tile = [&](auto par, int t, f32x16 (&sc)[2], f32x16 (&sn)[2], uint32_t (&pc)[16], uint32_t (&pn)[16]) {
+      tile_barrier();
+      slots<0, AH>([&](auto i) { request(par, i); });
+      const int tk = t + 2 < n ? t + 2 : n - 1;
+      const uint8_t* kr = kp + (long)tk * 64 * kst;
+      const uint8_t* vr = vp + (long)(t + 1) * 64 * vst;
+      uint8_t* kd = lds + decltype(par)::value * TILE;
+      uint8_t* vd = lds + (2 + (decltype(par)::value ^ 1)) * TILE;
+      float negm = -m * sl2;
+      mx = m;
+      mx1 = m;
+      slots<0, 4>([&](auto i) { step_d(i, pc); });
+      slot_end();
+      slots<0, NA>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        score_slot(i, sn);
+        request(par, std::integral_constant<int, x + AH>{});
+        if constexpr (x < 4) lk.issue_one(x, kr, kst, kd);
+        else if constexpr (x < 8) lv.issue_one(x - 4, vr, vst, vd);
+        run_slot(i, c4, sc, negm, pc);
+        if constexpr (x >= 9) max_pair(std::integral_constant<int, x - 9>{}, sn);
+        slot_end();
+      });
+      if (t + 1 == last) {
+        mask(t + 1, sn);
+        mx = m;
+        mx1 = m;
+        slots<0, 7>([&](auto j) { max_pair(j, sn); });
+      }
+      slots<0, 8>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        out_slot(i, pc);
+        request(par, std::integral_constant<int, x + AH + NA>{});
+        run_slot(std::integral_constant<int, x + NA>{}, c4, sc, negm, pc);
+        if constexpr (x == 0) max_pair(std::integral_constant<int, 7>{}, sn);
+        if constexpr (x >= 2 && x < 6) slots<2 * x + 4, 2 * x + 6>([&](auto j) { max_pair(j, sn); });
+        slot_end();
+      });
+      slots<4, 16>([&](auto i) { step_d(i, pc); });
+      const bool grow = follow_max();
+      negm = -m * sl2;
+      step_f(c0, sn, negm);
+      slots<8, NB>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        out_slot(i, pc);
+        request(par, std::integral_constant<int, x + AH + NA>{});
+        run_slot(std::integral_constant<int, x - 8>{}, c0, sn, negm, pn);
+        slot_end();
+      });
+      if (grow) rescale();
+    };
+    // the wavefront's last tile: no scores to make
+    auto last_tile = [&](auto par, f32x16 (&sc)[2], uint32_t (&pc)[16]) {
+      const float negm = -m * sl2;
+      slots<NA, NA + AH>([&](auto i) { request(par, i); });
+      slots<4, 8>([&](auto i) { exp_word(i, sc, negm, pc); });
+      slot_end();
+      slots<0, NB>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        out_slot(i, pc);
+        request(par, std::integral_constant<int, x + AH + NA>{});
+        if constexpr (x < 8) exp_word(std::integral_constant<int, x + 8>{}, sc, negm, pc);
+        slot_end();
+      });
+      slots<0, 16>([&](auto i) { step_d(i, pc); });
     };
 
-    const int n = (q0 + 128) / 64;           // even; tiles n - 2 and n - 1 cover the workgroup's own 128 tokens
-    const int t0 = band_first_tile(qb, nw);  // even
-    issue(st0, t0);
-    wait_all_loads();
-    __syncthreads();
-    for (int t = t0; t < n; t += 2) {
-      issue(st1, t + 1);
-      tile_step(st0, t);
-      __syncthreads();
-      if (t + 2 < n) issue(st0, t + 2);
-      tile_step(st1, t + 1);
-      __syncthreads();
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    asm volatile("s_waitcnt vmcnt(8)\n\ts_barrier" ::: "memory");  // tile t0's K
+    slots<0, AH>([&](auto i) { request(odd, i); });
+    slots<0, NA>([&](auto i) {
+      constexpr int x = decltype(i)::value;
+      if constexpr (x % 2 == 0) landed<(x + AH <= NA ? AH - 2 : NA - 2 - x)>(kf[x], kf[x + 1]);
+      const bf16x8 f = kf[x].get();
+      if constexpr (x % NKS == 0) scA[x / NKS] = mfma_bf16(f, qf[0], f32x16{});
+      else scA[x / NKS] = mfma_bf16(f, qf[x % NKS], scA[x / NKS]);
+      if constexpr (x + AH < NA) request(odd, std::integral_constant<int, x + AH>{});
+      slot_end();
+    });
+    if (t0 == last) mask(t0, scA);
+    mx = m;
+    mx1 = m;
+    slots<0, 16>([&](auto i) { max_pair(i, scA); });
+    follow_max();  // (O is zero)
+    slots<0, 4>([&](auto i) { exp_word(i, scA, -m * sl2, pA); });
+    step_f(c4, scA, -m * sl2);
+    for (int t = t0; t + 2 < n; t += 2) {
+      full_tile(even, t, scA, scB, pA, pB);
+      full_tile(odd, t + 1, scB, scA, pB, pA);
+    }
+    if (wave >= 2) {
+      full_tile(even, n - 2, scA, scB, pA, pB);
+      tile_barrier();
+      last_tile(odd, scB, pB);
+    } else {   // (V of the last tile is loaded for the others)
+      tile_barrier();
+      issue_v(n - 1);
+      last_tile(even, scA, pA);
+      tile_barrier();
     }
 
     const int myq = qw0 + lr;
@@ -285,6 +484,7 @@ __global__ __launch_bounds__(256, 2) void attnD_fwd_kernel(AttnT q, AttnT k, Att
         *(u32x2*)(op + (long)myq * o.st + d) = w;
       }
     if (lh == 0) lse[(long)bh * T + myq] = (m * sl2 + log2f(lt)) * LN2;  // m is the raw-score maximum
+    if (pass + 1 < npass) __syncthreads();  // the stages are free for the partner block
   }
 }
 
@@ -296,8 +496,9 @@ __global__ __launch_bounds__(256, 2) void attnD_dq_kernel(AttnT q, AttnT k, Attn
                                                                         const float* __restrict__ lse) {
   typedef Geo<D> G;
   constexpr int TILE = G::TILE, NKS = G::NKS, NDT = G::NDT;
-  __shared__ __attribute__((aligned(1024))) uint8_t st0[2 * TILE];
-  __shared__ __attribute__((aligned(1024))) uint8_t st1[2 * TILE];
+  constexpr int AH = 4;  // fragments asked for ahead of their MFMA: from slot 20 on, behind the barrier, the next half's
+  static_assert(NKS == 8 && NDT == 4, "three phases of eight slots");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * TILE];  // K even, K odd, V even, V odd tile
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int bx, bh;
@@ -312,13 +513,19 @@ __global__ __launch_bounds__(256, 2) void attnD_dq_kernel(AttnT q, AttnT k, Attn
   TileLoad<D, 16 / G::TPI> lk, lv;
   lk.init(kst, wave, lane);
   lv.init(vst, wave, lane);
-  auto issue = [&](uint8_t* st, int tile) {
-    lk.issue(kp + (long)tile * 64 * kst, kst, st);
-    lv.issue(vp + (long)tile * 64 * vst, vst, st + TILE);
-  };
+  auto issue_k = [&](int tile) { lk.issue(kp + (long)tile * 64 * kst, kst, lds + (tile & 1) * TILE); };
+  auto issue_v = [&](int tile) { lv.issue(vp + (long)tile * 64 * vst, vst, lds + (2 + (tile & 1)) * TILE); };
+  FragAddr<D> fa;
+  fa.init((uint32_t)(uintptr_t)(lds_void_t*)lds, lane);
   for (int pass = 0; pass < npass; ++pass) {
     const int qb = paired_block(nx, bx, pass, true);
     const int q0 = qb * 128, qw0 = q0 + wave * 32, myq = qw0 + lr;
+    const int n = (q0 + 128) / 64;           // even; tiles n - 2 and n - 1 cover the workgroup's own 128 tokens
+    const int t0 = band_first_tile(qb, nw);  // even
+    issue_k(t0);
+    issue_v(t0);
+    issue_k(t0 + 1);
+    issue_v(t0 + 1);
     bf16x8 qf[NKS], gf[NKS];
 #pragma unroll
     for (int s = 0; s < NKS; ++s) {
@@ -351,76 +558,191 @@ __global__ __launch_bounds__(256, 2) void attnD_dq_kernel(AttnT q, AttnT k, Attn
 #pragma unroll
       for (int e = 0; e < 16; ++e) dqa[i][e] = 0.f;
 
-    auto tile_step = [&](const uint8_t* st, int tile) {
+    // Half tiles of 32 keys, h = 2 tile + half, at LDS offset (h & 3) TILE / 2. While half h's dS and dQ += dS K are made, half
+    // h + 1's S and dP are: 24 slots of one MFMA, S (0 .. 7), dP (8 .. 15), dQ (16 .. 23). The wavefront's last half is the one on
+    // its diagonal. One barrier per half, before slot 20: this half's columns have been read and what the half before asked for has
+    // landed, so that V t + 2 (K t + 2) may replace V t (K t) behind an even (odd) half's barrier and the next half's rows be read.
+    f32x16 Sn, dP;
+    uint32_t pw[8], dsw[8];
+    float f0, f1;
+    RowFrag rf[16];
+    ColFrag cf[8];
+    constexpr int HALF = 32 * G::ROWB;
+    auto request_row = [&](auto slot, uint32_t off) {
+      constexpr int i = decltype(slot)::value;
+      rf[i].template request<i < 8 ? 0 : 2 * TILE>(fa.rows[i % 8] + off);
+    };
+    auto request_col = [&](auto slot, uint32_t off) {
+      constexpr int i = decltype(slot)::value - 16;
+      cf[i].template request<(i / NDT) * 16 * G::ROWB>(fa.lo[i % NDT] + off, fa.hi[i % NDT] + off);
+    };
+    // LDS instructions issued after fragment i + 1's when slot i waits for the two (0 behind the barrier, which waits for all but those after it)
+    auto after = [](int i) constexpr {
+      int c = 0;
+      for (int x = i + 2; x < i + AH; ++x) c += (x % 24) < 16 ? 1 : 2;
+      return c;
+    };
+    auto row_slot = [&](auto slot, auto aft) {
+      constexpr int i = decltype(slot)::value, s = i % 8;
+      if constexpr (i % 2 == 0) landed<decltype(aft)::value>(rf[i], rf[i + 1]);
+      const bf16x8 f = rf[i].get();
+      if constexpr (s == 0) {
+        float c = i < 8 ? myL : myD;
+        pin(c);  // (spread by moves each time: kept as constant operands the two would take 32 registers)
+        f32x16& x = i < 8 ? Sn : dP;
 #pragma unroll
-      for (int kt = 0; kt < 2; ++kt) {
-        const int klo = tile * 64 + kt * 32;
-        if (klo > qw0 + 31) continue;
-        f32x16 S, dP;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          S[e] = myL;
-          dP[e] = myD;
-        }
-#pragma unroll
-        for (int s = 0; s < NKS; ++s) S = mfma_bf16(frag_rows<D>(st, kt, s, lr, lh), qf[s], S);
-#pragma unroll
-        for (int s = 0; s < NKS; ++s) dP = mfma_bf16(frag_rows<D>(st + TILE, kt, s, lr, lh), gf[s], dP);
-        if (klo + 31 > qw0) {
-          const int kbase = klo + lh * 4 - myq;
-#pragma unroll
-          for (int e = 0; e < 16; ++e) S[e] = (kbase + (e >> 2) * 8 + (e & 3) > 0) ? -INFINITY : S[e];
-        }
-        uint32_t dsw[8];
-#pragma unroll
-        for (int e = 0; e < 16; e += 2) {
-          const float p0 = fast_exp2(S[e] * sl2), p1 = fast_exp2(S[e + 1] * sl2);
-          const uint32_t w = pack2bf(p0, p1);  // the reference multiplies dP - delta by the rounded P
-          dsw[e >> 1] = pack2bf(bflo(w) * dP[e], bfhi(w) * dP[e + 1]);
-        }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-          const bf16x8 db = frag_from(dsw[4 * ks], dsw[4 * ks + 1], dsw[4 * ks + 2], dsw[4 * ks + 3]);
-#pragma unroll
-          for (int dt = 0; dt < NDT; ++dt) dqa[dt] = mfma_bf16(frag_cols<D>(st, dt, kt * 32 + 16 * ks, lane), db, dqa[dt]);
-        }
+        for (int e = 0; e < 16; ++e) x[e] = c;
       }
+      if constexpr (i < 8) Sn = mfma_bf16(f, qf[s], Sn);
+      else dP = mfma_bf16(f, gf[s], dP);
+    };
+    auto col_slot = [&](auto slot, auto aft) {
+      constexpr int i = decltype(slot)::value - 16, ks = i / NDT, dt = i % NDT;
+      if constexpr (i % 2 == 0) landed<decltype(aft)::value>(cf[i], cf[i + 1]);
+      const bf16x8 f = cf[i].get();
+      dqa[dt] = mfma_bf16(f, frag_from(dsw[4 * ks], dsw[4 * ks + 1], dsw[4 * ks + 2], dsw[4 * ks + 3]), dqa[dt]);
+    };
+    auto ds_word = [&](auto word) {  // the reference multiplies dP - delta by the rounded P
+      constexpr int w = decltype(word)::value;
+      dsw[w] = pack2bf(bflo(pw[w]) * dP[2 * w], bfhi(pw[w]) * dP[2 * w + 1]);
+      pin(dsw[w]);
+    };
+    auto step_f = [&](auto word) {
+      constexpr int w = decltype(word)::value;
+      f0 = Sn[2 * w] * sl2;
+      f1 = Sn[2 * w + 1] * sl2;
+      pin(f0, f1);
+    };
+    auto step_x = [&]() {
+      f0 = fast_exp2(f0);
+      f1 = fast_exp2(f1);
+      pin(f0, f1);
+    };
+    auto step_c = [&](auto word) {
+      pw[decltype(word)::value] = pack2bf(f0, f1);
+      pin(pw[decltype(word)::value]);
+    };
+    auto mask = [&]() {  // Sn is the wavefront's diagonal
+      const int kbase = opaque(lh * 4 - lr);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) Sn[e] = (kbase + (e >> 2) * 8 + (e & 3) > 0) ? -INFINITY : Sn[e];
     };
 
-    const int n = (q0 + 128) / 64;
-    const int t0 = band_first_tile(qb, nw);
-    issue(st0, t0);
-    wait_all_loads();
-    __syncthreads();
-    for (int t = t0; t < n; t += 2) {
-      issue(st1, t + 1);
-      tile_step(st0, t);
-      __syncthreads();
-      if (t + 2 < n) issue(st0, t + 2);
-      tile_step(st1, t + 1);
-      __syncthreads();
+    const int h0 = 2 * t0, hl = 2 * (n - 2) + wave;
+    tile_barrier();
+    // half h0's S, dP and P
+    slots<0, AH>([&](auto i) { request_row(i, 0u); });
+    slots<0, 16>([&](auto i) {
+      constexpr int x = decltype(i)::value;
+      row_slot(i, std::integral_constant<int, (x + AH <= 16 ? AH - 2 : 14 - x) < 0 ? 0 : (x + AH <= 16 ? AH - 2 : 14 - x)>{});
+      if constexpr (x + AH < 16) request_row(std::integral_constant<int, x + AH>{}, 0u);
+      slot_end();
+    });
+    if (h0 == hl) mask();
+    slots<0, 8>([&](auto i) {
+      step_f(i);
+      step_x();
+      step_c(i);
+    });
+    slots<0, AH>([&](auto i) { request_row(i, (uint32_t)HALF); });
+    for (int hh = h0; hh < hl; ++hh) {
+      const uint32_t roff = ((hh + 1) & 3) * HALF, coff = (hh & 3) * HALF, noff = ((hh + 2) & 3) * HALF;
+      slot_end();
+      slots<0, 8>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        row_slot(i, std::integral_constant<int, after(x)>{});
+        request_row(std::integral_constant<int, x + AH>{}, roff);
+        ds_word(i);
+        slot_end();
+      });
+      row_slot(std::integral_constant<int, 8>{}, std::integral_constant<int, after(8)>{});
+      request_row(std::integral_constant<int, 8 + AH>{}, roff);
+      if (hh + 1 == hl) mask();
+      step_f(std::integral_constant<int, 0>{});
+      slot_end();
+      const int lt = (hh >> 1) + 2 < n ? (hh >> 1) + 2 : n - 1;
+      const bool odd = hh & 1;
+      const uint8_t* lp = odd ? kp + (long)lt * 64 * kst : vp + (long)lt * 64 * vst;
+      const long lst = odd ? kst : vst;
+      uint8_t* ld = lds + (odd ? 0 : 2 * TILE) + ((hh >> 1) & 1) * TILE;
+      slots<9, 24>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        if constexpr (x == 20) {
+          asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+          slot_end();
+        }
+        constexpr int aft = x < 20 ? after(x) : AH;  // (already there)
+        if constexpr (x < 16) row_slot(i, std::integral_constant<int, after(x)>{});
+        else col_slot(i, std::integral_constant<int, aft>{});
+        if constexpr (x + AH < 16) request_row(std::integral_constant<int, x + AH>{}, roff);
+        else if constexpr (x + AH < 24) request_col(std::integral_constant<int, x + AH>{}, coff);
+        else request_row(std::integral_constant<int, x + AH - 24>{}, noff);
+        if constexpr (x >= 20) (odd ? lk : lv).issue_one(x - 20, lp, lst, ld);
+        if constexpr (x % 2 == 1) {
+          step_x();
+        } else {
+          step_c(std::integral_constant<int, (x - 10) / 2>{});
+          step_f(std::integral_constant<int, (x - 8) / 2>{});
+        }
+        slot_end();
+      });
+      step_c(std::integral_constant<int, 7>{});
     }
+    // the wavefront's last half
+    {
+      const uint32_t coff = (hl & 3) * HALF;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the rows asked for are not used)
+      slots<0, AH>([&](auto i) { if constexpr (decltype(i)::value % 2 == 0) landed<0>(rf[decltype(i)::value], rf[decltype(i)::value + 1]); });
+      slots<16, 16 + AH>([&](auto i) { request_col(i, coff); });
+      slots<0, 8>([&](auto i) { ds_word(i); });
+      slot_end();
+      slots<16, 24>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        col_slot(i, std::integral_constant<int, x % 2 ? 0 : 2 * (x + AH <= 24 ? AH - 2 : 22 - x)>{});
+        if constexpr (x + AH < 24) request_col(std::integral_constant<int, x + AH>{}, coff);
+        slot_end();
+      });
+    }
+    for (int x = wave; x < 3; ++x) asm volatile("s_barrier" ::: "memory");  // the other wavefronts' halves
     bf16_t* dqp = dq.p + b * dq.sb + h * dq.sh + (long)myq * dq.st;
     store_grad_row<D>(dqa, scale, dqp, lh);
     if (lh == 0) {
       stats[(long)bh * T + myq] = myD;
       stats[rows + (long)bh * T + myq] = myL;
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (pass + 1 < npass) __syncthreads();  // the stages are free for the partner block
   }
 }
 
 // =========================================================================================== dK / dV
-template <int D, int R>  // R: queries per LDS stage (64 or 128)
-__global__ __launch_bounds__(256, D == 64 ? 2 : TFB_DKDV128_WPE) void attnD_dkdv_kernel(AttnT q, AttnT k, AttnT v, AttnT go, AttnT dk, AttnT dv,
+struct StatFrag {  // 32 rows' statistics as an accumulator's start: four 16-byte reads, into the half of the register file it is in
+  f32x4 v[4];
+  template <int OFF>
+  __device__ __forceinline__ void request(uint32_t addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=a"(v[0]) : "v"(addr), "n"(OFF));
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=a"(v[1]) : "v"(addr), "n"(OFF + 32));
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=a"(v[2]) : "v"(addr), "n"(OFF + 64));
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=a"(v[3]) : "v"(addr), "n"(OFF + 96));
+  }
+  template <int AFTER>
+  __device__ __forceinline__ void landed(f32x16& x) {
+    asm volatile("s_waitcnt lgkmcnt(%4)" : "+a"(v[0]), "+a"(v[1]), "+a"(v[2]), "+a"(v[3]) : "n"(AFTER));
+#pragma unroll
+    for (int e = 0; e < 16; ++e) x[e] = v[e >> 2][e & 3];
+  }
+};
+
+template <int D>
+__global__ __launch_bounds__(256, 1) void attnD_dkdv_kernel(AttnT q, AttnT k, AttnT v, AttnT go, AttnT dk, AttnT dv,
                                                                           const float* __restrict__ stats, long rows, int T,
                                                                           int H, float scale, float sl2, int nw) {
   typedef Geo<D> G;
-  constexpr int NKS = G::NKS, NDT = G::NDT;
-  constexpr int RT = R * G::ROWB;           // bytes of a staged Q (dO) tile
-  constexpr int RPB = 128 / R;              // stages per 128-token query tile
-  constexpr int STAGE = 2 * RT + 8 * R;     // Q tile, dO tile, R x (-lse / scale), R x (-delta)
-  __shared__ __attribute__((aligned(1024))) uint8_t st0[STAGE];
-  __shared__ __attribute__((aligned(1024))) uint8_t st1[STAGE];
+  constexpr int TILE = G::TILE, NKS = G::NKS, NDT = G::NDT, NI = 34;
+  constexpr int AH = 6;  // items asked for ahead of their use
+  static_assert(NKS == 8 && NDT == 4, "four phases of eight MFMAs");
+  constexpr int STAGE = 2 * TILE + 512;  // Q tile, dO tile, 64 x (-lse / scale), 64 x (-delta)
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * STAGE];
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int bx, bh;
@@ -434,33 +756,54 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : TFB_DKDV128_WPE) void attnD_dkdv
   const float* nlp = stats + rows + (long)bh * T;
   const int nx = T / 128, npass = paired_passes(nx);
   const long qst = q.st * 2, gst = go.st * 2;
-  TileLoad<D, R / 4 / G::TPI> lq, lg;
+  TileLoad<D, 16 / G::TPI> lq, lg;
   lq.init(qst, wave, lane);
   lg.init(gst, wave, lane);
+  FragAddr<D> fa;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t*)lds;
+  fa.init(lds0, lane);
+  const uint32_t sa = lds0 + 2 * TILE + 16 * lh;
   for (int pass = 0; pass < npass; ++pass) {
     const int kb = paired_block(nx, bx, pass, false);  // low key blocks see the most query tiles
     const int kw0 = kb * 128 + wave * 32, mykey = kw0 + lr;
+    // with a band the keys of tile kb are seen by the queries of tiles kb .. kb + nw - 1 only
+    const int nall = nx - kb, nt = 2 * (nw > 0 && nw < nall ? nw : nall), nh = 2 * nt;  // 64-query tiles, 32-query halves
+    // Half hh's share of the loads, five per wavefront: an odd half 2 i + 1 asks for Q and -lse / scale of tile i + 3 (whose stage tile
+    // i - 1 has left), the even half after it for that tile's dO and -delta. (All four wavefronts bring the 64 statistics.)
+    struct Part {
+      const uint8_t* p;
+      long st;
+      const float* s;
+      uint8_t* d;
+      uint8_t* ds;
+    };
+    auto part = [&](int tile, bool isq) {
+      const int tt = tile < nt ? tile : nt - 1;
+      const long r0 = (long)kb * 128 + (long)tt * 64;
+      uint8_t* d = lds + (tile & 3) * STAGE;
+      return Part{isq ? qp + r0 * qst : gp + r0 * gst, isq ? qst : gst, (isq ? nlp : delp) + r0, d + (isq ? 0 : TILE),
+                  d + 2 * TILE + (isq ? 0 : 256)};
+    };
+    auto load_one = [&](const Part& x, bool isq, int i) {
+      if (i < 4) (isq ? lq : lg).issue_one(i, x.p, x.st, x.d);
+      else __builtin_amdgcn_global_load_lds((glb_void_t*)(x.s + lane), (lds_void_t*)x.ds, 4, 0, 0);
+    };
+    auto load_part = [&](int tile, bool isq) {
+      const Part x = part(tile, isq);
+#pragma unroll
+      for (int i = 0; i < 5; ++i) load_one(x, isq, i);
+    };
+    load_part(0, true);
+    load_part(0, false);
+    load_part(1, true);
+    load_part(1, false);
+    load_part(2, true);
     bf16x8 kf[NKS], vf[NKS];
 #pragma unroll
     for (int s = 0; s < NKS; ++s) {
       kf[s] = *(const bf16x8*)(kp + (long)mykey * k.st + 16 * s + 8 * lh);
       vf[s] = *(const bf16x8*)(vp + (long)mykey * v.st + 16 * s + 8 * lh);
     }
-    // with a band the keys of tile kb are seen by the queries of tiles kb .. kb + nw - 1 only
-    const int nall = nx - kb, n = RPB * (nw > 0 && nw < nall ? nw : nall);
-    auto issue = [&](uint8_t* st, int i) {
-      const long r0 = (long)kb * 128 + (long)i * R;
-      lq.issue(qp + r0 * qst, qst, st);
-      lg.issue(gp + r0 * gst, gst, st + RT);
-      // the row statistics: R floats each, 4-byte loads (wavefront 0: -lse / scale, wavefront 1: -delta)
-      if (wave < 2) {
-        const float* src = (wave == 0 ? nlp : delp) + r0;
-#pragma unroll
-        for (int x = 0; x < R / 64; ++x)
-          __builtin_amdgcn_global_load_lds((glb_void_t*)(src + 64 * x + lane), (lds_void_t*)(st + 2 * RT + wave * 4 * R + 256 * x),
-                                           4, 0, 0);
-      }
-    };
     f32x16 dka[NDT], dva[NDT];
 #pragma unroll
     for (int i = 0; i < NDT; ++i)
@@ -470,79 +813,158 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : TFB_DKDV128_WPE) void attnD_dkdv
         dva[i][e] = 0.f;
       }
 
-    auto compute = [&](const uint8_t* st, int i) {
-      const uint8_t* qt_ = st;
-      const uint8_t* gt_ = st + RT;
-      const float* ls = (const float*)(st + 2 * RT);
-      const int qbase = kb * 128 + i * R;
-#pragma unroll
-      for (int qs = 0; qs < R / 32; ++qs) {
-        const int qlo = qbase + qs * 32;
-        if (qlo + 31 < kw0) continue;  // every key of this wavefront is in the future of these queries
-        // the accumulators start from the rows' -lse / scale and -delta
-        f32x16 S, dP;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const f32x4 L = *(const f32x4*)(ls + qs * 32 + 8 * j + 4 * lh);
-          const f32x4 Dl = *(const f32x4*)(ls + R + qs * 32 + 8 * j + 4 * lh);
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            S[4 * j + x] = L[x];
-            dP[4 * j + x] = Dl[x];
-          }
-        }
-#pragma unroll
-        for (int s = 0; s < NKS; ++s) S = mfma_bf16(frag_rows<D>(qt_, qs, s, lr, lh), kf[s], S);
-#pragma unroll
-        for (int s = 0; s < NKS; ++s) dP = mfma_bf16(frag_rows<D>(gt_, qs, s, lr, lh), vf[s], dP);
-        const int kq = mykey - (qlo + 4 * lh);  // key - q for element e is kq - (e>>2)*8 - (e&3)
-        if (kw0 + 31 > qlo) {
-#pragma unroll
-          for (int e = 0; e < 16; ++e) S[e] = (kq - 8 * (e >> 2) - (e & 3) > 0) ? -INFINITY : S[e];
-        }
-        uint32_t pw[8], dsw[8];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float p[4];
-#pragma unroll
-          for (int x = 0; x < 4; ++x) p[x] = fast_exp2(S[4 * j + x] * sl2);
-          const uint32_t w0 = pack2bf(p[0], p[1]), w1 = pack2bf(p[2], p[3]);
-          pw[2 * j] = w0;
-          pw[2 * j + 1] = w1;
-          dsw[2 * j] = pack2bf(bflo(w0) * dP[4 * j], bfhi(w0) * dP[4 * j + 1]);
-          dsw[2 * j + 1] = pack2bf(bflo(w1) * dP[4 * j + 2], bfhi(w1) * dP[4 * j + 3]);
-        }
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-          const bf16x8 pb = frag_from(pw[4 * ks], pw[4 * ks + 1], pw[4 * ks + 2], pw[4 * ks + 3]);
-          const bf16x8 db = frag_from(dsw[4 * ks], dsw[4 * ks + 1], dsw[4 * ks + 2], dsw[4 * ks + 3]);
-#pragma unroll
-          for (int dt = 0; dt < NDT; ++dt) {
-            dva[dt] = mfma_bf16(frag_cols<D>(gt_, dt, qs * 32 + 16 * ks, lane), pb, dva[dt]);
-            dka[dt] = mfma_bf16(frag_cols<D>(qt_, dt, qs * 32 + 16 * ks, lane), db, dka[dt]);
-          }
-        }
+    // Half h's dS, dV += dO P and dK += Q dS are made while half h + 1's S, dP and P are. Items in the order of their LDS reads:
+    // 0 .. 7 dV, 8 the start of S, 9 .. 16 S, 17 the start of dP, 18 .. 25 dP, 26 .. 33 dK.
+    f32x16 Sn, dP;
+    uint32_t pw[8], dsw[8];
+    float f0, f1;
+    RowFrag rf[16];
+    ColFrag cf[16];
+    StatFrag sf[2];
+    auto nlds = [](int i) constexpr { return i % 34 < 8 || i % 34 >= 26 ? 2 : i % 34 == 8 || i % 34 == 17 ? 4 : 1; };
+    auto after = [=](int i) constexpr {  // LDS instructions of the items asked for since
+      int c = 0;
+      for (int x = i + (i % 34 == 8 || i % 34 == 17 ? 1 : 2); x < i + AH; ++x) c += nlds(x);
+      return c;
+    };
+    // coff, roff: half h's and half h + 1's place, soff: half h + 1's statistics
+    auto request = [&](auto item, uint32_t coff, uint32_t roff, uint32_t soff) {
+      constexpr int i = decltype(item)::value;
+      if constexpr (i < 8) cf[i].template request<TILE + (i / NDT) * 16 * G::ROWB>(fa.lo[i % NDT] + coff, fa.hi[i % NDT] + coff);
+      else if constexpr (i == 8) sf[0].template request<0>(sa + soff);
+      else if constexpr (i < 17) rf[i - 9].template request<0>(fa.rows[i - 9] + roff);
+      else if constexpr (i == 17) sf[1].template request<256>(sa + soff);
+      else if constexpr (i < 26) rf[i - 10].template request<TILE>(fa.rows[i - 18] + roff);
+      else cf[i - 18].template request<((i - 26) / NDT) * 16 * G::ROWB>(fa.lo[(i - 26) % NDT] + coff, fa.hi[(i - 26) % NDT] + coff);
+    };
+    auto use = [&](auto item, auto aft) {
+      constexpr int i = decltype(item)::value, N = decltype(aft)::value;
+      if constexpr (i < 8) {
+        constexpr int w = 4 * (i / NDT);
+        if constexpr (i % 2 == 0) landed<N>(cf[i], cf[i + 1]);
+        const bf16x8 f = cf[i].get();
+        dva[i % NDT] = mfma_bf16(f, frag_from(pw[w], pw[w + 1], pw[w + 2], pw[w + 3]), dva[i % NDT]);
+      } else if constexpr (i == 8) {
+        sf[0].template landed<N>(Sn);
+      } else if constexpr (i < 17) {
+        if constexpr (i % 2 == 1) landed<N>(rf[i - 9], rf[i - 8]);
+        Sn = mfma_bf16(rf[i - 9].get(), kf[i - 9], Sn);
+      } else if constexpr (i == 17) {
+        sf[1].template landed<N>(dP);
+      } else if constexpr (i < 26) {
+        if constexpr (i % 2 == 0) landed<N>(rf[i - 10], rf[i - 9]);
+        dP = mfma_bf16(rf[i - 10].get(), vf[i - 18], dP);
+      } else {
+        constexpr int w = 4 * ((i - 26) / NDT);
+        if constexpr (i % 2 == 0) landed<N>(cf[i - 18], cf[i - 17]);
+        const bf16x8 f = cf[i - 18].get();
+        dka[(i - 26) % NDT] = mfma_bf16(f, frag_from(dsw[w], dsw[w + 1], dsw[w + 2], dsw[w + 3]), dka[(i - 26) % NDT]);
       }
     };
+    auto ds_word = [&](auto word) {  // the reference multiplies dP - delta by the rounded P
+      constexpr int w = decltype(word)::value;
+      dsw[w] = pack2bf(bflo(pw[w]) * dP[2 * w], bfhi(pw[w]) * dP[2 * w + 1]);
+      pin(dsw[w]);
+    };
+    auto step_f = [&](auto word) {
+      constexpr int w = decltype(word)::value;
+      f0 = Sn[2 * w] * sl2;
+      f1 = Sn[2 * w + 1] * sl2;
+      pin(f0, f1);
+    };
+    auto step_x = [&]() {
+      f0 = fast_exp2(f0);
+      f1 = fast_exp2(f1);
+      pin(f0, f1);
+    };
+    auto step_c = [&](auto word) {
+      pw[decltype(word)::value] = pack2bf(f0, f1);
+      pin(pw[decltype(word)::value]);
+    };
+    auto place = [](int hh) -> uint32_t { return ((hh >> 1) & 3) * STAGE + (hh & 1) * (TILE / 2); };
+    auto splace = [](int hh) -> uint32_t { return ((hh >> 1) & 3) * STAGE + (hh & 1) * 128; };
 
-    issue(st0, 0);
-    wait_all_loads();
-    __syncthreads();
-    for (int t = 0; t + 2 <= n; t += 2) {
-      issue(st1, t + 1);
-      compute(st0, t);
-      __syncthreads();
-      if (t + 2 < n) issue(st0, t + 2);
-      compute(st1, t + 1);
-      __syncthreads();
+    // tiles 0 and 1; then the halves before this wavefront's first, which is the one on its diagonal
+    asm volatile("s_waitcnt vmcnt(5)\n\ts_barrier" ::: "memory");
+    for (int x = 0; x < wave; ++x) {
+      if (x & 1) asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory");
+      load_part((x >> 1) + ((x & 1) ? 3 : 2), x & 1);
     }
-    if (n & 1) compute(st0, n - 1);
-    __syncthreads();  // the stages are free for the partner block
+    {
+      const uint32_t roff = place(wave), soff = splace(wave);
+      slots<8, 8 + AH>([&](auto i) { request(i, 0u, roff, soff); });
+      slots<8, 26>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        auto aft = [=]() constexpr {
+          int c = 0;
+          for (int y = x + (x == 8 || x == 17 ? 1 : 2); y < x + AH && y < 26; ++y) c += nlds(y);
+          return c;
+        };
+        use(i, std::integral_constant<int, aft()>{});
+        if constexpr (x + AH < 26) request(std::integral_constant<int, x + AH>{}, 0u, roff, soff);
+        slot_end();
+      });
+      const int kq = lr - 4 * lh;  // key - q for element e is kq - (e>>2)*8 - (e&3)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) Sn[e] = (kq - 8 * (e >> 2) - (e & 3) > 0) ? -INFINITY : Sn[e];
+      slots<0, 8>([&](auto i) {
+        step_f(i);
+        step_x();
+        step_c(i);
+      });
+    }
+    slots<0, AH>([&](auto i) { request(i, place(wave), 0u, 0u); });
+    static_assert(AH <= 8, "only columns of the first half are asked for here");
+    for (int hh = wave; hh + 1 < nh; ++hh) {
+      const bool isq = hh & 1;
+      // tile (hh + 1) / 2 is needed from here on: all but the ten newest loads have landed
+      if (isq) asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory");
+      const Part ld = part((hh >> 1) + (isq ? 3 : 2), isq);
+      const uint32_t coff = place(hh), roff = place(hh + 1), soff = splace(hh + 1);
+      slot_end();
+#pragma unroll
+      for (int i = 0; i < NDT; ++i) asm volatile("" : "+a"(dka[i]), "+a"(dva[i]));
+      slots<0, NI>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        use(i, std::integral_constant<int, after(x)>{});
+        if constexpr (x + AH < NI) request(std::integral_constant<int, x + AH>{}, coff, roff, soff);
+        else request(std::integral_constant<int, x + AH - NI>{}, roff, 0u, 0u);
+        if constexpr (x % 4 == 1 && x / 4 < 5) load_one(ld, isq, x / 4);
+        if constexpr (x < 16 && x % 2 == 0) ds_word(std::integral_constant<int, x / 2>{});
+        if constexpr (x == 18) step_f(std::integral_constant<int, 0>{});
+        if constexpr (x >= 19 && x % 2 == 1) step_x();
+        if constexpr (x >= 20 && x % 2 == 0) {
+          step_c(std::integral_constant<int, (x - 20) / 2>{});
+          step_f(std::integral_constant<int, (x - 18) / 2>{});
+        }
+        slot_end();
+      });
+      step_c(std::integral_constant<int, 7>{});
+    }
+    {  // the last half
+      const uint32_t coff = place(nh - 1);
+      slots<0, 8>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        use(i, std::integral_constant<int, 2 * (AH - 2)>{});
+        if constexpr (x + AH < 8) request(std::integral_constant<int, x + AH>{}, coff, 0u, 0u);
+        else request(std::integral_constant<int, x + AH + 18>{}, coff, 0u, 0u);
+        ds_word(i);
+        slot_end();
+      });
+      slots<26, NI>([&](auto i) {
+        constexpr int x = decltype(i)::value;
+        use(i, std::integral_constant<int, x % 2 ? 0 : 2 * (x + AH <= NI ? AH - 2 : NI - 2 - x)>{});
+        if constexpr (x + AH < NI) request(std::integral_constant<int, x + AH>{}, coff, 0u, 0u);
+        slot_end();
+      });
+    }
 
     bf16_t* dkp = dk.p + b * dk.sb + h * dk.sh + (long)mykey * dk.st;
     bf16_t* dvp = dv.p + b * dv.sb + h * dv.sh + (long)mykey * dv.st;
     store_grad_row<D>(dka, scale, dkp, lh);
     store_grad_row<D>(dva, 1.0f, dvp, lh);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (pass + 1 < npass) __syncthreads();  // the stages are free for the partner block
   }
 }
 
@@ -564,7 +986,7 @@ int bwd_launch(const void* q, const long* qs, const void* k, const long* ks, con
   hipLaunchKernelGGL(attnD_dq_kernel<D>, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
                      mk(go, gos), mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, nw, mk(o, os), lse);
   TFB_LAUNCH_CHECK();
-  hipLaunchKernelGGL((attnD_dkdv_kernel<D, TFB_DKDV128_R>), dim3(paired_grid(T / 128, B * H, D == 64 ? 2 : TFB_DKDV128_WPE), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
+  hipLaunchKernelGGL(attnD_dkdv_kernel<D>, dim3(paired_grid(T / 128, B * H, 1), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
                      mk(go, gos), mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale, scale * LOG2E, nw);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
