@@ -1026,6 +1026,21 @@ def test_attention_head_dim_128_pipelined_over_few_tiles(ops, dev, B, H, T, nw):
         assert rel_l2(got[sl], w) < BF16_TOL
 
 
+@pytest.mark.parametrize("D,H,T,nw", [(64, 2, 256, 0), (64, 12, 2048, 0), (64, 5, 512, 2), (128, 2, 256, 0), (128, 8, 1024, 0)])
+def test_attention_of_a_few_heads_equals_theirs_in_a_large_launch(ops, dev, D, H, T, nw):
+    """A launch that does not fill the chip runs one query (key) block per workgroup, a large one two: the same bits either way."""
+    g, B, kw = _g(D + H + T), 512 * 128 * 4 // (H * T), {"band": nw} if nw else {}
+    q, k, v = (torch.randn(1, H, T, D, generator=g).bfloat16().to(dev) for _ in range(3))
+    do = torch.randn(1, T, H, D, generator=g).bfloat16().to(dev)
+    outs = []
+    for n in (1, B):
+        Q, K, V = (x.expand(n, -1, -1, -1).contiguous() for x in (q, k, v))
+        G = do.expand(n, -1, -1, -1).contiguous()
+        o, lse = ops.attn_fwd(Q, K, V, D ** -0.5, **kw)
+        outs.append([x[-1] for x in (o, lse, *ops.attn_bwd(Q, K, V, o, G, lse, D ** -0.5, **kw))])
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+
+
 # ------------------------------------------------------------------------------------------ loss head
 @pytest.mark.parametrize("cap", [15.0, None])
 def test_loss_fwd_bwd(ops, dev, cap):

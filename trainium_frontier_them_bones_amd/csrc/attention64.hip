@@ -80,16 +80,34 @@ __device__ __forceinline__ bf16x8 frag_from(uint32_t a, uint32_t b, uint32_t c, 
   return __builtin_bit_cast(bf16x8, v);
 }
 __device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // s_waitcnt vmcnt(0)
+__device__ __forceinline__ float max_halves(float x) {  // the larger of the two lanes' that share a query
+  float y = x;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y));
+  return fmaxf(x, y);
+}
+// A stage's barrier: the loads into LDS that this wavefront has in flight are part of what the others read behind it (the compiler
+// may leave their wait to the first read of its own).
+__device__ __forceinline__ void stage_barrier() {
+  wait_all_loads();
+  __syncthreads();
+}
 
-// Workgroup -> (block along the sequence, batch*head): consecutive workgroup ids are dealt round-robin to the 8 XCDs,
-// each with its own L2, so the ids are re-dealt to keep all sequence blocks of one (batch, head) - which stream the same
-// K/V (or Q/dO) tiles - on one XCD. nx = blocks per (batch, head), nbh = batch*head count.
+// Workgroup -> (block along the sequence, batch*head): consecutive workgroup ids are dealt round-robin to the 8 XCDs, each with its own
+// L2, so the ids are re-dealt to keep all sequence blocks of one (batch, head) - which stream the same K/V (or Q/dO) tiles - on one
+// XCD; with one block per workgroup (gridDim.x = nx) in slot-major order, the heaviest block of each pair first. nx = blocks per
+// (batch, head), nbh = batch*head count.
 __device__ __forceinline__ void xcd_block(int nx, int nbh, int& bx, int& bh) {
-  const int lin = blockIdx.y * nx + blockIdx.x;
+  const int gx = gridDim.x, lin = blockIdx.y * gx + blockIdx.x;
   if (nbh % 8 == 0) {
     const int xcd = lin & 7, idx = lin >> 3;
-    bh = xcd + 8 * (idx / nx);
-    bx = idx % nx;
+    if (gx == nx) {
+      const int per = nbh >> 3;
+      bx = idx / per;
+      bh = xcd + 8 * (idx % per);
+    } else {
+      bh = xcd + 8 * (idx / gx);
+      bx = idx % gx;
+    }
   } else {
     bh = blockIdx.y;
     bx = blockIdx.x;
@@ -110,7 +128,13 @@ __device__ __forceinline__ int paired_block(int nx, int bx, int pass, bool heavy
 // First 64-key tile a 128-token query tile qb sees under a band of nw key tiles (a query of tile i sees the keys k <= q
 // of tiles i - nw + 1 .. i: band_mask, round2/source/kernels/nki_attn_bandpro.py:1654); 0 without a band (nw <= 0).
 __device__ __forceinline__ int band_first_tile(int qb, int nw) { return nw > 0 && qb - nw + 1 > 0 ? 2 * (qb - nw + 1) : 0; }
-__host__ inline unsigned paired_grid(int nx) { return (unsigned)(nx % 2 == 0 ? nx / 2 : nx); }
+// Blocks are paired when the paired grid fills its rounds of resident workgroups to 90 % (or is long enough not to care); otherwise
+// one block per workgroup, the heaviest first (B8 H8 T512 forward 14.3 -> 10.8 us, backward 43 -> 33; B1 H12 T2048 31 -> 27, 89 -> 80).
+__host__ inline unsigned paired_grid(int nx, int nbh, int per_cu) {
+  if (nx % 2) return (unsigned)nx;
+  const long wgs = (long)(nx / 2) * nbh, slots = tfb_resident_slots(per_cu), rounds = (wgs + slots - 1) / slots;
+  return (unsigned)(wgs * 10 >= rounds * slots * 9 ? nx / 2 : nx);
+}
 
 __device__ __forceinline__ int swz(int t) { return (((t >> 1) & 1) << 2) | ((t >> 2) & 3); }
 
@@ -209,7 +233,7 @@ __global__ __launch_bounds__(256, TFB_FWD64_WPE) void attn64_fwd_kernel(AttnT q,
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   stagger_start(slots);
   int bx, bh;
-  xcd_block(gridDim.x, gridDim.y, bx, bh);
+  xcd_block(T / 128, gridDim.y, bx, bh);
   const int b = bh / H, h = bh % H;
   const bf16_t* qp = q.p + b * q.sb + h * q.sh;
   const uint8_t* kp = (const uint8_t*)(k.p + b * k.sb + h * k.sh);
@@ -273,7 +297,7 @@ __global__ __launch_bounds__(256, TFB_FWD64_WPE) void attn64_fwd_kernel(AttnT q,
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int e = 0; e < 16; e += 2) mx = fmaxf(fmaxf(mx, sc[kt][e]), sc[kt][e + 1]);
-    return fmaxf(mx, __shfl_xor(mx, 32, 64));
+    return max_halves(mx);
   };
   // (4) The reference point m of the exponentials only has to keep them in range: it follows the running maximum when
   // some row's maximum has grown by more than 2^8 (always on a row's first tile, m = -1e30), which after the first few
@@ -348,7 +372,7 @@ __global__ __launch_bounds__(256, TFB_FWD64_WPE) void attn64_fwd_kernel(AttnT q,
     interleave(std::integral_constant<int, 3>{});
     follow_max(mx);
     load_vT(cur, pva);
-    __syncthreads();  // tile t + 1 has landed; every wavefront has its fragments of tile t
+    stage_barrier();  // tile t + 1 has landed; every wavefront has its fragments of tile t
     issue(cur, t + 2);
     scores(nxt, scN);
     softmax(scC, ppw);
@@ -379,8 +403,7 @@ __global__ __launch_bounds__(256, TFB_FWD64_WPE) void attn64_fwd_kernel(AttnT q,
   const int n = (q0 + 128) / 64;  // even; tiles n - 2 and n - 1 cover the workgroup's own 128 tokens
   const int t0 = band_first_tile(qb, nw);  // even; 0 without a band
   issue(st0, t0);
-  wait_all_loads();
-  __syncthreads();
+  stage_barrier();
   issue(st1, t0 + 1);
   scores(st0, scA);
   for (int t = t0; t + 2 < n; t += 2) {
@@ -389,7 +412,7 @@ __global__ __launch_bounds__(256, TFB_FWD64_WPE) void attn64_fwd_kernel(AttnT q,
   }
   accumulate(pva, ppw);  // the last full tile's product (zeros when there was none)
   diagonal_tile(st0, n - 2, scA);
-  __syncthreads();
+  stage_barrier();
   scores(st1, scB);
   diagonal_tile(st1, n - 1, scB);
 
@@ -458,7 +481,7 @@ __global__ __launch_bounds__(256, 2) void attn64_dkdv_kernel(AttnT q, AttnT k, A
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   stagger_start(slots);
   int bx, bh;
-  xcd_block(gridDim.x, gridDim.y, bx, bh);
+  xcd_block(T / 128, gridDim.y, bx, bh);
   const int b = bh / H, h = bh % H;
   const uint8_t* qp = (const uint8_t*)(q.p + b * q.sb + h * q.sh);
   const uint8_t* gp = (const uint8_t*)(go.p + b * go.sb + h * go.sh);
@@ -669,33 +692,32 @@ __global__ __launch_bounds__(256, 2) void attn64_dkdv_kernel(AttnT q, AttnT k, A
   };
 
   issue(st0, 0);
-  wait_all_loads();
-  __syncthreads();
+  stage_barrier();
   if (!TFB_DKDV64_PIPE) {
     for (int t = 0; t + 2 <= n; t += 2) {
       issue(st1, t + 1);
       compute(st0, t);
-      __syncthreads();
+      stage_barrier();
       issue(st0, t + 2 < n ? t + 2 : n - 1);
       compute(st1, t + 1);
-      __syncthreads();
+      stage_barrier();
     }
     if (n & 1) compute(st0, n - 1);
   } else {
     if (n > 1) issue(st1, 1);
     compute(st0, 0);  // the diagonal stage: blocks in a wavefront's past skipped, its own block masked
     if (n > 1) {
-      __syncthreads();
+      stage_barrier();
       issue(st0, 2 < n ? 2 : n - 1);
       full_stage(st1);
-      __syncthreads();
+      stage_barrier();
       for (int t = 2; t + 2 <= n; t += 2) {
         issue(st1, t + 1);
         full_stage(st0);
-        __syncthreads();
+        stage_barrier();
         issue(st0, t + 2 < n ? t + 2 : n - 1);
         full_stage(st1);
-        __syncthreads();
+        stage_barrier();
       }
       if (n & 1) full_stage(st0);
     }
@@ -721,7 +743,7 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   stagger_start(slots);
   int bx, bh;
-  xcd_block(gridDim.x, gridDim.y, bx, bh);
+  xcd_block(T / 128, gridDim.y, bx, bh);
   const int b = bh / H, h = bh % H;
   const bf16_t* qp = q.p + b * q.sb + h * q.sh;
   const bf16_t* gp = go.p + b * go.sb + h * go.sh;
@@ -852,7 +874,7 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
     accumulate(kTa, dsa);
     __builtin_amdgcn_sched_barrier(0);  // the second block's fragments are not requested while the first's are live
     load_kT(cur, 1, kTb);
-    __syncthreads();  // tile t + 1 has landed; every wavefront has its fragments of tile t
+    stage_barrier();  // tile t + 1 has landed; every wavefront has its fragments of tile t
     issue(cur, t + 2);
     scores(nxt, 0, Sa, dPa);
     softmax_ds(Sb, dPb, dsb, -1);
@@ -878,8 +900,7 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
   const int n = (q0 + 128) / 64;  // even; tiles n - 2 and n - 1 cover the workgroup's own 128 tokens
   const int t0 = band_first_tile(qb, nw);  // even; 0 without a band
   issue(st0, t0);
-  wait_all_loads();
-  __syncthreads();
+  stage_barrier();
   issue(st1, t0 + 1);
   scores(st0, 0, Sa, dPa);
   for (int t = t0; t + 2 < n; t += 2) {
@@ -887,7 +908,7 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
     full_tile(st1, st0, t + 1);
   }
   diagonal_tile(st0, n - 2, true);
-  __syncthreads();
+  stage_barrier();
   diagonal_tile(st1, n - 1, false);
 
   bf16_t* dqp = dq.p + b * dq.sb + h * dq.sh + (long)myq * dq.st;
@@ -907,7 +928,7 @@ AttnT mk(const void* p, const long* s) { return AttnT{(bf16_t*)p, s[0], s[1], s[
 // Called by tfb_attn_fwd / tfb_attn_bwd for D = 64 (arguments already validated there: T % 128 == 0, strides % 8 == 0).
 int tfb_attn64_fwd_impl(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, void* o,
                         const long* os, float* lse, int B, int H, int T, float scale, int nw, hipStream_t s) {
-  hipLaunchKernelGGL(attn64_fwd_kernel, dim3(paired_grid(T / 128), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(o, os), lse,
+  hipLaunchKernelGGL(attn64_fwd_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(o, os), lse,
                      T, H, scale * LOG2E, nw, tfb_resident_slots(2));
   TFB_LAUNCH_CHECK();
   return TFB_OK;
@@ -927,11 +948,11 @@ int tfb_attn64_bwd_impl(const void* q, const long* qs, const void* k, const long
                        stats, T, H, rows, 1.0f / scale);
     TFB_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(attn64_dq_kernel, dim3(paired_grid(T / 128), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
+  hipLaunchKernelGGL(attn64_dq_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
                      mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw,
                      tfb_resident_slots(2), mk(o, os), lse);
   TFB_LAUNCH_CHECK();
-  hipLaunchKernelGGL(attn64_dkdv_kernel, dim3(paired_grid(T / 128), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
+  hipLaunchKernelGGL(attn64_dkdv_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
                      mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw, tfb_resident_slots(2));
   TFB_LAUNCH_CHECK();
   return TFB_OK;
