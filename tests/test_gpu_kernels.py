@@ -1235,6 +1235,18 @@ def test_newton_schulz_stack(ops, dev, shape):
     assert rel_l2(v, y.float().square().sum(dim=-1 if r >= c else -2)) < 1e-6        # v is the row statistic of the y returned
 
 
+@pytest.mark.parametrize("K,M,N", [(14, 768, 768), (9, 1152, 1152), (60, 256, 256), (300, 128, 128), (7, 1280, 640)])
+def test_newton_schulz_of_a_stack_equals_that_of_its_matrices(ops, dev, K, M, N):
+    """The symmetric products take 64 x 64 tiles on a small stack and 128 x 128 on a large one, one tile of each diagonal pair stored
+    twice, a matrix's tiles in one run of workgroups: every matrix comes out as it does alone, bit for bit."""
+    g = torch.randn(K, M, N, generator=_g(K + M + N)).to(dev)
+    d = g.flatten(1).norm(dim=1) * 1.02
+    y, v = ops.ns5(g, d)
+    for i in (0, K // 2, K - 1):
+        yi, vi = ops.ns5(g[i:i + 1].contiguous(), d[i:i + 1].contiguous())
+        assert torch.equal(y[i], yi[0]) and torch.equal(v[i], vi[0])
+
+
 def test_newton_schulz_full_size_properties(ops, dev):
     """The 12 MLP matrices of the benchmark model in one call (K 12, 3072 x 768): singular values inside the Polar Express
     band, the same singular vectors as the input (cosine with the SVD polar factor), and the wide stack equal to the

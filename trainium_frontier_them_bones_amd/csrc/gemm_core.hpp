@@ -82,6 +82,7 @@ struct GemmArgs {
   FastDiv d_ntiles, d_per, d_nfast, d_blk, d_gblock, d_splits, d_split8;  // d_split8: by splits / 8
   int q_off;    // ring kernel: what the epilogue adds to its row numbers (a launch over the last rows of a larger one)
   int ranges;   // ring kernel: k ranges summed separately inside one workgroup, then added in order (see there)
+  long g_stride;  // ring kernel, symmetric products: both operands of group g start g_stride bytes * g further
   FastDiv d_ranges;
 };
 

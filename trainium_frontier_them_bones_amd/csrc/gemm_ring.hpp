@@ -23,6 +23,14 @@ struct has_ranges : std::false_type {};
 template <class T>
 struct has_ranges<T, std::void_t<decltype(T::kRanges)>> : std::true_type {};
 
+// Epilogues of products that are symmetric bit for bit (D[p][q] = D[q][p]: the same operand on both sides, the contraction in the same
+// order) declare  static constexpr bool kSymmetric : the launch is one workgroup per tile on and above the diagonal, and a tile above it
+// is stored a second time, transposed through LDS. They give  u32x4 value(v [, pre_t])  (eight rounded outputs),  out  and  ld.
+template <class T, class = void>
+struct is_symmetric : std::false_type {};
+template <class T>
+struct is_symmetric<T, std::void_t<decltype(T::kSymmetric)>> : std::true_type {};
+
 template <int BP_, int BQ_, int WP_, int WQ_, int ES_, int LAYP_, int LAYQ_, int FMTP_, int FMTQ_, int NS_>
 struct RingCfg {
   static constexpr int BP = BP_, BQ = BQ_, WP = WP_, WQ = WQ_, ES = ES_, NS = NS_;
@@ -152,7 +160,13 @@ struct RingFrags<ROWS, NTILE, ES, TFB_K_STRIDED> {
 };
 
 // The MFMAs that made x stay in front of this point (they have no side effects, and would otherwise sink across barriers).
-__device__ __forceinline__ void ring_pin(f32x16& x) { asm volatile("" : "+v"(x)); }
+// AGPR: with one workgroup per CU the compiler keeps accumulators in that half of the register file (pinned in the other they were
+// moved there and back, 128 moves per k-tile).
+template <bool AGPR>
+__device__ __forceinline__ void ring_pin(f32x16& x) {
+  if constexpr (AGPR) asm volatile("" : "+a"(x));
+  else asm volatile("" : "+v"(x));
+}
 
 // s_waitcnt vmcnt(tiles * PER): all but the newest `tiles` k-tiles of loads have landed (tiles is wavefront-uniform)
 template <int PER>
@@ -174,7 +188,21 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
   const int wp = wave % Cfg::WP, wq = wave / Cfg::WP;
   const int lr = lane & 31, lh = lane >> 5;
   int lid, split, tile_p, tile_q;
-  gemm_tile_of(a, blockIdx.x, lid, split, tile_p, tile_q);
+  [[maybe_unused]] int sym_group = 0;
+  if constexpr (is_symmetric<Epi>::value) {
+    static_assert(BP == BQ, "square tiles");
+    // an XCD's workgroups (id & 7) take a run of consecutive tiles, so that a group's operand is read into one or two L2s only
+    lid = (blockIdx.x & 7) * a.per + (blockIdx.x >> 3);
+    split = 0;
+    sym_group = fastdiv(lid, a.d_ntiles);
+    if (sym_group >= a.rows) return;   // (the whole workgroup: the runs are of equal length)
+    tile_p = lid - sym_group * a.ntiles;
+    tile_q = 0;
+    for (; tile_p >= a.ntp - tile_q; ++tile_q) tile_p -= a.ntp - tile_q;   // row tile_q has ntp - tile_q tiles
+    tile_p += tile_q;
+  } else {
+    gemm_tile_of(a, blockIdx.x, lid, split, tile_p, tile_q);
+  }
   const long p0 = (long)tile_p * BP, q0 = (long)tile_q * BQ;
   int kt0 = 0;
   if (a.splits > 1) {
@@ -188,10 +216,15 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
     a.P.base += (long)group * a.p_group_stride;
   }
   if (a.k_seg) {
-    group = blockIdx.y;
+    group = is_symmetric<Epi>::value ? sym_group : (int)blockIdx.y;
     const int k0 = a.k_seg[group], k1 = a.k_seg[group + 1];
     kt0 = k0 * ES / 128;
     a.nkt = (k1 - k0) * ES / 128;  // may be 0: the accumulators stay zero and are still written
+  }
+  if constexpr (is_symmetric<Epi>::value) {
+    group = sym_group;
+    a.P.base += group * a.g_stride;
+    a.Q.base += group * a.g_stride;
   }
   const int nkt = a.nkt;
 
@@ -302,7 +335,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
 #pragma unroll
     for (int i = 0; i < TP; ++i)
 #pragma unroll
-      for (int j = 0; j < TQ; ++j) ring_pin(acc[i][j]);
+      for (int j = 0; j < TQ; ++j) ring_pin<(Cfg::LDS_BYTES > 80 * 1024)>(acc[i][j]);
   };
 
   if (nkt > 0) {
@@ -341,6 +374,9 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
     // 32 output rows at a time through the wavefront's own LDS slice, then 8-element chunks, a row's on consecutive lanes
     constexpr int SLD = Cfg::STAGE_LD;
     float* stg = (float*)lds + wave * (32 * SLD);
+    constexpr int MLD = 40;   // (80-byte rows: 16-byte aligned, and a lane's column of eight on different banks)
+    static_assert(!is_symmetric<Epi>::value || Cfg::EPI_BYTES + NW * TP * 32 * MLD * 2 <= Cfg::LDS_BYTES, "mirror slices");
+    [[maybe_unused]] bf16_t* mirror = (bf16_t*)(lds + Cfg::EPI_BYTES) + wave * (TP * 32 * MLD);
 #pragma unroll
     for (int j = 0; j < TQ; ++j) {
 #pragma unroll
@@ -357,7 +393,16 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
         const int p = (int)p0 + pw + pc, q = a.q_off + (int)q0 + qw + j * 32 + row;
         const f32x4 lo = *(const f32x4*)(stg + row * SLD + pc), hi = *(const f32x4*)(stg + row * SLD + pc + 4);
         const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        if constexpr (has_partner32<Epi>::value) {
+        if constexpr (is_symmetric<Epi>::value) {
+          u32x4 w;
+          if constexpr (kPrefetch) w = epi.value(v, pre[j][k]);
+          else w = epi.value(v);
+          *(u32x4*)(epi.out + (long)q * epi.ld + p) = w;
+          if (tile_p != tile_q) {
+#pragma unroll
+            for (int x = 0; x < 8; ++x) mirror[(pc + x) * MLD + row] = (bf16_t)(x & 1 ? w[x >> 1] >> 16 : w[x >> 1]);
+          }
+        } else if constexpr (has_partner32<Epi>::value) {
           static_assert(TP == 2, "partner epilogue: 64 staged columns per wavefront");
           const f32x4 plo = *(const f32x4*)(stg + row * SLD + (pc ^ 32)), phi = *(const f32x4*)(stg + row * SLD + (pc ^ 32) + 4);
           const float vp[8] = {plo[0], plo[1], plo[2], plo[3], phi[0], phi[1], phi[2], phi[3]};
@@ -370,6 +415,16 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
         }
       }
       __builtin_amdgcn_wave_barrier();
+      if constexpr (is_symmetric<Epi>::value) {
+        if (tile_p != tile_q) {   // the 32 rows q of this pass as 64-byte pieces of the rows p
+#pragma unroll
+          for (int k = 0; k < NK; ++k) {
+            const int c = lane + 64 * k, row = c >> 2, qc = (c & 3) * 8;
+            *(u32x4*)(epi.out + ((long)p0 + pw + row) * epi.ld + q0 + qw + j * 32 + qc) = *(const u32x4*)(mirror + row * MLD + qc);
+          }
+          __builtin_amdgcn_wave_barrier();
+        }
+      }
     }
   }
 }
@@ -412,6 +467,39 @@ static inline int gemm_ring_pick(long np, long nq, long nkt, bool strided, long 
   const long cus = tfb_resident_slots(1), t64 = (np / 64) * (nq / 64) * groups;
   if (t64 <= cus) return 1;
   return 2 * t64 <= (strided ? 9 : 8) * cus ? 2 : 0;
+}
+
+// A stack of `groups` symmetric N x N products of one operand with itself (N a multiple of 128): 64 x 64 tiles while no CU has more
+// than two, else 128 x 128 with four stages (half the bytes per output, one workgroup per CU). What bounds them is a k-tile's trip
+// through one wavefront per SIMD and the operand's way into eight L2s, which the runs of tiles cut to one or two. The five iterations
+// of Muon with both symmetric products full -> this: 12 x 3072 x 768 810 -> 625 us, 12 x 2048 x 512 354 -> 251, 6 x 2304 x 768 369 -> 293.
+template <class Epi, int ES, int LAY>
+static int gemm_ring_symmetric(GemmOperand X, long g_stride, const int* k_seg, int N, int nkt, int groups, Epi e, hipStream_t s) {
+  GemmArgs a = {};
+  a.P = X;
+  a.Q = X;
+  a.np = N;
+  a.nq = N;
+  a.nkt = nkt;
+  a.k_seg = k_seg;
+  a.g_stride = g_stride;
+  const long n64 = N / 64, cus = tfb_resident_slots(1);
+  const bool small = n64 * (n64 + 1) / 2 * groups <= 2 * cus;
+  a.ntp = small ? N / 64 : N / 128;
+  using C64 = RingCfg<64, 64, 2, 2, ES, LAY, LAY, 0, 0, 4>;
+  using C128 = RingCfg<128, 128, 2, 2, ES, LAY, LAY, 0, 0, 4>;
+  const int st = small ? gemm_map_args<C64>(a, 1) : gemm_map_args<C128>(a, 1);
+  if (st != TFB_OK) return st;
+  a.ntiles = a.ntp * (a.ntp + 1) / 2;
+  a.d_ntiles = fastdiv_make(a.ntiles);
+  a.rows = groups;
+  if ((long)a.ntiles * groups > 0x7ffffff0L / 8) return TFB_ERR_SHAPE;
+  a.per = (a.ntiles * groups + 7) / 8;
+  const dim3 grid(8 * a.per);
+  if (small) hipLaunchKernelGGL((gemm_ring_kernel<C64, false, Epi>), grid, dim3(256), 0, s, a, e);
+  else hipLaunchKernelGGL((gemm_ring_kernel<C128, false, Epi>), grid, dim3(256), 0, s, a, e);
+  TFB_LAUNCH_CHECK();
+  return TFB_OK;
 }
 
 template <class Epi, int ES, int LAYP, int LAYQ, int FMTP, int FMTQ>

@@ -10,13 +10,24 @@
 // with the five (a, b, c) of the caller, then v[m] = sum_n X5[m][n]^2 in fp32 from the bf16 X5.
 //
 // The whole stack runs in three grouped GEMM launches per iteration (not three per matrix): the matrices are stacked
-// along the rows, G's contraction is segmented per matrix (k_seg), and the two products against the per-matrix [N][N]
-// operand pick it by the row tile's matrix (q_group). G and G G are symmetric bit for bit (the same products summed in
-// the same order on either side of the diagonal), so B^T = B and both products run in the k-contiguous "x @ w^T" form
-// with the [N][N] matrix as the weight; the reference's mirror fill of the lower blocks is therefore not needed.
+// along the rows, G's contraction is segmented per matrix (k_seg), and X B picks the [N][N] operand by the row tile's matrix
+// (q_group). G and G G are symmetric bit for bit (the same products summed in the same order on either side of the
+// diagonal): their tiles on and above the diagonal are computed, those above it stored a second time transposed, and with
+// B^T = B both products run in the k-contiguous "x @ w^T" form with the [N][N] matrix as the weight.
 #include "gemm_ring.hpp"
 
 namespace {
+
+__device__ __forceinline__ u32x4 axpby8(const float (&v)[8], const u32x4& zv, float alpha, float beta) {
+  float zf[8], r[8];
+  unpack8bf(zv, zf);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float t1 = v[k] * alpha, t2 = beta * zf[k];
+    r[k] = t1 + t2;
+  }
+  return pack8bf(r);
+}
 
 // out = bf16(fp32(alpha * D) + fp32(beta * z)), z and out [rows][ld] bf16; the z chunk is requested before the k-loop
 struct EpiAxpby {
@@ -27,22 +38,36 @@ struct EpiAxpby {
   using pre_t = u32x4;
   __device__ __forceinline__ pre_t prefetch(int p, int q) const { return *(const u32x4*)(z + (long)q * ld + p); }
   __device__ __forceinline__ void operator()(int p, int q, const float (&v)[8], const pre_t& zv, int) const {
-    float zf[8], r[8];
-    unpack8bf(zv, zf);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const float t1 = v[k] * alpha, t2 = beta * zf[k];
-      r[k] = t1 + t2;
-    }
-    *(u32x4*)(out + (long)q * ld + p) = pack8bf(r);
+    *(u32x4*)(out + (long)q * ld + p) = axpby8(v, zv, alpha, beta);
   }
 };
 
-// k_seg[i] = i * M (i <= K); gq[t] = t / (N / 128) for the K N / 128 row tiles of the stacked G; xq[t] = t / (M / 128)
-__global__ void ns_tables_kernel(int* k_seg, int* gq, int* xq, int K, int M, int N) {
+// A symmetric product of the stack, bf16 [K][N][N]: out = bf16(D), or bf16(fp32(alpha D) + fp32(beta z))
+struct EpiSym {
+  static constexpr bool kSymmetric = true;
+  bf16_t* out;
+  long ld, slab;
+  __device__ __forceinline__ EpiSym for_group(int g) const { return EpiSym{out + g * slab, ld, slab}; }
+  __device__ __forceinline__ u32x4 value(const float (&v)[8]) const { return pack8bf(v); }
+};
+struct EpiSymAxpby {
+  static constexpr bool kSymmetric = true;
+  bf16_t* out;
+  const bf16_t* z;
+  long ld, slab;
+  float alpha, beta;
+  using pre_t = u32x4;
+  __device__ __forceinline__ EpiSymAxpby for_group(int g) const { return EpiSymAxpby{out + g * slab, z + g * slab, ld, slab, alpha, beta}; }
+  __device__ __forceinline__ pre_t prefetch(int p, int q) const { return *(const u32x4*)(z + (long)q * ld + p); }
+  __device__ __forceinline__ u32x4 value(const float (&v)[8], const pre_t& zv) const {
+    return axpby8(v, zv, alpha, beta);
+  }
+};
+
+// k_seg[i] = i * M (i <= K); xq[t] = t / (M / 128) for the K M / 128 row tiles of the stacked X
+__global__ void ns_tables_kernel(int* k_seg, int* xq, int K, int M) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i <= K) k_seg[i] = i * M;
-  if (i < K * (N / 128)) gq[i] = i / (N / 128);
   if (i < K * (M / 128)) xq[i] = i / (M / 128);
 }
 
@@ -117,7 +142,7 @@ inline long align256(long b) { return (b + 255) & ~255L; }
 extern "C" long tfb_ns5_workspace_bytes(int K, int M, int N) {
   if (K <= 0 || M <= 0 || N <= 0) return 0;
   const long xb = align256((long)K * M * N * 2), gb = align256((long)K * N * N * 2);
-  return 2 * xb + 2 * gb + align256(((long)K + 1 + (long)K * (N / 128) + (long)K * (M / 128)) * 4);
+  return 2 * xb + 2 * gb + align256(((long)K + 1 + (long)K * (M / 128)) * 4);
 }
 
 // g: fp32 [K][M][N] (wide = 0) or [K][N][M] (wide = 1: each matrix is handled as its transpose), M >= N; inv_d: fp32 [K]
@@ -137,11 +162,10 @@ extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, vo
   bf16_t* G = (bf16_t*)(w + 2 * xb);
   bf16_t* Bm = (bf16_t*)(w + 2 * xb + gb);
   int* k_seg = (int*)(w + 2 * xb + 2 * gb);
-  int* gq = k_seg + K + 1;
-  int* xq = gq + (long)K * (N / 128);
+  int* xq = k_seg + K + 1;
 
   const int ntab = K * (M / 128) + 1;
-  hipLaunchKernelGGL(ns_tables_kernel, dim3((ntab + 255) / 256), dim3(256), 0, s, k_seg, gq, xq, K, M, N);
+  hipLaunchKernelGGL(ns_tables_kernel, dim3((ntab + 255) / 256), dim3(256), 0, s, k_seg, xq, K, M);
   TFB_LAUNCH_CHECK();
   if (wide)
     hipLaunchKernelGGL(ns_load_kernel<true>, dim3(M / 32, N / 32, K), dim3(256), 0, s, (const float*)g, (const float*)inv_d, X[0],
@@ -150,7 +174,6 @@ extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, vo
     hipLaunchKernelGGL(ns_load_kernel<false>, dim3(256, 1, K), dim3(256), 0, s, (const float*)g, (const float*)inv_d, X[0], M, N);
   TFB_LAUNCH_CHECK();
 
-  using CfgT = GemmCfg<128, 128, 2, 2, 2, TFB_K_STRIDED, TFB_K_STRIDED>;
   using CfgN = GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>;
   int cur = 0;
   for (int it = 0; it < 5; ++it) {
@@ -158,33 +181,13 @@ extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, vo
     bf16_t* xin = X[cur];
     // the tall stack's last iteration writes y itself
     bf16_t* xout = (it == 4 && !wide) ? (bf16_t*)y : X[cur ^ 1];
-    GemmArgs ga;
     // G[k] = X[k]^T X[k]: both operands k-strided (rows of the stacked X), the contraction segmented per matrix
-    ga.P = GemmOperand{(const uint8_t*)xin, (long)N * 2};
-    ga.Q = ga.P;
-    ga.np = N;
-    ga.nq = N;
-    ga.nkt = 0;
-    ga.ntp = N / 128;
-    ga.q_group = nullptr;
-    ga.p_group_stride = 0;
-    ga.k_seg = k_seg;
-    EpiStoreGrouped eg{EpiStore{G, (long)N, 0, 0}, (long)N * N};
-    int st = launch<CfgT>(ga, K, M / 64, eg, s);
+    int st = gemm_ring_symmetric<EpiSym, 2, TFB_K_STRIDED>(GemmOperand{(const uint8_t*)xin, (long)N * 2}, 0, k_seg, N, M / 64, K,
+                                                          EpiSym{G, (long)N, (long)N * N}, s);
     if (st != TFB_OK) return st;
-    // B = c G G + b G on the stacked G: rows of G[k] against G[k] as the weight (G G^T = G G)
-    GemmArgs gb2;
-    gb2.P = GemmOperand{(const uint8_t*)G, (long)N * 2};
-    gb2.Q = gb2.P;
-    gb2.np = N;
-    gb2.nq = K * N;
-    gb2.nkt = N * 2 / 128;
-    gb2.ntp = N / 128;
-    gb2.q_group = gq;
-    gb2.p_group_stride = (long)N * N * 2;
-    gb2.k_seg = nullptr;
-    EpiAxpby eb{Bm, G, (long)N, c, b};
-    st = launch<CfgN>(gb2, 1, gb2.nkt, eb, s);
+    // B = c G G + b G: G[k] against itself (G G^T = G G)
+    st = gemm_ring_symmetric<EpiSymAxpby, 2, TFB_K_CONTIG>(GemmOperand{(const uint8_t*)G, (long)N * 2}, (long)N * N * 2, nullptr, N,
+                                                          N * 2 / 128, K, EpiSymAxpby{Bm, G, (long)N, (long)N * N, c, b}, s);
     if (st != TFB_OK) return st;
     // X' = X B + a X on the stacked X: rows of X[k] against B[k] as the weight (X B^T = X B)
     GemmArgs gx;
