@@ -54,6 +54,9 @@ int tfb_rmsnorm_fwd(const void* x, const void* res, const void* w, void* s_out, 
  * weight gradients in fp8 too nothing reads the bf16 rows, and they are then not written. */
 int tfb_rmsnorm_fwd_q(const void* x, const void* res, const void* w, void* s_out, void* y, void* inv, void* y8,
                       float y8_scale, long nrows, int C, float eps, void* stream);
+/* tfb_rmsnorm_fwd_q of nrows rows with y and y8 of nrows_out >= nrows rows: the rows beyond nrows are zeros. */
+int tfb_rmsnorm_fwd_q_pad(const void* x, const void* res, const void* w, void* s_out, void* y, void* inv, void* y8,
+                          float y8_scale, long nrows, long nrows_out, int C, float eps, void* stream);
 
 /* dx = gs + inv * (gh - s * (gh . s) * inv^2 / C), gh = gy * w; dw fp32 [C] (+)= sum_rows gy * s * inv.
  * dw_part: fp32 [tfb_norm_bwd_blocks(nrows)][C] scratch (needed only with w).
@@ -168,6 +171,10 @@ int tfb_amax_scale(const void* x, long n, float limit, int e_lo, int e_hi, void*
 /* out8 = fp8(x * scale): scale read from scale_ptr (device fp32) when non-NULL, else scale_imm. fmt 0 e4m3, 1 e5m2.
  * The reference's q8 (nki_mlp_fused8.py:821-825) producing bytes. */
 int tfb_quant_fp8(const void* x, const void* scale_ptr, float scale_imm, int fmt, void* out8, long n, void* stream);
+/* tfb_quant_fp8 into n_out >= n bytes, those beyond n zero; copy (NULL to skip) bf16 [n_out]: x, then zeros. n, n_out
+ * multiples of 8. */
+int tfb_quant_fp8_pad(const void* x, const void* scale_ptr, float scale_imm, int fmt, void* out8, void* copy, long n, long n_out,
+                      void* stream);
 
 /* w8 uint8 [4][F*d] = e4m3(w_fc s_wfc) as [F][d] and [d][F], e4m3(w_proj s_wproj) as [d][F] and [F][d].
  * Replaces _precast8_kernel / precast_ref (round2/source/kernels/nki_mlp_l4t.py:392, 948-970). */
@@ -192,6 +199,9 @@ int tfb_mlp8_fwd(const void* x8, const void* w8, const void* row, void* y, void*
  * (round2/source/kernels/nki_mlp_nr8.py:1032: xo = bf16(x1 + y)). */
 int tfb_mlp8_fwd_res(const void* x8, const void* w8, const void* row, const void* res, void* y, void* r, void* h8, long M,
                      int d, int F, void* stream);
+/* tfb_mlp8_fwd_res where res has only the first `rows` of the M rows; y's rows from `rows` on hold no result. */
+int tfb_mlp8_fwd_res_rows(const void* x8, const void* w8, const void* row, const void* res, void* y, void* r, void* h8, long M,
+                          long rows, int d, int F, void* stream);
 
 /* Backward from dy8 = e5m2(dy s_dy) [M][d]: dx bf16 [M][d], dpre bf16 [M][F], h = bf16(r^2) [M][F] (NULL to skip),
  * dp8 [M][F] byte scratch. row = the backward row.

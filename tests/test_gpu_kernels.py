@@ -1397,3 +1397,29 @@ def test_mean_loss_with_a_target_beyond_the_vocabulary(ops, dev):
     assert abs(want.item() - ref.item()) < 1e-5
     got = A.LmHeadLossFn.apply(x.to(dev).requires_grad_(True), W.to(dev).requires_grad_(True), t.to(dev), 0.0, "mean")
     assert abs(got.item() - want.item()) < 1e-3 * want.item()
+
+
+@pytest.mark.parametrize("dw8", [True, False])
+@pytest.mark.parametrize("rows", [1, 127, 129, 300])
+def test_fp8_mlp_pads_its_rows_inside(ops, dev, rows, dw8):
+    """The fp8 MLP and the folded one on a row count that is no multiple of a tile against the same calls on rows padded with
+    zeros by hand: outputs and gradients are the same bit for bit, and no result depends on the padding's storage."""
+    from trainium_frontier_them_bones_amd import autograd as A
+    g = _g(rows)
+    d, F = 256, 512
+    wf, wp = ((0.05 * torch.randn(*s, generator=g)).bfloat16().to(dev).requires_grad_(True) for s in ((F, d), (d, F)))
+    st = A.Mlp8State(dw_fp8=dw8)
+    st.refresh(wf.detach(), wp.detach())
+    x = torch.randn(rows, d, generator=g).bfloat16().to(dev)
+    gy = torch.randn(rows, d, generator=g).bfloat16().to(dev)
+    pad = (0, 0, 0, (-rows) % 128)
+    for node in (A.Mlp8Fn, A.NrMlpFn):
+        xa, xb = x.clone().requires_grad_(True), torch.nn.functional.pad(x, pad).requires_grad_(True)
+        junk = torch.full((1 << 20,), float("nan"), dtype=torch.bfloat16, device=dev)
+        del junk                                                       # (the buffers of the call below start as NaN)
+        ya = node.apply(xa, wf, wp, st)
+        ga = torch.autograd.grad(ya, (xa, wf, wp), gy)
+        yb = node.apply(xb, wf, wp, st)
+        gb = torch.autograd.grad(yb, (xb, wf, wp), torch.nn.functional.pad(gy, pad))
+        assert ya.shape == x.shape and torch.equal(ya, yb[:rows]) and torch.equal(ga[0], gb[0][:rows])
+        assert torch.equal(ga[1], gb[1]) and torch.equal(ga[2], gb[2])

@@ -24,6 +24,7 @@ SIGNATURES = {
     "tfb_norm_bwd_blocks": [_l],
     "tfb_rmsnorm_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _l, _i, _f, _vp],
     "tfb_rmsnorm_fwd_q": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _f, _l, _i, _f, _vp],
+    "tfb_rmsnorm_fwd_q_pad": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _f, _l, _l, _i, _f, _vp],
     "tfb_rmsnorm_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _l, _i, _vp],
     "tfb_rmsnorm_bwd_amax": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _l, _i, _vp],
     "tfb_norm_dw_finish": [_vp, _vp, _i, _l, _l, _i, _l, _i, _vp],
@@ -35,10 +36,12 @@ SIGNATURES = {
     "tfb_mlp8_backward_scales_part": [_vp, _i, _vp, _vp, _i, _vp],
     "tfb_amax_scale": [_vp, _l, _f, _i, _i, _vp, _vp, _vp],
     "tfb_quant_fp8": [_vp, _vp, _f, _i, _vp, _l, _vp],
+    "tfb_quant_fp8_pad": [_vp, _vp, _f, _i, _vp, _vp, _l, _l, _vp],
     "tfb_mlp8_precast": [_vp, _vp, _vp, _vp, _i, _i, _vp],
     "tfb_mlp8_refresh_layers": [_vp, _vp, _l, _i, _vp, _vp, _vp, _i, _i, _f, _f, _vp],
     "tfb_mlp8_fwd": [_vp, _vp, _vp, _vp, _vp, _vp, _l, _i, _i, _vp],
     "tfb_mlp8_fwd_res": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _l, _i, _i, _vp],
+    "tfb_mlp8_fwd_res_rows": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _l, _l, _i, _i, _vp],
     "tfb_mlp8_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _l, _i, _i, _vp],
     "tfb_mlp8_bwd_q": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _f, _l, _i, _i, _vp],
     "tfb_gemm_fp8_tn": [_vp, _i, _vp, _i, _vp, _vp, _f, _vp, _l, _i, _i, _i, _i, _vp, _l, _vp],

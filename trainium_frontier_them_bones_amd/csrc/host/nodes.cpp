@@ -610,17 +610,17 @@ MlpGrads mlp8_backward(const Mlp8Attrs& st, const Tensor& gy_in, const Tensor& g
     o.dx = b.dx;
     return o;
   }
-  MlpBwd b = mlp8_bwd(gy, r, st.w8, rowb, false);
+  MlpBwd b = mlp8_bwd(gy, r, st.w8, rowb, false, true);
   o.dx = b.dx;
   if (!buffers) {
     o.dw_fc = make({F, d}, BF16, gy);
     gemm(b.dpre, xa, o.dw_fc, F, d, M, true, false, false);
-    o.dw_proj = mlp_dw_proj(gy, r, {}, false, BF16);
+    o.dw_proj = mlp_dw_proj(b.dyp, r, {}, false, BF16);
     return o;
   }
   o.dw_fc = weight_grad(w_fc, b.dpre, xa, M, F, d);
   GradBuf gp = accumulate_into(w_proj);
-  o.dw_proj = mlp_dw_proj(gy, r, gp.buf, gp.accumulate, BF16);
+  o.dw_proj = mlp_dw_proj(b.dyp, r, gp.buf, gp.accumulate, BF16);
   if (gp.buf.defined()) o.dw_proj = Tensor();
   return o;
 }
@@ -636,8 +636,8 @@ struct Mlp8 : Function<Mlp8> {
     const Tensor x8 = val(x8_), res = dense(val(res_));
     // with the bytes given and the weight gradients in fp8 nothing reads x itself (it may be a storage-less placeholder)
     const Tensor x = x8.defined() && st.dw_fp8 ? Tensor() : dense(x_);
-    MlpFwd f = mlp8_fwd(x, st.w8, st.row, w_fc.size(0), st.x_scale, x8, res);
-    ctx->save_for_backward({st.dw_fp8 ? f.x8 : x, f.r, w_fc, w_proj});
+    MlpFwd f = mlp8_fwd(x, st.w8, st.row, w_fc.size(0), st.x_scale, x8, res, !st.dw_fp8);
+    ctx->save_for_backward({st.dw_fp8 ? f.x8 : f.xp.defined() ? f.xp : x, f.r, w_fc, w_proj});
     S& s = keep<S>(ctx);
     s.state = PyRef(state), s.has_res = res_.has_value();
     return f.y;
@@ -660,7 +660,7 @@ struct NrMlp : Function<NrMlp> {
     const Mlp8Attrs st = mlp8_attrs(state);
     const Tensor x = dense(x_);
     // (with the weight gradients in fp8 too nothing reads the norm's bf16 rows: only its e4m3 bytes are written)
-    NormOut n = rmsnorm_fwd_q(x, {}, eps, {}, st.x_scale.host(), !st.dw_fp8);
+    NormOut n = rmsnorm_fwd_q(x, {}, eps, {}, st.x_scale.host(), !st.dw_fp8, tile_rows(x.numel() / x.size(-1)));
     MlpFwd f = mlp8_fwd(n.y, st.w8, st.row, w_fc.size(0), st.x_scale, n.y8, x);
     ctx->save_for_backward({x, st.dw_fp8 ? n.y8 : n.y, n.inv, f.r, w_fc, w_proj});
     keep<PyRef>(ctx) = PyRef(state);

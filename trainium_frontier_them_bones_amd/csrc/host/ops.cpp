@@ -89,14 +89,20 @@ NormOut rmsnorm_fwd(const Tensor& x, const Tensor& w, double eps, const Tensor& 
   return o;
 }
 
-NormOut rmsnorm_fwd_q(const Tensor& x, const Tensor& w, double eps, const Tensor& res, double y8_scale, bool want_y) {
+NormOut rmsnorm_fwd_q(const Tensor& x, const Tensor& w, double eps, const Tensor& res, double y8_scale, bool want_y, int64_t rows_out) {
   chk(x), chk(res), chk(w);
   const int64_t C = x.size(-1), rows = x.numel() / C;
   NormOut o;
-  if (want_y) o.y = make_like(x);
+  const bool pad = rows_out > rows;
+  if (want_y) o.y = pad ? make({rows_out, C}, BF16, x) : make_like(x);
   o.s = res.defined() ? make_like(x) : x;
   o.inv = scratch(x, rows);
-  o.y8 = make(x.sizes(), U8, x);
+  o.y8 = pad ? make({rows_out, C}, U8, x) : make(x.sizes(), U8, x);
+  if (pad) {
+    TFB_CALL(tfb_rmsnorm_fwd_q_pad, ptr(x), ptr(res), ptr(w), res.defined() ? ptr(o.s) : nullptr, ptr(o.y), ptr(o.inv), ptr(o.y8), y8_scale,
+             rows, rows_out, C, eps, stream());
+    return o;
+  }
   TFB_CALL(tfb_rmsnorm_fwd_q, ptr(x), ptr(res), ptr(w), res.defined() ? ptr(o.s) : nullptr, ptr(o.y), ptr(o.inv), ptr(o.y8), y8_scale, rows,
            C, eps, stream());
   return o;
@@ -191,6 +197,26 @@ Tensor quant_fp8(const Tensor& x, const void* scale_dev, double scale_imm, int f
   TFB_CALL(tfb_quant_fp8, ptr(x), scale_dev, scale_imm, fmt, ptr(out), x.numel(), stream());
   return out;
 }
+// The rows of x and then zeros up to M rows, as bytes; padded: the same in bf16 where x has fewer rows and it is asked for.
+static Tensor quant_rows(const Tensor& x, const void* scale_dev, double scale_imm, int fmt, int64_t M, Tensor* padded) {
+  const int64_t d = x.size(-1);
+  if (x.numel() == M * d) {
+    if (padded) *padded = x;
+    return quant_fp8(x, scale_dev, scale_imm, fmt);
+  }
+  Tensor out = make({M, d}, U8, x);
+  if (padded) *padded = make({M, d}, BF16, x);
+  TFB_CALL(tfb_quant_fp8_pad, ptr(x), scale_dev, scale_imm, fmt, ptr(out), padded ? ptr(*padded) : nullptr, x.numel(), M * d, stream());
+  return out;
+}
+
+// A tensor of like's shape whose storage holds M rows: the GEMM that writes it stores whole tiles.
+static Tensor make_rows(at::IntArrayRef shape, int64_t M, int64_t d, const Tensor& like) {
+  Tensor t = make({M, d}, BF16, like);
+  t.unsafeGetTensorImpl()->set_sizes_contiguous(shape);
+  return t;
+}
+
 Tensor quant_fp8(const Tensor& x, const Scale& s, int fmt) { return quant_fp8(x, ptr(s.dev), s.imm, fmt); }
 
 Tensor gemm_fp8(const Tensor& a8, const Tensor& b8, int fmt_a, const void* dq_a, const void* dq_b, double dq, const Tensor& res,
@@ -219,31 +245,35 @@ Tensor gemm_fp8_tn(const Tensor& g8, const Tensor& a8, int fmt_g, int fmt_a, con
   return out;
 }
 
-MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F, const Scale& x_scale, const Tensor& x8, const Tensor& res) {
+MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F, const Scale& x_scale, const Tensor& x8, const Tensor& res,
+                bool want_xp) {
   chk(x), chk(w8, U8), chk(row, F32), chk(x8, U8), chk(res);
   TORCH_CHECK_VALUE(x.defined() || x8.defined(), "give x2 or its bytes x8");
-  const Tensor& in = x.defined() ? x : x8;
-  const int64_t d = in.size(-1), M = in.numel() / d;
+  const Tensor& in = res.defined() ? res : x.defined() ? x : x8;   // (x and x8 may come padded already, res has the call's rows)
+  const int64_t d = in.size(-1), rows = in.numel() / d, M = tile_rows(rows);
+  const auto fits = [&](const Tensor& t) { return t.size(-1) == d && (t.numel() == rows * d || t.numel() == M * d); };
   TORCH_CHECK_VALUE(!x8.defined() || (x8.size(-1) == d && x8.numel() == M * d), "x8 shape");
-  TORCH_CHECK_VALUE(!res.defined() || (res.size(-1) == d && res.numel() == M * d), "res shape");
+  TORCH_CHECK_VALUE(!x.defined() || fits(x), "res shape");
   MlpFwd o;
-  o.x8 = x8.defined() ? x8 : quant_fp8(x, x_scale, E4M3);
-  o.y = make(in.sizes(), BF16, w8);
+  o.x8 = x8.defined() ? x8 : quant_rows(x, ptr(x_scale.dev), x_scale.imm, E4M3, M, want_xp ? &o.xp : nullptr);
+  o.y = make_rows(in.sizes(), M, d, w8);
   o.r = make({M, F}, BF16, w8);
   const Tensor h8 = make({M, F}, U8, w8);
-  if (res.defined())
+  if (res.defined() && rows < M)
+    TFB_CALL(tfb_mlp8_fwd_res_rows, ptr(o.x8), ptr(w8), ptr(row), ptr(res), ptr(o.y), ptr(o.r), ptr(h8), M, rows, d, F, stream());
+  else if (res.defined())
     TFB_CALL(tfb_mlp8_fwd_res, ptr(o.x8), ptr(w8), ptr(row), ptr(res), ptr(o.y), ptr(o.r), ptr(h8), M, d, F, stream());
   else
     TFB_CALL(tfb_mlp8_fwd, ptr(o.x8), ptr(w8), ptr(row), ptr(o.y), ptr(o.r), ptr(h8), M, d, F, stream());
   return o;
 }
 
-MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h) {
+MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h, bool want_dyp) {
   chk(dy), chk(r), chk(w8, U8), chk(row, F32);
-  const int64_t d = dy.size(-1), M = dy.numel() / d, F = r.size(1);
+  const int64_t d = dy.size(-1), M = tile_rows(dy.numel() / d), F = r.size(1);
   MlpBwd o;
-  o.dy8 = quant_fp8(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2);
-  o.dx = make_like(dy);
+  o.dy8 = quant_rows(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2, M, want_dyp ? &o.dyp : nullptr);
+  o.dx = make_rows(dy.sizes(), M, d, dy);
   o.dpre = make({M, F}, BF16, dy);
   if (want_h) o.h = make({M, F}, BF16, dy);
   o.dp8 = make({M, F}, U8, dy);
@@ -253,10 +283,10 @@ MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tenso
 
 MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, bool want_dpre) {
   chk(dy), chk(r), chk(w8, U8), chk(row, F32);
-  const int64_t d = dy.size(-1), M = dy.numel() / d, F = r.size(1);
+  const int64_t d = dy.size(-1), M = tile_rows(dy.numel() / d), F = r.size(1);
   MlpBwd o;
-  o.dy8 = quant_fp8(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2);
-  o.dx = make_like(dy);
+  o.dy8 = quant_rows(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2, M, nullptr);
+  o.dx = make_rows(dy.sizes(), M, d, dy);
   if (want_dpre) o.dpre = make({M, F}, BF16, dy);
   o.dp8 = make({M, F}, U8, dy);
   o.hq8 = make({M, F}, U8, dy);

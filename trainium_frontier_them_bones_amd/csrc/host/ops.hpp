@@ -17,7 +17,8 @@ Tensor workspace(const Tensor& like);   // fp32 split-K scratch of the current s
 // norms
 struct NormOut { Tensor s, y, inv, y8; };
 NormOut rmsnorm_fwd(const Tensor& x, const Tensor& w, double eps, const Tensor& res);
-NormOut rmsnorm_fwd_q(const Tensor& x, const Tensor& w, double eps, const Tensor& res, double y8_scale, bool want_y);
+// rows_out: the rows of y and y8 (0: x's); those beyond x's are zeros
+NormOut rmsnorm_fwd_q(const Tensor& x, const Tensor& w, double eps, const Tensor& res, double y8_scale, bool want_y, int64_t rows_out = 0);
 struct NormGrad { Tensor dx, dw, amax; };
 NormGrad rmsnorm_bwd(const Tensor& gy, const Tensor& s, const Tensor& inv, const Tensor& w, const Tensor& gs, const Tensor& dw,
                      bool accumulate, const Tensor& part, bool want_amax);
@@ -43,10 +44,14 @@ Tensor gemm_fp8(const Tensor& a8, const Tensor& b8, int fmt_a, const void* dq_a,
                 at::IntArrayRef out_shape);
 Tensor gemm_fp8_tn(const Tensor& g8, const Tensor& a8, int fmt_g, int fmt_a, const void* s_g, const void* s_a, double imm, Tensor out,
                    bool accumulate, at::ScalarType out_dtype);
-struct MlpFwd { Tensor y, r, x8; };
-MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F, const Scale& x_scale, const Tensor& x8, const Tensor& res);
-struct MlpBwd { Tensor dx, h, dpre, dp8, hq8, dy8; };
-MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h);
+// The fp8 MLP's calls take any number of rows; r and the byte operands have tile_rows(rows) rows, those beyond the given ones
+// from zeros. xp / dyp: x / dy with as many rows (themselves where nothing is to be padded), asked for by want_xp / want_dyp.
+inline int64_t tile_rows(int64_t rows) { return (rows + 127) / 128 * 128; }
+struct MlpFwd { Tensor y, r, x8, xp; };
+MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F, const Scale& x_scale, const Tensor& x8, const Tensor& res,
+                bool want_xp = false);
+struct MlpBwd { Tensor dx, h, dpre, dp8, hq8, dy8, dyp; };
+MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h, bool want_dyp = false);
 MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, bool want_dpre);
 void mlp8_dw8(const Tensor& x8, const Tensor& dp8, const Tensor& hq8, const Tensor& dy8, const Tensor& row, const Scale& x_scale,
               Tensor& dw_fc, Tensor& dw_proj, bool accumulate, at::ScalarType out_dtype);

@@ -306,12 +306,17 @@ __global__ __launch_bounds__(256) void amax_scale_kernel(const float* amax_part,
 }
 
 // ------------------------------------------------------------------------------------ casts
+// Elements n .. n_out are written as zeros: the rows up to a GEMM's next whole tile. copy (optional): the bf16 elements
+// too, padded alike, where the bf16 weight gradient contracts over the padded rows. Bound by memory; padding here instead
+// of in a copy of x saves a read and a write of x and three launches (8 x 2001 rows of 1536: 3 x 18 us of 1386).
 template <int FMT>
 __global__ __launch_bounds__(256) void quant_kernel(const bf16_t* __restrict__ x, const float* __restrict__ scale_ptr,
-                                                   float scale_imm, uint8_t* __restrict__ out, long n) {
+                                                   float scale_imm, uint8_t* __restrict__ out, bf16_t* __restrict__ copy, long n,
+                                                   long n_out) {
   const float s = scale_ptr ? *scale_ptr : scale_imm;
-  for (long i = ((long)blockIdx.x * 256 + threadIdx.x) * 8; i < n; i += (long)gridDim.x * 256 * 8) {
-    u32x4 u = *(const u32x4*)(x + i);
+  for (long i = ((long)blockIdx.x * 256 + threadIdx.x) * 8; i < n_out; i += (long)gridDim.x * 256 * 8) {
+    u32x4 u = i < n ? *(const u32x4*)(x + i) : u32x4{0u, 0u, 0u, 0u};
+    if (copy) *(u32x4*)(copy + i) = u;
     u32x2 o;
     o.x = cvt4_fp8<FMT>(bflo(u[0]) * s, bfhi(u[0]) * s, bflo(u[1]) * s, bfhi(u[1]) * s);
     o.y = cvt4_fp8<FMT>(bflo(u[2]) * s, bfhi(u[2]) * s, bflo(u[3]) * s, bfhi(u[3]) * s);
@@ -476,6 +481,7 @@ struct EpiDescaleRes {
   const bf16_t* res;
   bf16_t* out;
   long ld;
+  int last;        // res has rows 0 .. last: the rows beyond it that fill the last tile read row `last` and are no one's result
   float dq = 0.f;  // the descale factor, read once by prepare()
   using pre_t = u32x4;
   __device__ __forceinline__ EpiDescaleRes prepare() const {
@@ -489,7 +495,7 @@ struct EpiDescaleRes {
     }
     return e;
   }
-  __device__ __forceinline__ pre_t prefetch(int p, int q) const { return tfb_load_nt((const u32x4*)(res + (long)q * ld + p), TFB_NT_RES); }
+  __device__ __forceinline__ pre_t prefetch(int p, int q) const { return tfb_load_nt((const u32x4*)(res + (long)min(q, last) * ld + p), TFB_NT_RES); }
   __device__ __forceinline__ void operator()(int p, int q, const float (&v)[8], const pre_t& rv, int) const {
     float r[8], a[8], b[8];
 #pragma unroll
@@ -665,11 +671,12 @@ struct LoadSquare {
 inline bool shapes8(long M, int d, int F) { return M > 0 && M % 128 == 0 && d > 0 && d % 256 == 0 && F > 0 && F % 256 == 0; }
 
 template <int FMT>
-int launch_quant(const void* x, const float* sp, float si, void* out, long n, hipStream_t s) {
-  if (n % 8) return TFB_ERR_SHAPE;
-  long blocks = (n / 8 + 255) / 256;
+int launch_quant(const void* x, const float* sp, float si, void* out, void* copy, long n, long n_out, hipStream_t s) {
+  if (n % 8 || n_out % 8) return TFB_ERR_SHAPE;
+  long blocks = (n_out / 8 + 255) / 256;
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(quant_kernel<FMT>, dim3((unsigned)blocks), dim3(256), 0, s, (const bf16_t*)x, sp, si, (uint8_t*)out, n);
+  hipLaunchKernelGGL(quant_kernel<FMT>, dim3((unsigned)blocks), dim3(256), 0, s, (const bf16_t*)x, sp, si, (uint8_t*)out,
+                     (bf16_t*)copy, n, n_out);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
@@ -762,14 +769,21 @@ extern "C" int tfb_amax_scale(const void* x, long n, float limit, int e_lo, int 
   return TFB_OK;
 }
 
+// tfb_quant_fp8 into a longer buffer: bytes n .. n_out are zeros; copy (optional) [n_out] bf16 = x, then zeros.
+extern "C" int tfb_quant_fp8_pad(const void* x, const void* scale_ptr, float scale_imm, int fmt, void* out8, void* copy, long n,
+                                 long n_out, void* stream) {
+  if (!x || !out8) return TFB_ERR_ARG;
+  if (n <= 0 || n_out < n) return TFB_ERR_SHAPE;
+  const float* sp = (const float*)scale_ptr;
+  if (fmt == TFB_FMT_E4M3) return launch_quant<TFB_FMT_E4M3>(x, sp, scale_imm, out8, copy, n, n_out, (hipStream_t)stream);
+  if (fmt == TFB_FMT_E5M2) return launch_quant<TFB_FMT_E5M2>(x, sp, scale_imm, out8, copy, n, n_out, (hipStream_t)stream);
+  return TFB_ERR_ARG;
+}
+
 // out8 = fp8(x * scale): scale from device memory (scale_ptr) or immediate. fmt 0 = e4m3, 1 = e5m2.
 extern "C" int tfb_quant_fp8(const void* x, const void* scale_ptr, float scale_imm, int fmt, void* out8, long n,
                              void* stream) {
-  if (!x || !out8) return TFB_ERR_ARG;
-  if (n <= 0) return TFB_ERR_SHAPE;
-  if (fmt == TFB_FMT_E4M3) return launch_quant<TFB_FMT_E4M3>(x, (const float*)scale_ptr, scale_imm, out8, n, (hipStream_t)stream);
-  if (fmt == TFB_FMT_E5M2) return launch_quant<TFB_FMT_E5M2>(x, (const float*)scale_ptr, scale_imm, out8, n, (hipStream_t)stream);
-  return TFB_ERR_ARG;
+  return tfb_quant_fp8_pad(x, scale_ptr, scale_imm, fmt, out8, nullptr, n, n, stream);
 }
 
 // w8: uint8 [4][F*d] = wf8 [F][d], wf8T [d][F], wp8 [d][F], wp8T [F][d] (all e4m3, scaled by the row's s_w).
@@ -889,7 +903,7 @@ extern "C" int tfb_gemm_fp8_res(const void* a8, const void* b8, const void* dq_a
   if (!a8 || !b8 || !res || !out) return TFB_ERR_ARG;
   if (M <= 0 || N <= 0 || K <= 0 || M % 128 || N % 128 || K % 128 || M > 0x7fffffffL) return TFB_ERR_SHAPE;
   GemmOperand P{(const uint8_t*)b8, (long)K}, Q{(const uint8_t*)a8, (long)K};
-  EpiDescaleRes e{nullptr, 0, (const float*)dq_a, (const float*)dq_b, dq_imm, (const bf16_t*)res, (bf16_t*)out, (long)N};
+  EpiDescaleRes e{nullptr, 0, (const float*)dq_a, (const float*)dq_b, dq_imm, (const bf16_t*)res, (bf16_t*)out, (long)N, (int)M - 1};
   return launch8<Cfg8>(P, Q, N, (int)M, (long)K, e, (hipStream_t)stream);
 }
 
@@ -965,11 +979,11 @@ extern "C" int tfb_mlp8_fwd(const void* x8, const void* w8, const void* row, voi
 // tfb_mlp8_fwd with the block's residual add in the second GEMM's store: y = bf16(res + bf16(MLP(x))), res [M][d] bf16 (the
 // MLP's input before its norm). Equal to tfb_mlp8_fwd followed by a bf16 add, bit for bit.
 // Replaces the residual half of _mlp8_fwd_nr_kernel (round2/source/kernels/nki_mlp_nr8.py:1032); its norm half is
-// tfb_rmsnorm_fwd_q, which hands this call its x8.
-extern "C" int tfb_mlp8_fwd_res(const void* x8, const void* w8, const void* row, const void* res, void* y, void* r, void* h8,
-                                long M, int d, int F, void* stream) {
+// tfb_rmsnorm_fwd_q, which hands this call its x8. _rows: res has only the first `rows` rows, and only those of y count.
+extern "C" int tfb_mlp8_fwd_res_rows(const void* x8, const void* w8, const void* row, const void* res, void* y, void* r, void* h8,
+                                     long M, long rows, int d, int F, void* stream) {
   if (!x8 || !w8 || !row || !res || !y || !r || !h8) return TFB_ERR_ARG;
-  if (!shapes8(M, d, F)) return TFB_ERR_SHAPE;
+  if (!shapes8(M, d, F) || rows <= 0 || rows > M || M > 0x7fffffffL) return TFB_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
   const uint8_t* b = (const uint8_t*)w8;
   const long n = (long)F * d;
@@ -978,8 +992,13 @@ extern "C" int tfb_mlp8_fwd_res(const void* x8, const void* w8, const void* row,
   int st = launch_k768<Cfg8>(Pw, Qx, F, (int)M, (long)d, e1, s);
   if (st != TFB_OK) return st;
   GemmOperand Pp{b + 2 * n, (long)F}, Qh{(const uint8_t*)h8, (long)F};
-  EpiDescaleRes e2{(const float*)row, SC_DQ_PROJ, nullptr, nullptr, 1.0f, (const bf16_t*)res, (bf16_t*)y, (long)d};
+  EpiDescaleRes e2{(const float*)row, SC_DQ_PROJ, nullptr, nullptr, 1.0f, (const bf16_t*)res, (bf16_t*)y, (long)d,
+                   (int)rows - 1};
   return launch8<Cfg8>(Pp, Qh, d, (int)M, (long)F, e2, s);
+}
+extern "C" int tfb_mlp8_fwd_res(const void* x8, const void* w8, const void* row, const void* res, void* y, void* r, void* h8,
+                                long M, int d, int F, void* stream) {
+  return tfb_mlp8_fwd_res_rows(x8, w8, row, res, y, r, h8, M, M, d, F, stream);
 }
 
 // Backward: dy8 [M][d] e5m2 (cast at the row's s_dy), r [M][F] -> dx [M][d], dpre [M][F] bf16, h [M][F] bf16 (optional,

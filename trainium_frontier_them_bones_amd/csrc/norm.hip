@@ -112,7 +112,7 @@ template <int NCH, int G>
 __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                          const bf16_t* __restrict__ w, bf16_t* __restrict__ s_out,
                                                          bf16_t* __restrict__ y, float* __restrict__ inv, long nrows,
-                                                         int C, float eps, uint8_t* __restrict__ y8, float y8_scale) {
+                                                         int C, float eps, uint8_t* __restrict__ y8, float y8_scale, long nrows_out) {
   constexpr int RPW = 64 / G;  // rows per wavefront
   const int lane = threadIdx.x & (G - 1), sub = (threadIdx.x & 63) / G, wave = threadIdx.x >> 6;
   Row<NCH, G> wr;
@@ -161,6 +161,17 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restri
       }
     }
     if (inv && lane == 0) inv[row] = rs;
+  }
+  // rows nrows .. nrows_out of y and y8 are zeros, up to the next whole tile of the GEMM that reads them
+  for (; row < nrows_out; row += step) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int c = (lane + G * i) * 8;
+      if (c < C) {
+        if (y) *(u32x4*)(y + row * C + c) = u32x4{0u, 0u, 0u, 0u};
+        if (y8) *(u32x2*)(y8 + row * C + c) = u32x2{0u, 0u};
+      }
+    }
   }
 }
 
@@ -539,16 +550,16 @@ extern "C" int tfb_norm_bwd_blocks(long nrows) { return grid_for(nrows, 1024); }
 // y8 (optional): e4m3(bf16(y) * y8_scale), [nrows][C] bytes - the operand cast of the fp8 GEMM that consumes y, made here
 // instead of in a pass of its own.
 static int rmsnorm_fwd_impl(const void* x, const void* res, const void* w, void* s_out, void* y, void* inv, void* y8,
-                            float y8_scale, long nrows, int C, float eps, void* stream) {
+                            float y8_scale, long nrows, long nrows_out, int C, float eps, void* stream) {
   if (!x || (!y && !y8)) return TFB_ERR_ARG;   // y may be left out when only its fp8 cast is read (both MLP GEMM kinds in fp8)
   if (res && !s_out) return TFB_ERR_ARG;
-  if (!norm_shape_ok(nrows, C)) return TFB_ERR_SHAPE;
-  const long rpb = norm_rows_per_block(C), nb = (nrows + rpb - 1) / rpb;
+  if (!norm_shape_ok(nrows, C) || nrows_out < nrows) return TFB_ERR_SHAPE;
+  const long rpb = norm_rows_per_block(C), nb = (nrows_out + rpb - 1) / rpb;
   int grid = (int)(nb < 8192 ? nb : 8192);
 #define CALL(N, G)                                                                                                    \
   hipLaunchKernelGGL((rmsnorm_fwd_kernel<N, G>), dim3(grid), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)x,     \
                      (const bf16_t*)res, (const bf16_t*)w, (bf16_t*)s_out, (bf16_t*)y, (float*)inv, nrows, C, eps,    \
-                     (uint8_t*)y8, y8_scale)
+                     (uint8_t*)y8, y8_scale, nrows_out)
   DISPATCH_ROWS(C, CALL);
 #undef CALL
   TFB_LAUNCH_CHECK();
@@ -556,12 +567,16 @@ static int rmsnorm_fwd_impl(const void* x, const void* res, const void* w, void*
 }
 extern "C" int tfb_rmsnorm_fwd(const void* x, const void* res, const void* w, void* s_out, void* y, void* inv, long nrows,
                                int C, float eps, void* stream) {
-  return rmsnorm_fwd_impl(x, res, w, s_out, y, inv, nullptr, 0.f, nrows, C, eps, stream);
+  return rmsnorm_fwd_impl(x, res, w, s_out, y, inv, nullptr, 0.f, nrows, nrows, C, eps, stream);
+}
+extern "C" int tfb_rmsnorm_fwd_q_pad(const void* x, const void* res, const void* w, void* s_out, void* y, void* inv, void* y8,
+                                     float y8_scale, long nrows, long nrows_out, int C, float eps, void* stream) {
+  if (!y8) return TFB_ERR_ARG;
+  return rmsnorm_fwd_impl(x, res, w, s_out, y, inv, y8, y8_scale, nrows, nrows_out, C, eps, stream);
 }
 extern "C" int tfb_rmsnorm_fwd_q(const void* x, const void* res, const void* w, void* s_out, void* y, void* inv, void* y8,
                                  float y8_scale, long nrows, int C, float eps, void* stream) {
-  if (!y8) return TFB_ERR_ARG;
-  return rmsnorm_fwd_impl(x, res, w, s_out, y, inv, y8, y8_scale, nrows, C, eps, stream);
+  return tfb_rmsnorm_fwd_q_pad(x, res, w, s_out, y, inv, y8, y8_scale, nrows, nrows, C, eps, stream);
 }
 
 // dw_part: fp32 [tfb_norm_bwd_blocks(nrows)][C] scratch (only when w != NULL); dw: fp32 [C].

@@ -259,18 +259,13 @@ def fp8_refresh_weights(model, quantise_fn=None, *, e4m3_limit=240.0, x_scale=4.
 
 def mlp_fused8(mlp, x):
     """MLP.forward on [b, t, n_embd] with the four activation GEMMs in fp8 (R2:6947): c_proj(relu(c_fc(x))^2), weights
-    mlp.c_fc.weight [F, d] and mlp.c_proj.weight [d, F]; rows are padded with zeros to a multiple of 128 (a zero row
-    touches no other row). The scale row and weight bytes come from fp8_refresh_weights (made here on first use)."""
+    mlp.c_fc.weight [F, d] and mlp.c_proj.weight [d, F]; any number of rows: the byte operands
+    are padded with zeros to a multiple of 128 rows by the kernels that write them (a zero row touches no other row). The scale row and weight bytes come from fp8_refresh_weights (made here on first use)."""
     if getattr(mlp, "tfb_mlp8", None) is None or mlp.tfb_mlp8.row is None:
         fp8_refresh_weights([mlp])
-    b, t, c = x.shape
-    m = b * t
-    pad = (-m) % 128
-    x2 = torch.nn.functional.pad(x.reshape(m, c), (0, 0, 0, pad)) if pad else x
     w_fc = mlp.c_fc.weight if mlp.c_fc.weight.dtype == bf16 else mlp.c_fc.weight.to(bf16)
     w_proj = mlp.c_proj.weight if mlp.c_proj.weight.dtype == bf16 else mlp.c_proj.weight.to(bf16)
-    y = A.Mlp8Fn.apply(x2, w_fc, w_proj, mlp.tfb_mlp8)
-    return y[:m].reshape(b, t, c) if pad else y
+    return A.Mlp8Fn.apply(x, w_fc, w_proj, mlp.tfb_mlp8)
 
 
 def moe_refresh_weights(moe, *, e4m3_limit=240.0, x_scale=4.0):
@@ -323,20 +318,15 @@ def moe_mlp(moe, x, want_stats=False, aux_weights=(0.0, 0.0, 0.0)):
 def nr_mlp(mlp, x1):
     """x1 + MLP(rms_norm(x1)) on [b, t, n_embd] with the norm and the residual add folded into the fp8 MLP's two calls
     (R2:9202 nr_mlp / 9168 NrMlp; kernels K/nki_mlp_nr8.py:1032): the norm's pass also writes the e4m3 operand, the add
-    is made in the second GEMM's store, the backward's norm gradient and residual add are one launch. Rows are padded
-    with zeros to a multiple of 128 (a zero row normalises to zero and adds zero)."""
+    is made in the second GEMM's store, the backward's norm gradient and residual add are one launch. Any
+    number of rows, the byte operands padded with zeros to a multiple of 128 by the kernels that write them."""
     if getattr(mlp, "tfb_mlp8", None) is None or mlp.tfb_mlp8.row is None:
         fp8_refresh_weights([mlp])
-    b, t, c = x1.shape
     if x1.dtype != bf16:
         raise RuntimeError("the folded MLP takes bf16 rows, not %s" % x1.dtype)
-    m = b * t
-    pad = (-m) % 128
-    x2 = torch.nn.functional.pad(x1.reshape(m, c), (0, 0, 0, pad)) if pad else x1
     w_fc = mlp.c_fc.weight if mlp.c_fc.weight.dtype == bf16 else mlp.c_fc.weight.to(bf16)
     w_proj = mlp.c_proj.weight if mlp.c_proj.weight.dtype == bf16 else mlp.c_proj.weight.to(bf16)
-    xo = A.NrMlpFn.apply(x2, w_fc, w_proj, mlp.tfb_mlp8)
-    return xo[:m].reshape(b, t, c) if pad else xo
+    return A.NrMlpFn.apply(x1, w_fc, w_proj, mlp.tfb_mlp8)
 
 
 def proj_residual(x, w, res):
