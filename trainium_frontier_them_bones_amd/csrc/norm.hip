@@ -282,7 +282,14 @@ __global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ 
   out += (long)blockIdx.y * out_stride;
   float t = 0.f;
   if (c < C)
-    for (int r = ty; r < rows; r += 16) t += part[(long)r * C + c];
+    for (int r = ty; r < rows; r += 16 * 16) {   // sixteen rows in flight: the sum is a chain of load latencies otherwise (20 us of 1024 rows)
+      float v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v[k] = r + 16 * k < rows ? part[(long)(r + 16 * k) * C + c] : 0.f;
+#pragma unroll
+      for (int k = 0; k < 16; ++k)
+        if (r + 16 * k < rows) t += v[k];
+    }
   red[ty][tx] = t;
   __syncthreads();
   if (ty == 0 && c < C) {
