@@ -451,23 +451,32 @@ __global__ __launch_bounds__(256) void mix_tail_fwd_kernel(const bf16_t* __restr
 // g = bf16(ge + inv (gy - s (gy . s) inv^2 / C)) (the tail norm's backward, one rounding; ge and/or gy may be absent);
 // gx[t] = bf16(g[t] + bf16(lam g[t + 1])) (g[t + 1] = 0 at a sequence's last token: the shift's adjoint);
 // dlam partial [gridDim.x] = sum over the workgroup's rows of the bf16 products bf16(g[t] x[t - 1]) in fp32.
-// Row t + 1's g is recomputed by the wavefront that owns row t (the chain is per row: the same bits).
-template <int NCH>
+// Bound by memory: each group of lanes takes a run of rows from its last to its first, so that g[t + 1] is what it has just
+// made and only one row a run is made twice, and requests the next row before it works on this one. 32000 x 768: 81 us with
+// every g made twice from its three rows, DT with runs of eight.
+template <int NCH, int G>
 __global__ __launch_bounds__(256) void mix_tail_bwd_kernel(const bf16_t* __restrict__ s, const bf16_t* __restrict__ gy,
                                                           const bf16_t* __restrict__ ge, const float* __restrict__ inv,
                                                           const bf16_t* __restrict__ x, const float* __restrict__ lam,
                                                           bf16_t* __restrict__ gx, float* __restrict__ dlam_part, long nrows,
-                                                          int C, int T) {
+                                                          int C, int T, long run) {
+  constexpr int RPW = 64 / G;
   __shared__ float red[ROWS_PER_BLOCK];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & (G - 1), sub = (threadIdx.x & 63) / G, wave = threadIdx.x >> 6;
   const float l = lam[0];
-  float dl = 0.f;
-  auto g_row = [&](long row, Row<NCH>& g) {
-    Row<NCH> a;
-    a.load(s + row * C, C, lane);
+  float dl = 0.f, rs_next = 0.f;
+  RawRow<NCH, G> us, ug, ue, ux;
+  auto request = [&](long row, bool with_x) {
+    us.load(s + row * C, C, lane);
+    if (gy) ug.load(gy + row * C, C, lane), rs_next = inv[row];
+    if (ge) ue.load(ge + row * C, C, lane);
+    if (with_x) ux.load(x + (row - 1) * C, C, lane);
+  };
+  auto g_row = [&](Row<NCH, G>& g, const RawRow<NCH, G>& a_, const RawRow<NCH, G>& g_, const RawRow<NCH, G>& e_, float rs) {
+    Row<NCH, G> a;
     if (gy) {
-      g.load(gy + row * C, C, lane);
-      const float rs = inv[row];
+      a_.widen(a);
+      g_.widen(g);
       const float coef = row_dot(g, a) * rs * rs * (1.0f / C);
 #pragma unroll
       for (int i = 0; i < NCH; ++i)
@@ -477,34 +486,51 @@ __global__ __launch_bounds__(256) void mix_tail_bwd_kernel(const bf16_t* __restr
       g.zero();
     }
     if (ge) {
-      Row<NCH> e;
-      e.load(ge + row * C, C, lane);
+      e_.widen(a);
 #pragma unroll
       for (int i = 0; i < NCH; ++i)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) g.v[i][k] += e.v[i][k];
+        for (int k = 0; k < 8; ++k) g.v[i][k] += a.v[i][k];
     }
     g.round();
   };
-  for (long row = (long)blockIdx.x * ROWS_PER_BLOCK + wave; row < nrows; row += (long)gridDim.x * ROWS_PER_BLOCK) {
-    Row<NCH> g, gn, xp;
-    g_row(row, g);
-    if ((row + 1) % T) g_row(row + 1, gn);
-    else gn.zero();
-    if (row % T) xp.load(x + (row - 1) * C, C, lane);
-    else xp.zero();
-    float part = 0.f;
+  const long first = (((long)blockIdx.x * ROWS_PER_BLOCK + wave) * RPW + sub) * run, last = min(first + run, nrows) - 1;
+  if (first <= last) {
+    Row<NCH, G> gn;
+    const bool more = (last + 1) % T != 0;
+    request(more ? last + 1 : last, !more && last % T != 0);
+    if (more) {
+      const RawRow<NCH, G> a = us, g_ = ug, e = ue;
+      const float rs = rs_next;
+      request(last, last % T != 0);
+      g_row(gn, a, g_, e, rs);
+    } else {
+      gn.zero();
+    }
+    for (long row = last; row >= first; --row) {
+      Row<NCH, G> g, xp, out;
+      const RawRow<NCH, G> a = us, g_ = ug, e = ue, xr = ux;
+      const float rs = rs_next;
+      if (row > first) request(row - 1, (row - 1) % T != 0);
+      g_row(g, a, g_, e, rs);
+      if (row % T) xr.widen(xp);
+      else xp.zero();
+      if ((row + 1) % T == 0) gn.zero();
+      float part = 0.f;
 #pragma unroll
-    for (int i = 0; i < NCH; ++i)
+      for (int i = 0; i < NCH; ++i)
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        part += round_bf(g.v[i][k] * xp.v[i][k]);
-        g.v[i][k] = g.v[i][k] + round_bf(l * gn.v[i][k]);
-      }
-    dl += wave_sum(part);
-    g.store(gx + row * C, C, lane);
+        for (int k = 0; k < 8; ++k) {
+          part += round_bf(g.v[i][k] * xp.v[i][k]);
+          out.v[i][k] = g.v[i][k] + round_bf(l * gn.v[i][k]);
+        }
+      dl += part;
+      out.store(gx + row * C, C, lane);
+      gn = g;
+    }
   }
-  if (lane == 0) red[wave] = dl;
+  dl = wave_sum(dl);
+  if ((threadIdx.x & 63) == 0) red[wave] = dl;
   __syncthreads();
   if (threadIdx.x == 0) dlam_part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
@@ -698,12 +724,13 @@ extern "C" int tfb_mix_tail_bwd(const void* s1, const void* gy, const void* ge, 
                                 void* gx, void* part, void* dlam, long nrows, int C, int T, void* stream) {
   if (!s1 || (!gy && !ge) || !inv || !x || !lam || !gx || !part || !dlam) return TFB_ERR_ARG;
   if (!norm_shape_ok(nrows, C) || T <= 0 || nrows % T) return TFB_ERR_SHAPE;
-  int grid = grid_for(nrows, 1024);
-#define CALL(N)                                                                                                          \
-  hipLaunchKernelGGL(mix_tail_bwd_kernel<N>, dim3(grid), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)s1,           \
+  const long rpb = norm_rows_per_block(C), run = (nrows + 1024 * rpb - 1) / (1024 * rpb);
+  const int grid = (int)((nrows + rpb * run - 1) / (rpb * run));   // <= 1024 and <= tfb_norm_bwd_blocks(nrows)
+#define CALL(N, G)                                                                                                       \
+  hipLaunchKernelGGL((mix_tail_bwd_kernel<N, G>), dim3(grid), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)s1,      \
                      (const bf16_t*)gy, (const bf16_t*)ge, (const float*)inv, (const bf16_t*)x, (const float*)lam,       \
-                     (bf16_t*)gx, (float*)part, nrows, C, T)
-  DISPATCH_NCH(C, CALL);
+                     (bf16_t*)gx, (float*)part, nrows, C, T, run)
+  DISPATCH_ROWS(C, CALL);
 #undef CALL
   TFB_LAUNCH_CHECK();
   hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, (const float*)part, grid, (float*)dlam);
