@@ -21,11 +21,15 @@ namespace {
 
 __device__ __forceinline__ float fexp(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
 
-// c * tanh(x / c) and tanh(x / c)
-__device__ __forceinline__ float tanh_fast(float y) {
-  // tanh(y) = 1 - 2 / (exp(2y) + 1); exp overflow gives 1, underflow gives -1
-  float e = __builtin_amdgcn_exp2f(y * 2.8853900817779268f);
-  return 1.0f - 2.0f / (e + 1.0f);
+// tanh(y) = 1 - 2 / (exp(2 y) + 1), the exponential's overflow giving 1 and its underflow -1; with the hardware reciprocal (1
+// ulp, as the exponential): a correctly rounded division is ten more instructions a value, and made the softcap's pass over
+// the logits run at 2.3 TB/s
+__device__ __forceinline__ float tanh_rcp(float y) { return __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(y * 2.8853900817779268f) + 1.0f); }
+__device__ __forceinline__ float tanh_fast(float y) { return 1.0f - 2.0f * tanh_rcp(y); }
+// exp(cap tanh(x / cap) - cap) = exp(-2 cap / (exp(2 x / cap) + 1)): two exponentials and a reciprocal, half the instructions
+// of the tanh, its division and the exponential after it.
+__device__ __forceinline__ float capped_exp(float x, float icap, float cap) {
+  return __builtin_amdgcn_exp2f(-2.8853900817779268f * cap * tanh_rcp(x * icap));
 }
 
 struct MS {
@@ -70,205 +74,165 @@ __global__ __launch_bounds__(1024) void loss_row_weights_kernel(const IDX* __res
 }
 
 // ------------------------------------------------------------------------------------ loss on logits
-// One workgroup per row. loss_row = w * (lse - s_t) with w = row_w[row] (or 1), 0 for target < 0.
-template <typename IDX>
+// A row belongs to TPR threads: a workgroup of 256, or a wavefront (four rows a workgroup) where V <= 2048, whose rows would
+// leave half of a workgroup or more without a value (16384 x 1024, in place: 39 us with a workgroup a row, 20 with a wavefront).
+constexpr int WAVE_ROW_V = 2048;
+
+// The pairs (max, sum exp) of four chunks of eight logits, joined to a: one running maximum for the 32 values (none with a
+// softcap: cap bounds them). Chunks beyond V hold -inf; i, step: the first chunk's place in the row and the distance of two.
+__device__ __forceinline__ void ms_add4(MS& a, const u32x4* u, int i, int step, int V, float icap, float cap) {
+  if (cap > 0.f) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (i + step * c < V) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a.s += capped_exp(bflo(u[c][k]), icap, cap) + capped_exp(bfhi(u[c][k]), icap, cap);
+      }
+  } else {
+    float mx = a.m, t = 0.f;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) mx = fmaxf(fmaxf(mx, bflo(u[c][k])), bfhi(u[c][k]));
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) t += fexp(bflo(u[c][k]) - mx) + fexp(bfhi(u[c][k]) - mx);
+    a.s = a.s * fexp(a.m - mx) + t;
+    a.m = mx;
+  }
+}
+__device__ __forceinline__ u32x4 logits8(const bf16_t* x, int i, int V) {
+  return i < V ? *(const u32x4*)(x + i) : u32x4{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+}
+// The row's pair from its threads' pairs, in every one of them (TPR = 64) or in the workgroup's first thread (256).
+template <int TPR>
+__device__ __forceinline__ MS ms_row(MS a, float (&rm)[4], float (&rs)[4]) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) a = ms_merge(a, MS{__shfl_xor(a.m, o, 64), __shfl_xor(a.s, o, 64)});
+  if constexpr (TPR == 256) {
+    if ((threadIdx.x & 63) == 0) {
+      rm[threadIdx.x >> 6] = a.m;
+      rs[threadIdx.x >> 6] = a.s;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int i = 1; i < 4; ++i) a = ms_merge(a, MS{rm[i], rs[i]});
+  }
+  return a;
+}
+// d x_v = g (softmax_v - [v == t]) (1 - tanh^2) of eight values from v = i on; 1 - tanh^2 = 4 q (1 - q) with q = 1 / (e^2y + 1)
+__device__ __forceinline__ u32x4 loss_grad8(const u32x4& u, int i, long tt, float g, float l, float icap, float cap) {
+  float d[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float v = k & 1 ? bfhi(u[k >> 1]) : bflo(u[k >> 1]), hot = (i + k == tt) ? 1.0f : 0.0f;
+    if (cap > 0.f) {
+      const float q = tanh_rcp(v * icap);
+      d[k] = g * (fexp((cap - l) - 2.0f * cap * q) - hot) * (4.0f * q * (1.0f - q));
+    } else {
+      d[k] = g * (fexp(v - l) - hot);
+    }
+  }
+  return u32x4{pack2bf(d[0], d[1]), pack2bf(d[2], d[3]), pack2bf(d[4], d[5]), pack2bf(d[6], d[7])};
+}
+
+// loss_row = w * (lse - s_t) with w = row_w[row] (or 1), 0 for a target outside [0, V). Bound by memory: four 16-byte loads a
+// lane in flight. It is also the pass over the LM head's logits where the GEMM leaves it to one.
+template <typename IDX, int TPR>
 __global__ __launch_bounds__(256) void loss_fwd_kernel(const bf16_t* __restrict__ x, const IDX* __restrict__ tg,
                                                       const float* __restrict__ row_w, float* __restrict__ loss,
-                                                      float* __restrict__ lse, int V, float cap) {
+                                                      float* __restrict__ lse, long rows, int V, float cap) {
   __shared__ float rm[4], rs[4];
-  const long row = blockIdx.x;
+  const long row = (long)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  if (TPR < 256 && row >= rows) return;
   const bf16_t* xr = x + row * V;
+  const int t0 = threadIdx.x % TPR;
   const float icap = cap > 0.f ? 1.0f / cap : 0.f;
-  MS a{-1e30f, 0.f};
-  for (int i = threadIdx.x * 8; i < V; i += 256 * 8) {
-    u32x4 u = *(const u32x4*)(xr + i);
-    float v[8];
+  MS a{cap > 0.f ? cap : -1e30f, 0.f};
+  for (int i0 = t0 * 8; i0 < V; i0 += 4 * TPR * 8) {
+    u32x4 u[4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      v[2 * k] = bflo(u[k]);
-      v[2 * k + 1] = bfhi(u[k]);
-    }
-    if (cap > 0.f) {
-      // fixed shift: every s is in [-cap, cap]
-#pragma unroll
-      for (int k = 0; k < 8; ++k) a.s += fexp(cap * tanh_fast(v[k] * icap) - cap);
-      a.m = cap;
-    } else {
-      float mx = a.m;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) mx = fmaxf(mx, v[k]);
-      float sc = fexp(a.m - mx), t = 0.f;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) t += fexp(v[k] - mx);
-      a.s = a.s * sc + t;
-      a.m = mx;
-    }
+    for (int c = 0; c < 4; ++c) u[c] = logits8(xr, i0 + TPR * 8 * c, V);
+    ms_add4(a, u, i0, TPR * 8, V, icap, cap);
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    MS b{__shfl_xor(a.m, o, 64), __shfl_xor(a.s, o, 64)};
-    a = ms_merge(a, b);
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-    rm[wave] = a.m;
-    rs[wave] = a.s;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    MS t{rm[0], rs[0]};
-    for (int i = 1; i < 4; ++i) t = ms_merge(t, MS{rm[i], rs[i]});
-    float l = t.m + logf(t.s);
+  a = ms_row<TPR>(a, rm, rs);
+  if (t0 == 0) {
+    const float l = a.m + logf(a.s);
     lse[row] = l;
-    long tt = (long)tg[row];
+    const long tt = (long)tg[row];
     float out = 0.f;
     if ((unsigned long)tt < (unsigned long)V) {  // a target outside [0, V) is an ignored row, never an address
-      float xt = bf2f(xr[tt]);
-      float st = cap > 0.f ? cap * tanh_fast(xt * icap) : xt;
-      out = (l - st) * (row_w ? row_w[row] : 1.0f);
+      const float xt = bf2f(xr[tt]);
+      out = (l - (cap > 0.f ? cap * tanh_fast(xt * icap) : xt)) * (row_w ? row_w[row] : 1.0f);
     }
     loss[row] = out;
   }
 }
 
-// d x_v = g_row (softmax_v - [v == t]) (1 - tanh^2); g_row = grow[row] (upstream grad x row weight); target < 0 -> 0.
-template <typename IDX>
+// g_row = grow[row] (upstream grad x row weight); a target outside [0, V) -> 0.
+template <typename IDX, int TPR>
 __global__ __launch_bounds__(256) void loss_bwd_kernel(const bf16_t* __restrict__ x, const IDX* __restrict__ tg,
                                                       const float* __restrict__ lse, const float* __restrict__ grow,
-                                                      bf16_t* __restrict__ dx, int V, float cap) {
-  const long row = blockIdx.x;
+                                                      bf16_t* __restrict__ dx, long rows, int V, float cap) {
+  const long row = (long)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  if (TPR < 256 && row >= rows) return;
   const bf16_t* xr = x + row * V;
   bf16_t* dr = dx + row * V;
+  const int t0 = threadIdx.x % TPR;
   const long tt = (long)tg[row];
   const float g = (unsigned long)tt < (unsigned long)V ? grow[row] : 0.f;  // out of range = ignored
   const float l = lse[row];
   const float icap = cap > 0.f ? 1.0f / cap : 0.f;
   // (the next chunk is requested before this chunk's store: a wait for loaded data also waits for every older store)
-  u32x4 unext = {0u, 0u, 0u, 0u};
-  if ((int)threadIdx.x * 8 < V) unext = *(const u32x4*)(xr + threadIdx.x * 8);
-  for (int i = threadIdx.x * 8; i < V; i += 256 * 8) {
+  u32x4 unext = logits8(xr, t0 * 8, V);
+  for (int i = t0 * 8; i < V; i += TPR * 8) {
     const u32x4 u = unext;
-    if (i + 256 * 8 < V) unext = *(const u32x4*)(xr + i + 256 * 8);
-    float v[8], d[8];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      v[2 * k] = bflo(u[k]);
-      v[2 * k + 1] = bfhi(u[k]);
-    }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      float hot = (i + k == tt) ? 1.0f : 0.0f;
-      if (cap > 0.f) {
-        float t = tanh_fast(v[k] * icap);
-        float p = fexp(cap * t - l);
-        d[k] = g * (p - hot) * (1.0f - t * t);
-      } else {
-        d[k] = g * (fexp(v[k] - l) - hot);
-      }
-    }
-    u32x4 o = {pack2bf(d[0], d[1]), pack2bf(d[2], d[3]), pack2bf(d[4], d[5]), pack2bf(d[6], d[7])};
-    *(u32x4*)(dr + i) = o;
+    unext = logits8(xr, i + TPR * 8, V);
+    *(u32x4*)(dr + i) = loss_grad8(u, i, tt, g, l, icap, cap);
   }
 }
 
-// loss_fwd_kernel and loss_bwd_kernel for grow = row_w in ONE pass over the logits: a workgroup keeps its row in registers
-// (NCH chunks of eight values per thread, V <= 2048 NCH), reduces it to lse in the order of loss_fwd_kernel, writes lse and
-// the weighted row loss, and overwrites the row with d x_v = w (softmax_v - [v = t]) (1 - tanh^2): the gradient for an
+// loss_fwd_kernel and loss_bwd_kernel for grow = row_w in ONE pass over the logits: the threads of a row keep it in registers
+// (NCH chunks of eight values per thread, V <= 8 TPR NCH), reduce it to lse in the order of loss_fwd_kernel, write lse and
+// the weighted row loss, and overwrite the row with d x_v = w (softmax_v - [v = t]) (1 - tanh^2): the gradient for an
 // upstream gradient of one, which the caller's two gradient GEMMs scale by the real one. The logits are read once and
 // written once where the two kernels read them twice; values equal theirs bit for bit.
-template <typename IDX, int NCH>
+template <typename IDX, int NCH, int TPR>
 __global__ __launch_bounds__(256) void loss_fwd_bwd_kernel(bf16_t* x, const IDX* __restrict__ tg, const float* __restrict__ row_w,
-                                                          float* __restrict__ loss, float* __restrict__ lse, int V, float cap) {
+                                                          float* __restrict__ loss, float* __restrict__ lse, long rows, int V, float cap) {
   __shared__ float rm[4], rs[4], lsh;
-  const long row = blockIdx.x;
+  const long row = (long)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  if (TPR < 256 && row >= rows) return;
   bf16_t* xr = x + row * V;
+  const int t0 = threadIdx.x % TPR;
   const float icap = cap > 0.f ? 1.0f / cap : 0.f;
   u32x4 u[NCH];
 #pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    const int i = threadIdx.x * 8 + j * 2048;
-    u[j] = i < V ? *(const u32x4*)(xr + i) : u32x4{0u, 0u, 0u, 0u};
-  }
-  MS a{-1e30f, 0.f};
-#pragma unroll
-  for (int j = 0; j < NCH; ++j) {
-    if (threadIdx.x * 8 + j * 2048 < V) {
-      float v[8];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        v[2 * k] = bflo(u[j][k]);
-        v[2 * k + 1] = bfhi(u[j][k]);
-      }
-      if (cap > 0.f) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) a.s += fexp(cap * tanh_fast(v[k] * icap) - cap);
-        a.m = cap;
-      } else {
-        float mx = a.m;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) mx = fmaxf(mx, v[k]);
-        float sc = fexp(a.m - mx), t = 0.f;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) t += fexp(v[k] - mx);
-        a.s = a.s * sc + t;
-        a.m = mx;
-      }
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    MS b{__shfl_xor(a.m, o, 64), __shfl_xor(a.s, o, 64)};
-    a = ms_merge(a, b);
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-    rm[wave] = a.m;
-    rs[wave] = a.s;
-  }
-  __syncthreads();
+  for (int j = 0; j < NCH; ++j) u[j] = logits8(xr, (t0 + j * TPR) * 8, V);
   const long tt = (long)tg[row];
   const bool valid = (unsigned long)tt < (unsigned long)V;  // a target outside [0, V) is an ignored row, never an address
   const float w = valid ? (row_w ? row_w[row] : 1.0f) : 0.f;
-  if (threadIdx.x == 0) {
-    MS t{rm[0], rs[0]};
-    for (int i = 1; i < 4; ++i) t = ms_merge(t, MS{rm[i], rs[i]});
-    const float l = t.m + logf(t.s);
+  const float xt = valid ? bf2f(xr[tt]) : 0.f;              // (read before any thread overwrites the row)
+  MS a{cap > 0.f ? cap : -1e30f, 0.f};
+#pragma unroll
+  for (int j = 0; j < NCH; j += 4)
+    if ((t0 + j * TPR) * 8 < V) ms_add4(a, u + j, (t0 + j * TPR) * 8, TPR * 8, V, icap, cap);
+  a = ms_row<TPR>(a, rm, rs);
+  float l = a.m + logf(a.s);
+  if (t0 == 0) {
     lse[row] = l;
-    float out = 0.f;
-    if (valid) {
-      const float xt = bf2f(xr[tt]);   // (read before any thread overwrites the row: the barrier below)
-      const float st = cap > 0.f ? cap * tanh_fast(xt * icap) : xt;
-      out = (l - st) * w;
-    }
-    loss[row] = out;
-    lsh = l;
+    loss[row] = valid ? (l - (cap > 0.f ? cap * tanh_fast(xt * icap) : xt)) * w : 0.f;
   }
-  __syncthreads();
-  const float l = lsh;
+  if constexpr (TPR == 256) {
+    if (t0 == 0) lsh = l;
+    __syncthreads();
+    l = lsh;
+  }
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    const int i = threadIdx.x * 8 + j * 2048;
-    if (i < V) {
-      float v[8], d[8];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        v[2 * k] = bflo(u[j][k]);
-        v[2 * k + 1] = bfhi(u[j][k]);
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float hot = (i + k == tt) ? 1.0f : 0.0f;
-        if (cap > 0.f) {
-          const float t = tanh_fast(v[k] * icap);
-          const float p = fexp(cap * t - l);
-          d[k] = w * (p - hot) * (1.0f - t * t);
-        } else {
-          d[k] = w * (fexp(v[k] - l) - hot);
-        }
-      }
-      u32x4 o = {pack2bf(d[0], d[1]), pack2bf(d[2], d[3]), pack2bf(d[4], d[5]), pack2bf(d[6], d[7])};
-      *(u32x4*)(xr + i) = o;
-    }
+    const int i = (t0 + j * TPR) * 8;
+    if (i < V) *(u32x4*)(xr + i) = loss_grad8(u[j], i, tt, w, l, icap, cap);
   }
 }
 
@@ -404,13 +368,6 @@ __global__ __launch_bounds__(256) void loss_multi_bwd_kernel(const bf16_t* __res
 }
 
 // ------------------------------------------------------------------------------------ LM head GEMM + lse partials
-// exp(cap tanh(x / cap) - cap) = exp(-2 cap / (exp(2 x / cap) + 1)): two exponentials and a reciprocal, half the instructions
-// of the tanh, its division and the exponential after it.
-__device__ __forceinline__ float capped_exp(float x, float icap, float cap) {
-  const float e = __builtin_amdgcn_exp2f(x * (2.8853900817779268f * icap));
-  return __builtin_amdgcn_exp2f(-2.8853900817779268f * cap * __builtin_amdgcn_rcpf(e + 1.0f));
-}
-
 struct EpiLmHead {
   static constexpr bool kTileEpilogue = true;
   bf16_t* logits;  // [rows][V]
@@ -464,64 +421,6 @@ struct EpiLmHead {
   }
 };
 
-// lse and loss of one row of the logits per workgroup, for the launches whose GEMM leaves them to a pass of their own: four
-// 16-byte loads a lane in flight, one running maximum for the 32 values they bring (none with a softcap, where cap bounds them).
-template <typename IDX>
-__global__ __launch_bounds__(256) void lmhead_rows_kernel(const bf16_t* __restrict__ x, const IDX* __restrict__ tg,
-                                                         const float* __restrict__ row_w, float* __restrict__ loss,
-                                                         float* __restrict__ lse, int V, float cap) {
-  __shared__ float rm[4], rs[4];
-  const long row = blockIdx.x;
-  const bf16_t* xr = x + row * V;
-  const float icap = cap > 0.f ? 1.0f / cap : 0.f;
-  MS a{cap > 0.f ? cap : -1e30f, 0.f};
-  for (int i0 = threadIdx.x * 8; i0 < V; i0 += 4 * 2048) {
-    u32x4 u[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-      u[c] = i0 + 2048 * c < V ? *(const u32x4*)(xr + i0 + 2048 * c) : u32x4{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
-    if (cap > 0.f) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        if (i0 + 2048 * c < V) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) a.s += capped_exp(bflo(u[c][k]), icap, cap) + capped_exp(bfhi(u[c][k]), icap, cap);
-        }
-    } else {
-      float mx = a.m, t = 0.f;
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) mx = fmaxf(fmaxf(mx, bflo(u[c][k])), bfhi(u[c][k]));
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) t += fexp(bflo(u[c][k]) - mx) + fexp(bfhi(u[c][k]) - mx);
-      a.s = a.s * fexp(a.m - mx) + t;
-      a.m = mx;
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) a = ms_merge(a, MS{__shfl_xor(a.m, o, 64), __shfl_xor(a.s, o, 64)});
-  if ((threadIdx.x & 63) == 0) {
-    rm[threadIdx.x >> 6] = a.m;
-    rs[threadIdx.x >> 6] = a.s;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int i = 1; i < 4; ++i) a = ms_merge(a, MS{rm[i], rs[i]});
-    const float l = a.m + logf(a.s);
-    lse[row] = l;
-    const long tt = (long)tg[row];
-    float out = 0.f;
-    if ((unsigned long)tt < (unsigned long)V) {  // a target outside [0, V) is an ignored row, never an address
-      const float xt = bf2f(xr[tt]);
-      out = (l - (cap > 0.f ? cap * tanh_fast(xt * icap) : xt)) * (row_w ? row_w[row] : 1.0f);
-    }
-    loss[row] = out;
-  }
-}
-
 // A workgroup per 64 rows, a lane per row: each wavefront merges a quarter of the row's slab pairs (eight coalesced 512-byte
 // loads in flight), the four quarters meet in LDS, then the target logit is read and lse and the row loss are written.
 template <typename IDX>
@@ -564,6 +463,19 @@ __global__ __launch_bounds__(256) void lmhead_finish_kernel(const float* __restr
 
 }  // namespace
 
+static void launch_loss_fwd(const void* logits, const void* targets, int idx64, const void* row_w, void* loss, void* lse, long rows,
+                            int V, float softcap, hipStream_t s) {
+#define TFB_LF(IDX, TPR)                                                                                                     \
+  hipLaunchKernelGGL((loss_fwd_kernel<IDX, TPR>), dim3((unsigned)((rows + 256 / TPR - 1) / (256 / TPR))), dim3(256), 0, s,    \
+                     (const bf16_t*)logits, (const IDX*)targets, (const float*)row_w, (float*)loss, (float*)lse, rows, V, softcap)
+  if (V <= WAVE_ROW_V) {
+    if (idx64) TFB_LF(long, 64); else TFB_LF(int, 64);
+  } else {
+    if (idx64) TFB_LF(long, 256); else TFB_LF(int, 256);
+  }
+#undef TFB_LF
+}
+
 // logits bf16 [rows][V]; targets int64 (idx64) or int32, negative = ignored; row_w fp32 [rows] or NULL;
 // loss fp32 [rows] (already weighted); lse fp32 [rows]. softcap <= 0 means no softcap.
 extern "C" int tfb_loss_fwd(const void* logits, const void* targets, int idx64, const void* row_w, void* loss, void* lse,
@@ -571,12 +483,7 @@ extern "C" int tfb_loss_fwd(const void* logits, const void* targets, int idx64, 
   if (!logits || !targets || !loss || !lse) return TFB_ERR_ARG;
   if (rows <= 0 || V <= 0 || V % 8) return TFB_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-  if (idx64)
-    hipLaunchKernelGGL(loss_fwd_kernel<long>, dim3((unsigned)rows), dim3(256), 0, s, (const bf16_t*)logits, (const long*)targets,
-                       (const float*)row_w, (float*)loss, (float*)lse, V, softcap);
-  else
-    hipLaunchKernelGGL(loss_fwd_kernel<int>, dim3((unsigned)rows), dim3(256), 0, s, (const bf16_t*)logits, (const int*)targets,
-                       (const float*)row_w, (float*)loss, (float*)lse, V, softcap);
+  launch_loss_fwd(logits, targets, idx64, row_w, loss, lse, rows, V, softcap, s);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
@@ -606,15 +513,19 @@ extern "C" int tfb_loss_fwd_bwd(void* logits, const void* targets, int idx64, co
   if (!logits || !targets || !loss || !lse) return TFB_ERR_ARG;
   if (rows <= 0 || V <= 0 || V % 8 || V > 65536) return TFB_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-#define TFB_LFB(IDX, NCH)                                                                                                  \
-  hipLaunchKernelGGL((loss_fwd_bwd_kernel<IDX, NCH>), dim3((unsigned)rows), dim3(256), 0, s, (bf16_t*)logits,             \
-                     (const IDX*)targets, (const float*)row_w, (float*)loss, (float*)lse, V, softcap)
-  if (V <= 16384) {
-    if (idx64) TFB_LFB(long, 8); else TFB_LFB(int, 8);
+#define TFB_LFB(IDX, NCH, TPR)                                                                                              \
+  hipLaunchKernelGGL((loss_fwd_bwd_kernel<IDX, NCH, TPR>), dim3((unsigned)((rows + 256 / TPR - 1) / (256 / TPR))), dim3(256), 0, s, \
+                     (bf16_t*)logits, (const IDX*)targets, (const float*)row_w, (float*)loss, (float*)lse, rows, V, softcap)
+  if (V <= WAVE_ROW_V) {
+    if (idx64) TFB_LFB(long, 4, 64); else TFB_LFB(int, 4, 64);
+  } else if (V <= 8192) {
+    if (idx64) TFB_LFB(long, 4, 256); else TFB_LFB(int, 4, 256);
+  } else if (V <= 16384) {
+    if (idx64) TFB_LFB(long, 8, 256); else TFB_LFB(int, 8, 256);
   } else if (V <= 32768) {
-    if (idx64) TFB_LFB(long, 16); else TFB_LFB(int, 16);
+    if (idx64) TFB_LFB(long, 16, 256); else TFB_LFB(int, 16, 256);
   } else {
-    if (idx64) TFB_LFB(long, 32); else TFB_LFB(int, 32);
+    if (idx64) TFB_LFB(long, 32, 256); else TFB_LFB(int, 32, 256);
   }
 #undef TFB_LFB
   TFB_LAUNCH_CHECK();
@@ -627,12 +538,15 @@ extern "C" int tfb_loss_bwd(const void* logits, const void* targets, int idx64, 
   if (!logits || !targets || !lse || !grow || !dlogits) return TFB_ERR_ARG;
   if (rows <= 0 || V <= 0 || V % 8) return TFB_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-  if (idx64)
-    hipLaunchKernelGGL(loss_bwd_kernel<long>, dim3((unsigned)rows), dim3(256), 0, s, (const bf16_t*)logits, (const long*)targets,
-                       (const float*)lse, (const float*)grow, (bf16_t*)dlogits, V, softcap);
-  else
-    hipLaunchKernelGGL(loss_bwd_kernel<int>, dim3((unsigned)rows), dim3(256), 0, s, (const bf16_t*)logits, (const int*)targets,
-                       (const float*)lse, (const float*)grow, (bf16_t*)dlogits, V, softcap);
+#define TFB_LB(IDX, TPR)                                                                                                     \
+  hipLaunchKernelGGL((loss_bwd_kernel<IDX, TPR>), dim3((unsigned)((rows + 256 / TPR - 1) / (256 / TPR))), dim3(256), 0, s,    \
+                     (const bf16_t*)logits, (const IDX*)targets, (const float*)lse, (const float*)grow, (bf16_t*)dlogits, rows, V, softcap)
+  if (V <= WAVE_ROW_V) {
+    if (idx64) TFB_LB(long, 64); else TFB_LB(int, 64);
+  } else {
+    if (idx64) TFB_LB(long, 256); else TFB_LB(int, 256);
+  }
+#undef TFB_LB
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
@@ -690,12 +604,7 @@ extern "C" int tfb_lmhead_fwd(const void* x, const void* W, const void* targets,
   // 264 -> 210, 2048 x 32768 x 768 150 -> 118 / 161 -> 121, 32768 x 32768 x 768 2166 -> 2096 / 2292 -> 2047).
   if (gemm_pp_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, V, (int)rows, (long)d * 2, false, EpiStore{logits, (long)V, 0, 0}, s, st)) {
     if (st != TFB_OK) return st;
-    if (idx64)
-      hipLaunchKernelGGL(lmhead_rows_kernel<long>, dim3((unsigned)rows), dim3(256), 0, s, (const bf16_t*)logits, (const long*)targets,
-                         (const float*)row_w, (float*)loss, (float*)lse, V, softcap);
-    else
-      hipLaunchKernelGGL(lmhead_rows_kernel<int>, dim3((unsigned)rows), dim3(256), 0, s, (const bf16_t*)logits, (const int*)targets,
-                         (const float*)row_w, (float*)loss, (float*)lse, V, softcap);
+    launch_loss_fwd(logits, targets, idx64, row_w, loss, lse, rows, V, softcap, s);
     TFB_LAUNCH_CHECK();
     return TFB_OK;
   }
