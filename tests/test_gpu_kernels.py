@@ -1423,3 +1423,46 @@ def test_fp8_mlp_pads_its_rows_inside(ops, dev, rows, dw8):
         gb = torch.autograd.grad(yb, (xb, wf, wp), torch.nn.functional.pad(gy, pad))
         assert ya.shape == x.shape and torch.equal(ya, yb[:rows]) and torch.equal(ga[0], gb[0][:rows])
         assert torch.equal(ga[1], gb[1]) and torch.equal(ga[2], gb[2])
+
+
+@pytest.mark.parametrize("V", [8, 504, 1032, 2048, 2056, 8200])
+@pytest.mark.parametrize("cap", [0.0, 15.0])
+def test_loss_rows_of_a_wavefront_and_of_a_workgroup(ops, dev, V, cap):
+    """The loss kernels around V = 2048, where a row moves from a wavefront to a workgroup, with row counts that leave the last
+    workgroup partly empty: row losses and gradients against float64, the one-pass kernel against the two bit for bit."""
+    g = _g(V)
+    for N in (1, 7):
+        x = (3.0 * torch.randn(N, V, generator=g)).bfloat16()
+        t = torch.randint(0, V, (N,), generator=g)
+        t[0] = V - 1
+        w = torch.rand(N, generator=g)
+        z = x.double().requires_grad_(True)
+        sv = cap * torch.tanh(z / cap) if cap > 0 else z
+        want = torch.nn.functional.cross_entropy(sv, t, reduction="none") * w.double()
+        want.sum().backward()
+        xd, td, wd = x.to(dev), t.to(dev), w.to(dev)
+        rows, lse = ops.loss_fwd(xd, td, cap, wd)
+        d = ops.loss_bwd(xd, td, lse, wd, cap)
+        assert rel_l2(rows, want.detach()) < 1e-5 and rel_l2(d, z.grad) < BF16_TOL
+        y = xd.clone()
+        rows1, lse1 = ops.loss_fwd_bwd(y, td, wd, cap)
+        assert torch.equal(rows, rows1) and torch.equal(lse, lse1) and torch.equal(d, y)
+
+
+@pytest.mark.parametrize("B,T,C", [(3, 2731, 256), (1, 4097, 1536), (9, 911, 264), (5, 1, 768)])
+def test_mix_tail_backward_in_runs_of_rows(ops, dev, B, T, C):
+    """The mixer tail's backward where a group of lanes takes several rows, across sequence ends and with a last run cut short,
+    against float64 on the host."""
+    g = _g(B * T)
+    x, gy, ge = (torch.randn(B, T, C, generator=g).bfloat16() for _ in range(3))
+    lam = torch.tensor([0.3])
+    s1, y, inv = ops.mix_tail_fwd(x.to(dev), lam.to(dev), T, 1e-6)
+    gx, dl = ops.mix_tail_bwd(s1, inv, x.to(dev), lam.to(dev), T, gy.to(dev), ge.to(dev))
+    s, iv = s1.cpu().double().view(B, T, C), inv.cpu().double().view(B, T, 1)
+    gg = (ge.double() + iv * (gy.double() - s * (gy.double() * s).sum(-1, keepdim=True) * iv * iv / C)).bfloat16().double()
+    zero = torch.zeros(B, 1, C, dtype=torch.float64)
+    want = gg + 0.3 * torch.cat([gg[:, 1:], zero], 1)
+    assert rel_l2(gx, want.view_as(gx.cpu())) < BF16_TOL
+    wdl = (gg * torch.cat([zero, x.double()[:, :-1]], 1)).sum()
+    scale = (gg.square().sum() * x.double().square().sum()).sqrt() / (B * T * C) ** 0.5
+    assert abs(dl.item() - wdl.item()) < 2e-2 * scale.item() + 1e-6

@@ -21,16 +21,15 @@ namespace {
 
 __device__ __forceinline__ float fexp(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
 
-// tanh(y) = 1 - 2 / (exp(2 y) + 1), the exponential's overflow giving 1 and its underflow -1; with the hardware reciprocal (1
-// ulp, as the exponential): a correctly rounded division is ten more instructions a value, and made the softcap's pass over
-// the logits run at 2.3 TB/s
-__device__ __forceinline__ float tanh_rcp(float y) { return __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(y * 2.8853900817779268f) + 1.0f); }
-__device__ __forceinline__ float tanh_fast(float y) { return 1.0f - 2.0f * tanh_rcp(y); }
-// exp(cap tanh(x / cap) - cap) = exp(-2 cap / (exp(2 x / cap) + 1)): two exponentials and a reciprocal, half the instructions
-// of the tanh, its division and the exponential after it.
-__device__ __forceinline__ float capped_exp(float x, float icap, float cap) {
-  return __builtin_amdgcn_exp2f(-2.8853900817779268f * cap * tanh_rcp(x * icap));
+// 1 / (exp(2 y) + 1), correctly rounded: a Newton step on the hardware reciprocal gives the bits of an IEEE division for every
+// denominator from 1 to 2^24 (all of them compared on the GPU) at a third of its instructions; beyond, tanh is 1 either way.
+__device__ __forceinline__ float tanh_rcp(float y) {
+  const float d = fminf(__builtin_amdgcn_exp2f(y * 2.8853900817779268f), 0x1p100f) + 1.0f;
+  const float r = __builtin_amdgcn_rcpf(d);
+  return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
 }
+// tanh(y) = 1 - 2 / (exp(2 y) + 1)
+__device__ __forceinline__ float tanh_fast(float y) { return 1.0f - 2.0f * tanh_rcp(y); }
 
 struct MS {
   float m, s;
@@ -78,9 +77,34 @@ __global__ __launch_bounds__(1024) void loss_row_weights_kernel(const IDX* __res
 // leave half of a workgroup or more without a value (16384 x 1024, in place: 39 us with a workgroup a row, 20 with a wavefront).
 constexpr int WAVE_ROW_V = 2048;
 
-// The pairs (max, sum exp) of four chunks of eight logits, joined to a: one running maximum for the 32 values (none with a
-// softcap: cap bounds them). Chunks beyond V hold -inf; i, step: the first chunk's place in the row and the distance of two.
-__device__ __forceinline__ void ms_add4(MS& a, const u32x4* u, int i, int step, int V, float icap, float cap) {
+// The pair (max, sum exp) of eight logits joined to a (with a softcap cap is the maximum: it bounds every value).
+__device__ __forceinline__ void ms_add8(MS& a, const u32x4& u, float icap, float cap) {
+  float v[8];
+  unpack8bf(u, v);
+  if (cap > 0.f) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) a.s += fexp(cap * tanh_fast(v[k] * icap) - cap);
+  } else {
+    float mx = a.m, t = 0.f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) mx = fmaxf(mx, v[k]);
+    const float sc = fexp(a.m - mx);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) t += fexp(v[k] - mx);
+    a.s = a.s * sc + t;
+    a.m = mx;
+  }
+}
+
+// exp(cap tanh(x / cap) - cap) = exp(-2 cap / (exp(2 x / cap) + 1)): two exponentials and a reciprocal, half the instructions
+// of the tanh, its division and the exponential after it. For evaluation, where nothing repeats the gradient's bits.
+__device__ __forceinline__ float capped_exp(float x, float icap, float cap) {
+  const float e = __builtin_amdgcn_exp2f(x * (2.8853900817779268f * icap));
+  return __builtin_amdgcn_exp2f(-2.8853900817779268f * cap * __builtin_amdgcn_rcpf(e + 1.0f));
+}
+// Evaluation: four chunks with one running maximum for their 32 values. Chunks beyond V hold -inf; i, step: the first chunk's
+// place in the row and the distance of two.
+__device__ __forceinline__ void ms_add32(MS& a, const u32x4* u, int i, int step, int V, float icap, float cap) {
   if (cap > 0.f) {
 #pragma unroll
     for (int c = 0; c < 4; ++c)
@@ -105,31 +129,47 @@ __device__ __forceinline__ void ms_add4(MS& a, const u32x4* u, int i, int step, 
 __device__ __forceinline__ u32x4 logits8(const bf16_t* x, int i, int V) {
   return i < V ? *(const u32x4*)(x + i) : u32x4{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
 }
-// The row's pair from its threads' pairs, in every one of them (TPR = 64) or in the workgroup's first thread (256).
-template <int TPR>
-__device__ __forceinline__ MS ms_row(MS a, float (&rm)[4], float (&rs)[4]) {
+__device__ __forceinline__ MS ms_wave(MS a) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) a = ms_merge(a, MS{__shfl_xor(a.m, o, 64), __shfl_xor(a.s, o, 64)});
-  if constexpr (TPR == 256) {
-    if ((threadIdx.x & 63) == 0) {
-      rm[threadIdx.x >> 6] = a.m;
-      rs[threadIdx.x >> 6] = a.s;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0)
-      for (int i = 1; i < 4; ++i) a = ms_merge(a, MS{rm[i], rs[i]});
+  return a;
+}
+// A workgroup's row: the pair of all, in its first thread.
+__device__ __forceinline__ MS ms_group(MS a, float (&rm)[4], float (&rs)[4]) {
+  a = ms_wave(a);
+  if ((threadIdx.x & 63) == 0) {
+    rm[threadIdx.x >> 6] = a.m;
+    rs[threadIdx.x >> 6] = a.s;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int i = 1; i < 4; ++i) a = ms_merge(a, MS{rm[i], rs[i]});
+  return a;
+}
+// A wavefront's row of at most four chunks a lane, in all lanes: every chunk is what one wavefront of a workgroup would hold, and
+// they are joined in that order, so the row's lse has the same bits whichever way it is taken.
+__device__ __forceinline__ MS ms_wave_row(const u32x4 (&u)[4], int t0, int V, float icap, float cap) {
+  const MS none{cap > 0.f ? cap : -1e30f, 0.f};
+  MS a = none;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    if (c && 512 * c >= V) break;   // (a chunk that no lane has would change nothing)
+    MS b = none;
+    if ((t0 + 64 * c) * 8 < V) ms_add8(b, u[c], icap, cap);
+    b = ms_wave(b);
+    a = c ? ms_merge(a, b) : b;
   }
   return a;
 }
-// d x_v = g (softmax_v - [v == t]) (1 - tanh^2) of eight values from v = i on; 1 - tanh^2 = 4 q (1 - q) with q = 1 / (e^2y + 1)
+// d x_v = g (softmax_v - [v == t]) (1 - tanh^2) of eight values from v = i on
 __device__ __forceinline__ u32x4 loss_grad8(const u32x4& u, int i, long tt, float g, float l, float icap, float cap) {
   float d[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const float v = k & 1 ? bfhi(u[k >> 1]) : bflo(u[k >> 1]), hot = (i + k == tt) ? 1.0f : 0.0f;
     if (cap > 0.f) {
-      const float q = tanh_rcp(v * icap);
-      d[k] = g * (fexp((cap - l) - 2.0f * cap * q) - hot) * (4.0f * q * (1.0f - q));
+      const float t = tanh_fast(v * icap);
+      d[k] = g * (fexp(cap * t - l) - hot) * (1.0f - t * t);
     } else {
       d[k] = g * (fexp(v - l) - hot);
     }
@@ -138,8 +178,8 @@ __device__ __forceinline__ u32x4 loss_grad8(const u32x4& u, int i, long tt, floa
 }
 
 // loss_row = w * (lse - s_t) with w = row_w[row] (or 1), 0 for a target outside [0, V). Bound by memory: four 16-byte loads a
-// lane in flight. It is also the pass over the LM head's logits where the GEMM leaves it to one.
-template <typename IDX, int TPR>
+// lane in flight. EVAL: the pass over the LM head's logits where the GEMM leaves it to one.
+template <typename IDX, int TPR, bool EVAL>
 __global__ __launch_bounds__(256) void loss_fwd_kernel(const bf16_t* __restrict__ x, const IDX* __restrict__ tg,
                                                       const float* __restrict__ row_w, float* __restrict__ loss,
                                                       float* __restrict__ lse, long rows, int V, float cap) {
@@ -150,13 +190,22 @@ __global__ __launch_bounds__(256) void loss_fwd_kernel(const bf16_t* __restrict_
   const int t0 = threadIdx.x % TPR;
   const float icap = cap > 0.f ? 1.0f / cap : 0.f;
   MS a{cap > 0.f ? cap : -1e30f, 0.f};
-  for (int i0 = t0 * 8; i0 < V; i0 += 4 * TPR * 8) {
+  for (int i0 = t0 * 8; i0 < V || (TPR == 64 && i0 == t0 * 8); i0 += 4 * TPR * 8) {   // (a wavefront's row is one turn of all its lanes)
     u32x4 u[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) u[c] = logits8(xr, i0 + TPR * 8 * c, V);
-    ms_add4(a, u, i0, TPR * 8, V, icap, cap);
+    if constexpr (EVAL) {
+      ms_add32(a, u, i0, TPR * 8, V, icap, cap);
+    } else if constexpr (TPR == 64) {
+      a = ms_wave_row(u, t0, V, icap, cap);
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (i0 + TPR * 8 * c < V) ms_add8(a, u[c], icap, cap);
+    }
   }
-  a = ms_row<TPR>(a, rm, rs);
+  if constexpr (TPR == 256) a = ms_group(a, rm, rs);
+  else if constexpr (EVAL) a = ms_wave(a);
   if (t0 == 0) {
     const float l = a.m + logf(a.s);
     lse[row] = l;
@@ -215,10 +264,14 @@ __global__ __launch_bounds__(256) void loss_fwd_bwd_kernel(bf16_t* x, const IDX*
   const float w = valid ? (row_w ? row_w[row] : 1.0f) : 0.f;
   const float xt = valid ? bf2f(xr[tt]) : 0.f;              // (read before any thread overwrites the row)
   MS a{cap > 0.f ? cap : -1e30f, 0.f};
+  if constexpr (TPR == 64) {
+    a = ms_wave_row(u, t0, V, icap, cap);
+  } else {
 #pragma unroll
-  for (int j = 0; j < NCH; j += 4)
-    if ((t0 + j * TPR) * 8 < V) ms_add4(a, u + j, (t0 + j * TPR) * 8, TPR * 8, V, icap, cap);
-  a = ms_row<TPR>(a, rm, rs);
+    for (int j = 0; j < NCH; ++j)
+      if ((t0 + j * TPR) * 8 < V) ms_add8(a, u[j], icap, cap);
+    a = ms_group(a, rm, rs);
+  }
   float l = a.m + logf(a.s);
   if (t0 == 0) {
     lse[row] = l;
@@ -463,10 +516,11 @@ __global__ __launch_bounds__(256) void lmhead_finish_kernel(const float* __restr
 
 }  // namespace
 
+template <bool EVAL>
 static void launch_loss_fwd(const void* logits, const void* targets, int idx64, const void* row_w, void* loss, void* lse, long rows,
                             int V, float softcap, hipStream_t s) {
 #define TFB_LF(IDX, TPR)                                                                                                     \
-  hipLaunchKernelGGL((loss_fwd_kernel<IDX, TPR>), dim3((unsigned)((rows + 256 / TPR - 1) / (256 / TPR))), dim3(256), 0, s,    \
+  hipLaunchKernelGGL((loss_fwd_kernel<IDX, TPR, EVAL>), dim3((unsigned)((rows + 256 / TPR - 1) / (256 / TPR))), dim3(256), 0, s,    \
                      (const bf16_t*)logits, (const IDX*)targets, (const float*)row_w, (float*)loss, (float*)lse, rows, V, softcap)
   if (V <= WAVE_ROW_V) {
     if (idx64) TFB_LF(long, 64); else TFB_LF(int, 64);
@@ -483,7 +537,7 @@ extern "C" int tfb_loss_fwd(const void* logits, const void* targets, int idx64, 
   if (!logits || !targets || !loss || !lse) return TFB_ERR_ARG;
   if (rows <= 0 || V <= 0 || V % 8) return TFB_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-  launch_loss_fwd(logits, targets, idx64, row_w, loss, lse, rows, V, softcap, s);
+  launch_loss_fwd<false>(logits, targets, idx64, row_w, loss, lse, rows, V, softcap, s);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
@@ -604,7 +658,7 @@ extern "C" int tfb_lmhead_fwd(const void* x, const void* W, const void* targets,
   // 264 -> 210, 2048 x 32768 x 768 150 -> 118 / 161 -> 121, 32768 x 32768 x 768 2166 -> 2096 / 2292 -> 2047).
   if (gemm_pp_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, V, (int)rows, (long)d * 2, false, EpiStore{logits, (long)V, 0, 0}, s, st)) {
     if (st != TFB_OK) return st;
-    launch_loss_fwd(logits, targets, idx64, row_w, loss, lse, rows, V, softcap, s);
+    launch_loss_fwd<true>(logits, targets, idx64, row_w, loss, lse, rows, V, softcap, s);
     TFB_LAUNCH_CHECK();
     return TFB_OK;
   }
