@@ -490,6 +490,10 @@ int tfb_moe_backward_scales_rowmax(const void* rowmax, const void* seg, const vo
 /* out8 = fp8(x * rows[expert of the row's tile][col]); fmt 0 e4m3, 1 e5m2; padding tiles give zero bytes. */
 int tfb_moe_quant(const void* x, const void* tile_expert, const void* rows, int col, int fmt, void* out8, long rmax, int d,
                   void* stream);
+/* The e5m2 bytes of dys = bf16(bf16(gate) dout[tok]) at rows[expert][col], padding rows zero: tfb_moe_quant of what
+ * tfb_moe_combine_bwd_rowmax writes to dys, byte for byte; that call's dys may then be NULL. */
+int tfb_moe_quant_dout(const void* dout, const void* tok, const void* ksel, const void* gate, const void* tile_expert,
+                       const void* rows, int col, void* out8, long rmax, int d, int topk, void* stream);
 
 /* ---- Muon: Newton-Schulz ("Polar Express") orthogonalisation of a stack of gradient matrices -------------------------
  * Per matrix, held tall X [M][N] (M >= N): X0 = bf16(bf16(g) / d), then five times G = bf16(X^T X),

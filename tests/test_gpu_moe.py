@@ -490,3 +490,31 @@ def test_moe_layer_with_capacity_forward_backward(dev, experts):
     both = (info["slot"] < 0).all(1).reshape(b, t)
     if bool(both.any()):
         assert float(out.detach().cpu()[both].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("N", [1, 1024, 1025, 4096, 4097])
+@pytest.mark.parametrize("topk,E", [(2, 8), (1, 16), (2, 3)])
+def test_slot_tables_in_one_workgroup_and_in_four_launches(dev, N, topk, E):
+    """The slot tables on both sides of every size at which another kernel makes them, an expert without tokens among them:
+    a stable partition of the assignments by expert, segments padded to 128 rows, -1 in every row that nothing takes."""
+    from trainium_frontier_them_bones_amd import ops
+    g = torch.Generator().manual_seed(N + E)
+    idx = torch.stack([torch.randperm(E - 1, generator=g)[:topk] for _ in range(N)]).to(torch.int32)
+    tab = ops.moe_tables(idx.to(dev), E)
+    flat = idx.reshape(-1).long()
+    cnt = torch.bincount(flat, minlength=E)
+    seg = torch.cat([torch.zeros(1, dtype=torch.long), ((cnt + 127) // 128 * 128).cumsum(0)])
+    assert torch.equal(tab["cnt"].cpu().long(), cnt) and torch.equal(tab["seg"].cpu().long(), seg)
+    order = torch.argsort(flat, stable=True)
+    rank = torch.empty_like(flat)
+    rank[order] = torch.arange(len(flat)) - (cnt.cumsum(0) - cnt)[flat[order]]
+    slot = seg[flat] + rank
+    assert torch.equal(tab["slot"].cpu().long().reshape(-1), slot)
+    rmax = tab["tok"].numel()
+    tok = torch.full((rmax,), -1, dtype=torch.long)
+    tok[slot] = torch.arange(N).repeat_interleave(topk)
+    assert torch.equal(tab["tok"].cpu().long(), tok)
+    assert torch.equal(tab["ksel"].cpu().long()[slot], torch.arange(topk).repeat(N))
+    tiles = torch.arange(rmax // 128) * 128
+    want = torch.bucketize(tiles, seg[1:], right=True)
+    assert torch.equal(tab["tile_expert"].cpu().long(), torch.where(tiles < seg[E], want, torch.full_like(want, -1)))

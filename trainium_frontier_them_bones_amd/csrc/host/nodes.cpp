@@ -785,12 +785,12 @@ struct Moe : Function<Moe> {
       pybind11::gil_scoped_acquire gil;
       a = attrs(s.state.o);
     }
-    CombineGrad c = moe_combine_bwd(gout, ys, s.tab, gate, s.state.o != nullptr);
+    CombineGrad c = moe_combine_bwd(gout, ys, s.tab, gate, s.state.o != nullptr, !a.dw_fp8);
     Tensor rows_b;
     MlpBwd m;
     if (s.state.o) {   // the experts' amax(dys) rides the kernel that writes dys
       rows_b = moe_backward_scales_rowmax(c.rowmax, a.rows, s.tab, ys.size(1));
-      m = a.dw_fp8 ? moe_mlp8_bwd_q(c.dys, r, a.w8, rows_b, s.tab, a.limit) : moe_mlp8_bwd(c.dys, r, a.w8, rows_b, s.tab);
+      m = a.dw_fp8 ? moe_mlp8_bwd_q(moe_quant_dout(gout, gate, rows_b, s.tab), r, a.w8, rows_b, s.tab, a.limit) : moe_mlp8_bwd(c.dys, r, a.w8, rows_b, s.tab);
     } else {
       m = moe_mlp_bwd(c.dys, r, bf(w_fc), bf(w_proj), s.tab);
     }

@@ -554,10 +554,10 @@ Tensor moe_combine(const Tensor& ys, const MoeTab& tab, const Tensor& gate, at::
   return out;
 }
 
-CombineGrad moe_combine_bwd(const Tensor& dout, const Tensor& ys, const MoeTab& tab, const Tensor& gate, bool want_rowmax) {
+CombineGrad moe_combine_bwd(const Tensor& dout, const Tensor& ys, const MoeTab& tab, const Tensor& gate, bool want_rowmax, bool want_dys) {
   chk(dout), chk(ys), chk(gate, F32);
   const int64_t rmax = ys.size(0), d = ys.size(1);
-  CombineGrad o{make_like(ys), make_like(gate), {}};
+  CombineGrad o{want_dys ? make_like(ys) : Tensor(), make_like(gate), {}};
   // the kernel writes the gate gradient of every assignment that holds a row; a skipped one's is zero
   if (tab.capped) fill_f32(o.dgate, 0.0);
   if (want_rowmax) {
@@ -585,6 +585,15 @@ static Tensor moe_quant_dy(const Tensor& x, const Tensor& rows, const MoeTab& ta
   return out;
 }
 
+Tensor moe_quant_dout(const Tensor& dout, const Tensor& gate, const Tensor& rows, const MoeTab& tab) {
+  chk(dout), chk(gate, F32), chk(rows, F32);
+  const int64_t d = dout.size(-1);
+  Tensor out = make({tab.rmax, d}, U8, dout);
+  TFB_CALL(tfb_moe_quant_dout, ptr(dout), ptr(tab.tok), ptr(tab.ksel), ptr(gate), ptr(tab.tile_expert), ptr(rows), 5, ptr(out), tab.rmax, d,
+           gate.size(1), stream());
+  return out;
+}
+
 MlpBwd moe_mlp8_bwd(const Tensor& dys, const Tensor& r, const Tensor& w8, const Tensor& rows, const MoeTab& tab) {
   chk(dys), chk(r), chk(w8, U8);
   const int64_t rmax = dys.size(0), d = dys.size(1), F = r.size(1);
@@ -596,12 +605,12 @@ MlpBwd moe_mlp8_bwd(const Tensor& dys, const Tensor& r, const Tensor& w8, const 
   return o;
 }
 
-MlpBwd moe_mlp8_bwd_q(const Tensor& dys, const Tensor& r, const Tensor& w8, const Tensor& rows, const MoeTab& tab, double limit) {
-  chk(dys), chk(r), chk(w8, U8);
-  const int64_t rmax = dys.size(0), d = dys.size(1), F = r.size(1);
+MlpBwd moe_mlp8_bwd_q(const Tensor& dy8, const Tensor& r, const Tensor& w8, const Tensor& rows, const MoeTab& tab, double limit) {
+  chk(dy8, U8), chk(r), chk(w8, U8);
+  const int64_t rmax = dy8.size(0), d = dy8.size(1), F = r.size(1);
   MlpBwd o;
-  o.dy8 = moe_quant_dy(dys, rows, tab);
-  o.dx = make({rmax, d}, BF16, dys), o.dp8 = make({rmax, F}, U8, dys), o.hq8 = make({rmax, F}, U8, dys);
+  o.dy8 = dy8;
+  o.dx = make({rmax, d}, BF16, r), o.dp8 = make({rmax, F}, U8, r), o.hq8 = make({rmax, F}, U8, r);
   TFB_CALL(tfb_moe_mlp8_bwd_q, ptr(o.dy8), ptr(r), ptr(w8), ptr(rows), ptr(tab.tile_expert), ptr(o.dx), nullptr, ptr(o.dp8), ptr(o.hq8), limit,
            rmax, d, F, stream());
   return o;

@@ -110,10 +110,12 @@ std::tuple<Tensor, Tensor> moe_mlp8_fwd(const Tensor& xs8, const Tensor& w8, con
 std::tuple<Tensor, Tensor> moe_mlp_fwd(const Tensor& xs, const Tensor& w_fc, const Tensor& w_proj, const MoeTab& tab);
 Tensor moe_combine(const Tensor& ys, const MoeTab& tab, const Tensor& gate, at::IntArrayRef out_shape);
 struct CombineGrad { Tensor dys, dgate, rowmax; };
-CombineGrad moe_combine_bwd(const Tensor& dout, const Tensor& ys, const MoeTab& tab, const Tensor& gate, bool want_rowmax);
+// want_dys false (with want_rowmax): dys is left out, moe_quant_dout makes its bytes
+CombineGrad moe_combine_bwd(const Tensor& dout, const Tensor& ys, const MoeTab& tab, const Tensor& gate, bool want_rowmax, bool want_dys = true);
+Tensor moe_quant_dout(const Tensor& dout, const Tensor& gate, const Tensor& rows, const MoeTab& tab);
 Tensor moe_backward_scales_rowmax(const Tensor& rowmax, const Tensor& rows, const MoeTab& tab, int64_t d);
 MlpBwd moe_mlp8_bwd(const Tensor& dys, const Tensor& r, const Tensor& w8, const Tensor& rows, const MoeTab& tab);
-MlpBwd moe_mlp8_bwd_q(const Tensor& dys, const Tensor& r, const Tensor& w8, const Tensor& rows, const MoeTab& tab, double limit);
+MlpBwd moe_mlp8_bwd_q(const Tensor& dy8, const Tensor& r, const Tensor& w8, const Tensor& rows, const MoeTab& tab, double limit);
 MlpBwd moe_mlp_bwd(const Tensor& dys, const Tensor& r, const Tensor& w_fc, const Tensor& w_proj, const MoeTab& tab);
 void moe_dw8(const Tensor& xs8, const Tensor& dp8, const Tensor& hq8, const Tensor& dy8, const Tensor& rows, double x_scale,
              const MoeTab& tab, Tensor& dw_fc, Tensor& dw_proj, int64_t E, bool accumulate, at::ScalarType out_dtype);

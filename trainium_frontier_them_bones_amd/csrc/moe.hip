@@ -434,6 +434,98 @@ __global__ __launch_bounds__(256) void moe_place_kernel(const int* __restrict__ 
   }
 }
 
+// All of the above in one workgroup of sixteen wavefronts, for N <= 1024 PER tokens: wavefront v holds the assignments of the
+// 64-token groups v, v + 16, .. in registers from the count to the placing, the counts meet in LDS. Bound by its own chain of
+// barriers and, with more tokens, by the ballots: 4.8 us at 512 tokens where fill, count, scan and place took 17, and three
+// launches less, but 37 for 20 us at 16384. So up to 4096 tokens; beyond, the four launches, which use more than one CU.
+template <int PER>
+__global__ __launch_bounds__(1024) void moe_tables_kernel(const int* __restrict__ idx, int* __restrict__ cnt, int* __restrict__ seg,
+                                                         int* __restrict__ tile_expert, int* __restrict__ slot, int* __restrict__ tok,
+                                                         int* __restrict__ ksel, long N, int E, int topk, long rmax) {
+  __shared__ int s_off[16 * PER * MAXE], s_seg[MAXE + 1], s_cnt[MAXE];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int a0[PER], a1[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const long n = (long)(j * 16 + wave) * 64 + lane;
+    a0[j] = a1[j] = -1;
+    if (n < N) {
+      a0[j] = idx[n * topk];
+      if (topk == 2) a1[j] = idx[n * 2 + 1];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    for (int e = 0; e < E; ++e) {
+      const int c = __popcll(__ballot(a0[j] == e)) + __popcll(__ballot(a1[j] == e));
+      if (lane == 0) s_off[(j * 16 + wave) * E + e] = c;
+    }
+  __syncthreads();
+  if (wave < E) {   // the groups' counts of expert `wave` become their offsets in its segment: PER / 4 groups a lane
+    constexpr int RUN = (16 * PER + 63) / 64;
+    int c[RUN], tot = 0;
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) {
+      c[i] = lane * RUN + i < 16 * PER ? s_off[(lane * RUN + i) * E + wave] : 0;
+      tot += c[i];
+    }
+    int inc = tot;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(inc, o);
+      if (lane >= o) inc += t;
+    }
+    int run = inc - tot;
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) {
+      if (lane * RUN + i < 16 * PER) s_off[(lane * RUN + i) * E + wave] = run;
+      run += c[i];
+    }
+    if (lane == 63) cnt[wave] = s_cnt[wave] = inc;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int off = 0;
+    for (int e = 0; e < E; ++e) {
+      s_seg[e] = seg[e] = off;
+      off += (s_cnt[e] + 127) / 128 * 128;
+    }
+    s_seg[E] = seg[E] = off;
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < rmax / 128; t += 1024) {
+    int ex = -1;
+    for (int e = 0; e < E; ++e)
+      if (t * 128 >= s_seg[e] && t * 128 < s_seg[e + 1]) ex = e;
+    tile_expert[t] = ex;
+  }
+  if (wave < E)   // the rows that no assignment takes
+    for (int r = s_seg[wave] + s_cnt[wave] + lane; r < s_seg[wave + 1]; r += 64) tok[r] = -1;
+  for (long r = s_seg[E] + threadIdx.x; r < rmax; r += 1024) tok[r] = -1;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    int r0 = 0, r1 = 0;
+    for (int e = 0; e < E; ++e) {
+      const unsigned long long b0 = __ballot(a0[j] == e), b1 = __ballot(a1[j] == e);
+      int before = s_seg[e] + s_off[(j * 16 + wave) * E + e];
+      before = __builtin_amdgcn_mbcnt_hi((unsigned)(b0 >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b0, before));
+      before = __builtin_amdgcn_mbcnt_hi((unsigned)(b1 >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)b1, before));
+      if (a0[j] == e) r0 = before;
+      if (a1[j] == e) r1 = before;
+    }
+    const long n = (long)(j * 16 + wave) * 64 + lane;
+    if (n < N) {
+      slot[n * topk] = r0;
+      tok[r0] = (int)n;
+      ksel[r0] = 0;
+      if (topk == 2) {
+        slot[n * 2 + 1] = r1;
+        tok[r1] = (int)n;
+        ksel[r1] = 1;
+      }
+    }
+  }
+}
+
 __global__ void fill_i32_kernel(int* __restrict__ p, int val, long n) {
   for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) p[i] = val;
 }
@@ -491,7 +583,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16_t* __restri
 
 // One wavefront per slot row: dys[row] = bf16(bf16(g_k) dout[tok]); dgate[tok][k] = bf16(sum_d dout[tok] ys[row]).
 // ROWMAX: rowmax[row] = max |dys[row]| of the rounded values (0 for a padding row), from which the experts' backward scales
-// are taken without another pass over dys.
+// are taken without another pass over dys. dys may be left out then: where only its e5m2 bytes are read,
+// moe_quant_dout_kernel makes them from dout, half as many bytes as dys and mostly still in the caches.
 template <bool ROWMAX>
 __global__ __launch_bounds__(256) void moe_combine_bwd_kernel(const bf16_t* __restrict__ dout, const bf16_t* __restrict__ ys,
                                                              const int* __restrict__ tok, const int* __restrict__ ksel,
@@ -500,13 +593,13 @@ __global__ __launch_bounds__(256) void moe_combine_bwd_kernel(const bf16_t* __re
                                                              int d, int topk) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (long row = (long)blockIdx.x * 4 + wave; row < rmax; row += (long)gridDim.x * 4) {
-    const int t = tok[row];
+    const int t = tok[row], k = ksel[row];   // (a padding row's choice is not read)
     if (t < 0) {
-      for (int c = lane * 8; c < d; c += 512) *(u32x4*)(dys + row * d + c) = u32x4{0, 0, 0, 0};
+      if (dys)
+        for (int c = lane * 8; c < d; c += 512) *(u32x4*)(dys + row * d + c) = u32x4{0, 0, 0, 0};
       if (ROWMAX && lane == 0) rowmax[row] = 0.f;
       continue;
     }
-    const int k = ksel[row];
     const float g = round_bf(gate[(long)t * topk + k]);
     float dot = 0.f, m = 0.f;
     for (int c = lane * 8; c < d; c += 512) {
@@ -517,7 +610,7 @@ __global__ __launch_bounds__(256) void moe_combine_bwd_kernel(const bf16_t* __re
       for (int j = 0; j < 8; ++j) dot += go[j] * y[j];
       const u32x4 u = {pack2bf(g * go[0], g * go[1]), pack2bf(g * go[2], g * go[3]), pack2bf(g * go[4], g * go[5]),
                        pack2bf(g * go[6], g * go[7])};
-      *(u32x4*)(dys + row * d + c) = u;
+      if (dys) *(u32x4*)(dys + row * d + c) = u;
       if (ROWMAX) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) m = fmaxf(m, fmaxf(fabsf(bflo(u[j])), fabsf(bfhi(u[j]))));
@@ -964,6 +1057,39 @@ __global__ __launch_bounds__(256) void moe_quant_kernel(const bf16_t* __restrict
   }
 }
 
+// out8[row] = e5m2(dys[row] * rows[expert of row][col]) with dys[row] = bf16(bf16(g_k) dout[tok]) made here: the bytes of
+// moe_quant_kernel on the dys of moe_combine_bwd_kernel, which is then never written. One wavefront per row.
+// 32768 x 1024: the two kernels 33 + 19 us -> 24 + 20.
+__global__ __launch_bounds__(256) void moe_quant_dout_kernel(const bf16_t* __restrict__ dout, const int* __restrict__ tok,
+                                                            const int* __restrict__ ksel, const float* __restrict__ gate,
+                                                            const int* __restrict__ tile_expert, const float* __restrict__ rows,
+                                                            int col, uint8_t* __restrict__ out, long rmax, int d, int topk) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (long row = (long)blockIdx.x * 4 + wave; row < rmax; row += (long)gridDim.x * 4) {
+    const int t = tok[row], k = ksel[row], e = tile_expert[row >> 7];   // (one round trip for the three, one for what they name)
+    float g = 0.f, s = 0.f;
+    u32x4 u = {0u, 0u, 0u, 0u};
+    if (t >= 0) {
+      if (lane * 8 < d) u = *(const u32x4*)(dout + (long)t * d + lane * 8);
+      g = round_bf(gate[(long)t * topk + k]);
+      s = rows[e * 16 + col];
+    }
+    for (int c = lane * 8; c < d; c += 512) {
+      u32x2 o = {0, 0};
+      if (t >= 0) {
+        float v[8];
+        unpack8bf(u, v);
+        if (c + 512 < d) u = *(const u32x4*)(dout + (long)t * d + c + 512);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = round_bf(g * v[j]) * s;
+        o.x = cvt4_fp8<TFB_FMT_E5M2>(v[0], v[1], v[2], v[3]);
+        o.y = cvt4_fp8<TFB_FMT_E5M2>(v[4], v[5], v[6], v[7]);
+      }
+      *(u32x2*)(out + row * d + c) = o;
+    }
+  }
+}
+
 inline int nblocks(long n, int cap = 8192) {
   long b = (n + 255) / 256;
   return (int)(b < 1 ? 1 : (b < cap ? b : cap));
@@ -1003,6 +1129,16 @@ extern "C" int tfb_moe_tables(const void* idx, void* cnt, void* seg, void* tile_
   if (N <= 0 || E < 2 || E > MAXE || (topk != 1 && topk != 2) || rmax % 128 || rmax < tfb_moe_max_rows(N, E, topk))
     return TFB_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
+  if (N <= 4096) {
+#define TFB_MT(PER)                                                                                                       \
+  hipLaunchKernelGGL(moe_tables_kernel<PER>, dim3(1), dim3(1024), 0, s, (const int*)idx, (int*)cnt, (int*)seg,            \
+                     (int*)tile_expert, (int*)slot, (int*)tok, (int*)ksel, N, E, topk, rmax)
+    if (N <= 1024) TFB_MT(1);
+    else TFB_MT(4);
+#undef TFB_MT
+    TFB_LAUNCH_CHECK();
+    return TFB_OK;
+  }
   const int nwaves = (int)((N + 63) / 64);
   const int nb = (nwaves + 3) / 4;
   hipLaunchKernelGGL(fill_i32_kernel, dim3(nblocks(rmax)), dim3(256), 0, s, (int*)tok, -1, rmax);
@@ -1091,7 +1227,7 @@ extern "C" int tfb_moe_combine_bwd(const void* dout, const void* ys, const void*
 // tfb_moe_backward_scales_rowmax: the experts' backward scales then cost no pass of their own over dys.
 extern "C" int tfb_moe_combine_bwd_rowmax(const void* dout, const void* ys, const void* tok, const void* ksel, const void* gate,
                                           void* dys, void* dgate, void* rowmax, long rmax, int d, int topk, void* stream) {
-  if (!dout || !ys || !tok || !ksel || !gate || !dys || !dgate || !rowmax) return TFB_ERR_ARG;
+  if (!dout || !ys || !tok || !ksel || !gate || !dgate || !rowmax) return TFB_ERR_ARG;   // dys may be NULL (tfb_moe_quant_dout)
   if (rmax <= 0 || d <= 0 || d % 8 || (topk != 1 && topk != 2)) return TFB_ERR_SHAPE;
   hipLaunchKernelGGL(moe_combine_bwd_kernel<true>, dim3(nblocks(rmax * 64)), dim3(256), 0, (hipStream_t)stream,
                      (const bf16_t*)dout, (const bf16_t*)ys, (const int*)tok, (const int*)ksel, (const float*)gate, (bf16_t*)dys,
@@ -1239,6 +1375,19 @@ extern "C" int tfb_moe_backward_scales_rowmax(const void* rowmax, const void* se
   if (d <= 0 || d % 8 || E < 1 || E > MAXE) return TFB_ERR_SHAPE;
   hipLaunchKernelGGL(moe_backward_scales_rowmax_kernel, dim3(E), dim3(256), 0, (hipStream_t)stream, (const float*)rowmax,
                      (const int*)seg, (const float*)rows_in, (float*)rows_out, (float)(36.16 * (double)d));
+  TFB_LAUNCH_CHECK();
+  return TFB_OK;
+}
+
+// out8 [rmax][d] = e5m2(dys * rows[expert][col]) with dys = bf16(bf16(gate) dout[tok]), padding rows zero: tfb_moe_quant of the
+// dys that tfb_moe_combine_bwd_rowmax writes, byte for byte, without it.
+extern "C" int tfb_moe_quant_dout(const void* dout, const void* tok, const void* ksel, const void* gate, const void* tile_expert,
+                                  const void* rows, int col, void* out8, long rmax, int d, int topk, void* stream) {
+  if (!dout || !tok || !ksel || !gate || !tile_expert || !rows || !out8) return TFB_ERR_ARG;
+  if (rmax <= 0 || rmax % 128 || d <= 0 || d % 8 || col < 0 || col >= 16 || (topk != 1 && topk != 2)) return TFB_ERR_SHAPE;
+  hipLaunchKernelGGL(moe_quant_dout_kernel, dim3(nblocks(rmax * 64)), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)dout,
+                     (const int*)tok, (const int*)ksel, (const float*)gate, (const int*)tile_expert, (const float*)rows, col,
+                     (uint8_t*)out8, rmax, d, topk);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
