@@ -57,3 +57,28 @@ def test_a_nan_activation_reaches_the_loss_head(dev, N, V, cap):
     with torch.no_grad():
         ev = A.LmHeadLossFn.apply(x, W, t, cap, "mean")
     assert bool(loss.isnan()) and bool(ev.isnan()) and bool(gw.isnan().any())
+
+
+@pytest.mark.parametrize("cap", [7.0, 15.0, 30.0])
+@pytest.mark.parametrize("std", [0.5, 2.0])
+@pytest.mark.parametrize("N,V", [(128, 8192), (9600, 8192)])
+def test_lse_of_evaluation_is_as_exact_as_that_of_training(dev, N, V, std, cap):
+    """The log-sum-exp that evaluation takes in its GEMM's epilogue (first size) and in a pass over the logits (second) has no
+    larger error against float64, on the logits it returned, than the training kernels' with their exact tanh: in the mean
+    over the rows, where a bias of the terms stays and roundings cancel, and in the root mean square. The allowance of a
+    tenth of an ulp of lse (2^-20 to 2^-19 here) is what the sums' different order and 128 rows leave of chance."""
+    from trainium_frontier_them_bones_amd import ops
+    g = torch.Generator().manual_seed(V + int(cap))
+    d = 256
+    x = torch.randn(N, d, generator=g).to(bf16).to(dev)
+    W = (std / d ** 0.5 * torch.randn(V, d, generator=g)).to(bf16).to(dev)
+    t = torch.randint(0, V, (N,), generator=g).to(dev)
+    logits, _, lse = ops.lmhead_fwd(x, W, t, cap)
+    _, plain = ops.loss_fwd(logits, t, cap)
+    want = torch.cat([torch.logsumexp(cap * torch.tanh(part.double() / cap), -1) for part in logits.split(1024)])
+    e, p = lse.double() - want, plain.double() - want
+    ulp = 2.0 ** (torch.floor(torch.log2(want.mean())).item() - 23)
+    print("cap %g std %g rows %d: mean %.3g rms %.3g, training's %.3g %.3g, ulp %.3g"
+          % (cap, std, N, e.mean(), e.square().mean().sqrt(), p.mean(), p.square().mean().sqrt(), ulp))
+    assert abs(e.mean()) < abs(p.mean()) + 0.1 * ulp
+    assert e.square().mean().sqrt() < p.square().mean().sqrt() + 0.1 * ulp

@@ -30,8 +30,8 @@ __device__ __forceinline__ float tanh_rcp(float y) {
   const float r = __builtin_amdgcn_rcpf(d);
   return __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
 }
-// tanh(y) = 1 - 2 / (exp(2 y) + 1)
-__device__ __forceinline__ float tanh_fast(float y) { return 1.0f - 2.0f * tanh_rcp(y); }
+// tanh(y) = 1 - 2 / (exp(2 y) + 1) (doubling is exact: the fma has the bits of the product and the difference)
+__device__ __forceinline__ float tanh_fast(float y) { return __builtin_fmaf(-2.0f, tanh_rcp(y), 1.0f); }
 
 struct MS {
   float m, s;
@@ -79,13 +79,18 @@ __global__ __launch_bounds__(1024) void loss_row_weights_kernel(const IDX* __res
 // leave half of a workgroup or more without a value (16384 x 1024, in place: 39 us with a workgroup a row, 20 with a wavefront).
 constexpr int WAVE_ROW_V = 2048;
 
+// exp(cap tanh(x / cap) - cap). (exp2(-2 cap log2(e) / (exp(2 x / cap) + 1)) needs two instructions less; but the error of its
+// reciprocal and of the inner exponential counts 2 cap times over: the mean error of lse over 9600 rows x 8192 of deviation
+// 0.5, cap = 30, is then 0.42e-6 with the hardware's reciprocal and 0.61e-6 with an exact one, 0.16e-6 this way.)
+__device__ __forceinline__ float capped_exp(float x, float icap, float cap) { return fexp(cap * tanh_fast(x * icap) - cap); }
+
 // The pair (max, sum exp) of eight logits joined to a (with a softcap cap is the maximum: it bounds every value).
 __device__ __forceinline__ void ms_add8(MS& a, const u32x4& u, float icap, float cap) {
   float v[8];
   unpack8bf(u, v);
   if (cap > 0.f) {
 #pragma unroll
-    for (int k = 0; k < 8; ++k) a.s += fexp(cap * tanh_fast(v[k] * icap) - cap);
+    for (int k = 0; k < 8; ++k) a.s += capped_exp(v[k], icap, cap);
   } else {
     float mx = a.m, t = 0.f;
 #pragma unroll
@@ -98,12 +103,6 @@ __device__ __forceinline__ void ms_add8(MS& a, const u32x4& u, float icap, float
   }
 }
 
-// exp(cap tanh(x / cap) - cap) = exp(-2 cap / (exp(2 x / cap) + 1)): two exponentials and a reciprocal, half the instructions
-// of the tanh, its division and the exponential after it. For evaluation, where nothing repeats the gradient's bits.
-__device__ __forceinline__ float capped_exp(float x, float icap, float cap) {
-  const float e = __builtin_amdgcn_exp2f(x * (2.8853900817779268f * icap));
-  return __builtin_amdgcn_exp2f(-2.8853900817779268f * cap * __builtin_amdgcn_rcpf(e + 1.0f));
-}
 // Evaluation: four chunks with one running maximum for their 32 values. Chunks beyond V hold -inf; i, step: the first chunk's
 // place in the row and the distance of two.
 __device__ __forceinline__ void ms_add32(MS& a, const u32x4* u, int i, int step, int V, float icap, float cap) {
@@ -656,8 +655,8 @@ extern "C" int tfb_lmhead_fwd(const void* x, const void* W, const void* targets,
   GemmOperand P{(const uint8_t*)W, (long)d * 2}, Q{(const uint8_t*)x, (long)d * 2};
   int st;
   // Where the persistent 256 x 256 kernel takes the shape, its plain store and a pass over the logits are cheaper than the
-  // exponentials in an epilogue that nothing overlaps (the call, without / with a softcap: 9600 x 8192 x 1024 261 -> 193 us /
-  // 264 -> 210, 2048 x 32768 x 768 150 -> 118 / 161 -> 121, 32768 x 32768 x 768 2166 -> 2096 / 2292 -> 2047).
+  // exponentials in an epilogue that nothing overlaps (the call, without / with a softcap: 9600 x 8192 x 1024 261 -> 204 us /
+  // 264 -> 201, 2048 x 32768 x 768 150 -> 120 / 161 -> 138, 32768 x 32768 x 768 2166 -> 2005 / 2292 -> 2199).
   if (gemm_pp_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, V, (int)rows, (long)d * 2, false, EpiStore{logits, (long)V, 0, 0}, s, st)) {
     if (st != TFB_OK) return st;
     launch_loss_fwd<true>(logits, targets, idx64, row_w, loss, lse, rows, V, softcap, s);
