@@ -94,7 +94,9 @@ PyObject* attr(PyObject* o, PyObject* name);
 struct PyRef {
   PyObject* o = nullptr;
   PyRef() = default;
+  struct Steal {};
   explicit PyRef(PyObject* borrowed) : o(borrowed) { Py_XINCREF(o); }
+  PyRef(PyObject* owned, Steal) : o(owned) {}
   PyRef(PyRef&& r) noexcept : o(std::exchange(r.o, nullptr)) {}
   PyRef& operator=(PyRef&& r) noexcept {
     std::swap(o, r.o);

@@ -94,27 +94,31 @@ struct GradBuf {
   Tensor buf;
   bool accumulate = false;
 };
-// The weight's in-place gradient buffer (undefined: none) and whether it holds earlier micro-steps' sums; marks it written.
-GradBuf accumulate_into(const Tensor& w) {
+// The weight's in-place gradient buffer (undefined: none) and whether it holds earlier micro-steps' sums; marks it written. What
+// the kernels take for granted of it is checked first: a dense device tensor, of the weight's shape and bf16 or fp32 where a GEMM writes
+// it (flat: fp32 and as many elements).
+GradBuf accumulate_into(const Tensor& w, bool flat = false) {
   pybind11::gil_scoped_acquire gil;
-  PyObject* o = THPVariable_Wrap(w);
+  PyRef o(THPVariable_Wrap(w), PyRef::Steal{});
+  PyRef buf(attr(o.o, names().grad_buf), PyRef::Steal{});
   GradBuf g;
-  g.buf = tensor_of(attr(o, names().grad_buf));
-  if (g.buf.defined()) {
-    PyObject* fresh = attr(o, names().grad_fresh);
-    g.accumulate = fresh && PyObject_IsTrue(fresh) == 0;
-    Py_XDECREF(fresh);
-    PyObject_SetAttr(o, names().grad_fresh, Py_False);
-  }
-  Py_DECREF(o);
+  if (!buf.o || buf.o == Py_None) return g;
+  TORCH_CHECK_TYPE(THPVariable_Check(buf.o), "grad_buf must be a tensor, got ", Py_TYPE(buf.o)->tp_name);
+  g.buf = THPVariable_Unpack(buf.o);
+  chk(g.buf, flat ? F32 : g.buf.scalar_type());
+  const bool fits = flat ? g.buf.numel() == w.numel() : g.buf.sizes() == w.sizes();
+  TORCH_CHECK_VALUE((g.buf.scalar_type() == BF16 || g.buf.scalar_type() == F32) && fits,
+                    "grad_buf must be bf16 or fp32 in the weight's shape ", w.sizes(), ", not ", g.buf.scalar_type(), " ", g.buf.sizes());
+  PyRef fresh(attr(o.o, names().grad_fresh), PyRef::Steal{});
+  g.accumulate = fresh.o && PyObject_IsTrue(fresh.o) == 0;
+  PyObject_SetAttr(o.o, names().grad_fresh, Py_False);
   return g;
 }
 bool has_grad_buf(const Tensor& w) {
   pybind11::gil_scoped_acquire gil;
-  PyObject* o = THPVariable_Wrap(w);
-  const bool has = tensor_of(attr(o, names().grad_buf)).defined();
-  Py_DECREF(o);
-  return has;
+  PyRef o(THPVariable_Wrap(w), PyRef::Steal{});
+  PyRef buf(attr(o.o, names().grad_buf), PyRef::Steal{});
+  return buf.o && buf.o != Py_None;
 }
 
 // The norm's gain gradient: left as partial sums where the weight names a place for them (finished with the other norms' by
@@ -132,7 +136,7 @@ NormBack norm_backward(const Tensor& gy, const Tensor& s, const Tensor& inv, con
       part = tensor_of(attr(o, names().dw_part));
       Py_DECREF(o);
     }
-    if (!part.defined()) g = accumulate_into(w);
+    if (!part.defined()) g = accumulate_into(w, true);
   }
   NormGrad n = rmsnorm_bwd(dense(gy), s, inv, w, dense(gs), g.buf, g.accumulate, part, want_amax);
   NormBack b{n.dx, {}, n.amax};
@@ -802,6 +806,7 @@ struct Moe : Function<Moe> {
     if (in_place) {
       bf_ = accumulate_into(w_fc), bp = accumulate_into(w_proj);
       TORCH_CHECK(bf_.accumulate == bp.accumulate, "MoeMlp8Fn: the two expert weights' gradient buffers are in different states");
+      TORCH_CHECK_VALUE(bf_.buf.scalar_type() == bp.buf.scalar_type(), "MoeMlp8Fn: the two expert weights' gradient buffers differ in type");
     }
     Tensor dw_fc = bf_.buf, dw_proj = bp.buf;
     if (a.dw_fp8)
@@ -809,7 +814,7 @@ struct Moe : Function<Moe> {
     else
       moe_dw(m.dpre, xs, c.dys, r, s.tab, dw_fc, dw_proj, E, bf_.accumulate, BF16);
     if (in_place) dw_fc = dw_proj = Tensor();
-    GradBuf br = accumulate_into(router);
+    GradBuf br = accumulate_into(router, true);
     RouteGrad rg = moe_route_bwd(c.dgate, p, idx, m.dx, s.tab, h, wr, br.buf, br.accumulate, s.aux.empty() ? nullptr : &aux);
     return {rg.dh, br.buf.defined() ? Tensor() : rg.dwr.to(router.scalar_type()), dw_fc, dw_proj, Tensor(), Tensor(), Tensor(), Tensor(),
             Tensor(), Tensor()};
@@ -927,8 +932,8 @@ struct Embedding : Function<Embedding> {
   }
   static Vars backward(AutogradContext* ctx, Vars g) {
     const auto s = ctx->get_saved_variables();
-    GradBuf gb = accumulate_into(s[1]);
-    Tensor dw = gb.buf.defined() ? gb.buf : make(s[1].sizes(), F32, s[1]);
+    GradBuf gb = accumulate_into(s[1], true);
+    Tensor dw = gb.buf.defined() ? gb.buf.view(s[1].sizes()) : make(s[1].sizes(), F32, s[1]);
     if (!gb.accumulate) fill_f32(dw, 0.0);
     embedding_bwd(s[0], dense(g[0]), dw);
     return {Tensor(), gb.buf.defined() ? Tensor() : dw.to(s[1].scalar_type())};

@@ -113,6 +113,8 @@ NormGrad rmsnorm_bwd(const Tensor& gy, const Tensor& s, const Tensor& inv, const
   chk(gy), chk(s), chk(w), chk(gs), chk(inv, F32), chk(dw, F32), chk(part_given, F32);
   const int64_t C = s.size(-1), rows = s.numel() / C;
   const int64_t nb = w.defined() || want_amax ? tfb_norm_bwd_blocks(rows) : 0;
+  TORCH_CHECK_VALUE(!dw.defined() || dw.numel() == C, "dw is [C]");
+  TORCH_CHECK_VALUE(!w.defined() || !part_given.defined() || part_given.numel() >= nb * C, "part is [", nb, ", C]");
   NormGrad o;
   o.dx = make_like(s);
   Tensor part;
