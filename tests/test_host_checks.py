@@ -1,0 +1,61 @@
+"""The native host layer's checks of what a caller hands over, without a GPU: fake device tensors have shapes and types but no
+memory, so a call that passes its checks ends where it asks for its first output ("No HIP GPUs") and reaches no kernel."""
+import os
+
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+
+pytestmark = pytest.mark.filterwarnings("ignore:Accessing the data pointer of FakeTensor")
+bf16, f32, u8 = torch.bfloat16, torch.float32, torch.uint8
+
+
+@pytest.fixture
+def A():
+    from trainium_frontier_them_bones_amd import _lib, autograd
+    if not os.path.exists(_lib.HOST_PATH):
+        pytest.skip("host extension not built (run __graft_entry__.build())")
+    if torch.cuda.is_available():
+        pytest.skip("made for a machine without a GPU")
+    with FakeTensorMode(allow_non_fake_inputs=True):
+        yield autograd
+
+
+def _t(*shape, dtype=bf16):
+    return torch.empty(*shape, dtype=dtype, device="cuda")
+
+
+def _passes(fn):
+    """The call got through its checks."""
+    with pytest.raises(RuntimeError, match="No HIP GPUs"):
+        fn()
+
+
+def _refused(fn, exc=ValueError):
+    with pytest.raises(exc) as e:
+        fn()
+    assert "No HIP GPUs" not in str(e.value)
+
+
+def _linear8_state(A, N, K, dw_fp8=False):
+    st = A.Linear8State(dw_fp8=dw_fp8)
+    st.sc, st.w8, st.w8t = _t(3, dtype=f32), _t(N, K, dtype=u8), _t(K, N, dtype=u8)
+    return st
+
+
+@pytest.mark.parametrize("res", [False, True])
+@pytest.mark.parametrize("dw_fp8", [False, True])
+def test_fp8_projection_refuses_other_operands(A, dw_fp8, res):
+    """The rows come from x, its bytes may have any shape of as many; the bytes of the weight are the weight's."""
+    w, st = _t(512, 256), _linear8_state(A, 512, 256, dw_fp8)
+    x, r = _t(2, 128, 256), _t(2, 128, 512) if res else None
+    call = A.Linear8Fn.apply
+    _passes(lambda: call(x, w, st, 4.0, _t(256, 256, dtype=u8), r))
+    _passes(lambda: call(x, w, st, 4.0, None, r))
+    _passes(lambda: call(x, w, st, None, None, r))
+    for x8 in (_t(384, 256, dtype=u8), _t(128, 256, dtype=u8), _t(256, 512, dtype=u8), _t(256, 128, dtype=u8)):
+        _refused(lambda: call(x, w, st, 4.0, x8, r))
+    _refused(lambda: call(x, w, st, 4.0, _t(256, 256), r), TypeError)
+    for N, K in ((1024, 256), (256, 256), (512, 512), (512, 128)):
+        _refused(lambda: call(x, w, _linear8_state(A, N, K, dw_fp8), 4.0, None, r))
+    _refused(lambda: call(_t(2, 128, 512), w, st, 4.0, None, None))

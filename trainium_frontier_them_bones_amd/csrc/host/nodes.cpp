@@ -369,6 +369,10 @@ struct Linear8 : Function<Linear8> {
     const auto& n = names();
     const Tensor sc = tensor_attr(state, n.sc), w8 = tensor_attr(state, n.w8);
     const bool dw8 = bool_attr(state, n.dw_fp8);
+    chk(sc, F32);
+    TORCH_CHECK_VALUE(w.dim() == 2 && x.size(-1) == w.size(1), "inner dimensions differ: ", x.size(-1), " vs ", w.size(1));
+    TORCH_CHECK_VALUE(w8.sizes() == w.sizes() && sc.numel() >= 2, "the state holds another weight's bytes: ", w8.sizes(), " for ", w.sizes());
+    TORCH_CHECK_VALUE(!x8_ || x8_->numel() == x.numel(), "x8 has ", x8_ ? x8_->sizes() : x.sizes(), " bytes for x ", x.sizes());
     S& st = keep<S>(ctx);
     st.state = PyRef(state);
     st.has_res = res.has_value();
@@ -380,7 +384,7 @@ struct Linear8 : Function<Linear8> {
       x8 = quant_fp8(x, ptr(st.sx), 0, E4M3);
       dqa = static_cast<const float*>(ptr(st.sx)) + 1;
     } else {
-      x8 = x8_ ? *x8_ : quant_fp8(x, nullptr, *x_scale, E4M3);
+      x8 = x8_ ? dense(*x8_).view(x.sizes()) : quant_fp8(x, nullptr, *x_scale, E4M3);
       st.imm = 1.0 / *x_scale;
     }
     Tensor y = gemm_fp8(x8, w8, E4M3, dqa, dqw, st.imm, res ? dense(*res) : Tensor(), with_last(x, w.size(0)));

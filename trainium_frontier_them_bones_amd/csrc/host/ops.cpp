@@ -40,6 +40,9 @@ Tensor workspace(const Tensor& like) {
 // ---------------------------------------------------------------------------------------------------------------- GEMM
 void gemm(const Tensor& a, const Tensor& b, const Tensor& out, int64_t M, int64_t N, int64_t K, bool ta, bool tb, bool accumulate,
           const Tensor& alpha) {
+  chk(a), chk(b);
+  TORCH_CHECK_VALUE(a.numel() == M * K && b.numel() == K * N && out.numel() == M * N, "operands of ", a.numel(), " and ", b.numel(),
+                    " elements and an output of ", out.numel(), " for ", M, " x ", N, " x ", K);
   const Tensor ws = workspace(a);
   const int f32 = out.scalar_type() == F32;
   if (alpha.defined())
@@ -227,6 +230,7 @@ Tensor gemm_fp8(const Tensor& a8, const Tensor& b8, int fmt_a, const void* dq_a,
   const int64_t K = a8.size(-1), M = a8.numel() / K, N = b8.size(0);
   TORCH_CHECK_VALUE(b8.dim() == 2 && b8.size(1) == K, "inner dimensions differ");
   TORCH_CHECK_VALUE(!res.defined() || (res.size(-1) == N && res.numel() == M * N), "shapes differ");
+  TORCH_CHECK_VALUE(c10::multiply_integers(out_shape) == M * N, "an output ", out_shape, " for ", M, " x ", N);
   Tensor out = make(out_shape, BF16, a8);
   if (res.defined())
     TFB_CALL(tfb_gemm_fp8_res, ptr(a8), ptr(b8), dq_a, dq_b, dq, ptr(res), ptr(out), M, N, K, stream());
