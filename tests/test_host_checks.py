@@ -59,3 +59,30 @@ def test_fp8_projection_refuses_other_operands(A, dw_fp8, res):
     for N, K in ((1024, 256), (256, 256), (512, 512), (512, 128)):
         _refused(lambda: call(x, w, _linear8_state(A, N, K, dw_fp8), 4.0, None, r))
     _refused(lambda: call(_t(2, 128, 512), w, st, 4.0, None, None))
+
+
+def _mlp8_state(A, F, d, dw_fp8=False):
+    st = A.Mlp8State(dw_fp8=dw_fp8)
+    st.row, st.w8 = _t(16, dtype=f32), _t(4, F * d, dtype=u8)
+    return st
+
+
+@pytest.mark.parametrize("dw_fp8", [False, True])
+def test_fp8_mlp_refuses_other_operands(A, dw_fp8):
+    """The bytes are those of x itself (with bf16 weight gradients x is saved and contracted over the rows of the bytes), and
+    the state's those of the call's weights."""
+    d, F = 256, 512
+    wf, wp, st = _t(F, d), _t(d, F), _mlp8_state(A, F, d, dw_fp8)
+    call = A.Mlp8Fn.apply
+    x, ragged = _t(2, 128, d), _t(3, 100, d)
+    _passes(lambda: call(x, wf, wp, st))
+    _passes(lambda: call(ragged, wf, wp, st))
+    _passes(lambda: call(x, wf, wp, st, _t(256, d, dtype=u8), _t(2, 128, d)))
+    for res in (None, _t(3, 100, d)):
+        _refused(lambda: call(ragged, wf, wp, st, _t(384, d, dtype=u8), res))       # bytes of more rows than x has
+        _refused(lambda: call(ragged, wf, wp, st, _t(300, d, dtype=u8), res))       # no whole tiles to read
+    _refused(lambda: call(x, wf, wp, st, _t(128, d, dtype=u8)))
+    _refused(lambda: call(x, wf, wp, st, _t(256, d)), TypeError)
+    for F2, d2 in ((1024, d), (256, d), (F, 512)):
+        _refused(lambda: call(x, wf, wp, _mlp8_state(A, F2, d2, dw_fp8)))
+        _refused(lambda: call(_t(2, 128, d2), _t(F2, d2), _t(d2, F2), st))

@@ -641,7 +641,8 @@ struct Mlp8 : Function<Mlp8> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_fc, const Tensor& w_proj, PyObject* state,
                         const OptTensor& x8_, const OptTensor& res_) {
     const Mlp8Attrs st = mlp8_attrs(state);
-    const Tensor x8 = val(x8_), res = dense(val(res_));
+    TORCH_CHECK_VALUE(!x8_ || x8_->numel() == x_.numel(), "x8 has ", x8_ ? x8_->sizes() : x_.sizes(), " bytes for x ", x_.sizes());
+    const Tensor x8 = x8_ ? dense(*x8_).view(x_.sizes()) : Tensor(), res = dense(val(res_));
     // with the bytes given and the weight gradients in fp8 nothing reads x itself (it may be a storage-less placeholder)
     const Tensor x = x8.defined() && st.dw_fp8 ? Tensor() : dense(x_);
     MlpFwd f = mlp8_fwd(x, st.w8, st.row, w_fc.size(0), st.x_scale, x8, res, !st.dw_fp8);

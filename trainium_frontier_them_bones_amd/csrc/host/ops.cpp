@@ -251,6 +251,12 @@ Tensor gemm_fp8_tn(const Tensor& g8, const Tensor& a8, int fmt_g, int fmt_a, con
   return out;
 }
 
+// The bytes and scale row of an MLP state are those of weights [F, d] and [d, F].
+static void check_pack(const Tensor& w8, const Tensor& row, int64_t d, int64_t F) {
+  TORCH_CHECK_VALUE(w8.numel() == 4 * F * d && row.numel() >= 16, "the state holds another MLP's weights: ", w8.numel(), " bytes for d ", d,
+                    ", F ", F);
+}
+
 MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F, const Scale& x_scale, const Tensor& x8, const Tensor& res,
                 bool want_xp) {
   chk(x), chk(w8, U8), chk(row, F32), chk(x8, U8), chk(res);
@@ -260,6 +266,7 @@ MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F,
   const auto fits = [&](const Tensor& t) { return t.size(-1) == d && (t.numel() == rows * d || t.numel() == M * d); };
   TORCH_CHECK_VALUE(!x8.defined() || (x8.size(-1) == d && x8.numel() == M * d), "x8 shape");
   TORCH_CHECK_VALUE(!x.defined() || fits(x), "res shape");
+  check_pack(w8, row, d, F);
   MlpFwd o;
   o.x8 = x8.defined() ? x8 : quant_rows(x, ptr(x_scale.dev), x_scale.imm, E4M3, M, want_xp ? &o.xp : nullptr);
   o.y = make_rows(in.sizes(), M, d, w8);
