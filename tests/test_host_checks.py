@@ -86,3 +86,19 @@ def test_fp8_mlp_refuses_other_operands(A, dw_fp8):
     for F2, d2 in ((1024, d), (256, d), (F, 512)):
         _refused(lambda: call(x, wf, wp, _mlp8_state(A, F2, d2, dw_fp8)))
         _refused(lambda: call(_t(2, 128, d2), _t(F2, d2), _t(d2, F2), st))
+
+
+def test_fp8_mlp_backward_refuses_rows_of_another_forward(A):
+    """The backward rounds dy's rows up to whole tiles: r is compared with that count."""
+    from trainium_frontier_them_bones_amd import ops
+    d, F = 256, 512
+    w8, row = _t(4, F * d, dtype=u8), _t(16, dtype=f32)
+    for bwd in (lambda dy, r: ops.mlp8_bwd(dy, r, w8, row), lambda dy, r: ops.mlp8_bwd_q(dy, r, w8, row)):
+        _passes(lambda: bwd(_t(256, d), _t(256, F)))
+        _passes(lambda: bwd(_t(200, d), _t(256, F)))
+        for rows, r in ((200, 200), (256, 128), (129, 128), (256, 384)):
+            _refused(lambda: bwd(_t(rows, d), _t(r, F)))
+        _refused(lambda: bwd(_t(256, d), _t(256, 1024)))
+        _refused(lambda: bwd(_t(256, 512), _t(256, F)))
+    _passes(lambda: ops.mlp_dw_proj(_t(256, d), _t(256, F)))
+    _refused(lambda: ops.mlp_dw_proj(_t(256, d), _t(128, F)))

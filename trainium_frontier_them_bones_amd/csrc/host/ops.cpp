@@ -257,6 +257,11 @@ static void check_pack(const Tensor& w8, const Tensor& row, int64_t d, int64_t F
                     ", F ", F);
 }
 
+// r is what the forward of as many rows left: whole tiles where the forward padded.
+static void check_rows(const Tensor& r, int64_t M, int64_t F) {
+  TORCH_CHECK_VALUE(r.dim() == 2 && r.size(0) == M && r.size(1) == F, "r is [", M, ", F], not ", r.sizes());
+}
+
 MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F, const Scale& x_scale, const Tensor& x8, const Tensor& res,
                 bool want_xp) {
   chk(x), chk(w8, U8), chk(row, F32), chk(x8, U8), chk(res);
@@ -284,6 +289,8 @@ MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F,
 MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h, bool want_dyp) {
   chk(dy), chk(r), chk(w8, U8), chk(row, F32);
   const int64_t d = dy.size(-1), M = tile_rows(dy.numel() / d), F = r.size(1);
+  check_rows(r, M, F);
+  check_pack(w8, row, d, F);
   MlpBwd o;
   o.dy8 = quant_rows(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2, M, want_dyp ? &o.dyp : nullptr);
   o.dx = make_rows(dy.sizes(), M, d, dy);
@@ -297,6 +304,8 @@ MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tenso
 MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, bool want_dpre) {
   chk(dy), chk(r), chk(w8, U8), chk(row, F32);
   const int64_t d = dy.size(-1), M = tile_rows(dy.numel() / d), F = r.size(1);
+  check_rows(r, M, F);
+  check_pack(w8, row, d, F);
   MlpBwd o;
   o.dy8 = quant_rows(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2, M, nullptr);
   o.dx = make_rows(dy.sizes(), M, d, dy);
@@ -325,6 +334,7 @@ void mlp8_dw8(const Tensor& x8, const Tensor& dp8, const Tensor& hq8, const Tens
 Tensor mlp_dw_proj(const Tensor& dy, const Tensor& r, Tensor out, bool accumulate, at::ScalarType out_dtype) {
   chk(dy), chk(r);
   const int64_t d = dy.size(-1), M = dy.numel() / d, F = r.size(1);
+  check_rows(r, M, F);
   out = Out2::get(out, {d, F}, out_dtype, accumulate, dy);
   const Tensor ws = workspace(dy);
   TFB_CALL(tfb_mlp_dw_proj, ptr(dy), ptr(r), ptr(out), M, d, F, out.scalar_type() == F32, accumulate, ptr(ws), ws.numel() * 4, stream());
