@@ -102,3 +102,9 @@ def test_fp8_mlp_backward_refuses_rows_of_another_forward(A):
         _refused(lambda: bwd(_t(256, 512), _t(256, F)))
     _passes(lambda: ops.mlp_dw_proj(_t(256, d), _t(256, F)))
     _refused(lambda: ops.mlp_dw_proj(_t(256, d), _t(128, F)))
+
+
+def test_block_head_with_a_skip_needs_its_gain(A):
+    x, one = _t(4, 256), _t(1, dtype=f32)
+    _passes(lambda: A.BlockHeadFn.apply(x, x, one, one, x, one, 1e-6))
+    _refused(lambda: A.BlockHeadFn.apply(x, x, one, one, x, None, 1e-6), TypeError)

@@ -279,6 +279,7 @@ struct BlockHead : Function<BlockHead> {
                       const OptTensor& l3, double eps) {
     ctx->set_materialize_grads(false);
     const Tensor x = dense(x_), x0 = dense(x0_), skip = dense(val(skip_));
+    TORCH_CHECK_TYPE(!skip_ || l3, "a skip needs its gain l3");
     auto one = [](const Tensor& t) { return t.reshape(1).to(F32); };
     const Tensor g1 = one(l1), gains = at::cat({g1, one(l2), skip.defined() ? one(*l3) : g1});   // (the third is unused without a skip)
     auto [x_new, x_norm, inv] = block_head_fwd(x, x0, gains, skip, eps);
