@@ -108,3 +108,26 @@ def test_block_head_with_a_skip_needs_its_gain(A):
     x, one = _t(4, 256), _t(1, dtype=f32)
     _passes(lambda: A.BlockHeadFn.apply(x, x, one, one, x, one, 1e-6))
     _refused(lambda: A.BlockHeadFn.apply(x, x, one, one, x, None, 1e-6), TypeError)
+
+
+def test_an_empty_last_dimension_raises(A):
+    """Rows are counted by the last dimension: an empty one is an error, not a division by zero that ends the process."""
+    from trainium_frontier_them_bones_amd import ops
+    from trainium_frontier_them_bones_amd import train_api as api
+    e, one, tg = _t(4, 0), _t(1, dtype=f32), _t(4, dtype=torch.int64)
+    b = _t(4, 0, dtype=u8)
+    w, wt, w8 = _t(256, 0), _t(0, 256), _t(4, 0, dtype=u8)
+    row, rows = _t(16, dtype=f32), _t(2, 16, dtype=f32)
+    st, st8 = _mlp8_state(A, 256, 0), _linear8_state(A, 256, 0)
+    for fn in (
+            lambda: A.RMSNormFn.apply(e, None, 1e-6), lambda: A.RMSNormPassFn.apply(e, None, 1e-6, 4.0),
+            lambda: A.AddRMSNormFn.apply(e, e, None, 1e-6), lambda: A.BlockHeadFn.apply(e, e, one, one, None, None, 1e-6),
+            lambda: A.MixTailFn.apply(_t(1, 4, 0), one, 4), lambda: A.LinearFn.apply(e, w), lambda: A.LinearFn.apply(e, w, _t(4, 256)),
+            lambda: A.Linear8Fn.apply(e, w, st8, 4.0), lambda: A.Mlp8Fn.apply(e, w, wt, st), lambda: A.NrMlpFn.apply(e, w, wt, st),
+            lambda: A.MlpFusedFn.apply(e, w, wt), lambda: A.LmHeadLossFn.apply(e, w, tg, 0.0, "mean"),
+            lambda: A.MoeMlp8Fn.apply(e, _t(2, 0, dtype=f32), _t(2, 256, 0), _t(2, 0, 256), None, 1, None),
+            lambda: api.fused_loss(e, tg), lambda: api.fused_loss(e, tg, "none"), lambda: ops.matmul_res(e, wt, _t(4, 256)),
+            lambda: ops.gemm_fp8(b, w8), lambda: ops.gemm_fp8_tn(b, b), lambda: ops.mlp8_backward_scales(e, row),
+            lambda: ops.mlp8_fwd(e, w8, row, 256), lambda: ops.mlp8_bwd(e, _t(128, 256), w8, row), lambda: ops.mlp_dw_proj(e, _t(4, 256)),
+            lambda: ops.mlp_bwd(e, _t(4, 256), w, wt), lambda: ops.lmhead_fwd(e, w, tg, 0.0)):
+        _refused(fn)

@@ -42,6 +42,12 @@ inline Tensor make(at::IntArrayRef shape, at::ScalarType dt, const Tensor& like)
 }
 inline Tensor make_like(const Tensor& t) { return make(t.sizes(), t.scalar_type(), t); }
 
+// The size of t's last dimension, by which a number of rows is counted.
+inline int64_t last_dim(const Tensor& t) {
+  TORCH_CHECK_VALUE(t.dim() > 0 && t.size(-1) > 0, "a tensor ", t.sizes(), " has no rows");
+  return t.size(-1);
+}
+
 // The shape of t with its last dimension replaced.
 inline at::DimVector with_last(const Tensor& t, int64_t n) {
   at::DimVector s(t.sizes());

@@ -334,7 +334,7 @@ struct Linear : Function<Linear> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w, const OptTensor& res) {
     const Tensor x = dense(x_);
     chk(x), chk(w);
-    TORCH_CHECK_VALUE(w.dim() == 2 && x.size(-1) == w.size(1), "inner dimensions differ: ", x.size(-1), " vs ", w.size(1));
+    TORCH_CHECK_VALUE(w.dim() == 2 && last_dim(x) == w.size(1), "inner dimensions differ: ", x.size(-1), " vs ", w.size(1));
     Tensor y;
     if (res) {   // bf16(res + bf16(x @ w^T)): the residual add made in the GEMM's store (nki_attn_nr8.py:1003)
       y = matmul_res(x, w, dense(*res), true);
@@ -371,7 +371,7 @@ struct Linear8 : Function<Linear8> {
     const Tensor sc = tensor_attr(state, n.sc), w8 = tensor_attr(state, n.w8);
     const bool dw8 = bool_attr(state, n.dw_fp8);
     chk(sc, F32);
-    TORCH_CHECK_VALUE(w.dim() == 2 && x.size(-1) == w.size(1), "inner dimensions differ: ", x.size(-1), " vs ", w.size(1));
+    TORCH_CHECK_VALUE(w.dim() == 2 && last_dim(x) == w.size(1), "inner dimensions differ: ", x.size(-1), " vs ", w.size(1));
     TORCH_CHECK_VALUE(w8.sizes() == w.sizes() && sc.numel() >= 2, "the state holds another weight's bytes: ", w8.sizes(), " for ", w.sizes());
     TORCH_CHECK_VALUE(!x8_ || x8_->numel() == x.numel(), "x8 has ", x8_ ? x8_->sizes() : x.sizes(), " bytes for x ", x.sizes());
     S& st = keep<S>(ctx);
@@ -670,7 +670,7 @@ struct NrMlp : Function<NrMlp> {
     const Mlp8Attrs st = mlp8_attrs(state);
     const Tensor x = dense(x_);
     // (with the weight gradients in fp8 too nothing reads the norm's bf16 rows: only its e4m3 bytes are written)
-    NormOut n = rmsnorm_fwd_q(x, {}, eps, {}, st.x_scale.host(), !st.dw_fp8, tile_rows(x.numel() / x.size(-1)));
+    NormOut n = rmsnorm_fwd_q(x, {}, eps, {}, st.x_scale.host(), !st.dw_fp8, tile_rows(x.numel() / last_dim(x)));
     MlpFwd f = mlp8_fwd(n.y, st.w8, st.row, w_fc.size(0), st.x_scale, n.y8, x);
     ctx->save_for_backward({x, st.dw_fp8 ? n.y8 : n.y, n.inv, f.r, w_fc, w_proj});
     keep<PyRef>(ctx) = PyRef(state);
@@ -735,7 +735,7 @@ struct Moe : Function<Moe> {
     const Tensor h = dense(h_);
     const int64_t E = w_fc.size(0), F = w_fc.size(1), d = w_fc.size(2);
     const Tensor wr = dense(router.scalar_type() == F32 ? router : router.to(F32));
-    TORCH_CHECK_VALUE(h.size(-1) == d && wr.size(1) == d && wr.size(0) == E, "h [.., d], router [E, d], w_fc [E, F, d]");
+    TORCH_CHECK_VALUE(last_dim(h) == d && wr.size(1) == d && wr.size(0) == E, "h [.., d], router [E, d], w_fc [E, F, d]");
     S& s = keep<S>(ctx);
     s.aux = aux_weights, s.topk = topk;
     MoeRoute rt = moe_route(h, wr, topk, val(bias), !aux_weights.empty());
@@ -841,7 +841,7 @@ struct LmHeadLoss : Function<LmHeadLoss> {
                         bool one_pass) {
     const Tensor x = dense(x_), tg = targets_of(targets);
     chk(x), chk(W);
-    const int64_t d = x.size(-1), M = x.numel() / d, V = W.size(0);
+    const int64_t d = last_dim(x), M = x.numel() / d, V = W.size(0);
     TORCH_CHECK_VALUE(W.dim() == 2 && W.size(1) == d && tg.numel() == M, "x [.., d], W [V, d], one target a row");
     const Tensor w = loss_row_weights(tg, mean, V);
     keep<S>(ctx) = {one_pass, false, softcap, M, d, V};
@@ -891,7 +891,7 @@ struct LossRows : Function<LossRows> {
   };
   static Tensor forward(AutogradContext* ctx, const Tensor& logits, const Tensor& targets, double softcap) {
     const Tensor tg = targets_of(targets);
-    const int64_t V = logits.size(-1), N = logits.numel() / V;
+    const int64_t V = last_dim(logits), N = logits.numel() / V;
     TORCH_CHECK_VALUE(tg.numel() == N, "one target a row");
     auto [rows, lse] = loss_fwd(logits, tg, {}, softcap, N, V);
     ctx->save_for_backward({logits, tg, lse});
@@ -901,7 +901,7 @@ struct LossRows : Function<LossRows> {
   static Vars backward(AutogradContext* ctx, Vars g) {
     const auto s = ctx->get_saved_variables();
     Tensor out = make_like(s[0]);
-    const int64_t V = out.size(-1);
+    const int64_t V = last_dim(out);
     loss_bwd(s[0], s[1], s[2], dense(g[0].to(F32)), out, kept<S>(ctx).softcap, out.numel() / V, V);
     return {out, Tensor(), Tensor()};
   }
@@ -914,7 +914,7 @@ struct FusedLoss : Function<FusedLoss> {
   };
   static Tensor forward(AutogradContext* ctx, const Tensor& logits_, const Tensor& targets, bool mean, double softcap) {
     const Tensor logits = dense(logits_), tg = targets_of(targets);
-    const int64_t V = logits.size(-1), N = logits.numel() / V;
+    const int64_t V = last_dim(logits), N = logits.numel() / V;
     TORCH_CHECK_VALUE(tg.numel() == N, "one target a row");
     const Tensor w = loss_row_weights(tg, mean, V);
     auto [rows, lse] = loss_fwd(logits, tg, w, softcap, N, V);
@@ -925,7 +925,7 @@ struct FusedLoss : Function<FusedLoss> {
   static Vars backward(AutogradContext* ctx, Vars g) {
     const auto s = ctx->get_saved_variables();
     Tensor out = make_like(s[0]);
-    const int64_t V = out.size(-1);
+    const int64_t V = last_dim(out);
     loss_bwd(s[0], s[1], s[2], s[3] * g[0].to(F32), out, kept<S>(ctx).softcap, out.numel() / V, V);
     return {out, Tensor(), Tensor(), Tensor()};
   }

@@ -65,7 +65,7 @@ Tensor matmul(const Tensor& a, const Tensor& b, bool ta, bool tb, Tensor out, bo
 Tensor matmul_res(const Tensor& a, const Tensor& b, const Tensor& res, bool tb) {
   chk(a), chk(b), chk(res);
   TORCH_CHECK_VALUE(b.dim() == 2, "b is a matrix");
-  const int64_t K = a.size(-1), M = a.numel() / K, N = b.size(!tb);
+  const int64_t K = last_dim(a), M = a.numel() / K, N = b.size(!tb);
   TORCH_CHECK_VALUE(K == b.size(tb) && res.size(-1) == N && res.numel() == M * N, "shapes differ");
   Tensor out = make(res.sizes(), BF16, a);
   TFB_CALL(tfb_gemm_bf16_res, ptr(a), ptr(b), ptr(res), ptr(out), M, N, K, tb, stream());
@@ -74,7 +74,7 @@ Tensor matmul_res(const Tensor& a, const Tensor& b, const Tensor& res, bool tb) 
 
 Tensor qkv_rope(const Tensor& x, const Tensor& w, const Tensor& cos, const Tensor& sin, int64_t T, int64_t rot_cols) {
   chk(x), chk(w), chk(cos), chk(sin);
-  const int64_t K = x.size(-1), M = x.numel() / K, N = w.size(0);
+  const int64_t K = last_dim(x), M = x.numel() / K, N = w.size(0);
   Tensor out = make(with_last(x, N), BF16, x);
   TFB_CALL(tfb_qkv_rope_fwd, ptr(x), ptr(w), ptr(cos), ptr(sin), ptr(out), M, N, K, T, rot_cols, stream());
   return out;
@@ -83,7 +83,7 @@ Tensor qkv_rope(const Tensor& x, const Tensor& w, const Tensor& cos, const Tenso
 // --------------------------------------------------------------------------------------------------------------- norms
 NormOut rmsnorm_fwd(const Tensor& x, const Tensor& w, double eps, const Tensor& res) {
   chk(x), chk(res), chk(w);
-  const int64_t C = x.size(-1), rows = x.numel() / C;
+  const int64_t C = last_dim(x), rows = x.numel() / C;
   NormOut o;
   o.y = make_like(x);
   o.s = res.defined() ? make_like(x) : x;
@@ -94,7 +94,7 @@ NormOut rmsnorm_fwd(const Tensor& x, const Tensor& w, double eps, const Tensor& 
 
 NormOut rmsnorm_fwd_q(const Tensor& x, const Tensor& w, double eps, const Tensor& res, double y8_scale, bool want_y, int64_t rows_out) {
   chk(x), chk(res), chk(w);
-  const int64_t C = x.size(-1), rows = x.numel() / C;
+  const int64_t C = last_dim(x), rows = x.numel() / C;
   NormOut o;
   const bool pad = rows_out > rows;
   if (want_y) o.y = pad ? make({rows_out, C}, BF16, x) : make_like(x);
@@ -114,7 +114,7 @@ NormOut rmsnorm_fwd_q(const Tensor& x, const Tensor& w, double eps, const Tensor
 NormGrad rmsnorm_bwd(const Tensor& gy, const Tensor& s, const Tensor& inv, const Tensor& w, const Tensor& gs, const Tensor& dw,
                      bool accumulate, const Tensor& part_given, bool want_amax) {
   chk(gy), chk(s), chk(w), chk(gs), chk(inv, F32), chk(dw, F32), chk(part_given, F32);
-  const int64_t C = s.size(-1), rows = s.numel() / C;
+  const int64_t C = last_dim(s), rows = s.numel() / C;
   const int64_t nb = w.defined() || want_amax ? tfb_norm_bwd_blocks(rows) : 0;
   TORCH_CHECK_VALUE(!dw.defined() || dw.numel() == C, "dw is [C]");
   TORCH_CHECK_VALUE(!w.defined() || !part_given.defined() || part_given.numel() >= nb * C, "part is [", nb, ", C]");
@@ -140,7 +140,7 @@ NormGrad rmsnorm_bwd(const Tensor& gy, const Tensor& s, const Tensor& inv, const
 
 std::tuple<Tensor, Tensor, Tensor> block_head_fwd(const Tensor& x, const Tensor& x0, const Tensor& gains, const Tensor& skip, double eps) {
   chk(x), chk(x0), chk(skip), chk(gains, F32);
-  const int64_t C = x.size(-1), rows = x.numel() / C;
+  const int64_t C = last_dim(x), rows = x.numel() / C;
   Tensor x_new = make_like(x), x_norm = make_like(x), inv = scratch(x, rows);
   TFB_CALL(tfb_block_head_fwd, ptr(x), ptr(x0), ptr(skip), ptr(gains), ptr(x_new), ptr(x_norm), ptr(inv), rows, C, eps, stream());
   return {x_new, x_norm, inv};
@@ -149,7 +149,7 @@ std::tuple<Tensor, Tensor, Tensor> block_head_fwd(const Tensor& x, const Tensor&
 HeadGrad block_head_bwd(const Tensor& g_new, const Tensor& g_norm, const Tensor& x, const Tensor& x0, const Tensor& x_new,
                         const Tensor& inv, const Tensor& gains, const Tensor& skip) {
   chk(g_new), chk(g_norm), chk(x), chk(x0), chk(skip), chk(x_new);
-  const int64_t C = x.size(-1), rows = x.numel() / C;
+  const int64_t C = last_dim(x), rows = x.numel() / C;
   HeadGrad o{make_like(x), make_like(x), skip.defined() ? make_like(x) : Tensor(), scratch(x, 4)};
   const Tensor part = scratch(x, 4 * tfb_norm_bwd_blocks(rows));
   TFB_CALL(tfb_block_head_bwd, ptr(g_new), ptr(g_norm), ptr(x), ptr(x0), ptr(skip), ptr(x_new), ptr(inv), ptr(gains), ptr(o.dx), ptr(o.dx0),
@@ -159,7 +159,7 @@ HeadGrad block_head_bwd(const Tensor& g_new, const Tensor& g_norm, const Tensor&
 
 std::tuple<Tensor, Tensor, Tensor> mix_tail_fwd(const Tensor& x, const Tensor& lam, int64_t T, double eps) {
   chk(x), chk(lam, F32);
-  const int64_t C = x.size(-1), rows = x.numel() / C;
+  const int64_t C = last_dim(x), rows = x.numel() / C;
   Tensor s1 = make_like(x), xn2 = make_like(x), inv = scratch(x, rows);
   TFB_CALL(tfb_mix_tail_fwd, ptr(x), ptr(lam), ptr(s1), ptr(xn2), ptr(inv), rows, C, T, eps, stream());
   return {s1, xn2, inv};
@@ -169,7 +169,7 @@ std::tuple<Tensor, Tensor> mix_tail_bwd(const Tensor& s1, const Tensor& inv, con
                                         const Tensor& ge) {
   chk(s1), chk(x), chk(gy), chk(ge), chk(inv, F32), chk(lam, F32);
   TORCH_CHECK_VALUE(gy.defined() || ge.defined(), "give gy or ge");
-  const int64_t C = s1.size(-1), rows = s1.numel() / C;
+  const int64_t C = last_dim(s1), rows = s1.numel() / C;
   Tensor gx = make_like(s1), part = scratch(s1, tfb_norm_bwd_blocks(rows)), dlam = scratch(s1, 1);
   TFB_CALL(tfb_mix_tail_bwd, ptr(s1), ptr(gy), ptr(ge), ptr(inv), ptr(x), ptr(lam), ptr(gx), ptr(part), ptr(dlam), rows, C, T, stream());
   return {gx, dlam};
@@ -178,7 +178,7 @@ std::tuple<Tensor, Tensor> mix_tail_bwd(const Tensor& s1, const Tensor& inv, con
 // ------------------------------------------------------------------------------------------------------------- fp8 MLP
 Tensor mlp8_backward_scales(const Tensor& dy, const Tensor& row, const Tensor& amax_part) {
   chk(dy), chk(row, F32), chk(amax_part, F32);
-  const int64_t d = dy.size(-1), M = dy.numel() / d;
+  const int64_t d = last_dim(dy), M = dy.numel() / d;
   Tensor out = scratch(dy, 16);
   if (amax_part.defined()) {
     TFB_CALL(tfb_mlp8_backward_scales_part, ptr(amax_part), amax_part.numel(), ptr(row), ptr(out), d, stream());
@@ -204,7 +204,7 @@ Tensor quant_fp8(const Tensor& x, const void* scale_dev, double scale_imm, int f
 }
 // The rows of x and then zeros up to M rows, as bytes; padded: the same in bf16 where x has fewer rows and it is asked for.
 static Tensor quant_rows(const Tensor& x, const void* scale_dev, double scale_imm, int fmt, int64_t M, Tensor* padded) {
-  const int64_t d = x.size(-1);
+  const int64_t d = last_dim(x);
   if (x.numel() == M * d) {
     if (padded) *padded = x;
     return quant_fp8(x, scale_dev, scale_imm, fmt);
@@ -227,7 +227,7 @@ Tensor quant_fp8(const Tensor& x, const Scale& s, int fmt) { return quant_fp8(x,
 Tensor gemm_fp8(const Tensor& a8, const Tensor& b8, int fmt_a, const void* dq_a, const void* dq_b, double dq, const Tensor& res,
                 at::IntArrayRef out_shape) {
   chk(a8, U8), chk(b8, U8), chk(res);
-  const int64_t K = a8.size(-1), M = a8.numel() / K, N = b8.size(0);
+  const int64_t K = last_dim(a8), M = a8.numel() / K, N = b8.size(0);
   TORCH_CHECK_VALUE(b8.dim() == 2 && b8.size(1) == K, "inner dimensions differ");
   TORCH_CHECK_VALUE(!res.defined() || (res.size(-1) == N && res.numel() == M * N), "shapes differ");
   TORCH_CHECK_VALUE(c10::multiply_integers(out_shape) == M * N, "an output ", out_shape, " for ", M, " x ", N);
@@ -242,7 +242,7 @@ Tensor gemm_fp8(const Tensor& a8, const Tensor& b8, int fmt_a, const void* dq_a,
 Tensor gemm_fp8_tn(const Tensor& g8, const Tensor& a8, int fmt_g, int fmt_a, const void* s_g, const void* s_a, double imm, Tensor out,
                    bool accumulate, at::ScalarType out_dtype) {
   chk(g8, U8), chk(a8, U8);
-  const int64_t O = g8.size(-1), M = g8.numel() / O, D = a8.size(-1);
+  const int64_t O = last_dim(g8), M = g8.numel() / O, D = last_dim(a8);
   TORCH_CHECK_VALUE(a8.numel() / D == M, "token counts differ");
   out = Out2::get(out, {O, D}, out_dtype, accumulate, g8);
   const Tensor ws = workspace(g8);
@@ -267,7 +267,7 @@ MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F,
   chk(x), chk(w8, U8), chk(row, F32), chk(x8, U8), chk(res);
   TORCH_CHECK_VALUE(x.defined() || x8.defined(), "give x2 or its bytes x8");
   const Tensor& in = res.defined() ? res : x.defined() ? x : x8;   // (x and x8 may come padded already, res has the call's rows)
-  const int64_t d = in.size(-1), rows = in.numel() / d, M = tile_rows(rows);
+  const int64_t d = last_dim(in), rows = in.numel() / d, M = tile_rows(rows);
   const auto fits = [&](const Tensor& t) { return t.size(-1) == d && (t.numel() == rows * d || t.numel() == M * d); };
   TORCH_CHECK_VALUE(!x8.defined() || (x8.size(-1) == d && x8.numel() == M * d), "x8 shape");
   TORCH_CHECK_VALUE(!x.defined() || fits(x), "res shape");
@@ -288,7 +288,7 @@ MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F,
 
 MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h, bool want_dyp) {
   chk(dy), chk(r), chk(w8, U8), chk(row, F32);
-  const int64_t d = dy.size(-1), M = tile_rows(dy.numel() / d), F = r.size(1);
+  const int64_t d = last_dim(dy), M = tile_rows(dy.numel() / d), F = r.size(1);
   check_rows(r, M, F);
   check_pack(w8, row, d, F);
   MlpBwd o;
@@ -303,7 +303,7 @@ MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tenso
 
 MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, bool want_dpre) {
   chk(dy), chk(r), chk(w8, U8), chk(row, F32);
-  const int64_t d = dy.size(-1), M = tile_rows(dy.numel() / d), F = r.size(1);
+  const int64_t d = last_dim(dy), M = tile_rows(dy.numel() / d), F = r.size(1);
   check_rows(r, M, F);
   check_pack(w8, row, d, F);
   MlpBwd o;
@@ -320,7 +320,7 @@ MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Ten
 void mlp8_dw8(const Tensor& x8, const Tensor& dp8, const Tensor& hq8, const Tensor& dy8, const Tensor& row, const Scale& x_scale,
               Tensor& dw_fc, Tensor& dw_proj, bool accumulate, at::ScalarType out_dtype) {
   chk(x8, U8), chk(dp8, U8), chk(hq8, U8), chk(dy8, U8), chk(row, F32);
-  const int64_t d = x8.size(-1), M = x8.numel() / d, F = dp8.size(1);
+  const int64_t d = last_dim(x8), M = x8.numel() / d, F = dp8.size(1);
   TORCH_CHECK_VALUE(dp8.size(0) == M && hq8.sizes() == dp8.sizes() && dy8.numel() == M * d && dy8.size(-1) == d, "operand shapes");
   TORCH_CHECK_VALUE(dw_fc.defined() == dw_proj.defined(), "give both outputs or neither");
   dw_fc = Out2::get(dw_fc, {F, d}, out_dtype, accumulate, x8);
@@ -333,7 +333,7 @@ void mlp8_dw8(const Tensor& x8, const Tensor& dp8, const Tensor& hq8, const Tens
 
 Tensor mlp_dw_proj(const Tensor& dy, const Tensor& r, Tensor out, bool accumulate, at::ScalarType out_dtype) {
   chk(dy), chk(r);
-  const int64_t d = dy.size(-1), M = dy.numel() / d, F = r.size(1);
+  const int64_t d = last_dim(dy), M = dy.numel() / d, F = r.size(1);
   check_rows(r, M, F);
   out = Out2::get(out, {d, F}, out_dtype, accumulate, dy);
   const Tensor ws = workspace(dy);
@@ -343,7 +343,7 @@ Tensor mlp_dw_proj(const Tensor& dy, const Tensor& r, Tensor out, bool accumulat
 
 std::tuple<Tensor, Tensor> mlp_fwd(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj) {
   chk(x), chk(w_fc), chk(w_proj);
-  const int64_t d = x.size(-1), M = x.numel() / d, F = w_fc.size(0);
+  const int64_t d = last_dim(x), M = x.numel() / d, F = w_fc.size(0);
   TORCH_CHECK_VALUE(w_fc.sizes() == at::IntArrayRef({F, d}) && w_proj.sizes() == at::IntArrayRef({d, F}), "w_fc is [F, d], w_proj is [d, F]");
   Tensor y = make_like(x), r = make({M, F}, BF16, x), h = make({M, F}, BF16, x);
   TFB_CALL(tfb_mlp_fwd, ptr(x), ptr(w_fc), ptr(w_proj), ptr(y), ptr(r), ptr(h), M, d, F, stream());
@@ -352,7 +352,7 @@ std::tuple<Tensor, Tensor> mlp_fwd(const Tensor& x, const Tensor& w_fc, const Te
 
 MlpBwd mlp_bwd(const Tensor& dy, const Tensor& r, const Tensor& w_fc, const Tensor& w_proj, bool want_h) {
   chk(dy), chk(r), chk(w_fc), chk(w_proj);
-  const int64_t d = dy.size(-1), M = dy.numel() / d, F = w_fc.size(0);
+  const int64_t d = last_dim(dy), M = dy.numel() / d, F = w_fc.size(0);
   TORCH_CHECK_VALUE(r.sizes() == at::IntArrayRef({M, F}) && w_fc.sizes() == at::IntArrayRef({F, d}) &&
                         w_proj.sizes() == at::IntArrayRef({d, F}), "shapes differ");
   MlpBwd o;
@@ -503,7 +503,7 @@ void loss_bwd(const Tensor& logits, const Tensor& tg, const Tensor& lse, const T
 
 std::tuple<Tensor, Tensor, Tensor> lmhead_fwd(const Tensor& x, const Tensor& W, const Tensor& tg, double softcap, const Tensor& row_w) {
   chk(x), chk(W), chk(row_w, F32);
-  const int64_t d = x.size(-1), N = x.numel() / d, V = W.size(0);
+  const int64_t d = last_dim(x), N = x.numel() / d, V = W.size(0);
   Tensor logits = make({N, V}, BF16, x), part = scratch(x, N * (V / 64) * 2), loss = scratch(x, N), lse = scratch(x, N);
   TFB_CALL(tfb_lmhead_fwd, ptr(x), ptr(W), ptr(tg), is64(tg), ptr(row_w), ptr(logits), ptr(part), ptr(loss), ptr(lse), N, d, V, softcap,
            stream());
@@ -513,7 +513,7 @@ std::tuple<Tensor, Tensor, Tensor> lmhead_fwd(const Tensor& x, const Tensor& W, 
 // -------------------------------------------------------------------------------------------------- mixture of experts
 MoeRoute moe_route(const Tensor& h, const Tensor& wr, int64_t topk, const Tensor& bias, bool want_logits) {
   chk(h), chk(wr, F32), chk(bias, F32);
-  const int64_t d = h.size(-1), N = h.numel() / d, E = wr.size(0);
+  const int64_t d = last_dim(h), N = h.numel() / d, E = wr.size(0);
   MoeRoute o{make({N, E}, F32, h), make({N, topk}, I32, h), make({N, topk}, F32, h), want_logits ? make({N, E}, F32, h) : Tensor()};
   TFB_CALL(tfb_moe_route, ptr(h), ptr(wr), ptr(bias), ptr(o.logits), ptr(o.p), ptr(o.idx), ptr(o.gate), N, d, E, topk, stream());
   return o;
@@ -543,7 +543,7 @@ MoeTab moe_tables(const Tensor& idx, int64_t E, int64_t seq_len, int64_t capacit
 
 std::tuple<Tensor, Tensor> moe_gather(const Tensor& h, const MoeTab& tab, const Scale* x_scale, bool want_xs) {
   chk(h);
-  const int64_t d = h.size(-1);
+  const int64_t d = last_dim(h);
   Tensor xs, xs8;
   if (want_xs || !x_scale) xs = make({tab.rmax, d}, BF16, h);
   if (x_scale) xs8 = make({tab.rmax, d}, U8, h);
@@ -610,7 +610,7 @@ static Tensor moe_quant_dy(const Tensor& x, const Tensor& rows, const MoeTab& ta
 
 Tensor moe_quant_dout(const Tensor& dout, const Tensor& gate, const Tensor& rows, const MoeTab& tab) {
   chk(dout), chk(gate, F32), chk(rows, F32);
-  const int64_t d = dout.size(-1);
+  const int64_t d = last_dim(dout);
   Tensor out = make({tab.rmax, d}, U8, dout);
   TFB_CALL(tfb_moe_quant_dout, ptr(dout), ptr(tab.tok), ptr(tab.ksel), ptr(gate), ptr(tab.tile_expert), ptr(rows), 5, ptr(out), tab.rmax, d,
            gate.size(1), stream());
@@ -685,7 +685,7 @@ std::tuple<Tensor, Tensor> moe_aux_seq_fwd(const Tensor& p, const Tensor& idx, i
 
 RouteGrad moe_route_bwd(const Tensor& dgate, const Tensor& p, const Tensor& idx, const Tensor& dxs, const MoeTab& tab, const Tensor& h,
                         const Tensor& wr, Tensor dwr, bool accumulate, const MoeAux* aux) {
-  const int64_t d = h.size(-1), N = h.numel() / d, E = wr.size(0), topk = idx.size(1);
+  const int64_t d = last_dim(h), N = h.numel() / d, E = wr.size(0), topk = idx.size(1);
   if (!dwr.defined()) {
     dwr = make({E, d}, F32, h);
     accumulate = false;
