@@ -100,3 +100,31 @@ def test_a_buffer_for_the_norm_gradients_partial_sums_is_checked(dev):
     w.dw_part = torch.zeros(nb, 256, device=dev)
     A.RMSNormFn.apply(x, w, 1e-6).sum().backward()
     assert bool(w.dw_part.any()) and w.grad is None
+
+
+def test_operands_in_another_shape_give_the_same_results(dev):
+    """Residuals, the embedding stream and the skip given as [B, T, H, D] or as rows, or strided: outputs have x's leading shape,
+    values and gradients are those of the same operand in x's own shape, each gradient in its operand's shape."""
+    from trainium_frontier_them_bones_amd import autograd as A, train_api as api
+    B, T, C = 2, 128, 256
+    l = [torch.tensor([v], device=dev) for v in (1.0, 0.3, 0.5)]
+    w, wf, wp = _t(dev, C, C), _t(dev, 512, C), _t(dev, C, 512)
+    st8, st = A.Linear8State(), A.Mlp8State()
+    st8.refresh(w), st.refresh(wf, wp)
+    calls = [lambda x, r: api.tail_norm2(x, r), lambda x, r: (api.final_norm(x, r),), lambda x, r: api.block_head(x, r, l[0], l[1]),
+             lambda x, r: api.head_skip(x, r, r, *l), lambda x, r: (A.LinearFn.apply(x, w, r),),
+             lambda x, r: (A.Linear8Fn.apply(x, w, st8, 4.0, None, r),), lambda x, r: (A.Mlp8Fn.apply(x, wf, wp, st, None, r),)]
+    g = torch.Generator().manual_seed(3)
+    x0, r0, gy = (torch.randn(B, T, C, generator=g).to(bf16).to(dev) for _ in range(3))
+    for i, call in enumerate(calls):
+        want = None
+        for make in (lambda r: r.clone(), lambda r: r.view(B, T, 4, 64).clone(), lambda r: r.view(B * T, C).clone(),
+                     lambda r: r.transpose(1, 2).contiguous().transpose(1, 2)):
+            x, r = x0.clone().requires_grad_(True), make(r0).requires_grad_(True)
+            out = call(x, r)
+            assert all(o.shape == x.shape for o in out), i
+            got = [o.detach() for o in out] + list(torch.autograd.grad(out, (x, r), [gy] * len(out)))
+            assert got[-1].shape == r.shape
+            got[-1] = got[-1].reshape(B, T, C)
+            want = want or got
+            assert all(torch.equal(a, b) for a, b in zip(got, want)), i

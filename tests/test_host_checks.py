@@ -131,3 +131,24 @@ def test_an_empty_last_dimension_raises(A):
             lambda: ops.mlp8_fwd(e, w8, row, 256), lambda: ops.mlp8_bwd(e, _t(128, 256), w8, row), lambda: ops.mlp_dw_proj(e, _t(4, 256)),
             lambda: ops.mlp_bwd(e, _t(4, 256), w, wt), lambda: ops.lmhead_fwd(e, w, tg, 0.0)):
         _refused(fn)
+
+
+def test_operands_of_the_same_rows_may_have_another_shape(A):
+    """An operand that is added to x's rows or mixed into them has x's elements, in any shape; other counts are refused."""
+    from trainium_frontier_them_bones_amd import train_api as api
+    x, heads, more, less = _t(2, 128, 256), _t(2, 128, 4, 64), _t(3, 128, 256), _t(128, 256)
+    one, w = _t(1, dtype=f32), _t(512, 256)
+    wf, wp, st, st8 = _t(512, 256), _t(256, 512), _mlp8_state(A, 512, 256), _linear8_state(A, 512, 256)
+    flat, wide = _t(256, 256), _t(256, 512)
+    for fn in (lambda r: api.tail_norm2(x, r), lambda r: api.final_norm(x, r), lambda r: api.block_head(x, r, one, one),
+               lambda r: api.head_skip(x, r, x, one, one, one), lambda r: api.head_skip(x, x, r, one, one, one),
+               lambda r: A.Mlp8Fn.apply(x, wf, wp, st, None, r)):
+        for r in (x, heads, flat, _t(2, 256, 128).transpose(1, 2)):
+            _passes(lambda: fn(r))
+        for r in (more, less, _t(1, 128, 256)):
+            _refused(lambda: fn(r))
+    for fn in (lambda r: A.LinearFn.apply(x, w, r), lambda r: A.Linear8Fn.apply(x, w, st8, 4.0, None, r)):
+        _passes(lambda: fn(wide))
+        _passes(lambda: fn(_t(2, 128, 8, 64)))
+        _refused(lambda: fn(_t(128, 512)))
+        _refused(lambda: fn(x))

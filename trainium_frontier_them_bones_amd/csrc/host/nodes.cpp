@@ -35,6 +35,14 @@ Tensor val(const OptTensor& t) { return t ? *t : Tensor(); }
 
 at::DimVector dims(const Tensor& t) { return at::DimVector(t.sizes()); }
 
+// An operand that belongs to another's rows may come in any shape of as many elements; its gradient goes back in that shape
+// (and as the very same tensor where the shapes agree: amax partials may hang on it).
+Tensor in_shape(const Tensor& t, at::IntArrayRef shape, const char* what) {
+  TORCH_CHECK_VALUE(t.numel() == c10::multiply_integers(shape), what, " ", t.sizes(), " has not the elements of ", shape);
+  return t.sizes() == shape ? dense(t) : dense(t).view(shape);
+}
+Tensor back_in_shape(const Tensor& g, at::IntArrayRef shape) { return !g.defined() || g.sizes() == shape ? g : g.reshape(shape); }
+
 // ------------------------------------------------------------------------------------------- Python-side conventions
 PyObject* interned(const char* s) { return PyUnicode_InternFromString(s); }
 struct Names {
@@ -256,35 +264,37 @@ struct RmsNormPass : Function<RmsNormPass> {
 struct AddRmsNorm : Function<AddRmsNorm> {
   static Vars forward(AutogradContext* ctx, const Tensor& x, const Tensor& res, const OptTensor& w_, double eps) {
     ctx->set_materialize_grads(false);
-    TORCH_CHECK_VALUE(x.sizes() == res.sizes(), "x and res differ in shape");
     const Tensor w = val(w_);
-    NormOut o = rmsnorm_fwd(dense(x), w, eps, dense(res));
+    NormOut o = rmsnorm_fwd(dense(x), w, eps, in_shape(res, x.sizes(), "res"));
     ctx->save_for_backward({o.s, o.inv, w});
+    keep<at::DimVector>(ctx) = dims(res);
     return {o.s, o.y};
   }
   static Vars backward(AutogradContext* ctx, Vars g) {
-    if (!g[1].defined()) return {g[0], g[0], Tensor(), Tensor()};
+    const at::DimVector& res = kept<at::DimVector>(ctx);
+    if (!g[1].defined()) return {g[0], back_in_shape(g[0], res), Tensor(), Tensor()};
     const auto s = ctx->get_saved_variables();
     NormBack b = norm_backward(g[1], s[0], s[1], s[2], g[0], false);
-    return {b.dx, b.dx, b.gw, Tensor()};
+    return {b.dx, back_in_shape(b.dx, res), b.gw, Tensor()};
   }
 };
 
 struct BlockHead : Function<BlockHead> {
   struct S {
-    bool skip;
-    at::DimVector l1, l2, l3;
+    bool has_skip;
+    at::DimVector l1, l2, l3, x0, skip;
   };
   static Vars forward(AutogradContext* ctx, const Tensor& x_, const Tensor& x0_, const Tensor& l1, const Tensor& l2, const OptTensor& skip_,
                       const OptTensor& l3, double eps) {
     ctx->set_materialize_grads(false);
-    const Tensor x = dense(x_), x0 = dense(x0_), skip = dense(val(skip_));
+    const Tensor x = dense(x_), x0 = in_shape(x0_, x.sizes(), "x0"), skip = skip_ ? in_shape(*skip_, x.sizes(), "skip") : Tensor();
     TORCH_CHECK_TYPE(!skip_ || l3, "a skip needs its gain l3");
     auto one = [](const Tensor& t) { return t.reshape(1).to(F32); };
     const Tensor g1 = one(l1), gains = at::cat({g1, one(l2), skip.defined() ? one(*l3) : g1});   // (the third is unused without a skip)
     auto [x_new, x_norm, inv] = block_head_fwd(x, x0, gains, skip, eps);
     ctx->save_for_backward({x, x0, skip, x_new, inv, gains});
-    keep<S>(ctx) = {skip.defined(), dims(l1), dims(l2), skip.defined() ? dims(*l3) : at::DimVector()};
+    keep<S>(ctx) = {skip.defined(), dims(l1), dims(l2), skip.defined() ? dims(*l3) : at::DimVector(), dims(x0_),
+                    skip.defined() ? dims(*skip_) : at::DimVector()};
     return {x_new, x_norm};
   }
   static Vars backward(AutogradContext* ctx, Vars g) {
@@ -293,7 +303,8 @@ struct BlockHead : Function<BlockHead> {
     const Tensor gn = g[1].defined() ? dense(g[1]) : at::zeros_like(s[0]);
     HeadGrad h = block_head_bwd(dense(g[0]), gn, s[0], s[1], s[3], s[4], s[5], s[2]);
     auto gain = [&](int i, const at::DimVector& shape) { return h.dgains.narrow(0, i, 1).view(shape); };
-    return {h.dx, h.dx0, gain(0, st.l1), gain(1, st.l2), h.dskip, st.skip ? gain(2, st.l3) : Tensor(), Tensor()};
+    return {h.dx, back_in_shape(h.dx0, st.x0), gain(0, st.l1), gain(1, st.l2), back_in_shape(h.dskip, st.skip),
+            st.has_skip ? gain(2, st.l3) : Tensor(), Tensor()};
   }
 };
 
@@ -331,19 +342,23 @@ struct Relu2 : Function<Relu2> {
 
 // ------------------------------------------------------------------------------------------------------ projections
 struct Linear : Function<Linear> {
+  struct S {
+    bool has_res;
+    at::DimVector res;
+  };
   static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w, const OptTensor& res) {
     const Tensor x = dense(x_);
     chk(x), chk(w);
     TORCH_CHECK_VALUE(w.dim() == 2 && last_dim(x) == w.size(1), "inner dimensions differ: ", x.size(-1), " vs ", w.size(1));
     Tensor y;
     if (res) {   // bf16(res + bf16(x @ w^T)): the residual add made in the GEMM's store (nki_attn_nr8.py:1003)
-      y = matmul_res(x, w, dense(*res), true);
+      y = matmul_res(x, w, in_shape(*res, with_last(x, w.size(0)), "res"), true);
     } else {
       y = make(with_last(x, w.size(0)), BF16, x);
       gemm(x, w, y, x.numel() / w.size(1), w.size(0), w.size(1), false, true, false);
     }
     ctx->save_for_backward({x, w});
-    keep<bool>(ctx) = res.has_value();
+    keep<S>(ctx) = {res.has_value(), res ? dims(*res) : at::DimVector()};
     return y;
   }
   static Vars backward(AutogradContext* ctx, Vars g) {
@@ -353,7 +368,8 @@ struct Linear : Function<Linear> {
     chk(gy);
     Tensor dx = make_like(x);
     gemm(gy, w, dx, M, K, N, false, false, false);
-    return {dx, weight_grad(w, gy, x, M, N, K), kept<bool>(ctx) ? g[0] : Tensor()};
+    const S& st = kept<S>(ctx);
+    return {dx, weight_grad(w, gy, x, M, N, K), st.has_res ? back_in_shape(g[0], st.res) : Tensor()};
   }
 };
 
@@ -363,6 +379,7 @@ struct Linear8 : Function<Linear8> {
     Tensor sx;         // the activation's (s, 1/s, amax), or undefined with a constant scale
     double imm = 1;    // 1 / the constant scale
     bool has_res;
+    at::DimVector res;
   };
   static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w, PyObject* state, std::optional<double> x_scale,
                         const OptTensor& x8_, const OptTensor& res) {
@@ -373,10 +390,11 @@ struct Linear8 : Function<Linear8> {
     chk(sc, F32);
     TORCH_CHECK_VALUE(w.dim() == 2 && last_dim(x) == w.size(1), "inner dimensions differ: ", x.size(-1), " vs ", w.size(1));
     TORCH_CHECK_VALUE(w8.sizes() == w.sizes() && sc.numel() >= 2, "the state holds another weight's bytes: ", w8.sizes(), " for ", w.sizes());
-    TORCH_CHECK_VALUE(!x8_ || x8_->numel() == x.numel(), "x8 has ", x8_ ? x8_->sizes() : x.sizes(), " bytes for x ", x.sizes());
+    const Tensor r = res ? in_shape(*res, with_last(x, w.size(0)), "res") : Tensor();
     S& st = keep<S>(ctx);
     st.state = PyRef(state);
     st.has_res = res.has_value();
+    if (res) st.res = dims(*res);
     const float* dqw = static_cast<const float*>(ptr(sc)) + 1;
     const float* dqa = nullptr;
     Tensor x8;
@@ -385,10 +403,10 @@ struct Linear8 : Function<Linear8> {
       x8 = quant_fp8(x, ptr(st.sx), 0, E4M3);
       dqa = static_cast<const float*>(ptr(st.sx)) + 1;
     } else {
-      x8 = x8_ ? dense(*x8_).view(x.sizes()) : quant_fp8(x, nullptr, *x_scale, E4M3);
+      x8 = x8_ ? in_shape(*x8_, x.sizes(), "x8") : quant_fp8(x, nullptr, *x_scale, E4M3);
       st.imm = 1.0 / *x_scale;
     }
-    Tensor y = gemm_fp8(x8, w8, E4M3, dqa, dqw, st.imm, res ? dense(*res) : Tensor(), with_last(x, w.size(0)));
+    Tensor y = gemm_fp8(x8, w8, E4M3, dqa, dqw, st.imm, r, with_last(x, w.size(0)));
     ctx->save_for_backward({dw8 ? x8 : x, w});
     return y;
   }
@@ -415,7 +433,7 @@ struct Linear8 : Function<Linear8> {
     } else {
       dw = weight_grad(w, gy, xa, M, N, K);
     }
-    return {dx, dw, Tensor(), Tensor(), Tensor(), st.has_res ? g[0] : Tensor()};
+    return {dx, dw, Tensor(), Tensor(), Tensor(), st.has_res ? back_in_shape(g[0], st.res) : Tensor()};
   }
 };
 
@@ -638,18 +656,19 @@ struct Mlp8 : Function<Mlp8> {
   struct S {
     PyRef state;
     bool has_res;
+    at::DimVector res;
   };
   static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_fc, const Tensor& w_proj, PyObject* state,
                         const OptTensor& x8_, const OptTensor& res_) {
     const Mlp8Attrs st = mlp8_attrs(state);
-    TORCH_CHECK_VALUE(!x8_ || x8_->numel() == x_.numel(), "x8 has ", x8_ ? x8_->sizes() : x_.sizes(), " bytes for x ", x_.sizes());
-    const Tensor x8 = x8_ ? dense(*x8_).view(x_.sizes()) : Tensor(), res = dense(val(res_));
+    const Tensor x8 = x8_ ? in_shape(*x8_, x_.sizes(), "x8") : Tensor(), res = res_ ? in_shape(*res_, x_.sizes(), "res") : Tensor();
     // with the bytes given and the weight gradients in fp8 nothing reads x itself (it may be a storage-less placeholder)
     const Tensor x = x8.defined() && st.dw_fp8 ? Tensor() : dense(x_);
     MlpFwd f = mlp8_fwd(x, st.w8, st.row, w_fc.size(0), st.x_scale, x8, res, !st.dw_fp8);
     ctx->save_for_backward({st.dw_fp8 ? f.x8 : f.xp.defined() ? f.xp : x, f.r, w_fc, w_proj});
     S& s = keep<S>(ctx);
     s.state = PyRef(state), s.has_res = res_.has_value();
+    if (res_) s.res = dims(*res_);
     return f.y;
   }
   static Vars backward(AutogradContext* ctx, Vars g) {
@@ -661,7 +680,7 @@ struct Mlp8 : Function<Mlp8> {
       st = mlp8_attrs(k.state.o);
     }
     MlpGrads m = mlp8_backward(st, g[0], dense(g[0]), s[0], s[1], s[2], s[3], true);
-    return {m.dx, m.dw_fc, m.dw_proj, Tensor(), Tensor(), k.has_res ? g[0] : Tensor()};
+    return {m.dx, m.dw_fc, m.dw_proj, Tensor(), Tensor(), k.has_res ? back_in_shape(g[0], k.res) : Tensor()};
   }
 };
 
