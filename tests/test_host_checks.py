@@ -152,3 +152,56 @@ def test_operands_of_the_same_rows_may_have_another_shape(A):
         _passes(lambda: fn(_t(2, 128, 8, 64)))
         _refused(lambda: fn(_t(128, 512)))
         _refused(lambda: fn(x))
+
+
+def _node_calls(A):
+    """class -> (all arguments, how many of them are needed)."""
+    x, w, one = _t(2, 128, 256), _t(512, 256), _t(1, dtype=f32)
+    qkv, cos = _t(2, 128, 768), _t(128, 32)
+    q, wf, wp = _t(2, 4, 128, 64), _t(512, 256), _t(256, 512)
+    st, st8, tg = _mlp8_state(A, 512, 256), _linear8_state(A, 512, 256), _t(256, dtype=torch.int64)
+    gain, u, res, logits = _t(256), _t(2, 128, 256, dtype=u8), _t(2, 128, 512), _t(256, 512)
+    router, ef, ep, bias = _t(4, 256, dtype=f32), _t(4, 512, 256), _t(4, 256, 512), _t(4, dtype=f32)
+    return {
+        A.RMSNormFn: ((x, gain, 1e-6), 3), A.RMSNormPassFn: ((x, gain, 1e-6, 4.0, False), 3), A.AddRMSNormFn: ((x, x, gain, 1e-6), 4),
+        A.BlockHeadFn: ((x, x, one, one, x, one, 1e-6), 7), A.MixTailFn: ((x, one, 128), 3), A.Relu2Fn: ((x,), 1),
+        A.LinearFn: ((x, w, res), 2), A.Linear8Fn: ((x, w, st8, 4.0, u, res), 4),
+        A.CausalAttentionFn: ((q, q, q, 0.125, 0), 4), A.RopeAttentionFn: ((qkv, cos, cos, 4, 0.125), 5),
+        A.RopeNormFn: ((_t(2, 128, 4, 64), cos, cos, 1e-6), 4), A.RopeNormAttentionFn: ((qkv, cos, cos, 4, 0.125, 1e-6, 0), 6),
+        A.QkvRopeAttentionFn: ((x, _t(768, 256), cos, cos, 4, 0.125), 6), A.Mlp8Fn: ((x, wf, wp, st, u, x), 4),
+        A.NrMlpFn: ((x, wf, wp, st, 1e-6), 4), A.MlpFusedFn: ((x, wf, wp), 3), A.LmHeadLossFn: ((x, w, tg, 15.0, "mean"), 5),
+        A.EmbeddingFn: ((tg, w), 2), A.MoeMlp8Fn: ((x, router, ef, ep, None, 2, bias, (0.1, 0.1), 8, {}), 7),
+    }
+
+
+def test_nodes_take_their_arguments_and_no_others(A):
+    """A missing argument raises instead of standing for zero (a scale, an epsilon), one too many is not passed over."""
+    for cls, (args, needed) in _node_calls(A).items():
+        for n in range(needed, len(args) + 1):
+            _passes(lambda: cls.apply(*args[:n]))
+        _refused(lambda: cls.apply(*args[:needed - 1]), TypeError)
+        _refused(lambda: cls.apply(*args, None), TypeError)
+        for k, a in enumerate(args[:needed]):
+            if isinstance(a, (float, A.Mlp8State, A.Linear8State)) and (cls, k) not in ((A.Linear8Fn, 3), (A.LmHeadLossFn, 3)):
+                _refused(lambda: cls.apply(*args[:k], None, *args[k + 1:]), TypeError)
+            if type(a) is int:
+                _refused(lambda: cls.apply(*args[:k], None, *args[k + 1:]), TypeError)
+    q = _t(2, 4, 128, 64)
+    _passes(lambda: A.CausalAttentionFn.apply(q, q, q, 0.125, None))                        # no band
+    _passes(lambda: A.LmHeadLossFn.apply(_t(256, 256), _t(512, 256), _t(256, dtype=torch.int64), None, "sum"))   # no softcap
+
+
+def test_wrappers_for_sequences_take_three_dimensions(A):
+    from trainium_frontier_them_bones_amd import train_api as api
+
+    class Module:
+        pass
+
+    mlp = Module()
+    mlp.c_fc, mlp.c_proj, mlp.tfb_mlp8 = Module(), Module(), _mlp8_state(A, 512, 256)
+    mlp.c_fc.weight, mlp.c_proj.weight = _t(512, 256), _t(256, 512)
+    for fn in (lambda x: api.mlp_fused8(mlp, x), lambda x: api.nr_mlp(mlp, x), lambda x: api.mlp_fused(mlp, x),
+               lambda x: api.mix_tail(x, None, _t(1, dtype=f32))):
+        _passes(lambda: fn(_t(2, 128, 256)))
+        _refused(lambda: fn(_t(256, 256)))
+        _refused(lambda: fn(_t(2, 2, 64, 256)))

@@ -35,18 +35,25 @@ struct Args {
     return opt(i);
   }
   OptTensor maybe(int i) const { return has(i) ? OptTensor(opt(i)) : OptTensor(); }
-  double f(int i, double missing = 0.0) const {
-    if (!has(i)) return missing;
+  PyObject* need(int i) const {   // an object that is not None
+    TORCH_CHECK_TYPE(has(i), "argument ", i + 1, " is missing");
+    return a[i];
+  }
+  double f(int i) const {
+    TORCH_CHECK_TYPE(has(i), "argument ", i + 1, " (a number) is missing");
     const double v = PyFloat_AsDouble(a[i]);
     if (v == -1.0 && PyErr_Occurred()) raise_python();
     return v;
   }
-  int64_t i(int k, int64_t missing = 0) const {
-    if (!has(k)) return missing;
+  double f_or(int i, double missing) const { return i < n ? f(i) : missing; }
+  double cap(int i) const { return has(i) ? f(i) : 0.0; }   // a softcap: None stands for none
+  int64_t i(int k) const {
+    TORCH_CHECK_TYPE(has(k), "argument ", k + 1, " (a whole number) is missing");
     const int64_t v = PyLong_AsLongLong(a[k]);
     if (v == -1 && PyErr_Occurred()) raise_python();
     return v;
   }
+  int64_t i_or(int k, int64_t none) const { return has(k) ? i(k) : none; }   // missing or None
   bool b(int i, bool missing = false) const {
     if (i >= n) return missing;
     const int v = PyObject_IsTrue(a[i]);
@@ -86,9 +93,10 @@ PyObject* outs(const Tensors& v) {
 }
 PyObject* none() { Py_RETURN_NONE; }
 
-template <PyObject* (*F)(const Args&)>
+template <PyObject* (*F)(const Args&), int LO, int HI>   // a function of LO to HI arguments
 PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
+  TORCH_CHECK_TYPE(n >= LO && n <= HI, "takes ", LO, LO == HI ? "" : " to " + std::to_string(HI), " arguments (", n, " given)");
   return F({a, n});
   END_HANDLE_TH_ERRORS
 }
@@ -106,17 +114,17 @@ PyObject* py_mix_tail(const Args& a) { return outs(mix_tail_node(a.t(0), a.t(1),
 PyObject* py_relu2(const Args& a) { return out(relu2_node(a.t(0))); }
 PyObject* py_linear(const Args& a) { return out(linear_node(a.t(0), a.t(1), a.maybe(2))); }
 PyObject* py_linear8(const Args& a) {
-  return out(linear8_node(a.t(0), a.t(1), a.obj(2), a.has(3) ? std::optional<double>(a.f(3)) : std::nullopt, a.maybe(4), a.maybe(5)));
+  return out(linear8_node(a.t(0), a.t(1), a.need(2), a.has(3) ? std::optional<double>(a.f(3)) : std::nullopt, a.maybe(4), a.maybe(5)));
 }
-PyObject* py_attention(const Args& a) { return out(attention_node(a.t(0), a.t(1), a.t(2), a.f(3), a.i(4))); }
+PyObject* py_attention(const Args& a) { return out(attention_node(a.t(0), a.t(1), a.t(2), a.f(3), a.i_or(4, 0))); }
 PyObject* py_rope_attention(const Args& a) { return out(rope_attention_node(a.t(0), a.t(1), a.t(2), a.i(3), a.f(4))); }
 PyObject* py_rope_norm(const Args& a) { return out(rope_norm_node(a.t(0), a.t(1), a.t(2), a.f(3))); }
 PyObject* py_rope_norm_attention(const Args& a) {
-  return out(rope_norm_attention_node(a.t(0), a.t(1), a.t(2), a.i(3), a.f(4), a.f(5), a.i(6)));
+  return out(rope_norm_attention_node(a.t(0), a.t(1), a.t(2), a.i(3), a.f(4), a.f(5), a.i_or(6, 0)));
 }
 PyObject* py_qkv_rope_attention(const Args& a) { return out(qkv_rope_attention_node(a.t(0), a.t(1), a.t(2), a.t(3), a.i(4), a.f(5))); }
-PyObject* py_mlp8(const Args& a) { return out(mlp8_node(a.t(0), a.t(1), a.t(2), a.obj(3), a.maybe(4), a.maybe(5))); }
-PyObject* py_nr_mlp(const Args& a) { return out(nr_mlp_node(a.t(0), a.t(1), a.t(2), a.obj(3), a.f(4, std::ldexp(1.0, -23)))); }
+PyObject* py_mlp8(const Args& a) { return out(mlp8_node(a.t(0), a.t(1), a.t(2), a.need(3), a.maybe(4), a.maybe(5))); }
+PyObject* py_nr_mlp(const Args& a) { return out(nr_mlp_node(a.t(0), a.t(1), a.t(2), a.need(3), a.f_or(4, std::ldexp(1.0, -23)))); }
 PyObject* py_mlp_fused(const Args& a) { return out(mlp_fused_node(a.t(0), a.t(1), a.t(2))); }
 PyObject* py_moe(const Args& a) {
   std::vector<double> aux;
@@ -130,17 +138,17 @@ PyObject* py_moe(const Args& a) {
       if (PyErr_Occurred()) raise_python();
     }
   }
-  Tensors r = moe_node(a.t(0), a.t(1), a.t(2), a.t(3), a.obj(4), a.i(5), a.maybe(6), aux, a.i(8, -1), a.obj(9));
+  Tensors r = moe_node(a.t(0), a.t(1), a.t(2), a.t(3), a.obj(4), a.i(5), a.maybe(6), aux, a.i_or(8, -1), a.obj(9));
   return r.size() == 1 ? out(r[0]) : outs(r);
 }
 PyObject* py_lm_head_loss(const Args& a) {
-  return out(lm_head_loss_node(a.t(0), a.t(1), a.t(2), a.f(3), a.is(4, "mean"), a.b(5, true)));
+  return out(lm_head_loss_node(a.t(0), a.t(1), a.t(2), a.cap(3), a.is(4, "mean"), true));
 }
-PyObject* py_loss_rows(const Args& a) { return out(loss_rows_node(a.t(0), a.t(1), a.f(2))); }
-PyObject* py_fused_loss(const Args& a) { return out(fused_loss_node(a.t(0), a.t(1), a.b(2), a.f(3))); }
+PyObject* py_loss_rows(const Args& a) { return out(loss_rows_node(a.t(0), a.t(1), a.cap(2))); }
+PyObject* py_fused_loss(const Args& a) { return out(fused_loss_node(a.t(0), a.t(1), a.b(2), a.cap(3))); }
 PyObject* py_embedding(const Args& a) { return out(embedding_node(a.t(0), a.t(1))); }
 PyObject* py_attach_amax(const Args& a) {
-  attach_amax(a.t(0), a.obj(1));
+  attach_amax(a.t(0), a.need(1));
   return none();
 }
 PyObject* py_amax_hint(const Args& a) {
@@ -222,22 +230,22 @@ PyObject* op_adamw(const Args& a) {   // p, g, m, v, step, lr, beta1, beta2, eps
   adamw(a.t(0), a.t(1), a.t(2), a.t(3), a.f(4), a.f(5), a.f(6), a.f(7), a.f(8), a.f(9), a.opt(10));
   return none();
 }
-PyObject* op_row_weights(const Args& a) { return out(loss_row_weights(targets_of(a.t(0)), a.b(1), a.i(2))); }
+PyObject* op_row_weights(const Args& a) { return out(loss_row_weights(targets_of(a.t(0)), a.b(1), a.i_or(2, 0))); }
 PyObject* op_loss_fwd(const Args& a) {   // logits [N, V], targets, row_w, softcap
   const Tensor x = a.t(0);
-  return outs(loss_fwd(x, targets_of(a.t(1)), a.opt(2), a.f(3), x.size(0), x.size(1)));
+  return outs(loss_fwd(x, targets_of(a.t(1)), a.opt(2), a.cap(3), x.size(0), x.size(1)));
 }
 PyObject* op_loss_fwd_bwd(const Args& a) {
   const Tensor x = a.t(0);
-  return outs(loss_fwd_bwd(x, targets_of(a.t(1)), a.opt(2), a.f(3), x.size(0), x.size(1)));
+  return outs(loss_fwd_bwd(x, targets_of(a.t(1)), a.opt(2), a.cap(3), x.size(0), x.size(1)));
 }
 PyObject* op_loss_bwd(const Args& a) {   // logits, targets, lse, grow, softcap, in place
   const Tensor x = a.t(0), o = a.b(5) ? x : make_like(x);
-  loss_bwd(x, targets_of(a.t(1)), a.t(2), a.t(3), o, a.f(4), x.size(0), x.size(1));
+  loss_bwd(x, targets_of(a.t(1)), a.t(2), a.t(3), o, a.cap(4), x.size(0), x.size(1));
   return out(o);
 }
 PyObject* op_lmhead_fwd(const Args& a) {
-  return outs(lmhead_fwd(a.t(0), a.t(1), targets_of(a.t(2)), a.f(3), a.opt(4)));
+  return outs(lmhead_fwd(a.t(0), a.t(1), targets_of(a.t(2)), a.cap(3), a.opt(4)));
 }
 
 PyObject* set_timed(const Args& a) {
@@ -245,25 +253,31 @@ PyObject* set_timed(const Args& a) {
   return none();
 }
 
-#define FN(name, f) {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<f>)), METH_FASTCALL, nullptr}
+// name, function, the least and the largest number of arguments
+#define FN(name, f, lo, hi) \
+  {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<f, lo, hi>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    FN("rmsnorm", py_rmsnorm), FN("rmsnorm_pass", py_rmsnorm_pass), FN("add_rmsnorm", py_add_rmsnorm), FN("block_head", py_block_head),
-    FN("mix_tail", py_mix_tail), FN("relu2", py_relu2), FN("linear", py_linear), FN("linear8", py_linear8), FN("attention", py_attention),
-    FN("rope_attention", py_rope_attention), FN("rope_norm", py_rope_norm), FN("rope_norm_attention", py_rope_norm_attention),
-    FN("qkv_rope_attention", py_qkv_rope_attention), FN("mlp8", py_mlp8), FN("nr_mlp", py_nr_mlp), FN("mlp_fused", py_mlp_fused),
-    FN("moe", py_moe), FN("lm_head_loss", py_lm_head_loss), FN("loss_rows", py_loss_rows), FN("fused_loss", py_fused_loss),
-    FN("embedding", py_embedding), FN("attach_amax", py_attach_amax), FN("amax_hint", py_amax_hint), FN("set_timed", set_timed),
-    FN("tfb_gemm_bf16", op_gemm), FN("tfb_gemm_bf16_scaled", op_gemm), FN("tfb_gemm_bf16_res", op_gemm_res), FN("tfb_qkv_rope_fwd", op_qkv_rope),
-    FN("tfb_rmsnorm_fwd", op_rmsnorm_fwd), FN("tfb_rmsnorm_fwd_q", op_rmsnorm_fwd_q), FN("tfb_rmsnorm_bwd", op_rmsnorm_bwd),
-    FN("tfb_rmsnorm_bwd_amax", op_rmsnorm_bwd), FN("tfb_block_head_fwd", op_block_head_fwd), FN("tfb_block_head_bwd", op_block_head_bwd),
-    FN("tfb_mix_tail_fwd", op_mix_tail_fwd), FN("tfb_mix_tail_bwd", op_mix_tail_bwd), FN("tfb_mlp8_backward_scales", op_mlp8_backward_scales),
-    FN("tfb_mlp8_backward_scales_part", op_mlp8_backward_scales), FN("tfb_amax_scale", op_amax_scale), FN("tfb_quant_fp8", op_quant_fp8),
-    FN("tfb_gemm_fp8", op_gemm_fp8), FN("tfb_gemm_fp8_res", op_gemm_fp8), FN("tfb_gemm_fp8_tn", op_gemm_fp8_tn), FN("tfb_mlp8_fwd", op_mlp8_fwd),
-    FN("tfb_mlp8_fwd_res", op_mlp8_fwd), FN("tfb_mlp8_bwd", op_mlp8_bwd), FN("tfb_mlp8_bwd_q", op_mlp8_bwd_q), FN("tfb_mlp8_dw8", op_mlp8_dw8),
-    FN("tfb_mlp_dw_proj", op_mlp_dw_proj), FN("tfb_mlp_fwd", op_mlp_fwd), FN("tfb_mlp_bwd", op_mlp_bwd), FN("tfb_relu2", op_relu2),
-    FN("tfb_embedding_fwd", op_embedding_fwd), FN("tfb_fill_f32", op_fill),
-    FN("tfb_adamw", op_adamw), FN("tfb_loss_row_weights", op_row_weights), FN("tfb_loss_fwd", op_loss_fwd),
-    FN("tfb_loss_fwd_bwd", op_loss_fwd_bwd), FN("tfb_loss_bwd", op_loss_bwd), FN("tfb_lmhead_fwd", op_lmhead_fwd),
+    FN("rmsnorm", py_rmsnorm, 3, 3), FN("rmsnorm_pass", py_rmsnorm_pass, 3, 5), FN("add_rmsnorm", py_add_rmsnorm, 4, 4),
+    FN("block_head", py_block_head, 7, 7), FN("mix_tail", py_mix_tail, 3, 3), FN("relu2", py_relu2, 1, 1), FN("linear", py_linear, 2, 3),
+    FN("linear8", py_linear8, 4, 6), FN("attention", py_attention, 4, 5), FN("rope_attention", py_rope_attention, 5, 5),
+    FN("rope_norm", py_rope_norm, 4, 4), FN("rope_norm_attention", py_rope_norm_attention, 6, 7),
+    FN("qkv_rope_attention", py_qkv_rope_attention, 6, 6), FN("mlp8", py_mlp8, 4, 6), FN("nr_mlp", py_nr_mlp, 4, 5),
+    FN("mlp_fused", py_mlp_fused, 3, 3), FN("moe", py_moe, 7, 10), FN("lm_head_loss", py_lm_head_loss, 5, 5), FN("loss_rows", py_loss_rows, 3, 3),
+    FN("fused_loss", py_fused_loss, 4, 4), FN("embedding", py_embedding, 2, 2), FN("attach_amax", py_attach_amax, 2, 2),
+    FN("amax_hint", py_amax_hint, 2, 2), FN("set_timed", set_timed, 1, 1), FN("tfb_gemm_bf16", op_gemm, 7, 7),
+    FN("tfb_gemm_bf16_scaled", op_gemm, 8, 8), FN("tfb_gemm_bf16_res", op_gemm_res, 4, 4), FN("tfb_qkv_rope_fwd", op_qkv_rope, 6, 6),
+    FN("tfb_rmsnorm_fwd", op_rmsnorm_fwd, 4, 4), FN("tfb_rmsnorm_fwd_q", op_rmsnorm_fwd_q, 6, 6), FN("tfb_rmsnorm_bwd", op_rmsnorm_bwd, 9, 9),
+    FN("tfb_rmsnorm_bwd_amax", op_rmsnorm_bwd, 9, 9), FN("tfb_block_head_fwd", op_block_head_fwd, 5, 5),
+    FN("tfb_block_head_bwd", op_block_head_bwd, 8, 8), FN("tfb_mix_tail_fwd", op_mix_tail_fwd, 4, 4), FN("tfb_mix_tail_bwd", op_mix_tail_bwd, 7, 7),
+    FN("tfb_mlp8_backward_scales", op_mlp8_backward_scales, 2, 2), FN("tfb_mlp8_backward_scales_part", op_mlp8_backward_scales, 3, 3),
+    FN("tfb_amax_scale", op_amax_scale, 4, 4), FN("tfb_quant_fp8", op_quant_fp8, 3, 3), FN("tfb_gemm_fp8", op_gemm_fp8, 6, 6),
+    FN("tfb_gemm_fp8_res", op_gemm_fp8, 7, 7), FN("tfb_gemm_fp8_tn", op_gemm_fp8_tn, 10, 10), FN("tfb_mlp8_fwd", op_mlp8_fwd, 6, 6),
+    FN("tfb_mlp8_fwd_res", op_mlp8_fwd, 7, 7), FN("tfb_mlp8_bwd", op_mlp8_bwd, 5, 5), FN("tfb_mlp8_bwd_q", op_mlp8_bwd_q, 6, 6),
+    FN("tfb_mlp8_dw8", op_mlp8_dw8, 10, 10), FN("tfb_mlp_dw_proj", op_mlp_dw_proj, 5, 5), FN("tfb_mlp_fwd", op_mlp_fwd, 3, 3),
+    FN("tfb_mlp_bwd", op_mlp_bwd, 5, 5), FN("tfb_relu2", op_relu2, 3, 3), FN("tfb_embedding_fwd", op_embedding_fwd, 2, 2),
+    FN("tfb_fill_f32", op_fill, 2, 2), FN("tfb_adamw", op_adamw, 11, 11), FN("tfb_loss_row_weights", op_row_weights, 3, 3),
+    FN("tfb_loss_fwd", op_loss_fwd, 4, 4), FN("tfb_loss_fwd_bwd", op_loss_fwd_bwd, 4, 4), FN("tfb_loss_bwd", op_loss_bwd, 6, 6),
+    FN("tfb_lmhead_fwd", op_lmhead_fwd, 5, 5),
     {nullptr, nullptr, 0, nullptr}};
 #undef FN
 

@@ -260,7 +260,9 @@ def fp8_refresh_weights(model, quantise_fn=None, *, e4m3_limit=240.0, x_scale=4.
 def mlp_fused8(mlp, x):
     """MLP.forward on [b, t, n_embd] with the four activation GEMMs in fp8 (R2:6947): c_proj(relu(c_fc(x))^2), weights
     mlp.c_fc.weight [F, d] and mlp.c_proj.weight [d, F]; any number of rows: the byte operands
-    are padded with zeros to a multiple of 128 rows by the kernels that write them (a zero row touches no other row). The scale row and weight bytes come from fp8_refresh_weights (made here on first use)."""
+    are padded with zeros to a multiple of 128 rows by the kernels that write them (a zero row touches no other row). The
+    scale row and weight bytes come from fp8_refresh_weights (made here on first use)."""
+    b, t, c = x.shape   # (another number of dimensions raises)
     if getattr(mlp, "tfb_mlp8", None) is None or mlp.tfb_mlp8.row is None:
         fp8_refresh_weights([mlp])
     w_fc = mlp.c_fc.weight if mlp.c_fc.weight.dtype == bf16 else mlp.c_fc.weight.to(bf16)
@@ -320,6 +322,7 @@ def nr_mlp(mlp, x1):
     (R2:9202 nr_mlp / 9168 NrMlp; kernels K/nki_mlp_nr8.py:1032): the norm's pass also writes the e4m3 operand, the add
     is made in the second GEMM's store, the backward's norm gradient and residual add are one launch. Any
     number of rows, the byte operands padded with zeros to a multiple of 128 by the kernels that write them."""
+    b, t, c = x1.shape   # (another number of dimensions raises)
     if getattr(mlp, "tfb_mlp8", None) is None or mlp.tfb_mlp8.row is None:
         fp8_refresh_weights([mlp])
     if x1.dtype != bf16:
@@ -467,6 +470,7 @@ def mlp_bwd_kernel(dy2, rT, w_fc, w_proj, tb=None, dw_mode=0):
 def mlp_fused(mlp, x):
     """MLP.forward on [b, t, n_embd] through the dense bf16 fused kernels (R2:6782): `mlp` has c_fc.weight [F, d] and
     c_proj.weight [d, F]. Raises TfbError for a shape the kernels do not take (the round-2 policy)."""
+    b, t, c = x.shape   # (another number of dimensions raises)
     return A.MlpFusedFn.apply(x, mlp.c_fc.weight.to(dtype=x.dtype), mlp.c_proj.weight.to(dtype=x.dtype))
 
 
@@ -488,4 +492,5 @@ def shift1(x):
 def mix_tail(x, xn_dead, lam):
     """(s1, xn2) = (x + lam * shift1(x), RMSNorm(s1)) for a [B, T, C] stream in one launch each way (R1:7308). xn_dead (the
     head's unused x_norm) is accepted for the reference's signature and not read."""
-    return A.MixTailFn.apply(x, lam, x.shape[1])
+    B, T, C = x.shape
+    return A.MixTailFn.apply(x, lam, T)
