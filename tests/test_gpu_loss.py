@@ -82,3 +82,20 @@ def test_lse_of_evaluation_is_as_exact_as_that_of_training(dev, N, V, std, cap):
           % (cap, std, N, e.mean(), e.square().mean().sqrt(), p.mean(), p.square().mean().sqrt(), ulp))
     assert abs(e.mean()) < abs(p.mean()) + 0.1 * ulp
     assert e.square().mean().sqrt() < p.square().mean().sqrt() + 0.1 * ulp
+
+
+@pytest.mark.parametrize("cap", [None, 15.0])
+def test_fused_loss_node_gives_the_rows(dev, cap):
+    """FusedLossFn.apply(logits, targets, softcap) is the loss of every row, ReducedLossFn their mean or sum."""
+    from trainium_frontier_them_bones_amd import autograd as A, ops
+    x, t = _rows(dev, 9, 264, 5)
+    t[4] = -1
+    want, _ = ops.loss_fwd(x, t, cap)
+    rows = A.FusedLossFn.apply(x, t, cap)
+    assert rows.shape == (9,) and torch.equal(rows, want)
+    assert torch.allclose(A.ReducedLossFn.apply(x, t, False, cap), want.sum(), rtol=1e-6)
+    assert torch.allclose(A.ReducedLossFn.apply(x, t, True, cap), want.sum() / 8, rtol=1e-6)
+    a, b = x.clone().requires_grad_(True), x.clone().requires_grad_(True)
+    (ga,) = torch.autograd.grad(A.FusedLossFn.apply(a, t, cap).sum(), a)
+    (gb,) = torch.autograd.grad(A.ReducedLossFn.apply(b, t, False, cap), b)
+    assert torch.equal(ga, gb)

@@ -170,19 +170,20 @@ def _node_calls(A):
         A.RopeNormFn: ((_t(2, 128, 4, 64), cos, cos, 1e-6), 4), A.RopeNormAttentionFn: ((qkv, cos, cos, 4, 0.125, 1e-6, 0), 6),
         A.QkvRopeAttentionFn: ((x, _t(768, 256), cos, cos, 4, 0.125), 6), A.Mlp8Fn: ((x, wf, wp, st, u, x), 4),
         A.NrMlpFn: ((x, wf, wp, st, 1e-6), 4), A.MlpFusedFn: ((x, wf, wp), 3), A.LmHeadLossFn: ((x, w, tg, 15.0, "mean"), 5),
-        A.EmbeddingFn: ((tg, w), 2), A.MoeMlp8Fn: ((x, router, ef, ep, None, 2, bias, (0.1, 0.1), 8, {}), 7),
+        A.FusedLossFn: ((logits, tg, 15.0), 3), A.ReducedLossFn: ((logits, tg, True, 15.0), 4), A.EmbeddingFn: ((tg, w), 2), A.MoeMlp8Fn: ((x, router, ef, ep, None, 2, bias, (0.1, 0.1), 8, {}), 7),
     }
 
 
 def test_nodes_take_their_arguments_and_no_others(A):
     """A missing argument raises instead of standing for zero (a scale, an epsilon), one too many is not passed over."""
+    may_be_none = ((A.Linear8Fn, 3), (A.LmHeadLossFn, 3), (A.FusedLossFn, 2), (A.ReducedLossFn, 3))   # a scale, a softcap
     for cls, (args, needed) in _node_calls(A).items():
         for n in range(needed, len(args) + 1):
             _passes(lambda: cls.apply(*args[:n]))
         _refused(lambda: cls.apply(*args[:needed - 1]), TypeError)
         _refused(lambda: cls.apply(*args, None), TypeError)
         for k, a in enumerate(args[:needed]):
-            if isinstance(a, (float, A.Mlp8State, A.Linear8State)) and (cls, k) not in ((A.Linear8Fn, 3), (A.LmHeadLossFn, 3)):
+            if isinstance(a, (float, A.Mlp8State, A.Linear8State)) and (cls, k) not in may_be_none:
                 _refused(lambda: cls.apply(*args[:k], None, *args[k + 1:]), TypeError)
             if type(a) is int:
                 _refused(lambda: cls.apply(*args[:k], None, *args[k + 1:]), TypeError)

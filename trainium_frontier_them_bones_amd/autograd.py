@@ -184,15 +184,15 @@ class LmHeadLossFn:
     apply = _Node("lm_head_loss")
 
 
-class LossRowsFn:
-    """(logits, targets, softcap): the row losses [N] of materialised logits (round1/source/train.py:4691, reduction "none")."""
-    apply = _Node("loss_rows")
-
-
 class FusedLossFn:
+    """(logits, targets, softcap): the row losses [N] of materialised logits (round1/source/train.py:4691, reduction "none")."""
+    apply = _Node("fused_loss")
+
+
+class ReducedLossFn:
     """(logits, targets, mean, softcap): the reduced loss of materialised logits, the mean over the rows whose target counts or
     the sum (round1/source/train.py:4691): the reduction is a weight per row, made in one launch."""
-    apply = _Node("fused_loss")
+    apply = _Node("reduced_loss")
 
 
 class FusedLossMultiFn(torch.autograd.Function):

@@ -144,8 +144,8 @@ PyObject* py_moe(const Args& a) {
 PyObject* py_lm_head_loss(const Args& a) {
   return out(lm_head_loss_node(a.t(0), a.t(1), a.t(2), a.cap(3), a.is(4, "mean"), true));
 }
-PyObject* py_loss_rows(const Args& a) { return out(loss_rows_node(a.t(0), a.t(1), a.cap(2))); }
-PyObject* py_fused_loss(const Args& a) { return out(fused_loss_node(a.t(0), a.t(1), a.b(2), a.cap(3))); }
+PyObject* py_fused_loss(const Args& a) { return out(fused_loss_node(a.t(0), a.t(1), a.cap(2))); }
+PyObject* py_reduced_loss(const Args& a) { return out(reduced_loss_node(a.t(0), a.t(1), a.b(2), a.cap(3))); }
 PyObject* py_embedding(const Args& a) { return out(embedding_node(a.t(0), a.t(1))); }
 PyObject* py_attach_amax(const Args& a) {
   attach_amax(a.t(0), a.need(1));
@@ -262,8 +262,8 @@ PyMethodDef methods[] = {
     FN("linear8", py_linear8, 4, 6), FN("attention", py_attention, 4, 5), FN("rope_attention", py_rope_attention, 5, 5),
     FN("rope_norm", py_rope_norm, 4, 4), FN("rope_norm_attention", py_rope_norm_attention, 6, 7),
     FN("qkv_rope_attention", py_qkv_rope_attention, 6, 6), FN("mlp8", py_mlp8, 4, 6), FN("nr_mlp", py_nr_mlp, 4, 5),
-    FN("mlp_fused", py_mlp_fused, 3, 3), FN("moe", py_moe, 7, 10), FN("lm_head_loss", py_lm_head_loss, 5, 5), FN("loss_rows", py_loss_rows, 3, 3),
-    FN("fused_loss", py_fused_loss, 4, 4), FN("embedding", py_embedding, 2, 2), FN("attach_amax", py_attach_amax, 2, 2),
+    FN("mlp_fused", py_mlp_fused, 3, 3), FN("moe", py_moe, 7, 10), FN("lm_head_loss", py_lm_head_loss, 5, 5), FN("fused_loss", py_fused_loss, 3, 3),
+    FN("reduced_loss", py_reduced_loss, 4, 4), FN("embedding", py_embedding, 2, 2), FN("attach_amax", py_attach_amax, 2, 2),
     FN("amax_hint", py_amax_hint, 2, 2), FN("set_timed", set_timed, 1, 1), FN("tfb_gemm_bf16", op_gemm, 7, 7),
     FN("tfb_gemm_bf16_scaled", op_gemm, 8, 8), FN("tfb_gemm_bf16_res", op_gemm_res, 4, 4), FN("tfb_qkv_rope_fwd", op_qkv_rope, 6, 6),
     FN("tfb_rmsnorm_fwd", op_rmsnorm_fwd, 4, 4), FN("tfb_rmsnorm_fwd_q", op_rmsnorm_fwd_q, 6, 6), FN("tfb_rmsnorm_bwd", op_rmsnorm_bwd, 9, 9),

@@ -904,7 +904,7 @@ struct LmHeadLoss : Function<LmHeadLoss> {
   }
 };
 
-struct LossRows : Function<LossRows> {
+struct FusedLoss : Function<FusedLoss> {
   struct S {
     double softcap;
   };
@@ -927,7 +927,7 @@ struct LossRows : Function<LossRows> {
 };
 
 // The reduced loss (sum, or mean over the rows whose target counts) as one node: the reduction is a weight per row.
-struct FusedLoss : Function<FusedLoss> {
+struct ReducedLoss : Function<ReducedLoss> {
   struct S {
     double softcap;
   };
@@ -1034,9 +1034,9 @@ Tensor lm_head_loss_node(const Tensor& x, const Tensor& W, const Tensor& targets
   const bool one = allow_one_pass && at::GradMode::is_enabled() && (x.requires_grad() || W.requires_grad()) && W.size(0) <= 65536;
   return LmHeadLoss::apply(x, W, targets, softcap, mean, one);
 }
-Tensor loss_rows_node(const Tensor& logits, const Tensor& targets, double softcap) { return LossRows::apply(logits, targets, softcap); }
-Tensor fused_loss_node(const Tensor& logits, const Tensor& targets, bool mean, double softcap) {
-  return FusedLoss::apply(logits, targets, mean, softcap);
+Tensor fused_loss_node(const Tensor& logits, const Tensor& targets, double softcap) { return FusedLoss::apply(logits, targets, softcap); }
+Tensor reduced_loss_node(const Tensor& logits, const Tensor& targets, bool mean, double softcap) {
+  return ReducedLoss::apply(logits, targets, mean, softcap);
 }
 Tensor embedding_node(const Tensor& idx, const Tensor& w) { return Embedding::apply(idx, w); }
 

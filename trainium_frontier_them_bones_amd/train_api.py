@@ -82,10 +82,10 @@ def fused_loss(logits, targets, reduction="mean", softcap=LOGIT_SOFTCAP):
     """The static cross-entropy chain on the raw lm_head output (R1:4691): softcap * tanh(logits / softcap), log-softmax,
     ignore_index -1; reduction "mean" (over the targets not ignored), "sum" or "none" (rows in targets' shape)."""
     if reduction == "none":
-        return A.LossRowsFn.apply(logits.contiguous(), targets, softcap).view(targets.shape)
+        return A.FusedLossFn.apply(logits.contiguous(), targets, softcap).view(targets.shape)
     if reduction not in ("mean", "sum"):
         raise ValueError("reduction must be 'mean', 'sum' or 'none'")
-    return A.FusedLossFn.apply(logits, targets, reduction == "mean", softcap)   # (the rows the kernel gives a loss to)
+    return A.ReducedLossFn.apply(logits, targets, reduction == "mean", softcap)   # (the rows the kernel gives a loss to)
 
 
 def fused_loss_multi(logits, tg, rw, softcap=LOGIT_SOFTCAP, ref=None):
