@@ -128,3 +128,19 @@ def test_operands_in_another_shape_give_the_same_results(dev):
             got[-1] = got[-1].reshape(B, T, C)
             want = want or got
             assert all(torch.equal(a, b) for a, b in zip(got, want)), i
+
+
+def test_attention_nodes_on_a_projection_give_rows(dev):
+    """The nodes that take the fused projection [B, T, 3C] return [B, T, C]; the wrapper returns the heads [B, T, H, D] of the
+    same values, and their gradients agree."""
+    from oracle import attention as O
+    from trainium_frontier_them_bones_amd import autograd as A, train_api as api
+    B, T, H, D = 2, 128, 2, 64
+    cos, sin = (t.to(dev) for t in O.rope_tables(T, D))
+    qkv, gy = _t(dev, B, T, 3 * H * D, grad=True), _t(dev, B, T, H * D)
+    y = A.RopeNormAttentionFn.apply(qkv, cos, sin, H, 0.125, api.RMS_EPS)
+    z = api.nki_rope_attention(qkv, cos, sin, H, 0.125)
+    assert y.shape == (B, T, H * D) and z.shape == (B, T, H, D) and torch.equal(y, z.reshape(B, T, H * D))
+    (ga,), (gb,) = torch.autograd.grad(y, qkv, gy), torch.autograd.grad(z, qkv, gy.view(B, T, H, D))
+    assert torch.equal(ga, gb)
+    assert A.RopeAttentionFn.apply(qkv, cos, sin, H, 0.125).shape == (B, T, H * D)

@@ -168,7 +168,7 @@ def _node_calls(A):
         A.LinearFn: ((x, w, res), 2), A.Linear8Fn: ((x, w, st8, 4.0, u, res), 4),
         A.CausalAttentionFn: ((q, q, q, 0.125, 0), 4), A.RopeAttentionFn: ((qkv, cos, cos, 4, 0.125), 5),
         A.RopeNormFn: ((_t(2, 128, 4, 64), cos, cos, 1e-6), 4), A.RopeNormAttentionFn: ((qkv, cos, cos, 4, 0.125, 1e-6, 0), 6),
-        A.QkvRopeAttentionFn: ((x, _t(768, 256), cos, cos, 4, 0.125), 6), A.Mlp8Fn: ((x, wf, wp, st, u, x), 4),
+        A.RopeNormAttentionHeadsFn: ((qkv, cos, cos, 4, 0.125, 1e-6, 0), 6), A.QkvRopeAttentionFn: ((x, _t(768, 256), cos, cos, 4, 0.125), 6), A.Mlp8Fn: ((x, wf, wp, st, u, x), 4),
         A.NrMlpFn: ((x, wf, wp, st, 1e-6), 4), A.MlpFusedFn: ((x, wf, wp), 3), A.LmHeadLossFn: ((x, w, tg, 15.0, "mean"), 5),
         A.FusedLossFn: ((logits, tg, 15.0), 3), A.ReducedLossFn: ((logits, tg, True, 15.0), 4), A.EmbeddingFn: ((tg, w), 2), A.MoeMlp8Fn: ((x, router, ef, ep, None, 2, bias, (0.1, 0.1), 8, {}), 7),
     }

@@ -103,10 +103,15 @@ class RopeNormFn:
 
 class RopeNormAttentionFn:
     """(qkv, cos, sin, n_head, scale, eps[, band]): nki_rope_attention (round1/source/train.py:8197, NkiRopeAttnFn 8135): causal
-    SDPA(QKnorm(RoPE(q)), QKnorm(RoPE(k)), v) straight from the fused projection output qkv [B, T, 3C] -> [B, T, H, D], one dqkv
+    SDPA(QKnorm(RoPE(q)), QKnorm(RoPE(k)), v) straight from the fused projection output qkv [B, T, 3C] -> [B, T, C], one dqkv
     [B, T, 3C] back. The input is not modified: the normalised q and k go to a fresh buffer, v is read in place through strides.
     band = nw > 0: the tile-band form (round2/source/train.py:4925 fused_rope_attention_band)."""
     apply = _Node("rope_norm_attention")
+
+
+class RopeNormAttentionHeadsFn:
+    """RopeNormAttentionFn with the result as [B, T, H, D], without a view node after it."""
+    apply = _Node("rope_norm_attention_heads")
 
 
 class QkvRopeAttentionFn:

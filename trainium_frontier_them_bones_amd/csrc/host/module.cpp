@@ -119,8 +119,9 @@ PyObject* py_linear8(const Args& a) {
 PyObject* py_attention(const Args& a) { return out(attention_node(a.t(0), a.t(1), a.t(2), a.f(3), a.i_or(4, 0))); }
 PyObject* py_rope_attention(const Args& a) { return out(rope_attention_node(a.t(0), a.t(1), a.t(2), a.i(3), a.f(4))); }
 PyObject* py_rope_norm(const Args& a) { return out(rope_norm_node(a.t(0), a.t(1), a.t(2), a.f(3))); }
+template <bool HEADS>
 PyObject* py_rope_norm_attention(const Args& a) {
-  return out(rope_norm_attention_node(a.t(0), a.t(1), a.t(2), a.i(3), a.f(4), a.f(5), a.i_or(6, 0)));
+  return out(rope_norm_attention_node(a.t(0), a.t(1), a.t(2), a.i(3), a.f(4), a.f(5), a.i_or(6, 0), HEADS));
 }
 PyObject* py_qkv_rope_attention(const Args& a) { return out(qkv_rope_attention_node(a.t(0), a.t(1), a.t(2), a.t(3), a.i(4), a.f(5))); }
 PyObject* py_mlp8(const Args& a) { return out(mlp8_node(a.t(0), a.t(1), a.t(2), a.need(3), a.maybe(4), a.maybe(5))); }
@@ -260,7 +261,8 @@ PyMethodDef methods[] = {
     FN("rmsnorm", py_rmsnorm, 3, 3), FN("rmsnorm_pass", py_rmsnorm_pass, 3, 5), FN("add_rmsnorm", py_add_rmsnorm, 4, 4),
     FN("block_head", py_block_head, 7, 7), FN("mix_tail", py_mix_tail, 3, 3), FN("relu2", py_relu2, 1, 1), FN("linear", py_linear, 2, 3),
     FN("linear8", py_linear8, 4, 6), FN("attention", py_attention, 4, 5), FN("rope_attention", py_rope_attention, 5, 5),
-    FN("rope_norm", py_rope_norm, 4, 4), FN("rope_norm_attention", py_rope_norm_attention, 6, 7),
+    FN("rope_norm", py_rope_norm, 4, 4), FN("rope_norm_attention", py_rope_norm_attention<false>, 6, 7),
+    FN("rope_norm_attention_heads", py_rope_norm_attention<true>, 6, 7),
     FN("qkv_rope_attention", py_qkv_rope_attention, 6, 6), FN("mlp8", py_mlp8, 4, 6), FN("nr_mlp", py_nr_mlp, 4, 5),
     FN("mlp_fused", py_mlp_fused, 3, 3), FN("moe", py_moe, 7, 10), FN("lm_head_loss", py_lm_head_loss, 5, 5), FN("fused_loss", py_fused_loss, 3, 3),
     FN("reduced_loss", py_reduced_loss, 4, 4), FN("embedding", py_embedding, 2, 2), FN("attach_amax", py_attach_amax, 2, 2),

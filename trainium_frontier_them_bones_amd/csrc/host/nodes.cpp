@@ -542,13 +542,13 @@ struct RopeNorm : Function<RopeNorm> {
 
 struct RopeNormAttention : Function<RopeNormAttention> {
   static Tensor forward(AutogradContext* ctx, const Tensor& qkv_, const Tensor& cos, const Tensor& sin, int64_t n_head, double scale,
-                        double eps, int64_t band) {
+                        double eps, int64_t band, bool heads) {
     const Tensor qkv = dense(qkv_);
     const QkvDims m = qkv_dims(qkv, n_head, scale, band);
     const int64_t rows = m.B * m.T, R = 2 * m.C;
     const Tensor qk = make({rows, R}, BF16, qkv), r = make({rows, R}, BF16, qkv), inv = make({rows, 2 * m.H}, F32, qkv);
     rope_norm_fwd(qkv, cos, sin, r, qk, inv, rows, m.T, 2 * m.H, m.D, 3 * m.C, eps);
-    Tensor o = make({m.B, m.T, m.H, m.D}, BF16, qkv), lse = make({m.B, m.H, m.T}, F32, qkv);
+    Tensor o = heads ? make({m.B, m.T, m.H, m.D}, BF16, qkv) : make({m.B, m.T, m.C}, BF16, qkv), lse = make({m.B, m.H, m.T}, F32, qkv);
     attn_fwd(third(qk, 0, m.T, m.C, m.D, R), third(qk, 1, m.T, m.C, m.D, R), third(qkv, 2, m.T, m.C, m.D, 3 * m.C), o, lse, m.B, m.H, m.T, m.D,
              scale, band);
     ctx->save_for_backward({qkv, qk, r, inv, o, lse, cos, sin});
@@ -566,7 +566,7 @@ struct RopeNormAttention : Function<RopeNormAttention> {
              third(dqkv, 0, m.T, m.C, m.D, F), third(dqkv, 1, m.T, m.C, m.D, F), third(dqkv, 2, m.T, m.C, m.D, F), s[5], {}, {}, m.B, m.H, m.T,
              m.D, m.scale, m.band);
     rope_norm_bwd(dqkv, s[2], s[3], s[6], s[7], dqkv, m.B * m.T, m.T, 2 * m.H, m.D, F, F);   // in place on the q and k thirds
-    return {dqkv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    return {dqkv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -1012,8 +1012,8 @@ Tensor rope_attention_node(const Tensor& qkv, const Tensor& cos, const Tensor& s
 }
 Tensor rope_norm_node(const Tensor& x, const Tensor& cos, const Tensor& sin, double eps) { return RopeNorm::apply(x, cos, sin, eps); }
 Tensor rope_norm_attention_node(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t n_head, double scale, double eps,
-                                int64_t band) {
-  return RopeNormAttention::apply(qkv, cos, sin, n_head, scale, eps, band);
+                                int64_t band, bool heads) {
+  return RopeNormAttention::apply(qkv, cos, sin, n_head, scale, eps, band, heads);
 }
 Tensor qkv_rope_attention_node(const Tensor& x, const Tensor& w, const Tensor& cos, const Tensor& sin, int64_t n_head, double scale) {
   return QkvRopeAttention::apply(x, w, cos, sin, n_head, scale);

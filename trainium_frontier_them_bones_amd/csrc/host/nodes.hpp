@@ -22,7 +22,7 @@ Tensor attention_node(const Tensor& q, const Tensor& k, const Tensor& v, double 
 Tensor rope_attention_node(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t n_head, double scale);
 Tensor rope_norm_node(const Tensor& x, const Tensor& cos, const Tensor& sin, double eps);
 Tensor rope_norm_attention_node(const Tensor& qkv, const Tensor& cos, const Tensor& sin, int64_t n_head, double scale, double eps,
-                                int64_t band);
+                                int64_t band, bool heads);   // [B, T, C], or [B, T, H, D]
 Tensor qkv_rope_attention_node(const Tensor& x, const Tensor& w, const Tensor& cos, const Tensor& sin, int64_t n_head, double scale);
 Tensor mlp8_node(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj, PyObject* state, const OptTensor& x8, const OptTensor& res);
 Tensor nr_mlp_node(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj, PyObject* state, double eps);

@@ -73,8 +73,7 @@ def nki_rope_attention(qkv, cos, sin, n_head, scale=None, nw=None):
         return None
     sc = float(scale) if scale is not None else 1.0 / math.sqrt(D)
     c, s = _tables_2d(cos, sin, T, D // 2)
-    y = _none_if_shape(A.RopeNormAttentionFn.apply, qkv, c, s, n_head, sc, RMS_EPS, int(nw) if nw else 0)
-    return y
+    return _none_if_shape(A.RopeNormAttentionHeadsFn.apply, qkv, c, s, n_head, sc, RMS_EPS, int(nw) if nw else 0)
 
 
 # ------------------------------------------------------------------------------------------ loss head (R1:4691, 4908; R2:6364)
