@@ -99,3 +99,31 @@ def test_fused_loss_node_gives_the_rows(dev, cap):
     (ga,) = torch.autograd.grad(A.FusedLossFn.apply(a, t, cap).sum(), a)
     (gb,) = torch.autograd.grad(A.ReducedLossFn.apply(b, t, False, cap), b)
     assert torch.equal(ga, gb)
+
+
+def test_the_switch_for_the_one_pass_loss_head(dev, monkeypatch):
+    """autograd.LM_HEAD_ONE_PASS = False takes the loss and its gradient in two passes: other launches, the same values."""
+    from trainium_frontier_them_bones_amd import _lib, autograd as A
+    g = torch.Generator().manual_seed(8)
+    x = torch.randn(128, 128, generator=g).to(bf16).to(dev).requires_grad_(True)
+    W = (0.05 * torch.randn(1024, 128, generator=g)).to(bf16).to(dev).requires_grad_(True)
+    t = torch.randint(0, 1024, (128,), generator=g).to(dev)
+
+    def step():
+        rec = []
+        _lib.TIMED["*"] = rec
+        try:
+            loss = A.LmHeadLossFn.apply(x, W, t, 15.0, "mean")
+            grads = torch.autograd.grad(loss, (x, W))
+        finally:
+            del _lib.TIMED["*"]
+        return loss.item(), grads, {r[2] for r in rec}
+
+    one, grads1, names1 = step()
+    monkeypatch.setattr(A, "LM_HEAD_ONE_PASS", False)
+    two, grads2, names2 = step()
+    assert "tfb_loss_fwd_bwd" in names1 and "tfb_loss_fwd_bwd" not in names2
+    assert {"tfb_lmhead_fwd", "tfb_loss_bwd"} <= names2
+    assert abs(one - two) < 1e-6 * one
+    for a, b in zip(grads1, grads2):
+        assert (a.float() - b.float()).norm() < 5e-3 * b.float().norm()

@@ -179,6 +179,9 @@ class NrMlpFn:
     apply = _Node("nr_mlp")
 
 
+LM_HEAD_ONE_PASS = True   # False: LmHeadLossFn always takes the GEMM with the lse epilogue and the separate loss backward
+
+
 class LmHeadLossFn:
     """(x, W, targets, softcap, reduction): loss = reduce(CE(softcap(x @ W^T), targets)). When a gradient is wanted the forward is
     the plain LM-head GEMM followed by ONE pass over the logits that writes lse and the row losses and leaves, in place of the

@@ -143,7 +143,7 @@ PyObject* py_moe(const Args& a) {
   return r.size() == 1 ? out(r[0]) : outs(r);
 }
 PyObject* py_lm_head_loss(const Args& a) {
-  return out(lm_head_loss_node(a.t(0), a.t(1), a.t(2), a.cap(3), a.is(4, "mean"), true));
+  return out(lm_head_loss_node(a.t(0), a.t(1), a.t(2), a.cap(3), a.is(4, "mean")));
 }
 PyObject* py_fused_loss(const Args& a) { return out(fused_loss_node(a.t(0), a.t(1), a.cap(2))); }
 PyObject* py_reduced_loss(const Args& a) { return out(reduced_loss_node(a.t(0), a.t(1), a.b(2), a.cap(3))); }

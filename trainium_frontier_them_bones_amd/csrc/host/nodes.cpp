@@ -49,7 +49,7 @@ struct Names {
   PyObject *grad_buf = interned("grad_buf"), *grad_fresh = interned("grad_fresh"), *dw_part = interned("dw_part"),
            *amax = interned("_tfb_amax_part"), *w8 = interned("w8"), *w8t = interned("w8t"), *row = interned("row"), *rows = interned("rows"),
            *x_scale = interned("x_scale"), *limit = interned("limit"), *e4m3_limit = interned("e4m3_limit"), *dw_fp8 = interned("dw_fp8"),
-           *sc = interned("sc"), *use_amax = interned("USE_AMAX_HINT");
+           *sc = interned("sc"), *use_amax = interned("USE_AMAX_HINT"), *one_pass = interned("LM_HEAD_ONE_PASS");
 };
 const Names& names() {
   static const Names* n = new Names;
@@ -96,6 +96,13 @@ Scale scale_attr(PyObject* o, PyObject* name) {   // a float, or a one-element f
   Py_XDECREF(a);
   s.imm = float_attr(o, name);
   return s;
+}
+
+// A switch of the Python module autograd (missing: off). Under the GIL.
+bool switched_on(PyObject* name) {
+  static PyObject* dict = PyModule_GetDict(PyImport_ImportModule("trainium_frontier_them_bones_amd.autograd"));
+  PyObject* v = PyDict_GetItem(dict, name);
+  return v && PyObject_IsTrue(v) == 1;
 }
 
 struct GradBuf {
@@ -190,9 +197,7 @@ PyObject* call_python(PyObject* fn, std::initializer_list<PyObject*> args) {   /
 // it.
 Tensor backward_scales(const Tensor& gy, const Tensor& g2, const Tensor& row) {
   pybind11::gil_scoped_acquire gil;
-  static PyObject* fn_dict = PyModule_GetDict(PyImport_ImportModule("trainium_frontier_them_bones_amd.autograd"));
-  PyObject* use = PyDict_GetItem(fn_dict, names().use_amax);
-  PyObject* hint = use && PyObject_IsTrue(use) ? amax_hint(gy, g2) : nullptr;
+  PyObject* hint = switched_on(names().use_amax) ? amax_hint(gy, g2) : nullptr;
   if (PyObject* fn = replaced("mlp8_backward_scales")) return tensor_of(call_python(fn, {THPVariable_Wrap(g2), THPVariable_Wrap(row), hint}));
   return mlp8_backward_scales(g2, row, tensor_of(hint));
 }
@@ -1029,9 +1034,10 @@ Tensors moe_node(const Tensor& h, const Tensor& router, const Tensor& w_fc, cons
                  const OptTensor& bias, const std::vector<double>& aux, int64_t capacity, PyObject* info) {
   return Moe::apply(h, router, w_fc, w_proj, st, topk, bias, aux, capacity, info);
 }
-Tensor lm_head_loss_node(const Tensor& x, const Tensor& W, const Tensor& targets, double softcap, bool mean, bool allow_one_pass) {
+Tensor lm_head_loss_node(const Tensor& x, const Tensor& W, const Tensor& targets, double softcap, bool mean) {
   // the one-pass form pays when a gradient is wanted and a row of logits fits the kernel's registers
-  const bool one = allow_one_pass && at::GradMode::is_enabled() && (x.requires_grad() || W.requires_grad()) && W.size(0) <= 65536;
+  const bool one = at::GradMode::is_enabled() && (x.requires_grad() || W.requires_grad()) && W.size(0) <= 65536 &&
+                   switched_on(names().one_pass);
   return LmHeadLoss::apply(x, W, targets, softcap, mean, one);
 }
 Tensor fused_loss_node(const Tensor& logits, const Tensor& targets, double softcap) { return FusedLoss::apply(logits, targets, softcap); }

@@ -29,7 +29,7 @@ Tensor nr_mlp_node(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj, Py
 Tensor mlp_fused_node(const Tensor& x, const Tensor& w_fc, const Tensor& w_proj);
 Tensors moe_node(const Tensor& h, const Tensor& router, const Tensor& w_fc, const Tensor& w_proj, PyObject* state, int64_t topk,
                  const OptTensor& bias, const std::vector<double>& aux_weights, int64_t capacity, PyObject* info);
-Tensor lm_head_loss_node(const Tensor& x, const Tensor& W, const Tensor& targets, double softcap, bool mean, bool allow_one_pass);
+Tensor lm_head_loss_node(const Tensor& x, const Tensor& W, const Tensor& targets, double softcap, bool mean);
 Tensor fused_loss_node(const Tensor& logits, const Tensor& targets, double softcap);
 Tensor reduced_loss_node(const Tensor& logits, const Tensor& targets, bool mean, double softcap);
 Tensor embedding_node(const Tensor& idx, const Tensor& w);
