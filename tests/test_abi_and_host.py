@@ -147,3 +147,23 @@ def test_every_entry_point_rejects_null_pointers_and_empty_shapes_on_the_host():
                 else:
                     args.append(0)
             assert getattr(L, name)(*args) in (1, 2), (name, null)
+
+
+def test_every_change_of_the_table_of_timed_entry_points_is_told_to_the_native_layer(monkeypatch):
+    """The native layer asks for events only while the table holds something: each way to change a dict tells it, before the
+    extension is loaded (the state is handed over at the load) and after."""
+    from trainium_frontier_them_bones_amd import _lib
+    told = []
+    monkeypatch.setitem(_lib.native.__dict__, "set_timed", told.append)
+    t = _lib.TIMED
+    assert not t
+    steps = [(lambda: t.__setitem__("a", []), True), (lambda: t.__delitem__("a"), False), (lambda: t.update(a=[], b=[]), True),
+             (lambda: t.pop("a"), True), (lambda: t.popitem(), False), (lambda: t.setdefault("c", []), True), (lambda: t.clear(), False),
+             (lambda: t.__ior__({"d": []}), True), (lambda: t.pop("nothing", None), True), (lambda: t.clear(), False)]
+    for step, want in steps:
+        step()
+        assert told.pop() is want and not told and bool(t) is want
+    monkeypatch.delitem(_lib.native.__dict__, "set_timed")
+    t["a"] = []                                            # nothing is loaded for it
+    assert "set_timed" not in _lib.native.__dict__
+    t.clear()

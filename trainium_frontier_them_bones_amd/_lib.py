@@ -147,15 +147,21 @@ def lib():
 class _Timed(dict):
     """name -> list: when an entry point is listed here every call is bracketed by events on torch's current stream (the
     stream the kernels are launched on) and (start, end, name, args) appended; the key "*" takes every entry point not
-    listed by name. Used by the benchmark only. The native layer is told whether the table is empty."""
+    listed by name. Used by the benchmark only. Whatever changes the table tells the native layer whether it is empty."""
 
-    def __setitem__(self, name, rec):
-        super().__setitem__(name, rec)
-        native.set_timed(True)
 
-    def __delitem__(self, name):
-        super().__delitem__(name)
-        native.set_timed(bool(self))
+def _telling(name):
+    def method(self, *args, **kw):
+        try:
+            return getattr(dict, name)(self, *args, **kw)
+        finally:
+            native.timed_changed()
+    method.__name__ = name
+    return method
+
+
+for _name in ("__setitem__", "__delitem__", "__ior__", "update", "setdefault", "pop", "popitem", "clear"):
+    setattr(_Timed, _name, _telling(_name))
 
 
 TIMED = _Timed()
@@ -198,6 +204,12 @@ HOST_PATH = os.path.join(HERE, "_tfb_host.so")
 class _Native:
     """The extension module, loaded on first use (the package imports without a built library)."""
 
+    def timed_changed(self):
+        """Tells the extension, once it is loaded, whether any entry point is timed."""
+        tell = self.__dict__.get("set_timed")
+        if tell is not None:
+            tell(bool(TIMED))
+
     def __getattr__(self, name):
         lib()      # first: the extension binds to the library loaded from LIB_PATH
         if not os.path.exists(HOST_PATH):
@@ -210,6 +222,7 @@ class _Native:
         mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_tfb_host", loader))
         loader.exec_module(mod)
         self.__dict__.update((k, v) for k, v in vars(mod).items() if not k.startswith("__"))
+        self.timed_changed()
         try:
             return self.__dict__[name]
         except KeyError:
