@@ -1,4 +1,4 @@
-"""The entry points whose outputs have more rows than their inputs, called through the C-ABI: what they write equals the
+"""Entry points called through the C-ABI, above all those whose outputs have more rows than their inputs: what they write equals the
 plain forms on the given rows bit for bit and is zero beyond, whatever the output buffers held."""
 import pytest
 import torch
@@ -95,3 +95,19 @@ def test_expert_gradient_bytes_without_the_bf16_rows(dev, N, topk):
               _p(out), tab["rmax"], d, topk, _stream())
     used = int(tab["seg"][-1])
     assert torch.equal(out[:used], ops.moe_quant(dys, rows_b, 5, ops.FMT_E5M2, tab)[:used])
+
+
+@pytest.mark.parametrize("n,V", [(1, 8), (1000, 512), (5000, 32768), (300, 50304)])
+def test_embedding_backward_stays_within_the_scratch_it_asks_for(dev, n, V):
+    """tfb_embedding_bwd_grouped with exactly tfb_embedding_bwd_scratch_ints ints, a guard behind them, against the op."""
+    from trainium_frontier_them_bones_amd import _lib, ops
+    g = torch.Generator().manual_seed(n)
+    idx = torch.randint(0, V, (n,), generator=g).to(dev)
+    dy = torch.randn(n, 64, generator=g).to(bf16).to(dev)
+    ints = int(_lib.lib().tfb_embedding_bwd_scratch_ints(n, V))
+    scr = torch.full((ints + 64,), 0x5a5a5a5a, dtype=torch.int32, device=dev)
+    dw, want = torch.zeros(V, 64, device=dev), torch.zeros(V, 64, device=dev)
+    _lib.call("tfb_embedding_bwd_grouped", _p(idx), 1, _p(dy), _p(dw), n, 64, V, _p(scr), _stream())
+    ops.embedding_bwd(idx, dy, want)
+    assert torch.equal(scr[ints:], torch.full_like(scr[ints:], 0x5a5a5a5a))
+    assert torch.equal(want, dw) or (want - dw).norm() < 1e-6 * want.norm()

@@ -68,6 +68,8 @@ struct Args {
     return {0.0, d};
   }
   at::ScalarType dtype(int i) const { return has(i) && b(i) ? F32 : BF16; }   // "fp32 output?"
+  bool bthd(int i) const { return !is(i, "bhtd"); }   // a layout's name
+  MoeTab tab(int i) const;                            // the dict that tfb_moe_tables returns
   bool is(int i, const char* s) const { return has(i) && PyUnicode_Check(a[i]) && PyUnicode_CompareWithASCIIString(a[i], s) == 0; }
 };
 
@@ -92,6 +94,36 @@ PyObject* outs(const Tensors& v) {
   return r;
 }
 PyObject* none() { Py_RETURN_NONE; }
+
+// A dict's entry as a tensor (undefined: none of that name).
+Tensor dict_tensor(PyObject* d, const char* key) {
+  PyObject* v = PyDict_GetItemString(d, key);
+  return v && THPVariable_Check(v) ? THPVariable_Unpack(v) : Tensor();
+}
+MoeTab Args::tab(int i) const {
+  PyObject* d = need(i);
+  TORCH_CHECK_TYPE(PyDict_Check(d), "argument ", i + 1, " must be the dict of the slot tables");
+  MoeTab t{dict_tensor(d, "cnt"), dict_tensor(d, "seg"), dict_tensor(d, "tile_expert"), dict_tensor(d, "slot"), dict_tensor(d, "tok"),
+           dict_tensor(d, "ksel"), dict_tensor(d, "cnt_all")};
+  for (const Tensor* x : {&t.cnt, &t.seg, &t.tile_expert, &t.slot, &t.tok, &t.ksel}) {
+    TORCH_CHECK_TYPE(x->defined(), "the slot tables are incomplete");
+    chk(*x, I32);
+  }
+  t.rmax = t.tok.numel();
+  t.capped = PyDict_GetItemString(d, "capacity") != nullptr;
+  return t;
+}
+PyObject* out(const MoeTab& t, int64_t capacity) {
+  PyObject* d = PyDict_New();
+  auto put = [&](const char* key, PyObject* v) {
+    PyDict_SetItemString(d, key, v);
+    Py_DECREF(v);
+  };
+  put("cnt", out(t.cnt)), put("seg", out(t.seg)), put("tile_expert", out(t.tile_expert)), put("slot", out(t.slot));
+  put("tok", out(t.tok)), put("ksel", out(t.ksel)), put("rmax", PyLong_FromLongLong(t.rmax));
+  if (t.capped) put("cnt_all", out(t.cnt_all)), put("capacity", PyLong_FromLongLong(capacity));
+  return d;
+}
 
 template <PyObject* (*F)(const Args&), int LO, int HI>   // a function of LO to HI arguments
 PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -249,6 +281,105 @@ PyObject* op_lmhead_fwd(const Args& a) {
   return outs(lmhead_fwd(a.t(0), a.t(1), targets_of(a.t(2)), a.cap(3), a.opt(4)));
 }
 
+// attention and rotary embedding
+PyObject* op_attn_fwd(const Args& a) {   // q, k, v, scale, layout, band
+  return outs(attention(a.t(0), a.t(1), a.t(2), a.f(3), a.bthd(4), a.i_or(5, 0)));
+}
+PyObject* op_attn_bwd(const Args& a) {   // q, k, v, o, do, lse, scale, layout, dq, dk, dv, their layout, cos, sin, band
+  attention_bwd(a.t(0), a.t(1), a.t(2), a.t(3), a.t(4), a.t(5), a.f(6), a.bthd(7), a.t(8), a.t(9), a.t(10), a.bthd(11), a.opt(12), a.opt(13),
+                a.i_or(14, 0));
+  return none();
+}
+PyObject* op_attn_bwd_static(const Args& a) {   // as far as the layout of dq, dk, dv
+  attention_bwd_static(a.t(0), a.t(1), a.t(2), a.t(3), a.t(4), a.t(5), a.f(6), a.bthd(7), a.t(8), a.t(9), a.t(10), a.bthd(11));
+  return none();
+}
+PyObject* op_rope(const Args& a) {   // x, cos, sin, T, heads, D, inverse, out
+  const Tensor x = a.t(0), o = a.has(7) ? a.t(7) : x;
+  const RowView rx = row_view(x), ro = row_view(o);
+  rope(x, a.t(1), a.t(2), o, rx.rows, a.i(3), a.i(4), a.i(5), rx.stride, ro.stride, a.b(6));
+  return none();
+}
+PyObject* op_rope_norm_fwd(const Args& a) {   // x, cos, sin, T, heads, D, eps, want_r
+  const Tensor x = a.t(0);
+  const RowView v = row_view(x);
+  const int64_t H = a.i(4), D = a.i(5);
+  Tensor y = make({v.rows, H * D}, BF16, x), r = a.b(7) ? make_like(y) : Tensor(), inv = make({v.rows, H}, F32, x);
+  rope_norm_fwd(x, a.t(1), a.t(2), r, y, inv, v.rows, a.i(3), H, D, v.stride, a.f(6));
+  return outs(y, r, inv);
+}
+PyObject* op_rope_norm_bwd(const Args& a) {   // g, r, inv, cos, sin, T, heads, D, out
+  const Tensor g = a.t(0);
+  const RowView v = row_view(g);
+  const int64_t H = a.i(6), D = a.i(7);
+  const Tensor o = a.has(8) ? a.t(8) : make({v.rows, H * D}, BF16, g);
+  rope_norm_bwd(g, a.t(1), a.t(2), a.t(3), a.t(4), o, v.rows, a.i(5), H, D, v.stride, row_view(o).stride);
+  return out(o);
+}
+PyObject* op_embedding_bwd(const Args& a) {   // idx, dy, dw
+  embedding_bwd(a.t(0), a.t(1), a.t(2));
+  return none();
+}
+
+// mixture of experts
+PyObject* op_moe_route(const Args& a) {   // h, wr, topk, bias, want_logits
+  MoeRoute o = moe_route(a.t(0), a.t(1), a.i(2), a.opt(3), a.b(4));
+  return outs(o.p, o.idx, o.gate, o.logits);
+}
+PyObject* op_moe_tables(const Args& a) {   // idx, E, seq_len, capacity
+  const int64_t cap = a.i_or(3, -1);
+  return out(moe_tables(a.t(0), a.i(1), a.i_or(2, -1), cap), cap);
+}
+PyObject* op_moe_gather(const Args& a) {   // h, tab, x_scale, want_xs
+  const Scale s = a.has(2) ? a.scale(2) : Scale{};
+  return outs(moe_gather(a.t(0), a.tab(1), a.has(2) ? &s : nullptr, a.b(3)));
+}
+PyObject* op_moe_mlp8_fwd(const Args& a) { return outs(moe_mlp8_fwd(a.t(0), a.t(1), a.t(2), a.tab(3), a.i(4))); }
+PyObject* op_moe_mlp_fwd(const Args& a) { return outs(moe_mlp_fwd(a.t(0), a.t(1), a.t(2), a.tab(3))); }
+PyObject* op_moe_mlp_bwd(const Args& a) {   // dys, r, w_fc, w_proj, tab
+  MlpBwd o = moe_mlp_bwd(a.t(0), a.t(1), a.t(2), a.t(3), a.tab(4));
+  return outs(o.dx, o.dpre);
+}
+PyObject* op_moe_backward_scales_rowmax(const Args& a) { return out(moe_backward_scales_rowmax(a.t(0), a.t(1), a.tab(2), a.i(3))); }
+PyObject* op_moe_quant(const Args& a) { return out(moe_quant(a.t(0), a.t(1), a.i(2), a.i(3), a.tab(4))); }
+PyObject* op_moe_quant_dout(const Args& a) { return out(moe_quant_dout(a.t(0), a.t(1), a.t(2), a.tab(3))); }
+PyObject* op_moe_mlp8_bwd(const Args& a) {   // dys, r, w8, rows, tab
+  MlpBwd o = moe_mlp8_bwd(a.t(0), a.t(1), a.t(2), a.t(3), a.tab(4));
+  return outs(o.dx, o.dpre);
+}
+PyObject* op_moe_mlp8_bwd_q(const Args& a) {   // dy8, r, w8, rows, tab, limit
+  MlpBwd o = moe_mlp8_bwd_q(a.t(0), a.t(1), a.t(2), a.t(3), a.tab(4), a.f(5));
+  return outs(o.dx, o.dp8, o.hq8);
+}
+PyObject* op_moe_dw8(const Args& a) {   // xs8, dp8, hq8, dy8, rows, x_scale, tab, E, dw_fc, dw_proj, accumulate, fp32
+  Tensor f = a.opt(8), p = a.opt(9);
+  moe_dw8(a.t(0), a.t(1), a.t(2), a.t(3), a.t(4), a.scale(5).host(), a.tab(6), f, p, a.i(7), a.b(10), a.dtype(11));
+  return outs(f, p);
+}
+PyObject* op_moe_dw(const Args& a) {   // dpre, xs, dys, r, tab, E, dw_fc, dw_proj, accumulate, fp32
+  Tensor f = a.opt(6), p = a.opt(7);
+  moe_dw(a.t(0), a.t(1), a.t(2), a.t(3), a.tab(4), f, p, a.i(5), a.b(8), a.dtype(9));
+  return outs(f, p);
+}
+PyObject* op_moe_combine(const Args& a) {   // ys, tab, gate
+  const Tensor ys = a.t(0), gate = a.t(2);
+  return out(moe_combine(ys, a.tab(1), gate, {gate.size(0), ys.size(1)}));
+}
+PyObject* op_moe_combine_bwd(const Args& a) {   // dout, ys, tab, gate, want_rowmax
+  CombineGrad o = moe_combine_bwd(a.t(0), a.t(1), a.tab(2), a.t(3), a.b(4));
+  return a.b(4) ? outs(o.dys, o.dgate, o.rowmax) : outs(o.dys, o.dgate);
+}
+PyObject* op_moe_aux_fwd(const Args& a) { return outs(moe_aux_fwd(a.t(0), a.t(1), a.tab(2), a.i(3))); }
+PyObject* op_moe_aux_seq_fwd(const Args& a) { return outs(moe_aux_seq_fwd(a.t(0), a.t(1), a.i(2), a.i(3))); }
+PyObject* op_moe_route_bwd(const Args& a) {
+  // dgate, p, idx, dxs, tab, h, wr, dwr, accumulate[, terms, lse, gaux, alpha, beta[, fs, gamma, seq_len]]
+  MoeAux x;
+  if (a.n > 9) x.terms = a.t(9), x.lse = a.t(10), x.gaux = a.t(11), x.alpha = a.f(12), x.beta = a.f(13);
+  if (a.n > 14) x.fs = a.t(14), x.gamma = a.f(15), x.seq_len = a.i(16);
+  RouteGrad o = moe_route_bwd(a.t(0), a.t(1), a.t(2), a.t(3), a.tab(4), a.t(5), a.t(6), a.opt(7), a.b(8), a.n > 9 ? &x : nullptr);
+  return outs(o.dh, o.dwr, o.dlogits);
+}
+
 PyObject* set_timed(const Args& a) {
   timed = a.b(0);
   return none();
@@ -280,6 +411,21 @@ PyMethodDef methods[] = {
     FN("tfb_fill_f32", op_fill, 2, 2), FN("tfb_adamw", op_adamw, 11, 11), FN("tfb_loss_row_weights", op_row_weights, 3, 3),
     FN("tfb_loss_fwd", op_loss_fwd, 4, 4), FN("tfb_loss_fwd_bwd", op_loss_fwd_bwd, 4, 4), FN("tfb_loss_bwd", op_loss_bwd, 6, 6),
     FN("tfb_lmhead_fwd", op_lmhead_fwd, 5, 5),
+    FN("tfb_attn_fwd", op_attn_fwd, 5, 5), FN("tfb_attn_fwd_band", op_attn_fwd, 6, 6), FN("tfb_attn_bwd", op_attn_bwd, 12, 12),
+    FN("tfb_attn_bwd_rope", op_attn_bwd, 14, 14), FN("tfb_attn_bwd_band", op_attn_bwd, 15, 15),
+    FN("tfb_attn_bwd_static", op_attn_bwd_static, 12, 12),
+    FN("tfb_rope", op_rope, 8, 8), FN("tfb_rope_norm_fwd", op_rope_norm_fwd, 8, 8), FN("tfb_rope_norm_bwd", op_rope_norm_bwd, 9, 9),
+    FN("tfb_embedding_bwd_grouped", op_embedding_bwd, 3, 3), FN("tfb_moe_route", op_moe_route, 5, 5),
+    FN("tfb_moe_tables", op_moe_tables, 2, 2), FN("tfb_moe_tables_cap", op_moe_tables, 4, 4), FN("tfb_moe_gather", op_moe_gather, 4, 4), FN("tfb_moe_mlp8_fwd", op_moe_mlp8_fwd, 5, 5),
+    FN("tfb_moe_mlp_fwd", op_moe_mlp_fwd, 4, 4), FN("tfb_moe_mlp_bwd", op_moe_mlp_bwd, 5, 5),
+    FN("tfb_moe_backward_scales_rowmax", op_moe_backward_scales_rowmax, 4, 4), FN("tfb_moe_quant", op_moe_quant, 5, 5),
+    FN("tfb_moe_quant_dout", op_moe_quant_dout, 4, 4), FN("tfb_moe_mlp8_bwd", op_moe_mlp8_bwd, 5, 5),
+    FN("tfb_moe_mlp8_bwd_q", op_moe_mlp8_bwd_q, 6, 6), FN("tfb_moe_dw8", op_moe_dw8, 12, 12), FN("tfb_moe_dw", op_moe_dw, 10, 10),
+    FN("tfb_moe_combine", op_moe_combine, 3, 3), FN("tfb_moe_combine_bwd", op_moe_combine_bwd, 4, 4),
+    FN("tfb_moe_combine_bwd_rowmax", op_moe_combine_bwd, 5, 5),
+    FN("tfb_moe_aux_fwd", op_moe_aux_fwd, 4, 4), FN("tfb_moe_aux_seq_fwd", op_moe_aux_seq_fwd, 4, 4),
+    FN("tfb_moe_route_bwd", op_moe_route_bwd, 9, 9), FN("tfb_moe_route_bwd_aux", op_moe_route_bwd, 14, 14),
+    FN("tfb_moe_route_bwd_aux_seq", op_moe_route_bwd, 17, 17),
     {nullptr, nullptr, 0, nullptr}};
 #undef FN
 

@@ -443,12 +443,6 @@ struct Linear8 : Function<Linear8> {
 };
 
 // -------------------------------------------------------------------------------------------------------- attention
-void check_qkv(const Tensor& q, const Tensor& k, const Tensor& v) {
-  for (const Tensor* t : {&q, &k, &v}) {
-    TORCH_CHECK_TYPE(t->is_cuda() && t->scalar_type() == BF16, "attention takes bf16 device tensors");
-    TORCH_CHECK_VALUE(t->dim() == 4 && t->sizes() == q.sizes(), "q, k, v shapes differ");
-  }
-}
 void check_grad(const Tensor& go, int64_t n) {
   TORCH_CHECK_TYPE(go.is_cuda() && go.scalar_type() == BF16, "attention takes bf16 device tensors");
   TORCH_CHECK_VALUE(go.numel() == n, "o and do are [B, T, H, D]");
@@ -461,10 +455,7 @@ struct Attention : Function<Attention> {
   };
   static Tensor forward(AutogradContext* ctx, const Tensor& q_, const Tensor& k_, const Tensor& v_, double scale, int64_t band) {
     const Tensor q = dense(q_), k = dense(k_), v = dense(v_);
-    check_qkv(q, k, v);
-    const int64_t B = q.size(0), H = q.size(1), T = q.size(2), D = q.size(3);
-    Tensor o = make({B, T, H, D}, BF16, q), lse = make({B, H, T}, F32, q);
-    attn_fwd(bhtd(q), bhtd(k), bhtd(v), o, lse, B, H, T, D, scale, band);
+    auto [o, lse] = attention(q, k, v, scale, false, band);
     ctx->save_for_backward({q, k, v, o, lse});
     keep<S>(ctx) = {scale, band};
     return o;
@@ -476,8 +467,7 @@ struct Attention : Function<Attention> {
     check_grad(go, o.numel());
     // gradients in the inputs' own (contiguous [B, H, T, D]) layout: autograd keeps them as they are
     Tensor dq = make_like(q), dk = make_like(k), dv = make_like(v);
-    attn_bwd(bhtd(q), bhtd(k), bhtd(v), o, go, bhtd(dq), bhtd(dk), bhtd(dv), s[4], {}, {}, q.size(0), q.size(1), q.size(2), q.size(3),
-             st.scale, st.band);
+    attention_bwd(q, k, v, o, go.view(o.sizes()), s[4], st.scale, false, dq, dk, dv, false, {}, {}, st.band);
     return {dq, dk, dv, Tensor(), Tensor()};
   }
 };
@@ -486,6 +476,8 @@ struct QkvDims {
   int64_t B, T, C, H, D;
   double scale;
   int64_t band = 0;
+  View third(const Tensor& t, int i, int64_t row) const { return tfb::third(t, i, T, C, D, row); }
+  View whole(const Tensor& t) const { return tfb::whole(t, T, H, D); }
 };
 QkvDims qkv_dims(const Tensor& qkv, int64_t n_head, double scale, int64_t band = 0) {
   TORCH_CHECK_TYPE(qkv.is_cuda() && qkv.scalar_type() == BF16, "attention takes bf16 device tensors");
@@ -502,8 +494,7 @@ struct RopeAttention : Function<RopeAttention> {
     const Tensor rot = make({m.B, m.T, 2 * m.C}, BF16, qkv);
     rope(qkv, cos, sin, rot, rows, m.T, 2 * m.H, m.D, 3 * m.C, 2 * m.C, false);
     Tensor o = make({m.B, m.T, m.C}, BF16, qkv), lse = make({m.B, m.H, m.T}, F32, qkv);
-    attn_fwd(third(rot, 0, m.T, m.C, m.D, 2 * m.C), third(rot, 1, m.T, m.C, m.D, 2 * m.C), third(qkv, 2, m.T, m.C, m.D, 3 * m.C), o, lse, m.B,
-             m.H, m.T, m.D, scale, 0);
+    attn_fwd(m.third(rot, 0, 2 * m.C), m.third(rot, 1, 2 * m.C), m.third(qkv, 2, 3 * m.C), o, lse, m.B, m.H, m.T, m.D, scale, 0);
     ctx->save_for_backward({qkv, rot, o, lse, cos, sin});
     keep<QkvDims>(ctx) = m;
     return o;
@@ -516,9 +507,8 @@ struct RopeAttention : Function<RopeAttention> {
     const int64_t R = 3 * m.C;
     Tensor dqkv = make_like(qkv);
     const bool fused = m.D == 64;   // the inverse rotation of dq, dk rides the backward kernels' stores
-    attn_bwd(third(rot, 0, m.T, m.C, m.D, 2 * m.C), third(rot, 1, m.T, m.C, m.D, 2 * m.C), third(qkv, 2, m.T, m.C, m.D, R), s[2], go,
-             third(dqkv, 0, m.T, m.C, m.D, R), third(dqkv, 1, m.T, m.C, m.D, R), third(dqkv, 2, m.T, m.C, m.D, R), s[3], fused ? cos : Tensor(),
-             fused ? sin : Tensor(), m.B, m.H, m.T, m.D, m.scale, 0);
+    attn_bwd(m.third(rot, 0, 2 * m.C), m.third(rot, 1, 2 * m.C), m.third(qkv, 2, R), m.whole(s[2]), m.whole(go), m.third(dqkv, 0, R),
+             m.third(dqkv, 1, R), m.third(dqkv, 2, R), s[3], fused ? cos : Tensor(), fused ? sin : Tensor(), m.B, m.H, m.T, m.D, m.scale, 0);
     if (!fused) rope(dqkv, cos, sin, dqkv, m.B * m.T, m.T, 2 * m.H, m.D, R, R, true);
     return {dqkv, Tensor(), Tensor(), Tensor(), Tensor()};
   }
@@ -554,8 +544,7 @@ struct RopeNormAttention : Function<RopeNormAttention> {
     const Tensor qk = make({rows, R}, BF16, qkv), r = make({rows, R}, BF16, qkv), inv = make({rows, 2 * m.H}, F32, qkv);
     rope_norm_fwd(qkv, cos, sin, r, qk, inv, rows, m.T, 2 * m.H, m.D, 3 * m.C, eps);
     Tensor o = heads ? make({m.B, m.T, m.H, m.D}, BF16, qkv) : make({m.B, m.T, m.C}, BF16, qkv), lse = make({m.B, m.H, m.T}, F32, qkv);
-    attn_fwd(third(qk, 0, m.T, m.C, m.D, R), third(qk, 1, m.T, m.C, m.D, R), third(qkv, 2, m.T, m.C, m.D, 3 * m.C), o, lse, m.B, m.H, m.T, m.D,
-             scale, band);
+    attn_fwd(m.third(qk, 0, R), m.third(qk, 1, R), m.third(qkv, 2, 3 * m.C), o, lse, m.B, m.H, m.T, m.D, scale, band);
     ctx->save_for_backward({qkv, qk, r, inv, o, lse, cos, sin});
     keep<QkvDims>(ctx) = m;
     return o;
@@ -567,9 +556,8 @@ struct RopeNormAttention : Function<RopeNormAttention> {
     check_grad(go, s[4].numel());
     const int64_t R = 2 * m.C, F = 3 * m.C;
     Tensor dqkv = make_like(qkv);
-    attn_bwd(third(qk, 0, m.T, m.C, m.D, R), third(qk, 1, m.T, m.C, m.D, R), third(qkv, 2, m.T, m.C, m.D, F), s[4], go,
-             third(dqkv, 0, m.T, m.C, m.D, F), third(dqkv, 1, m.T, m.C, m.D, F), third(dqkv, 2, m.T, m.C, m.D, F), s[5], {}, {}, m.B, m.H, m.T,
-             m.D, m.scale, m.band);
+    attn_bwd(m.third(qk, 0, R), m.third(qk, 1, R), m.third(qkv, 2, F), m.whole(s[4]), m.whole(go), m.third(dqkv, 0, F), m.third(dqkv, 1, F),
+             m.third(dqkv, 2, F), s[5], {}, {}, m.B, m.H, m.T, m.D, m.scale, m.band);
     rope_norm_bwd(dqkv, s[2], s[3], s[6], s[7], dqkv, m.B * m.T, m.T, 2 * m.H, m.D, F, F);   // in place on the q and k thirds
     return {dqkv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
@@ -586,7 +574,7 @@ struct QkvRopeAttention : Function<QkvRopeAttention> {
     const QkvDims m = qkv_dims(qkv, n_head, scale);
     Tensor o = make({B, T, C}, BF16, x), lse = make({B, m.H, T}, F32, x);
     const int64_t R = 3 * C;
-    attn_fwd(third(qkv, 0, T, C, m.D, R), third(qkv, 1, T, C, m.D, R), third(qkv, 2, T, C, m.D, R), o, lse, B, m.H, T, m.D, scale, 0);
+    attn_fwd(m.third(qkv, 0, R), m.third(qkv, 1, R), m.third(qkv, 2, R), o, lse, B, m.H, T, m.D, scale, 0);
     ctx->save_for_backward({x, w, qkv, o, lse, cos, sin});
     keep<QkvDims>(ctx) = m;
     return o;
@@ -598,9 +586,8 @@ struct QkvRopeAttention : Function<QkvRopeAttention> {
     check_grad(go, s[3].numel());
     const int64_t R = 3 * m.C, K = w.size(1), M = m.B * m.T;
     const Tensor dqkv = make_like(qkv);
-    attn_bwd(third(qkv, 0, m.T, m.C, m.D, R), third(qkv, 1, m.T, m.C, m.D, R), third(qkv, 2, m.T, m.C, m.D, R), s[3], go,
-             third(dqkv, 0, m.T, m.C, m.D, R), third(dqkv, 1, m.T, m.C, m.D, R), third(dqkv, 2, m.T, m.C, m.D, R), s[4], s[5], s[6], m.B, m.H,
-             m.T, m.D, m.scale, 0);
+    attn_bwd(m.third(qkv, 0, R), m.third(qkv, 1, R), m.third(qkv, 2, R), m.whole(s[3]), m.whole(go), m.third(dqkv, 0, R), m.third(dqkv, 1, R),
+             m.third(dqkv, 2, R), s[4], s[5], s[6], m.B, m.H, m.T, m.D, m.scale, 0);
     Tensor dx = make_like(x);
     gemm(dqkv, w, dx, M, K, R, false, false, false);
     return {dx, weight_grad(w, dqkv, x, M, R, K), Tensor(), Tensor(), Tensor(), Tensor()};
@@ -773,7 +760,7 @@ struct Moe : Function<Moe> {
       if (!a.dw_fp8) xs8 = Tensor();   // only the fp8 weight gradient reads the bytes again
     } else {
       std::tie(xs, xs8) = moe_gather(h, s.tab, nullptr, true);
-      std::tie(ys, r) = moe_mlp_fwd(xs, bf(w_fc), bf(w_proj), s.tab);
+      std::tie(ys, r, std::ignore) = moe_mlp_fwd(xs, bf(w_fc), bf(w_proj), s.tab);
     }
     Tensor out = moe_combine(ys, s.tab, rt.gate, h.sizes());
     if (info) {

@@ -385,21 +385,87 @@ void attn_fwd(const View& q, const View& k, const View& v, const Tensor& o, cons
     TFB_CALL(tfb_attn_fwd, q.p, q.s, k.p, k.s, v.p, v.s, ptr(o), os, ptr(lse), B, H, T, D, scale, stream());
 }
 
-void attn_bwd(const View& q, const View& k, const View& v, const Tensor& o, const Tensor& go, const View& dq, const View& dk,
+void attn_bwd(const View& q, const View& k, const View& v, const View& o, const View& go, const View& dq, const View& dk,
               const View& dv, const Tensor& lse, const Tensor& cos, const Tensor& sin, int64_t B, int64_t H, int64_t T, int64_t D,
               double scale, int64_t band) {
   chk(cos), chk(sin);
-  const long os[3] = {T * H * D, D, H * D};
-  const Tensor delta = scratch(o, 2 * B * H * T);
+  const Tensor delta = scratch(lse, 2 * B * H * T);
   if (band)
-    TFB_CALL(tfb_attn_bwd_band, q.p, q.s, k.p, k.s, v.p, v.s, ptr(o), os, ptr(go), os, dq.p, dq.s, dk.p, dk.s, dv.p, dv.s, ptr(lse),
+    TFB_CALL(tfb_attn_bwd_band, q.p, q.s, k.p, k.s, v.p, v.s, o.p, o.s, go.p, go.s, dq.p, dq.s, dk.p, dk.s, dv.p, dv.s, ptr(lse),
              ptr(delta), ptr(cos), ptr(sin), B, H, T, D, scale, band, stream());
   else if (cos.defined())
-    TFB_CALL(tfb_attn_bwd_rope, q.p, q.s, k.p, k.s, v.p, v.s, ptr(o), os, ptr(go), os, dq.p, dq.s, dk.p, dk.s, dv.p, dv.s, ptr(lse),
+    TFB_CALL(tfb_attn_bwd_rope, q.p, q.s, k.p, k.s, v.p, v.s, o.p, o.s, go.p, go.s, dq.p, dq.s, dk.p, dk.s, dv.p, dv.s, ptr(lse),
              ptr(delta), ptr(cos), ptr(sin), B, H, T, D, scale, stream());
   else
-    TFB_CALL(tfb_attn_bwd, q.p, q.s, k.p, k.s, v.p, v.s, ptr(o), os, ptr(go), os, dq.p, dq.s, dk.p, dk.s, dv.p, dv.s, ptr(lse), ptr(delta),
+    TFB_CALL(tfb_attn_bwd, q.p, q.s, k.p, k.s, v.p, v.s, o.p, o.s, go.p, go.s, dq.p, dq.s, dk.p, dk.s, dv.p, dv.s, ptr(lse), ptr(delta),
              B, H, T, D, scale, stream());
+}
+
+namespace {
+
+struct AttnDims {
+  int64_t B, H, T, D;
+  at::DimVector shape(bool bthd) const { return bthd ? at::DimVector{B, T, H, D} : at::DimVector{B, H, T, D}; }
+};
+void check_attn(const Tensor& t) {
+  TORCH_CHECK_TYPE(t.is_cuda() && t.scalar_type() == BF16, "attention takes bf16 device tensors");
+  TORCH_CHECK_VALUE(t.dim() == 4, "attention tensors are 4-D");
+}
+AttnDims attn_dims(const Tensor& q, bool bthd) {
+  check_attn(q);
+  return {q.size(0), q.size(bthd ? 2 : 1), q.size(bthd ? 1 : 2), q.size(3)};
+}
+// The entry points see only pointers and strides: a tensor of the wrong shape, or a log-sum-exp that is not fp32 [B, H, T] dense,
+// would be an out-of-bounds access on the device.
+AttnDims check_attn_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& go, const Tensor& lse,
+                        const Tensor& dq, const Tensor& dk, const Tensor& dv, bool bthd, bool out_bthd) {
+  for (const Tensor* t : {&q, &k, &v, &o, &go, &dq, &dk, &dv}) check_attn(*t);
+  const AttnDims m = attn_dims(q, bthd);
+  TORCH_CHECK_VALUE(m.T % 128 == 0 && (m.D == 64 || m.D == 128), "attention takes T % 128 == 0 and D 64 or 128");
+  TORCH_CHECK_VALUE(k.sizes() == q.sizes() && v.sizes() == q.sizes(), "q, k, v shapes differ");
+  for (const Tensor* t : {&o, &go}) TORCH_CHECK_VALUE(t->sizes() == m.shape(true), "o and do are [B, T, H, D]");
+  for (const Tensor* t : {&dq, &dk, &dv}) TORCH_CHECK_VALUE(t->sizes() == m.shape(out_bthd), "dq, dk, dv shapes do not match out_layout");
+  TORCH_CHECK_VALUE(lse.is_cuda() && lse.scalar_type() == F32 && lse.is_contiguous() && lse.numel() == m.B * m.H * m.T,
+                    "lse is fp32 [B, H, T] contiguous");
+  return m;
+}
+
+}  // namespace
+
+std::tuple<Tensor, Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool bthd, int64_t band) {
+  const AttnDims m = attn_dims(q, bthd);
+  for (const Tensor* t : {&k, &v}) {
+    check_attn(*t);
+    TORCH_CHECK_VALUE(t->sizes() == q.sizes(), "q, k, v shapes differ");
+  }
+  Tensor o = make(m.shape(true), BF16, q), lse = make({m.B, m.H, m.T}, F32, q);
+  attn_fwd(layout(q, bthd), layout(k, bthd), layout(v, bthd), o, lse, m.B, m.H, m.T, m.D, scale, band);
+  return {o, lse};
+}
+
+void attention_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& go, const Tensor& lse, double scale,
+                   bool bthd_, const Tensor& dq, const Tensor& dk, const Tensor& dv, bool out_bthd, const Tensor& cos, const Tensor& sin,
+                   int64_t band) {
+  const AttnDims m = check_attn_bwd(q, k, v, o, go, lse, dq, dk, dv, bthd_, out_bthd);
+  attn_bwd(layout(q, bthd_), layout(k, bthd_), layout(v, bthd_), bthd(o), bthd(go), layout(dq, out_bthd), layout(dk, out_bthd),
+           layout(dv, out_bthd), lse, cos, sin, m.B, m.H, m.T, m.D, scale, band);
+}
+
+void attention_bwd_static(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o_, const Tensor& go_, const Tensor& lse,
+                          double scale, bool bthd_, const Tensor& dq_, const Tensor& dk_, const Tensor& dv_, bool out_bthd) {
+  const AttnDims m = check_attn_bwd(q_, k_, v_, o_, go_, lse, dq_, dk_, dv_, bthd_, out_bthd);
+  const View q = layout(q_, bthd_), k = layout(k_, bthd_), v = layout(v_, bthd_), o = bthd(o_), go = bthd(go_), dq = layout(dq_, out_bthd),
+             dk = layout(dk_, out_bthd), dv = layout(dv_, out_bthd);
+  TFB_CALL(tfb_attn_bwd_static, q.p, q.s, k.p, k.s, v.p, v.s, o.p, o.s, go.p, go.s, dq.p, dq.s, dk.p, dk.s, dv.p, dv.s, ptr(lse), m.B, m.H,
+           m.T, m.D, scale, stream());
+}
+
+RowView row_view(const Tensor& t) {
+  TORCH_CHECK_TYPE(t.is_cuda() && t.scalar_type() == BF16 && t.dim() > 0 && t.stride(-1) == 1,
+                   "expected a bf16 device tensor with contiguous rows");
+  if (t.is_contiguous()) return {t.numel() / last_dim(t), t.size(-1)};
+  TORCH_CHECK_VALUE(t.dim() == 2, "a strided operand is a matrix");
+  return {t.size(0), t.stride(0)};
 }
 
 void rope(const Tensor& x, const Tensor& cos, const Tensor& sin, const Tensor& out, int64_t rows, int64_t T, int64_t nheads, int64_t D,
@@ -560,14 +626,14 @@ std::tuple<Tensor, Tensor> moe_mlp8_fwd(const Tensor& xs8, const Tensor& w8, con
   return {ys, r};
 }
 
-std::tuple<Tensor, Tensor> moe_mlp_fwd(const Tensor& xs, const Tensor& w_fc, const Tensor& w_proj, const MoeTab& tab) {
+std::tuple<Tensor, Tensor, Tensor> moe_mlp_fwd(const Tensor& xs, const Tensor& w_fc, const Tensor& w_proj, const MoeTab& tab) {
   chk(xs), chk(w_fc), chk(w_proj);
   const int64_t rmax = xs.size(0), d = xs.size(1), E = w_fc.size(0), F = w_fc.size(1);
   TORCH_CHECK_VALUE(w_fc.sizes() == at::IntArrayRef({E, F, d}) && w_proj.sizes() == at::IntArrayRef({E, d, F}),
                     "moe_mlp_fwd: w_fc [E,F,d] and w_proj [E,d,F] expected");
   Tensor ys = make({rmax, d}, BF16, xs), r = make({rmax, F}, BF16, xs), h = make({rmax, F}, BF16, xs);
   TFB_CALL(tfb_moe_mlp_fwd, ptr(xs), ptr(w_fc), ptr(w_proj), ptr(tab.tile_expert), ptr(ys), ptr(r), ptr(h), rmax, d, F, stream());
-  return {ys, r};
+  return {ys, r, h};
 }
 
 Tensor moe_combine(const Tensor& ys, const MoeTab& tab, const Tensor& gate, at::IntArrayRef out_shape) {
@@ -601,10 +667,10 @@ Tensor moe_backward_scales_rowmax(const Tensor& rowmax, const Tensor& rows, cons
   return out;
 }
 
-static Tensor moe_quant_dy(const Tensor& x, const Tensor& rows, const MoeTab& tab) {
+Tensor moe_quant(const Tensor& x, const Tensor& rows, int64_t col, int64_t fmt, const MoeTab& tab) {
   chk(x), chk(rows, F32);
   Tensor out = make(x.sizes(), U8, x);
-  TFB_CALL(tfb_moe_quant, ptr(x), ptr(tab.tile_expert), ptr(rows), 5, E5M2, ptr(out), x.size(0), x.size(1), stream());
+  TFB_CALL(tfb_moe_quant, ptr(x), ptr(tab.tile_expert), ptr(rows), col, fmt, ptr(out), x.size(0), x.size(1), stream());
   return out;
 }
 
@@ -621,7 +687,7 @@ MlpBwd moe_mlp8_bwd(const Tensor& dys, const Tensor& r, const Tensor& w8, const 
   chk(dys), chk(r), chk(w8, U8);
   const int64_t rmax = dys.size(0), d = dys.size(1), F = r.size(1);
   MlpBwd o;
-  o.dy8 = moe_quant_dy(dys, rows, tab);
+  o.dy8 = moe_quant(dys, rows, 5, E5M2, tab);
   o.dx = make({rmax, d}, BF16, dys), o.dpre = make({rmax, F}, BF16, dys), o.dp8 = make({rmax, F}, U8, dys);
   TFB_CALL(tfb_moe_mlp8_bwd, ptr(o.dy8), ptr(r), ptr(w8), ptr(rows), ptr(tab.tile_expert), ptr(o.dx), ptr(o.dpre), ptr(o.dp8), rmax, d, F,
            stream());
@@ -648,11 +714,19 @@ MlpBwd moe_mlp_bwd(const Tensor& dys, const Tensor& r, const Tensor& w_fc, const
   return o;
 }
 
+static void moe_dw_outputs(Tensor& dw_fc, Tensor& dw_proj, int64_t E, int64_t F, int64_t d, bool accumulate, at::ScalarType out_dtype,
+                           const Tensor& like) {
+  TORCH_CHECK_VALUE(dw_fc.defined() == dw_proj.defined(), "give both outputs or neither");
+  dw_fc = Out2::get(dw_fc, {E, F, d}, out_dtype, accumulate, like);
+  dw_proj = Out2::get(dw_proj, {E, d, F}, out_dtype, accumulate, like);
+  TORCH_CHECK_VALUE(dw_fc.scalar_type() == dw_proj.scalar_type(), "bad outputs");
+}
+
 void moe_dw8(const Tensor& xs8, const Tensor& dp8, const Tensor& hq8, const Tensor& dy8, const Tensor& rows, double x_scale,
              const MoeTab& tab, Tensor& dw_fc, Tensor& dw_proj, int64_t E, bool accumulate, at::ScalarType out_dtype) {
   chk(xs8, U8), chk(dp8, U8), chk(hq8, U8), chk(dy8, U8), chk(rows, F32);
   const int64_t d = xs8.size(1), F = dp8.size(1);
-  if (!dw_fc.defined()) dw_fc = make({E, F, d}, out_dtype, xs8), dw_proj = make({E, d, F}, out_dtype, xs8);
+  moe_dw_outputs(dw_fc, dw_proj, E, F, d, accumulate, out_dtype, xs8);
   TFB_CALL(tfb_moe_dw8, ptr(xs8), ptr(dp8), ptr(hq8), ptr(dy8), ptr(rows), x_scale, ptr(tab.seg), ptr(dw_fc), ptr(dw_proj), E, d, F,
            dw_fc.scalar_type() == F32, accumulate, stream());
 }
@@ -660,7 +734,8 @@ void moe_dw8(const Tensor& xs8, const Tensor& dp8, const Tensor& hq8, const Tens
 void moe_dw(const Tensor& dpre, const Tensor& xs, const Tensor& dys, const Tensor& r, const MoeTab& tab, Tensor& dw_fc, Tensor& dw_proj,
             int64_t E, bool accumulate, at::ScalarType out_dtype) {
   const int64_t d = xs.size(1), F = r.size(1);
-  if (!dw_fc.defined()) dw_fc = make({E, F, d}, out_dtype, xs), dw_proj = make({E, d, F}, out_dtype, xs);
+  chk(dpre), chk(xs), chk(dys), chk(r);
+  moe_dw_outputs(dw_fc, dw_proj, E, F, d, accumulate, out_dtype, xs);
   TFB_CALL(tfb_moe_dw, ptr(dpre), ptr(xs), ptr(dys), ptr(r), ptr(tab.seg), ptr(dw_fc), ptr(dw_proj), E, d, F, dw_fc.scalar_type() == F32,
            accumulate, stream());
 }

@@ -66,12 +66,26 @@ struct View {
 };
 View bhtd(const Tensor& t);                                      // a 4-D tensor [B, H, T, D]
 View bthd(const Tensor& t);                                      // a 4-D tensor [B, T, H, D]
+inline View layout(const Tensor& t, bool bthd_) { return bthd_ ? bthd(t) : bhtd(t); }
 View third(const Tensor& t, int i, int64_t T, int64_t C, int64_t D, int64_t row);   // columns i C .. of a [B T, row] tensor, heads of D
 void attn_fwd(const View& q, const View& k, const View& v, const Tensor& o, const Tensor& lse, int64_t B, int64_t H, int64_t T, int64_t D,
               double scale, int64_t band);
-void attn_bwd(const View& q, const View& k, const View& v, const Tensor& o, const Tensor& go, const View& dq, const View& dk,
+void attn_bwd(const View& q, const View& k, const View& v, const View& o, const View& go, const View& dq, const View& dk,
               const View& dv, const Tensor& lse, const Tensor& cos, const Tensor& sin, int64_t B, int64_t H, int64_t T, int64_t D,
               double scale, int64_t band);
+// on 4-D tensors [B, H, T, D] or [B, T, H, D], a flag for q, k, v and one for dq, dk, dv
+std::tuple<Tensor, Tensor> attention(const Tensor& q, const Tensor& k, const Tensor& v, double scale, bool bthd, int64_t band);
+void attention_bwd(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& go, const Tensor& lse, double scale,
+                   bool bthd, const Tensor& dq, const Tensor& dk, const Tensor& dv, bool out_bthd, const Tensor& cos, const Tensor& sin,
+                   int64_t band);
+void attention_bwd_static(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& go, const Tensor& lse,
+                          double scale, bool bthd, const Tensor& dq, const Tensor& dk, const Tensor& dv, bool out_bthd);
+inline View whole(const Tensor& t, int64_t T, int64_t H, int64_t D) { return {ptr(t), {T * H * D, D, H * D}}; }   // dense [B, T, H, D]
+// a 2-D view with contiguous rows, or a dense tensor as rows of its last dimension
+struct RowView {
+  int64_t rows, stride;
+};
+RowView row_view(const Tensor& t);
 void rope(const Tensor& x, const Tensor& cos, const Tensor& sin, const Tensor& out, int64_t rows, int64_t T, int64_t nheads, int64_t D,
           int64_t x_stride, int64_t out_stride, bool inverse);
 void rope_norm_fwd(const Tensor& x, const Tensor& cos, const Tensor& sin, const Tensor& r, const Tensor& y, const Tensor& inv,
@@ -107,11 +121,12 @@ MoeRoute moe_route(const Tensor& h, const Tensor& wr, int64_t topk, const Tensor
 MoeTab moe_tables(const Tensor& idx, int64_t E, int64_t seq_len, int64_t capacity);   // capacity < 0: dropless
 std::tuple<Tensor, Tensor> moe_gather(const Tensor& h, const MoeTab& tab, const Scale* x_scale, bool want_xs);
 std::tuple<Tensor, Tensor> moe_mlp8_fwd(const Tensor& xs8, const Tensor& w8, const Tensor& rows, const MoeTab& tab, int64_t F);
-std::tuple<Tensor, Tensor> moe_mlp_fwd(const Tensor& xs, const Tensor& w_fc, const Tensor& w_proj, const MoeTab& tab);
+std::tuple<Tensor, Tensor, Tensor> moe_mlp_fwd(const Tensor& xs, const Tensor& w_fc, const Tensor& w_proj, const MoeTab& tab);
 Tensor moe_combine(const Tensor& ys, const MoeTab& tab, const Tensor& gate, at::IntArrayRef out_shape);
 struct CombineGrad { Tensor dys, dgate, rowmax; };
 // want_dys false (with want_rowmax): dys is left out, moe_quant_dout makes its bytes
 CombineGrad moe_combine_bwd(const Tensor& dout, const Tensor& ys, const MoeTab& tab, const Tensor& gate, bool want_rowmax, bool want_dys = true);
+Tensor moe_quant(const Tensor& x, const Tensor& rows, int64_t col, int64_t fmt, const MoeTab& tab);
 Tensor moe_quant_dout(const Tensor& dout, const Tensor& gate, const Tensor& rows, const MoeTab& tab);
 Tensor moe_backward_scales_rowmax(const Tensor& rowmax, const Tensor& rows, const MoeTab& tab, int64_t d);
 MlpBwd moe_mlp8_bwd(const Tensor& dys, const Tensor& r, const Tensor& w8, const Tensor& rows, const MoeTab& tab);

@@ -252,93 +252,40 @@ _L3 = _ct.c_long * 3
 
 
 def _bht(t, layout):
-    """(batch, head, token) element strides of a 4-D tensor given as "bhtd" or "bthd" (head dim contiguous)."""
-    if t.stride(3) != 1:
-        raise RuntimeError("head dimension must be contiguous")
+    """(batch, head, token) element strides of a 4-D tensor given as "bhtd" or "bthd", for a call of the C-ABI itself."""
     if layout == "bhtd":
         return _L3(t.stride(0), t.stride(1), t.stride(2))
     return _L3(t.stride(0), t.stride(2), t.stride(1))
-
-
-def _attn_chk(t):
-    if not t.is_cuda or t.dtype != bf16:
-        raise TypeError("attention takes bf16 device tensors")
-
-
-def _attn_bwd_chk(q, k, v, o, do, lse, dq, dk, dv, layout, out_layout):
-    """Host checks of an attention backward call: a tensor of the wrong shape, or a log-sum-exp that is not fp32
-    [B, H, T] contiguous, would be an out-of-bounds access on the device (the entry point sees only pointers and strides)."""
-    for t in (q, k, v, o, do, dq, dk, dv):
-        _attn_chk(t)
-        if t.dim() != 4:
-            raise ValueError("attention tensors are 4-D")
-    B, H, T, D = q.shape if layout == "bhtd" else (q.shape[0], q.shape[2], q.shape[1], q.shape[3])
-    if T % 128 or D not in (64, 128):
-        raise ValueError("attention takes T % 128 == 0 and D 64 or 128")
-    inp = (B, H, T, D) if layout == "bhtd" else (B, T, H, D)
-    outp = (B, H, T, D) if out_layout == "bhtd" else (B, T, H, D)
-    if tuple(k.shape) != inp or tuple(v.shape) != inp or tuple(q.shape) != inp:
-        raise ValueError("q, k, v shapes differ")
-    if tuple(o.shape) != (B, T, H, D) or tuple(do.shape) != (B, T, H, D):
-        raise ValueError("o and do are [B, T, H, D]")
-    for t in (dq, dk, dv):
-        if tuple(t.shape) != outp:
-            raise ValueError("dq, dk, dv shapes do not match out_layout")
-    if not lse.is_cuda or lse.dtype != torch.float32 or not lse.is_contiguous() or lse.numel() != B * H * T:
-        raise ValueError("lse is fp32 [B, H, T] contiguous")
-    return B, H, T, D
 
 
 def attn_fwd(q, k, v, scale, layout="bhtd", band=0):
     """q, k, v: 4-D views [B,H,T,D] ("bhtd") or [B,T,H,D] ("bthd"), arbitrary batch/head/token strides.
     Returns o [B,T,H,D] contiguous and lse [B,H,T] fp32. band = nw > 0: the reference's tile band (a query of 128-token
     tile i sees the keys k <= q of tiles i - nw + 1 .. i; K/nki_attn_bandpro.py:1654); 0: all keys k <= q."""
-    for t in (q, k, v):
-        _attn_chk(t)
-    if layout == "bhtd":
-        B, H, T, D = q.shape
-    else:
-        B, T, H, D = q.shape
-    o = torch.empty(B, T, H, D, dtype=bf16, device=q.device)
-    lse = torch.empty(B, H, T, dtype=torch.float32, device=q.device)
     if band:
-        _lib.call("tfb_attn_fwd_band", _p(q), _bht(q, layout), _p(k), _bht(k, layout), _p(v), _bht(v, layout), _p(o),
-                  _bht(o, "bthd"), _p(lse), B, H, T, D, float(scale), int(band), _stream())
-    else:
-        _lib.call("tfb_attn_fwd", _p(q), _bht(q, layout), _p(k), _bht(k, layout), _p(v), _bht(v, layout), _p(o),
-                  _bht(o, "bthd"), _p(lse), B, H, T, D, float(scale), _stream())
-    return o, lse
+        return native.tfb_attn_fwd_band(q, k, v, scale, layout, band)
+    return native.tfb_attn_fwd(q, k, v, scale, layout)
 
 
 def attn_bwd(q, k, v, o, do, lse, scale, layout="bhtd", dq=None, dk=None, dv=None, out_layout="bhtd", rope=None, band=0):
     """Gradients of attn_fwd. o, do are [B,T,H,D]. dq/dk/dv may be given as (strided) views with `out_layout`;
     otherwise dq, dk are allocated [B,H,T,D] and dv [B,T,H,D] (returned as a [B,H,T,D] view), as the reference returns.
     rope = (cos, sin) (bf16 [T, D/2]): dq and dk come back with the inverse rotation applied (D = 64)."""
-    _attn_chk(q)
-    if q.dim() != 4:
-        raise ValueError("attention tensors are 4-D")
-    if layout == "bhtd":
-        B, H, T, D = q.shape
-    else:
-        B, T, H, D = q.shape
     if dq is None:
+        if q.dim() != 4:
+            raise ValueError("attention tensors are 4-D")
+        B, H, T, D = q.shape if layout == "bhtd" else (q.shape[0], q.shape[2], q.shape[1], q.shape[3])
         dq = torch.empty(B, H, T, D, dtype=bf16, device=q.device)
         dk = torch.empty(B, H, T, D, dtype=bf16, device=q.device)
         dv = torch.empty(B, T, H, D, dtype=bf16, device=q.device).permute(0, 2, 1, 3)
         out_layout = "bhtd"
-    _attn_bwd_chk(q, k, v, o, do, lse, dq, dk, dv, layout, out_layout)
-    delta = torch.empty(2, B, H, T, dtype=torch.float32, device=q.device)
-    cos, sin = rope if rope is not None else (None, None)
-    _chk(cos), _chk(sin)
-    ptrs = (_p(q), _bht(q, layout), _p(k), _bht(k, layout), _p(v), _bht(v, layout), _p(o), _bht(o, "bthd"), _p(do),
-            _bht(do, "bthd"), _p(dq), _bht(dq, out_layout), _p(dk), _bht(dk, out_layout), _p(dv), _bht(dv, out_layout), _p(lse),
-            _p(delta))
+    args = (q, k, v, o, do, lse, scale, layout, dq, dk, dv, out_layout)
     if band:
-        _lib.call("tfb_attn_bwd_band", *ptrs, _p(cos), _p(sin), B, H, T, D, float(scale), int(band), _stream())
+        native.tfb_attn_bwd_band(*args, *(rope or (None, None)), band)
     elif rope is not None:
-        _lib.call("tfb_attn_bwd_rope", *ptrs, _p(cos), _p(sin), B, H, T, D, float(scale), _stream())
+        native.tfb_attn_bwd_rope(*args, *rope)
     else:
-        _lib.call("tfb_attn_bwd", *ptrs, B, H, T, D, float(scale), _stream())
+        native.tfb_attn_bwd(*args)
     return dq, dk, dv
 
 
@@ -352,10 +299,7 @@ def attn_bwd_static(q, k, v, o, do, lse, scale, dq, dk, dv, layout="bhtd", out_l
     is a static device array inside the library (B * H * T <= tfb_attn_bwd_static_max_rows(); TfbError status 4 beyond).
     Calls that overlap on one GPU share that array and race; this wrapper creates no tensor either. The FIRST call on a
     device looks up the array's address: make one call eagerly before capturing this one into a HIP graph."""
-    B, H, T, D = _attn_bwd_chk(q, k, v, o, do, lse, dq, dk, dv, layout, out_layout)
-    _lib.call("tfb_attn_bwd_static", _p(q), _bht(q, layout), _p(k), _bht(k, layout), _p(v), _bht(v, layout), _p(o),
-              _bht(o, "bthd"), _p(do), _bht(do, "bthd"), _p(dq), _bht(dq, out_layout), _p(dk), _bht(dk, out_layout), _p(dv),
-              _bht(dv, out_layout), _p(lse), B, H, T, D, float(scale), _stream())
+    native.tfb_attn_bwd_static(q, k, v, o, do, lse, scale, layout, dq, dk, dv, out_layout)
     return dq, dk, dv
 
 
@@ -375,47 +319,21 @@ def relu2_bwd_from_h(h, dh):
 def rope_(x, cos, sin, T, nheads, D, inverse=False, out=None):
     """Rotate the first nheads*D columns of each row of x ([rows, row_stride] view, contiguous rows) in place
     (or into `out`). cos, sin: bf16 [T, D/2]; row r is token r % T."""
-    _chk(cos), _chk(sin)
-    if not x.is_cuda or x.dtype != bf16 or x.stride(-1) != 1:
-        raise TypeError("rope_ takes a bf16 device tensor with contiguous rows")
-    x2 = x.reshape(-1, x.shape[-1]) if x.is_contiguous() else x
-    rows, stride = x2.shape[0], x2.stride(0)
-    o = x2 if out is None else out
-    _lib.call("tfb_rope", _p(x2), _p(cos), _p(sin), _p(o), rows, T, nheads, D, stride, o.stride(0), int(inverse), _stream())
+    native.tfb_rope(x, cos, sin, T, nheads, D, inverse, out)
     return x if out is None else out
-
-
-def _rows2d(x):
-    if not x.is_cuda or x.dtype != bf16 or x.stride(-1) != 1:
-        raise TypeError("expected a bf16 device tensor with contiguous rows")
-    return x.reshape(-1, x.shape[-1]) if x.is_contiguous() else x
 
 
 def rope_norm_fwd(x, cos, sin, T, nheads, D, eps=2.0 ** -23, want_r=True):
     """RoPE then parameter-free RMSNorm of each of the first `nheads` heads (D columns each) of every row of x
     ([rows, row_stride] view). Returns (y [rows, nheads*D] normalised, r [rows, nheads*D] rotated or None,
     inv [rows, nheads] fp32)."""
-    _chk(cos), _chk(sin)
-    x2 = _rows2d(x)
-    rows = x2.shape[0]
-    y = torch.empty(rows, nheads * D, dtype=bf16, device=x.device)
-    r = torch.empty(rows, nheads * D, dtype=bf16, device=x.device) if want_r else None
-    inv = torch.empty(rows, nheads, dtype=torch.float32, device=x.device)
-    _lib.call("tfb_rope_norm_fwd", _p(x2), _p(cos), _p(sin), _p(r), _p(y), _p(inv), rows, T, nheads, D, x2.stride(0),
-              nheads * D, nheads * D, float(eps), _stream())
-    return y, r, inv
+    return native.tfb_rope_norm_fwd(x, cos, sin, T, nheads, D, eps, want_r)
 
 
 def rope_norm_bwd(g, r, inv, cos, sin, T, nheads, D, out=None):
     """The gradient of rope_norm_fwd's input from g (gradient of y; [rows, row_stride] view), the saved r and inv; written
     into `out` ([rows, row_stride] view) or a fresh [rows, nheads*D] tensor."""
-    _chk(cos), _chk(sin), _chk(r), _chk(inv, torch.float32)
-    g2 = _rows2d(g)
-    rows = g2.shape[0]
-    o = torch.empty(rows, nheads * D, dtype=bf16, device=g.device) if out is None else _rows2d(out)
-    _lib.call("tfb_rope_norm_bwd", _p(g2), _p(r), _p(inv), _p(cos), _p(sin), _p(o), rows, T, nheads, D, g2.stride(0),
-              r.stride(0), o.stride(0), _stream())
-    return o if out is None else out
+    return native.tfb_rope_norm_bwd(g, r, inv, cos, sin, T, nheads, D, out)
 
 
 def resmix_bwd(g, x, x0, ab):
@@ -437,16 +355,13 @@ def embedding_fwd(idx, weight):
 def embedding_bwd(idx, dy, dw, grouped=True):
     """dw (fp32 [V, C]) += scatter of dy rows by idx. grouped: rows sorted by token on the device and summed per token
     (deterministic order inside a token's run); False: one fp32 atomic add per element (the plain entry point)."""
+    if grouped:
+        native.tfb_embedding_bwd_grouped(idx, dy, dw)
+        return dw
     _chk(dy), _chk(dw, torch.float32)
     idx = idx.contiguous()
-    n, V = idx.numel(), dw.shape[0]
-    if not grouped:
-        _lib.call("tfb_embedding_bwd", _p(idx), int(idx.dtype == torch.int64), _p(dy), _p(dw), n, dy.shape[-1], V,
-                  _stream())
-        return dw
-    scr = _scratch(dw.device, _lib.lib().tfb_embedding_bwd_scratch_ints(n, V))  # 4-byte elements, used as int32
-    _lib.call("tfb_embedding_bwd_grouped", _p(idx), int(idx.dtype == torch.int64), _p(dy), _p(dw), n, dy.shape[-1], V,
-              _p(scr), _stream())
+    _lib.call("tfb_embedding_bwd", _p(idx), int(idx.dtype == torch.int64), _p(dy), _p(dw), idx.numel(), dy.shape[-1], dw.shape[0],
+              _stream())
     return dw
 
 
@@ -537,98 +452,38 @@ def moe_max_rows(N, E, topk):
 
 def moe_route(h2, wr, topk, bias=None, want_logits=False):
     """(p fp32 [N,E], idx int32 [N,topk], gate fp32 [N,topk], logits or None) from h2 bf16 [N,d], wr fp32 [E,d]."""
-    _chk(h2), _chk(wr, torch.float32), _chk(bias, torch.float32)
-    N, d = h2.shape
-    E = wr.shape[0]
-    dev = h2.device
-    p = torch.empty(N, E, dtype=torch.float32, device=dev)
-    idx = torch.empty(N, topk, dtype=torch.int32, device=dev)
-    gate = torch.empty(N, topk, dtype=torch.float32, device=dev)
-    logits = torch.empty(N, E, dtype=torch.float32, device=dev) if want_logits else None
-    _lib.call("tfb_moe_route", _p(h2), _p(wr), _p(bias), _p(logits), _p(p), _p(idx), _p(gate), N, d, E, topk, _stream())
-    return p, idx, gate, logits
+    return native.tfb_moe_route(h2, wr, topk, bias, want_logits)
 
 
 def moe_tables(idx, E, seq_len=None, capacity=None):
     """Slot tables for the ragged layout: dict(cnt, seg, tile_expert, slot, tok, ksel, rmax). Dropless by default; with
     seq_len and capacity the reference's per-sequence capacity (round2/source/train.py:10555-10634): each sequence keeps its
     first `capacity` assignments per expert, the rest get slot -1; the dict then also holds cnt_all (every assignment)."""
-    _chk(idx, torch.int32)
-    N, topk = idx.shape
-    dev = idx.device
-    rmax = moe_max_rows(N, E, topk)
-    i32 = dict(dtype=torch.int32, device=dev)
-    t = {"cnt": torch.empty(E, **i32), "seg": torch.empty(E + 1, **i32), "tile_expert": torch.empty(rmax // 128, **i32),
-         "slot": torch.empty(N, topk, **i32), "tok": torch.empty(rmax, **i32), "ksel": torch.empty(rmax, **i32), "rmax": rmax}
-    nw = (N + 63) // 64
     if capacity is None:
-        scratch = torch.empty(nw * E, **i32)
-        _lib.call("tfb_moe_tables", _p(idx), _p(t["cnt"]), _p(t["seg"]), _p(t["tile_expert"]), _p(t["slot"]), _p(t["tok"]),
-                  _p(t["ksel"]), _p(scratch), N, E, topk, rmax, _stream())
-        return t
-    if seq_len is None:
-        raise ValueError("a capacity is counted per sequence: seq_len is needed")
-    t["cnt_all"] = torch.empty(E, **i32)
-    t["capacity"] = int(capacity)
-    scratch = torch.empty(2 * nw * E, **i32)
-    _lib.call("tfb_moe_tables_cap", _p(idx), _p(t["cnt"]), _p(t["cnt_all"]), _p(t["seg"]), _p(t["tile_expert"]), _p(t["slot"]),
-              _p(t["tok"]), _p(t["ksel"]), _p(scratch), N, int(seq_len), int(capacity), E, topk, rmax, _stream())
-    return t
+        return native.tfb_moe_tables(idx, E)
+    return native.tfb_moe_tables_cap(idx, E, seq_len, capacity)
 
 
 def moe_gather(h2, tab, x_scale=4.0, want_xs=True):
     """(xs bf16 [rmax,d], xs8 uint8 [rmax,d]); x_scale None: no fp8 copy (xs8 is None); want_xs False: no bf16 copy (xs is
     None: fp8 experts whose weight gradients are in fp8 too never read it)."""
-    _chk(h2)
-    d = h2.shape[1]
-    rmax = tab["rmax"]
-    xs = torch.empty(rmax, d, dtype=bf16, device=h2.device) if want_xs or x_scale is None else None
-    if x_scale is None:
-        _lib.call("tfb_moe_gather", _p(h2), _p(tab["tok"]), None, 1.0, _p(xs), None, rmax, d, _stream())
-        return xs, None
-    xs8 = torch.empty(rmax, d, dtype=torch.uint8, device=h2.device)
-    if isinstance(x_scale, torch.Tensor):
-        _lib.call("tfb_moe_gather", _p(h2), _p(tab["tok"]), _p(x_scale), 0.0, _p(xs), _p(xs8), rmax, d, _stream())
-    else:
-        _lib.call("tfb_moe_gather", _p(h2), _p(tab["tok"]), None, float(x_scale), _p(xs), _p(xs8), rmax, d, _stream())
-    return xs, xs8
+    return native.tfb_moe_gather(h2, tab, x_scale, want_xs)
 
 
 def moe_mlp8_fwd(xs8, w8, rows, tab, F):
     """Grouped fp8 expert MLP forward: (ys bf16 [rmax,d], r bf16 [rmax,F]). w8 uint8 [E,4,F*d], rows fp32 [E,16]."""
-    _chk(xs8, torch.uint8), _chk(w8, torch.uint8), _chk(rows, torch.float32)
-    rmax, d = xs8.shape
-    ys = torch.empty(rmax, d, dtype=bf16, device=xs8.device)
-    r = torch.empty(rmax, F, dtype=bf16, device=xs8.device)
-    h8 = torch.empty(rmax, F, dtype=torch.uint8, device=xs8.device)
-    _lib.call("tfb_moe_mlp8_fwd", _p(xs8), _p(w8), _p(rows), _p(tab["tile_expert"]), _p(ys), _p(r), _p(h8), rmax, d, F, _stream())
-    return ys, r
+    return native.tfb_moe_mlp8_fwd(xs8, w8, rows, tab, F)
 
 
 def moe_mlp_fwd(xs, w_fc, w_proj, tab):
     """Grouped bf16 expert MLP forward: (ys bf16 [rmax,d], r bf16 [rmax,F] = relu(pre), h bf16 [rmax,F] = r^2).
     w_fc bf16 [E,F,d], w_proj bf16 [E,d,F]."""
-    _chk(xs), _chk(w_fc), _chk(w_proj)
-    rmax, d = xs.shape
-    E, F, _ = w_fc.shape
-    if tuple(w_fc.shape) != (E, F, d) or tuple(w_proj.shape) != (E, d, F):
-        raise ValueError("moe_mlp_fwd: w_fc [E,F,d] and w_proj [E,d,F] expected")
-    ys = torch.empty(rmax, d, dtype=bf16, device=xs.device)
-    r = torch.empty(rmax, F, dtype=bf16, device=xs.device)
-    h = torch.empty(rmax, F, dtype=bf16, device=xs.device)
-    _lib.call("tfb_moe_mlp_fwd", _p(xs), _p(w_fc), _p(w_proj), _p(tab["tile_expert"]), _p(ys), _p(r), _p(h), rmax, d, F, _stream())
-    return ys, r, h
+    return native.tfb_moe_mlp_fwd(xs, w_fc, w_proj, tab)
 
 
 def moe_mlp_bwd(dys, r, w_fc, w_proj, tab):
     """Grouped bf16 expert MLP backward: (dxs bf16 [rmax,d], dpre bf16 [rmax,F])."""
-    _chk(dys), _chk(r), _chk(w_fc), _chk(w_proj)
-    rmax, d = dys.shape
-    F = r.shape[1]
-    dxs = torch.empty(rmax, d, dtype=bf16, device=dys.device)
-    dpre = torch.empty(rmax, F, dtype=bf16, device=dys.device)
-    _lib.call("tfb_moe_mlp_bwd", _p(dys), _p(r), _p(w_fc), _p(w_proj), _p(tab["tile_expert"]), _p(dxs), _p(dpre), rmax, d, F, _stream())
-    return dxs, dpre
+    return native.tfb_moe_mlp_bwd(dys, r, w_fc, w_proj, tab)
 
 
 def moe_backward_scales(dys, rows, tab):
@@ -643,154 +498,77 @@ def moe_backward_scales(dys, rows, tab):
 
 def moe_backward_scales_rowmax(rowmax, rows, tab, d):
     """moe_backward_scales from the row maxima moe_combine_bwd(..., want_rowmax=True) left: the same rows, no pass over dys."""
-    _chk(rowmax, torch.float32), _chk(rows, torch.float32)
-    E = rows.shape[0]
-    out = torch.empty_like(rows)
-    _lib.call("tfb_moe_backward_scales_rowmax", _p(rowmax), _p(tab["seg"]), _p(rows), _p(out), d, E, _stream())
-    return out
+    return native.tfb_moe_backward_scales_rowmax(rowmax, rows, tab, d)
 
 
 def moe_quant(x, rows, col, fmt, tab):
-    _chk(x), _chk(rows, torch.float32)
-    out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    _lib.call("tfb_moe_quant", _p(x), _p(tab["tile_expert"]), _p(rows), col, fmt, _p(out), x.shape[0], x.shape[1], _stream())
-    return out
+    """fp8 bytes of x [rmax,d] at its rows' experts' scales rows[expert][col]; rows that no expert has are zero."""
+    return native.tfb_moe_quant(x, rows, col, fmt, tab)
+
+
+def moe_quant_dout(dout, gate, rows, tab):
+    """moe_quant(dys, rows, 5, FMT_E5M2, tab) of the dys that moe_combine_bwd writes, from dout itself."""
+    return native.tfb_moe_quant_dout(dout, gate, rows, tab)
 
 
 def moe_mlp8_bwd(dys, r, w8, rows_bwd, tab):
     """(dxs bf16 [rmax,d], dpre bf16 [rmax,F]) from dys; rows_bwd from moe_backward_scales."""
-    _chk(dys), _chk(r)
-    rmax, d = dys.shape
-    F = r.shape[1]
-    dy8 = moe_quant(dys, rows_bwd, 5, FMT_E5M2, tab)
-    dxs = torch.empty(rmax, d, dtype=bf16, device=dys.device)
-    dpre = torch.empty(rmax, F, dtype=bf16, device=dys.device)
-    dp8 = torch.empty(rmax, F, dtype=torch.uint8, device=dys.device)
-    _lib.call("tfb_moe_mlp8_bwd", _p(dy8), _p(r), _p(w8), _p(rows_bwd), _p(tab["tile_expert"]), _p(dxs), _p(dpre), _p(dp8), rmax, d,
-              F, _stream())
-    return dxs, dpre
+    return native.tfb_moe_mlp8_bwd(dys, r, w8, rows_bwd, tab)
 
 
 def moe_mlp8_bwd_q(dys, r, w8, rows_bwd, tab, hq_limit):
     """The grouped fp8 backward for the fp8 weight gradients: (dxs bf16 [rmax,d], dp8 e5m2 [rmax,F], hq8 e4m3 [rmax,F],
     dy8 e5m2 [rmax,d]); no bf16 dpre is written."""
-    _chk(dys), _chk(r)
-    rmax, d = dys.shape
-    F = r.shape[1]
     dy8 = moe_quant(dys, rows_bwd, 5, FMT_E5M2, tab)
-    dxs = torch.empty(rmax, d, dtype=bf16, device=dys.device)
-    dp8 = torch.empty(rmax, F, dtype=torch.uint8, device=dys.device)
-    hq8 = torch.empty(rmax, F, dtype=torch.uint8, device=dys.device)
-    _lib.call("tfb_moe_mlp8_bwd_q", _p(dy8), _p(r), _p(w8), _p(rows_bwd), _p(tab["tile_expert"]), _p(dxs), None, _p(dp8), _p(hq8),
-              float(hq_limit), rmax, d, F, _stream())
-    return dxs, dp8, hq8, dy8
+    return native.tfb_moe_mlp8_bwd_q(dy8, r, w8, rows_bwd, tab, hq_limit) + (dy8,)
 
 
 def moe_dw8(xs8, dp8, hq8, dy8, rows_bwd, x_scale, tab, E, dw_fc=None, dw_proj=None, accumulate=False, out_dtype=bf16):
     """(dw_fc [E,F,d], dw_proj [E,d,F]) in fp8 over each expert's row segment, from the bytes the other GEMMs multiplied."""
-    _chk(xs8, torch.uint8), _chk(dp8, torch.uint8), _chk(hq8, torch.uint8), _chk(dy8, torch.uint8), _chk(rows_bwd, torch.float32)
-    d, F = xs8.shape[1], dp8.shape[1]
-    if dw_fc is None:
-        dw_fc = torch.empty(E, F, d, dtype=out_dtype, device=xs8.device)
-        dw_proj = torch.empty(E, d, F, dtype=out_dtype, device=xs8.device)
-    _lib.call("tfb_moe_dw8", _p(xs8), _p(dp8), _p(hq8), _p(dy8), _p(rows_bwd), float(x_scale), _p(tab["seg"]), _p(dw_fc), _p(dw_proj),
-              E, d, F, int(dw_fc.dtype == torch.float32), int(accumulate), _stream())
-    return dw_fc, dw_proj
+    return native.tfb_moe_dw8(xs8, dp8, hq8, dy8, rows_bwd, x_scale, tab, E, dw_fc, dw_proj, accumulate, out_dtype == torch.float32)
 
 
 def moe_dw(dpre, xs, dys, r, tab, E, dw_fc=None, dw_proj=None, accumulate=False, out_dtype=bf16):
     """(dw_fc [E,F,d], dw_proj [E,d,F]) over each expert's row segment."""
-    d, F = xs.shape[1], r.shape[1]
-    if dw_fc is None:
-        dw_fc = torch.empty(E, F, d, dtype=out_dtype, device=xs.device)
-        dw_proj = torch.empty(E, d, F, dtype=out_dtype, device=xs.device)
-    _lib.call("tfb_moe_dw", _p(dpre), _p(xs), _p(dys), _p(r), _p(tab["seg"]), _p(dw_fc), _p(dw_proj), E, d, F,
-              int(dw_fc.dtype == torch.float32), int(accumulate), _stream())
-    return dw_fc, dw_proj
+    return native.tfb_moe_dw(dpre, xs, dys, r, tab, E, dw_fc, dw_proj, accumulate, out_dtype == torch.float32)
 
 
 def moe_combine(ys, tab, gate, N):
-    _chk(ys), _chk(gate, torch.float32)
-    d = ys.shape[1]
-    out = torch.empty(N, d, dtype=bf16, device=ys.device)
-    _lib.call("tfb_moe_combine", _p(ys), _p(tab["slot"]), _p(gate), _p(out), N, d, gate.shape[1], _stream())
-    return out
+    """out [N,d]: the sum over a token's experts of its gates times their rows."""
+    if gate.shape[0] != N:
+        raise ValueError("gate [N, topk]")
+    return native.tfb_moe_combine(ys, tab, gate)
 
 
 def moe_combine_bwd(dout, ys, tab, gate, want_rowmax=False):
     """(dys, dgate), and with want_rowmax the fp32 [rmax] maxima of |dys| per row for moe_backward_scales_rowmax."""
-    _chk(dout), _chk(ys), _chk(gate, torch.float32)
-    rmax, d = ys.shape
-    dys = torch.empty_like(ys)
-    # the kernel writes the gate gradient of every assignment that holds a row; a skipped one's is zero
-    dgate = torch.zeros_like(gate) if "capacity" in tab else torch.empty_like(gate)
     if want_rowmax:
-        rowmax = torch.empty(rmax, dtype=torch.float32, device=ys.device)
-        _lib.call("tfb_moe_combine_bwd_rowmax", _p(dout), _p(ys), _p(tab["tok"]), _p(tab["ksel"]), _p(gate), _p(dys), _p(dgate),
-                  _p(rowmax), rmax, d, gate.shape[1], _stream())
-        return dys, dgate, rowmax
-    _lib.call("tfb_moe_combine_bwd", _p(dout), _p(ys), _p(tab["tok"]), _p(tab["ksel"]), _p(gate), _p(dys), _p(dgate), rmax, d,
-              gate.shape[1], _stream())
-    return dys, dgate
+        return native.tfb_moe_combine_bwd_rowmax(dout, ys, tab, gate, True)
+    return native.tfb_moe_combine_bwd(dout, ys, tab, gate)
 
 
 def moe_route_bwd(dgate, p, idx, dxs, tab, h2, wr, dwr=None, accumulate=False, aux=None):
     """(dh bf16 [N,d], dwr fp32 [E,d], dlogits fp32 [N,E]). aux = (terms, lse, gaux, alpha, beta): the gradient gaux
     (1-element fp32 device tensor) of the weighted auxiliary terms alpha lb + beta z of moe_aux_fwd is folded into dlogits;
     aux = (terms, lse, gaux, alpha, beta, fs, gamma, seq_len) adds the per-sequence term gamma seq of moe_aux_seq_fwd."""
-    N, d = h2.shape
-    E = wr.shape[0]
-    dlogits = torch.empty(N, E, dtype=torch.float32, device=h2.device)
-    dh = torch.empty_like(h2)
-    if dwr is None:
-        dwr = torch.empty(E, d, dtype=torch.float32, device=h2.device)
-        accumulate = False
-    scr = _scratch(h2.device, 64 * E * d)
+    args = (dgate, p, idx, dxs, tab, h2, wr, dwr, accumulate)
     if aux is None:
-        _lib.call("tfb_moe_route_bwd", _p(dgate), _p(p), _p(idx), _p(dxs), _p(tab["slot"]), _p(h2), _p(wr), _p(dlogits), _p(dh),
-                  _p(dwr), int(accumulate), _p(scr), N, d, E, idx.shape[1], _stream())
-    elif len(aux) == 8:
-        terms, lse, gaux, alpha, beta, fs, gamma, seq_len = aux
-        _chk(terms, torch.float32), _chk(lse, torch.float32), _chk(gaux, torch.float32), _chk(fs, torch.float32)
-        if N % int(seq_len) or tuple(fs.shape) != (N // int(seq_len), E):
-            raise ValueError("moe_route_bwd: fs must be [N / seq_len, E]")
-        _lib.call("tfb_moe_route_bwd_aux_seq", _p(dgate), _p(p), _p(idx), _p(dxs), _p(tab["slot"]), _p(h2), _p(wr), _p(dlogits),
-                  _p(dh), _p(dwr), int(accumulate), _p(scr), _p(terms), _p(lse), _p(gaux), float(alpha), float(beta), _p(fs),
-                  float(gamma), int(seq_len), N, d, E, idx.shape[1], _stream())
-    else:
-        terms, lse, gaux, alpha, beta = aux
-        _chk(terms, torch.float32), _chk(lse, torch.float32), _chk(gaux, torch.float32)
-        _lib.call("tfb_moe_route_bwd_aux", _p(dgate), _p(p), _p(idx), _p(dxs), _p(tab["slot"]), _p(h2), _p(wr), _p(dlogits),
-                  _p(dh), _p(dwr), int(accumulate), _p(scr), _p(terms), _p(lse), _p(gaux), float(alpha), float(beta), N, d, E,
-                  idx.shape[1], _stream())
-    return dh, dwr, dlogits
+        return native.tfb_moe_route_bwd(*args)
+    if len(aux) == 8:
+        return native.tfb_moe_route_bwd_aux_seq(*args, *aux)
+    return native.tfb_moe_route_bwd_aux(*args, *aux)
 
 
 def moe_aux_fwd(p, logits, tab, topk):
     """(terms fp32 [2 + E] = (lb, z, f_e), lse fp32 [N]): the router's load-balance term E sum_e f_e P_e, its z term
     mean(logsumexp(logits)^2) and the experts' load shares (round2/source/train.py:10779 moe_aux_terms)."""
-    _chk(p, torch.float32), _chk(logits, torch.float32)
-    N, E = p.shape
-    terms = torch.empty(2 + E, dtype=torch.float32, device=p.device)
-    lse = torch.empty(N, dtype=torch.float32, device=p.device)
-    scr = torch.empty(64 * 17, dtype=torch.float32, device=p.device)
-    _lib.call("tfb_moe_aux_fwd", _p(p), _p(logits), _p(tab.get("cnt_all", tab["cnt"])), _p(terms), _p(lse), _p(scr), N, E, topk, _stream())
-    return terms, lse
+    return native.tfb_moe_aux_fwd(p, logits, tab, topk)
 
 
 def moe_aux_seq_fwd(p, idx, seq_len, topk):
     """(term fp32 [1], fs fp32 [N / seq_len, E]): the per-sequence balance term of moe_aux_terms
     (round2/source/train.py:10789-10792) = mean over sequences of E sum_e fs ps, and the sequences' load shares."""
-    _chk(p, torch.float32), _chk(idx, torch.int32)
-    N, E = p.shape
-    T = int(seq_len)
-    if T <= 0 or N % T:
-        raise ValueError("moe_aux_seq_fwd: %d tokens are not whole sequences of %d" % (N, T))
-    fs = torch.empty(N // T, E, dtype=torch.float32, device=p.device)
-    term = torch.empty(1, dtype=torch.float32, device=p.device)
-    scr = torch.empty(N // T, dtype=torch.float32, device=p.device)
-    _lib.call("tfb_moe_aux_seq_fwd", _p(p), _p(idx), _p(fs), _p(term), _p(scr), N, T, E, topk, _stream())
-    return term, fs
+    return native.tfb_moe_aux_seq_fwd(p, idx, seq_len, topk)
 
 
 # ------------------------------------------------------------------------------------------ Muon Newton-Schulz
