@@ -22,30 +22,11 @@
 // Before, with plain loops whose LDS reads stood right in front of their MFMAs -> now: B3 H8 T1664 forward 52 -> 35 us, backward
 // 164 -> 118; B1 H8 T2048 56 -> 35, 177 -> 122; B16 H6 T2048 155 -> 120, 600 -> 475.
 #include <type_traits>
-#include "common.hpp"
+#include "attention_core.hpp"
 
 namespace {
 
-struct AttnT {
-  bf16_t* p;
-  long sb, sh, st;
-};
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef const __attribute__((address_space(1))) void glb_void_t;
 typedef __attribute__((address_space(1))) uint8_t glb_u8_t;
-
-constexpr float LOG2E = 1.4426950408889634f;
-constexpr float LN2 = 0.6931471805599453f;
-
-__device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-__device__ __forceinline__ bf16x8 frag_from(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-  u32x4 v = {a, b, c, d};
-  return __builtin_bit_cast(bf16x8, v);
-}
 
 template <int D>
 struct Geo {
@@ -61,43 +42,6 @@ struct Geo {
     return ((t & 3) << 2) | ((t >> 2) & 3);
   }
 };
-
-// Workgroup -> (sequence block slot bx, batch x head index bh). Workgroup ids are dealt round-robin over the 8 XCDs, so
-// id & 7 is the XCD: every (batch, head) pair is given to one XCD. With paired blocks (gridDim.x = nx / 2, equal work per
-// workgroup) a pair's workgroups are consecutive on their XCD; with one block per workgroup (gridDim.x = nx) the order on
-// an XCD is slot-major - the heaviest block of each of its pairs first, then the next heaviest of each - which is
-// longest-first scheduling of the unequal causal work, and the blocks of one pair that run together stream the same
-// K/V (Q/dO) tiles at the same time.
-__device__ __forceinline__ void xcd_block(int nx, int nbh, int& bx, int& bh) {
-  const int gx = gridDim.x, lin = blockIdx.y * gx + blockIdx.x;
-  if (nbh % 8 == 0) {
-    const int xcd = lin & 7, idx = lin >> 3;
-    if (gx == nx) {
-      const int per = nbh >> 3;
-      bx = idx / per;
-      bh = xcd + 8 * (idx % per);
-    } else {
-      bh = xcd + 8 * (idx / gx);
-      bx = idx % gx;
-    }
-  } else {
-    bh = blockIdx.y;
-    bx = blockIdx.x;
-  }
-}
-__device__ __forceinline__ int paired_passes(int nx) { return (int)gridDim.x * 2 == nx ? 2 : 1; }
-__device__ __forceinline__ int paired_block(int nx, int bx, int pass, bool heavy_last) {
-  const int first = heavy_last ? nx - 1 - bx : bx;
-  return pass == 0 ? first : nx - 1 - first;
-}
-// first 64-key tile a 128-token query tile qb sees under a band of nw key tiles; 0 without a band
-__device__ __forceinline__ int band_first_tile(int qb, int nw) { return nw > 0 && qb - nw + 1 > 0 ? 2 * (qb - nw + 1) : 0; }
-// Blocks are paired when the paired grid fills its rounds of resident workgroups to 90 % (or is long enough not to care).
-__host__ inline unsigned paired_grid(int nx, int nbh, int per_cu) {
-  if (nx % 2) return (unsigned)nx;
-  const long wgs = (long)(nx / 2) * nbh, slots = tfb_resident_slots(per_cu), rounds = (wgs + slots - 1) / slots;
-  return (unsigned)(wgs * 10 >= rounds * slots * 9 ? nx / 2 : nx);
-}
 
 // This wavefront's share of a (16 NI TPI / 4 ...)-token tile load: instructions g = wave + 4 i, i < NI, each TPI tokens.
 template <int D, int NI>
@@ -215,12 +159,6 @@ struct FragAddr {
 };
 // all of this wavefront's loads into LDS have landed, and every wavefront is here
 __device__ __forceinline__ void tile_barrier() { asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); }
-__device__ __forceinline__ float max_halves(float x) {  // the larger of the two lanes' that share a query
-  float y = x;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y));
-  return fmaxf(x, y);
-}
-
 // =========================================================================================== forward
 template <int D>
 __global__ __launch_bounds__(256, 2) void attnD_fwd_kernel(AttnT q, AttnT k, AttnT v, AttnT o, float* __restrict__ lse, int T,
@@ -967,8 +905,6 @@ __global__ __launch_bounds__(256, 1) void attnD_dkdv_kernel(AttnT q, AttnT k, At
     if (pass + 1 < npass) __syncthreads();  // the stages are free for the partner block
   }
 }
-
-AttnT mk(const void* p, const long* s) { return AttnT{(bf16_t*)p, s[0], s[1], s[2]}; }
 
 template <int D>
 int fwd_launch(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, void* o,

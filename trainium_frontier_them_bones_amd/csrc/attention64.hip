@@ -26,7 +26,7 @@
 // being in the opposite phase. dK/dV has no registers left for a second set of scores at two wavefronts per SIMD and
 // keeps the plain loop.
 #include <type_traits>
-#include "common.hpp"
+#include "attention_core.hpp"
 
 // wavefronts per SIMD the kernels are compiled for (register budget 512 / n)
 #ifndef TFB_DKDV64_QT
@@ -56,84 +56,18 @@
 
 namespace {
 
-struct AttnT {
-  bf16_t* p;
-  long sb, sh, st;
-};
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-typedef const __attribute__((address_space(1))) void glb_void_t;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4_t;
 
-constexpr float LOG2E = 1.4426950408889634f;
-constexpr float LN2 = 0.6931471805599453f;
 constexpr int TILE = 64 * 128;  // bytes of one staged tile
 
-__device__ __forceinline__ f32x16 mfma_bf16(bf16x8 a, bf16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
-__device__ __forceinline__ bf16x8 frag_from(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
-  u32x4 v = {a, b, c, d};
-  return __builtin_bit_cast(bf16x8, v);
-}
 __device__ __forceinline__ void wait_all_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // s_waitcnt vmcnt(0)
-__device__ __forceinline__ float max_halves(float x) {  // the larger of the two lanes' that share a query
-  float y = x;
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y));
-  return fmaxf(x, y);
-}
 // A stage's barrier: the loads into LDS that this wavefront has in flight are part of what the others read behind it (the compiler
 // may leave their wait to the first read of its own).
 __device__ __forceinline__ void stage_barrier() {
   wait_all_loads();
   __syncthreads();
-}
-
-// Workgroup -> (block along the sequence, batch*head): consecutive workgroup ids are dealt round-robin to the 8 XCDs, each with its own
-// L2, so the ids are re-dealt to keep all sequence blocks of one (batch, head) - which stream the same K/V (or Q/dO) tiles - on one
-// XCD; with one block per workgroup (gridDim.x = nx) in slot-major order, the heaviest block of each pair first. nx = blocks per
-// (batch, head), nbh = batch*head count.
-__device__ __forceinline__ void xcd_block(int nx, int nbh, int& bx, int& bh) {
-  const int gx = gridDim.x, lin = blockIdx.y * gx + blockIdx.x;
-  if (nbh % 8 == 0) {
-    const int xcd = lin & 7, idx = lin >> 3;
-    if (gx == nx) {
-      const int per = nbh >> 3;
-      bx = idx / per;
-      bh = xcd + 8 * (idx % per);
-    } else {
-      bh = xcd + 8 * (idx / gx);
-      bx = idx % gx;
-    }
-  } else {
-    bh = blockIdx.y;
-    bx = blockIdx.x;
-  }
-}
-
-// Causal work per 128-token block grows linearly along the sequence, and workgroups are dispatched in id order: with one
-// block per workgroup the heaviest blocks of the last (batch, head) pairs start when most of the grid has drained and
-// run on alone (for 16 blocks x 192 pairs on 512 slots: 17 % of the kernel's time). When the block count nx is even a
-// workgroup therefore does block i and then block nx - 1 - i (gridDim.x = nx / 2): every workgroup carries the same
-// work. `heavy_last` = the work grows with the block index (query blocks) rather than falls (key blocks); the heavier
-// block of the pair runs first either way.
-__device__ __forceinline__ int paired_passes(int nx) { return (int)gridDim.x * 2 == nx ? 2 : 1; }
-__device__ __forceinline__ int paired_block(int nx, int bx, int pass, bool heavy_last) {
-  const int first = heavy_last ? nx - 1 - bx : bx;
-  return pass == 0 ? first : nx - 1 - first;
-}
-// First 64-key tile a 128-token query tile qb sees under a band of nw key tiles (a query of tile i sees the keys k <= q
-// of tiles i - nw + 1 .. i: band_mask, round2/source/kernels/nki_attn_bandpro.py:1654); 0 without a band (nw <= 0).
-__device__ __forceinline__ int band_first_tile(int qb, int nw) { return nw > 0 && qb - nw + 1 > 0 ? 2 * (qb - nw + 1) : 0; }
-// Blocks are paired when the paired grid fills its rounds of resident workgroups to 90 % (or is long enough not to care); otherwise
-// one block per workgroup, the heaviest first (B8 H8 T512 forward 14.3 -> 10.8 us, backward 43 -> 33; B1 H12 T2048 31 -> 27, 89 -> 80).
-__host__ inline unsigned paired_grid(int nx, int nbh, int per_cu) {
-  if (nx % 2) return (unsigned)nx;
-  const long wgs = (long)(nx / 2) * nbh, slots = tfb_resident_slots(per_cu), rounds = (wgs + slots - 1) / slots;
-  return (unsigned)(wgs * 10 >= rounds * slots * 9 ? nx / 2 : nx);
 }
 
 __device__ __forceinline__ int swz(int t) { return (((t >> 1) & 1) << 2) | ((t >> 2) & 3); }
@@ -920,8 +854,6 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
   __syncthreads();  // the stages are free for the partner block
   }
 }
-
-AttnT mk(const void* p, const long* s) { return AttnT{(bf16_t*)p, s[0], s[1], s[2]}; }
 
 }  // namespace
 
