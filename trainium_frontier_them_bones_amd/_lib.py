@@ -155,7 +155,7 @@ def _telling(name):
         try:
             return getattr(dict, name)(self, *args, **kw)
         finally:
-            native.timed_changed()
+            native.told()
     method.__name__ = name
     return method
 
@@ -165,6 +165,8 @@ for _name in ("__setitem__", "__delitem__", "__ior__", "update", "setdefault", "
 
 
 TIMED = _Timed()
+
+REPLACED = {}   # name -> function: what a program has put in the place of functions of ops (kept there)
 
 
 def _timed_begin(name):
@@ -204,11 +206,12 @@ HOST_PATH = os.path.join(HERE, "_tfb_host.so")
 class _Native:
     """The extension module, loaded on first use (the package imports without a built library)."""
 
-    def timed_changed(self):
-        """Tells the extension, once it is loaded, whether any entry point is timed."""
-        tell = self.__dict__.get("set_timed")
-        if tell is not None:
-            tell(bool(TIMED))
+    def told(self):
+        """Tells the extension, once it is loaded, whether any entry point is timed and any function of ops replaced."""
+        for name, table in (("set_timed", TIMED), ("set_replaced", REPLACED)):
+            tell = self.__dict__.get(name)
+            if tell is not None:
+                tell(bool(table))
 
     def __getattr__(self, name):
         lib()      # first: the extension binds to the library loaded from LIB_PATH
@@ -222,7 +225,7 @@ class _Native:
         mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_tfb_host", loader))
         loader.exec_module(mod)
         self.__dict__.update((k, v) for k, v in vars(mod).items() if not k.startswith("__"))
-        self.timed_changed()
+        self.told()
         try:
             return self.__dict__[name]
         except KeyError:

@@ -1,6 +1,7 @@
 // Python bindings of the native host layer (module _tfb_host): the nodes under their Python class names and the tensor-level ops under
 // the names of the entry points they run. Plain vectorcall functions: positional arguments, None for "not given".
 #include "nodes.hpp"
+#include "wrapped.hpp"
 
 namespace tfb {
 
@@ -69,7 +70,7 @@ struct Args {
   }
   at::ScalarType dtype(int i) const { return has(i) && b(i) ? F32 : BF16; }   // "fp32 output?"
   bool bthd(int i) const { return !is(i, "bhtd"); }   // a layout's name
-  MoeTab tab(int i) const;                            // the dict that tfb_moe_tables returns
+  MoeTab tab(int i) const { return from_dict(need(i)); }
   bool is(int i, const char* s) const { return has(i) && PyUnicode_Check(a[i]) && PyUnicode_CompareWithASCIIString(a[i], s) == 0; }
 };
 
@@ -94,36 +95,6 @@ PyObject* outs(const Tensors& v) {
   return r;
 }
 PyObject* none() { Py_RETURN_NONE; }
-
-// A dict's entry as a tensor (undefined: none of that name).
-Tensor dict_tensor(PyObject* d, const char* key) {
-  PyObject* v = PyDict_GetItemString(d, key);
-  return v && THPVariable_Check(v) ? THPVariable_Unpack(v) : Tensor();
-}
-MoeTab Args::tab(int i) const {
-  PyObject* d = need(i);
-  TORCH_CHECK_TYPE(PyDict_Check(d), "argument ", i + 1, " must be the dict of the slot tables");
-  MoeTab t{dict_tensor(d, "cnt"), dict_tensor(d, "seg"), dict_tensor(d, "tile_expert"), dict_tensor(d, "slot"), dict_tensor(d, "tok"),
-           dict_tensor(d, "ksel"), dict_tensor(d, "cnt_all")};
-  for (const Tensor* x : {&t.cnt, &t.seg, &t.tile_expert, &t.slot, &t.tok, &t.ksel}) {
-    TORCH_CHECK_TYPE(x->defined(), "the slot tables are incomplete");
-    chk(*x, I32);
-  }
-  t.rmax = t.tok.numel();
-  t.capped = PyDict_GetItemString(d, "capacity") != nullptr;
-  return t;
-}
-PyObject* out(const MoeTab& t, int64_t capacity) {
-  PyObject* d = PyDict_New();
-  auto put = [&](const char* key, PyObject* v) {
-    PyDict_SetItemString(d, key, v);
-    Py_DECREF(v);
-  };
-  put("cnt", out(t.cnt)), put("seg", out(t.seg)), put("tile_expert", out(t.tile_expert)), put("slot", out(t.slot));
-  put("tok", out(t.tok)), put("ksel", out(t.ksel)), put("rmax", PyLong_FromLongLong(t.rmax));
-  if (t.capped) put("cnt_all", out(t.cnt_all)), put("capacity", PyLong_FromLongLong(capacity));
-  return d;
-}
 
 template <PyObject* (*F)(const Args&), int LO, int HI>   // a function of LO to HI arguments
 PyObject* entry(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -198,7 +169,7 @@ PyObject* op_rmsnorm_fwd(const Args& a) {
   return outs(o.s, o.y, o.inv);
 }
 PyObject* op_rmsnorm_fwd_q(const Args& a) {
-  NormOut o = rmsnorm_fwd_q(a.t(0), a.opt(1), a.f(2), a.opt(3), a.f(4), a.b(5));
+  NormOut o = rmsnorm_fwd_q(a.t(0), a.opt(1), a.f(2), a.opt(3), a.f(4), a.b(5), a.n > 6 ? a.i(6) : 0);
   return outs(o.s, o.y, o.inv, o.y8);
 }
 PyObject* op_rmsnorm_bwd(const Args& a) {
@@ -327,8 +298,7 @@ PyObject* op_moe_route(const Args& a) {   // h, wr, topk, bias, want_logits
   return outs(o.p, o.idx, o.gate, o.logits);
 }
 PyObject* op_moe_tables(const Args& a) {   // idx, E, seq_len, capacity
-  const int64_t cap = a.i_or(3, -1);
-  return out(moe_tables(a.t(0), a.i(1), a.i_or(2, -1), cap), cap);
+  return to_dict(moe_tables(a.t(0), a.i(1), a.i_or(2, -1), a.i_or(3, -1)));
 }
 PyObject* op_moe_gather(const Args& a) {   // h, tab, x_scale, want_xs
   const Scale s = a.has(2) ? a.scale(2) : Scale{};
@@ -385,6 +355,11 @@ PyObject* set_timed(const Args& a) {
   return none();
 }
 
+PyObject* set_replaced(const Args& a) {
+  any_replaced = a.b(0);
+  return none();
+}
+
 // name, function, the least and the largest number of arguments
 #define FN(name, f, lo, hi) \
   {name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<f, lo, hi>)), METH_FASTCALL, nullptr}
@@ -397,9 +372,9 @@ PyMethodDef methods[] = {
     FN("qkv_rope_attention", py_qkv_rope_attention, 6, 6), FN("mlp8", py_mlp8, 4, 6), FN("nr_mlp", py_nr_mlp, 4, 5),
     FN("mlp_fused", py_mlp_fused, 3, 3), FN("moe", py_moe, 7, 10), FN("lm_head_loss", py_lm_head_loss, 5, 5), FN("fused_loss", py_fused_loss, 3, 3),
     FN("reduced_loss", py_reduced_loss, 4, 4), FN("embedding", py_embedding, 2, 2), FN("attach_amax", py_attach_amax, 2, 2),
-    FN("amax_hint", py_amax_hint, 2, 2), FN("set_timed", set_timed, 1, 1), FN("tfb_gemm_bf16", op_gemm, 7, 7),
+    FN("amax_hint", py_amax_hint, 2, 2), FN("set_timed", set_timed, 1, 1), FN("set_replaced", set_replaced, 1, 1), FN("tfb_gemm_bf16", op_gemm, 7, 7),
     FN("tfb_gemm_bf16_scaled", op_gemm, 8, 8), FN("tfb_gemm_bf16_res", op_gemm_res, 4, 4), FN("tfb_qkv_rope_fwd", op_qkv_rope, 6, 6),
-    FN("tfb_rmsnorm_fwd", op_rmsnorm_fwd, 4, 4), FN("tfb_rmsnorm_fwd_q", op_rmsnorm_fwd_q, 6, 6), FN("tfb_rmsnorm_bwd", op_rmsnorm_bwd, 9, 9),
+    FN("tfb_rmsnorm_fwd", op_rmsnorm_fwd, 4, 4), FN("tfb_rmsnorm_fwd_q", op_rmsnorm_fwd_q, 6, 6), FN("tfb_rmsnorm_fwd_q_pad", op_rmsnorm_fwd_q, 7, 7), FN("tfb_rmsnorm_bwd", op_rmsnorm_bwd, 9, 9),
     FN("tfb_rmsnorm_bwd_amax", op_rmsnorm_bwd, 9, 9), FN("tfb_block_head_fwd", op_block_head_fwd, 5, 5),
     FN("tfb_block_head_bwd", op_block_head_bwd, 8, 8), FN("tfb_mix_tail_fwd", op_mix_tail_fwd, 4, 4), FN("tfb_mix_tail_bwd", op_mix_tail_bwd, 7, 7),
     FN("tfb_mlp8_backward_scales", op_mlp8_backward_scales, 2, 2), FN("tfb_mlp8_backward_scales_part", op_mlp8_backward_scales, 3, 3),

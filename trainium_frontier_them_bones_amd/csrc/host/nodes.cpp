@@ -3,6 +3,7 @@
 // the reference (round1/source/train.py:8463-8472): a weight with a `grad_buf` attribute gets its gradient added into that
 // buffer and None is handed to autograd.
 #include "nodes.hpp"
+#include "wrapped.hpp"
 
 #include <torch/csrc/autograd/custom_function.h>
 
@@ -11,6 +12,7 @@ namespace tfb {
 using torch::autograd::AutogradContext;
 using torch::autograd::Function;
 using Vars = torch::autograd::variable_list;
+namespace op = wrapped;
 
 namespace {
 
@@ -153,7 +155,7 @@ NormBack norm_backward(const Tensor& gy, const Tensor& s, const Tensor& inv, con
     }
     if (!part.defined()) g = accumulate_into(w, true);
   }
-  NormGrad n = rmsnorm_bwd(dense(gy), s, inv, w, dense(gs), g.buf, g.accumulate, part, want_amax);
+  NormGrad n = op::rmsnorm_bwd(dense(gy), s, inv, w, dense(gs), g.buf, g.accumulate, part, want_amax);
   NormBack b{n.dx, {}, n.amax};
   if (w.defined() && !part.defined() && !g.buf.defined()) b.gw = n.dw.to(w.scalar_type());
   return b;
@@ -163,43 +165,23 @@ NormBack norm_backward(const Tensor& gy, const Tensor& s, const Tensor& inv, con
 Tensor weight_grad(const Tensor& w, const Tensor& g, const Tensor& a, int64_t M, int64_t N, int64_t K) {
   GradBuf gb = accumulate_into(w);
   if (gb.buf.defined()) {
-    gemm(g, a, gb.buf, N, K, M, true, false, gb.accumulate);
+    op::gemm(g, a, gb.buf, N, K, M, true, false, gb.accumulate);
     return {};
   }
   Tensor dw = make({N, K}, BF16, g);
-  gemm(g, a, dw, N, K, M, true, false, false);
+  op::gemm(g, a, dw, N, K, M, true, false, false);
   return dw;
-}
-
-// The function that a program has put in the place of ops.<name> on the Python side (instrumentation wraps an op that way), or
-// nullptr while the package's own is there. A borrowed reference; under the GIL.
-PyObject* replaced(const char* name) {
-  static PyObject* ops_dict = PyModule_GetDict(PyImport_ImportModule("trainium_frontier_them_bones_amd.ops"));
-  static PyObject* own = PyDict_GetItemString(ops_dict, "_WRAPPABLE");
-  PyObject* fn = PyDict_GetItemString(ops_dict, name);
-  return fn == PyDict_GetItemString(own, name) ? nullptr : fn;
-}
-PyObject* call_python(PyObject* fn, std::initializer_list<PyObject*> args) {   // steals the arguments; nullptr stands for None
-  PyObject* t = PyTuple_New(args.size());
-  Py_ssize_t i = 0;
-  for (PyObject* a : args) PyTuple_SET_ITEM(t, i++, a ? a : (Py_INCREF(Py_None), Py_None));
-  PyObject* r = PyObject_CallObject(fn, t);
-  Py_DECREF(t);
-  if (!r) {
-    python_error e;
-    e.persist();
-    throw e;
-  }
-  return r;
 }
 
 // The scale row of an fp8 MLP backward: from the amax partials on the gradient when they are still valid, else from a pass over
 // it.
 Tensor backward_scales(const Tensor& gy, const Tensor& g2, const Tensor& row) {
-  pybind11::gil_scoped_acquire gil;
-  PyObject* hint = switched_on(names().use_amax) ? amax_hint(gy, g2) : nullptr;
-  if (PyObject* fn = replaced("mlp8_backward_scales")) return tensor_of(call_python(fn, {THPVariable_Wrap(g2), THPVariable_Wrap(row), hint}));
-  return mlp8_backward_scales(g2, row, tensor_of(hint));
+  Tensor hint;
+  {
+    pybind11::gil_scoped_acquire gil;
+    if (switched_on(names().use_amax)) hint = tensor_of(amax_hint(gy, g2));
+  }
+  return op::mlp8_backward_scales(g2, row, hint);
 }
 
 void attach(const Tensor& dx, const Tensor& amax) {
@@ -228,7 +210,7 @@ struct RmsNorm : Function<RmsNorm> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x_, const OptTensor& w_, double eps) {
     ctx->set_materialize_grads(false);
     const Tensor x = dense(x_), w = val(w_);
-    NormOut o = rmsnorm_fwd(x, w, eps, {});
+    NormOut o = op::rmsnorm_fwd(x, w, eps, {});
     ctx->save_for_backward({x, o.inv, w});
     return o.y;
   }
@@ -247,11 +229,11 @@ struct RmsNormPass : Function<RmsNormPass> {
     TORCH_CHECK_VALUE(y8_scale || !bytes_only, "bytes_only needs y8_scale");
     const Tensor x = dense(x_), w = val(w_);
     if (!y8_scale) {
-      NormOut o = rmsnorm_fwd(x, w, eps, {});
+      NormOut o = op::rmsnorm_fwd(x, w, eps, {});
       ctx->save_for_backward({x, o.inv, w});
       return {x, o.y};
     }
-    NormOut o = rmsnorm_fwd_q(x, w, eps, {}, *y8_scale, !bytes_only);
+    NormOut o = op::rmsnorm_fwd_q(x, w, eps, {}, *y8_scale, !bytes_only);
     ctx->mark_non_differentiable({o.y8});
     ctx->save_for_backward({x, o.inv, w});
     return {x, bytes_only ? nan_placeholder(x) : o.y, o.y8};
@@ -270,7 +252,7 @@ struct AddRmsNorm : Function<AddRmsNorm> {
   static Vars forward(AutogradContext* ctx, const Tensor& x, const Tensor& res, const OptTensor& w_, double eps) {
     ctx->set_materialize_grads(false);
     const Tensor w = val(w_);
-    NormOut o = rmsnorm_fwd(dense(x), w, eps, in_shape(res, x.sizes(), "res"));
+    NormOut o = op::rmsnorm_fwd(dense(x), w, eps, in_shape(res, x.sizes(), "res"));
     ctx->save_for_backward({o.s, o.inv, w});
     keep<at::DimVector>(ctx) = dims(res);
     return {o.s, o.y};
@@ -296,7 +278,7 @@ struct BlockHead : Function<BlockHead> {
     TORCH_CHECK_TYPE(!skip_ || l3, "a skip needs its gain l3");
     auto one = [](const Tensor& t) { return t.reshape(1).to(F32); };
     const Tensor g1 = one(l1), gains = at::cat({g1, one(l2), skip.defined() ? one(*l3) : g1});   // (the third is unused without a skip)
-    auto [x_new, x_norm, inv] = block_head_fwd(x, x0, gains, skip, eps);
+    auto [x_new, x_norm, inv] = op::block_head_fwd(x, x0, gains, skip, eps);
     ctx->save_for_backward({x, x0, skip, x_new, inv, gains});
     keep<S>(ctx) = {skip.defined(), dims(l1), dims(l2), skip.defined() ? dims(*l3) : at::DimVector(), dims(x0_),
                     skip.defined() ? dims(*skip_) : at::DimVector()};
@@ -306,7 +288,7 @@ struct BlockHead : Function<BlockHead> {
     const auto s = ctx->get_saved_variables();
     const S& st = kept<S>(ctx);
     const Tensor gn = g[1].defined() ? dense(g[1]) : at::zeros_like(s[0]);
-    HeadGrad h = block_head_bwd(dense(g[0]), gn, s[0], s[1], s[3], s[4], s[5], s[2]);
+    HeadGrad h = op::block_head_bwd(dense(g[0]), gn, s[0], s[1], s[3], s[4], s[5], s[2]);
     auto gain = [&](int i, const at::DimVector& shape) { return h.dgains.narrow(0, i, 1).view(shape); };
     return {h.dx, back_in_shape(h.dx0, st.x0), gain(0, st.l1), gain(1, st.l2), back_in_shape(h.dskip, st.skip),
             st.has_skip ? gain(2, st.l3) : Tensor(), Tensor()};
@@ -322,7 +304,7 @@ struct MixTail : Function<MixTail> {
   static Vars forward(AutogradContext* ctx, const Tensor& x_, const Tensor& lam, int64_t T) {
     ctx->set_materialize_grads(false);
     const Tensor x = dense(x_), lam32 = lam.reshape(1).to(F32);
-    auto [s1, xn2, inv] = mix_tail_fwd(x, lam32, T, std::ldexp(1.0, -23));
+    auto [s1, xn2, inv] = op::mix_tail_fwd(x, lam32, T, std::ldexp(1.0, -23));
     ctx->save_for_backward({x, s1, inv, lam32});
     keep<S>(ctx) = {T, dims(lam), lam.scalar_type()};
     return {s1, xn2};
@@ -331,7 +313,7 @@ struct MixTail : Function<MixTail> {
     if (!g[0].defined() && !g[1].defined()) return {Tensor(), Tensor(), Tensor()};
     const auto s = ctx->get_saved_variables();
     const S& st = kept<S>(ctx);
-    auto [gx, dlam] = mix_tail_bwd(s[1], s[2], s[0], s[3], st.T, dense(g[1]), dense(g[0]));
+    auto [gx, dlam] = op::mix_tail_bwd(s[1], s[2], s[0], s[3], st.T, dense(g[1]), dense(g[0]));
     return {gx, dlam.to(st.dt).view(st.shape), Tensor()};
   }
 };
@@ -340,9 +322,9 @@ struct Relu2 : Function<Relu2> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x_) {
     const Tensor x = dense(x_);
     ctx->save_for_backward({x});
-    return relu2(x, {}, 0);
+    return op::relu2(x);
   }
-  static Vars backward(AutogradContext* ctx, Vars g) { return {relu2(ctx->get_saved_variables()[0], dense(g[0]), 1)}; }
+  static Vars backward(AutogradContext* ctx, Vars g) { return {op::relu2_bwd(ctx->get_saved_variables()[0], dense(g[0]))}; }
 };
 
 // ------------------------------------------------------------------------------------------------------ projections
@@ -357,10 +339,10 @@ struct Linear : Function<Linear> {
     TORCH_CHECK_VALUE(w.dim() == 2 && last_dim(x) == w.size(1), "inner dimensions differ: ", x.size(-1), " vs ", w.size(1));
     Tensor y;
     if (res) {   // bf16(res + bf16(x @ w^T)): the residual add made in the GEMM's store (nki_attn_nr8.py:1003)
-      y = matmul_res(x, w, in_shape(*res, with_last(x, w.size(0)), "res"), true);
+      y = op::matmul_res(x, w, in_shape(*res, with_last(x, w.size(0)), "res"), true);
     } else {
       y = make(with_last(x, w.size(0)), BF16, x);
-      gemm(x, w, y, x.numel() / w.size(1), w.size(0), w.size(1), false, true, false);
+      op::gemm(x, w, y, x.numel() / w.size(1), w.size(0), w.size(1), false, true, false);
     }
     ctx->save_for_backward({x, w});
     keep<S>(ctx) = {res.has_value(), res ? dims(*res) : at::DimVector()};
@@ -372,7 +354,7 @@ struct Linear : Function<Linear> {
     const int64_t N = w.size(0), K = w.size(1), M = x.numel() / K;
     chk(gy);
     Tensor dx = make_like(x);
-    gemm(gy, w, dx, M, K, N, false, false, false);
+    op::gemm(gy, w, dx, M, K, N, false, false, false);
     const S& st = kept<S>(ctx);
     return {dx, weight_grad(w, gy, x, M, N, K), st.has_res ? back_in_shape(g[0], st.res) : Tensor()};
   }
@@ -400,18 +382,15 @@ struct Linear8 : Function<Linear8> {
     st.state = PyRef(state);
     st.has_res = res.has_value();
     if (res) st.res = dims(*res);
-    const float* dqw = static_cast<const float*>(ptr(sc)) + 1;
-    const float* dqa = nullptr;
     Tensor x8;
     if (!x_scale) {
-      st.sx = amax_scale(x, float_attr(state, n.limit), -24, 40);
-      x8 = quant_fp8(x, ptr(st.sx), 0, E4M3);
-      dqa = static_cast<const float*>(ptr(st.sx)) + 1;
+      st.sx = op::amax_scale(x, float_attr(state, n.limit), -24, 40);
+      x8 = op::quant_fp8(x, st.sx, 0, E4M3);
     } else {
-      x8 = x8_ ? in_shape(*x8_, x.sizes(), "x8") : quant_fp8(x, nullptr, *x_scale, E4M3);
+      x8 = x8_ ? in_shape(*x8_, x.sizes(), "x8") : op::quant_fp8(x, {}, *x_scale, E4M3);
       st.imm = 1.0 / *x_scale;
     }
-    Tensor y = gemm_fp8(x8, w8, E4M3, dqa, dqw, st.imm, r, with_last(x, w.size(0)));
+    Tensor y = op::gemm_fp8(x8, w8, E4M3, st.sx, sc, st.imm, r, with_last(x, w.size(0)));
     ctx->save_for_backward({dw8 ? x8 : x, w});
     return y;
   }
@@ -426,14 +405,13 @@ struct Linear8 : Function<Linear8> {
       sc = tensor_attr(st.state.o, names().sc), w8t = tensor_attr(st.state.o, names().w8t), dw8 = bool_attr(st.state.o, names().dw_fp8);
     }
     const int64_t N = w.size(0), K = w.size(1), M = xa.numel() / K;
-    const Tensor sg = amax_scale(gy, 57344.0 / 2.0, -40, 60);
-    const float* psg = static_cast<const float*>(ptr(sg));
-    const Tensor g8 = quant_fp8(gy, psg, 0, E5M2);
-    Tensor dx = gemm_fp8(g8, w8t, E5M2, psg + 1, static_cast<const float*>(ptr(sc)) + 1, 1.0, {}, xa.sizes());
+    const Tensor sg = op::amax_scale(gy, 57344.0 / 2.0, -40, 60);
+    const Tensor g8 = op::quant_fp8(gy, sg, 0, E5M2);
+    Tensor dx = op::gemm_fp8(g8, w8t, E5M2, sg, sc, 1.0, {}, xa.sizes());
     Tensor dw;
     if (dw8) {
       GradBuf gb = accumulate_into(w);
-      dw = gemm_fp8_tn(g8, xa, E5M2, E4M3, psg, ptr(st.sx), st.imm, gb.buf, gb.accumulate, BF16);
+      dw = op::gemm_fp8_tn(g8, xa, E5M2, E4M3, sg, st.sx, st.imm, gb.buf, gb.accumulate, BF16);
       if (gb.buf.defined()) dw = Tensor();
     } else {
       dw = weight_grad(w, gy, xa, M, N, K);
@@ -455,7 +433,7 @@ struct Attention : Function<Attention> {
   };
   static Tensor forward(AutogradContext* ctx, const Tensor& q_, const Tensor& k_, const Tensor& v_, double scale, int64_t band) {
     const Tensor q = dense(q_), k = dense(k_), v = dense(v_);
-    auto [o, lse] = attention(q, k, v, scale, false, band);
+    auto [o, lse] = op::attention(q, k, v, scale, band);
     ctx->save_for_backward({q, k, v, o, lse});
     keep<S>(ctx) = {scale, band};
     return o;
@@ -467,7 +445,7 @@ struct Attention : Function<Attention> {
     check_grad(go, o.numel());
     // gradients in the inputs' own (contiguous [B, H, T, D]) layout: autograd keeps them as they are
     Tensor dq = make_like(q), dk = make_like(k), dv = make_like(v);
-    attention_bwd(q, k, v, o, go.view(o.sizes()), s[4], st.scale, false, dq, dk, dv, false, {}, {}, st.band);
+    op::attention_bwd(q, k, v, o, go.view(o.sizes()), s[4], st.scale, dq, dk, dv, st.band);
     return {dq, dk, dv, Tensor(), Tensor()};
   }
 };
@@ -476,8 +454,7 @@ struct QkvDims {
   int64_t B, T, C, H, D;
   double scale;
   int64_t band = 0;
-  View third(const Tensor& t, int i, int64_t row) const { return tfb::third(t, i, T, C, D, row); }
-  View whole(const Tensor& t) const { return tfb::whole(t, T, H, D); }
+  op::Third third(const Tensor& t, int i, int64_t row) const { return {t, i, row, B, H, T, D}; }
 };
 QkvDims qkv_dims(const Tensor& qkv, int64_t n_head, double scale, int64_t band = 0) {
   TORCH_CHECK_TYPE(qkv.is_cuda() && qkv.scalar_type() == BF16, "attention takes bf16 device tensors");
@@ -492,9 +469,9 @@ struct RopeAttention : Function<RopeAttention> {
     const QkvDims m = qkv_dims(qkv, n_head, scale);
     const int64_t rows = m.B * m.T;
     const Tensor rot = make({m.B, m.T, 2 * m.C}, BF16, qkv);
-    rope(qkv, cos, sin, rot, rows, m.T, 2 * m.H, m.D, 3 * m.C, 2 * m.C, false);
+    op::rope(qkv, cos, sin, rot, rows, m.T, 2 * m.H, m.D, 3 * m.C, 2 * m.C, false);
     Tensor o = make({m.B, m.T, m.C}, BF16, qkv), lse = make({m.B, m.H, m.T}, F32, qkv);
-    attn_fwd(m.third(rot, 0, 2 * m.C), m.third(rot, 1, 2 * m.C), m.third(qkv, 2, 3 * m.C), o, lse, m.B, m.H, m.T, m.D, scale, 0);
+    op::attn_fwd(m.third(rot, 0, 2 * m.C), m.third(rot, 1, 2 * m.C), m.third(qkv, 2, 3 * m.C), o, lse, scale, 0);
     ctx->save_for_backward({qkv, rot, o, lse, cos, sin});
     keep<QkvDims>(ctx) = m;
     return o;
@@ -507,9 +484,9 @@ struct RopeAttention : Function<RopeAttention> {
     const int64_t R = 3 * m.C;
     Tensor dqkv = make_like(qkv);
     const bool fused = m.D == 64;   // the inverse rotation of dq, dk rides the backward kernels' stores
-    attn_bwd(m.third(rot, 0, 2 * m.C), m.third(rot, 1, 2 * m.C), m.third(qkv, 2, R), m.whole(s[2]), m.whole(go), m.third(dqkv, 0, R),
-             m.third(dqkv, 1, R), m.third(dqkv, 2, R), s[3], fused ? cos : Tensor(), fused ? sin : Tensor(), m.B, m.H, m.T, m.D, m.scale, 0);
-    if (!fused) rope(dqkv, cos, sin, dqkv, m.B * m.T, m.T, 2 * m.H, m.D, R, R, true);
+    op::attn_bwd(m.third(rot, 0, 2 * m.C), m.third(rot, 1, 2 * m.C), m.third(qkv, 2, R), s[2], go, m.third(dqkv, 0, R),
+             m.third(dqkv, 1, R), m.third(dqkv, 2, R), s[3], fused ? cos : Tensor(), fused ? sin : Tensor(), m.scale, 0);
+    if (!fused) op::rope(dqkv, cos, sin, dqkv, m.B * m.T, m.T, 2 * m.H, m.D, R, R, true);
     return {dqkv, Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
@@ -521,7 +498,7 @@ struct RopeNorm : Function<RopeNorm> {
     TORCH_CHECK_VALUE(x.dim() == 4, "x is [B, T, H, D]");
     const int64_t T = x.size(1), H = x.size(2), D = x.size(3), rows = x.size(0) * T;
     Tensor y = make_like(x), r = make_like(x), inv = make({rows, H}, F32, x);
-    rope_norm_fwd(x, cos, sin, r, y, inv, rows, T, H, D, H * D, eps);
+    op::rope_norm_fwd(x, cos, sin, r, y, inv, rows, T, H, D, H * D, eps);
     ctx->save_for_backward({r, inv, cos, sin});
     return y;
   }
@@ -530,7 +507,7 @@ struct RopeNorm : Function<RopeNorm> {
     const Tensor gy = dense(g[0]), &r = s[0];
     const int64_t T = r.size(1), H = r.size(2), D = r.size(3);
     Tensor dx = make_like(r);
-    rope_norm_bwd(gy, r, s[1], s[2], s[3], dx, r.size(0) * T, T, H, D, H * D, H * D);
+    op::rope_norm_bwd(gy, r, s[1], s[2], s[3], dx, r.size(0) * T, T, H, D, H * D, H * D);
     return {dx, Tensor(), Tensor(), Tensor()};
   }
 };
@@ -541,10 +518,10 @@ struct RopeNormAttention : Function<RopeNormAttention> {
     const Tensor qkv = dense(qkv_);
     const QkvDims m = qkv_dims(qkv, n_head, scale, band);
     const int64_t rows = m.B * m.T, R = 2 * m.C;
-    const Tensor qk = make({rows, R}, BF16, qkv), r = make({rows, R}, BF16, qkv), inv = make({rows, 2 * m.H}, F32, qkv);
-    rope_norm_fwd(qkv, cos, sin, r, qk, inv, rows, m.T, 2 * m.H, m.D, 3 * m.C, eps);
+    Tensor qk = make({rows, R}, BF16, qkv), r = make({rows, R}, BF16, qkv), inv = make({rows, 2 * m.H}, F32, qkv);
+    op::rope_norm_fwd(qkv, cos, sin, r, qk, inv, rows, m.T, 2 * m.H, m.D, 3 * m.C, eps);
     Tensor o = heads ? make({m.B, m.T, m.H, m.D}, BF16, qkv) : make({m.B, m.T, m.C}, BF16, qkv), lse = make({m.B, m.H, m.T}, F32, qkv);
-    attn_fwd(m.third(qk, 0, R), m.third(qk, 1, R), m.third(qkv, 2, 3 * m.C), o, lse, m.B, m.H, m.T, m.D, scale, band);
+    op::attn_fwd(m.third(qk, 0, R), m.third(qk, 1, R), m.third(qkv, 2, 3 * m.C), o, lse, scale, band);
     ctx->save_for_backward({qkv, qk, r, inv, o, lse, cos, sin});
     keep<QkvDims>(ctx) = m;
     return o;
@@ -556,9 +533,9 @@ struct RopeNormAttention : Function<RopeNormAttention> {
     check_grad(go, s[4].numel());
     const int64_t R = 2 * m.C, F = 3 * m.C;
     Tensor dqkv = make_like(qkv);
-    attn_bwd(m.third(qk, 0, R), m.third(qk, 1, R), m.third(qkv, 2, F), m.whole(s[4]), m.whole(go), m.third(dqkv, 0, F), m.third(dqkv, 1, F),
-             m.third(dqkv, 2, F), s[5], {}, {}, m.B, m.H, m.T, m.D, m.scale, m.band);
-    rope_norm_bwd(dqkv, s[2], s[3], s[6], s[7], dqkv, m.B * m.T, m.T, 2 * m.H, m.D, F, F);   // in place on the q and k thirds
+    op::attn_bwd(m.third(qk, 0, R), m.third(qk, 1, R), m.third(qkv, 2, F), s[4], go, m.third(dqkv, 0, F), m.third(dqkv, 1, F),
+             m.third(dqkv, 2, F), s[5], {}, {}, m.scale, m.band);
+    op::rope_norm_bwd(dqkv, s[2], s[3], s[6], s[7], dqkv, m.B * m.T, m.T, 2 * m.H, m.D, F, F);   // in place on the q and k thirds
     return {dqkv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
@@ -570,11 +547,11 @@ struct QkvRopeAttention : Function<QkvRopeAttention> {
     chk(x), chk(w);
     TORCH_CHECK_VALUE(x.dim() == 3 && w.dim() == 2 && x.size(2) == w.size(1), "x is [B, T, in], w [3C, in]");
     const int64_t B = x.size(0), T = x.size(1), C = w.size(0) / 3;
-    const Tensor qkv = qkv_rope(x, w, cos, sin, T, 2 * C);
+    const Tensor qkv = op::qkv_rope(x, w, cos, sin, T, 2 * C);
     const QkvDims m = qkv_dims(qkv, n_head, scale);
     Tensor o = make({B, T, C}, BF16, x), lse = make({B, m.H, T}, F32, x);
     const int64_t R = 3 * C;
-    attn_fwd(m.third(qkv, 0, R), m.third(qkv, 1, R), m.third(qkv, 2, R), o, lse, B, m.H, T, m.D, scale, 0);
+    op::attn_fwd(m.third(qkv, 0, R), m.third(qkv, 1, R), m.third(qkv, 2, R), o, lse, scale, 0);
     ctx->save_for_backward({x, w, qkv, o, lse, cos, sin});
     keep<QkvDims>(ctx) = m;
     return o;
@@ -586,10 +563,10 @@ struct QkvRopeAttention : Function<QkvRopeAttention> {
     check_grad(go, s[3].numel());
     const int64_t R = 3 * m.C, K = w.size(1), M = m.B * m.T;
     const Tensor dqkv = make_like(qkv);
-    attn_bwd(m.third(qkv, 0, R), m.third(qkv, 1, R), m.third(qkv, 2, R), m.whole(s[3]), m.whole(go), m.third(dqkv, 0, R), m.third(dqkv, 1, R),
-             m.third(dqkv, 2, R), s[4], s[5], s[6], m.B, m.H, m.T, m.D, m.scale, 0);
+    op::attn_bwd(m.third(qkv, 0, R), m.third(qkv, 1, R), m.third(qkv, 2, R), s[3], go, m.third(dqkv, 0, R), m.third(dqkv, 1, R),
+             m.third(dqkv, 2, R), s[4], s[5], s[6], m.scale, 0);
     Tensor dx = make_like(x);
-    gemm(dqkv, w, dx, M, K, R, false, false, false);
+    op::gemm(dqkv, w, dx, M, K, R, false, false, false);
     return {dx, weight_grad(w, dqkv, x, M, R, K), Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
@@ -617,29 +594,29 @@ MlpGrads mlp8_backward(const Mlp8Attrs& st, const Tensor& gy_in, const Tensor& g
   const int64_t F = w_fc.size(0), d = w_fc.size(1), M = r.size(0);
   MlpGrads o;
   if (st.dw_fp8) {
-    MlpBwd b = mlp8_bwd_q(gy, r, st.w8, rowb, st.limit, false);
+    MlpBwd b = op::mlp8_bwd_q(gy, r, st.w8, rowb, st.limit, false);
     GradBuf bf, bp;
     if (buffers) bf = accumulate_into(w_fc), bp = accumulate_into(w_proj);
     TORCH_CHECK(bf.buf.defined() == bp.buf.defined() && bf.accumulate == bp.accumulate,
                 "the fp8 weight gradients write both MLP weights' gradient buffers in one call");
     const bool in_place = bf.buf.defined();
     o.dw_fc = bf.buf, o.dw_proj = bp.buf;
-    mlp8_dw8(xa, b.dp8, b.hq8, b.dy8, rowb, st.x_scale, o.dw_fc, o.dw_proj, bf.accumulate, BF16);
+    op::mlp8_dw8(xa, b.dp8, b.hq8, b.dy8, rowb, st.x_scale, o.dw_fc, o.dw_proj, bf.accumulate, BF16);
     if (in_place) o.dw_fc = o.dw_proj = Tensor();
     o.dx = b.dx;
     return o;
   }
-  MlpBwd b = mlp8_bwd(gy, r, st.w8, rowb, false, true);
+  MlpBwd b = op::mlp8_bwd(gy, r, st.w8, rowb, false, true);
   o.dx = b.dx;
   if (!buffers) {
     o.dw_fc = make({F, d}, BF16, gy);
-    gemm(b.dpre, xa, o.dw_fc, F, d, M, true, false, false);
-    o.dw_proj = mlp_dw_proj(b.dyp, r, {}, false, BF16);
+    op::gemm(b.dpre, xa, o.dw_fc, F, d, M, true, false, false);
+    o.dw_proj = op::mlp_dw_proj(b.dyp, r, {}, false, BF16);
     return o;
   }
   o.dw_fc = weight_grad(w_fc, b.dpre, xa, M, F, d);
   GradBuf gp = accumulate_into(w_proj);
-  o.dw_proj = mlp_dw_proj(b.dyp, r, gp.buf, gp.accumulate, BF16);
+  o.dw_proj = op::mlp_dw_proj(b.dyp, r, gp.buf, gp.accumulate, BF16);
   if (gp.buf.defined()) o.dw_proj = Tensor();
   return o;
 }
@@ -656,7 +633,7 @@ struct Mlp8 : Function<Mlp8> {
     const Tensor x8 = x8_ ? in_shape(*x8_, x_.sizes(), "x8") : Tensor(), res = res_ ? in_shape(*res_, x_.sizes(), "res") : Tensor();
     // with the bytes given and the weight gradients in fp8 nothing reads x itself (it may be a storage-less placeholder)
     const Tensor x = x8.defined() && st.dw_fp8 ? Tensor() : dense(x_);
-    MlpFwd f = mlp8_fwd(x, st.w8, st.row, w_fc.size(0), st.x_scale, x8, res, !st.dw_fp8);
+    MlpFwd f = op::mlp8_fwd(x, st.w8, st.row, w_fc.size(0), st.x_scale, x8, res, !st.dw_fp8);
     ctx->save_for_backward({st.dw_fp8 ? f.x8 : f.xp.defined() ? f.xp : x, f.r, w_fc, w_proj});
     S& s = keep<S>(ctx);
     s.state = PyRef(state), s.has_res = res_.has_value();
@@ -681,8 +658,8 @@ struct NrMlp : Function<NrMlp> {
     const Mlp8Attrs st = mlp8_attrs(state);
     const Tensor x = dense(x_);
     // (with the weight gradients in fp8 too nothing reads the norm's bf16 rows: only its e4m3 bytes are written)
-    NormOut n = rmsnorm_fwd_q(x, {}, eps, {}, st.x_scale.host(), !st.dw_fp8, tile_rows(x.numel() / last_dim(x)));
-    MlpFwd f = mlp8_fwd(n.y, st.w8, st.row, w_fc.size(0), st.x_scale, n.y8, x);
+    NormOut n = op::rmsnorm_fwd_q(x, {}, eps, {}, st.x_scale.host(), !st.dw_fp8, tile_rows(x.numel() / last_dim(x)));
+    MlpFwd f = op::mlp8_fwd(n.y, st.w8, st.row, w_fc.size(0), st.x_scale, n.y8, x);
     ctx->save_for_backward({x, st.dw_fp8 ? n.y8 : n.y, n.inv, f.r, w_fc, w_proj});
     keep<PyRef>(ctx) = PyRef(state);
     return f.y;
@@ -696,7 +673,7 @@ struct NrMlp : Function<NrMlp> {
     }
     const Tensor gy = dense(g[0]);
     MlpGrads m = mlp8_backward(st, g[0], gy, s[1], s[3], s[4], s[5], false);
-    NormGrad n = rmsnorm_bwd(m.dx, s[0], s[2], {}, gy, {}, false, {}, true);
+    NormGrad n = op::rmsnorm_bwd(m.dx, s[0], s[2], {}, gy, {}, false, {}, true);
     attach(n.dx, n.amax);   // for the block before this one, whose backward receives this as its dy
     return {n.dx, m.dw_fc, m.dw_proj, Tensor(), Tensor()};
   }
@@ -705,7 +682,7 @@ struct NrMlp : Function<NrMlp> {
 struct MlpFused : Function<MlpFused> {
   static Tensor forward(AutogradContext* ctx, const Tensor& x_, const Tensor& w_fc, const Tensor& w_proj) {
     const Tensor x = dense(x_);
-    auto [y, r] = mlp_fwd(x, w_fc, w_proj);
+    auto [y, r] = op::mlp_fwd(x, w_fc, w_proj);
     ctx->save_for_backward({x, r, w_fc, w_proj});
     return y;
   }
@@ -713,7 +690,7 @@ struct MlpFused : Function<MlpFused> {
     const auto s = ctx->get_saved_variables();
     const Tensor gy = dense(g[0]);
     const int64_t F = s[2].size(0), d = s[2].size(1), M = s[1].size(0);
-    MlpBwd b = mlp_bwd(gy, s[1], s[2], s[3], true);
+    MlpBwd b = op::mlp_bwd(gy, s[1], s[2], s[3], true);
     Tensor dw_fc = weight_grad(s[2], b.dpre, s[0], M, F, d);   // dpre^T x
     return {b.dx, dw_fc, weight_grad(s[3], gy, b.h, M, d, F)};   // dy^T h
   }
@@ -749,20 +726,20 @@ struct Moe : Function<Moe> {
     TORCH_CHECK_VALUE(last_dim(h) == d && wr.size(1) == d && wr.size(0) == E, "h [.., d], router [E, d], w_fc [E, F, d]");
     S& s = keep<S>(ctx);
     s.aux = aux_weights, s.topk = topk;
-    MoeRoute rt = moe_route(h, wr, topk, val(bias), !aux_weights.empty());
-    s.tab = moe_tables(rt.idx, E, h.dim() >= 2 ? h.size(-2) : -1, capacity);
+    MoeRoute rt = op::moe_route(h, wr, topk, val(bias), !aux_weights.empty());
+    s.tab = op::moe_tables(rt.idx, E, h.dim() >= 2 ? h.size(-2) : -1, capacity);
     Tensor xs, xs8, ys, r;
     if (state) {
       s.state = PyRef(state);
       const Attrs a = attrs(state);
-      std::tie(xs, xs8) = moe_gather(h, s.tab, &a.x_scale, !a.dw_fp8);
-      std::tie(ys, r) = moe_mlp8_fwd(xs8, a.w8, a.rows, s.tab, F);
+      std::tie(xs, xs8) = op::moe_gather(h, s.tab, &a.x_scale, !a.dw_fp8);
+      std::tie(ys, r) = op::moe_mlp8_fwd(xs8, a.w8, a.rows, s.tab, F);
       if (!a.dw_fp8) xs8 = Tensor();   // only the fp8 weight gradient reads the bytes again
     } else {
-      std::tie(xs, xs8) = moe_gather(h, s.tab, nullptr, true);
-      std::tie(ys, r, std::ignore) = moe_mlp_fwd(xs, bf(w_fc), bf(w_proj), s.tab);
+      std::tie(xs, xs8) = op::moe_gather(h, s.tab, nullptr, true);
+      std::tie(ys, r) = op::moe_mlp_fwd(xs, bf(w_fc), bf(w_proj), s.tab);
     }
-    Tensor out = moe_combine(ys, s.tab, rt.gate, h.sizes());
+    Tensor out = op::moe_combine(ys, s.tab, rt.gate, h.sizes());
     if (info) {
       const Tensor share = s.tab.cnt.sum().to(F32) / double(rt.idx.numel());
       PyObject* k = THPVariable_Wrap(share);
@@ -773,14 +750,14 @@ struct Moe : Function<Moe> {
       ctx->save_for_backward({h, wr, rt.p, rt.idx, rt.gate, xs, xs8, ys, r, router, w_fc, w_proj});
       return {out};
     }
-    auto [terms, lse] = moe_aux_fwd(rt.p, rt.logits, s.tab, topk);
+    auto [terms, lse] = op::moe_aux_fwd(rt.p, rt.logits, s.tab, topk);
     Tensor aux = terms.select(0, 0) * aux_weights[0] + terms.select(0, 1) * aux_weights[1];
     Tensor fs;
     if (aux_weights.size() > 2 && aux_weights[2] != 0.0) {
       TORCH_CHECK_VALUE(h.dim() >= 3, "MoeMlp8Fn: the per-sequence balance term needs h [b, t, d]");
       s.seq_len = h.size(-2);
       Tensor term;
-      std::tie(term, fs) = moe_aux_seq_fwd(rt.p, rt.idx, s.seq_len, topk);
+      std::tie(term, fs) = op::moe_aux_seq_fwd(rt.p, rt.idx, s.seq_len, topk);
       aux = aux + term.select(0, 0) * aux_weights[2];
     }
     ctx->save_for_backward({h, wr, rt.p, rt.idx, rt.gate, xs, xs8, ys, r, router, w_fc, w_proj, terms, lse, fs});
@@ -806,14 +783,14 @@ struct Moe : Function<Moe> {
       pybind11::gil_scoped_acquire gil;
       a = attrs(s.state.o);
     }
-    CombineGrad c = moe_combine_bwd(gout, ys, s.tab, gate, s.state.o != nullptr, !a.dw_fp8);
+    CombineGrad c = op::moe_combine_bwd(gout, ys, s.tab, gate, s.state.o != nullptr, !a.dw_fp8);
     Tensor rows_b;
     MlpBwd m;
     if (s.state.o) {   // the experts' amax(dys) rides the kernel that writes dys
-      rows_b = moe_backward_scales_rowmax(c.rowmax, a.rows, s.tab, ys.size(1));
-      m = a.dw_fp8 ? moe_mlp8_bwd_q(moe_quant_dout(gout, gate, rows_b, s.tab), r, a.w8, rows_b, s.tab, a.limit) : moe_mlp8_bwd(c.dys, r, a.w8, rows_b, s.tab);
+      rows_b = op::moe_backward_scales_rowmax(c.rowmax, a.rows, s.tab, ys.size(1));
+      m = a.dw_fp8 ? op::moe_mlp8_bwd_q(c.dys, gout, gate, r, a.w8, rows_b, s.tab, a.limit) : op::moe_mlp8_bwd(c.dys, r, a.w8, rows_b, s.tab);
     } else {
-      m = moe_mlp_bwd(c.dys, r, bf(w_fc), bf(w_proj), s.tab);
+      m = op::moe_mlp_bwd(c.dys, r, bf(w_fc), bf(w_proj), s.tab);
     }
     // one grouped launch writes both gradients: both weights carry a gradient buffer (in the same state) or neither does; the
     // "fresh" flags are only touched on the branch that really writes the buffers
@@ -827,12 +804,12 @@ struct Moe : Function<Moe> {
     }
     Tensor dw_fc = bf_.buf, dw_proj = bp.buf;
     if (a.dw_fp8)
-      moe_dw8(xs8, m.dp8, m.hq8, m.dy8, rows_b, a.x_scale.host(), s.tab, dw_fc, dw_proj, E, bf_.accumulate, BF16);
+      op::moe_dw8(xs8, m.dp8, m.hq8, m.dy8, rows_b, a.x_scale.host(), s.tab, dw_fc, dw_proj, E, bf_.accumulate, BF16);
     else
-      moe_dw(m.dpre, xs, c.dys, r, s.tab, dw_fc, dw_proj, E, bf_.accumulate, BF16);
+      op::moe_dw(m.dpre, xs, c.dys, r, s.tab, dw_fc, dw_proj, E, bf_.accumulate, BF16);
     if (in_place) dw_fc = dw_proj = Tensor();
     GradBuf br = accumulate_into(router, true);
-    RouteGrad rg = moe_route_bwd(c.dgate, p, idx, m.dx, s.tab, h, wr, br.buf, br.accumulate, s.aux.empty() ? nullptr : &aux);
+    RouteGrad rg = op::moe_route_bwd(c.dgate, p, idx, m.dx, s.tab, h, wr, br.buf, br.accumulate, s.aux.empty() ? nullptr : &aux);
     return {rg.dh, br.buf.defined() ? Tensor() : rg.dwr.to(router.scalar_type()), dw_fc, dw_proj, Tensor(), Tensor(), Tensor(), Tensor(),
             Tensor(), Tensor()};
   }
@@ -854,21 +831,15 @@ struct LmHeadLoss : Function<LmHeadLoss> {
     chk(x), chk(W);
     const int64_t d = last_dim(x), M = x.numel() / d, V = W.size(0);
     TORCH_CHECK_VALUE(W.dim() == 2 && W.size(1) == d && tg.numel() == M, "x [.., d], W [V, d], one target a row");
-    const Tensor w = loss_row_weights(tg, mean, V);
+    const Tensor w = op::loss_row_weights(tg, mean, V);
     keep<S>(ctx) = {one_pass, false, softcap, M, d, V};
     if (one_pass) {
       Tensor dl = make({M, V}, BF16, x);
-      gemm(x, W, dl, M, V, d, false, true, false);
+      op::gemm(x, W, dl, M, V, d, false, true, false);
       ctx->save_for_backward({x, W, dl});
-      if (PyObject* fn = replaced("loss_fwd_bwd")) {
-        PyObject* r = call_python(fn, {THPVariable_Wrap(dl), THPVariable_Wrap(tg), THPVariable_Wrap(w), PyFloat_FromDouble(softcap)});
-        const Tensor rows = tensor_of(PySequence_GetItem(r, 0));
-        Py_DECREF(r);
-        return rows.sum();
-      }
-      return std::get<0>(loss_fwd_bwd(dl, tg, w, softcap, M, V)).sum();
+      return std::get<0>(op::loss_fwd_bwd(dl, tg, w, softcap, M, V)).sum();
     }
-    auto [logits, rows, lse] = lmhead_fwd(x, W, tg, softcap, w);
+    auto [logits, rows, lse] = op::lmhead_fwd(x, W, tg, softcap, w);
     ctx->save_for_backward({x, W, tg, logits, lse, w});
     return rows.sum();
   }
@@ -884,14 +855,13 @@ struct LmHeadLoss : Function<LmHeadLoss> {
       TORCH_CHECK(!k.consumed, "LmHeadLossFn: second backward through the same node (retain_graph): the saved logits were overwritten by "
                                "their gradient in the first one");
       k.consumed = true;
-      dl = s[3];
-      loss_bwd(dl, s[2], s[4], s[5] * g[0].to(F32), dl, k.softcap, k.M, k.V);
+      dl = op::loss_bwd(s[3], s[2], s[4], s[5] * g[0].to(F32), true, k.softcap, k.M, k.V);
     }
     Tensor dx = make_like(x);
-    gemm(dl, W, dx, k.M, k.d, k.V, false, false, false, alpha);
+    op::gemm(dl, W, dx, k.M, k.d, k.V, false, false, false, alpha);
     GradBuf gb = accumulate_into(W);
     Tensor dw = gb.buf.defined() ? gb.buf : make({k.V, k.d}, BF16, x);
-    gemm(dl, x, dw, k.V, k.d, k.M, true, false, gb.accumulate, alpha);
+    op::gemm(dl, x, dw, k.V, k.d, k.M, true, false, gb.accumulate, alpha);
     return {dx, gb.buf.defined() ? Tensor() : dw, Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
@@ -904,17 +874,15 @@ struct FusedLoss : Function<FusedLoss> {
     const Tensor tg = targets_of(targets);
     const int64_t V = last_dim(logits), N = logits.numel() / V;
     TORCH_CHECK_VALUE(tg.numel() == N, "one target a row");
-    auto [rows, lse] = loss_fwd(logits, tg, {}, softcap, N, V);
+    auto [rows, lse] = op::loss_fwd(logits, tg, {}, softcap, N, V);
     ctx->save_for_backward({logits, tg, lse});
     keep<S>(ctx) = {softcap};
     return rows;
   }
   static Vars backward(AutogradContext* ctx, Vars g) {
     const auto s = ctx->get_saved_variables();
-    Tensor out = make_like(s[0]);
-    const int64_t V = last_dim(out);
-    loss_bwd(s[0], s[1], s[2], dense(g[0].to(F32)), out, kept<S>(ctx).softcap, out.numel() / V, V);
-    return {out, Tensor(), Tensor()};
+    const int64_t V = last_dim(s[0]);
+    return {op::loss_bwd(s[0], s[1], s[2], dense(g[0].to(F32)), false, kept<S>(ctx).softcap, s[0].numel() / V, V), Tensor(), Tensor()};
   }
 };
 
@@ -927,37 +895,130 @@ struct ReducedLoss : Function<ReducedLoss> {
     const Tensor logits = dense(logits_), tg = targets_of(targets);
     const int64_t V = last_dim(logits), N = logits.numel() / V;
     TORCH_CHECK_VALUE(tg.numel() == N, "one target a row");
-    const Tensor w = loss_row_weights(tg, mean, V);
-    auto [rows, lse] = loss_fwd(logits, tg, w, softcap, N, V);
+    const Tensor w = op::loss_row_weights(tg, mean, V);
+    auto [rows, lse] = op::loss_fwd(logits, tg, w, softcap, N, V);
     ctx->save_for_backward({logits, tg, lse, w});
     keep<S>(ctx) = {softcap};
     return rows.sum();
   }
   static Vars backward(AutogradContext* ctx, Vars g) {
     const auto s = ctx->get_saved_variables();
-    Tensor out = make_like(s[0]);
-    const int64_t V = last_dim(out);
-    loss_bwd(s[0], s[1], s[2], s[3] * g[0].to(F32), out, kept<S>(ctx).softcap, out.numel() / V, V);
-    return {out, Tensor(), Tensor(), Tensor()};
+    const int64_t V = last_dim(s[0]);
+    return {op::loss_bwd(s[0], s[1], s[2], s[3] * g[0].to(F32), false, kept<S>(ctx).softcap, s[0].numel() / V, V), Tensor(), Tensor(), Tensor()};
   }
 };
 
 struct Embedding : Function<Embedding> {
   static Tensor forward(AutogradContext* ctx, const Tensor& idx, const Tensor& w) {
     ctx->save_for_backward({idx, w});
-    return embedding_fwd(idx, w);
+    return op::embedding_fwd(idx, w);
   }
   static Vars backward(AutogradContext* ctx, Vars g) {
     const auto s = ctx->get_saved_variables();
     GradBuf gb = accumulate_into(s[1], true);
     Tensor dw = gb.buf.defined() ? gb.buf.view(s[1].sizes()) : make(s[1].sizes(), F32, s[1]);
-    if (!gb.accumulate) fill_f32(dw, 0.0);
-    embedding_bwd(s[0], dense(g[0]), dw);
+    if (!gb.accumulate) op::fill_f32(dw, 0.0);
+    op::embedding_bwd(s[0], dense(g[0]), dw);
     return {Tensor(), gb.buf.defined() ? Tensor() : dw.to(s[1].scalar_type())};
   }
 };
 
 }  // namespace
+
+// ------------------------------------------------------------------------------------- replaced ops (see wrapped.hpp)
+bool any_replaced = false;
+
+namespace {
+PyObject* replaced_dict() {   // name -> function, kept by ops.py
+  static PyObject* d = PyObject_GetAttrString(PyImport_ImportModule("trainium_frontier_them_bones_amd._lib"), "REPLACED");
+  return d;
+}
+[[noreturn]] void throw_python() {
+  python_error e;
+  e.persist();
+  throw e;
+}
+}  // namespace
+
+PyObject* replaced_fn(const char* name) { return PyDict_GetItemString(replaced_dict(), name); }
+
+std::vector<Tensor> call_replaced(PyObject* fn, PyObject* args) {
+  PyRef a(args, PyRef::Steal{});
+  PyRef r(PyObject_CallObject(fn, args), PyRef::Steal{});
+  if (!r.o) throw_python();
+  std::vector<Tensor> v;
+  auto add = [&](PyObject* o) { v.push_back(THPVariable_Check(o) ? THPVariable_Unpack(o) : Tensor()); };
+  if (PyTuple_Check(r.o))
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(r.o); ++i) add(PyTuple_GET_ITEM(r.o, i));
+  else
+    add(r.o);
+  return v;
+}
+
+PyObject* to_dict(const MoeTab& t) {
+  PyObject* d = PyDict_New();
+  auto put = [&](const char* key, PyObject* v) {
+    PyDict_SetItemString(d, key, v);
+    Py_DECREF(v);
+  };
+  for (const auto& [key, v] : {std::pair<const char*, const Tensor&>{"cnt", t.cnt}, {"seg", t.seg}, {"tile_expert", t.tile_expert},
+                               {"slot", t.slot}, {"tok", t.tok}, {"ksel", t.ksel}})
+    put(key, THPVariable_Wrap(v));
+  put("rmax", PyLong_FromLongLong(t.rmax));
+  if (t.capped) put("cnt_all", THPVariable_Wrap(t.cnt_all)), put("capacity", PyLong_FromLongLong(t.capacity));
+  return d;
+}
+MoeTab from_dict(PyObject* d) {
+  TORCH_CHECK_TYPE(PyDict_Check(d), "the slot tables are a dict");
+  auto get = [&](const char* key) {
+    PyObject* v = PyDict_GetItemString(d, key);
+    return v && THPVariable_Check(v) ? THPVariable_Unpack(v) : Tensor();
+  };
+  MoeTab t{get("cnt"), get("seg"), get("tile_expert"), get("slot"), get("tok"), get("ksel"), get("cnt_all")};
+  for (const Tensor* x : {&t.cnt, &t.seg, &t.tile_expert, &t.slot, &t.tok, &t.ksel}) {
+    TORCH_CHECK_TYPE(x->defined(), "the slot tables are incomplete");
+    chk(*x, I32);
+  }
+  t.rmax = t.tok.numel();
+  if (PyObject* c = PyDict_GetItemString(d, "capacity")) t.capped = true, t.capacity = PyLong_AsLongLong(c);
+  return t;
+}
+
+namespace wrapped {
+
+PyObject* py(const Tensor& t) {
+  if (!t.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(t);
+}
+PyObject* py(const Scale& s) { return s.dev.defined() ? py(s.dev) : py(s.imm); }
+PyObject* py(at::ScalarType dt) {
+  static PyObject* torch = PyImport_ImportModule("torch");
+  return PyObject_GetAttrString(torch, dt == F32 ? "float32" : "bfloat16");
+}
+PyObject* py(const Rope& r) { return r.cos.defined() ? Py_BuildValue("(NN)", py(r.cos), py(r.sin)) : py(None{}); }
+PyObject* py(const Aux& x) {
+  if (!x.p) return py(None{});
+  const MoeAux& a = *x.p;
+  if (!a.fs.defined()) return Py_BuildValue("(NNNdd)", py(a.terms), py(a.lse), py(a.gaux), a.alpha, a.beta);
+  return Py_BuildValue("(NNNddNdL)", py(a.terms), py(a.lse), py(a.gaux), a.alpha, a.beta, py(a.fs), a.gamma, static_cast<long long>(a.seq_len));
+}
+
+MoeTab moe_tables(const Tensor& idx, int64_t E, int64_t seq_len, int64_t capacity) {
+  if (C10_UNLIKELY(any_replaced)) {
+    pybind11::gil_scoped_acquire gil;
+    if (PyObject* fn = replaced_fn("moe_tables")) {
+      const bool capped = capacity >= 0;
+      PyRef a(Py_BuildValue("(NLNN)", py(idx), static_cast<long long>(E), capped ? py(seq_len) : py(None{}), capped ? py(capacity) : py(None{})),
+              PyRef::Steal{});
+      PyRef r(PyObject_CallObject(fn, a.o), PyRef::Steal{});
+      if (!r.o) throw_python();
+      return from_dict(r.o);
+    }
+  }
+  return tfb::moe_tables(idx, E, seq_len, capacity);
+}
+
+}  // namespace wrapped
 
 void attach_amax(const Tensor& t, PyObject* amax) {
   PyObject* o = THPVariable_Wrap(t);

@@ -592,7 +592,7 @@ MoeTab moe_tables(const Tensor& idx, int64_t E, int64_t seq_len, int64_t capacit
   t.rmax = tfb_moe_max_rows(N, E, topk);
   t.cnt = make({E}, I32, idx), t.seg = make({E + 1}, I32, idx), t.tile_expert = make({t.rmax / 128}, I32, idx);
   t.slot = make({N, topk}, I32, idx), t.tok = make({t.rmax}, I32, idx), t.ksel = make({t.rmax}, I32, idx);
-  t.capped = capacity >= 0;
+  t.capped = capacity >= 0, t.capacity = capacity;
   if (!t.capped) {
     const Tensor scr = make({nw * E}, I32, idx);
     TFB_CALL(tfb_moe_tables, ptr(idx), ptr(t.cnt), ptr(t.seg), ptr(t.tile_expert), ptr(t.slot), ptr(t.tok), ptr(t.ksel), ptr(scr), N, E, topk,

@@ -113,7 +113,7 @@ std::tuple<Tensor, Tensor, Tensor> lmhead_fwd(const Tensor& x, const Tensor& W, 
 // mixture of experts
 struct MoeTab {
   Tensor cnt, seg, tile_expert, slot, tok, ksel, cnt_all;
-  int64_t rmax = 0;
+  int64_t rmax = 0, capacity = 0;
   bool capped = false;
 };
 struct MoeRoute { Tensor p, idx, gate, logits; };

@@ -3,6 +3,9 @@ short fixed sequence of launches) per call on torch's current stream. No autogra
 autograd.py) and no fallbacks: every function requires CUDA(ROCm) tensors and the built
 library. torch supplies device memory and the stream; all arithmetic is in the HIP kernels.
 """
+import sys
+import types
+
 import torch
 
 from . import _lib
@@ -58,10 +61,12 @@ def rmsnorm_fwd(x, weight=None, eps=2.0 ** -23, res=None):
     return native.tfb_rmsnorm_fwd(x, weight, eps, res)
 
 
-def rmsnorm_fwd_q(x, weight=None, eps=2.0 ** -23, res=None, y8_scale=4.0, want_y=True):
+def rmsnorm_fwd_q(x, weight=None, eps=2.0 ** -23, res=None, y8_scale=4.0, want_y=True, rows_out=0):
     """rmsnorm_fwd that also returns y8 = e4m3(bf16(y) * y8_scale) bytes, the operand cast of the fp8 GEMM that consumes y
     (equal to quant_fp8(y, y8_scale), bit for bit). Returns (s, y, inv, y8); want_y False: the bf16 rows are not written and
-    y is None (for a consumer that reads only the bytes)."""
+    y is None (for a consumer that reads only the bytes). rows_out: y and y8 get that many rows, those beyond x's zero."""
+    if rows_out:
+        return native.tfb_rmsnorm_fwd_q_pad(x, weight, eps, res, y8_scale, want_y, rows_out)
     return native.tfb_rmsnorm_fwd_q(x, weight, eps, res, y8_scale, want_y)
 
 
@@ -407,10 +412,6 @@ def loss_fwd_bwd(logits2, targets, row_w=None, softcap=15.0):
     return native.tfb_loss_fwd_bwd(logits2, targets, row_w, softcap)
 
 
-# The functions a program may wrap by assigning to this module's name: the native nodes call what stands there.
-_WRAPPABLE = {"mlp8_backward_scales": mlp8_backward_scales, "loss_fwd_bwd": loss_fwd_bwd}
-
-
 def loss_multi_fwd(logits2, targets, row_w, softcap=15.0, eps=0.0):
     """Row losses sum_k row_w[k] (lse - (1 - eps) s_{t_k} - eps mean_v s_v) and lse; targets [K, N] (int64 / int32, < 0 =
     weight 0), row_w fp32 [K, N]."""
@@ -647,3 +648,23 @@ def mix_tail_fwd(x2, lam, T, eps=2.0 ** -23):
 def mix_tail_bwd(s1, inv, x2, lam, T, gy=None, ge=None):
     """(gx bf16 [rows,C], dlam fp32 [1]) from the gradients gy of xn2 and ge of s1 (either may be None) (R1:7145)."""
     return native.tfb_mix_tail_bwd(s1, inv, x2, lam, T, gy, ge)
+
+
+# ------------------------------------------------------------------------------------------ replaced functions
+# A program may put a function of its own in the place of any function here (ops.<name> = f, monkeypatch.setattr, ...): the
+# autograd nodes then call that one. The native layer looks for it only while there is one.
+_OWN = {name: fn for name, fn in list(globals().items()) if isinstance(fn, types.FunctionType) and not name.startswith("_")}
+
+
+class _Module(types.ModuleType):
+    def __setattr__(self, name, value):
+        super().__setattr__(name, value)
+        own = _OWN.get(name)
+        if own is not None:
+            _lib.REPLACED.pop(name, None)
+            if value is not own:
+                _lib.REPLACED[name] = value
+            native.told()
+
+
+sys.modules[__name__].__class__ = _Module
