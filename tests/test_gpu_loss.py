@@ -127,3 +127,22 @@ def test_the_switch_for_the_one_pass_loss_head(dev, monkeypatch):
     assert abs(one - two) < 1e-6 * one
     for a, b in zip(grads1, grads2):
         assert (a.float() - b.float()).norm() < 5e-3 * b.float().norm()
+
+
+@pytest.mark.parametrize("cap", [0.5, 7.0, 15.0, 30.0, 50.0])
+def test_tanh_has_the_bits_of_an_ieee_division(dev, cap):
+    """The gradient factor 1 - tanh^2 of every bf16 bit pattern, each the target of a row of its own, with the kernels'
+    reciprocal and with a division in the same fp32 expressions (NaN where the logit is one)."""
+    from trainium_frontier_them_bones_amd import ops
+    x = torch.arange(65536, dtype=torch.int32, device=dev).to(torch.int16).view(bf16)
+    z = torch.zeros(65536, 8, dtype=bf16, device=dev)
+    z[:, 3] = x
+    t = torch.full((65536,), 3, device=dev)
+    lse = torch.full((65536,), cap + 200.0, device=dev)              # no softmax left: -1 at the target, 0 elsewhere
+    got = ops.loss_bwd(z, t, lse, torch.ones(65536, device=dev), cap)
+    y = x.float() * (1.0 / torch.tensor(cap, device=dev))
+    th = 1.0 - 2.0 / (torch.exp2(y * 2.8853900817779268) + 1.0)
+    want = (-(1.0 - th * th)).to(bf16)
+    nan = x.isnan()
+    assert bool(got[nan, 3].isnan().all()) and torch.equal(got[~nan, 3], want[~nan])
+    assert not bool(got[~nan][:, [0, 1, 2, 4, 5, 6, 7]].any())

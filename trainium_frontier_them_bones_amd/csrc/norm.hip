@@ -453,7 +453,7 @@ __global__ __launch_bounds__(256) void mix_tail_fwd_kernel(const bf16_t* __restr
 // dlam partial [gridDim.x] = sum over the workgroup's rows of the bf16 products bf16(g[t] x[t - 1]) in fp32.
 // Bound by memory: each group of lanes takes a run of rows from its last to its first, so that g[t + 1] is what it has just
 // made and only one row a run is made twice, and requests the next row before it works on this one. 32000 x 768: 81 us with
-// every g made twice from its three rows, DT with runs of eight.
+// every g made twice from its three rows, 45 in runs of four rows (the run is the shortest that leaves 1024 workgroups).
 template <int NCH, int G>
 __global__ __launch_bounds__(256) void mix_tail_bwd_kernel(const bf16_t* __restrict__ s, const bf16_t* __restrict__ gy,
                                                           const bf16_t* __restrict__ ge, const float* __restrict__ inv,
