@@ -54,7 +54,7 @@ def cpu_baseline_and_parity(cfg, dev):
     from oracle.model import OracleGPT
     from trainium_frontier_them_bones_amd.model import GPT, zipf_tokens
     host = os.cpu_count() or 1
-    threads = min(host, 16)            # the GPU box gives one GPU's job 16 cores, whatever os.cpu_count() shows
+    threads = min(host, 16)            # one GPU's share of its host, whatever os.cpu_count() shows
     torch.set_num_threads(threads)
     m = GPT(cfg, dev, seed=0)
     o = OracleGPT(cfg, m.init_values)

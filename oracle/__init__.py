@@ -3,7 +3,7 @@ kernels (attention, fp8 fused MLP, RMSNorm / residual blocks, loss head, AdamW, 
 model that strings them together).
 
 THIS PACKAGE IS TEST INFRASTRUCTURE. Only tests/, __graft_entry__.smoke() and bench.py's
-cpu_baseline leg may import it, and only as the checker / the timed CPU baseline. Nothing under
+cpu_baseline leg may import it, and only as the oracle of a comparison / the timed CPU baseline. Nothing under
 trainium_frontier_them_bones_amd/ imports it and the HIP path never routes through it.
 
 Every function cites the reference lines it restates (paths relative to the reference repo:

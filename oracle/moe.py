@@ -106,7 +106,7 @@ def moe_forward(h, router, w_fc, w_proj, topk, bias=None, fp8=True, e4m3_limit=2
     fp8 False: the experts in bf16, the kit's expression per expert (round2/source/train.py:10716 moe_experts_local).
     dys_amax (optional, fp32 [E]): per-expert amax of the expert outputs' gradients to take the backward scales from,
     for a call that holds only some of the layer's tokens. idx (optional, [N, k]): selections to use instead of the
-    oracle's own (a checker passes the kernel's, so that a near-tie cannot route a token differently); the gates are
+    oracle's own (a test passes the kernel's, so that a near-tie cannot route a token differently); the gates are
     still this function's, from its own probabilities at those experts."""
     d = h.shape[-1]
     h2 = h.reshape(-1, d)

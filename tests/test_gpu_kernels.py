@@ -560,7 +560,7 @@ def test_mlp8_refresh_of_all_layers_equals_per_layer_calls(ops, dev):
 
 
 def test_mlp8_full_size_properties(ops, dev):
-    """configuration 3 of BASELINE.json sizes: exact equivariance under a permutation of the tokens and agreement of 512-row slices
+    """sizes of the benchmark's configuration 3: exact equivariance under a permutation of the tokens and agreement of 512-row slices
     with the oracle."""
     from oracle import mlp8 as O
     M, d, F = 16384, 768, 3072
@@ -733,7 +733,7 @@ def test_fp8_projection_weight_stationary_kernel_equals_the_tiled_kernel(ops, de
 
 @pytest.mark.parametrize("shape", [(512, 256, 512), (16384, 768, 3072)])
 def test_mlp8_as_the_benchmark_times_it(ops, dev, shape):
-    """Configuration 3 of BASELINE.json in the form bench.py times: OCP e4m3 at 448, the activation scale from the tensor's
+    """Configuration 3 of the benchmark in the form bench.py times: OCP e4m3 at 448, the activation scale from the tensor's
     amax (a power of two, left on the device), all six GEMMs in fp8 (weight gradients from the bytes the other GEMMs
     multiplied), through the autograd wrapper. Against the oracle with the same limit and the same activation scale:
     y and dx on two 512-row slices (2e-2), both weight gradients over all rows (2e-2)."""
@@ -945,7 +945,7 @@ def test_attention_strided_qkv_and_rejects(ops, dev):
 
 
 def test_attention_full_size_properties(ops, dev):
-    """configuration 2 of BASELINE.json (B16 H12 T2048 D64, RoPE'd q and k): two (b, h) pairs against the oracle, causality by
+    """configuration 2 of the benchmark (B16 H12 T2048 D64, RoPE'd q and k): two (b, h) pairs against the oracle, causality by
     perturbing the future, and dV with dO = 1 equal to the column sums of P."""
     from oracle import attention as O
     B, H, T, D = 16, 12, 2048, 64
@@ -1069,7 +1069,7 @@ def test_loss_fwd_bwd(ops, dev, cap):
 
 
 def test_lmhead_config1(ops, dev):
-    """configuration 1 of BASELINE.json at full size through the autograd layer: RMSNorm -> LM-head GEMM (+lse) -> CE, fwd + bwd."""
+    """configuration 1 of the benchmark at full size through the autograd layer: RMSNorm -> LM-head GEMM (+lse) -> CE, fwd + bwd."""
     from oracle import loss as O
     from trainium_frontier_them_bones_amd import autograd as A
     g = _g(20261)

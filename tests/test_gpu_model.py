@@ -64,7 +64,7 @@ def test_each_half_block_against_the_oracle_on_its_own_inputs(dev):
 
 
 def test_full_size_model_on_one_sequence_against_the_oracle(dev):
-    """Configuration 4 of BASELINE.json at its real model size (12 layers, d 768, 12 heads, MLP 3072, vocab 32768) on ONE
+    """Configuration 4 of the benchmark at its real model size (12 layers, d 768, 12 heads, MLP 3072, vocab 32768) on ONE
     sequence of 2048 tokens: the loss of the first step and, after one AdamW update of every parameter, of the second,
     against the oracle model on the same tokens, within 1e-3 relative."""
     from oracle.model import OracleGPT
@@ -118,7 +118,7 @@ def test_gradient_accumulation_in_place(dev):
 
 
 def test_full_size_batch_first_loss_against_the_oracle(dev):
-    """Configuration 4 of BASELINE.json at its stated batch (16 sequences of 2048 tokens): the loss of the first forward pass
+    """Configuration 4 of the benchmark at its stated batch (16 sequences of 2048 tokens): the loss of the first forward pass
     against the mean of the oracle's sixteen per-sequence forward losses (equal lengths, no ignored target: the batch mean),
     within 1e-3 relative."""
     from oracle.model import OracleGPT

@@ -1,4 +1,4 @@
-"""MoE layer on the HIP kernels against the oracle (configuration 5 of BASELINE.json shapes in the last test)."""
+"""MoE layer on the HIP kernels against the oracle (the shapes of the benchmark's configuration 5 in the last test)."""
 import pytest
 import torch
 
