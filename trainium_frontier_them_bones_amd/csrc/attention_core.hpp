@@ -33,8 +33,11 @@ __device__ __forceinline__ float max_halves(float x) {  // the larger of the two
 
 // Workgroup -> (block along the sequence, batch*head): consecutive workgroup ids are dealt round-robin to the 8 XCDs, each with its own
 // L2, so the ids are re-dealt to keep all sequence blocks of one (batch, head) - which stream the same K/V (or Q/dO) tiles - on one
-// XCD; with one block per workgroup (gridDim.x = nx) in slot-major order, the heaviest block of each pair first. nx = blocks per
-// (batch, head), nbh = batch*head count.
+// XCD. With one block per workgroup (gridDim.x = nx) the order is slot-major, the heaviest block of each pair first: workgroups start in
+// id order, and the causal blocks differ in work by a factor of nx. That order matters more than the XCD: where the pairs are no
+// multiple of 8 and cannot be dealt to the XCDs evenly, it is kept without that (pair by pair in order, the last pairs' heavy blocks
+// ran on alone; T2048 D64 12 heads B3 forward 57 -> 34 us, backward 165 -> 96; B7 103 -> 73, 297 -> 195; T3072 D128 6 heads B2
+// 64 -> 52, 230 -> 174). nx = blocks per (batch, head), nbh = batch*head count.
 __device__ __forceinline__ void xcd_block(int nx, int nbh, int& bx, int& bh) {
   const int gx = gridDim.x, lin = blockIdx.y * gx + blockIdx.x;
   if (nbh % 8 == 0) {
@@ -47,6 +50,9 @@ __device__ __forceinline__ void xcd_block(int nx, int nbh, int& bx, int& bh) {
       bh = xcd + 8 * (idx / gx);
       bx = idx % gx;
     }
+  } else if (gx == nx) {
+    bx = lin / nbh;
+    bh = lin - bx * nbh;
   } else {
     bh = blockIdx.y;
     bx = blockIdx.x;
