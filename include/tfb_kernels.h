@@ -37,6 +37,13 @@ int tfb_gemm_bf16_scaled(const void* A, const void* B, void* C, int M, int N, in
  * The bf16 form of _proj8_fwd_ra_kernel (round2/source/kernels/nki_attn_nr8.py:1003: out = bf16(res + bf16(acc dq))). */
 int tfb_gemm_bf16_res(const void* A, const void* B, const void* res, void* C, int M, int N, int K, int trans_b, void* stream);
 
+/* The two gradients of y [M][N] = x [M][K] @ w [N][K]^T in one launch: dx [M][K] = dy @ w and dw [N][K] (+)= dy^T @ x (bf16 or fp32,
+ * optionally accumulated into), each equal bit for bit to its tfb_gemm_bf16 call with a workspace of workspace_bytes (it fixes the
+ * order of the sums; none is used). For calls of few rows: status 1 for M rows that it does not take, which _applies tells without a launch (0 / 1). */
+int tfb_linear_bwd_applies(int M, int N, int K, long workspace_bytes);
+int tfb_linear_bwd(const void* dy, const void* x, const void* w, void* dx, void* dw, int M, int N, int K, int dw_f32, int dw_accumulate,
+                   long workspace_bytes, void* stream);
+
 /* ---- RMSNorm family --------------------------------------------------------------------------------------------
  * Number of partial-sum rows the backward kernels write for `nrows` rows (host helper, no GPU work). */
 int tfb_norm_bwd_blocks(long nrows);
@@ -236,6 +243,13 @@ int tfb_mlp8_bwd_q(const void* dy8, const void* r, const void* w8, const void* r
 int tfb_mlp8_dw8(const void* x8, const void* dp8, const void* hq8, const void* dy8, const void* row, float x_scale, void* dw_fc,
                  void* dw_proj, long M, int d, int F, int out_f32, int accumulate, void* workspace, long workspace_bytes,
                  const void* x_scale_dev, void* stream);
+/* tfb_mlp8_bwd_q (h and dpre NULL) followed by tfb_mlp8_dw8, bit for bit, with dx and the two weight gradients as jobs of one launch.
+ * For calls of few rows: status 1 for M rows that it does not take, which _applies tells without a launch (0 / 1). workspace_bytes: of the workspace
+ * that the two calls would be given (it fixes the order of their sums); none is used. */
+int tfb_mlp8_bwd_dw8_applies(long M, int d, int F, long workspace_bytes);
+int tfb_mlp8_bwd_dw8(const void* dy8, const void* r, const void* w8, const void* row, void* dx, void* dp8, void* hq8, float hq_limit,
+                     const void* x8, float x_scale, const void* x_scale_dev, void* dw_fc, void* dw_proj, long M, int d, int F, int out_f32,
+                     int accumulate, long workspace_bytes, void* stream);
 
 /* ---- fp8 projections (attention QKV / output projection in fp8) -----------------------------------------------------
  * out8 [R][C], outT8 [C][R] = e4m3(w [R][C] * *scale_ptr): a weight pre-cast once per optimizer step in both byte layouts.

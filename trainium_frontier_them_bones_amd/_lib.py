@@ -19,6 +19,8 @@ _fp = ctypes.POINTER(ctypes.c_float)   # a HOST array of floats (tfb_ns5's coeff
 # name -> argtypes (restype is always int status unless listed in _RESTYPE)
 SIGNATURES = {
     "tfb_gemm_bf16": [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _l, _vp],
+    "tfb_linear_bwd_applies": [_i, _i, _i, _l],
+    "tfb_linear_bwd": [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _l, _vp],
     "tfb_gemm_bf16_scaled": [_vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp, _l, _vp, _vp],
     "tfb_gemm_bf16_res": [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     "tfb_norm_bwd_blocks": [_l],
@@ -45,6 +47,8 @@ SIGNATURES = {
     "tfb_mlp8_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _l, _i, _i, _vp],
     "tfb_mlp8_bwd_q": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _f, _l, _i, _i, _vp],
     "tfb_gemm_fp8_tn": [_vp, _i, _vp, _i, _vp, _vp, _f, _vp, _l, _i, _i, _i, _i, _vp, _l, _vp],
+    "tfb_mlp8_bwd_dw8_applies": [_l, _i, _i, _l],
+    "tfb_mlp8_bwd_dw8": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _f, _vp, _f, _vp, _vp, _vp, _l, _i, _i, _i, _i, _l, _vp],
     "tfb_mlp8_dw8": [_vp, _vp, _vp, _vp, _vp, _f, _vp, _vp, _l, _i, _i, _i, _i, _vp, _l, _vp, _vp],
     "tfb_attn_fwd": [_vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _i, _i, _i, _i, _f, _vp],
     "tfb_attn_fwd_band": [_vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _i, _i, _i, _i, _f, _i, _vp],

@@ -179,10 +179,10 @@ __device__ __forceinline__ void ring_wait(int tiles) {
 #undef TFB_RING_WAIT
 }
 
+// Workgroup `block` of the launch: one output tile.
 template <class Cfg, bool RANGES, class Epi>
-__global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi epi_in) {
+__device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, int block, uint8_t* lds) {
   constexpr int BP = Cfg::BP, BQ = Cfg::BQ, NW = Cfg::NW, TP = Cfg::TP, TQ = Cfg::TQ, ES = Cfg::ES, NS = Cfg::NS;
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[Cfg::LDS_BYTES];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wp = wave % Cfg::WP, wq = wave / Cfg::WP;
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
   if constexpr (is_symmetric<Epi>::value) {
     static_assert(BP == BQ, "square tiles");
     // an XCD's workgroups (id & 7) take a run of consecutive tiles, so that a group's operand is read into one or two L2s only
-    lid = (blockIdx.x & 7) * a.per + (blockIdx.x >> 3);
+    lid = (block & 7) * a.per + (block >> 3);
     split = 0;
     sym_group = fastdiv(lid, a.d_ntiles);
     if (sym_group >= a.rows) return;   // (the whole workgroup: the runs are of equal length)
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
     for (; tile_p >= a.ntp - tile_q; ++tile_q) tile_p -= a.ntp - tile_q;   // row tile_q has ntp - tile_q tiles
     tile_p += tile_q;
   } else {
-    gemm_tile_of(a, blockIdx.x, lid, split, tile_p, tile_q);
+    gemm_tile_of(a, block, lid, split, tile_p, tile_q);
   }
   const long p0 = (long)tile_p * BP, q0 = (long)tile_q * BQ;
   int kt0 = 0;
@@ -361,10 +361,12 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
     if (t + 1 < nkt) step(1, t + 1, std::false_type{});
   }
   if constexpr (RANGES) {
+    if (range > 1) {
 #pragma unroll
-    for (int i = 0; i < TP; ++i)
+      for (int i = 0; i < TP; ++i)
 #pragma unroll
-      for (int j = 0; j < TQ; ++j) acc[i][j] = total[i][j] + acc[i][j];
+        for (int j = 0; j < TQ; ++j) acc[i][j] = total[i][j] + acc[i][j];
+    }
   }
   __syncthreads();
 
@@ -429,9 +431,15 @@ __global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi e
   }
 }
 
+template <class Cfg, bool RANGES, class Epi>
+__global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_kernel(GemmArgs a, Epi epi_in) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[Cfg::LDS_BYTES];
+  gemm_ring_tile<Cfg, RANGES>(a, epi_in, blockIdx.x, lds);
+}
+
 // ranges > 1: the k ranges summed inside the workgroup (at most nkt of them; not with a k_seg)
-template <class Cfg, class Epi>
-static int gemm_ring_launch_args(GemmArgs a, int groups_y, int splits, int ranges, Epi epi, hipStream_t stream) {
+template <class Cfg>
+static int gemm_ring_args(GemmArgs& a, int splits, int ranges) {
   const int st = gemm_map_args<Cfg>(a, splits);
   if (st != TFB_OK) return st;
   a.slots = 0;
@@ -439,6 +447,12 @@ static int gemm_ring_launch_args(GemmArgs a, int groups_y, int splits, int range
   if (ranges > 1 && (splits > 1 || ranges > a.nkt)) return TFB_ERR_SHAPE;
   a.ranges = ranges;
   a.d_ranges = fastdiv_make(ranges);
+  return TFB_OK;
+}
+template <class Cfg, class Epi>
+static int gemm_ring_launch_args(GemmArgs a, int groups_y, int splits, int ranges, Epi epi, hipStream_t stream) {
+  const int st = gemm_ring_args<Cfg>(a, splits, ranges);
+  if (st != TFB_OK) return st;
   const dim3 grid(a.ntiles * splits, groups_y, 1);
   if constexpr (has_ranges<Epi>::value) {
     if (ranges > 1) {
@@ -547,4 +561,114 @@ static bool gemm_pp_try(GemmOperand P, GemmOperand Q, int np, int nq, long kbyte
   a.nkt = (int)(kbytes / 128);
   st = gemm_ring_launch<Epi, ES, LAYP, LAYQ, FMTP, FMTQ>(128L * np <= 4096L * tfb_resident_slots(1) ? 1 : 2, a, 1, 1, e, s, 1, main);
   return true;
+}
+
+// ---- several independent contractions in one launch ------------------------------------------------------------------
+// What bounds a ring launch is the rate at which a CU's loads go into LDS (some 100 KB a microsecond, whatever the tile or the number
+// of stages; the loads alone take 12.5 of the 13.9 us of a 2048 x 768 x 2304 launch), and a launch of fewer tiles than CUs leaves the
+// others idle for its whole length. The gradients of one layer - the input's and the weights' - are independent of each other, so they
+// run as jobs of one launch: the tiles of the second start where the first leaves room, and a launch's fixed 3 - 4 us are paid once.
+// The same tiles, the same sums as in launches of their own.
+template <int LAYP_, int LAYQ_, int ES_, int FMTP_, int FMTQ_, bool RANGES_, class Epi_>
+struct RingJob {
+  typedef Epi_ Epi;
+  static constexpr bool RANGES = RANGES_;
+  template <int BP, int NS>
+  using Cfg = RingCfg<BP, 64, 2, 2, ES_, LAYP_, LAYQ_, FMTP_, FMTQ_, NS>;
+  typedef Cfg<64, 4> Small;
+  typedef Cfg<128, 3> Large;
+  GemmArgs a = {};
+  Epi e;
+  int ranges = 1;
+  RingJob(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Epi e_, int ranges_ = 1) : e(e_), ranges(ranges_) {
+    a.P = P;
+    a.Q = Q;
+    a.np = np;
+    a.nq = nq;
+    a.nkt = (int)(kbytes / 128);
+  }
+  // whether it would go through the ring by itself
+  bool applies() const {
+    return a.np > 0 && a.nq > 0 && a.np % 128 == 0 && a.nq % 128 == 0 && gemm_ring_pick(a.np, a.nq, a.nkt, LAYP_ == TFB_K_STRIDED && LAYQ_ == TFB_K_STRIDED) != 0;
+  }
+  double bytes() const { return (double)(a.np / 128) * (a.nq / 64) * a.nkt * 24576; }   // through LDS, in tiles of 128 x 64
+};
+template <class Cfg_, class Job>
+struct RingPart {
+  typedef Cfg_ Cfg;
+  GemmArgs a;
+  typename Job::Epi e;
+  int first, blocks;   // its workgroups; a multiple of 8, so that an id keeps its XCD
+};
+struct RingNoJob {
+  typedef RingNoJob Small, Large, Epi;
+  static constexpr int LDS_BYTES = 0;
+  static constexpr bool RANGES = false;
+  GemmArgs a = {};
+  double bytes() const { return 0; }
+};
+
+template <class J, class Part>
+__device__ __forceinline__ void gemm_ring_part(const Part& p, uint8_t* lds) {
+  const int block = (int)blockIdx.x - p.first;
+  if (block >= 0 && block < p.a.ntiles) gemm_ring_tile<typename Part::Cfg, J::RANGES>(p.a, p.e, block, lds);
+}
+template <class J0, class J1, class J2, class P0, class P1, class P2>
+__global__ __launch_bounds__(256, 2) void gemm_ring_jobs_kernel(P0 p0, P1 p1, P2 p2) {
+  constexpr int B01 = P0::Cfg::LDS_BYTES > P1::Cfg::LDS_BYTES ? P0::Cfg::LDS_BYTES : P1::Cfg::LDS_BYTES;
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[B01 > P2::Cfg::LDS_BYTES ? B01 : P2::Cfg::LDS_BYTES];
+  gemm_ring_part<J0>(p0, lds);
+  gemm_ring_part<J1>(p1, lds);
+  if constexpr (!std::is_same<J2, RingNoJob>::value) gemm_ring_part<J2>(p2, lds);
+}
+
+template <class Cfg, class Job>
+static int gemm_ring_make(const Job& j, RingPart<Cfg, Job>& p, int& blocks, long& tile) {
+  p.first = p.blocks = 0;
+  if constexpr (std::is_same<Job, RingNoJob>::value) {
+    return TFB_OK;
+  } else {
+    p.a = j.a;
+    p.e = j.e;
+    p.a.ntp = j.a.np / Cfg::BP;
+    const int st = gemm_ring_args<Cfg>(p.a, 1, j.ranges);
+    p.blocks = (p.a.ntiles + 7) & ~7;
+    blocks += p.blocks;
+    tile = (long)j.a.nkt * Cfg::STAGE_BYTES;
+    return st;
+  }
+}
+template <class C0, class C1, class C2, class J0, class J1, class J2>
+static int gemm_ring_jobs_launch(const J0& j0, const J1& j1, const J2& j2, hipStream_t s) {
+  RingPart<C0, J0> p0 = {};
+  RingPart<C1, J1> p1 = {};
+  RingPart<C2, J2> p2 = {};
+  int n = 0;
+  long t0 = 0, t1 = 0, t2 = 0;   // bytes of a tile: the longest tiles start first
+  int st = gemm_ring_make(j0, p0, n, t0);
+  if (st == TFB_OK) st = gemm_ring_make(j1, p1, n, t1);
+  if (st == TFB_OK) st = gemm_ring_make(j2, p2, n, t2);
+  if (st != TFB_OK) return st;
+  p0.first = (t1 > t0 ? p1.blocks : 0) + (t2 > t0 ? p2.blocks : 0);
+  p1.first = (t0 >= t1 ? p0.blocks : 0) + (t2 > t1 ? p2.blocks : 0);
+  p2.first = (t0 >= t2 ? p0.blocks : 0) + (t1 >= t2 ? p1.blocks : 0);
+  hipLaunchKernelGGL((gemm_ring_jobs_kernel<J0, J1, J2, RingPart<C0, J0>, RingPart<C1, J1>, RingPart<C2, J2>>), dim3(n), dim3(256), 0, s, p0, p1,
+                     p2);
+  TFB_LAUNCH_CHECK();
+  return TFB_OK;
+}
+// Two jobs, or three of which the last two have the same tiles. 64 x 64 tiles for a job whose 128 x 64 tile would be longer than what a
+// CU has to do on average (the output projection's weight gradient of 2048 tokens: 72 such tiles of 32 k-tiles).
+template <class J0, class J1, class J2 = RingNoJob>
+static int gemm_ring_jobs(const J0& j0, const J1& j1, hipStream_t s, const J2& j2 = {}) {
+  const double most = 1.2 * (j0.bytes() + j1.bytes() + j2.bytes()) / tfb_resident_slots(1);
+  const bool s0 = j0.a.nkt * 24576.0 > most, s1 = j1.a.nkt * 24576.0 > most;
+  typedef typename J0::Small S0;
+  typedef typename J0::Large L0;
+  typedef typename J1::Small S1;
+  typedef typename J1::Large L1;
+  typedef typename J2::Small S2;
+  typedef typename J2::Large L2;
+  if (s0) return s1 ? gemm_ring_jobs_launch<S0, S1, S2>(j0, j1, j2, s) : gemm_ring_jobs_launch<S0, L1, L2>(j0, j1, j2, s);
+  return s1 ? gemm_ring_jobs_launch<L0, S1, S2>(j0, j1, j2, s) : gemm_ring_jobs_launch<L0, L1, L2>(j0, j1, j2, s);
 }

@@ -173,6 +173,22 @@ Tensor weight_grad(const Tensor& w, const Tensor& g, const Tensor& a, int64_t M,
   return dw;
 }
 
+// dx and the weight gradient of y = x w^T for x of M rows, w [N, K].
+std::pair<Tensor, Tensor> linear_backward(const Tensor& gy, const Tensor& x, const Tensor& w, int64_t M, int64_t N, int64_t K) {
+  Tensor dx = make_like(x);
+  if (any_replaced || !linear_bwd_applies(M, N, K)) {
+    op::gemm(gy, w, dx, M, K, N, false, false, false);
+    return {dx, weight_grad(w, gy, x, M, N, K)};
+  }
+  chk(gy), chk(x), chk(w);
+  TORCH_CHECK_VALUE(gy.numel() == M * N && x.numel() == M * K && w.numel() == N * K, "operands of ", gy.numel(), ", ", x.numel(), " and ",
+                    w.numel(), " elements for ", M, " x ", N, " x ", K);
+  GradBuf gb = accumulate_into(w);
+  const Tensor dw = gb.buf.defined() ? gb.buf : make({N, K}, BF16, gy);
+  linear_bwd(gy, x, w, dx, dw, M, N, K, gb.accumulate);
+  return {dx, gb.buf.defined() ? Tensor() : dw};
+}
+
 // The scale row of an fp8 MLP backward: from the amax partials on the gradient when they are still valid, else from a pass over
 // it.
 Tensor backward_scales(const Tensor& gy, const Tensor& g2, const Tensor& row) {
@@ -353,10 +369,9 @@ struct Linear : Function<Linear> {
     const Tensor &x = s[0], &w = s[1], gy = dense(g[0]);
     const int64_t N = w.size(0), K = w.size(1), M = x.numel() / K;
     chk(gy);
-    Tensor dx = make_like(x);
-    op::gemm(gy, w, dx, M, K, N, false, false, false);
+    auto [dx, dw] = linear_backward(gy, x, w, M, N, K);
     const S& st = kept<S>(ctx);
-    return {dx, weight_grad(w, gy, x, M, N, K), st.has_res ? back_in_shape(g[0], st.res) : Tensor()};
+    return {dx, dw, st.has_res ? back_in_shape(g[0], st.res) : Tensor()};
   }
 };
 
@@ -565,9 +580,8 @@ struct QkvRopeAttention : Function<QkvRopeAttention> {
     const Tensor dqkv = make_like(qkv);
     op::attn_bwd(m.third(qkv, 0, R), m.third(qkv, 1, R), m.third(qkv, 2, R), s[3], go, m.third(dqkv, 0, R), m.third(dqkv, 1, R),
              m.third(dqkv, 2, R), s[4], s[5], s[6], m.scale, 0);
-    Tensor dx = make_like(x);
-    op::gemm(dqkv, w, dx, M, K, R, false, false, false);
-    return {dx, weight_grad(w, dqkv, x, M, R, K), Tensor(), Tensor(), Tensor(), Tensor()};
+    auto [dx, dw] = linear_backward(dqkv, x, w, M, R, K);
+    return {dx, dw, Tensor(), Tensor(), Tensor(), Tensor()};
   }
 };
 
@@ -594,16 +608,29 @@ MlpGrads mlp8_backward(const Mlp8Attrs& st, const Tensor& gy_in, const Tensor& g
   const int64_t F = w_fc.size(0), d = w_fc.size(1), M = r.size(0);
   MlpGrads o;
   if (st.dw_fp8) {
-    MlpBwd b = op::mlp8_bwd_q(gy, r, st.w8, rowb, st.limit, false);
-    GradBuf bf, bp;
-    if (buffers) bf = accumulate_into(w_fc), bp = accumulate_into(w_proj);
-    TORCH_CHECK(bf.buf.defined() == bp.buf.defined() && bf.accumulate == bp.accumulate,
-                "the fp8 weight gradients write both MLP weights' gradient buffers in one call");
-    const bool in_place = bf.buf.defined();
-    o.dw_fc = bf.buf, o.dw_proj = bp.buf;
-    op::mlp8_dw8(xa, b.dp8, b.hq8, b.dy8, rowb, st.x_scale, o.dw_fc, o.dw_proj, bf.accumulate, BF16);
+    bool in_place = false;
+    auto outputs = [&]() -> DwOut {
+      GradBuf bf, bp;
+      if (buffers) bf = accumulate_into(w_fc), bp = accumulate_into(w_proj);
+      TORCH_CHECK(bf.buf.defined() == bp.buf.defined() && bf.accumulate == bp.accumulate,
+                  "the fp8 weight gradients write both MLP weights' gradient buffers in one call");
+      in_place = bf.buf.defined();
+      o.dw_fc = bf.buf, o.dw_proj = bp.buf;
+      return {bf.buf, bp.buf, bf.accumulate};
+    };
+    if (!any_replaced && mlp8_bwd_dw8_applies(r, d)) {
+      o.dx = mlp8_bwd_dw8(gy, r, st.w8, rowb, st.limit, xa, st.x_scale, [&]() -> DwOut {
+        DwOut w = outputs();
+        if (!in_place) w.fc = o.dw_fc = make({F, d}, BF16, gy), w.proj = o.dw_proj = make({d, F}, BF16, gy);
+        return w;
+      });
+    } else {
+      MlpBwd b = op::mlp8_bwd_q(gy, r, st.w8, rowb, st.limit, false);
+      const bool accumulate = outputs().accumulate;
+      op::mlp8_dw8(xa, b.dp8, b.hq8, b.dy8, rowb, st.x_scale, o.dw_fc, o.dw_proj, accumulate, BF16);
+      o.dx = b.dx;
+    }
     if (in_place) o.dw_fc = o.dw_proj = Tensor();
-    o.dx = b.dx;
     return o;
   }
   MlpBwd b = op::mlp8_bwd(gy, r, st.w8, rowb, false, true);

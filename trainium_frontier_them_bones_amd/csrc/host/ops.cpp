@@ -7,6 +7,8 @@ namespace tfb {
 
 namespace {
 
+constexpr int64_t WORKSPACE_BYTES = 256 << 20;   // holds the largest split any entry point asks for
+
 Tensor scratch(const Tensor& like, int64_t nfloats) { return make({nfloats}, F32, like); }
 
 void want_shape(const Tensor& t, at::IntArrayRef s, const char* what) { TORCH_CHECK_VALUE(t.sizes() == s, what); }
@@ -26,14 +28,12 @@ struct Out2 {   // a given output is checked, a missing one made
 }  // namespace
 
 Tensor workspace(const Tensor& like) {
-  // One per (device, stream): launches on different streams would otherwise race on the same partial sums. 256 MB holds the
-  // largest split any entry point asks for. Kept for the life of the process (streams are few: torch hands out a fixed pool).
-  constexpr int64_t BYTES = 256 << 20;
+  // One per (device, stream): launches on different streams would otherwise race on the same partial sums. Kept for the life of the process (streams are few: torch hands out a fixed pool).
   static std::mutex mu;
   static auto* pool = new std::map<std::pair<int, void*>, Tensor>;   // never destroyed: the device may be gone by then
   std::lock_guard<std::mutex> lock(mu);
   Tensor& ws = (*pool)[{like.get_device(), stream()}];
-  if (!ws.defined()) ws = make({BYTES / 4}, F32, like);
+  if (!ws.defined()) ws = make({WORKSPACE_BYTES / 4}, F32, like);
   return ws;
 }
 
@@ -49,6 +49,13 @@ void gemm(const Tensor& a, const Tensor& b, const Tensor& out, int64_t M, int64_
     TFB_CALL(tfb_gemm_bf16_scaled, ptr(a), ptr(b), ptr(out), M, N, K, ta, tb, f32, accumulate, ptr(ws), ws.numel() * 4, ptr(alpha), stream());
   else
     TFB_CALL(tfb_gemm_bf16, ptr(a), ptr(b), ptr(out), M, N, K, ta, tb, f32, accumulate, ptr(ws), ws.numel() * 4, stream());
+}
+
+bool linear_bwd_applies(int64_t M, int64_t N, int64_t K) { return M < INT32_MAX && tfb_linear_bwd_applies(M, N, K, WORKSPACE_BYTES) == 0; }
+
+void linear_bwd(const Tensor& gy, const Tensor& x, const Tensor& w, const Tensor& dx, const Tensor& dw, int64_t M, int64_t N, int64_t K,
+                bool accumulate) {
+  TFB_CALL(tfb_linear_bwd, ptr(gy), ptr(x), ptr(w), ptr(dx), ptr(dw), M, N, K, dw.scalar_type() == F32, accumulate, WORKSPACE_BYTES, stream());
 }
 
 Tensor matmul(const Tensor& a, const Tensor& b, bool ta, bool tb, Tensor out, bool accumulate, at::ScalarType out_dtype, const Tensor& alpha) {
@@ -315,6 +322,24 @@ MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Ten
   TFB_CALL(tfb_mlp8_bwd_q, ptr(o.dy8), ptr(r), ptr(w8), ptr(row), ptr(o.dx), nullptr, ptr(o.dpre), ptr(o.dp8), ptr(o.hq8), limit, M, d, F,
            stream());
   return o;
+}
+
+bool mlp8_bwd_dw8_applies(const Tensor& r, int64_t d) { return tfb_mlp8_bwd_dw8_applies(r.size(0), d, r.size(1), WORKSPACE_BYTES) == 0; }
+
+Tensor mlp8_bwd_dw8(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, const Tensor& x8, const Scale& x_scale,
+                    const std::function<DwOut()>& outputs) {
+  chk(dy), chk(r), chk(w8, U8), chk(row, F32), chk(x8, U8);
+  const int64_t d = last_dim(dy), M = tile_rows(dy.numel() / d), F = r.size(1);
+  check_rows(r, M, F);
+  check_pack(w8, row, d, F);
+  TORCH_CHECK_VALUE(x8.numel() == M * d && last_dim(x8) == d, "operand shapes");
+  const DwOut o = outputs();
+  TORCH_CHECK_VALUE(o.fc.numel() == F * d && o.proj.numel() == F * d && o.fc.scalar_type() == o.proj.scalar_type(), "bad outputs");
+  const Tensor dy8 = quant_rows(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2, M, nullptr);
+  const Tensor dx = make_rows(dy.sizes(), M, d, dy), dp8 = make({M, F}, U8, dy), hq8 = make({M, F}, U8, dy);
+  TFB_CALL(tfb_mlp8_bwd_dw8, ptr(dy8), ptr(r), ptr(w8), ptr(row), ptr(dx), ptr(dp8), ptr(hq8), limit, ptr(x8), x_scale.imm, ptr(x_scale.dev),
+           ptr(o.fc), ptr(o.proj), M, d, F, o.fc.scalar_type() == F32, o.accumulate, WORKSPACE_BYTES, stream());
+  return dx;
 }
 
 void mlp8_dw8(const Tensor& x8, const Tensor& dp8, const Tensor& hq8, const Tensor& dy8, const Tensor& row, const Scale& x_scale,

@@ -1,6 +1,8 @@
 // The entry points on tensors: checks, outputs and scratch from torch's allocator, one library call (or a short fixed
 // sequence) on the current stream. No autograd here. An undefined Tensor stands for "not given".
 #pragma once
+#include <functional>
+
 #include "common.hpp"
 
 namespace tfb {
@@ -8,6 +10,10 @@ namespace tfb {
 // GEMM. The explicit sizes let the callers hand over tensors of any leading shape.
 void gemm(const Tensor& a, const Tensor& b, const Tensor& out, int64_t M, int64_t N, int64_t K, bool ta, bool tb, bool accumulate,
           const Tensor& alpha = {});
+// dx = gy w and dw (+)= gy^T x in one launch, where linear_bwd_applies; bf16 operands, checked by the caller
+bool linear_bwd_applies(int64_t M, int64_t N, int64_t K);
+void linear_bwd(const Tensor& gy, const Tensor& x, const Tensor& w, const Tensor& dx, const Tensor& dw, int64_t M, int64_t N, int64_t K,
+                bool accumulate);
 Tensor matmul(const Tensor& a, const Tensor& b, bool ta, bool tb, Tensor out, bool accumulate, at::ScalarType out_dtype,
               const Tensor& alpha);
 Tensor matmul_res(const Tensor& a, const Tensor& b, const Tensor& res, bool tb);
@@ -53,6 +59,14 @@ MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F,
 struct MlpBwd { Tensor dx, h, dpre, dp8, hq8, dy8, dyp; };
 MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h, bool want_dyp = false);
 MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, bool want_dpre);
+// dx and both weight gradients at once, where mlp8_bwd_dw8_applies; outputs() is asked for the latter once the operands are checked
+struct DwOut {
+  Tensor fc, proj;
+  bool accumulate;
+};
+bool mlp8_bwd_dw8_applies(const Tensor& r, int64_t d);
+Tensor mlp8_bwd_dw8(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, const Tensor& x8, const Scale& x_scale,
+                    const std::function<DwOut()>& outputs);
 void mlp8_dw8(const Tensor& x8, const Tensor& dp8, const Tensor& hq8, const Tensor& dy8, const Tensor& row, const Scale& x_scale,
               Tensor& dw_fc, Tensor& dw_proj, bool accumulate, at::ScalarType out_dtype);
 Tensor mlp_dw_proj(const Tensor& dy, const Tensor& r, Tensor out, bool accumulate, at::ScalarType out_dtype);
