@@ -17,148 +17,14 @@
 // The tile loops are software-pipelined by hand, slot by slot: an MFMA, the LDS read of a fragment that a later slot uses, and a
 // share of the elementwise work of the neighbouring tile. What bounds them: two wavefronts per SIMD (forward, dQ: all 256 registers)
 // share the matrix pipe, which an MFMA holds for 32 cycles and a dot product (the rounded row sum) for about 16; one wavefront alone
-// on its SIMD (dK/dV with K, V and both gradients in 340 registers, and every kernel when the grid leaves CUs half empty) issues an
-// instruction every five cycles, so there the count of instructions per MFMA is the time.
-// Before, with plain loops whose LDS reads stood right in front of their MFMAs -> now: B3 H8 T1664 forward 52 -> 35 us, backward
-// 164 -> 118; B1 H8 T2048 56 -> 35, 177 -> 122; B16 H6 T2048 155 -> 120, 600 -> 475.
-#include <type_traits>
-#include "attention_core.hpp"
+// on its SIMD (when the grid leaves CUs half empty) issues an instruction every five cycles, so there the count of instructions per MFMA
+// is the time. dK/dV runs in pairs of wavefronts (attention_dkdv.hip).
+// Before, with plain loops whose LDS reads stood right in front of their MFMAs -> now: B3 H8 T1664 forward 52 -> 35 us; B1 H8 T2048
+// 56 -> 35; B16 H6 T2048 155 -> 120.
+#include "attention_slots.hpp"
 
 namespace {
 
-typedef __attribute__((address_space(1))) uint8_t glb_u8_t;
-
-template <int D>
-struct Geo {
-  static constexpr int ROWB = 2 * D;        // bytes of a token's row
-  static constexpr int TILE = 64 * ROWB;    // bytes of a 64-token tile
-  static constexpr int NKS = D / 16;        // MFMA k-steps over the head dimension
-  static constexpr int NDT = D / 32;        // 32-element tiles of the head dimension
-  static constexpr int LPT = ROWB / 16;     // lanes (16-byte chunks) per token
-  static constexpr int TPI = 64 / LPT;      // tokens per 1 KB load instruction
-  // slot swizzle: chunk c of token t at slot c ^ swz(t)
-  __device__ static __forceinline__ int swz(int t) {
-    if (D == 64) return (((t >> 1) & 1) << 2) | ((t >> 2) & 3);
-    return ((t & 3) << 2) | ((t >> 2) & 3);
-  }
-};
-
-// This wavefront's share of a (16 NI TPI / 4 ...)-token tile load: instructions g = wave + 4 i, i < NI, each TPI tokens.
-template <int D, int NI>
-struct TileLoad {
-  typedef Geo<D> G;
-  uint32_t voff;
-  int wave;
-  __device__ __forceinline__ void init(long stride, int wave_, int lane) {
-    wave = wave_;
-    const int lrow = lane / G::LPT;
-    // token = TPI g + lrow with g = wave + 4 i: the swizzle depends on g only through bits that 4 i does not touch
-    const int chunk = (lane % G::LPT) ^ G::swz(G::TPI * wave + lrow);
-    voff = (uint32_t)((G::TPI * wave + lrow) * stride + chunk * 16);
-  }
-  __device__ __forceinline__ void issue_one(int i, const uint8_t* rows, long stride, uint8_t* lds) const {
-    const glb_u8_t* r = (const glb_u8_t*)rows;
-    uint32_t o = voff;
-    asm volatile("" : "+v"(o));   // (its widening stays in this block, where the load takes it as a 32-bit offset)
-    __builtin_amdgcn_global_load_lds((glb_void_t*)(r + i * (4 * G::TPI) * stride + o), (lds_void_t*)(lds + (wave + 4 * i) * 1024), 16, 0, 0);
-  }
-  __device__ __forceinline__ void issue(const uint8_t* rows, long stride, uint8_t* lds) const {
-    const glb_u8_t* r = (const glb_u8_t*)rows;   // (uniform base + 32-bit lane offset: no 64-bit address per lane)
-#pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      __builtin_amdgcn_global_load_lds((glb_void_t*)(r + voff), (lds_void_t*)(lds + (wave + 4 * i) * 1024), 16, 0, 0);
-      r += 4 * G::TPI * stride;
-    }
-  }
-};
-
-// One token's gradient row from the NDT accumulators a lane holds (elements 32 dt + 8 j + 4 lh + i), scaled and rounded
-// once to bf16.
-template <int D>
-__device__ __forceinline__ void store_grad_row(const f32x16 (&acc)[Geo<D>::NDT], float scale, bf16_t* row, int lh) {
-#pragma unroll
-  for (int dt = 0; dt < Geo<D>::NDT; ++dt)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      u32x2 w = {pack2bf(acc[dt][4 * j] * scale, acc[dt][4 * j + 1] * scale),
-                 pack2bf(acc[dt][4 * j + 2] * scale, acc[dt][4 * j + 3] * scale)};
-      *(u32x2*)(row + 32 * dt + 8 * j + 4 * lh) = w;
-    }
-}
-
-// ------------------------------------------------------------------------------------ pipelined fragment reads
-// The tile loops below are written slot by slot: one MFMA, the LDS read of the fragment that a later slot needs, and this slot's
-// share of the elementwise work, kept in that order by sched_barrier(0). Fragments are read by inline assembly and tied to an
-// explicit s_waitcnt lgkmcnt(n) right before their MFMA: left to the compiler, each read sits in front of its MFMA and every one
-// pays the LDS latency.
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
-
-template <int I, int N, class F>
-__device__ __forceinline__ void slots(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    slots<I + 1, N>(f);
-  }
-}
-__device__ __forceinline__ void slot_end() { __builtin_amdgcn_sched_barrier(0); }
-
-// values made in this slot (they would otherwise sink to the block that uses them)
-__device__ __forceinline__ void pin(float& a, float& b) { asm volatile("" : "+v"(a), "+v"(b)); }
-template <class T>
-__device__ __forceinline__ void pin(T& a) { asm volatile("" : "+v"(a)); }
-__device__ __forceinline__ int opaque(int x) {  // (comparisons against it stay where they are used, not in registers across the loop)
-  asm volatile("" : "+v"(x));
-  return x;
-}
-struct RowFrag {  // a token-major fragment on its way: one 16-byte read
-  i32x4_t v;
-  template <int OFF>
-  __device__ __forceinline__ void request(uint32_t addr) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-  }
-  __device__ __forceinline__ bf16x8 get() const { return __builtin_bit_cast(bf16x8, v); }
-};
-struct ColFrag {  // a transposed fragment: two 8-byte reads
-  u32x2 a, b;
-  template <int OFF>
-  __device__ __forceinline__ void request(uint32_t lo, uint32_t hi) {
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(a) : "v"(lo), "n"(OFF));
-    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(b) : "v"(hi), "n"(OFF));
-  }
-  __device__ __forceinline__ bf16x8 get() const { return frag_from(a.x, a.y, b.x, b.y); }
-};
-// Two fragments are waited for together: one wavefront alone on its SIMD issues an instruction every five cycles, seven under an MFMA.
-// AFTER: LDS instructions issued since the second's.
-template <int AFTER>
-__device__ __forceinline__ void landed(RowFrag& x, RowFrag& y) {
-  asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(x.v), "+v"(y.v) : "n"(AFTER));
-}
-template <int AFTER>
-__device__ __forceinline__ void landed(ColFrag& x, ColFrag& y) {
-  asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(x.a), "+v"(x.b), "+v"(y.a), "+v"(y.b) : "n"(AFTER));
-}
-// Per-lane addresses of the fragments of a tile at `base`. Token-major, rows[s]: token lane & 31, elements 16 s + 8 (lane >> 5) .. + 7.
-// Transposed, lo[dt] and hi[dt]: element (MFMA row) 32 dt + (lane & 31), tokens 4 lh + {0..3} and 8 + 4 lh + {0..3}. A tile's place,
-// the 32-token half and the 16-token step are added, as the instruction's offset where they are constants.
-template <int D>
-struct FragAddr {
-  uint32_t rows[Geo<D>::NKS], lo[Geo<D>::NDT], hi[Geo<D>::NDT];
-  __device__ __forceinline__ void init(uint32_t base, int lane) {
-    typedef Geo<D> G;
-    const int lr = lane & 31, lh = lane >> 5, g4 = lane >> 4, j = lane & 15;
-#pragma unroll
-    for (int s = 0; s < G::NKS; ++s) rows[s] = base + lr * G::ROWB + (((2 * s + lh) ^ G::swz(lr)) << 4);
-    const int t = 4 * (g4 >> 1) + (j >> 2);
-#pragma unroll
-    for (int dt = 0; dt < G::NDT; ++dt) {
-      const int d = 32 * dt + 16 * (g4 & 1) + 4 * (j & 3);
-      lo[dt] = base + t * G::ROWB + (((d >> 3) ^ G::swz(t)) << 4) + ((d & 4) << 1);
-      hi[dt] = base + (t + 8) * G::ROWB + (((d >> 3) ^ G::swz(t + 8)) << 4) + ((d & 4) << 1);
-    }
-  }
-};
-// all of this wavefront's loads into LDS have landed, and every wavefront is here
-__device__ __forceinline__ void tile_barrier() { asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); }
 // =========================================================================================== forward
 template <int D>
 __global__ __launch_bounds__(256, 2) void attnD_fwd_kernel(AttnT q, AttnT k, AttnT v, AttnT o, float* __restrict__ lse, int T,
@@ -653,259 +519,6 @@ __global__ __launch_bounds__(256, 2) void attnD_dq_kernel(AttnT q, AttnT k, Attn
   }
 }
 
-// =========================================================================================== dK / dV
-struct StatFrag {  // 32 rows' statistics as an accumulator's start: four 16-byte reads, into the half of the register file it is in
-  f32x4 v[4];
-  template <int OFF>
-  __device__ __forceinline__ void request(uint32_t addr) {
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=a"(v[0]) : "v"(addr), "n"(OFF));
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=a"(v[1]) : "v"(addr), "n"(OFF + 32));
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=a"(v[2]) : "v"(addr), "n"(OFF + 64));
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=a"(v[3]) : "v"(addr), "n"(OFF + 96));
-  }
-  template <int AFTER>
-  __device__ __forceinline__ void landed(f32x16& x) {
-    asm volatile("s_waitcnt lgkmcnt(%4)" : "+a"(v[0]), "+a"(v[1]), "+a"(v[2]), "+a"(v[3]) : "n"(AFTER));
-#pragma unroll
-    for (int e = 0; e < 16; ++e) x[e] = v[e >> 2][e & 3];
-  }
-};
-
-template <int D>
-__global__ __launch_bounds__(256, 1) void attnD_dkdv_kernel(AttnT q, AttnT k, AttnT v, AttnT go, AttnT dk, AttnT dv,
-                                                                          const float* __restrict__ stats, long rows, int T,
-                                                                          int H, float scale, float sl2, int nw) {
-  typedef Geo<D> G;
-  constexpr int TILE = G::TILE, NKS = G::NKS, NDT = G::NDT, NI = 34;
-  constexpr int AH = 6;  // items asked for ahead of their use
-  static_assert(NKS == 8 && NDT == 4, "four phases of eight MFMAs");
-  constexpr int STAGE = 2 * TILE + 512;  // Q tile, dO tile, 64 x (-lse / scale), 64 x (-delta)
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * STAGE];
-  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int bx, bh;
-  xcd_block(T / 128, gridDim.y, bx, bh);
-  const int b = bh / H, h = bh % H;
-  const uint8_t* qp = (const uint8_t*)(q.p + b * q.sb + h * q.sh);
-  const uint8_t* gp = (const uint8_t*)(go.p + b * go.sb + h * go.sh);
-  const bf16_t* kp = k.p + b * k.sb + h * k.sh;
-  const bf16_t* vp = v.p + b * v.sb + h * v.sh;
-  const float* delp = stats + (long)bh * T;
-  const float* nlp = stats + rows + (long)bh * T;
-  const int nx = T / 128, npass = paired_passes(nx);
-  const long qst = q.st * 2, gst = go.st * 2;
-  TileLoad<D, 16 / G::TPI> lq, lg;
-  lq.init(qst, wave, lane);
-  lg.init(gst, wave, lane);
-  FragAddr<D> fa;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t*)lds;
-  fa.init(lds0, lane);
-  const uint32_t sa = lds0 + 2 * TILE + 16 * lh;
-  for (int pass = 0; pass < npass; ++pass) {
-    const int kb = paired_block(nx, bx, pass, false);  // low key blocks see the most query tiles
-    const int kw0 = kb * 128 + wave * 32, mykey = kw0 + lr;
-    // with a band the keys of tile kb are seen by the queries of tiles kb .. kb + nw - 1 only
-    const int nall = nx - kb, nt = 2 * (nw > 0 && nw < nall ? nw : nall), nh = 2 * nt;  // 64-query tiles, 32-query halves
-    // Half hh's share of the loads, five per wavefront: an odd half 2 i + 1 asks for Q and -lse / scale of tile i + 3 (whose stage tile
-    // i - 1 has left), the even half after it for that tile's dO and -delta. (All four wavefronts bring the 64 statistics.)
-    struct Part {
-      const uint8_t* p;
-      long st;
-      const float* s;
-      uint8_t* d;
-      uint8_t* ds;
-    };
-    auto part = [&](int tile, bool isq) {
-      const int tt = tile < nt ? tile : nt - 1;
-      const long r0 = (long)kb * 128 + (long)tt * 64;
-      uint8_t* d = lds + (tile & 3) * STAGE;
-      return Part{isq ? qp + r0 * qst : gp + r0 * gst, isq ? qst : gst, (isq ? nlp : delp) + r0, d + (isq ? 0 : TILE),
-                  d + 2 * TILE + (isq ? 0 : 256)};
-    };
-    auto load_one = [&](const Part& x, bool isq, int i) {
-      if (i < 4) (isq ? lq : lg).issue_one(i, x.p, x.st, x.d);
-      else __builtin_amdgcn_global_load_lds((glb_void_t*)(x.s + lane), (lds_void_t*)x.ds, 4, 0, 0);
-    };
-    auto load_part = [&](int tile, bool isq) {
-      const Part x = part(tile, isq);
-#pragma unroll
-      for (int i = 0; i < 5; ++i) load_one(x, isq, i);
-    };
-    load_part(0, true);
-    load_part(0, false);
-    load_part(1, true);
-    load_part(1, false);
-    load_part(2, true);
-    bf16x8 kf[NKS], vf[NKS];
-#pragma unroll
-    for (int s = 0; s < NKS; ++s) {
-      kf[s] = *(const bf16x8*)(kp + (long)mykey * k.st + 16 * s + 8 * lh);
-      vf[s] = *(const bf16x8*)(vp + (long)mykey * v.st + 16 * s + 8 * lh);
-    }
-    f32x16 dka[NDT], dva[NDT];
-#pragma unroll
-    for (int i = 0; i < NDT; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        dka[i][e] = 0.f;
-        dva[i][e] = 0.f;
-      }
-
-    // Half h's dS, dV += dO P and dK += Q dS are made while half h + 1's S, dP and P are. Items in the order of their LDS reads:
-    // 0 .. 7 dV, 8 the start of S, 9 .. 16 S, 17 the start of dP, 18 .. 25 dP, 26 .. 33 dK.
-    f32x16 Sn, dP;
-    uint32_t pw[8], dsw[8];
-    float f0, f1;
-    RowFrag rf[16];
-    ColFrag cf[16];
-    StatFrag sf[2];
-    auto nlds = [](int i) constexpr { return i % 34 < 8 || i % 34 >= 26 ? 2 : i % 34 == 8 || i % 34 == 17 ? 4 : 1; };
-    auto after = [=](int i) constexpr {  // LDS instructions of the items asked for since
-      int c = 0;
-      for (int x = i + (i % 34 == 8 || i % 34 == 17 ? 1 : 2); x < i + AH; ++x) c += nlds(x);
-      return c;
-    };
-    // coff, roff: half h's and half h + 1's place, soff: half h + 1's statistics
-    auto request = [&](auto item, uint32_t coff, uint32_t roff, uint32_t soff) {
-      constexpr int i = decltype(item)::value;
-      if constexpr (i < 8) cf[i].template request<TILE + (i / NDT) * 16 * G::ROWB>(fa.lo[i % NDT] + coff, fa.hi[i % NDT] + coff);
-      else if constexpr (i == 8) sf[0].template request<0>(sa + soff);
-      else if constexpr (i < 17) rf[i - 9].template request<0>(fa.rows[i - 9] + roff);
-      else if constexpr (i == 17) sf[1].template request<256>(sa + soff);
-      else if constexpr (i < 26) rf[i - 10].template request<TILE>(fa.rows[i - 18] + roff);
-      else cf[i - 18].template request<((i - 26) / NDT) * 16 * G::ROWB>(fa.lo[(i - 26) % NDT] + coff, fa.hi[(i - 26) % NDT] + coff);
-    };
-    auto use = [&](auto item, auto aft) {
-      constexpr int i = decltype(item)::value, N = decltype(aft)::value;
-      if constexpr (i < 8) {
-        constexpr int w = 4 * (i / NDT);
-        if constexpr (i % 2 == 0) landed<N>(cf[i], cf[i + 1]);
-        const bf16x8 f = cf[i].get();
-        dva[i % NDT] = mfma_bf16(f, frag_from(pw[w], pw[w + 1], pw[w + 2], pw[w + 3]), dva[i % NDT]);
-      } else if constexpr (i == 8) {
-        sf[0].template landed<N>(Sn);
-      } else if constexpr (i < 17) {
-        if constexpr (i % 2 == 1) landed<N>(rf[i - 9], rf[i - 8]);
-        Sn = mfma_bf16(rf[i - 9].get(), kf[i - 9], Sn);
-      } else if constexpr (i == 17) {
-        sf[1].template landed<N>(dP);
-      } else if constexpr (i < 26) {
-        if constexpr (i % 2 == 0) landed<N>(rf[i - 10], rf[i - 9]);
-        dP = mfma_bf16(rf[i - 10].get(), vf[i - 18], dP);
-      } else {
-        constexpr int w = 4 * ((i - 26) / NDT);
-        if constexpr (i % 2 == 0) landed<N>(cf[i - 18], cf[i - 17]);
-        const bf16x8 f = cf[i - 18].get();
-        dka[(i - 26) % NDT] = mfma_bf16(f, frag_from(dsw[w], dsw[w + 1], dsw[w + 2], dsw[w + 3]), dka[(i - 26) % NDT]);
-      }
-    };
-    auto ds_word = [&](auto word) {  // the reference multiplies dP - delta by the rounded P
-      constexpr int w = decltype(word)::value;
-      dsw[w] = pack2bf(bflo(pw[w]) * dP[2 * w], bfhi(pw[w]) * dP[2 * w + 1]);
-      pin(dsw[w]);
-    };
-    auto step_f = [&](auto word) {
-      constexpr int w = decltype(word)::value;
-      f0 = Sn[2 * w] * sl2;
-      f1 = Sn[2 * w + 1] * sl2;
-      pin(f0, f1);
-    };
-    auto step_x = [&]() {
-      f0 = fast_exp2(f0);
-      f1 = fast_exp2(f1);
-      pin(f0, f1);
-    };
-    auto step_c = [&](auto word) {
-      pw[decltype(word)::value] = pack2bf(f0, f1);
-      pin(pw[decltype(word)::value]);
-    };
-    auto place = [](int hh) -> uint32_t { return ((hh >> 1) & 3) * STAGE + (hh & 1) * (TILE / 2); };
-    auto splace = [](int hh) -> uint32_t { return ((hh >> 1) & 3) * STAGE + (hh & 1) * 128; };
-
-    // tiles 0 and 1; then the halves before this wavefront's first, which is the one on its diagonal
-    asm volatile("s_waitcnt vmcnt(5)\n\ts_barrier" ::: "memory");
-    for (int x = 0; x < wave; ++x) {
-      if (x & 1) asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory");
-      load_part((x >> 1) + ((x & 1) ? 3 : 2), x & 1);
-    }
-    {
-      const uint32_t roff = place(wave), soff = splace(wave);
-      slots<8, 8 + AH>([&](auto i) { request(i, 0u, roff, soff); });
-      slots<8, 26>([&](auto i) {
-        constexpr int x = decltype(i)::value;
-        auto aft = [=]() constexpr {
-          int c = 0;
-          for (int y = x + (x == 8 || x == 17 ? 1 : 2); y < x + AH && y < 26; ++y) c += nlds(y);
-          return c;
-        };
-        use(i, std::integral_constant<int, aft()>{});
-        if constexpr (x + AH < 26) request(std::integral_constant<int, x + AH>{}, 0u, roff, soff);
-        slot_end();
-      });
-      const int kq = lr - 4 * lh;  // key - q for element e is kq - (e>>2)*8 - (e&3)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) Sn[e] = (kq - 8 * (e >> 2) - (e & 3) > 0) ? -INFINITY : Sn[e];
-      slots<0, 8>([&](auto i) {
-        step_f(i);
-        step_x();
-        step_c(i);
-      });
-    }
-    slots<0, AH>([&](auto i) { request(i, place(wave), 0u, 0u); });
-    static_assert(AH <= 8, "only columns of the first half are asked for here");
-    for (int hh = wave; hh + 1 < nh; ++hh) {
-      const bool isq = hh & 1;
-      // tile (hh + 1) / 2 is needed from here on: all but the ten newest loads have landed
-      if (isq) asm volatile("s_waitcnt vmcnt(10)\n\ts_barrier" ::: "memory");
-      const Part ld = part((hh >> 1) + (isq ? 3 : 2), isq);
-      const uint32_t coff = place(hh), roff = place(hh + 1), soff = splace(hh + 1);
-      slot_end();
-#pragma unroll
-      for (int i = 0; i < NDT; ++i) asm volatile("" : "+a"(dka[i]), "+a"(dva[i]));
-      slots<0, NI>([&](auto i) {
-        constexpr int x = decltype(i)::value;
-        use(i, std::integral_constant<int, after(x)>{});
-        if constexpr (x + AH < NI) request(std::integral_constant<int, x + AH>{}, coff, roff, soff);
-        else request(std::integral_constant<int, x + AH - NI>{}, roff, 0u, 0u);
-        if constexpr (x % 4 == 1 && x / 4 < 5) load_one(ld, isq, x / 4);
-        if constexpr (x < 16 && x % 2 == 0) ds_word(std::integral_constant<int, x / 2>{});
-        if constexpr (x == 18) step_f(std::integral_constant<int, 0>{});
-        if constexpr (x >= 19 && x % 2 == 1) step_x();
-        if constexpr (x >= 20 && x % 2 == 0) {
-          step_c(std::integral_constant<int, (x - 20) / 2>{});
-          step_f(std::integral_constant<int, (x - 18) / 2>{});
-        }
-        slot_end();
-      });
-      step_c(std::integral_constant<int, 7>{});
-    }
-    {  // the last half
-      const uint32_t coff = place(nh - 1);
-      slots<0, 8>([&](auto i) {
-        constexpr int x = decltype(i)::value;
-        use(i, std::integral_constant<int, 2 * (AH - 2)>{});
-        if constexpr (x + AH < 8) request(std::integral_constant<int, x + AH>{}, coff, 0u, 0u);
-        else request(std::integral_constant<int, x + AH + 18>{}, coff, 0u, 0u);
-        ds_word(i);
-        slot_end();
-      });
-      slots<26, NI>([&](auto i) {
-        constexpr int x = decltype(i)::value;
-        use(i, std::integral_constant<int, x % 2 ? 0 : 2 * (x + AH <= NI ? AH - 2 : NI - 2 - x)>{});
-        if constexpr (x + AH < NI) request(std::integral_constant<int, x + AH>{}, coff, 0u, 0u);
-        slot_end();
-      });
-    }
-
-    bf16_t* dkp = dk.p + b * dk.sb + h * dk.sh + (long)mykey * dk.st;
-    bf16_t* dvp = dv.p + b * dv.sb + h * dv.sh + (long)mykey * dv.st;
-    store_grad_row<D>(dka, scale, dkp, lh);
-    store_grad_row<D>(dva, 1.0f, dvp, lh);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (pass + 1 < npass) __syncthreads();  // the stages are free for the partner block
-  }
-}
-
 template <int D>
 int fwd_launch(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, void* o,
                const long* os, float* lse, int B, int H, int T, float scale, int nw, hipStream_t s) {
@@ -922,10 +535,7 @@ int bwd_launch(const void* q, const long* qs, const void* k, const long* ks, con
   hipLaunchKernelGGL(attnD_dq_kernel<D>, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
                      mk(go, gos), mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, nw, mk(o, os), lse);
   TFB_LAUNCH_CHECK();
-  hipLaunchKernelGGL(attnD_dkdv_kernel<D>, dim3(paired_grid(T / 128, B * H, 1), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
-                     mk(go, gos), mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale, scale * LOG2E, nw);
-  TFB_LAUNCH_CHECK();
-  return TFB_OK;
+  return tfb_attn_dkdv_impl(q, qs, k, ks, v, vs, go, gos, dk, dks, dv, dvs, stats, B, H, T, D, scale, nullptr, nullptr, nw, s);
 }
 
 }  // namespace

@@ -127,37 +127,6 @@ __device__ __forceinline__ bf16x8 frag_cols(const uint8_t* tile, int dt, int tok
   return __builtin_bit_cast(bf16x8, v);
 }
 
-// Store one token's gradient row from the two 32-element halves a lane's accumulators hold (elements 8 j + 4 lh + i of
-// each half), scaled and rounded once to bf16; with cos / sin tables ([T][32] bf16) the inverse RoPE rotation
-// (y1 = x1 c - x2 s, y2 = x2 c + x1 s on the rounded values, rounded again: what a separate pass over the bf16
-// gradient computes) is applied on the way out.
-__device__ __forceinline__ void store_grad_row(const f32x16 (&acc)[2], float scale, bf16_t* row, const bf16_t* cs,
-                                               const bf16_t* sn, int tok, int lh) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int d = 8 * j + 4 * lh;
-    u32x2 w1 = {pack2bf(acc[0][4 * j] * scale, acc[0][4 * j + 1] * scale),
-                pack2bf(acc[0][4 * j + 2] * scale, acc[0][4 * j + 3] * scale)};
-    u32x2 w2 = {pack2bf(acc[1][4 * j] * scale, acc[1][4 * j + 1] * scale),
-                pack2bf(acc[1][4 * j + 2] * scale, acc[1][4 * j + 3] * scale)};
-    if (cs) {
-      const u32x2 c = *(const u32x2*)(cs + (long)tok * 32 + d), s = *(const u32x2*)(sn + (long)tok * 32 + d);
-      u32x2 o1, o2;
-#pragma unroll
-      for (int x = 0; x < 2; ++x) {
-        const float a0 = bflo(w1[x]), a1 = bfhi(w1[x]), b0 = bflo(w2[x]), b1 = bfhi(w2[x]);
-        const float c0 = bflo(c[x]), c1 = bfhi(c[x]), s0 = -bflo(s[x]), s1 = -bfhi(s[x]);
-        o1[x] = pack2bf(a0 * c0 + b0 * s0, a1 * c1 + b1 * s1);
-        o2[x] = pack2bf(b0 * c0 - a0 * s0, b1 * c1 - a1 * s1);
-      }
-      w1 = o1;
-      w2 = o2;
-    }
-    *(u32x2*)(row + d) = w1;
-    *(u32x2*)(row + 32 + d) = w2;
-  }
-}
-
 // =========================================================================================== forward
 __global__ __launch_bounds__(256, TFB_FWD64_WPE) void attn64_fwd_kernel(AttnT q, AttnT k, AttnT v, AttnT o, float* __restrict__ lse,
                                                             int T, int H, float sl2, int nw, int slots) {
@@ -884,6 +853,14 @@ int tfb_attn64_bwd_impl(const void* q, const long* qs, const void* k, const long
                      mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw,
                      tfb_resident_slots(2), mk(o, os), lse);
   TFB_LAUNCH_CHECK();
+  // Few key blocks: pairs of wavefronts (one workgroup of eight wavefronts on a CU, two on each SIMD) in place of one or two workgroups of
+  // four, up to one and a half blocks for each CU, and up to two where the blocks of a sequence are twelve or more: the longest then sets
+  // the time (dQ and dK/dV, us, that kernel -> pairs: T2048 192 blocks 76 -> 68, 384 81 -> 72, 512 88 -> 86, T4096 384 148 -> 130, T8192
+  // 128 258 -> 220, T1024 320 47 -> 43, T512 64 26.4 -> 24.6; beyond, T768 432 41.9 -> 44.5, T3072 576 132 -> 134, T256 384 25.7 ->
+  // 30.6; sequences of one block 12.7 -> 14.1).
+  const long nx = T / 128, blocks = nx * B * H, cus = tfb_resident_slots(1);
+  if (nx > 1 && 2 * blocks <= (nx >= 12 ? 4 : 3) * cus && tfb_attn_dkdv_strides_ok(qs, gos))
+    return tfb_attn_dkdv_impl(q, qs, k, ks, v, vs, go, gos, dk, dks, dv, dvs, stats, B, H, T, 64, scale, cos_t, sin_t, nw, s);
   hipLaunchKernelGGL(attn64_dkdv_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
                      mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw, tfb_resident_slots(2));
   TFB_LAUNCH_CHECK();

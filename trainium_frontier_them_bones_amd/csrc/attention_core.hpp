@@ -3,6 +3,14 @@
 #pragma once
 #include "common.hpp"
 
+// dK and dV by pairs of wavefronts (attention_dkdv.hip). Its loads address 32 tokens by a 32-bit offset.
+int tfb_attn_dkdv_impl(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, const void* go,
+                       const long* gos, void* dk, const long* dks, void* dv, const long* dvs, const float* stats, int B, int H, int T,
+                       int D, float scale, const void* cos_t, const void* sin_t, int nw, hipStream_t s);
+static inline bool tfb_attn_dkdv_strides_ok(const long* qs, const long* gos) {
+  return qs[2] >= 0 && qs[2] < (1L << 25) && gos[2] >= 0 && gos[2] < (1L << 25);
+}
+
 namespace {
 
 struct AttnT {
@@ -29,6 +37,37 @@ __device__ __forceinline__ float max_halves(float x) {  // the larger of the two
   float y = x;
   asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y));
   return fmaxf(x, y);
+}
+
+// Store one token's gradient row from the two 32-element halves a lane's accumulators hold (elements 8 j + 4 lh + i of
+// each half), scaled and rounded once to bf16; with cos / sin tables ([T][32] bf16) the inverse RoPE rotation
+// (y1 = x1 c - x2 s, y2 = x2 c + x1 s on the rounded values, rounded again: what a separate pass over the bf16
+// gradient computes) is applied on the way out.
+__device__ __forceinline__ void store_grad_row(const f32x16 (&acc)[2], float scale, bf16_t* row, const bf16_t* cs,
+                                               const bf16_t* sn, int tok, int lh) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int d = 8 * j + 4 * lh;
+    u32x2 w1 = {pack2bf(acc[0][4 * j] * scale, acc[0][4 * j + 1] * scale),
+                pack2bf(acc[0][4 * j + 2] * scale, acc[0][4 * j + 3] * scale)};
+    u32x2 w2 = {pack2bf(acc[1][4 * j] * scale, acc[1][4 * j + 1] * scale),
+                pack2bf(acc[1][4 * j + 2] * scale, acc[1][4 * j + 3] * scale)};
+    if (cs) {
+      const u32x2 c = *(const u32x2*)(cs + (long)tok * 32 + d), s = *(const u32x2*)(sn + (long)tok * 32 + d);
+      u32x2 o1, o2;
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const float a0 = bflo(w1[x]), a1 = bfhi(w1[x]), b0 = bflo(w2[x]), b1 = bfhi(w2[x]);
+        const float c0 = bflo(c[x]), c1 = bfhi(c[x]), s0 = -bflo(s[x]), s1 = -bfhi(s[x]);
+        o1[x] = pack2bf(a0 * c0 + b0 * s0, a1 * c1 + b1 * s1);
+        o2[x] = pack2bf(b0 * c0 - a0 * s0, b1 * c1 - a1 * s1);
+      }
+      w1 = o1;
+      w2 = o2;
+    }
+    *(u32x2*)(row + d) = w1;
+    *(u32x2*)(row + 32 + d) = w2;
+  }
 }
 
 // Workgroup -> (block along the sequence, batch*head): consecutive workgroup ids are dealt round-robin to the 8 XCDs, each with its own
