@@ -32,3 +32,25 @@ def test_many_rows_equal_few(M, d, F):
     # and every row against its own group of 1024: the tiles of every XCD
     r = torch.cat([ops.mlp8_fwd(c.contiguous(), w8, row, F)[1] for c in x.split(1024)])
     assert torch.equal(all_rows[1], r)
+
+
+# the clamped square of the up-projection, read through a second GEMM that is the identity: a power of two as the clamp's scale (one multiplication
+# and the scale in the conversion), one that is not, sums beyond the clamp, infinite and tiny ones
+@pytest.mark.parametrize("times", [1.0, 0.75])
+@pytest.mark.parametrize("M", [128, 16384])
+def test_clamped_square_of_the_up_projection(M, times):
+    dev = torch.device("cuda:0")
+    d, F = (256, 256) if M == 128 else (1024, 2048)
+    g = torch.Generator(device=dev).manual_seed(M)
+    w_fc = (torch.randn(F, d, generator=g, device=dev) * d ** -0.5).bfloat16()
+    w_proj = torch.zeros(d, F, device=dev, dtype=torch.bfloat16)
+    w_proj[:, :d] = torch.eye(d, device=dev).bfloat16()
+    row = ops.mlp8_forward_scales(w_fc, w_proj)
+    w8 = ops.mlp8_precast(w_fc, w_proj, row)
+    row[2] *= times                                                  # c
+    x = torch.randn(M, d, generator=g, device=dev) * torch.logspace(-6, 2, M, device=dev)[:, None]
+    y, r = ops.mlp8_fwd(x.bfloat16(), w8, row, F)[:2]
+    rc = (r.float() * row[2]).bfloat16().float().clamp(max=15.375)
+    h8 = (rc * rc).to(torch.float8_e4m3fn).float()
+    one = w8[2].view(torch.float8_e4m3fn).float().view(d, F)[0, 0]   # the identity's entries as cast
+    assert torch.equal(y, (h8[:, :d] * one * row[4]).bfloat16())

@@ -82,15 +82,20 @@ __device__ __forceinline__ void unpack8bf(u32x4 u, float (&v)[8]) {
 #define TFB_FMT_E4M3 0
 #define TFB_FMT_E5M2 1
 
+// x within [-limit, limit]; a NaN stays one (two instructions: fminf and fmaxf drop it, and a comparison and a choice cost two more)
+__device__ __forceinline__ float clamp_keeping_nan(float x, float limit) {
+  return __builtin_elementwise_minimum(__builtin_elementwise_maximum(x, -limit), limit);
+}
+
 // CLAMP = false: for values the caller has already bounded inside the format's range.
 template <int FMT, bool CLAMP = true>
 __device__ __forceinline__ uint32_t cvt4_fp8(float a, float b, float c, float d) {
   if (CLAMP) {  // saturate the finite values; a NaN stays a NaN (fminf / fmaxf alone would turn it into -max)
     const float mx = FMT == TFB_FMT_E4M3 ? TFB_E4M3_MAX : TFB_E5M2_MAX;
-    a = a != a ? a : fminf(fmaxf(a, -mx), mx);
-    b = b != b ? b : fminf(fmaxf(b, -mx), mx);
-    c = c != c ? c : fminf(fmaxf(c, -mx), mx);
-    d = d != d ? d : fminf(fmaxf(d, -mx), mx);
+    a = clamp_keeping_nan(a, mx);
+    b = clamp_keeping_nan(b, mx);
+    c = clamp_keeping_nan(c, mx);
+    d = clamp_keeping_nan(d, mx);
   }
   int w = 0;
   if (FMT == TFB_FMT_E4M3) {

@@ -52,6 +52,13 @@ __device__ __forceinline__ void ws8_unroll(F&& f) {
   }
 }
 
+// An epilogue may take an element's place in its outputs (place(p, q), linear in q) instead of its coordinates: put(place, v [, prefetched]).
+// A product of 64 bits for every row of a lane is a large part of what it does.
+template <class T, class = void>
+struct has_place : std::false_type {};
+template <class T>
+struct has_place<T, std::void_t<decltype(std::declval<const T&>().place(0, 0))>> : std::true_type {};
+
 // NK: the contraction in k-tiles of 128 bytes
 template <int NK, int FMTP, int FMTQ, class Epi>
 __global__ __launch_bounds__(512, 2) void gemm_ws8_kernel(Ws8Args a, Epi epi_in) {
@@ -205,14 +212,26 @@ __global__ __launch_bounds__(512, 2) void gemm_ws8_kernel(Ws8Args a, Epi epi_in)
     where(t, panel, q0);
     const int p = panel * 256 + 64 * (wave >> 1) + 8 * (lane & 7);
     const int ql = (TT / 2) * (wave & 1) + (lane >> 3);
+    [[maybe_unused]] long off = 0, down = 0;
+    if constexpr (has_place<Epi>::value) {
+      off = epi.place(p, (int)q0 + ql);
+      down = epi.place(0, 8);
+    }
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
       const int row = ql + 8 * k, c = 2 * (lane & 7);
       const f32x4 lo = *(const f32x4*)(stg + row * 256 + ((c ^ (row & 15)) << 4));
       const f32x4 hi = *(const f32x4*)(stg + row * 256 + (((c + 1) ^ (row & 15)) << 4));
       const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      if constexpr (kPrefetch) epi(p, (int)q0 + row, v, pre[k], 0);
-      else epi(p, (int)q0 + row, v, 0);
+      if constexpr (has_place<Epi>::value) {
+        if constexpr (kPrefetch) epi.put(off, v, pre[k]);
+        else epi.put(off, v);
+        off += down;
+      } else if constexpr (kPrefetch) {
+        epi(p, (int)q0 + row, v, pre[k], 0);
+      } else {
+        epi(p, (int)q0 + row, v, 0);
+      }
     }
   };
 

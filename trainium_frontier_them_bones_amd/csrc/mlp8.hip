@@ -384,12 +384,23 @@ __global__ __launch_bounds__(256) void precast_mlp_kernel(const bf16_t* __restri
 // All activation GEMMs: P side = the weight pack layout whose rows are the output's contiguous
 // dimension, Q side = the token-major fp8 activation. p = output column (4 consecutive), q = token.
 
+// x is a power of two whose square and reciprocal are too
+__device__ __forceinline__ bool is_pow2(float x) {
+  const uint32_t b = __float_as_uint(x);
+  return (b & 0x807fffffu) == 0 && (b >> 23) > 67 && (b >> 23) < 187;
+}
+
 struct EpiUp {  // pre = x8 @ wf8^T: r, h8
   const float* sc;
   bf16_t* r;     // [M][F]
   uint8_t* h8;   // [M][F]
   long F;
   float dq = 0.f, c = 0.f;  // sc[SC_DQ_FC], sc[SC_C_H], read once by prepare()
+  // With c a power of two (what the scale search produces) r c is a bf16 value as r is, and min(r c, 15.375)^2 = min(r^2, (15.375 / c)^2)
+  // c^2 with every product exact: one multiplication, one minimum, and the scale in the conversion, instead of two, one and a rounding.
+  // (4096 x 4096 x 1024 on the 128 x 128 kernel 29.6 -> 27.5 us; the kernel with the weights in registers is bound by its stores: 92)
+  float inv_c2 = 0.f, lim = 0.f;
+  bool fast = false;
   __device__ __forceinline__ EpiUp for_group(int g) const {
     EpiUp e = *this;
     e.sc = sc + g * NSC;
@@ -399,48 +410,51 @@ struct EpiUp {  // pre = x8 @ wf8^T: r, h8
     EpiUp e = *this;
     e.dq = sc[SC_DQ_FC];
     e.c = sc[SC_C_H];
+    e.fast = is_pow2(e.c);
+    e.inv_c2 = 1.0f / (e.c * e.c);
+    e.lim = H_CLAMP * H_CLAMP * e.inv_c2;
     return e;
   }
-  __device__ __forceinline__ void operator()(int p, int q, const float (&v)[8], int) const {
+  typedef short s2_t __attribute__((ext_vector_type(2)));
+  __device__ __forceinline__ uint32_t cast4(float a, float b, float x, float y) const {
+    s2_t o = {0, 0};
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(o, a, b, inv_c2, false);
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(o, x, y, inv_c2, true);
+    return __builtin_bit_cast(uint32_t, o);
+  }
+  __device__ __forceinline__ long place(int p, int q) const { return (long)q * F + p; }
+  __device__ __forceinline__ void put(long off, const float (&v)[8]) const {
     float hh[8];
     u32x4 rbits;
 #pragma unroll
     for (int i = 0; i < 8; i += 2) {
-      float a = fmaxf(v[i] * dq, 0.f), b = fmaxf(v[i + 1] * dq, 0.f);
-      rbits[i >> 1] = round2_bf(a, b);                       // r = bf16(max(acc dq, 0)): saved before the clamp
-      float ca = fminf(a * c, H_CLAMP), cb = fminf(b * c, H_CLAMP);
-      round2_bf(ca, cb);                                     // rc = bf16(min(r c_h, 15.375))
-      hh[i] = ca * ca;
-      hh[i + 1] = cb * cb;
+      hh[i] = fmaxf(v[i] * dq, 0.f);
+      hh[i + 1] = fmaxf(v[i + 1] * dq, 0.f);
+      rbits[i >> 1] = round2_bf(hh[i], hh[i + 1]);             // r = bf16(max(acc dq, 0)): saved before the clamp
     }
-    const long off = (long)q * F + p;
     // r is read again only by the backward: a non-temporal store keeps its 201 MB per layer from pushing the operand
     // tiles the other workgroups re-read out of the L2 (forward 2.69 -> 2.29 ms per step); full lines only: the same hint
     // on stores of part of a line (the LM head's logits, 16 bytes a row) bypasses the L2's merging and costs 2x
     __builtin_nontemporal_store(rbits, (u32x4*)(r + off));
-    // 0 <= rc^2 <= 15.375^2 < 240: inside the e4m3 range, no saturation clamp needed
-    u32x2 o = {cvt4_fp8<TFB_FMT_E4M3, false>(hh[0], hh[1], hh[2], hh[3]),
-               cvt4_fp8<TFB_FMT_E4M3, false>(hh[4], hh[5], hh[6], hh[7])};
+    u32x2 o;
+    if (fast) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) hh[i] = fminf(hh[i] * hh[i], lim);
+      o = u32x2{cast4(hh[0], hh[1], hh[2], hh[3]), cast4(hh[4], hh[5], hh[6], hh[7])};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        float ca = fminf(hh[i] * c, H_CLAMP), cb = fminf(hh[i + 1] * c, H_CLAMP);
+        round2_bf(ca, cb);                                     // rc = bf16(min(r c_h, 15.375))
+        hh[i] = ca * ca;
+        hh[i + 1] = cb * cb;
+      }
+      // 0 <= rc^2 <= 15.375^2 < 240: inside the e4m3 range, no saturation clamp needed
+      o = u32x2{cvt4_fp8<TFB_FMT_E4M3, false>(hh[0], hh[1], hh[2], hh[3]), cvt4_fp8<TFB_FMT_E4M3, false>(hh[4], hh[5], hh[6], hh[7])};
+    }
     *(u32x2*)(h8 + off) = o;   // (read by the next GEMM: a non-temporal store here costs 0.2 ms per step)
   }
-  // the 256 x 256 kernel's protocol (pre() before the rounding to bf16, chunk() on the 8 rounded values): the same values
-  __device__ __forceinline__ float pre(float x) const { return fmaxf(x * dq, 0.f); }
-  __device__ __forceinline__ void chunk(int p, int q, const u32x4& rbits) const {
-    float a[8], hh[8];
-    unpack8bf(rbits, a);
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      float ca = fminf(a[i] * c, H_CLAMP), cb = fminf(a[i + 1] * c, H_CLAMP);
-      round2_bf(ca, cb);
-      hh[i] = ca * ca;
-      hh[i + 1] = cb * cb;
-    }
-    const long off = (long)q * F + p;
-    __builtin_nontemporal_store(rbits, (u32x4*)(r + off));
-    u32x2 o = {cvt4_fp8<TFB_FMT_E4M3, false>(hh[0], hh[1], hh[2], hh[3]),
-               cvt4_fp8<TFB_FMT_E4M3, false>(hh[4], hh[5], hh[6], hh[7])};
-    *(u32x2*)(h8 + off) = o;
-  }
+  __device__ __forceinline__ void operator()(int p, int q, const float (&v)[8], int) const { put(place(p, q), v); }
 };
 
 struct EpiScaleStore {  // out = bf16(acc * sc[col])
@@ -605,8 +619,11 @@ struct EpiDh {  // dh = dy8 @ wp8: dpre = bf16((acc*dq_dh2)*r), dp8 = e5m2(dpre*
     }
     return __builtin_bit_cast(uint32_t, o);
   }
-  __device__ __forceinline__ void operator()(int p, int q, const float (&v)[8], const pre_t& rv, int) const {
-    const long off = (long)q * F + p;
+  __device__ __forceinline__ long place(int p, int q) const { return (long)q * F + p; }
+  __device__ __forceinline__ void operator()(int p, int q, const float (&v)[8], const pre_t& rv, int) const { put(place(p, q), v, rv); }
+  // What bounds the dH kernels is this: some ten instructions an element, by a wavefront alone on its SIMD's vector unit. With the clamp as two
+  // of them instead of three or four and the place kept as an offset, 32768 x 3072 x 768 117 -> 109 us, 16384 x 4096 x 1024 106 -> 93.
+  __device__ __forceinline__ void put(long off, const float (&v)[8], const pre_t& rv) const {
     float rr[8], dp[8];
     unpack8bf(rv, rr);
     u32x4 dbits;
@@ -615,7 +632,7 @@ struct EpiDh {  // dh = dy8 @ wp8: dpre = bf16((acc*dq_dh2)*r), dp8 = e5m2(dpre*
       for (int i = 0; i < 8; ++i) dp[i] = (v[i] * dq) * rr[i];
       if (dpre) *(u32x4*)(dpre + off) = pack8bf(dp);                 // dpre = bf16((acc dq_dh2) r)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) dp[i] = dp[i] != dp[i] ? dp[i] : fminf(fmaxf(dp[i], -lim_dp), lim_dp);
+      for (int i = 0; i < 8; ++i) dp[i] = clamp_keeping_nan(dp[i], lim_dp);
       dbits = pack8bf(dp);
       u32x2 o = {cast4_scaled<TFB_FMT_E5M2>(dbits[0], dbits[1], inv_sdp), cast4_scaled<TFB_FMT_E5M2>(dbits[2], dbits[3], inv_sdp)};
       *(u32x2*)(dp8 + off) = o;
