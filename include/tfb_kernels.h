@@ -170,6 +170,10 @@ int tfb_mlp8_backward_scales(const void* dy, const void* row_in, void* row_out, 
 /* The same row from npart amax partials whose maximum is amax(dy) (as tfb_rmsnorm_bwd_amax leaves them): no pass over dy.
  * Replaces backward_scales (nki_mlp_fused8.py:803-813). */
 int tfb_mlp8_backward_scales_part(const void* amax_part, int npart, const void* row_in, void* row_out, int d, void* stream);
+/* The same row (amax_part null: from dy, its maxima in scratch) and out8 [n_out] = e5m2(dy s_dy), zeros from n on, copy (optional) bf16
+ * alike: one launch behind the maxima. n, n_out % 8 == 0. */
+int tfb_mlp8_backward_quant(const void* dy, const void* amax_part, int npart, void* scratch, const void* row_in, void* row_out, void* out8,
+                            void* copy, long n, long n_out, int d, void* stream);
 
 /* out fp32 [3] = (s, 1/s, amax): s = 2^e the largest with amax(x) s <= limit, e in [e_lo, e_hi]; scratch fp32 [1024].
  * The reference's _pow2_le (nki_mlp_fused8.py:742) applied to a tensor's amax. */

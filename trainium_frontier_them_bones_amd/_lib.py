@@ -36,6 +36,7 @@ SIGNATURES = {
     "tfb_mlp8_forward_scales": [_vp, _vp, _vp, _vp, _i, _i, _f, _f, _vp, _vp],
     "tfb_mlp8_backward_scales": [_vp, _vp, _vp, _vp, _l, _i, _vp],
     "tfb_mlp8_backward_scales_part": [_vp, _i, _vp, _vp, _i, _vp],
+    "tfb_mlp8_backward_quant": [_vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _l, _l, _i, _vp],
     "tfb_amax_scale": [_vp, _l, _f, _i, _i, _vp, _vp, _vp],
     "tfb_quant_fp8": [_vp, _vp, _f, _i, _vp, _l, _vp],
     "tfb_quant_fp8_pad": [_vp, _vp, _f, _i, _vp, _vp, _l, _l, _vp],

@@ -189,15 +189,10 @@ std::pair<Tensor, Tensor> linear_backward(const Tensor& gy, const Tensor& x, con
   return {dx, gb.buf.defined() ? Tensor() : dw};
 }
 
-// The scale row of an fp8 MLP backward: from the amax partials on the gradient when they are still valid, else from a pass over
-// it.
-Tensor backward_scales(const Tensor& gy, const Tensor& g2, const Tensor& row) {
-  Tensor hint;
-  {
-    pybind11::gil_scoped_acquire gil;
-    if (switched_on(names().use_amax)) hint = tensor_of(amax_hint(gy, g2));
-  }
-  return op::mlp8_backward_scales(g2, row, hint);
+// The amax partials on a gradient that an fp8 MLP backward starts from, when they are still valid (else it makes a pass over it).
+Tensor amax_of(const Tensor& gy, const Tensor& g2) {
+  pybind11::gil_scoped_acquire gil;
+  return switched_on(names().use_amax) ? tensor_of(amax_hint(gy, g2)) : Tensor();
 }
 
 void attach(const Tensor& dx, const Tensor& amax) {
@@ -604,7 +599,10 @@ struct MlpGrads {
 };
 MlpGrads mlp8_backward(const Mlp8Attrs& st, const Tensor& gy_in, const Tensor& gy, const Tensor& xa, const Tensor& r, const Tensor& w_fc,
                        const Tensor& w_proj, bool buffers) {
-  const Tensor rowb = backward_scales(gy_in, gy, st.row);
+  const Tensor amax = amax_of(gy_in, gy);
+  // (where an op of the package is replaced, the ops one by one)
+  const ScaledGrad sg = any_replaced ? ScaledGrad{op::mlp8_backward_scales(gy, st.row, amax), {}, {}} : mlp8_scaled_grad(gy, st.row, amax, !st.dw_fp8);
+  const Tensor& rowb = sg.row;
   const int64_t F = w_fc.size(0), d = w_fc.size(1), M = r.size(0);
   MlpGrads o;
   if (st.dw_fp8) {
@@ -619,13 +617,13 @@ MlpGrads mlp8_backward(const Mlp8Attrs& st, const Tensor& gy_in, const Tensor& g
       return {bf.buf, bp.buf, bf.accumulate};
     };
     if (!any_replaced && mlp8_bwd_dw8_applies(r, d)) {
-      o.dx = mlp8_bwd_dw8(gy, r, st.w8, rowb, st.limit, xa, st.x_scale, [&]() -> DwOut {
+      o.dx = mlp8_bwd_dw8(gy, r, st.w8, sg, st.limit, xa, st.x_scale, [&]() -> DwOut {
         DwOut w = outputs();
         if (!in_place) w.fc = o.dw_fc = make({F, d}, BF16, gy), w.proj = o.dw_proj = make({d, F}, BF16, gy);
         return w;
       });
     } else {
-      MlpBwd b = op::mlp8_bwd_q(gy, r, st.w8, rowb, st.limit, false);
+      MlpBwd b = any_replaced ? op::mlp8_bwd_q(gy, r, st.w8, rowb, st.limit, false) : mlp8_bwd_q(gy, r, st.w8, sg, st.limit, false);
       const bool accumulate = outputs().accumulate;
       op::mlp8_dw8(xa, b.dp8, b.hq8, b.dy8, rowb, st.x_scale, o.dw_fc, o.dw_proj, accumulate, BF16);
       o.dx = b.dx;
@@ -633,7 +631,7 @@ MlpGrads mlp8_backward(const Mlp8Attrs& st, const Tensor& gy_in, const Tensor& g
     if (in_place) o.dw_fc = o.dw_proj = Tensor();
     return o;
   }
-  MlpBwd b = op::mlp8_bwd(gy, r, st.w8, rowb, false, true);
+  MlpBwd b = any_replaced ? op::mlp8_bwd(gy, r, st.w8, rowb, false, true) : mlp8_bwd(gy, r, st.w8, sg, false);
   o.dx = b.dx;
   if (!buffers) {
     o.dw_fc = make({F, d}, BF16, gy);

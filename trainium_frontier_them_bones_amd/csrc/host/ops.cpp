@@ -196,6 +196,18 @@ Tensor mlp8_backward_scales(const Tensor& dy, const Tensor& row, const Tensor& a
   return out;
 }
 
+ScaledGrad mlp8_scaled_grad(const Tensor& dy, const Tensor& row, const Tensor& amax_part, bool want_padded) {
+  chk(dy), chk(row, F32), chk(amax_part, F32);
+  TORCH_CHECK_VALUE(row.numel() >= 16, "the scale row has ", row.numel(), " entries");
+  const int64_t d = last_dim(dy), n = dy.numel(), M = tile_rows(n / d);
+  ScaledGrad o{scratch(dy, 16), make({M, d}, U8, dy), want_padded && n == M * d ? dy : want_padded ? make({M, d}, BF16, dy) : Tensor()};
+  const Tensor scr = amax_part.defined() ? Tensor() : scratch(dy, 4096);
+  const bool copy = want_padded && n != M * d;
+  TFB_CALL(tfb_mlp8_backward_quant, ptr(dy), ptr(amax_part), amax_part.defined() ? amax_part.numel() : 0, ptr(scr), ptr(row), ptr(o.row),
+           ptr(o.bytes), copy ? ptr(o.padded) : nullptr, n, M * d, d, stream());
+  return o;
+}
+
 Tensor amax_scale(const Tensor& x, double limit, int64_t e_lo, int64_t e_hi) {
   chk(x);
   Tensor out = scratch(x, 3), scr = scratch(x, 4096);
@@ -293,13 +305,29 @@ MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F,
   return o;
 }
 
-MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h, bool want_dyp) {
+// What a backward of dy's rows is given; the rows in whole tiles.
+static int64_t check_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row) {
   chk(dy), chk(r), chk(w8, U8), chk(row, F32);
   const int64_t d = last_dim(dy), M = tile_rows(dy.numel() / d), F = r.size(1);
   check_rows(r, M, F);
   check_pack(w8, row, d, F);
+  return M;
+}
+// dy's bytes at a row's scale
+static ScaledGrad at_scale(const Tensor& dy, const Tensor& row, int64_t M, bool want_padded) {
+  ScaledGrad o{row, {}, {}};
+  o.bytes = quant_rows(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2, M, want_padded ? &o.padded : nullptr);
+  return o;
+}
+
+MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h, bool want_dyp) {
+  return mlp8_bwd(dy, r, w8, at_scale(dy, row, check_bwd(dy, r, w8, row), want_dyp), want_h);
+}
+MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const ScaledGrad& sg, bool want_h) {
+  const Tensor& row = sg.row;
+  const int64_t M = check_bwd(dy, r, w8, row), d = last_dim(dy), F = r.size(1);
   MlpBwd o;
-  o.dy8 = quant_rows(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2, M, want_dyp ? &o.dyp : nullptr);
+  o.dy8 = sg.bytes, o.dyp = sg.padded;
   o.dx = make_rows(dy.sizes(), M, d, dy);
   o.dpre = make({M, F}, BF16, dy);
   if (want_h) o.h = make({M, F}, BF16, dy);
@@ -309,12 +337,13 @@ MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tenso
 }
 
 MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, bool want_dpre) {
-  chk(dy), chk(r), chk(w8, U8), chk(row, F32);
-  const int64_t d = last_dim(dy), M = tile_rows(dy.numel() / d), F = r.size(1);
-  check_rows(r, M, F);
-  check_pack(w8, row, d, F);
+  return mlp8_bwd_q(dy, r, w8, at_scale(dy, row, check_bwd(dy, r, w8, row), false), limit, want_dpre);
+}
+MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const ScaledGrad& sg, double limit, bool want_dpre) {
+  const Tensor& row = sg.row;
+  const int64_t M = check_bwd(dy, r, w8, row), d = last_dim(dy), F = r.size(1);
   MlpBwd o;
-  o.dy8 = quant_rows(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2, M, nullptr);
+  o.dy8 = sg.bytes;
   o.dx = make_rows(dy.sizes(), M, d, dy);
   if (want_dpre) o.dpre = make({M, F}, BF16, dy);
   o.dp8 = make({M, F}, U8, dy);
@@ -326,16 +355,14 @@ MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Ten
 
 bool mlp8_bwd_dw8_applies(const Tensor& r, int64_t d) { return tfb_mlp8_bwd_dw8_applies(r.size(0), d, r.size(1), WORKSPACE_BYTES) == 0; }
 
-Tensor mlp8_bwd_dw8(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, const Tensor& x8, const Scale& x_scale,
+Tensor mlp8_bwd_dw8(const Tensor& dy, const Tensor& r, const Tensor& w8, const ScaledGrad& sg, double limit, const Tensor& x8, const Scale& x_scale,
                     const std::function<DwOut()>& outputs) {
-  chk(dy), chk(r), chk(w8, U8), chk(row, F32), chk(x8, U8);
-  const int64_t d = last_dim(dy), M = tile_rows(dy.numel() / d), F = r.size(1);
-  check_rows(r, M, F);
-  check_pack(w8, row, d, F);
+  const Tensor &row = sg.row, &dy8 = sg.bytes;
+  chk(x8, U8);
+  const int64_t M = check_bwd(dy, r, w8, row), d = last_dim(dy), F = r.size(1);
   TORCH_CHECK_VALUE(x8.numel() == M * d && last_dim(x8) == d, "operand shapes");
   const DwOut o = outputs();
   TORCH_CHECK_VALUE(o.fc.numel() == F * d && o.proj.numel() == F * d && o.fc.scalar_type() == o.proj.scalar_type(), "bad outputs");
-  const Tensor dy8 = quant_rows(dy, static_cast<const float*>(ptr(row)) + 5, 0, E5M2, M, nullptr);
   const Tensor dx = make_rows(dy.sizes(), M, d, dy), dp8 = make({M, F}, U8, dy), hq8 = make({M, F}, U8, dy);
   TFB_CALL(tfb_mlp8_bwd_dw8, ptr(dy8), ptr(r), ptr(w8), ptr(row), ptr(dx), ptr(dp8), ptr(hq8), limit, ptr(x8), x_scale.imm, ptr(x_scale.dev),
            ptr(o.fc), ptr(o.proj), M, d, F, o.fc.scalar_type() == F32, o.accumulate, WORKSPACE_BYTES, stream());

@@ -43,6 +43,11 @@ struct Scale {
   double host() const { return dev.defined() ? dev.item<double>() : imm; }   // (reads the device value back)
 };
 Tensor mlp8_backward_scales(const Tensor& dy, const Tensor& row, const Tensor& amax_part);
+// The scale row and dy's bytes at its scale, whole tiles of rows; padded: dy in bf16 of as many, where it is asked for
+struct ScaledGrad {
+  Tensor row, bytes, padded;
+};
+ScaledGrad mlp8_scaled_grad(const Tensor& dy, const Tensor& row, const Tensor& amax_part, bool want_padded);
 Tensor amax_scale(const Tensor& x, double limit, int64_t e_lo, int64_t e_hi);
 Tensor quant_fp8(const Tensor& x, const void* scale_dev, double scale_imm, int fmt);
 Tensor quant_fp8(const Tensor& x, const Scale& s, int fmt);
@@ -58,14 +63,16 @@ MlpFwd mlp8_fwd(const Tensor& x, const Tensor& w8, const Tensor& row, int64_t F,
                 bool want_xp = false);
 struct MlpBwd { Tensor dx, h, dpre, dp8, hq8, dy8, dyp; };
 MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, bool want_h, bool want_dyp = false);
+MlpBwd mlp8_bwd(const Tensor& dy, const Tensor& r, const Tensor& w8, const ScaledGrad& sg, bool want_h);
 MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, bool want_dpre);
+MlpBwd mlp8_bwd_q(const Tensor& dy, const Tensor& r, const Tensor& w8, const ScaledGrad& sg, double limit, bool want_dpre);
 // dx and both weight gradients at once, where mlp8_bwd_dw8_applies; outputs() is asked for the latter once the operands are checked
 struct DwOut {
   Tensor fc, proj;
   bool accumulate;
 };
 bool mlp8_bwd_dw8_applies(const Tensor& r, int64_t d);
-Tensor mlp8_bwd_dw8(const Tensor& dy, const Tensor& r, const Tensor& w8, const Tensor& row, double limit, const Tensor& x8, const Scale& x_scale,
+Tensor mlp8_bwd_dw8(const Tensor& dy, const Tensor& r, const Tensor& w8, const ScaledGrad& sg, double limit, const Tensor& x8, const Scale& x_scale,
                     const std::function<DwOut()>& outputs);
 void mlp8_dw8(const Tensor& x8, const Tensor& dp8, const Tensor& hq8, const Tensor& dy8, const Tensor& row, const Scale& x_scale,
               Tensor& dw_fc, Tensor& dw_proj, bool accumulate, at::ScalarType out_dtype);

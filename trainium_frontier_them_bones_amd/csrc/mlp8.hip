@@ -14,6 +14,7 @@
 //   x8 = e4m3(x * s_x); r = bf16(max(acc * dq_fc, 0)); rc = bf16(min(r * c_h, 15.375));
 //   h8 = e4m3(rc^2); y = bf16(acc * dq_proj); dy8 = e5m2(dy * s_dy);
 //   dpre = bf16((acc * dq_dh2) * r); dp8 = e5m2(dpre * s_dp); dx = bf16(acc * dq_dx).
+#include <algorithm>
 #include "gemm_ring.hpp"
 #include "gemm_ws8.hpp"
 
@@ -272,16 +273,12 @@ __global__ __launch_bounds__(256) void forward_scales_kernel(const float* rowss,
   }
 }
 
-// One workgroup: the backward call's row from amax(dy) (nki_mlp_fused8.py:803-813).
-__global__ __launch_bounds__(256) void backward_scales_kernel(const float* amax_part, int npart, const float* row_in,
-                                                             float dp_factor, float* row_out) {
-  __shared__ float red[4];
-  float amax_dy = reduce_max_array(amax_part, npart, red);
+// One workgroup: the backward call's row from amax(dy) (nki_mlp_fused8.py:803-813), whose scale of dy is s_dy.
+__device__ __forceinline__ void backward_row(float amax_dy, float s_dy, float i_dy, const float* row_in, float dp_factor, float* row_out) {
   if (threadIdx.x < NSC) row_out[threadIdx.x] = row_in[threadIdx.x];
   __syncthreads();
   if (threadIdx.x == 0) {
-    float s_dy, i_dy, s_dp, i_dp;
-    pow2_le(amax_dy, TFB_E5M2_MAX / 2.0f, -40, 60, &s_dy, &i_dy);
+    float s_dp, i_dp;
     float bound = sqrtf(row_in[SC_RHO2] * row_in[SC_KAPPA2]) * amax_dy * dp_factor;
     pow2_le(bound, TFB_E5M2_MAX, -40, 60, &s_dp, &i_dp);
     row_out[SC_S_DY] = s_dy;
@@ -289,6 +286,14 @@ __global__ __launch_bounds__(256) void backward_scales_kernel(const float* amax_
     row_out[SC_S_DP] = s_dp;
     row_out[SC_DQ_DX] = i_dp * row_in[SC_I_WFC];
   }
+}
+__global__ __launch_bounds__(256) void backward_scales_kernel(const float* amax_part, int npart, const float* row_in,
+                                                             float dp_factor, float* row_out) {
+  __shared__ float red[4];
+  const float amax_dy = reduce_max_array(amax_part, npart, red);
+  float s_dy, i_dy;
+  pow2_le(amax_dy, TFB_E5M2_MAX / 2.0f, -40, 60, &s_dy, &i_dy);
+  backward_row(amax_dy, s_dy, i_dy, row_in, dp_factor, row_out);
 }
 
 // One workgroup: out[0] = s = 2^e (largest with amax * s <= limit), out[1] = 1/s.
@@ -321,6 +326,30 @@ __global__ __launch_bounds__(256) void quant_kernel(const bf16_t* __restrict__ x
     o.x = cvt4_fp8<FMT>(bflo(u[0]) * s, bfhi(u[0]) * s, bflo(u[1]) * s, bfhi(u[1]) * s);
     o.y = cvt4_fp8<FMT>(bflo(u[2]) * s, bfhi(u[2]) * s, bflo(u[3]) * s, bfhi(u[3]) * s);
     *(u32x2*)(out + i) = o;
+  }
+}
+
+// backward_scales_kernel and quant_kernel of dy at the scale it finds: every workgroup reduces the maxima (a few KB out of the L2, under its
+// first load of dy), the first leaves the row. A launch by itself for one workgroup's work takes 3 to 5 us of a backward call.
+// (a training step of 2048 tokens, twelve such calls, 4574 -> 4533 us; fp8 MLP of 16384 tokens 294 -> 292)
+__global__ __launch_bounds__(256) void backward_quant_kernel(const float* amax_part, int npart, const float* row_in, float dp_factor,
+                                                            float* row_out, const bf16_t* __restrict__ x, uint8_t* __restrict__ out,
+                                                            bf16_t* __restrict__ copy, long n, long n_out) {
+  __shared__ float red[4];
+  long i = ((long)blockIdx.x * 256 + threadIdx.x) * 8;
+  u32x4 u = i < n ? *(const u32x4*)(x + i) : u32x4{0u, 0u, 0u, 0u};
+  const float amax_dy = reduce_max_array(amax_part, npart, red);
+  float s, inv;
+  pow2_le(amax_dy, TFB_E5M2_MAX / 2.0f, -40, 60, &s, &inv);
+  if (blockIdx.x == 0) backward_row(amax_dy, s, inv, row_in, dp_factor, row_out);
+  while (i < n_out) {
+    if (copy) *(u32x4*)(copy + i) = u;
+    u32x2 o;
+    o.x = cvt4_fp8<TFB_FMT_E5M2>(bflo(u[0]) * s, bfhi(u[0]) * s, bflo(u[1]) * s, bfhi(u[1]) * s);
+    o.y = cvt4_fp8<TFB_FMT_E5M2>(bflo(u[2]) * s, bfhi(u[2]) * s, bflo(u[3]) * s, bfhi(u[3]) * s);
+    *(u32x2*)(out + i) = o;
+    i += (long)gridDim.x * 256 * 8;
+    u = i < n ? *(const u32x4*)(x + i) : u32x4{0u, 0u, 0u, 0u};
   }
 }
 
@@ -766,6 +795,26 @@ extern "C" int tfb_mlp8_backward_scales_part(const void* amax_part, int npart, c
   if (npart <= 0 || d <= 0) return TFB_ERR_SHAPE;
   hipLaunchKernelGGL(backward_scales_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, (const float*)amax_part, npart,
                      (const float*)row_in, (float)(36.16 * (double)d), (float*)row_out);
+  TFB_LAUNCH_CHECK();
+  return TFB_OK;
+}
+
+// tfb_mlp8_backward_scales(_part) and tfb_quant_fp8_pad of dy at the row's s_dy as one launch behind the maxima: out8 = e5m2(dy s_dy), bytes
+// n .. n_out zeros, copy (optional) [n_out] bf16 = dy, then zeros. amax_part null: the maxima are made here, in scratch.
+extern "C" int tfb_mlp8_backward_quant(const void* dy, const void* amax_part, int npart, void* scratch, const void* row_in, void* row_out,
+                                       void* out8, void* copy, long n, long n_out, int d, void* stream) {
+  if (!dy || !row_in || !row_out || !out8 || (!amax_part && !scratch)) return TFB_ERR_ARG;
+  if (n <= 0 || n_out < n || n % 8 || n_out % 8 || d <= 0 || (amax_part && npart <= 0)) return TFB_ERR_SHAPE;
+  hipStream_t s = (hipStream_t)stream;
+  if (!amax_part) {
+    npart = (int)std::min<long>((n / 8 + 255) / 256, AMAX_BLOCKS);
+    hipLaunchKernelGGL(amax_partial_kernel, dim3((unsigned)npart), dim3(256), 0, s, (const bf16_t*)dy, n, (float*)scratch);
+    TFB_LAUNCH_CHECK();
+    amax_part = scratch;
+  }
+  const long blocks = std::min<long>((n_out / 8 + 255) / 256, 8L * tfb_resident_slots(1));
+  hipLaunchKernelGGL(backward_quant_kernel, dim3((unsigned)blocks), dim3(256), 0, s, (const float*)amax_part, npart, (const float*)row_in,
+                     (float)(36.16 * (double)d), (float*)row_out, (const bf16_t*)dy, (uint8_t*)out8, (bf16_t*)copy, n, n_out);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
