@@ -75,7 +75,16 @@ struct PpArgs {
   GemmOperand P1, Q1;
   int nout0, p_fast1, nfast1;
   FastDiv d_nfast1;
+  // Contractions over segments of the rows (an epilogue with kExperts): group e's is seg[e] .. seg[e + 1] in rows, multiples of 128. A workgroup
+  // has one output tile of one group: XCD x tiles x ipx .. of the group with the most rows, then of the next
+  const int* seg;
+  int ngroups;
+  FastDiv d_ipx;
 };
+template <class T, class = void>
+struct has_experts : std::false_type {};
+template <class T>
+struct has_experts<T, std::void_t<decltype(T::kExperts)>> : std::true_type {};
 template <class T, class = void>
 struct has_second : std::false_type {};
 template <class T>
@@ -190,8 +199,25 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     return sd;
   };
   [[maybe_unused]] int first = 0;  // the first output tile of this workgroup's contraction
+  [[maybe_unused]] int group_tile = 0, group_k0 = 0, group_nkt = 0;
+  if constexpr (has_experts<Epi>::value) {
+    const int j = blockIdx.x >> 3, rank = fastdiv(j, a.d_ipx);
+    group_tile = (blockIdx.x & 7) * a.ipx + j - rank * a.ipx;
+    if (group_tile >= a.nout) return;  // (whole workgroup)
+    // the group of that rank: more rows first, of equal ones the lower index
+    const int rows = lane < a.ngroups ? a.seg[lane + 1] - a.seg[lane] : -1;
+    int before = 0;
+    for (int m = 0; m < a.ngroups; ++m) {
+      const int other = __builtin_amdgcn_readlane(rows, m);
+      before += other > rows || (other == rows && m < lane);
+    }
+    const int group = __builtin_ctzll(__ballot(lane < a.ngroups && before == rank));
+    group_k0 = __builtin_amdgcn_readfirstlane(a.seg[group]) / 128;
+    group_nkt = __builtin_amdgcn_readlane(rows, group) / 128;
+    epi_in = epi_in.for_group(group);
+  }
   if constexpr (has_second<Epi>::value) {
-    const int item = (blockIdx.x & 7) * a.ipx + (blockIdx.x >> 3);
+    const int item = has_experts<Epi>::value ? group_tile : (int)((blockIdx.x & 7) * a.ipx + (blockIdx.x >> 3));
     if (item - fastdiv(item, a.d_nout) * a.nout >= a.nout0) {
       first = a.nout0;
       a.P = a.P1;
@@ -232,6 +258,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   auto krange = [&](int split, int& k0, int& n) {
     k0 = 0;
     n = a.nk_total;
+    if constexpr (has_experts<Epi>::value) {
+      k0 = group_k0;
+      n = group_nkt;
+    }
     if (a.splits > 1) {
       k0 = (int)((long)split * a.nk_total / a.splits);
       n = (int)((long)(split + 1) * a.nk_total / a.splits) - k0;
@@ -385,7 +415,9 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
 
   const Epi epi = epi_prepare(epi_in);
   int w = blockIdx.x;
-  if (a.ipx > 0) {
+  if constexpr (has_experts<Epi>::value) {
+    w = group_tile;
+  } else if (a.ipx > 0) {
     if ((w >> 3) >= a.ipx) return;
     w = (w & 7) * a.ipx + (w >> 3);
   }
@@ -397,14 +429,24 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   const uint8_t* gp = origin(sp, p0, k0);  // current work item: the sides' addresses of its first k-tile
   const uint8_t* gq = origin(sq, q0, k0);
 
+  // A segment without rows: nothing is loaded, its product is zero.
+  if constexpr (has_experts<Epi>::value) {
+    if (nkt == 0) {
+      const float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int i = tid; i < 256 * 32; i += 512) epi((int)p0 + 8 * (i & 31), (int)q0 + (i >> 5), v, 0);
+      return;
+    }
+  }
+
   // ---- prologue: all of k-tile 0 into stage 0, three quarters of k-tile 1 into stage 1
   dma(0, 1, 0, gq);
   dma(0, 0, 0, gp);
   dma(0, 1, 1, gq);
   dma(0, 0, 1, gp);
-  dma(1, 0, 0, gp + sp.kstep);
-  dma(1, 1, 0, gq + sq.kstep);
-  dma(1, 1, 1, gq + sq.kstep);
+  const long k_one = has_experts<Epi>::value && nkt < 2 ? 0 : 1;  // (a segment of one k-tile: that one again)
+  dma(1, 0, 0, gp + k_one * sp.kstep);
+  dma(1, 1, 0, gq + k_one * sq.kstep);
+  dma(1, 1, 1, gq + k_one * sq.kstep);
   asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
   TFB_SBAR();               // k-tile 0 is there for everybody
   if (wr == 1) TFB_SBAR();  // group 1 runs one cluster behind from here on
@@ -516,7 +558,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       constexpr bool first = decltype(FIRST)::value;
       // k positions one and two ahead in the workgroup's stream of k-tiles
       const bool in1 = kt + 1 < nkt, in2 = kt + 2 < nkt;
-      const long k1 = in1 ? kt + 1 : 0, k2 = in2 ? kt + 2 : kt + 2 - nkt;
+      const long k1 = in1 ? kt + 1 : 0, k2 = in2 ? kt + 2 : has_experts<Epi>::value && nkt < 2 ? 0 : kt + 2 - nkt;
       const uint8_t* gp1 = (in1 ? gp : gpn) + k1 * sp.kstep;
       const uint8_t* gp2 = (in2 ? gp : gpn) + k2 * sp.kstep;
       const uint8_t* gq2 = (in2 ? gq : gqn) + k2 * sq.kstep;
@@ -759,6 +801,46 @@ static int gemm_pp_launch_two(GemmOperand P0, GemmOperand Q0, int np0, int nq0, 
   const long n0 = (long)np0 * nq0, n1 = (long)np1 * nq1;
   EpiSplitTwo e{{ws, (long)np0, n0 + n1}, n0, (long)np1};
   hipLaunchKernelGGL((gemm_pp_kernel<1, TFB_FMT_E4M3, TFB_FMT_E5M2, TFB_K_STRIDED, TFB_K_STRIDED, EpiSplitTwo>), dim3(a.nwg), dim3(512), 0, stream, a, e);
+  TFB_LAUNCH_CHECK();
+  return TFB_OK;
+}
+
+// Two weight gradients of each of `groups` experts over its rows: P_i e4m3, Q_i e5m2, row segments seg (device, multiples of 128 rows). The
+// experts' loads are the router's and often far apart: tiles of the heaviest expert first, so that the others' fill the CUs beside its long
+// ones (and both gradients in one launch, so that these are twice as many).
+template <class Epi>
+static int gemm_pp_launch_experts(GemmOperand P0, GemmOperand Q0, int np0, int nq0, GemmOperand P1, GemmOperand Q1, int np1, int nq1, const int* seg,
+                                  int groups, Epi epi, hipStream_t stream) {
+  if (np0 <= 0 || nq0 <= 0 || np1 <= 0 || nq1 <= 0 || (np0 | nq0 | np1 | nq1) % 256 || groups <= 0 || groups > 64 || !seg) return TFB_ERR_SHAPE;
+  for (const GemmOperand& o : {P0, Q0, P1, Q1}) {
+    if (o.ld <= 0 || o.ld > (1L << 28)) return TFB_ERR_SHAPE;
+    if (((uintptr_t)o.base | (uintptr_t)o.ld) & 15) return TFB_ERR_ARG;
+  }
+  const long t0 = (long)(np0 / 256) * (nq0 / 256), t1 = (long)(np1 / 256) * (nq1 / 256);
+  if ((t0 + t1) * groups >= (1L << 24)) return TFB_ERR_SHAPE;
+  PpArgs a = {};
+  a.P = P0;
+  a.Q = Q0;
+  a.P1 = P1;
+  a.Q1 = Q1;
+  a.splits = 1;
+  a.nout0 = (int)t0;
+  a.nout = a.ntiles = (int)(t0 + t1);
+  a.ipx = (a.nout + 7) / 8;
+  a.nwg = 8 * a.ipx * groups;
+  a.p_fast = np0 <= nq0;
+  a.nfast = (a.p_fast ? np0 : nq0) / 256;
+  a.p_fast1 = np1 <= nq1;
+  a.nfast1 = (a.p_fast1 ? np1 : nq1) / 256;
+  a.R = a.GW = a.panel = a.gw_last = 1;
+  a.d_nfast = fastdiv_make(a.nfast);
+  a.d_nfast1 = fastdiv_make(a.nfast1);
+  a.d_panel = a.d_gw = a.d_gw_last = fastdiv_make(1);
+  a.d_nout = fastdiv_make(a.nout);
+  a.d_ipx = fastdiv_make(a.ipx);
+  a.seg = seg;
+  a.ngroups = groups;
+  hipLaunchKernelGGL((gemm_pp_kernel<1, TFB_FMT_E4M3, TFB_FMT_E5M2, TFB_K_STRIDED, TFB_K_STRIDED, Epi>), dim3(a.nwg), dim3(512), 0, stream, a, epi);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }

@@ -1298,6 +1298,13 @@ struct EpiDescaleGrouped {
     base(p, q, w, s);
   }
 };
+struct EpiExperts : EpiDescaleGrouped {  // both gradients', for the persistent kernel
+  static constexpr bool kExperts = true, kSplitF32 = true;
+  EpiDescaleGrouped other;
+  __device__ __forceinline__ EpiExperts for_group(int g) const { return EpiExperts{EpiDescaleGrouped::for_group(g), other.for_group(g)}; }
+  __device__ __forceinline__ EpiExperts for_second() const { return EpiExperts{other, other}; }
+  __device__ __forceinline__ EpiExperts prepare() const { return EpiExperts{EpiDescaleGrouped::prepare(), other}; }
+};
 }  // namespace
 
 // The experts' two weight gradients in fp8 over each expert's row segment [seg[e], seg[e+1]) of the grouped byte buffers
@@ -1325,6 +1332,13 @@ extern "C" int tfb_moe_dw8(const void* xs8, const void* dp8, const void* hq8, co
   a.nq = F;
   a.ntp = d / 128;
   EpiDescaleGrouped e1{EpiStore{dw_fc, (long)d, out_f32, accumulate}, (long)F * d, (const float*)rows, SC_S_DP, -1, 1.0f / x_scale};
+  EpiDescaleGrouped e2{EpiStore{dw_proj, (long)F, out_f32, accumulate}, (long)F * d, (const float*)rows, SC_S_DY, SC_S_H, 1.0f};
+  // whole 256 x 256 tiles: both gradients as one launch of the persistent kernel, one tile of one expert a workgroup, the same bits (us, 8 experts
+  // 1024 x 2816, two launches of the 128 x 128 kernel -> this: 13000 rows to each of two experts and 1200 to the others 247 -> 185, 4200 to
+  // each 247 -> 172, 512 55 -> 49, 256 41 -> 39, 128 31 -> 34; 4 experts 768 x 3072, 4096 rows each 115 -> 94)
+  if (TFB_PP && d % 256 == 0 && F % 256 == 0 && E <= 64)
+    return gemm_pp_launch_experts(a.P, a.Q, d, F, GemmOperand{(const uint8_t*)hq8, (long)F}, GemmOperand{(const uint8_t*)dy8, (long)d}, F, d,
+                                  (const int*)seg, E, EpiExperts{e1, e2}, s);
   int st = gemm_launch_args<Cfg>(a, E, 1, LoadIdentity{}, LoadIdentity{}, e1, s);
   if (st != TFB_OK) return st;
   // dw_proj[e][j][f] = sum_m dy8[m][j] hq8[m][f]: output contiguous in f -> P = hq8 (e4m3), Q = dy8 (e5m2)
@@ -1333,7 +1347,6 @@ extern "C" int tfb_moe_dw8(const void* xs8, const void* dp8, const void* hq8, co
   a.np = F;
   a.nq = d;
   a.ntp = F / 128;
-  EpiDescaleGrouped e2{EpiStore{dw_proj, (long)F, out_f32, accumulate}, (long)F * d, (const float*)rows, SC_S_DY, SC_S_H, 1.0f};
   return gemm_launch_args<Cfg>(a, E, 1, LoadIdentity{}, LoadIdentity{}, e2, s);
 }
 
