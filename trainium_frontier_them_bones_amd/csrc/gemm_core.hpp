@@ -777,11 +777,13 @@ struct EpiSplit {
 
 // out (+)= scale * (sum over splits of ws), rounded once; scale = imm / (*sa * *sb) (absent factors are 1: the fp8
 // GEMMs' power-of-two descale, exact), times *alpha when given
-// (elements i .. i + 3 of a slab of `slab` at ws)
-static __device__ __forceinline__ void splitk_reduce4(const float* __restrict__ ws, long slab, void* out, long i, int splits, int f32,
-                                                      int accumulate, const float* sa, const float* sb, float imm, const float* alpha) {
+static __global__ void splitk_reduce_kernel(const float* __restrict__ ws, void* out, long n, int splits, int f32,
+                                            int accumulate, const float* sa, const float* sb, float imm,
+                                            const float* alpha) {
+  long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (i >= n) return;
   f32x4 s = *(const f32x4*)(ws + i);
-  for (int k = 1; k < splits; ++k) s += *(const f32x4*)(ws + (long)k * slab + i);
+  for (int k = 1; k < splits; ++k) s += *(const f32x4*)(ws + (long)k * n + i);
   if (sa || sb || imm != 1.0f) {
     float d = 1.0f;
     if (sa) d *= *sa;
@@ -805,28 +807,6 @@ static __device__ __forceinline__ void splitk_reduce4(const float* __restrict__ 
     u32x2 r = {pack2bf(s[0], s[1]), pack2bf(s[2], s[3])};
     *(u32x2*)o = r;
   }
-}
-
-static __global__ void splitk_reduce_kernel(const float* __restrict__ ws, void* out, long n, int splits, int f32,
-                                            int accumulate, const float* sa, const float* sb, float imm,
-                                            const float* alpha) {
-  long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (i >= n) return;
-  splitk_reduce4(ws, n, out, i, splits, f32, accumulate, sa, sb, imm, alpha);
-}
-// One of two outputs whose partials lie side by side in a slab (each a multiple of 1024 elements, so a workgroup has one of them).
-struct SplitOut {
-  void* out;
-  const float *sa, *sb;
-  float imm;
-};
-static __global__ void splitk_reduce_two_kernel(const float* __restrict__ ws, SplitOut o0, SplitOut o1, long n0, long n1, int splits, int f32,
-                                                int accumulate) {
-  const long first = (long)blockIdx.x * blockDim.x * 4;
-  const bool second = first >= n0;
-  const SplitOut o = second ? o1 : o0;
-  const long i = first - (second ? n0 : 0) + threadIdx.x * 4;
-  splitk_reduce4(ws + (second ? n0 : 0), n0 + n1, o.out, i, splits, f32, accumulate, o.sa, o.sb, o.imm, nullptr);
 }
 
 static inline int splitk_reduce(const float* ws, void* out, long n, int splits, int f32, int accumulate, hipStream_t s,

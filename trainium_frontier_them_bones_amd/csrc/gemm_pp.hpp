@@ -70,13 +70,12 @@ struct PpArgs {
   int rect, R, GW, panel;  // panel = GW * R
   int gw_last;             // width of the last panel (nfast % GW, or GW)
   FastDiv d_nfast, d_panel, d_gw, d_gw_last;
-  // Two contractions of the same length in one launch (an epilogue with for_second(), one work item per workgroup): output tiles from nout0 on
-  // are the second's
+  // Two contractions of the same rows (an epilogue with kExperts): output tiles from nout0 on are the second's
   GemmOperand P1, Q1;
   int nout0, p_fast1, nfast1;
   FastDiv d_nfast1;
-  // Contractions over segments of the rows (an epilogue with kExperts): group e's is seg[e] .. seg[e + 1] in rows, multiples of 128. A workgroup
-  // has one output tile of one group: XCD x tiles x ipx .. of the group with the most rows, then of the next
+  // over segments of them: group e's is seg[e] .. seg[e + 1], multiples of 128 rows. A workgroup has one output tile of one group:
+  // XCD x tiles x ipx .. of the group with the most rows, then of the next
   const int* seg;
   int ngroups;
   FastDiv d_ipx;
@@ -85,20 +84,6 @@ template <class T, class = void>
 struct has_experts : std::false_type {};
 template <class T>
 struct has_experts<T, std::void_t<decltype(T::kExperts)>> : std::true_type {};
-template <class T, class = void>
-struct has_second : std::false_type {};
-template <class T>
-struct has_second<T, std::void_t<decltype(std::declval<const T&>().for_second())>> : std::true_type {};
-// EpiSplit of two outputs: a split's slab holds the first's partials, then the second's
-struct EpiSplitTwo : EpiSplit {
-  long n0, ld1;
-  __device__ __forceinline__ EpiSplitTwo for_second() const {
-    EpiSplitTwo e = *this;
-    e.ws += n0;
-    e.ld = ld1;
-    return e;
-  }
-};
 
 // Epilogue protocol of this kernel (every epilogue of the library rounds f(accumulator) to bf16 first):
 //   float pre(float acc)                      applied to every accumulator before its rounding to bf16;
@@ -215,10 +200,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     group_k0 = __builtin_amdgcn_readfirstlane(a.seg[group]) / 128;
     group_nkt = __builtin_amdgcn_readlane(rows, group) / 128;
     epi_in = epi_in.for_group(group);
-  }
-  if constexpr (has_second<Epi>::value) {
-    const int item = has_experts<Epi>::value ? group_tile : (int)((blockIdx.x & 7) * a.ipx + (blockIdx.x >> 3));
-    if (item - fastdiv(item, a.d_nout) * a.nout >= a.nout0) {
+    if (group_tile >= a.nout0) {
       first = a.nout0;
       a.P = a.P1;
       a.Q = a.Q1;
@@ -237,7 +219,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       split = fastdiv(w, a.d_nout);
       w -= split * a.nout;
     }
-    if constexpr (has_second<Epi>::value) w -= first;
+    if constexpr (has_experts<Epi>::value) w -= first;
     int fast, slow;
     if (a.rect) {
       const int x = w & 7, j = w >> 3;
@@ -762,47 +744,6 @@ static inline int gemm_pp_fewtile_splits(long t256, long nkt, long out_elems, lo
   int c = t256 * 8 <= cus ? 8 * (int)(cus / 8 / t256) : (int)(cus / t256);
   while (c > 1 && (nkt / c < 16 || (long)c * out_elems * 4 > ws_bytes)) --c;
   return (c > 1 && (double)(t256 * c) >= 0.8 * (double)cus) ? c : 0;
-}
-
-// Two weight gradients of one length of contraction, O_i x D_i over kbytes of strided fp8 (P_i e4m3, Q_i e5m2), as one launch of
-// `splits` k ranges; their partials side by side in ws. The partials are written and read again, and two launches of few tiles need twice the
-// ranges of one: 16384 rows, 768 x 3072 (36 tiles each): 7 ranges each -> 3 of both, 132 MB -> 57 MB each way.
-static int gemm_pp_launch_two(GemmOperand P0, GemmOperand Q0, int np0, int nq0, GemmOperand P1, GemmOperand Q1, int np1, int nq1, long kbytes,
-                              int splits, float* ws, hipStream_t stream) {
-  if (np0 <= 0 || nq0 <= 0 || np1 <= 0 || nq1 <= 0 || (np0 | nq0 | np1 | nq1) % 256 || kbytes % 128 || splits < 2 || kbytes / 128 / splits < 2)
-    return TFB_ERR_SHAPE;
-  for (const GemmOperand& o : {P0, Q0, P1, Q1}) {
-    if (o.ld <= 0 || o.ld > (1L << 28)) return TFB_ERR_SHAPE;
-    if (((uintptr_t)o.base | (uintptr_t)o.ld) & 15) return TFB_ERR_ARG;
-  }
-  const long t0 = (long)(np0 / 256) * (nq0 / 256), t1 = (long)(np1 / 256) * (nq1 / 256);
-  if ((t0 + t1) * splits > tfb_resident_slots(1)) return TFB_ERR_SHAPE;
-  PpArgs a = {};
-  a.P = P0;
-  a.Q = Q0;
-  a.P1 = P1;
-  a.Q1 = Q1;
-  a.splits = splits;
-  a.nk_total = (int)(kbytes / 128);
-  a.nout0 = (int)t0;
-  a.nout = (int)(t0 + t1);
-  a.ntiles = a.nout * splits;
-  a.ipx = (a.ntiles + 7) / 8;
-  a.nwg = 8 * a.ipx;
-  a.p_fast = np0 <= nq0;
-  a.nfast = (a.p_fast ? np0 : nq0) / 256;
-  a.p_fast1 = np1 <= nq1;
-  a.nfast1 = (a.p_fast1 ? np1 : nq1) / 256;
-  a.R = a.GW = a.panel = a.gw_last = 1;
-  a.d_nfast = fastdiv_make(a.nfast);
-  a.d_nfast1 = fastdiv_make(a.nfast1);
-  a.d_panel = a.d_gw = a.d_gw_last = fastdiv_make(1);
-  a.d_nout = fastdiv_make(a.nout);
-  const long n0 = (long)np0 * nq0, n1 = (long)np1 * nq1;
-  EpiSplitTwo e{{ws, (long)np0, n0 + n1}, n0, (long)np1};
-  hipLaunchKernelGGL((gemm_pp_kernel<1, TFB_FMT_E4M3, TFB_FMT_E5M2, TFB_K_STRIDED, TFB_K_STRIDED, EpiSplitTwo>), dim3(a.nwg), dim3(512), 0, stream, a, e);
-  TFB_LAUNCH_CHECK();
-  return TFB_OK;
 }
 
 // Two weight gradients of each of `groups` experts over its rows: P_i e4m3, Q_i e5m2, row segments seg (device, multiples of 128 rows). The

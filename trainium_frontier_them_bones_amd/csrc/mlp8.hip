@@ -1068,22 +1068,11 @@ extern "C" int tfb_mlp8_fwd_res(const void* x8, const void* w8, const void* row,
   return tfb_mlp8_fwd_res_rows(x8, w8, row, res, y, r, h8, M, M, d, F, stream);
 }
 
-// k ranges of the two weight gradients of an F x d MLP over M rows as one launch of the persistent kernel: as many as give every CU one
-// work item at most; 0 where that leaves more than a fifth of the CUs idle, a range has fewer than 16 k-tiles, or there are fewer than 48
-// in all (us, two launches or ring jobs -> this: 768 x 3072, 6144 rows 53 -> 48, 8192 69 -> 55, 16384 115 -> 93, 32768 174 -> 161; 1024 x
-// 4096, 4096 rows 51.4 -> 52.8, 6144 76 -> 66, 8192 102 -> 78, 16384 258 -> 127; 512 x 2048, 16384 rows 61 -> 51).
-static int dw8_two_splits(long M, int d, int F, long workspace_bytes) {
-  if (!TFB_PP || d % 256 || F % 256 || M / 128 < 48) return 0;
-  const long cus = tfb_resident_slots(1), tiles = 2L * (F / 256) * (d / 256), c = cus / tiles;
-  if (c < 2 || M / 128 / c < 16 || c * 2 * F * (long)d * 4 > workspace_bytes) return 0;
-  return 10 * tiles * c >= 8 * cus ? (int)c : 0;
-}
-
 // The weight gradients of an MLP of M rows as ring jobs (see tfb_mlp8_dw8): j[0] dw_fc, j[1] dw_proj; false where either is no ring
-// launch by itself, or the persistent kernel's.
+// launch by itself, or the persistent kernel's (tfb_gemm_fp8_tn).
 typedef RingJob<TFB_K_STRIDED, TFB_K_STRIDED, 1, TFB_FMT_E4M3, TFB_FMT_E5M2, true, EpiDescaleStore> JobDw8;
 static int dw8_ranges(long M, int d, int F, long ws_bytes) {   // k ranges of either (one tile count), 0: not as jobs
-  if (M <= 0 || M > 0x7fffffffL || M % 128 || d % 128 || F % 128 || M / 128 >= 128 || dw8_two_splits(M, d, F, ws_bytes) || !gemm_ring_pick(d, F, M / 128, true)) return 0;
+  if (M <= 0 || M > 0x7fffffffL || M % 128 || d % 128 || F % 128 || M / 128 >= 128 || !gemm_ring_pick(d, F, M / 128, true)) return 0;
   return choose_splits((long)(d / 128) * (F / 128), (int)(M / 128), (long)d * F, ws_bytes);
 }
 static JobDw8 dw8_job(const void* g8, const void* a8, const float* s_g, const float* s_a, float imm, void* out, long M, int O, int D,
@@ -1135,19 +1124,6 @@ extern "C" int tfb_mlp8_dw8(const void* x8, const void* dp8, const void* hq8, co
   if (const int ranges = dw8_ranges(M, d, F, workspace_bytes))   // launches of few tiles: the two as jobs of one (2048 rows, 768 x 3072: 25.3 -> 20.7 us)
     return gemm_ring_jobs(dw8_job(dp8, x8, sc + SC_S_DP, (const float*)x_scale_dev, x_imm, dw_fc, M, F, d, out_f32, accumulate, ranges),
                           dw8_job(dy8, hq8, sc + SC_S_DY, sc + SC_S_H, 1.0f, dw_proj, M, d, F, out_f32, accumulate, ranges), (hipStream_t)stream);
-  hipStream_t s = (hipStream_t)stream;
-  if (const int sp = dw8_two_splits(M, d, F, workspace_bytes)) {
-    float* ws = (float*)workspace;
-    const long n = (long)F * d;
-    int st = gemm_pp_launch_two(GemmOperand{(const uint8_t*)x8, (long)d}, GemmOperand{(const uint8_t*)dp8, (long)F}, d, F,
-                                GemmOperand{(const uint8_t*)hq8, (long)F}, GemmOperand{(const uint8_t*)dy8, (long)d}, F, d, M, sp, ws, s);
-    if (st != TFB_OK) return st;
-    hipLaunchKernelGGL(splitk_reduce_two_kernel, dim3((unsigned)(2 * n / 1024)), dim3(256), 0, s, ws,
-                       SplitOut{dw_fc, sc + SC_S_DP, (const float*)x_scale_dev, x_imm}, SplitOut{dw_proj, sc + SC_S_DY, sc + SC_S_H, 1.0f}, n, n, sp,
-                       out_f32, accumulate);
-    TFB_LAUNCH_CHECK();
-    return TFB_OK;
-  }
   // dw_fc[f][dd] = sum_m dp8[m][f] x8[m][dd]: g = dp8 (e5m2), a = x8 (e4m3); x8's scale from the device when it lives there
   int st = tfb_gemm_fp8_tn(dp8, TFB_FMT_E5M2, x8, TFB_FMT_E4M3, sc + SC_S_DP, x_scale_dev, x_imm, dw_fc, M, F, d, out_f32, accumulate, workspace, workspace_bytes, stream);
   if (st != TFB_OK) return st;
