@@ -507,7 +507,10 @@ __global__ __launch_bounds__(256, 2) void attnD_dq_kernel(AttnT q, AttnT k, Attn
         slot_end();
       });
     }
-    for (int x = wave; x < 3; ++x) asm volatile("s_barrier" ::: "memory");  // the other wavefronts' halves
+    // The other wavefronts' halves. They read what this one's last loads bring (the first wavefront's share of the last K tile): those have
+    // to have landed before its next barrier. (Without the wait rare launches had 45 of a block's rows of dQ wrong.)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    for (int x = wave; x < 3; ++x) asm volatile("s_barrier" ::: "memory");
     bf16_t* dqp = dq.p + b * dq.sb + h * dq.sh + (long)myq * dq.st;
     store_grad_row<D>(dqa, scale, dqp, lh);
     if (lh == 0) {
