@@ -535,9 +535,14 @@ int bwd_launch(const void* q, const long* qs, const void* k, const long* ks, con
                const long* os, const void* go, const long* gos, void* dq, const long* dqs, void* dk, const long* dks, void* dv,
                const long* dvs, const float* lse, float* stats, int B, int H, int T, float scale, int nw, hipStream_t s) {
   const long rows = (long)B * H * T;
-  hipLaunchKernelGGL(attnD_dq_kernel<D>, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
-                     mk(go, gos), mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, nw, mk(o, os), lse);
-  TFB_LAUNCH_CHECK();
+  if (tfb_attn_dq_pair_applies(D, T, (long)B * H, ks, vs)) {
+    const int st = tfb_attn_dq_pair_impl(q, qs, k, ks, v, vs, o, os, go, gos, dq, dqs, lse, stats, B, H, T, D, scale, nullptr, nullptr, nw, s);
+    if (st != TFB_OK) return st;
+  } else {
+    hipLaunchKernelGGL(attnD_dq_kernel<D>, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
+                       mk(go, gos), mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, nw, mk(o, os), lse);
+    TFB_LAUNCH_CHECK();
+  }
   return tfb_attn_dkdv_impl(q, qs, k, ks, v, vs, go, gos, dk, dks, dv, dvs, stats, B, H, T, D, scale, nullptr, nullptr, nw, s);
 }
 

@@ -849,10 +849,15 @@ int tfb_attn64_bwd_impl(const void* q, const long* qs, const void* k, const long
                        stats, T, H, rows, 1.0f / scale);
     TFB_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(attn64_dq_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
-                     mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw,
-                     tfb_resident_slots(2), mk(o, os), lse);
-  TFB_LAUNCH_CHECK();
+  if (tfb_attn_dq_pair_applies(64, T, (long)B * H, ks, vs)) {
+    const int st = tfb_attn_dq_pair_impl(q, qs, k, ks, v, vs, o, os, go, gos, dq, dqs, lse, stats, B, H, T, 64, scale, cos_t, sin_t, nw, s);
+    if (st != TFB_OK) return st;
+  } else {
+    hipLaunchKernelGGL(attn64_dq_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
+                       mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw,
+                       tfb_resident_slots(2), mk(o, os), lse);
+    TFB_LAUNCH_CHECK();
+  }
   // Few key blocks: pairs of wavefronts (one workgroup of eight wavefronts on a CU, two on each SIMD) in place of one or two workgroups of
   // four, up to one and a half blocks for each CU, and up to two where the blocks of a sequence are twelve or more: the longest then sets
   // the time (dQ and dK/dV, us, that kernel -> pairs: T2048 192 blocks 76 -> 68, 384 81 -> 72, 512 88 -> 86, T4096 384 148 -> 130, T8192

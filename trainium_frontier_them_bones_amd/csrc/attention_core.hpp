@@ -11,6 +11,19 @@ static inline bool tfb_attn_dkdv_strides_ok(const long* qs, const long* gos) {
   return qs[2] >= 0 && qs[2] < (1L << 25) && gos[2] >= 0 && gos[2] < (1L << 25);
 }
 
+// dQ and the row statistics by pairs of wavefronts, 64 queries a workgroup (attention_dq.hip). The same holds of its loads.
+int tfb_attn_dq_pair_impl(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, const void* o,
+                          const long* os, const void* go, const long* gos, void* dq, const long* dqs, const float* lse, float* stats, int B, int H,
+                          int T, int D, float scale, const void* cos_t, const void* sin_t, int nw, hipStream_t s);
+// Where: up to one 128-query block for each CU, or one and a half (D = 64) where a sequence has twelve or more: the longest block then sets
+// the time. dQ and dK/dV, us, one wavefront to 32 queries -> pairs, D = 64: T2048 192 blocks 69 -> 61, 64 blocks 63 -> 53, 384 blocks 73 ->
+// 73, 576 94 -> 99; T1920 360 70 -> 66; T4096 384 129 -> 123; T1024 192 40 -> 36; T512 256 27.4 -> 26.1; T384 288 28.8 -> 31.3; T128 80
+// 13.3 -> 12.5; D = 128: T2048 128 blocks 103 -> 84, 256 107 -> 96; T1664 312 99 -> 99; T1920 600 162 -> 188; T384 36 34 -> 30, 288 47.6 -> 54.
+static inline bool tfb_attn_dq_pair_applies(int D, int T, long nbh, const long* ks, const long* vs) {
+  const long nx = T / 128, blocks = nx * nbh, cus = tfb_resident_slots(1);
+  return 2 * blocks <= (D == 64 && nx >= 12 ? 3 : 2) * cus && tfb_attn_dkdv_strides_ok(ks, vs);
+}
+
 namespace {
 
 struct AttnT {
