@@ -860,7 +860,7 @@ int tfb_attn64_bwd_impl(const void* q, const long* qs, const void* k, const long
   }
   // Few key blocks: pairs of wavefronts (one workgroup of eight wavefronts on a CU, two on each SIMD) in place of one or two workgroups of
   // four, up to one and a half blocks for each CU, and up to two where the blocks of a sequence are twelve or more: the longest then sets
-  // the time (dQ and dK/dV, us, that kernel -> pairs: T2048 192 blocks 76 -> 68, 384 81 -> 72, 512 88 -> 86, T4096 384 148 -> 130, T8192
+  // the time (us, that kernel -> pairs, with a dQ launch of one wavefront to 32 queries: T2048 192 blocks 76 -> 68, 384 81 -> 72, 512 88 -> 86, T4096 384 148 -> 130, T8192
   // 128 258 -> 220, T1024 320 47 -> 43, T512 64 26.4 -> 24.6; beyond, T768 432 41.9 -> 44.5, T3072 576 132 -> 134, T256 384 25.7 ->
   // 30.6; sequences of one block 12.7 -> 14.1).
   const long nx = T / 128, blocks = nx * B * H, cus = tfb_resident_slots(1);
