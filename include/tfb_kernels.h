@@ -429,6 +429,12 @@ int tfb_moe_mlp8_bwd_q(const void* dy8, const void* r, const void* w8, const voi
  * backward (moe_expert8_mlp, round2/source/train.py:10731), expert by expert. */
 int tfb_moe_dw8(const void* xs8, const void* dp8, const void* hq8, const void* dy8, const void* rows, float x_scale,
                 const void* seg, void* dw_fc, void* dw_proj, int E, int d, int F, int out_f32, int accumulate, void* stream);
+/* tfb_moe_dw8 told the rows rmax of the grouped buffers (tfb_moe_max_rows; 0: not known): both gradients of all experts in one
+ * launch where tfb_moe_dw8_one_launch_applies (0 = it does), else a launch for each; the same bits. */
+int tfb_moe_dw8_rows(const void* xs8, const void* dp8, const void* hq8, const void* dy8, const void* rows, float x_scale,
+                     const void* seg, void* dw_fc, void* dw_proj, int E, int d, int F, int out_f32, int accumulate, long rmax,
+                     void* stream);
+int tfb_moe_dw8_one_launch_applies(int E, int d, int F, long rmax);
 
 /* dw_fc [E][F][d] (+)= dpre_e^T xs_e, dw_proj [E][d][F] (+)= dys_e^T bf16(r_e^2) over each expert's row segment.
  * Replaces the per-expert weight_grads (round2/source/kernels/nki_mlp_fused8.py:706-711). */

@@ -167,3 +167,21 @@ def test_every_change_of_the_table_of_timed_entry_points_is_told_to_the_native_l
     t["a"] = []                                            # nothing is loaded for it
     assert "set_timed" not in _lib.native.__dict__
     t.clear()
+
+
+@pytest.mark.parametrize("E,d,F,rows,one", [
+    (8, 512, 1024, 64, False), (8, 512, 1024, 512, True),          # 128 tiles: half a round
+    (4, 256, 512, 128, False), (4, 256, 512, 256, False), (4, 256, 512, 1024, True), (2, 256, 256, 256, False), (2, 256, 256, 1024, True),
+    (8, 1024, 2816, 64, False), (8, 1024, 2816, 256, True), (8, 1024, 2816, 4096, True),
+    (8, 768, 1536, 128, False), (8, 768, 1536, 512, True),         # 288 tiles: a little more than a round
+    (16, 512, 1024, 1, True),                                      # exactly one
+    (8, 512, 1024, 0, True),                                       # rows not known
+    (8, 384, 1024, 4096, False), (8, 512, 1152, 4096, False), (65, 512, 1024, 4096, False)])   # not the kernel's
+def test_expert_gradients_run_as_one_launch_where_rows_and_tiles_fill_it(E, d, F, rows, one):
+    """The rule on sizes alone (256 CUs where there is no device to ask)."""
+    from trainium_frontier_them_bones_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built (run __graft_entry__.build())")
+    L = _lib.lib()
+    rmax = L.tfb_moe_max_rows(rows * E, E, 1) if rows else 0
+    assert (L.tfb_moe_dw8_one_launch_applies(E, d, F, rmax) == 0) == one

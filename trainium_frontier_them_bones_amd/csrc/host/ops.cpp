@@ -779,8 +779,8 @@ void moe_dw8(const Tensor& xs8, const Tensor& dp8, const Tensor& hq8, const Tens
   chk(xs8, U8), chk(dp8, U8), chk(hq8, U8), chk(dy8, U8), chk(rows, F32);
   const int64_t d = xs8.size(1), F = dp8.size(1);
   moe_dw_outputs(dw_fc, dw_proj, E, F, d, accumulate, out_dtype, xs8);
-  TFB_CALL(tfb_moe_dw8, ptr(xs8), ptr(dp8), ptr(hq8), ptr(dy8), ptr(rows), x_scale, ptr(tab.seg), ptr(dw_fc), ptr(dw_proj), E, d, F,
-           dw_fc.scalar_type() == F32, accumulate, stream());
+  TFB_CALL(tfb_moe_dw8_rows, ptr(xs8), ptr(dp8), ptr(hq8), ptr(dy8), ptr(rows), x_scale, ptr(tab.seg), ptr(dw_fc), ptr(dw_proj), E, d, F,
+           dw_fc.scalar_type() == F32, accumulate, xs8.size(0), stream());
 }
 
 void moe_dw(const Tensor& dpre, const Tensor& xs, const Tensor& dys, const Tensor& r, const MoeTab& tab, Tensor& dw_fc, Tensor& dw_proj,

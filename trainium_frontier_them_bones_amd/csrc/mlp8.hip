@@ -1283,15 +1283,43 @@ struct EpiExperts : EpiDescaleGrouped {  // both gradients', for the persistent 
 };
 }  // namespace
 
+// Both gradients of all experts as one launch of the persistent kernel (TFB_OK), or a launch of the 128 x 128 kernel for each; the same bits.
+// It needs whole 256 x 256 tiles, and an expert's rows must be enough for what its tiles cost beside the k-loop: a CU works on one of them at a
+// time (fill and store are its own), where two of the 128 x 128 tiles share it, four to each output, spread over more CUs. What matters is how far the
+// tiles fill their rounds of the CUs, and the rows per expert, of which the host knows the mean (tokens x choices / experts): the loads beyond
+// it are the router's. Measured, us, two launches -> one, operands and outputs out of the L2s, loads even (and skewed, two experts e^2 as likely):
+//   tiles    at few rows                                              at more
+//      4   256 rows 11.1 -> 12.1, 512 13.7 -> 14.2                     1024 19.0 -> 18.4
+//     16   256 11.7 -> 12.6 (13.5 -> 13.7), 512 14.4 -> 14.8           1024 20.0 -> 18.9 (28.2 -> 24.9)
+//     64   16 9.4 -> 11.3, 256 12.7 -> 13.3 (14.4 -> 14.5)             384 14.7 -> 14.4, 1024 21.4 -> 19.9 (28.9 -> 25.7)
+//    128   64 11.2 -> 12.8                                             192 14.2 -> 14.1, 512 18.5 -> 17.5 (26.8 -> 23.5)
+//    256   -                                                           16 15.3 -> 14.7, 128 17.9 -> 16.0, 2048 64 -> 43
+//    288   128 19.1 -> 22.5, 256 24.6 -> 24.8 (20.3 -> 22.4)           512 31.5 -> 28.5 (29.4 -> 25.6), 2048 69 -> 57
+//    352   64 18.9 -> 21.6                                             384 26.8 -> 26.3, 2048 66 -> 57
+//    704   64 29.0 -> 32.1 (30.4 -> 32.1)                              256 39.8 -> 38.1 (35.6 -> 37.2), 512 50.0 -> 45.5, 4096 239 -> 170
+//   1408   64 65.4 -> 69.9                                             192 86.5 -> 81.9, 1024 169 -> 136
+// Up to five eighths of a round the line falls from 512 rows with the tiles; a full round has none; a launch of more rounds starts at 128 rows,
+// or 256 where its rounds are less than three quarters full. With unknown rows: one launch.
+extern "C" int tfb_moe_dw8_one_launch_applies(int E, int d, int F, long rmax) {
+  if (!TFB_PP || E <= 0 || E > 64 || d <= 0 || F <= 0 || d % 256 || F % 256 || rmax < 0) return TFB_ERR_SHAPE;
+  if (rmax == 0) return TFB_OK;
+  const long tiles = 2L * E * (d / 256) * (F / 256), cus = tfb_resident_slots(1), rounds = (tiles + cus - 1) / cus, mean = std::max(rmax / E - 127, 0L);
+  long least = 0;
+  if (rounds > 1) least = 4 * tiles < 3 * rounds * cus ? 256 : 128;
+  else if (8 * tiles < 5 * cus) least = 512 - 512 * 8 * tiles / (5 * cus);
+  return mean >= least ? TFB_OK : TFB_ERR_SHAPE;
+}
+
 // The experts' two weight gradients in fp8 over each expert's row segment [seg[e], seg[e+1]) of the grouped byte buffers
 // (every segment a multiple of 128 rows): dw_fc [E][F][d] (+)= bf16((dp8_e^T @ xs8_e) / (s_dp[e] x_scale)), dw_proj [E][d][F]
 // (+)= bf16((dy8_e^T @ hq8_e) / (s_dy[e] s_h[e])), with the scales of rows fp32 [E][16] (the backward call's rows).
 // xs8 e4m3 (the gather's), dp8 e5m2 and hq8 e4m3 (tfb_moe_mlp8_bwd_q's), dy8 e5m2 (the backward's input bytes).
 // Replaces mlp8_weight_grads under its fp8 weight-gradient switch (round2/source/train.py:8209-8229) inside
 // moe_expert8_mlp's backward, expert by expert.
-extern "C" int tfb_moe_dw8(const void* xs8, const void* dp8, const void* hq8, const void* dy8, const void* rows, float x_scale,
-                           const void* seg, void* dw_fc, void* dw_proj, int E, int d, int F, int out_f32, int accumulate,
-                           void* stream) {
+// rmax = the rows of the grouped buffers, as tfb_moe_max_rows gives them (0: not known): what the host knows of the loads.
+extern "C" int tfb_moe_dw8_rows(const void* xs8, const void* dp8, const void* hq8, const void* dy8, const void* rows, float x_scale,
+                                const void* seg, void* dw_fc, void* dw_proj, int E, int d, int F, int out_f32, int accumulate, long rmax,
+                                void* stream) {
   if (!xs8 || !dp8 || !hq8 || !dy8 || !rows || !seg || !dw_fc || !dw_proj) return TFB_ERR_ARG;
   if (E <= 0 || d <= 0 || F <= 0 || d % 128 || F % 128 || !(x_scale > 0.f)) return TFB_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
@@ -1309,10 +1337,7 @@ extern "C" int tfb_moe_dw8(const void* xs8, const void* dp8, const void* hq8, co
   a.ntp = d / 128;
   EpiDescaleGrouped e1{EpiStore{dw_fc, (long)d, out_f32, accumulate}, (long)F * d, (const float*)rows, SC_S_DP, -1, 1.0f / x_scale};
   EpiDescaleGrouped e2{EpiStore{dw_proj, (long)F, out_f32, accumulate}, (long)F * d, (const float*)rows, SC_S_DY, SC_S_H, 1.0f};
-  // whole 256 x 256 tiles: both gradients as one launch of the persistent kernel, one tile of one expert a workgroup, the same bits (us, 8 experts
-  // 1024 x 2816, two launches of the 128 x 128 kernel -> this: 13000 rows to each of two experts and 1200 to the others 247 -> 185, 4200 to
-  // each 247 -> 172, 512 55 -> 49, 256 41 -> 39, 128 31 -> 34; 4 experts 768 x 3072, 4096 rows each 115 -> 94)
-  if (TFB_PP && d % 256 == 0 && F % 256 == 0 && E <= 64)
+  if (tfb_moe_dw8_one_launch_applies(E, d, F, rmax) == TFB_OK)
     return gemm_pp_launch_experts(a.P, a.Q, d, F, GemmOperand{(const uint8_t*)hq8, (long)F}, GemmOperand{(const uint8_t*)dy8, (long)d}, F, d,
                                   (const int*)seg, E, EpiExperts{e1, e2}, s);
   int st = gemm_launch_args<Cfg>(a, E, 1, LoadIdentity{}, LoadIdentity{}, e1, s);
@@ -1324,6 +1349,11 @@ extern "C" int tfb_moe_dw8(const void* xs8, const void* dp8, const void* hq8, co
   a.nq = d;
   a.ntp = F / 128;
   return gemm_launch_args<Cfg>(a, E, 1, LoadIdentity{}, LoadIdentity{}, e2, s);
+}
+extern "C" int tfb_moe_dw8(const void* xs8, const void* dp8, const void* hq8, const void* dy8, const void* rows, float x_scale,
+                           const void* seg, void* dw_fc, void* dw_proj, int E, int d, int F, int out_f32, int accumulate,
+                           void* stream) {
+  return tfb_moe_dw8_rows(xs8, dp8, hq8, dy8, rows, x_scale, seg, dw_fc, dw_proj, E, d, F, out_f32, accumulate, 0, stream);
 }
 
 // Per-expert weight gradients over the expert's row segment [seg[e], seg[e+1]) of the grouped buffers:
