@@ -10,6 +10,9 @@
 // whose place in a tile is known (addresses move on once a tile, accumulators alternate without copies).
 // One wavefront doing both -> pairs, us: D = 128 (340 registers, alone on its SIMD) B1 H8 T2048 66 -> 52; with dQ's launch B3 H8 T1664
 // 109 -> 98, B16 H6 T2048 435 -> 409, B2 H16 T4096 498 -> 466; D = 64 B1 H12 T2048 45 -> 35.6.
+// D = 128 has no other kernel: with dQ's launch, over 1 to 512 heads (up to 1536 blocks), pairs take 0.85 - 0.94 of the time at T4096 and T2048,
+// 0.89 - 0.97 at T1024 to T512, 0.93 - 1.00 at T384 (96 heads 46.1 -> 46.1), 0.96 - 0.99 at T256 (512 heads 117.8 -> 116.3), and 0.1 - 0.4 us more where a sequence is one
+// block (8 heads 22.2 -> 22.4, 256 30.4 -> 30.8, 512 55.5 -> 55.8).
 #include "attention_slots.hpp"
 
 namespace {
