@@ -185,3 +185,23 @@ def test_expert_gradients_run_as_one_launch_where_rows_and_tiles_fill_it(E, d, F
     L = _lib.lib()
     rmax = L.tfb_moe_max_rows(rows * E, E, 1) if rows else 0
     assert (L.tfb_moe_dw8_one_launch_applies(E, d, F, rmax) == 0) == one
+
+
+# dQ's and dK/dV's kernels by pairs of wavefronts (1, 2) where a launch's longest block sets the time: as many blocks as that holds for (B H T / 128),
+# and some more. A band leaves the blocks alike, so few of them fill the chip.
+@pytest.mark.parametrize("D,T,nw,counts", [
+    (64, 128, 0, [(128, 1), (192, 0)]), (64, 256, 0, [(128, 3), (192, 2), (384, 0)]), (64, 384, 0, [(384, 0)]), (64, 512, 0, [(192, 3), (384, 0)]),
+    (64, 1024, 0, [(288, 3), (384, 2), (448, 0)]), (64, 2048, 0, [(384, 3), (512, 2), (576, 0)]), (64, 4096, 0, [(384, 3), (512, 2), (576, 0)]),
+    (64, 2048, 1, [(128, 1), (192, 0), (384, 0)]), (64, 2048, 2, [(128, 3), (192, 2), (384, 0)]), (64, 2048, 8, [(192, 3), (256, 2), (320, 0)]),
+    (64, 640, 2, [(320, 0)]), (64, 1024, 2, [(192, 2)]), (64, 2048, 16, [(512, 2)]), (64, 2048, 99, [(512, 2)]),
+    (128, 128, 0, [(128, 3), (192, 2), (256, 2)]), (128, 256, 0, [(128, 3), (192, 2)]), (128, 1024, 0, [(256, 3), (320, 2)]),
+    (128, 2048, 0, [(288, 3), (384, 2)]), (128, 1024, 2, [(128, 3), (192, 2)]), (128, 2048, 8, [(128, 3), (256, 2)]),
+    (96, 2048, 0, [(16, 0)]), (64, 2050, 0, [(16, 0)])])
+def test_attention_runs_by_pairs_where_the_longest_block_sets_the_time(D, T, nw, counts):
+    """The rule on sizes alone (256 CUs where there is no device to ask)."""
+    from trainium_frontier_them_bones_amd import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built (run __graft_entry__.build())")
+    for blocks, want in counts:
+        got = sum(w for w in (1, 2) if _lib.lib().tfb_attn_bwd_pairs_applies(w, 1, blocks * 128 // T, T, D, nw) == 0)
+        assert got == want, blocks

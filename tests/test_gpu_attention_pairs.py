@@ -1,8 +1,10 @@
-"""dK and dV by pairs of wavefronts: the bits of one wavefront doing both, over the forms a call may have."""
+"""dK and dV by pairs of wavefronts, and dQ, over the forms a call may have. At D = 64, and for dQ at D = 128, a launch of many blocks runs one
+wavefront to 32 tokens, and a launch of few in pairs has its bits. dK and dV of D = 128 always run in pairs: there the launches say that the
+grid does not matter, and the comparison with fp32 is what holds the values."""
 import pytest
 import torch
 
-from trainium_frontier_them_bones_amd import ops
+from trainium_frontier_them_bones_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -17,15 +19,20 @@ def _grads(B, T, H, D, band, rope, qkv, do):
     return out
 
 
-# two blocks (the fewest that D = 64 has in pairs) and one (which it has not), odd and even numbers of blocks, bands of one block and more,
-# the most blocks: 1.5 per CU, and two per CU at twelve blocks a sequence. The other launch has so many that D = 64 runs one wavefront.
+# two blocks (the fewest that D = 64 has in pairs) and one (which it has not, nor has a band of one), odd and even numbers of blocks, bands,
+# and the most blocks: about one for each CU of short sequences and two of long ones, less for dQ. pairs: what runs in pairs at D = 64 and at
+# D = 128 (1 = dQ, 2 = dK and dV); of the other launch nothing may at D = 64.
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("T,H,band,rope", [(128, 3, 0, True), (256, 2, 0, True), (256, 2, 1, False), (384, 1, 0, False), (640, 2, 2, True), (1024, 3, 0, True),
-                                           (1152, 1, 3, False), (1536, 2, 0, True), (2048, 1, 1, False)])
-def test_key_and_value_gradients_in_pairs(T, H, band, rope, D):
+@pytest.mark.parametrize("T,H,band,rope,pairs", [
+    (128, 3, 0, True, (1, 3)), (256, 2, 0, True, (3, 3)), (256, 2, 1, False, (1, 3)), (384, 1, 0, False, (3, 3)), (640, 2, 2, True, (3, 3)),
+    (1024, 3, 0, True, (3, 3)), (1152, 1, 3, False, (3, 3)), (1536, 2, 0, True, (3, 3)), (2048, 1, 1, False, (1, 3)), (512, 64, 0, False, (2, 2)),
+    (2048, 19, 0, True, (3, 3)), (2048, 24, 0, False, (3, 2)), (2048, 33, 0, True, (2, 2)), (1024, 32, 2, False, (2, 2))])
+def test_key_and_value_gradients_in_pairs(T, H, band, rope, pairs, D):
     dev = torch.device("cuda:0")
     g = torch.Generator(device=dev).manual_seed(T + H + band)
     many = -(-4 * 256 * 128 // (T * H))
+    routes = [sum(w for w in (1, 2) if _lib.lib().tfb_attn_bwd_pairs_applies(w, n, H, T, D, band) == 0) for n in (1, many)]
+    assert routes == [pairs[D // 128], 0 if D == 64 else 2]
     qkv = torch.randn(1, T, 3 * H * D, generator=g, device=dev).bfloat16()
     do = torch.randn(1, T, H, D, generator=g, device=dev).bfloat16()
     tables = None

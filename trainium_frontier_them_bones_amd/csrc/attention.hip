@@ -18,7 +18,7 @@
 // Tensors are addressed by (batch, head, token) element strides with the head dimension
 // contiguous, so q/k/v may be thirds of a fused qkv [B,T,3C] buffer and o / dO are [B,T,H,D].
 #include <cstdlib>
-#include "common.hpp"
+#include "attention_core.hpp"
 
 namespace {
 bool strides_ok(const long* s) { return s[0] % 8 == 0 && s[1] % 8 == 0 && s[2] % 8 == 0; }
@@ -96,6 +96,14 @@ extern "C" int tfb_attn_bwd(const void* q, const long* qs, const void* k, const 
                             float scale, void* stream) {
   return tfb_attn_bwd_rope(q, qs, k, ks, v, vs, o, os, go, gos, dq, dqs, dk, dks, dv, dvs, lse, delta, nullptr, nullptr, B, H, T,
                            D, scale, stream);
+}
+
+// Whether a backward's dQ kernel (which 1) or its dK/dV kernel (2) is the one by pairs of wavefronts, for token strides that it takes.
+extern "C" int tfb_attn_bwd_pairs_applies(int which, int B, int H, int T, int D, int nw) {
+  if (which < 1 || which > 2 || B <= 0 || H <= 0 || T <= 0 || T % 128 || (D != 64 && D != 128) || nw < 0) return TFB_ERR_SHAPE;
+  const long st[3] = {0, 0, D}, nbh = (long)B * H;
+  const bool yes = which == 1 ? tfb_attn_dq_pair_applies(D, T, nbh, nw, st, st) : D == 128 || tfb_attn_dkdv_pair_applies(T, nbh, nw, st, st);
+  return yes ? TFB_OK : TFB_ERR_SHAPE;
 }
 
 // ---- attention backward for callers that cannot allocate --------------------------------------------------------------

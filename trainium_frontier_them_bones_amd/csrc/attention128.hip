@@ -535,7 +535,7 @@ int bwd_launch(const void* q, const long* qs, const void* k, const long* ks, con
                const long* os, const void* go, const long* gos, void* dq, const long* dqs, void* dk, const long* dks, void* dv,
                const long* dvs, const float* lse, float* stats, int B, int H, int T, float scale, int nw, hipStream_t s) {
   const long rows = (long)B * H * T;
-  if (tfb_attn_dq_pair_applies(D, T, (long)B * H, ks, vs)) {
+  if (tfb_attn_dq_pair_applies(D, T, (long)B * H, nw, ks, vs)) {
     const int st = tfb_attn_dq_pair_impl(q, qs, k, ks, v, vs, o, os, go, gos, dq, dqs, lse, stats, B, H, T, D, scale, nullptr, nullptr, nw, s);
     if (st != TFB_OK) return st;
   } else {

@@ -849,7 +849,7 @@ int tfb_attn64_bwd_impl(const void* q, const long* qs, const void* k, const long
                        stats, T, H, rows, 1.0f / scale);
     TFB_LAUNCH_CHECK();
   }
-  if (tfb_attn_dq_pair_applies(64, T, (long)B * H, ks, vs)) {
+  if (tfb_attn_dq_pair_applies(64, T, (long)B * H, nw, ks, vs)) {
     const int st = tfb_attn_dq_pair_impl(q, qs, k, ks, v, vs, o, os, go, gos, dq, dqs, lse, stats, B, H, T, 64, scale, cos_t, sin_t, nw, s);
     if (st != TFB_OK) return st;
   } else {
@@ -858,13 +858,7 @@ int tfb_attn64_bwd_impl(const void* q, const long* qs, const void* k, const long
                        tfb_resident_slots(2), mk(o, os), lse);
     TFB_LAUNCH_CHECK();
   }
-  // Few key blocks: pairs of wavefronts (one workgroup of eight wavefronts on a CU, two on each SIMD) in place of one or two workgroups of
-  // four, up to one and a half blocks for each CU, and up to two where the blocks of a sequence are twelve or more: the longest then sets
-  // the time (us, that kernel -> pairs, with a dQ launch of one wavefront to 32 queries: T2048 192 blocks 76 -> 68, 384 81 -> 72, 512 88 -> 86, T4096 384 148 -> 130, T8192
-  // 128 258 -> 220, T1024 320 47 -> 43, T512 64 26.4 -> 24.6; beyond, T768 432 41.9 -> 44.5, T3072 576 132 -> 134, T256 384 25.7 ->
-  // 30.6; sequences of one block 12.7 -> 14.1).
-  const long nx = T / 128, blocks = nx * B * H, cus = tfb_resident_slots(1);
-  if (nx > 1 && 2 * blocks <= (nx >= 12 ? 4 : 3) * cus && tfb_attn_dkdv_strides_ok(qs, gos))
+  if (tfb_attn_dkdv_pair_applies(T, (long)B * H, nw, qs, gos))
     return tfb_attn_dkdv_impl(q, qs, k, ks, v, vs, go, gos, dk, dks, dv, dvs, stats, B, H, T, 64, scale, cos_t, sin_t, nw, s);
   hipLaunchKernelGGL(attn64_dkdv_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
                      mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw, tfb_resident_slots(2));

@@ -1,6 +1,7 @@
 // What the attention kernels of both head dimensions share: operand views, MFMA and lane helpers, and the rules by which a
 // workgroup gets its blocks.
 #pragma once
+#include <algorithm>
 #include "common.hpp"
 
 // dK and dV by pairs of wavefronts (attention_dkdv.hip). Its loads address 32 tokens by a 32-bit offset.
@@ -15,13 +16,41 @@ static inline bool tfb_attn_dkdv_strides_ok(const long* qs, const long* gos) {
 int tfb_attn_dq_pair_impl(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, const void* o,
                           const long* os, const void* go, const long* gos, void* dq, const long* dqs, const float* lse, float* stats, int B, int H,
                           int T, int D, float scale, const void* cos_t, const void* sin_t, int nw, hipStream_t s);
-// Where: up to one 128-query block for each CU, or one and a half (D = 64) where a sequence has twelve or more: the longest block then sets
-// the time. dQ and dK/dV, us, one wavefront to 32 queries -> pairs, D = 64: T2048 192 blocks 69 -> 61, 64 blocks 63 -> 53, 384 blocks 73 ->
-// 73, 576 94 -> 99; T1920 360 70 -> 66; T4096 384 129 -> 123; T1024 192 40 -> 36; T512 256 27.4 -> 26.1; T384 288 28.8 -> 31.3; T128 80
-// 13.3 -> 12.5; D = 128: T2048 128 blocks 103 -> 84, 256 107 -> 96; T1664 312 99 -> 99; T1920 600 162 -> 188; T384 36 34 -> 30, 288 47.6 -> 54.
-static inline bool tfb_attn_dq_pair_applies(int D, int T, long nbh, const long* ks, const long* vs) {
-  const long nx = T / 128, blocks = nx * nbh, cus = tfb_resident_slots(1);
-  return 2 * blocks <= (D == 64 && nx >= 12 ? 3 : 2) * cus && tfb_attn_dkdv_strides_ok(ks, vs);
+// Pairs divide a block's work between twice the wavefronts and do a little more of it. That shortens a launch whose longest block sets the
+// time and not one whose blocks keep the SIMDs busy, so what counts is the work a CU has in units of the longest block. A causal
+// block i of nx has i + 1 tiles, a band leaves it nw at most: the blocks of a short sequence or a narrow band are nearly alike and fill the
+// chip with half as many as those of a long sequence.
+struct AttnLoad {
+  long longest, work, blocks;   // tiles of the longest block; of all blocks; how many they are
+};
+static inline AttnLoad attn_load(int T, long nbh, int nw) {
+  const long nx = T / 128, w = nw > 0 && nw < nx ? nw : nx;
+  return AttnLoad{w, nbh * (w * (w + 1) / 2 + (nx - w) * w), nbh * nx};
+}
+// dQ: half a block for each CU (its workgroups of 64 queries are twice the blocks and then have a CU each), or as much work as the line
+// below (D = 128 has one such workgroup on a CU, D = 64 two). dQ and dK/dV, us, one wavefront to 32 queries -> pairs, blocks in brackets:
+//   D = 64   T128 [128] 14.6 -> 14.5, [160] 14.8 -> 16.3; T256 [128] 20.0 -> 19.2, [192] 20.5 -> 21.1; T512 [192] 28.5 -> 27.8, [288] 30.5 -> 31.9;
+//            T1024 [288] 46.1 -> 43.2, [384] 47.9 -> 50.6; T2048 [384] 80.6 -> 79.7, [512] 87.2 -> 88.8; T4096 [384] 147 -> 139, [576] 168 -> 172;
+//            bands: 1 T2048 [192] 15.8 -> 17.1; 2 T2048 [128] 20.2 -> 19.3, [192] 21.0 -> 22.7; 4 T1024 [128] 28.4 -> 26.2, [256] 29.3 -> 30.8;
+//            8 T2048 [192] 44.2 -> 43.2, [320] 49.1 -> 52.6
+//   D = 128  T128 [128] 25.1 -> 23.5, [192] 27.1 -> 31.4; T256 [128] 30.9 -> 28.1, [192] 32.5 -> 34.8; T512 [160] 42.0 -> 40.3, [288] 49.9 -> 55.5;
+//            T1024 [256] 65.4 -> 60.8, [320] 69.9 -> 74.6; T2048 [288] 112 -> 110, [384] 120 -> 124; T4096 [320] 207 -> 198, [448] 234 -> 245;
+//            bands: 1 T2048 [192] 28.7 -> 32.9; 4 T1024 [128] 41.8 -> 36.7, [192] 43.1 -> 47.1; 8 T2048 [128] 62.7 -> 52.9, [256] 67.0 -> 73.7
+static inline bool tfb_attn_dq_pair_applies(int D, int T, long nbh, int nw, const long* ks, const long* vs) {
+  const AttnLoad l = attn_load(T, nbh, nw);
+  const long cus = tfb_resident_slots(1), line = D == 64 ? std::min(l.longest + 7, 16L) : std::min(l.longest + 7, 17L);
+  return (2 * l.blocks <= cus || (D == 64 ? 20 : 26) * l.work <= line * cus * l.longest) && tfb_attn_dkdv_strides_ok(ks, vs);
+}
+// dK/dV at D = 64 (a workgroup of eight wavefronts on a CU, in place of one or two of four): one block for each CU, or as much work as this line,
+// but not where every block is one tile. dQ and dK/dV, us, one or two workgroups of four -> pairs:
+//   T128 [64] 14.0 -> 15.3; T256 [192] 20.5 -> 20.3, [288] 25.1 -> 27.7; T512 [256] 29.1 -> 27.6, [320] 31.0 -> 32.3;
+//   T1024 [384] 47.9 -> 46.4, [448] 50.0 -> 51.4; T2048 [512] 87.2 -> 82.2, [576] 91.2 -> 98.0; T4096 [512] 160 -> 146, [576] 168 -> 169; bands:
+//   1 T2048 [128] 14.6 -> 15.8; 2 T2048 [256] 22.0 -> 21.6, [320] 30.9 -> 35.6; 4 T2048 [256] 29.8 -> 28.1, [320] 42.6 -> 46.2;
+//   8 T2048 [256] 45.5 -> 41.0, [320] 49.1 -> 51.9
+static inline bool tfb_attn_dkdv_pair_applies(int T, long nbh, int nw, const long* qs, const long* gos) {
+  const AttnLoad l = attn_load(T, nbh, nw);
+  const long cus = tfb_resident_slots(1);
+  return l.longest > 1 && (l.blocks <= cus || 32 * l.work <= std::min(l.longest + 20, 36L) * cus * l.longest) && tfb_attn_dkdv_strides_ok(qs, gos);
 }
 
 namespace {
