@@ -50,9 +50,6 @@
 #ifndef TFB_FWD64_WPE
 #define TFB_FWD64_WPE 2
 #endif
-#ifndef TFB_ATTN_DELTA_IN_DQ
-#define TFB_ATTN_DELTA_IN_DQ 1  // the dQ kernel makes the rows' -delta and -lse / scale itself (0: the separate pre-pass)
-#endif
 
 namespace {
 
@@ -333,40 +330,6 @@ __global__ __launch_bounds__(256, TFB_FWD64_WPE) void attn64_fwd_kernel(AttnT q,
     }
   if (lh == 0) lse[(long)bh * T + myq] = (m * sl2 + log2f(lt)) * LN2;  // m is the raw-score maximum
   __syncthreads();  // the stages are free for the partner block
-  }
-}
-
-// =========================================================================================== delta
-// stats[0][bh][t] = -sum_d dO * O (fp32 of the bf16 values); stats[1][bh][t] = -lse / scale; 4 lanes per row. Both are
-// the values the backward kernels start their dP and S accumulators from: the MFMAs then deliver dP - delta and
-// S - lse / scale, and P = exp2(scale log2(e) (S - lse / scale)) needs no further row term.
-__global__ __launch_bounds__(256) void attn64_delta_kernel(AttnT o, AttnT go, const float* __restrict__ lse,
-                                                           float* __restrict__ stats, int T, int H, long rows, float inv_scale) {
-  const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-  const long row = idx >> 2;
-  const int part = (int)(idx & 3);
-  if (row >= rows) return;
-  const int t = (int)(row % T);
-  const long bh = row / T;
-  const int b = (int)(bh / H), h = (int)(bh % H);
-  const bf16_t* op = o.p + b * o.sb + h * o.sh + (long)t * o.st + part * 16;
-  const bf16_t* gp = go.p + b * go.sb + h * go.sh + (long)t * go.st + part * 16;
-  float s = 0.f;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    u32x4 a = *(const u32x4*)(op + 8 * i);
-    u32x4 g = *(const u32x4*)(gp + 8 * i);
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      s += bflo(a[w]) * bflo(g[w]);
-      s += bfhi(a[w]) * bfhi(g[w]);
-    }
-  }
-  s += __shfl_xor(s, 1, 64);
-  s += __shfl_xor(s, 2, 64);
-  if (part == 0) {
-    stats[row] = -s;
-    stats[rows + row] = -lse[row] * inv_scale;
   }
 }
 
@@ -664,30 +627,25 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
     qf[s] = *(const bf16x8*)(qp + (long)myq * q.st + 16 * s + 8 * lh);
     gf[s] = *(const bf16x8*)(gp + (long)myq * go.st + 16 * s + 8 * lh);
   }
-  float myD, myL;
-  if (TFB_ATTN_DELTA_IN_DQ) {
-    // the row statistics of this wavefront's queries, made here (this kernel runs first) from the dO fragments it holds
-    // anyway and the same elements of O, and left in `stats` for the dK/dV kernel: -sum_d dO O and -lse / scale
-    const bf16_t* orow = o.p + b * o.sb + h * o.sh + (long)myq * o.st;
-    float dot = 0.f;
+  // the row statistics of this wavefront's queries, made here (this kernel runs first) from the dO fragments it holds
+  // anyway and the same elements of O, and left in `stats` for the dK/dV kernel: -sum_d dO O and -lse / scale, the values both kernels start
+  // their dP and S accumulators from. The MFMAs then deliver dP - delta and S - lse / scale, and P needs no further row term.
+  const bf16_t* orow = o.p + b * o.sb + h * o.sh + (long)myq * o.st;
+  float dot = 0.f;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const u32x4 ov = *(const u32x4*)(orow + 16 * s + 8 * lh);
-      const u32x4 gv = __builtin_bit_cast(u32x4, gf[s]);
+  for (int s = 0; s < 4; ++s) {
+    const u32x4 ov = *(const u32x4*)(orow + 16 * s + 8 * lh);
+    const u32x4 gv = __builtin_bit_cast(u32x4, gf[s]);
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        dot += bflo(ov[w]) * bflo(gv[w]);
-        dot += bfhi(ov[w]) * bfhi(gv[w]);
-      }
+    for (int w = 0; w < 4; ++w) {
+      dot += bflo(ov[w]) * bflo(gv[w]);
+      dot += bfhi(ov[w]) * bfhi(gv[w]);
     }
-    dot += __shfl_xor(dot, 32, 64);
-    myD = -dot;
-    myL = -lse[(long)bh * T + myq] * (1.0f / scale);   // (stored with the block's dQ at the end: a store here would sit in
-                                                       // front of the first tile's wait for its loads)
-  } else {
-    myD = stats[(long)bh * T + myq];
-    myL = stats[rows + (long)bh * T + myq];
   }
+  dot += __shfl_xor(dot, 32, 64);
+  const float myD = -dot;
+  const float myL = -lse[(long)bh * T + myq] * (1.0f / scale);   // (stored with the block's dQ at the end: a store here would sit
+                                                                     // in front of the first tile's wait for its loads)
 
   TileLoad<2> lk, lv;
   lk.init(kst, wave, lane);
@@ -816,7 +774,7 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
 
   bf16_t* dqp = dq.p + b * dq.sb + h * dq.sh + (long)myq * dq.st;
   store_grad_row(dqa, scale, dqp, cs, sn, myq, lh);
-  if (TFB_ATTN_DELTA_IN_DQ && lh == 0) {
+  if (lh == 0) {
     stats[(long)bh * T + myq] = myD;
     stats[rows + (long)bh * T + myq] = myL;
   }
@@ -844,11 +802,6 @@ int tfb_attn64_bwd_impl(const void* q, const long* qs, const void* k, const long
   const long rows = (long)B * H * T;
   // dQ first: it makes the row statistics of its own queries on the way (from fragments it loads anyway) and leaves them
   // for dK/dV, so no pass of its own reads O and dO for them (the separate pre-pass took 16.6 us at B16 H12 T2048)
-  if (!TFB_ATTN_DELTA_IN_DQ) {
-    hipLaunchKernelGGL(attn64_delta_kernel, dim3((unsigned)((rows * 4 + 255) / 256)), dim3(256), 0, s, mk(o, os), mk(go, gos), lse,
-                       stats, T, H, rows, 1.0f / scale);
-    TFB_LAUNCH_CHECK();
-  }
   if (tfb_attn_dq_pair_applies(64, T, (long)B * H, nw, ks, vs)) {
     const int st = tfb_attn_dq_pair_impl(q, qs, k, ks, v, vs, o, os, go, gos, dq, dqs, lse, stats, B, H, T, 64, scale, cos_t, sin_t, nw, s);
     if (st != TFB_OK) return st;

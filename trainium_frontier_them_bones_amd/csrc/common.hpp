@@ -12,8 +12,6 @@
 #define TFB_ERR_LAUNCH 3    // hipGetLastError() after the launch was not hipSuccess
 #define TFB_ERR_WORKSPACE 4 // workspace too small
 
-#define TFB_WAVE 64
-
 typedef uint16_t bf16_t;  // raw bf16 bits; arithmetic is always done in fp32
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));

@@ -90,14 +90,6 @@ struct has_experts<T, std::void_t<decltype(T::kExperts)>> : std::true_type {};
 //   void chunk(p, q, v [, vp] [, pre_t])      8 consecutive rounded outputs D[p .. p + 7][q] as four packed bf16 pairs
 //                                             (p % 8 == 0); with kPartner32 also the 8 values 32 outputs away (p ^ 32); with a
 //                                             pre_t / prefetch(p, q) the operand requested before the block was staged.
-// Plain bf16 store: out [q][ld] = bf16(D)
-struct EpiStoreBf16 {
-  bf16_t* out;
-  long ld;
-  __device__ __forceinline__ float pre(float x) const { return x; }
-  __device__ __forceinline__ void chunk(int p, int q, const u32x4& v) const { *(u32x4*)(out + (long)q * ld + p) = v; }
-};
-
 #ifdef PP_DBG
 __device__ unsigned long long pp_dbg[256 * 4];
 #endif

@@ -587,10 +587,6 @@ struct RingJob {
     a.nq = nq;
     a.nkt = (int)(kbytes / 128);
   }
-  // whether it would go through the ring by itself
-  bool applies() const {
-    return a.np > 0 && a.nq > 0 && a.np % 128 == 0 && a.nq % 128 == 0 && gemm_ring_pick(a.np, a.nq, a.nkt, LAYP_ == TFB_K_STRIDED && LAYQ_ == TFB_K_STRIDED) != 0;
-  }
   double bytes() const { return (double)(a.np / 128) * (a.nq / 64) * a.nkt * 24576; }   // through LDS, in tiles of 128 x 64
 };
 template <class Cfg_, class Job>

@@ -1068,10 +1068,9 @@ extern "C" int tfb_mlp8_fwd_res(const void* x8, const void* w8, const void* row,
   return tfb_mlp8_fwd_res_rows(x8, w8, row, res, y, r, h8, M, M, d, F, stream);
 }
 
-// The weight gradients of an MLP of M rows as ring jobs (see tfb_mlp8_dw8): j[0] dw_fc, j[1] dw_proj; false where either is no ring
-// launch by itself, or the persistent kernel's (tfb_gemm_fp8_tn).
+// The weight gradients of an MLP of M rows as ring jobs (tfb_mlp8_dw8, tfb_mlp8_bwd_dw8): both outputs have the same tiles and k ranges.
 typedef RingJob<TFB_K_STRIDED, TFB_K_STRIDED, 1, TFB_FMT_E4M3, TFB_FMT_E5M2, true, EpiDescaleStore> JobDw8;
-static int dw8_ranges(long M, int d, int F, long ws_bytes) {   // k ranges of either (one tile count), 0: not as jobs
+static int dw8_ranges(long M, int d, int F, long ws_bytes) {   // k ranges of either; 0: not as jobs (no ring launch by itself, or the persistent kernel's: tfb_gemm_fp8_tn)
   if (M <= 0 || M > 0x7fffffffL || M % 128 || d % 128 || F % 128 || M / 128 >= 128 || !gemm_ring_pick(d, F, M / 128, true)) return 0;
   return choose_splits((long)(d / 128) * (F / 128), (int)(M / 128), (long)d * F, ws_bytes);
 }
