@@ -427,7 +427,8 @@ struct EpiUp {  // pre = x8 @ wf8^T: r, h8
   float dq = 0.f, c = 0.f;  // sc[SC_DQ_FC], sc[SC_C_H], read once by prepare()
   // With c a power of two (what the scale search produces) r c is a bf16 value as r is, and min(r c, 15.375)^2 = min(r^2, (15.375 / c)^2)
   // c^2 with every product exact: one multiplication, one minimum, and the scale in the conversion, instead of two, one and a rounding.
-  // (4096 x 4096 x 1024 on the 128 x 128 kernel 29.6 -> 27.5 us; the kernel with the weights in registers is bound by its stores: 92)
+  // (4096 x 4096 x 1024 on the 128 x 128 kernel 29.6 -> 27.5 us; the kernel with the weights in registers is bound by its stores: 92. Ring launches:
+  // with the down-projection, 768 x 3072, 2048 rows 20.7 -> 20.3, 256 rows 11.1 -> 11.4, as of 128 to 640 rows at every width)
   float inv_c2 = 0.f, lim = 0.f;
   bool fast = false;
   __device__ __forceinline__ EpiUp for_group(int g) const {
