@@ -14,6 +14,10 @@
 // tile, and the epilogue (accumulators -> bf16 -> global, straight from registers: a lane pair exchange with
 // v_permlane32_swap gives every lane 8 consecutive outputs of a row) runs while those loads are in flight.
 //
+// Narrow tiles (192 x 256, 256 x 192) fill rounds of the CUs that 256 x 256 leaves part empty: an output of 768 columns is four tiles
+// of 192, so 16384 rows are 256 tiles instead of 192. The operand with 192 rows is the one of which a wavefront owns two halves; of the
+// second it then owns one MFMA tile, and the two blocks of that half share a cluster: six clusters a k-tile, every one 8 MFMAs.
+//
 // Fragment reads are inline assembly (ds_read_b128 with immediate offsets) with explicit s_waitcnt: left to the compiler,
 // every LDS read beside global -> LDS loads in flight would wait for vmcnt(0).
 //
@@ -30,10 +34,6 @@
 // fp32) and splitk_reduce_kernel finishes them.
 #pragma once
 #include "gemm_core.hpp"
-
-#ifndef TFB_PP_EARLYB
-#define TFB_PP_EARLYB 1  // a k-tile's first Q fragments requested in the previous k-tile's last MFMA cluster
-#endif
 
 typedef __attribute__((address_space(3))) uint8_t tfb_lds_u8;
 typedef unsigned tfb_u32x2 __attribute__((ext_vector_type(2)));
@@ -58,8 +58,8 @@ struct PpArgs {
   int ntiles;   // work items = output tiles * splits (item w: split w / nout, output tile w % nout)
   int nout;     // output tiles
   int splits;
-  int ipx;      // > 0 (few output tiles, one work item per workgroup): XCD x (= workgroup & 7) takes the ipx consecutive
-                // work items from x * ipx, so that an XCD's workgroups share one or two k ranges of the operands in its L2
+  int ipx;      // > 0 (k ranges of one round; slow tile rows that are no multiple of 8): XCD x (= workgroup & 7) takes the ipx consecutive
+                // work items from x * ipx, so that an XCD's workgroups share k ranges or slow rows of the operands in its L2
   FastDiv d_nout;
   int nwg;      // workgroups launched (a multiple of 8 when rect)
   int p_fast;   // the fast-walking operand is P
@@ -90,9 +90,6 @@ struct has_experts<T, std::void_t<decltype(T::kExperts)>> : std::true_type {};
 //   void chunk(p, q, v [, vp] [, pre_t])      8 consecutive rounded outputs D[p .. p + 7][q] as four packed bf16 pairs
 //                                             (p % 8 == 0); with kPartner32 also the 8 values 32 outputs away (p ^ 32); with a
 //                                             pre_t / prefetch(p, q) the operand requested before the block was staged.
-#ifdef PP_DBG
-__device__ unsigned long long pp_dbg[256 * 4];
-#endif
 typedef short tfb_s16x8 __attribute__((ext_vector_type(8)));
 template <int OFF>
 __device__ __forceinline__ tfb_s16x4 tfb_lds_read_tr64(uint32_t addr) {
@@ -115,16 +112,22 @@ struct has_split_f32 : std::false_type {};
 template <class T>
 struct has_split_f32<T, std::void_t<decltype(T::kSplitF32)>> : std::true_type {};
 
+// SHAPE: the output tile, rows of p x rows of q.
+#define TFB_PP_256x256 0
+#define TFB_PP_192x256 1
+#define TFB_PP_256x192 2
+
 // ES: element size (2: bf16, 1: OCP fp8 with FMTP / FMTQ = 0 e4m3, 1 e5m2 per side); LAYP / LAYQ: TFB_K_CONTIG or
 // TFB_K_STRIDED
-template <int ES, int FMTP, int FMTQ, int LAYP, int LAYQ, class Epi>
+template <int ES, int FMTP, int FMTQ, int LAYP, int LAYQ, class Epi, int SHAPE = TFB_PP_256x256>
 __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   constexpr bool kF32 = has_split_f32<Epi>::value;
-#ifdef PP_DBG
-  const unsigned long long c_start = __builtin_readcyclecounter();
-  unsigned long long c_epi = 0, c_loop = 0;
-  int n_tiles = 0;
-#endif
+  // X is the operand of which a wavefront owns up to 2 x 64 rows (wr), Y the one of which it owns 2 x 32 (wc)
+  constexpr bool NARROW = SHAPE != TFB_PP_256x256, QX = SHAPE == TFB_PP_256x192;
+  constexpr int TP = SHAPE == TFB_PP_192x256 ? 192 : 256, TQ = QX ? 192 : 256;
+  constexpr int LAYX = QX ? LAYQ : LAYP, LAYY = QX ? LAYP : LAYQ;
+  static_assert(!NARROW || (!kF32 && !has_experts<Epi>::value && !has_partner32<Epi>::value), "a narrow tile's half 1 has 32 rows of a wavefront");
+  static_assert(!NARROW || LAYX == TFB_K_CONTIG || ES == 2, "half a quarter of fp8 rows");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * 65536];
   __shared__ __attribute__((aligned(1024))) uint8_t stg_all[8 * 4096];  // epilogue staging, 4 KB per wavefront
   const int tid = threadIdx.x;
@@ -202,9 +205,9 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       epi_in = epi_in.for_second();
     }
   }
-  const Side sp = make_side(a.P, LAYP), sq = make_side(a.Q, LAYQ);
+  const Side sx = make_side(QX ? a.Q : a.P, LAYX), sy = make_side(QX ? a.P : a.Q, LAYY);
 
-  // work item -> operand addresses of its first k-tile (P side, Q side), output tile origin and split
+  // work item -> output tile origin and split
   auto tile_of = [&](int w, long& p0, long& q0, int& split) {
     split = 0;
     if (a.splits > 1) {
@@ -226,8 +229,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       slow = fastdiv(w, a.d_nfast);
       fast = w - slow * a.nfast;
     }
-    p0 = (long)(a.p_fast ? fast : slow) * 256;
-    q0 = (long)(a.p_fast ? slow : fast) * 256;
+    p0 = (long)(a.p_fast ? fast : slow) * TP;
+    q0 = (long)(a.p_fast ? slow : fast) * TQ;
   };
   auto krange = [&](int split, int& k0, int& n) {
     k0 = 0;
@@ -243,31 +246,38 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   };
   auto origin = [&](const Side& sd, long r0, int k0) { return sd.base + r0 * sd.tstep + (long)k0 * sd.kstep; };
 
-  // quarter (X: 0 P, 1 Q; half h) of stage S <- the k-tile at g (the side's address of that k-tile of the output tile)
-  auto dma = [&](int S, int X, int h, const uint8_t* g) {
-    const Side& sd = X ? sq : sp;
-    uint8_t* d = lds + S * 65536 + X * 32768 + h * 16384 + wave * 1024;
+  // quarter (X / Y, half h) of stage S <- the k-tile at g (the side's address of that k-tile of the output tile). The 64 rows of a
+  // narrow tile's X half 1: k-contiguous, the first instruction alone; k-strided, both with the lanes of the chunks beyond them off.
+  [[maybe_unused]] const bool in_half = ((lane & 15) ^ (4 * (lane >> 4))) < 8;
+  auto dma = [&](int S, int Y, int h, const uint8_t* g) __attribute__((always_inline)) {
+    const Side& sd = Y ? sy : sx;
+    uint8_t* d = lds + S * 65536 + Y * 32768 + h * 16384 + wave * 1024;
+    const bool half = NARROW && !Y && h;
+    if (half && LAYX == TFB_K_STRIDED && !in_half) return;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < (half && LAYX == TFB_K_CONTIG ? 1 : 2); ++i)
       __builtin_amdgcn_global_load_lds((tfb_glb_void_t*)(g + h * sd.hstep + i * sd.istep + (size_t)sd.v),
                                        (tfb_lds_void_t*)(d + i * 8192), 16, 0, 0);
   };
+  constexpr int NX1 = NARROW && LAYX == TFB_K_CONTIG ? 1 : 2;  // a wavefront's load instructions for X half 1
 
   // ---- fragment addresses (stage 0; the stage bit is toggled after every k-tile)
-  uint32_t ap[4], aq[4];
+  uint32_t ax[4], ay[4];
+  [[maybe_unused]] uint32_t ax1[4];  // of X half 1 of a narrow tile, where a wavefront's rows are wr * 32 ..
   {
     const uint32_t lbase = (uint32_t)(size_t)(tfb_lds_u8*)lds;
-    const int rp = wr * 64 + lr, rq = wc * 32 + lr;
+    const int rx = wr * 64 + lr, rx1 = wr * 32 + lr, ry = wc * 32 + lr;
     // k-contiguous, one address per k-step. bf16: k-step s (16 k) of a row is chunk 2 s + lh; fp8: k-step s (64 k) is
     // chunks 4 s + 2 lh, + 1: entry 2 s + u
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       const int c = ES == 2 ? 2 * s + lh : 4 * (s >> 1) + 2 * lh + (s & 1);
-      ap[s] = lbase + rp * 128 + (((c ^ tfb_kc_swz(rp)) & 7) << 4);
-      aq[s] = lbase + 32768 + rq * 128 + (((c ^ tfb_kc_swz(rq)) & 7) << 4);
+      ax[s] = lbase + rx * 128 + (((c ^ tfb_kc_swz(rx)) & 7) << 4);
+      ax1[s] = lbase + rx1 * 128 + (((c ^ tfb_kc_swz(rx1)) & 7) << 4);
+      ay[s] = lbase + 32768 + ry * 128 + (((c ^ tfb_kc_swz(ry)) & 7) << 4);
     }
     // k-strided: 16-lane group g4 reads rows 16 (g4 & 1) .. + 15 of an MFMA tile, k-group g4 >> 1; lane j of the group
-    // points at k-row j / 4 (of four consecutive k), rows 4 (j % 4) .. + 3. One address per 32-row tile (ap[0], ap[1]:
+    // points at k-row j / 4 (of four consecutive k), rows 4 (j % 4) .. + 3. One address per 32-row tile (ax[0], ax[1]:
     // the second tile's chunk index differs in bit 2, which the swizzle also touches, so it is not an immediate offset);
     // k-step s is 16 k-rows further (an immediate), the fragment's upper four k another 4 k-rows.
     const int g4 = lane >> 4, j = lane & 15, kq = j >> 2;
@@ -281,15 +291,17 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       const int p = row0 + 16 * (g4 & 1) + 8 * (j & 1), k8 = j >> 1;
       return (uint32_t)((32 * (g4 >> 1) + k8) * 128 + ((((p >> 4) ^ (2 * ((k8 >> 1) & 3))) << 4) | (p & 8)));
     };
-    if (LAYP == TFB_K_STRIDED) {
-      ap[0] = lbase + tr_addr(wr * 64);
-      ap[1] = lbase + tr_addr(wr * 64 + 32);
+    if (LAYX == TFB_K_STRIDED) {
+      ax[0] = lbase + tr_addr(wr * 64);
+      ax[1] = lbase + tr_addr(wr * 64 + 32);
+      ax1[0] = lbase + tr_addr(wr * 32);
     }
-    if (LAYQ == TFB_K_STRIDED) aq[0] = lbase + 32768 + tr_addr(wc * 32);
+    if (LAYY == TFB_K_STRIDED) ay[0] = lbase + 32768 + tr_addr(wc * 32);
   }
-  constexpr int NAP = LAYP == TFB_K_STRIDED ? 2 : 4, NAQ = LAYQ == TFB_K_STRIDED ? 1 : 4;  // addresses in use
+  // addresses in use
+  constexpr int NAX = LAYX == TFB_K_STRIDED ? 2 : 4, NAX1 = !NARROW ? 0 : LAYX == TFB_K_STRIDED ? 1 : 4, NAY = LAYY == TFB_K_STRIDED ? 1 : 4;
 
-  f32x16 acc[2][2][2];  // [P half][i][Q half]
+  f32x16 acc[2][2][2];  // [X half][i][Y half]
   // fragments: bf16 four k-steps of 16 (one 128-bit read each), fp8 two k-steps of 64 (two 128-bit reads each)
   typedef std::conditional_t<ES == 2, bf16x8, i32x4> r128_t;
   r128_t fa[2][4], fb0[4], fb1[4];
@@ -308,34 +320,44 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   constexpr int TR1 = ES == 2 ? 4096 : 2048, TR2 = 8192, TR3 = ES == 2 ? 12288 : 8192 + 2048;
   auto readA = [&](auto H) __attribute__((always_inline)) {
     constexpr int h = decltype(H)::value;
-    if constexpr (LAYP == TFB_K_CONTIG) {
+    if constexpr (NARROW && h) {
+      if constexpr (LAYX == TFB_K_CONTIG) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) fa[0][s] = tfb_lds_read128<16384, r128_t>(ax1[s]);
+      } else {
+        fa[0][0] = tr_frag(std::integral_constant<int, 16384>{}, ax1[0]);
+        fa[0][1] = tr_frag(std::integral_constant<int, 16384 + TR1>{}, ax1[0]);
+        fa[0][2] = tr_frag(std::integral_constant<int, 16384 + TR2>{}, ax1[0]);
+        fa[0][3] = tr_frag(std::integral_constant<int, 16384 + TR3>{}, ax1[0]);
+      }
+    } else if constexpr (LAYX == TFB_K_CONTIG) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        fa[0][s] = tfb_lds_read128<h * 16384, r128_t>(ap[s]);
-        fa[1][s] = tfb_lds_read128<h * 16384 + 4096, r128_t>(ap[s]);
+        fa[0][s] = tfb_lds_read128<h * 16384, r128_t>(ax[s]);
+        fa[1][s] = tfb_lds_read128<h * 16384 + 4096, r128_t>(ax[s]);
       }
     } else {
-      fa[0][0] = tr_frag(std::integral_constant<int, h * 16384>{}, ap[0]);
-      fa[1][0] = tr_frag(std::integral_constant<int, h * 16384>{}, ap[1]);
-      fa[0][1] = tr_frag(std::integral_constant<int, h * 16384 + TR1>{}, ap[0]);
-      fa[1][1] = tr_frag(std::integral_constant<int, h * 16384 + TR1>{}, ap[1]);
-      fa[0][2] = tr_frag(std::integral_constant<int, h * 16384 + TR2>{}, ap[0]);
-      fa[1][2] = tr_frag(std::integral_constant<int, h * 16384 + TR2>{}, ap[1]);
-      fa[0][3] = tr_frag(std::integral_constant<int, h * 16384 + TR3>{}, ap[0]);
-      fa[1][3] = tr_frag(std::integral_constant<int, h * 16384 + TR3>{}, ap[1]);
+      fa[0][0] = tr_frag(std::integral_constant<int, h * 16384>{}, ax[0]);
+      fa[1][0] = tr_frag(std::integral_constant<int, h * 16384>{}, ax[1]);
+      fa[0][1] = tr_frag(std::integral_constant<int, h * 16384 + TR1>{}, ax[0]);
+      fa[1][1] = tr_frag(std::integral_constant<int, h * 16384 + TR1>{}, ax[1]);
+      fa[0][2] = tr_frag(std::integral_constant<int, h * 16384 + TR2>{}, ax[0]);
+      fa[1][2] = tr_frag(std::integral_constant<int, h * 16384 + TR2>{}, ax[1]);
+      fa[0][3] = tr_frag(std::integral_constant<int, h * 16384 + TR3>{}, ax[0]);
+      fa[1][3] = tr_frag(std::integral_constant<int, h * 16384 + TR3>{}, ax[1]);
     }
   };
   // flip = 0x10000: the fragments of the OTHER stage (the next k-tile)
   auto readB = [&](auto H, r128_t(&fb)[4], uint32_t flip = 0) __attribute__((always_inline)) {
     constexpr int h = decltype(H)::value;
-    if constexpr (LAYQ == TFB_K_CONTIG) {
+    if constexpr (LAYY == TFB_K_CONTIG) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) fb[s] = tfb_lds_read128<h * 16384, r128_t>(aq[s] ^ flip);
+      for (int s = 0; s < 4; ++s) fb[s] = tfb_lds_read128<h * 16384, r128_t>(ay[s] ^ flip);
     } else {
-      fb[0] = tr_frag(std::integral_constant<int, h * 16384>{}, aq[0] ^ flip);
-      fb[1] = tr_frag(std::integral_constant<int, h * 16384 + TR1>{}, aq[0] ^ flip);
-      fb[2] = tr_frag(std::integral_constant<int, h * 16384 + TR2>{}, aq[0] ^ flip);
-      fb[3] = tr_frag(std::integral_constant<int, h * 16384 + TR3>{}, aq[0] ^ flip);
+      fb[0] = tr_frag(std::integral_constant<int, h * 16384>{}, ay[0] ^ flip);
+      fb[1] = tr_frag(std::integral_constant<int, h * 16384 + TR1>{}, ay[0] ^ flip);
+      fb[2] = tr_frag(std::integral_constant<int, h * 16384 + TR2>{}, ay[0] ^ flip);
+      fb[3] = tr_frag(std::integral_constant<int, h * 16384 + TR3>{}, ay[0] ^ flip);
     }
   };
   // the fragments pass through the wait as in/out operands, so that no MFMA that reads them is scheduled ahead of it
@@ -344,64 +366,62 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
                  : "+v"(fa[0][0]), "+v"(fa[0][1]), "+v"(fa[0][2]), "+v"(fa[0][3]), "+v"(fa[1][0]), "+v"(fa[1][1]),
                    "+v"(fa[1][2]), "+v"(fa[1][3]));
   };
+  auto waitA1 = [&]() {  // (X half 1 of a narrow tile: one tile of 32 rows)
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[0][0]), "+v"(fa[0][1]), "+v"(fa[0][2]), "+v"(fa[0][3]));
+  };
   auto waitB = [&](r128_t(&fb)[4]) {
     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fb[0]), "+v"(fb[1]), "+v"(fb[2]), "+v"(fb[3]));
   };
-  auto mma = [&](auto FIRST, auto HP, auto HQ, const r128_t(&fb)[4]) __attribute__((always_inline)) {
+  auto mma = [&](auto FIRST, auto HX, auto HY, const r128_t(&fb)[4]) __attribute__((always_inline)) {
     constexpr bool first = decltype(FIRST)::value;
-    constexpr int hp = decltype(HP)::value, hq = decltype(HQ)::value;
+    constexpr int hx = decltype(HX)::value, hy = decltype(HY)::value, NI = NARROW && hx ? 1 : 2;
     __builtin_amdgcn_s_setprio(1);
-    if constexpr (ES == 2) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s)
+    for (int s = 0; s < (ES == 2 ? 4 : 2); ++s)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          f32x16 c = acc[hp][i][hq];
-          if (first && s == 0) {
+      for (int i = 0; i < NI; ++i) {
+        f32x16 c = acc[hx][i][hy];
+        if (first && s == 0) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) c[e] = 0.f;
-          }
-          acc[hp][i][hq] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i][s], fb[s], c, 0, 0, 0);
+          for (int e = 0; e < 16; ++e) c[e] = 0.f;
         }
-    } else {
-#pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          f32x16 c = acc[hp][i][hq];
-          if (first && s == 0) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) c[e] = 0.f;
-          }
-          const i32x4 al = fa[i][2 * s], ah = fa[i][2 * s + 1], bl = fb[2 * s], bh = fb[2 * s + 1];
-          const i32x8 av = {al.x, al.y, al.z, al.w, ah.x, ah.y, ah.z, ah.w};
-          const i32x8 bv = {bl.x, bl.y, bl.z, bl.w, bh.x, bh.y, bh.z, bh.w};
+        // the P fragment is the MFMA's A operand
+        if constexpr (ES == 2) {
+          acc[hx][i][hy] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(QX ? fb[s] : fa[i][s], QX ? fa[i][s] : fb[s], c, 0, 0, 0);
+        } else {
+          const i32x4 xl = fa[i][2 * s], xh = fa[i][2 * s + 1], yl = fb[2 * s], yh = fb[2 * s + 1];
+          const i32x8 xv = {xl.x, xl.y, xl.z, xl.w, xh.x, xh.y, xh.z, xh.w};
+          const i32x8 yv = {yl.x, yl.y, yl.z, yl.w, yh.x, yh.y, yh.z, yh.w};
           // formats: 0 = e4m3, 1 = e5m2; E8M0 scale byte 127 = 2^0
-          acc[hp][i][hq] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv, c, FMTP, FMTQ, 0, 127, 0, 127);
+          acc[hx][i][hy] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(QX ? yv : xv, QX ? xv : yv, c, FMTP, FMTQ, 0, 127, 0, 127);
         }
-    }
+      }
     __builtin_amdgcn_s_setprio(0);
     // the MFMAs have no side effects: without a use here they may sink below the barriers that follow
-    asm volatile("" : "+v"(acc[hp][0][hq]), "+v"(acc[hp][1][hq]));
+    if constexpr (NI == 2) asm volatile("" : "+v"(acc[hx][0][hy]), "+v"(acc[hx][1][hy]));
+    else asm volatile("" : "+v"(acc[hx][0][hy]));
   };
   typedef std::integral_constant<int, 0> H0;
   typedef std::integral_constant<int, 1> H1;
 
   const Epi epi = epi_prepare(epi_in);
-  int w = blockIdx.x;
+  int w = blockIdx.x, w_step = a.nwg, w_end = a.ntiles;  // this workgroup's items: w, w + w_step, .. below w_end
   if constexpr (has_experts<Epi>::value) {
     w = group_tile;
+    w_end = 0;
   } else if (a.ipx > 0) {
-    if ((w >> 3) >= a.ipx) return;
-    w = (w & 7) * a.ipx + (w >> 3);
+    const int x0 = (w & 7) * a.ipx;
+    w = x0 + (w >> 3);
+    w_step = a.nwg >> 3;
+    w_end = x0 + a.ipx < a.ntiles ? x0 + a.ipx : a.ntiles;
+    if (w >= w_end) return;  // (whole workgroup)
   }
-  if (w >= a.ntiles) return;  // (whole workgroup)
   long p0, q0;
   int split, k0;
   tile_of(w, p0, q0, split);
   krange(split, k0, nkt);
-  const uint8_t* gp = origin(sp, p0, k0);  // current work item: the sides' addresses of its first k-tile
-  const uint8_t* gq = origin(sq, q0, k0);
+  const uint8_t* gx = origin(sx, QX ? q0 : p0, k0);  // current work item: the sides' addresses of its first k-tile
+  const uint8_t* gy = origin(sy, QX ? p0 : q0, k0);
 
   // A segment without rows: nothing is loaded, its product is zero.
   if constexpr (has_experts<Epi>::value) {
@@ -412,56 +432,62 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     }
   }
 
-  // ---- prologue: all of k-tile 0 into stage 0, three quarters of k-tile 1 into stage 1
-  dma(0, 1, 0, gq);
-  dma(0, 0, 0, gp);
-  dma(0, 1, 1, gq);
-  dma(0, 0, 1, gp);
+  // ---- prologue: all of k-tile 0 into stage 0, three quarters of k-tile 1 into stage 1 (narrow tiles: the two quarters 0)
+  dma(0, 1, 0, gy);
+  dma(0, 0, 0, gx);
+  dma(0, 1, 1, gy);
+  dma(0, 0, 1, gx);
   const long k_one = has_experts<Epi>::value && nkt < 2 ? 0 : 1;  // (a segment of one k-tile: that one again)
-  dma(1, 0, 0, gp + k_one * sp.kstep);
-  dma(1, 1, 0, gq + k_one * sq.kstep);
-  dma(1, 1, 1, gq + k_one * sq.kstep);
-  asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+  dma(1, 0, 0, gx + k_one * sx.kstep);
+  dma(1, 1, 0, gy + k_one * sy.kstep);
+  if constexpr (!NARROW) dma(1, 1, 1, gy + k_one * sy.kstep);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NARROW ? 4 : 6) : "memory");
   TFB_SBAR();               // k-tile 0 is there for everybody
   if (wr == 1) TFB_SBAR();  // group 1 runs one cluster behind from here on
 
-  // ---- epilogue of one 64 (p) x 32 (q) accumulator block, acc[hp][i][hq][4 jj + e] = D[pb + 32 i + 8 jj + 4 lh + e][qb + lr]:
-  // every accumulator goes through epi.pre() and is rounded to bf16, the block passes through the wavefront's own 4 KB of
-  // LDS (row q = 128 bytes, 16-byte chunk c at slot c ^ ((q >> 1) & 7): the 8-byte writes and the 16-byte reads then use
-  // the banks evenly), and every lane finishes 8 consecutive outputs of a row, a row's 64 outputs (128 bytes) on 8
-  // consecutive lanes: epi.chunk(p, q, v [, partner] [, prefetched]).
+  // ---- epilogue of one accumulator block, acc[hx][i][hy][4 jj + e] = D[pb + 8 jj + 4 lh + e][qb + lr] of MFMA tile i: every
+  // accumulator goes through epi.pre() and is rounded to bf16, the block passes through the wavefront's own 4 KB of LDS, and every
+  // lane finishes 8 consecutive outputs of a row: epi.chunk(p, q, v [, partner] [, prefetched]). Two forms:
+  //   64 p (X = P, two tiles): row q = 128 bytes, 16-byte chunk c at slot c ^ ((q >> 1) & 7) (the 8-byte writes and the 16-byte
+  //   reads then use the banks evenly), a row's 64 outputs on 8 consecutive lanes;
+  //   32 p: row q = 64 bytes, chunk c at slot c ^ ((q >> 2) & 3), a row's outputs on 4 lanes; X = Q: tile i is rows 32 i .. of q.
   constexpr bool kPrefetch = has_prefetch<Epi>::value;
-  auto store_block = [&](auto HP, auto HQ, long tp0, long tq0) __attribute__((always_inline)) {
-    constexpr int hp = decltype(HP)::value, hq = decltype(HQ)::value;
-    const int pb = (int)tp0 + hp * 128 + wr * 64, qb = (int)tq0 + hq * 128 + wc * 32;
-    const int ch = lane & 7, r8 = lane >> 3;
-    // the epilogue's own operand: all four chunks requested up front when that is 16 registers, else one ahead
+  auto store_block = [&](auto HX, auto HY, long tp0, long tq0) __attribute__((always_inline)) {
+    constexpr int hx = decltype(HX)::value, hy = decltype(HY)::value, NI = NARROW && hx ? 1 : 2;
+    constexpr bool wide = !QX && NI == 2;
+    const int x = hx * 128 + wr * (32 * NI), y = hy * 128 + wc * 32;
+    const int pb = (int)tp0 + (QX ? y : x), qb = (int)tq0 + (QX ? x : y);
+    constexpr int NCH = wide ? 4 : QX ? 2 * NI : 2, RSTEP = wide ? 8 : 16;  // chunks of a lane, rows apart
+    const int ch = wide ? lane & 7 : lane & 3, row0 = wide ? lane >> 3 : lane >> 2;
+    // the epilogue's own operand: all chunks requested up front when that is 16 registers, else one ahead
     typedef typename prefetch_type<Epi>::type pre_t;
-    constexpr int kAhead = sizeof(pre_t) <= 16 ? 4 : 1;
-    [[maybe_unused]] pre_t pre[4];
+    constexpr int kAhead = sizeof(pre_t) <= 16 ? NCH : 1;
+    [[maybe_unused]] pre_t pre[NCH];
     if constexpr (kPrefetch) {
 #pragma unroll
-      for (int k = 0; k < kAhead; ++k) pre[k] = epi.prefetch(pb + 8 * ch, qb + r8 + 8 * k);
+      for (int k = 0; k < kAhead; ++k) pre[k] = epi.prefetch(pb + 8 * ch, qb + row0 + RSTEP * k);
     }
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
-        const f32x16& c = acc[hp][i][hq];
+        const f32x16& c = acc[hx][i][hy];
         if constexpr (!kF32) {
           u32x2 v = {pack2bf(epi.pre(c[4 * jj + 0]), epi.pre(c[4 * jj + 1])),
                      pack2bf(epi.pre(c[4 * jj + 2]), epi.pre(c[4 * jj + 3]))};
-          *(u32x2*)(stg + lr * 128 + (((4 * i + jj) ^ ((lr >> 1) & 7)) << 4) + 8 * lh) = v;
+          if constexpr (wide) *(u32x2*)(stg + lr * 128 + (((4 * i + jj) ^ ((lr >> 1) & 7)) << 4) + 8 * lh) = v;
+          else *(u32x2*)(stg + (32 * i + lr) * 64 + ((jj ^ ((lr >> 2) & 3)) << 4) + 8 * lh) = v;
         }
       }
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int row = r8 + 8 * k;
-      const u32x4 v = *(const u32x4*)(stg + row * 128 + ((ch ^ ((row >> 1) & 7)) << 4));
+    for (int k = 0; k < NCH; ++k) {
+      const int row = row0 + RSTEP * k;
+      const u32x4 v = wide ? *(const u32x4*)(stg + row * 128 + ((ch ^ ((row >> 1) & 7)) << 4))
+                           : *(const u32x4*)(stg + row * 64 + ((ch ^ ((row >> 2) & 3)) << 4));
       const int p = pb + 8 * ch, q = qb + row;
-      if constexpr (kPrefetch && kAhead < 4) {
-        if (k + kAhead < 4) pre[k + kAhead] = epi.prefetch(pb + 8 * ch, qb + r8 + 8 * (k + kAhead));
+      if constexpr (kPrefetch) {
+        if (k + kAhead < NCH) pre[k + kAhead] = epi.prefetch(p, qb + row0 + RSTEP * (k + kAhead));
       }
       if constexpr (has_partner32<Epi>::value) {
         const u32x4 vp = *(const u32x4*)(stg + row * 128 + (((ch ^ 4) ^ ((row >> 1) & 7)) << 4));  // 32 outputs away
@@ -509,21 +535,21 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   };
 
   int S = 0;
-  if (TFB_PP_EARLYB) readB(H0{}, fb0);
+  readB(H0{}, fb0);
   bool have_prev = false;  // the previous tile's accumulators are still to be stored
   long pp0 = 0, pq0 = 0;   // its origin
   for (;;) {
     // the workgroup's next work item (its first k-tiles are requested by this one's last iterations); past the end: this
     // one again (loads nobody reads, from valid memory)
-    const int wn = a.ipx > 0 ? a.ntiles : w + a.nwg;
+    const int wn = w + w_step;
     long pn = p0, qn = q0;
     int splitn = split, k0n = k0, nktn = nkt;
-    if (wn < a.ntiles) {
+    if (wn < w_end) {
       tile_of(wn, pn, qn, splitn);
       krange(splitn, k0n, nktn);
     }
-    const uint8_t* gpn = origin(sp, pn, k0n);
-    const uint8_t* gqn = origin(sq, qn, k0n);
+    const uint8_t* gxn = origin(sx, QX ? qn : pn, k0n);
+    const uint8_t* gyn = origin(sy, QX ? pn : qn, k0n);
 
     // One k-tile. In a tile's first iteration the MFMAs start from zero, and each accumulator block of the PREVIOUS tile is
     // stored in the memory cluster in front of the MFMA cluster that overwrites it: the stores of one group (4 KB per
@@ -533,84 +559,118 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       // k positions one and two ahead in the workgroup's stream of k-tiles
       const bool in1 = kt + 1 < nkt, in2 = kt + 2 < nkt;
       const long k1 = in1 ? kt + 1 : 0, k2 = in2 ? kt + 2 : has_experts<Epi>::value && nkt < 2 ? 0 : kt + 2 - nkt;
-      const uint8_t* gp1 = (in1 ? gp : gpn) + k1 * sp.kstep;
-      const uint8_t* gp2 = (in2 ? gp : gpn) + k2 * sp.kstep;
-      const uint8_t* gq2 = (in2 ? gq : gqn) + k2 * sq.kstep;
-      // c0 (the Q fragments of half 0 were requested in the previous k-tile's c7)
-      if (!TFB_PP_EARLYB) readB(H0{}, fb0);
-      readA(H0{});
-      dma(S ^ 1, 0, 1, gp1);
-      if constexpr (!kF32) {
-        if (first && have_prev) store_block(H0{}, H0{}, pp0, pq0);
-      }
-      TFB_SBAR();
-      // c1
-      waitB(fb0);
-      waitA();
-      mma(FIRST, H0{}, H0{}, fb0);
-      TFB_SBAR();
-      // c2
-      readB(H1{}, fb1);
-      dma(S, 0, 0, gp2);
-      if constexpr (!kF32) {
-        if (first && have_prev) store_block(H0{}, H1{}, pp0, pq0);
-      }
-      TFB_SBAR();
-      // c3
-      waitB(fb1);
-      mma(FIRST, H0{}, H1{}, fb1);
-      TFB_SBAR();
-      // c4
-      readA(H1{});
-      dma(S, 1, 0, gq2);
-      if constexpr (!kF32) {
-        if (first && have_prev) store_block(H1{}, H0{}, pp0, pq0);
-      }
-      TFB_SBAR();
-      // c5
-      waitA();
-      mma(FIRST, H1{}, H0{}, fb0);
-      if (TFB_PP_EARLYB) {
+      const uint8_t* gx1 = (in1 ? gx : gxn) + k1 * sx.kstep;
+      const uint8_t* gx2 = (in2 ? gx : gxn) + k2 * sx.kstep;
+      const uint8_t* gy2 = (in2 ? gy : gyn) + k2 * sy.kstep;
+      auto store = [&](auto HX, auto HY) __attribute__((always_inline)) {
+        if constexpr (!kF32) {
+          if (first && have_prev) store_block(HX, HY, pp0, pq0);
+        }
+      };
+      if constexpr (!NARROW) {
+        // c0 (the Y fragments of half 0 were requested in the previous k-tile's c7)
+        readA(H0{});
+        dma(S ^ 1, 0, 1, gx1);
+        store(H0{}, H0{});
+        TFB_SBAR();
+        // c1
+        waitB(fb0);
+        waitA();
+        mma(FIRST, H0{}, H0{}, fb0);
+        TFB_SBAR();
+        // c2
+        readB(H1{}, fb1);
+        dma(S, 0, 0, gx2);
+        store(H0{}, H1{});
+        TFB_SBAR();
+        // c3
+        waitB(fb1);
+        mma(FIRST, H0{}, H1{}, fb1);
+        TFB_SBAR();
+        // c4
+        readA(H1{});
+        dma(S, 1, 0, gy2);
+        store(H1{}, H0{});
+        TFB_SBAR();
+        // c5
+        waitA();
+        mma(FIRST, H1{}, H0{}, fb0);
         // Completion is reported in issue order, stores included. Everything up to the quarter requested in c0 has to be
         // there one cluster before the other group's matching wait: all but the two quarters requested since (4
         // instructions), and in a first iteration with stores all but those and the 12 stores (c0's four were issued
         // behind its loads). After the barrier that ends c6 both groups have waited, so the next k-tile is complete.
         if (!kF32 && first && have_prev) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
         else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-      }
-      TFB_SBAR();
-      // c6
-      dma(S, 1, 1, gq2);
-      if (!kF32 && first && have_prev) {
-        if constexpr (!kF32) store_block(H1{}, H1{}, pp0, pq0);
-        if (!TFB_PP_EARLYB) asm volatile("s_waitcnt vmcnt(22)" ::: "memory");
+        TFB_SBAR();
+        // c6
+        dma(S, 1, 1, gy2);
+        store(H1{}, H1{});
+        TFB_SBAR();
+        // c7: the next k-tile's first Y fragments are requested under this cluster's MFMAs (fb0 was last read in c5)
+        readB(H0{}, fb0, 0x10000u);
+        mma(FIRST, H1{}, H1{}, fb1);
+        TFB_SBAR();
       } else {
-        if (!TFB_PP_EARLYB) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+        // X half 1 is one MFMA tile a wavefront: three MFMA clusters of 8 instead of four. Quarters 0 are requested two k-tiles
+        // ahead, quarters 1 one ahead. A cluster's reads are waited for in front of its barrier (the requests behind them take longer),
+        // so a quarter is requested again only when a barrier has passed since either group had the old one in registers.
+        const uint8_t* gy1 = (in1 ? gy : gyn) + k1 * sy.kstep;
+        // c0 (Y half 0: see c5)
+        readA(H0{});
+        dma(S ^ 1, 1, 1, gy1);
+        dma(S ^ 1, 0, 1, gx1);
+        store(H0{}, H0{});
+        waitB(fb0);
+        waitA();
+        TFB_SBAR();
+        // c1
+        mma(FIRST, H0{}, H0{}, fb0);
+        TFB_SBAR();
+        // c2
+        readB(H1{}, fb1);
+        store(H0{}, H1{});
+        waitB(fb1);
+        TFB_SBAR();
+        // c3
+        mma(FIRST, H0{}, H1{}, fb1);
+        // The next k-tile's quarters 0 (requested in the previous iteration's c4) have to be there: all but what was requested
+        // since, c0's loads and in a first iteration with stores the 8 stores of c0 and c2. c5 reads them behind two more barriers.
+        if (first && have_prev) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + NX1 + 8) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + NX1) : "memory");
+        TFB_SBAR();
+        // c4
+        readA(H1{});
+        dma(S, 0, 0, gx2);
+        dma(S, 1, 0, gy2);
+        store(H1{}, H0{});
+        store(H1{}, H1{});
+        waitA1();
+        TFB_SBAR();
+        // c5
+        mma(FIRST, H1{}, H0{}, fb0);
+        readB(H0{}, fb0, 0x10000u);
+        mma(FIRST, H1{}, H1{}, fb1);
+        // The next k-tile's quarters 1 (c0) likewise: all but c4's four loads, and with stores the 8 of c0 and c2 and c4's 4.
+        if (first && have_prev) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        TFB_SBAR();
       }
-      TFB_SBAR();
-      // c7: the next k-tile's first Q fragments are requested under this cluster's MFMAs (fb0 was last read in c5)
-      if (TFB_PP_EARLYB) readB(H0{}, fb0, 0x10000u);
-      mma(FIRST, H1{}, H1{}, fb1);
-      TFB_SBAR();
       S ^= 1;
 #pragma unroll
-      for (int s = 0; s < NAP; ++s) ap[s] ^= 0x10000u;
+      for (int s = 0; s < NAX; ++s) ax[s] ^= 0x10000u;
 #pragma unroll
-      for (int s = 0; s < NAQ; ++s) aq[s] ^= 0x10000u;
+      for (int s = 0; s < NAX1; ++s) ax1[s] ^= 0x10000u;
+#pragma unroll
+      for (int s = 0; s < NAY; ++s) ay[s] ^= 0x10000u;
     };
-#ifdef PP_DBG
-    const unsigned long long c_l0 = __builtin_readcyclecounter();
-#endif
     iter(std::true_type{}, 0);
-#ifdef PP_DBG
-    const unsigned long long c_e0 = __builtin_readcyclecounter();
-    c_epi += c_e0 - c_l0;
-#endif
-    for (int kt = 1; kt < nkt; ++kt) iter(std::false_type{}, kt);
-#ifdef PP_DBG
-    c_loop += __builtin_readcyclecounter() - c_e0;
-    ++n_tiles;
-#endif
+    if constexpr (has_experts<Epi>::value) {
+      for (int kt = 1; kt < nkt; ++kt) iter(std::false_type{}, kt);
+    } else {
+      int kt = 1;
+      do iter(std::false_type{}, kt);
+      while (++kt < nkt);
+    }
     if constexpr (kF32) {
       // a k-split's partial tile: stored here, both groups together (a work item is hundreds of k-tiles long)
       if (wr == 0) TFB_SBAR();  // group 0 waits for group 1's last cluster
@@ -624,14 +684,14 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       pq0 = q0;
     }
     w = wn;
-    if (w >= a.ntiles) break;
+    if (w >= w_end) break;
     p0 = pn;
     q0 = qn;
     split = splitn;
     k0 = k0n;
     nkt = nktn;
-    gp = gpn;
-    gq = gqn;
+    gx = gxn;
+    gy = gyn;
     if constexpr (kF32) {
       if (wr == 1) TFB_SBAR();  // group 1 falls one cluster behind again
     }
@@ -643,18 +703,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     store_block(H1{}, H0{}, pp0, pq0);
     store_block(H1{}, H1{}, pp0, pq0);
   }
-#ifdef PP_DBG
-  if (tid == 0 && blockIdx.x < 256) {
-    pp_dbg[blockIdx.x * 4 + 0] = __builtin_readcyclecounter() - c_start;
-    pp_dbg[blockIdx.x * 4 + 1] = c_loop;
-    pp_dbg[blockIdx.x * 4 + 2] = c_epi;
-    pp_dbg[blockIdx.x * 4 + 3] = n_tiles;
-  }
-#endif
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stream's last (unused) loads must have landed before LDS is released
 }
 
-// Shapes this kernel takes: np, nq multiples of 256, at least two k-tiles of 128 bytes.
+// Shapes this kernel takes: np, nq multiples of 256 (192 on a narrow tile's side), at least two k-tiles of 128 bytes.
 // Shapes it is USED for: its tiles have to fill their rounds of the CUs, to 60 % where there is one round and to 70 % otherwise,
 // because a CU works on one tile at a time; then the half operand traffic per output wins against the 128 x 128 kernel at every
 // contraction length (standalone, us, that kernel -> this one): bf16 2048 x 32768 x 768 (4.0 rounds) 140 -> 105, 8192 x 4096 x 768
@@ -662,25 +714,55 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
 // at the line 8192 x 3072 x 768 (1.5) 46.4 -> 47.2, and below it 8192 x 2304 x 768 (1.12) 37.6 -> 41.8, 8192 x 1024 x 768 (0.5)
 // 18.5 -> 23.7. A heavy epilogue per tile (rotary embedding, residual add, the MLP's activation) is serial with the k-loop here and runs
 // under another workgroup's MFMAs there: those need 16 k-tiles or 4096 tiles as well (in the training step, 6 to 12 k-tiles:
-// 141 -> 148, 55 -> 60, 112 -> 111 us).
+// 141 -> 148, 55 -> 60, 112 -> 111 us); 24 on a narrow tile (bf16 9600 x 1024 x 1024 with a residual 32.8 -> 34.2).
+// A narrow tile takes 0.75 / 0.92 (192 x 256) or 0.75 / 0.84 (256 x 192) of a 256 x 256 tile's time, so it is taken where its rounds save
+// that much (us, the kernel of before -> this one): fp8 16384 x 768 x 3072 40.9 -> 36.8, 32768 rows 73.0 -> 65.5, 9600 x 1024 x 4096 51.7 ->
+// 40.3, 11904 x 768 x 3072 50.6 -> 30.3; bf16 32768 x 768 x 2304 118 -> 104, 30336 x 768 x 768 55 -> 43, 12672 x 768 x 3072 95 -> 62; not in
+// place of a 256 x 256 launch of as many rounds for 256 x 192 (fp8 11520 x 1024 x 2816 38.2 -> 40.3). Against the 128 x 128 kernel: its two
+// workgroups a CU run a round in 0.65 of a 256 x 256 tile's time, half a round or less (one a CU) in 0.38 (4992 x 1536 x 1536, 0.91 of a
+// round: 28.6 there, 34.9 here).
 #ifndef TFB_PP
 #define TFB_PP 1  // 0: every GEMM on the 128 x 128 kernel; 2: every shape the kernel takes (for comparisons)
 #endif
-static inline bool gemm_pp_applies(long np, long nq, long kbytes, bool heavy_epilogue = false) {
-  if (!TFB_PP || np <= 0 || nq <= 0 || np % 256 || nq % 256 || kbytes < 256 || kbytes % 128) return false;
-  const long tiles = (np / 256) * (nq / 256), cus = tfb_resident_slots(1), rounds = (tiles + cus - 1) / cus;
-  if (tiles < 8) return false;
-  if (TFB_PP == 2) return true;
-  if (10 * tiles < (rounds == 1 ? 6 : 7) * rounds * cus) return false;
-  return !heavy_epilogue || kbytes / 128 >= 16 || tiles >= 4096;
+#ifndef TFB_PP_SHAPE
+#define TFB_PP_SHAPE -1  // 0, 1, 2: that tile only (for comparisons)
+#endif
+// The tile for an output of np x nq, or -1: the one that keeps the CUs busiest (256 x 256 also for all but the last 128 rows of q, where
+// it has a full round without them: a launch of the ring more, 0.15 of a round).
+static inline int gemm_pp_shape(long np, long nq, long kbytes, bool heavy_epilogue, bool narrow_ok) {
+  if (!TFB_PP || np <= 0 || nq <= 0 || kbytes < 256 || kbytes % 128) return -1;
+  const long cus = tfb_resident_slots(1);
+  const double core_rounds = (double)((np + 127) / 128) * (double)((nq + 127) / 128) / (double)(2 * cus), whole = (double)(long)core_rounds;
+  const double core = 0.65 * whole + (core_rounds == whole ? 0.0 : core_rounds - whole > 0.5 ? 0.65 : 0.38);
+  int best = -1;
+  double best_cost = 1e30, whole_tiles = 1e30;
+  for (int shape = 0; shape < (narrow_ok ? 3 : 1); ++shape) {
+    if (TFB_PP_SHAPE >= 0 && shape != TFB_PP_SHAPE) continue;
+    const long tp = shape == TFB_PP_192x256 ? 192 : 256, tq = shape == TFB_PP_256x192 ? 192 : 256;
+    const long rest = nq % tq, tiles = (np / tp) * (nq / tq), rounds = (tiles + cus - 1) / cus;
+    if (np % tp || tiles < 8 || (rest && (shape || rest != 128 || tiles < cus))) continue;
+    const double cost = (double)rounds * (shape == 0 ? 1.0 : shape == TFB_PP_192x256 ? 0.75 / 0.92 : 0.75 / 0.84) + (rest ? 0.15 : 0.0);
+    if (TFB_PP != 2 && TFB_PP_SHAPE < 0) {
+      if ((double)tiles < (rounds == 1 ? 0.6 : 0.7) * (double)(rounds * cus)) continue;
+      if (heavy_epilogue && kbytes / 128 < (shape ? 24 : 16) && tiles < 4096) continue;
+      if (shape && (cost > (heavy_epilogue ? 0.9 : 0.95) * core || cost > 0.88 * whole_tiles)) continue;
+    }
+    if (shape == 0) whole_tiles = cost;
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = shape;
+    }
+  }
+  return best;
 }
 
-// np, nq multiples of 256; kbytes = the contraction in bytes of a k-contiguous row (elements * ES), a multiple of 128
+// np, nq multiples of the tile; kbytes = the contraction in bytes of a k-contiguous row (elements * ES), a multiple of 128
 // with at least two k-tiles per split. With splits > 1 the epilogue is one with kSplitF32 (EpiSplit); when all work items
 // fit one round of the CUs they are dealt to the XCDs in consecutive runs (PpArgs::ipx).
-template <int ES, int FMTP, int FMTQ, int LAYP, int LAYQ, class Epi>
+template <int ES, int FMTP, int FMTQ, int LAYP, int LAYQ, int SHAPE = TFB_PP_256x256, class Epi>
 static int gemm_pp_launch_lay(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, int splits, Epi epi, hipStream_t stream) {
-  if (np <= 0 || nq <= 0 || splits <= 0 || np % 256 || nq % 256 || kbytes % 128 || kbytes / 128 / splits < 2)
+  constexpr int TP = SHAPE == TFB_PP_192x256 ? 192 : 256, TQ = SHAPE == TFB_PP_256x192 ? 192 : 256;
+  if (np <= 0 || nq <= 0 || splits <= 0 || np % TP || nq % TQ || kbytes % 128 || kbytes / 128 / splits < 2)
     return TFB_ERR_SHAPE;
   if (P.ld <= 0 || Q.ld <= 0 || P.ld > (1L << 28) || Q.ld > (1L << 28)) return TFB_ERR_SHAPE;
   if (((uintptr_t)P.base | (uintptr_t)Q.base | (uintptr_t)P.ld | (uintptr_t)Q.ld) & 15) return TFB_ERR_ARG;
@@ -690,7 +772,7 @@ static int gemm_pp_launch_lay(GemmOperand P, GemmOperand Q, int np, int nq, long
   a.Q = Q;
   a.splits = splits;
   a.nk_total = (int)(kbytes / 128);
-  const int ntp = np / 256, ntq = nq / 256;
+  const int ntp = np / TP, ntq = nq / TQ;
   if ((long)ntp * ntq * splits >= (1L << 30)) return TFB_ERR_SHAPE;
   a.nout = ntp * ntq;
   a.ntiles = a.nout * splits;
@@ -700,10 +782,14 @@ static int gemm_pp_launch_lay(GemmOperand P, GemmOperand Q, int np, int nq, long
   const int nslow = a.p_fast ? ntq : ntp;
   a.rect = (nslow % 8 == 0) && a.nout >= 8;
   a.nwg = a.ntiles < cus ? a.ntiles : cus;
-  if (splits > 1 && a.ntiles <= cus) {
+  // Slow rows that are no multiple of 8: consecutive items per XCD too while it can keep the fast operand beside them (us, dealt over the
+  // XCDs one by one -> so: fp8 16128 x 768 x 3072 on 192 x 256 tiles 45.8 -> 35; bf16 12032 x 2304 x 768 51.3 -> 47.5, 9600 x 3072 x 1024 65.6 ->
+  // 64.7, 18816 x 4096 x 1024 156.3 -> 155.8; 9600 x 8192 x 1024, 16.8 MB, 154.6 -> 159.4).
+  const long fast_bytes = (long)(a.p_fast ? np : nq) * kbytes;
+  if (splits > 1 ? a.ntiles <= cus : !a.rect && a.ntiles >= 8 && fast_bytes <= (8L << 20) + (1L << 19)) {
     a.rect = 0;
     a.ipx = (a.ntiles + 7) / 8;
-    a.nwg = 8 * a.ipx;
+    a.nwg = 8 * a.ipx < cus ? 8 * a.ipx : cus & ~7;
   }
   if (a.rect) a.nwg &= ~7;
   if (a.nwg <= 0) return TFB_ERR_SHAPE;
@@ -721,7 +807,7 @@ static int gemm_pp_launch_lay(GemmOperand P, GemmOperand Q, int np, int nq, long
   a.d_gw = fastdiv_make(a.GW);
   a.d_gw_last = fastdiv_make(a.gw_last);
   a.d_nout = fastdiv_make(a.nout);
-  hipLaunchKernelGGL((gemm_pp_kernel<ES, FMTP, FMTQ, LAYP, LAYQ, Epi>), dim3(a.nwg), dim3(512), 0, stream, a, epi);
+  hipLaunchKernelGGL((gemm_pp_kernel<ES, FMTP, FMTQ, LAYP, LAYQ, Epi, SHAPE>), dim3(a.nwg), dim3(512), 0, stream, a, epi);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }

@@ -544,13 +544,19 @@ static bool gemm_ring_try(GemmOperand P, GemmOperand Q, int np, int nq, long kby
   return true;
 }
 
-// A dense launch through the persistent kernel where gemm_pp_applies takes it, or takes all but the last 128 rows of q (which then go
+// A dense launch through the persistent kernel where gemm_pp_shape gives it a tile (all but the last 128 rows of q, it may be: those go
 // through the ring: 9600 x 3072 x 1024 in bf16 79 -> 62 us): true, with its status in st. heavy: the epilogue is heavy there.
 template <int ES, int LAYP, int LAYQ, int FMTP, int FMTQ, class Epi>
 static bool gemm_pp_try(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, bool heavy, Epi e, hipStream_t s, int& st) {
+  constexpr bool narrow_ok = LAYQ == TFB_K_CONTIG && !has_partner32<Epi>::value;
+  const int shape = gemm_pp_shape(np, nq, kbytes, heavy, narrow_ok);
+  if (shape < 0) return false;
+  if constexpr (narrow_ok) {
+    if (shape == TFB_PP_192x256) st = gemm_pp_launch_lay<ES, FMTP, FMTQ, LAYP, LAYQ, TFB_PP_192x256>(P, Q, np, nq, kbytes, 1, e, s);
+    if (shape == TFB_PP_256x192) st = gemm_pp_launch_lay<ES, FMTP, FMTQ, LAYP, LAYQ, TFB_PP_256x192>(P, Q, np, nq, kbytes, 1, e, s);
+    if (shape != TFB_PP_256x256) return true;
+  }
   const int rest = nq % 256, main = nq - rest;
-  if (!gemm_pp_applies(np, main, kbytes, heavy)) return false;
-  if (rest && (rest != 128 || (long)(np / 256) * (main / 256) < tfb_resident_slots(1))) return false;
   st = gemm_pp_launch_lay<ES, FMTP, FMTQ, LAYP, LAYQ>(P, Q, np, main, kbytes, 1, e, s);
   if (st != TFB_OK || !rest) return true;
   GemmArgs a = {};
