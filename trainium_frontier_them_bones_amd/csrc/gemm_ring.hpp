@@ -31,6 +31,36 @@ struct is_symmetric : std::false_type {};
 template <class T>
 struct is_symmetric<T, std::void_t<decltype(T::kSymmetric)>> : std::true_type {};
 
+// A wavefront's 32 (q) x PC (p) block of finished outputs, transposed: out[p][q]. put() takes its 8-element chunks of rows q, store()
+// fetches them as columns with ds_read_b64_tr_b16 (a lane: 8 consecutive q of one p) and writes 64-byte pieces of the rows p. Both
+// areas are the wavefront's own (LDS operations of one wavefront execute in order); the paddings spread rows over the banks.
+// (Element by element, 32 two-byte writes a lane, this was 4 of 31 us of a 12 x 768 x 768 product over 3072.)
+template <int PC>
+struct MirrorBlock {
+  static constexpr int QP = PC * 2 + 16, PP = 80;              // bytes of a row q, of a row p
+  static constexpr int BYTES = 32 * QP, OUT_BYTES = PC * PP;
+  static __device__ __forceinline__ void put(uint8_t* t, int row, int pc, const u32x4& w) { *(u32x4*)(t + row * QP + pc * 2) = w; }
+  static __device__ __forceinline__ void store(const uint8_t* t, uint8_t* o, bf16_t* out, long ld, int lane) {
+    const int g4 = lane >> 4, j = lane & 15;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int r = 0; r < PC / 16; ++r) {   // lane group g4: rows p 16 r .. + 15, q 8 g4 .. + 7
+      const uint8_t* a = t + (8 * g4 + (j >> 2)) * QP + 32 * r + 8 * (j & 3);
+      const tfb_s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tfb_lds_s16x4_t*)a);
+      const tfb_s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tfb_lds_s16x4_t*)(a + 4 * QP));
+      typedef short s16x8 __attribute__((ext_vector_type(8)));
+      *(s16x8*)(o + (16 * r + j) * PP + 16 * g4) = s16x8{lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int k = 0; k < PC / 16; ++k) {
+      const int row = (lane >> 2) + 16 * k, qc = (lane & 3) * 16;
+      *(u32x4*)((uint8_t*)(out + (long)row * ld) + qc) = *(const u32x4*)(o + row * PP + qc);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+};
+
 template <int BP_, int BQ_, int WP_, int WQ_, int ES_, int LAYP_, int LAYQ_, int FMTP_, int FMTQ_, int NS_>
 struct RingCfg {
   static constexpr int BP = BP_, BQ = BQ_, WP = WP_, WQ = WQ_, ES = ES_, NS = NS_;
@@ -160,13 +190,7 @@ struct RingFrags<ROWS, NTILE, ES, TFB_K_STRIDED> {
 };
 
 // The MFMAs that made x stay in front of this point (they have no side effects, and would otherwise sink across barriers).
-// AGPR: with one workgroup per CU the compiler keeps accumulators in that half of the register file (pinned in the other they were
-// moved there and back, 128 moves per k-tile).
-template <bool AGPR>
-__device__ __forceinline__ void ring_pin(f32x16& x) {
-  if constexpr (AGPR) asm volatile("" : "+a"(x));
-  else asm volatile("" : "+v"(x));
-}
+__device__ __forceinline__ void ring_pin(f32x16& x) { asm volatile("" : "+v"(x)); }
 
 // s_waitcnt vmcnt(tiles * PER): all but the newest `tiles` k-tiles of loads have landed (tiles is wavefront-uniform)
 template <int PER>
@@ -266,6 +290,16 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
+  // symmetric products: the second half of every k-tile has sums of its own, as in gemm_sym.hpp
+  constexpr bool HALVES = is_symmetric<Epi>::value;
+  [[maybe_unused]] f32x16 upper[HALVES ? TP : 1][HALVES ? TQ : 1];
+  if constexpr (HALVES) {
+#pragma unroll
+    for (int i = 0; i < TP; ++i)
+#pragma unroll
+      for (int j = 0; j < TQ; ++j) upper[i][j] = acc[i][j];
+  }
+
   // a.ranges k ranges [z nkt / Z, (z + 1) nkt / Z), as a k-split cuts them: total = range 0 + range 1 + ...
   [[maybe_unused]] f32x16 total[RANGES ? TP : 1][RANGES ? TQ : 1];
   [[maybe_unused]] int range = 1, range_end = RANGES ? fastdiv(nkt, a.d_ranges) : 0;
@@ -295,7 +329,11 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
     constexpr int s = decltype(s_)::value;
     auto one = [&](auto i_, auto j_) {
       constexpr int i = decltype(i_)::value, j = decltype(j_)::value;
-      acc[i][j] = mfma32<ES, Cfg::FMTP, Cfg::FMTQ>(fp[set].template get<i, s>(), fq[set].template get<j, s>(), acc[i][j]);
+      auto& c = [&]() -> f32x16& {
+        if constexpr (HALVES && 2 * s >= Cfg::KS) return upper[i][j];
+        else return acc[i][j];
+      }();
+      c = mfma32<ES, Cfg::FMTP, Cfg::FMTQ>(fp[set].template get<i, s>(), fq[set].template get<j, s>(), c);
     };
     using N0 = std::integral_constant<int, 0>;
     using N1 = std::integral_constant<int, 1>;
@@ -335,7 +373,10 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
 #pragma unroll
     for (int i = 0; i < TP; ++i)
 #pragma unroll
-      for (int j = 0; j < TQ; ++j) ring_pin<(Cfg::LDS_BYTES > 80 * 1024)>(acc[i][j]);
+      for (int j = 0; j < TQ; ++j) {
+        ring_pin(acc[i][j]);
+        if constexpr (HALVES) ring_pin(upper[i][j]);
+      }
   };
 
   if (nkt > 0) {
@@ -368,6 +409,12 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
         for (int j = 0; j < TQ; ++j) acc[i][j] = total[i][j] + acc[i][j];
     }
   }
+  if constexpr (HALVES) {
+#pragma unroll
+    for (int i = 0; i < TP; ++i)
+#pragma unroll
+      for (int j = 0; j < TQ; ++j) acc[i][j] = acc[i][j] + upper[i][j];
+  }
   __syncthreads();
 
   if constexpr (has_tile_epilogue<Epi>::value) {
@@ -376,9 +423,9 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
     // 32 output rows at a time through the wavefront's own LDS slice, then 8-element chunks, a row's on consecutive lanes
     constexpr int SLD = Cfg::STAGE_LD;
     float* stg = (float*)lds + wave * (32 * SLD);
-    constexpr int MLD = 40;   // (80-byte rows: 16-byte aligned, and a lane's column of eight on different banks)
-    static_assert(!is_symmetric<Epi>::value || Cfg::EPI_BYTES + NW * TP * 32 * MLD * 2 <= Cfg::LDS_BYTES, "mirror slices");
-    [[maybe_unused]] bf16_t* mirror = (bf16_t*)(lds + Cfg::EPI_BYTES) + wave * (TP * 32 * MLD);
+    typedef MirrorBlock<TP * 32> Mirror;
+    static_assert(!is_symmetric<Epi>::value || Cfg::EPI_BYTES + NW * (Mirror::BYTES + Mirror::OUT_BYTES) <= Cfg::LDS_BYTES, "mirror slices");
+    [[maybe_unused]] uint8_t* mirror = lds + Cfg::EPI_BYTES + wave * (Mirror::BYTES + Mirror::OUT_BYTES);
 #pragma unroll
     for (int j = 0; j < TQ; ++j) {
 #pragma unroll
@@ -400,10 +447,7 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
           if constexpr (kPrefetch) w = epi.value(v, pre[j][k]);
           else w = epi.value(v);
           *(u32x4*)(epi.out + (long)q * epi.ld + p) = w;
-          if (tile_p != tile_q) {
-#pragma unroll
-            for (int x = 0; x < 8; ++x) mirror[(pc + x) * MLD + row] = (bf16_t)(x & 1 ? w[x >> 1] >> 16 : w[x >> 1]);
-          }
+          if (tile_p != tile_q) Mirror::put(mirror, row, pc, w);
         } else if constexpr (has_partner32<Epi>::value) {
           static_assert(TP == 2, "partner epilogue: 64 staged columns per wavefront");
           const f32x4 plo = *(const f32x4*)(stg + row * SLD + (pc ^ 32)), phi = *(const f32x4*)(stg + row * SLD + (pc ^ 32) + 4);
@@ -418,14 +462,7 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
       }
       __builtin_amdgcn_wave_barrier();
       if constexpr (is_symmetric<Epi>::value) {
-        if (tile_p != tile_q) {   // the 32 rows q of this pass as 64-byte pieces of the rows p
-#pragma unroll
-          for (int k = 0; k < NK; ++k) {
-            const int c = lane + 64 * k, row = c >> 2, qc = (c & 3) * 8;
-            *(u32x4*)(epi.out + ((long)p0 + pw + row) * epi.ld + q0 + qw + j * 32 + qc) = *(const u32x4*)(mirror + row * MLD + qc);
-          }
-          __builtin_amdgcn_wave_barrier();
-        }
+        if (tile_p != tile_q) Mirror::store(mirror, mirror + Mirror::BYTES, epi.out + ((long)p0 + pw) * epi.ld + q0 + qw + j * 32, epi.ld, lane);
       }
     }
   }
@@ -483,10 +520,7 @@ static inline int gemm_ring_pick(long np, long nq, long nkt, bool strided, long 
   return 2 * t64 <= (strided ? 9 : 8) * cus ? 2 : 0;
 }
 
-// A stack of `groups` symmetric N x N products of one operand with itself (N a multiple of 128): 64 x 64 tiles while no CU has more
-// than two, else 128 x 128 with four stages (half the bytes per output, one workgroup per CU). What bounds them is a k-tile's trip
-// through one wavefront per SIMD and the operand's way into eight L2s, which the runs of tiles cut to one or two. The five iterations
-// of Muon with both symmetric products full -> this: 12 x 3072 x 768 810 -> 625 us, 12 x 2048 x 512 354 -> 251, 6 x 2304 x 768 369 -> 293.
+// A stack of `groups` symmetric N x N products of one operand with itself (N a multiple of 128) on 64 x 64 tiles: gemm_sym.hpp has the rule.
 template <class Epi, int ES, int LAY>
 static int gemm_ring_symmetric(GemmOperand X, long g_stride, const int* k_seg, int N, int nkt, int groups, Epi e, hipStream_t s) {
   GemmArgs a = {};
@@ -497,21 +531,16 @@ static int gemm_ring_symmetric(GemmOperand X, long g_stride, const int* k_seg, i
   a.nkt = nkt;
   a.k_seg = k_seg;
   a.g_stride = g_stride;
-  const long n64 = N / 64, cus = tfb_resident_slots(1);
-  const bool small = n64 * (n64 + 1) / 2 * groups <= 2 * cus;
-  a.ntp = small ? N / 64 : N / 128;
-  using C64 = RingCfg<64, 64, 2, 2, ES, LAY, LAY, 0, 0, 4>;
-  using C128 = RingCfg<128, 128, 2, 2, ES, LAY, LAY, 0, 0, 4>;
-  const int st = small ? gemm_map_args<C64>(a, 1) : gemm_map_args<C128>(a, 1);
+  a.ntp = N / 64;
+  using Cfg = RingCfg<64, 64, 2, 2, ES, LAY, LAY, 0, 0, 4>;
+  const int st = gemm_map_args<Cfg>(a, 1);
   if (st != TFB_OK) return st;
   a.ntiles = a.ntp * (a.ntp + 1) / 2;
   a.d_ntiles = fastdiv_make(a.ntiles);
   a.rows = groups;
   if ((long)a.ntiles * groups > 0x7ffffff0L / 8) return TFB_ERR_SHAPE;
   a.per = (a.ntiles * groups + 7) / 8;
-  const dim3 grid(8 * a.per);
-  if (small) hipLaunchKernelGGL((gemm_ring_kernel<C64, false, Epi>), grid, dim3(256), 0, s, a, e);
-  else hipLaunchKernelGGL((gemm_ring_kernel<C128, false, Epi>), grid, dim3(256), 0, s, a, e);
+  hipLaunchKernelGGL((gemm_ring_kernel<Cfg, false, Epi>), dim3(8 * a.per), dim3(256), 0, s, a, e);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }

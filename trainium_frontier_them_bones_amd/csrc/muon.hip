@@ -14,7 +14,7 @@
 // (q_group). G and G G are symmetric bit for bit (the same products summed in the same order on either side of the
 // diagonal): their tiles on and above the diagonal are computed, those above it stored a second time transposed, and with
 // B^T = B both products run in the k-contiguous "x @ w^T" form with the [N][N] matrix as the weight.
-#include "gemm_ring.hpp"
+#include "gemm_sym.hpp"
 
 namespace {
 
@@ -182,11 +182,11 @@ extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, vo
     // the tall stack's last iteration writes y itself
     bf16_t* xout = (it == 4 && !wide) ? (bf16_t*)y : X[cur ^ 1];
     // G[k] = X[k]^T X[k]: both operands k-strided (rows of the stacked X), the contraction segmented per matrix
-    int st = gemm_ring_symmetric<EpiSym, 2, TFB_K_STRIDED>(GemmOperand{(const uint8_t*)xin, (long)N * 2}, 0, k_seg, N, M / 64, K,
+    int st = gemm_symmetric<EpiSym, TFB_K_STRIDED>(GemmOperand{(const uint8_t*)xin, (long)N * 2}, 0, k_seg, N, M / 64, K,
                                                           EpiSym{G, (long)N, (long)N * N}, s);
     if (st != TFB_OK) return st;
     // B = c G G + b G: G[k] against itself (G G^T = G G)
-    st = gemm_ring_symmetric<EpiSymAxpby, 2, TFB_K_CONTIG>(GemmOperand{(const uint8_t*)G, (long)N * 2}, (long)N * N * 2, nullptr, N,
+    st = gemm_symmetric<EpiSymAxpby, TFB_K_CONTIG>(GemmOperand{(const uint8_t*)G, (long)N * 2}, (long)N * N * 2, nullptr, N,
                                                           N * 2 / 128, K, EpiSymAxpby{Bm, G, (long)N, (long)N * N, c, b}, s);
     if (st != TFB_OK) return st;
     // X' = X B + a X on the stacked X: rows of X[k] against B[k] as the weight (X B^T = X B)
