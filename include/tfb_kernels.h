@@ -529,10 +529,16 @@ int tfb_moe_quant_dout(const void* dout, const void* tok, const void* ksel, cons
  * g fp32 [K][M][N] (wide 0) or [K][N][M] (wide 1: handled as the transposes); inv_d fp32 [K] device (1 / d). M, N % 128.
  * workspace: tfb_ns5_workspace_bytes(K, M, N) bytes of device memory. The whole stack takes 3 grouped GEMM launches per
  * iteration. Replaces _nsk_kernel(ga, gb, sc) -> ya, yb, va, vb (round2/source/kernels/nki_nsk.py:370; arithmetic
- * emulate_nsk :452) = the loop of muon_math_body (reference_ns :471); one call per stack. */
+ * emulate_nsk :452) = the loop of muon_math_body (reference_ns :471). */
 long tfb_ns5_workspace_bytes(int K, int M, int N);
 int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, void* y, void* v, int K, int M, int N, int wide,
             void* workspace, long workspace_bytes, void* stream);
+/* Both stacks of a Muon step at once, of the same tall shape [M][N] but each in its own layout, one launch of every kind for all matrices:
+ * each comes out as tfb_ns5 leaves it, bit for bit. da, db: the denominators (d_type 1 fp32, 2 bf16, 3 fp16; the reciprocal is taken in
+ * fp32, round2/source/kernels/nki_nsk.py:406). Kb 0: one stack, B's pointers may be NULL. workspace: tfb_ns5_workspace_bytes(Ka + Kb, M, N). */
+int tfb_ns5_stacks(const void* ga, const void* da, void* ya, void* va, int Ka, int wide_a, const void* gb, const void* db, void* yb,
+                   void* vb, int Kb, int wide_b, int d_type, const float* coeffs, int M, int N, void* workspace, long workspace_bytes,
+                   void* stream);
 
 /* ---- dense bf16 fused MLP ---------------------------------------------------------------------------------------------
  * x bf16 [M][d], w_fc bf16 [F][d], w_proj bf16 [d][F] (nn.Linear layouts) -> y bf16 [M][d] = bf16(h @ w_proj^T) with

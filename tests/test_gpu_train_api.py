@@ -294,6 +294,29 @@ def test_nsk_both_stacks(api, dev):
     assert e[0].shape == (0, 512, 256) and torch.equal(e[1], yb)
 
 
+@pytest.mark.parametrize("Ka,sa,Kb,sb", [(2, (512, 256), 3, (256, 512)), (1, (384, 384), 4, (384, 384)), (3, (128, 256), 1, (128, 256)),
+                                         (40, (256, 256), 24, (256, 256)), (5, (1152, 640), 9, (640, 1152))])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+def test_nsk_of_both_stacks_equals_that_of_each(api, dev, Ka, sa, Kb, sb, dtype):
+    """Stacks of the same long and short side run as one, in every combination of layouts and with either tile of the symmetric
+    products: bit for bit what each gives alone; a function in the place of ops.ns5 is called."""
+    from trainium_frontier_them_bones_amd import ops
+    g = torch.Generator(device=dev).manual_seed(Ka + Kb)
+    ga, gb = (torch.randn(K, *s, generator=g, device=dev) * 0.02 for K, s in ((Ka, sa), (Kb, sb)))
+    da, db = (x.norm(dim=(-2, -1)).mul(1.01).to(dtype) for x in (ga, gb))
+    ya, yb, va, vb = api.nsk(ga, gb, da.reshape(-1, 1, 1), db)
+    for y, v, x, d in ((ya, va, ga, da), (yb, vb, gb, db)):
+        y1, v1 = ops.ns5(x, d)
+        assert torch.equal(y, y1) and torch.equal(v, v1)
+    own, calls = ops.ns5, []
+    try:
+        ops.ns5 = lambda x, d, *c: calls.append(x.shape) or own(x, d, *c)
+        r = api.nsk(ga, gb, da, db)
+    finally:
+        ops.ns5 = own
+    assert calls == [ga.shape, gb.shape] and torch.equal(r[0], ya) and torch.equal(r[3], vb)
+
+
 def test_head2_and_adamw_fused_step(api, dev):
     from oracle import norm as ON
     g = _g(14)

@@ -119,6 +119,7 @@ SIGNATURES = {
     "tfb_moe_quant": [_vp, _vp, _vp, _i, _i, _vp, _l, _i, _vp],
     "tfb_moe_quant_dout": [_vp, _vp, _vp, _vp, _vp, _vp, _i, _vp, _l, _i, _i, _vp],
     "tfb_ns5_workspace_bytes": [_i, _i, _i],
+    "tfb_ns5_stacks": [_vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp, _i, _i, _i, _fp, _i, _i, _vp, _l, _vp],
     "tfb_ns5": [_vp, _vp, _fp, _vp, _vp, _i, _i, _i, _i, _vp, _l, _vp],
     "tfb_mlp_dw_proj": [_vp, _vp, _vp, _l, _i, _i, _i, _i, _vp, _l, _vp],
 }

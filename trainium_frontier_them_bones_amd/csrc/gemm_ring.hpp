@@ -240,7 +240,7 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
     a.P.base += (long)group * a.p_group_stride;
   }
   if (a.k_seg) {
-    group = is_symmetric<Epi>::value ? sym_group : (int)blockIdx.y;
+    group = blockIdx.y;
     const int k0 = a.k_seg[group], k1 = a.k_seg[group + 1];
     kt0 = k0 * ES / 128;
     a.nkt = (k1 - k0) * ES / 128;  // may be 0: the accumulators stay zero and are still written
@@ -522,14 +522,13 @@ static inline int gemm_ring_pick(long np, long nq, long nkt, bool strided, long 
 
 // A stack of `groups` symmetric N x N products of one operand with itself (N a multiple of 128) on 64 x 64 tiles: gemm_sym.hpp has the rule.
 template <class Epi, int ES, int LAY>
-static int gemm_ring_symmetric(GemmOperand X, long g_stride, const int* k_seg, int N, int nkt, int groups, Epi e, hipStream_t s) {
+static int gemm_ring_symmetric(GemmOperand X, long g_stride, int N, int nkt, int groups, Epi e, hipStream_t s) {
   GemmArgs a = {};
   a.P = X;
   a.Q = X;
   a.np = N;
   a.nq = N;
   a.nkt = nkt;
-  a.k_seg = k_seg;
   a.g_stride = g_stride;
   a.ntp = N / 64;
   using Cfg = RingCfg<64, 64, 2, 2, ES, LAY, LAY, 0, 0, 4>;

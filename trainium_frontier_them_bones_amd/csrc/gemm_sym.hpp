@@ -21,10 +21,9 @@
 
 struct SymArgs {
   GemmOperand X;
-  long g_stride;      // the operand of group g starts g_stride bytes * g further, and
-  const int* k_seg;   // (optional) its contraction is elements k_seg[g] .. k_seg[g + 1], multiples of 128, at least 128
-  int nkt;            // k-tiles of 64 without k_seg: an even number
-  int nt;             // tiles of a side
+  long g_stride;   // the operand of group g starts g_stride bytes * g further
+  int nkt;         // k-tiles of 64: an even number
+  int nt;          // tiles of a side
   int ntiles, groups, per;   // nt (nt + 1) / 2 tiles a group; XCD x (= workgroup & 7) takes `per` consecutive tiles of the stack
   FastDiv d_ntiles;
 };
@@ -93,17 +92,13 @@ __global__ __launch_bounds__(512, 2) void gemm_sym_kernel(SymArgs a, Epi epi_in)
   for (; tile_p >= a.nt - tile_q; ++tile_q) tile_p -= a.nt - tile_q;   // row tile_q has nt - tile_q tiles
   tile_p += tile_q;
   const int p0 = tile_p * 128, q0 = tile_q * 128;
-  int k0 = 0, nkt = a.nkt;
-  if (a.k_seg) {
-    k0 = a.k_seg[group];
-    nkt = (a.k_seg[group + 1] - k0) / 64;
-  }
+  const int nkt = a.nkt;
   GemmOperand X = a.X;
   X.base += group * a.g_stride;
 
   TileDma<128, 8, LAY, 2> dp, dq;
-  dp.init(X, p0, (long)k0 * 2, wave, lane);
-  dq.init(X, q0, (long)k0 * 2, wave, lane);
+  dp.init(X, p0, 0, wave, lane);
+  dq.init(X, q0, 0, wave, lane);
   auto issue = [&](int t) __attribute__((always_inline)) {   // four loads a wavefront
     uint8_t* d = lds + (t & (NS - 1)) * STAGE;
     dp.issue(d, t, wave);
@@ -274,13 +269,13 @@ __global__ __launch_bounds__(512, 2) void gemm_sym_kernel(SymArgs a, Epi epi_in)
 // tiles of the ring kernel while no CU has more than two, else 128 x 128 (half the bytes per output, one workgroup per CU). An XCD's
 // workgroups take a run of consecutive tiles, so that a matrix's operand is read into one or two L2s only.
 template <class Epi, int LAY>
-static int gemm_symmetric(GemmOperand X, long g_stride, const int* k_seg, int N, int nkt, int groups, Epi e, hipStream_t s) {
+static int gemm_symmetric(GemmOperand X, long g_stride, int N, int nkt, int groups, Epi e, hipStream_t s) {
   if (N <= 0 || N % 128 || groups <= 0 || nkt < 2 || nkt % 2) return TFB_ERR_SHAPE;
   const long n64 = N / 64, cus = tfb_resident_slots(1);
-  if (n64 * (n64 + 1) / 2 * groups <= 2 * cus) return gemm_ring_symmetric<Epi, 2, LAY>(X, g_stride, k_seg, N, nkt, groups, e, s);
+  if (n64 * (n64 + 1) / 2 * groups <= 2 * cus) return gemm_ring_symmetric<Epi, 2, LAY>(X, g_stride, N, nkt, groups, e, s);
   if (X.ld <= 0 || X.ld > (1L << 28)) return TFB_ERR_SHAPE;
   if (((uintptr_t)X.base | (uintptr_t)X.ld) & 15) return TFB_ERR_ARG;
-  SymArgs a = {X, g_stride, k_seg, nkt, N / 128, 0, groups, 0, {}};
+  SymArgs a = {X, g_stride, nkt, N / 128, 0, groups, 0, {}};
   a.ntiles = a.nt * (a.nt + 1) / 2;
   if ((long)a.ntiles * groups > 0x7ffffff0L / 8) return TFB_ERR_SHAPE;
   a.per = (a.ntiles * groups + 7) / 8;

@@ -10,11 +10,13 @@
 // with the five (a, b, c) of the caller, then v[m] = sum_n X5[m][n]^2 in fp32 from the bf16 X5.
 //
 // The whole stack runs in three grouped GEMM launches per iteration (not three per matrix): the matrices are stacked
-// along the rows, G's contraction is segmented per matrix (k_seg), and X B picks the [N][N] operand by the row tile's matrix
+// along the rows, G's contraction is over a matrix's own rows, and X B picks the [N][N] operand by the row tile's matrix
 // (q_group). G and G G are symmetric bit for bit (the same products summed in the same order on either side of the
 // diagonal): their tiles on and above the diagonal are computed, those above it stored a second time transposed, and with
 // B^T = B both products run in the k-contiguous "x @ w^T" form with the [N][N] matrix as the weight.
 #include "gemm_sym.hpp"
+
+extern "C" long tfb_ns5_workspace_bytes(int K, int M, int N);
 
 namespace {
 
@@ -29,16 +31,19 @@ __device__ __forceinline__ u32x4 axpby8(const float (&v)[8], const u32x4& zv, fl
   return pack8bf(r);
 }
 
-// out = bf16(fp32(alpha * D) + fp32(beta * z)), z and out [rows][ld] bf16; the z chunk is requested before the k-loop
+// out = bf16(fp32(alpha * D) + fp32(beta * z)), z and out [rows][ld] bf16; the z chunk is requested before the k-loop. Rows from `split` on
+// go to out2 (at the same offsets)
 struct EpiAxpby {
   bf16_t* out;
+  bf16_t* out2;
+  int split;
   const bf16_t* z;
   long ld;
   float alpha, beta;
   using pre_t = u32x4;
   __device__ __forceinline__ pre_t prefetch(int p, int q) const { return *(const u32x4*)(z + (long)q * ld + p); }
   __device__ __forceinline__ void operator()(int p, int q, const float (&v)[8], const pre_t& zv, int) const {
-    *(u32x4*)(out + (long)q * ld + p) = axpby8(v, zv, alpha, beta);
+    *(u32x4*)((q < split ? out : out2) + (long)q * ld + p) = axpby8(v, zv, alpha, beta);
   }
 };
 
@@ -64,20 +69,28 @@ struct EpiSymAxpby {
   }
 };
 
-// k_seg[i] = i * M (i <= K); xq[t] = t / (M / 128) for the K M / 128 row tiles of the stacked X
-__global__ void ns_tables_kernel(int* k_seg, int* xq, int K, int M) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i <= K) k_seg[i] = i * M;
-  if (i < K * (M / 128)) xq[i] = i / (M / 128);
+// The reciprocals of a stack's denominators: what the caller computed, or 1 / fp32(d) of its denominators
+#define NS_INV 0
+#define NS_D_F32 1
+#define NS_D_BF16 2
+#define NS_D_F16 3
+__device__ __forceinline__ float ns_inverse(const void* d, int type, int k) {
+  if (type == NS_INV) return ((const float*)d)[k];
+  if (type == NS_D_F32) return 1.0f / ((const float*)d)[k];
+  if (type == NS_D_BF16) return 1.0f / __uint_as_float((uint32_t)((const bf16_t*)d)[k] << 16);
+  return 1.0f / (float)((const _Float16*)d)[k];
 }
 
-// X0 [K][M][N] bf16 = bf16(bf16(g) * inv_d[k]); g fp32 [K][M][N], or with WIDE [K][N][M] (32 x 32 tiles through LDS)
+// X0 [K][M][N] bf16 = bf16(bf16(g) * inv_d[k]); g fp32 [K][M][N], or with WIDE [K][N][M] (32 x 32 tiles through LDS). Also the table of the
+// matrix that a row tile of 128 belongs to: xq[k M / 128 ..] = first + k.
 template <bool WIDE>
-__global__ __launch_bounds__(256) void ns_load_kernel(const float* __restrict__ g, const float* __restrict__ inv_d,
-                                                     bf16_t* __restrict__ x, int M, int N) {
+__global__ __launch_bounds__(256) void ns_load_kernel(const float* __restrict__ g, const void* __restrict__ d, int type,
+                                                     bf16_t* __restrict__ x, int* __restrict__ xq, int first, int M, int N) {
   const int k = blockIdx.z;
-  const float r = inv_d[k];
+  const float r = ns_inverse(d, type, k);
   const long mat = (long)k * M * N;
+  if (blockIdx.x == 0 && blockIdx.y == 0)
+    for (int i = threadIdx.x; i < M / 128; i += 256) xq[k * (M / 128) + i] = first + k;
   if (!WIDE) {
     const long n = (long)M * N;
     for (long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4; i < n; i += (long)gridDim.x * 256 * 4) {
@@ -97,11 +110,17 @@ __global__ __launch_bounds__(256) void ns_load_kernel(const float* __restrict__ 
   }
 }
 
-// v[k][m] = sum_n X[k][m][n]^2 (fp32, from the bf16 values): one wavefront per row
-__global__ __launch_bounds__(256) void ns_rowsq_kernel(const bf16_t* __restrict__ x, float* __restrict__ v, long rows, int N) {
+// v[k][m] = sum_n X[k][m][n]^2 (fp32, from the bf16 values): one wavefront per row. Rows from `split` on are x2's and go to v2 (at the
+// same offsets).
+__global__ __launch_bounds__(256) void ns_rowsq_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ x2, float* __restrict__ v,
+                                                      float* __restrict__ v2, long split, long rows, int N) {
   const int lane = threadIdx.x & 63;
   const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
+  if (row >= split) {
+    x = x2;
+    v = v2;
+  }
   float s = 0.f;
   for (int c = lane * 8; c < N; c += 512) {
     float f[8];
@@ -138,56 +157,57 @@ inline long align256(long b) { return (b + 255) & ~255L; }
 
 }  // namespace
 
-// Bytes of device workspace tfb_ns5 needs for a stack of K matrices with long side M and short side N.
-extern "C" long tfb_ns5_workspace_bytes(int K, int M, int N) {
-  if (K <= 0 || M <= 0 || N <= 0) return 0;
-  const long xb = align256((long)K * M * N * 2), gb = align256((long)K * N * N * 2);
-  return 2 * xb + 2 * gb + align256(((long)K + 1 + (long)K * (M / 128)) * 4);
-}
+namespace {
 
-// g: fp32 [K][M][N] (wide = 0) or [K][N][M] (wide = 1: each matrix is handled as its transpose), M >= N; inv_d: fp32 [K]
-// device (1 / d of each matrix, d as the caller's optimizer computes it); coeffs: 15 HOST floats, (a, b, c) of the five
-// iterations; y: bf16, the layout of g; v: fp32 [K][M]. M, N multiples of 128. The call enqueues 3 + 15 (+1) launches
-// on `stream` and returns; the workspace must stay untouched until they have run.
-extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, void* y, void* v, int K, int M, int N, int wide,
-                       void* workspace, long workspace_bytes, void* stream) {
-  if (!g || !inv_d || !coeffs || !y || !v || !workspace) return TFB_ERR_ARG;
-  if (K <= 0 || M <= 0 || N <= 0 || M % 128 || N % 128 || M < N || (long)K * M > 0x7fffffffL / 2 || K > 65535)
-    return TFB_ERR_SHAPE;
+struct NsStack {   // K matrices of one layout; d: their reciprocals or denominators (NS_*)
+  const void *g, *d;
+  void *y, *v;
+  int K, wide;
+};
+
+// Both stacks, the matrices of A in front of B's: one launch of every kind for all of them (a stack of few matrices leaves most CUs idle: 1 + 1
+// matrices of 3072 x 768, their reciprocals included, in two calls 326 us, in one 193), a stack's own only where its layout differs.
+int ns_run(const NsStack& A, const NsStack& B, int d_type, const float* coeffs, int M, int N, void* workspace, long workspace_bytes, hipStream_t s) {
+  const int K = A.K + B.K;
+  if (!A.g || !A.d || !A.y || !A.v || (B.K && (!B.g || !B.d || !B.y || !B.v)) || !coeffs || !workspace) return TFB_ERR_ARG;
+  if (A.K <= 0 || B.K < 0 || M <= 0 || N <= 0 || M % 128 || N % 128 || M < N || (long)A.K + B.K > 65535 || (long)K * M > 0x7fffffffL / 2) return TFB_ERR_SHAPE;
   if (workspace_bytes < tfb_ns5_workspace_bytes(K, M, N)) return TFB_ERR_WORKSPACE;
-  hipStream_t s = (hipStream_t)stream;
   uint8_t* w = (uint8_t*)workspace;
-  const long xb = align256((long)K * M * N * 2), gb = align256((long)K * N * N * 2);
+  const long xb = align256((long)K * M * N * 2), gb = align256((long)K * N * N * 2), mat = (long)M * N;
   bf16_t* X[2] = {(bf16_t*)w, (bf16_t*)(w + xb)};
   bf16_t* G = (bf16_t*)(w + 2 * xb);
   bf16_t* Bm = (bf16_t*)(w + 2 * xb + gb);
-  int* k_seg = (int*)(w + 2 * xb + 2 * gb);
-  int* xq = k_seg + K + 1;
+  int* xq = (int*)(w + 2 * xb + 2 * gb);
 
-  const int ntab = K * (M / 128) + 1;
-  hipLaunchKernelGGL(ns_tables_kernel, dim3((ntab + 255) / 256), dim3(256), 0, s, k_seg, xq, K, M);
-  TFB_LAUNCH_CHECK();
-  if (wide)
-    hipLaunchKernelGGL(ns_load_kernel<true>, dim3(M / 32, N / 32, K), dim3(256), 0, s, (const float*)g, (const float*)inv_d, X[0],
-                       M, N);
-  else
-    hipLaunchKernelGGL(ns_load_kernel<false>, dim3(256, 1, K), dim3(256), 0, s, (const float*)g, (const float*)inv_d, X[0], M, N);
-  TFB_LAUNCH_CHECK();
+  auto load = [&](const NsStack& S, int first) {
+    if (S.K == 0) return TFB_OK;
+    if (S.wide)
+      hipLaunchKernelGGL(ns_load_kernel<true>, dim3(M / 32, N / 32, S.K), dim3(256), 0, s, (const float*)S.g, S.d, d_type, X[0] + first * mat,
+                         xq + first * (M / 128), first, M, N);
+    else
+      hipLaunchKernelGGL(ns_load_kernel<false>, dim3(256, 1, S.K), dim3(256), 0, s, (const float*)S.g, S.d, d_type, X[0] + first * mat,
+                         xq + first * (M / 128), first, M, N);
+    TFB_LAUNCH_CHECK();
+    return TFB_OK;
+  };
+  int st = load(A, 0);
+  if (st == TFB_OK) st = load(B, A.K);
+  if (st != TFB_OK) return st;
 
   using CfgN = GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>;
-  int cur = 0;
+  bf16_t *x5a = nullptr, *x5b = nullptr;   // the last iterate's rows of either stack, from row 0 of all of them
   for (int it = 0; it < 5; ++it) {
     const float a = coeffs[3 * it], b = coeffs[3 * it + 1], c = coeffs[3 * it + 2];
-    bf16_t* xin = X[cur];
-    // the tall stack's last iteration writes y itself
-    bf16_t* xout = (it == 4 && !wide) ? (bf16_t*)y : X[cur ^ 1];
-    // G[k] = X[k]^T X[k]: both operands k-strided (rows of the stacked X), the contraction segmented per matrix
-    int st = gemm_symmetric<EpiSym, TFB_K_STRIDED>(GemmOperand{(const uint8_t*)xin, (long)N * 2}, 0, k_seg, N, M / 64, K,
-                                                          EpiSym{G, (long)N, (long)N * N}, s);
+    bf16_t *xin = X[it & 1], *xout = X[(it & 1) ^ 1];
+    // a tall stack's last iteration writes y itself
+    x5a = it == 4 && !A.wide ? (bf16_t*)A.y : xout;
+    x5b = it == 4 && B.K && !B.wide ? (bf16_t*)B.y - A.K * mat : xout;
+    // G[k] = X[k]^T X[k]: both operands k-strided (rows of X[k])
+    st = gemm_symmetric<EpiSym, TFB_K_STRIDED>(GemmOperand{(const uint8_t*)xin, (long)N * 2}, mat * 2, N, M / 64, K, EpiSym{G, (long)N, (long)N * N}, s);
     if (st != TFB_OK) return st;
     // B = c G G + b G: G[k] against itself (G G^T = G G)
-    st = gemm_symmetric<EpiSymAxpby, TFB_K_CONTIG>(GemmOperand{(const uint8_t*)G, (long)N * 2}, (long)N * N * 2, nullptr, N,
-                                                          N * 2 / 128, K, EpiSymAxpby{Bm, G, (long)N, (long)N * N, c, b}, s);
+    st = gemm_symmetric<EpiSymAxpby, TFB_K_CONTIG>(GemmOperand{(const uint8_t*)G, (long)N * 2}, (long)N * N * 2, N, N / 64, K,
+                                                   EpiSymAxpby{Bm, G, (long)N, (long)N * N, c, b}, s);
     if (st != TFB_OK) return st;
     // X' = X B + a X on the stacked X: rows of X[k] against B[k] as the weight (X B^T = X B)
     GemmArgs gx;
@@ -200,18 +220,45 @@ extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, vo
     gx.q_group = xq;
     gx.p_group_stride = (long)N * N * 2;
     gx.k_seg = nullptr;
-    EpiAxpby ex{xout, xin, (long)N, 1.0f, a};
-    st = launch<CfgN>(gx, 1, gx.nkt, ex, s);
+    st = launch<CfgN>(gx, 1, gx.nkt, EpiAxpby{x5a, x5b, A.K * M, xin, (long)N, 1.0f, a}, s);
     if (st != TFB_OK) return st;
-    cur ^= 1;
   }
-  const bf16_t* x5 = wide ? X[cur] : (const bf16_t*)y;
-  const long rows = (long)K * M;
-  hipLaunchKernelGGL(ns_rowsq_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, x5, (float*)v, rows, N);
+  const long rows = (long)K * M, split = (long)A.K * M;
+  hipLaunchKernelGGL(ns_rowsq_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, x5a, x5b, (float*)A.v, (float*)B.v - split, split, rows, N);
   TFB_LAUNCH_CHECK();
-  if (wide) {
-    hipLaunchKernelGGL(ns_transpose_out_kernel, dim3(M / 32, N / 32, K), dim3(256), 0, s, x5, (bf16_t*)y, M, N);
+  auto transpose = [&](const NsStack& S, const bf16_t* x5) {
+    if (S.K == 0 || !S.wide) return TFB_OK;
+    hipLaunchKernelGGL(ns_transpose_out_kernel, dim3(M / 32, N / 32, S.K), dim3(256), 0, s, x5, (bf16_t*)S.y, M, N);
     TFB_LAUNCH_CHECK();
-  }
-  return TFB_OK;
+    return TFB_OK;
+  };
+  st = transpose(A, x5a);
+  return st != TFB_OK ? st : transpose(B, x5b + A.K * mat);
+}
+
+}  // namespace
+
+// Bytes of device workspace tfb_ns5 needs for a stack of K matrices (tfb_ns5_stacks: of both stacks' together) with long side M and short side N.
+extern "C" long tfb_ns5_workspace_bytes(int K, int M, int N) {
+  if (K <= 0 || M <= 0 || N <= 0) return 0;
+  const long xb = align256((long)K * M * N * 2), gb = align256((long)K * N * N * 2);
+  return 2 * xb + 2 * gb + align256((long)K * (M / 128) * 4);
+}
+
+// g: fp32 [K][M][N] (wide = 0) or [K][N][M] (wide = 1: each matrix is handled as its transpose), M >= N; inv_d: fp32 [K]
+// device (1 / d of each matrix, d as the caller's optimizer computes it); coeffs: 15 HOST floats, (a, b, c) of the five
+// iterations; y: bf16, the layout of g; v: fp32 [K][M]. M, N multiples of 128. The call enqueues 2 + 15 (+1) launches
+// on `stream` and returns; the workspace must stay untouched until they have run.
+extern "C" int tfb_ns5(const void* g, const void* inv_d, const float* coeffs, void* y, void* v, int K, int M, int N, int wide,
+                       void* workspace, long workspace_bytes, void* stream) {
+  return ns_run(NsStack{g, inv_d, y, v, K, wide}, NsStack{}, NS_INV, coeffs, M, N, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+// tfb_ns5 of two stacks of the same tall shape, each in its own layout, from the denominators themselves (d_type: 1 fp32, 2 bf16, 3 fp16; the
+// reciprocal is taken in fp32): every matrix comes out as tfb_ns5 leaves it, bit for bit. Kb 0: one stack, B's pointers may be NULL.
+extern "C" int tfb_ns5_stacks(const void* ga, const void* da, void* ya, void* va, int Ka, int wide_a, const void* gb, const void* db, void* yb,
+                              void* vb, int Kb, int wide_b, int d_type, const float* coeffs, int M, int N, void* workspace,
+                              long workspace_bytes, void* stream) {
+  if (d_type != NS_D_F32 && d_type != NS_D_BF16 && d_type != NS_D_F16) return TFB_ERR_ARG;
+  return ns_run(NsStack{ga, da, ya, va, Ka, wide_a}, NsStack{gb, db, yb, vb, Kb, wide_b}, d_type, coeffs, M, N, workspace, workspace_bytes, (hipStream_t)stream);
 }

@@ -584,30 +584,47 @@ NS_COEFFS = (
 _NS_WS = {}
 
 
-def ns5(g, d, coeffs=NS_COEFFS):
-    """Five Newton-Schulz iterations on a stack g fp32 [K, r, c] (tall r >= c, or wide: handled as the transposes) from
-    X0 = bf16(bf16(g) / d), d [K] (any float dtype; the reciprocal is taken in fp32 as the reference's sc_tile does).
-    Returns (y bf16 [K, r, c], v fp32 [K, max(r, c)] = the sums of y^2 along the short side)."""
+_NS_D_TYPES = {torch.float32: 1, bf16: 2, torch.float16: 3}
+
+
+def ns5_stacks(stacks, coeffs=NS_COEFFS):
+    """Five Newton-Schulz iterations on one or two stacks [(g, d), ..] whose matrices have the same long and short side: g fp32 [K, r, c]
+    (tall r >= c, or wide: handled as the transposes) from X0 = bf16(bf16(g) / d), d [K] (any float dtype; the reciprocal is taken in
+    fp32 as the reference's sc_tile does). Returns [(y bf16 [K, r, c], v fp32 [K, max(r, c)] = the sums of y^2 along the short side), ..]."""
     import ctypes
-    _chk(g, torch.float32)
-    K, r, c = g.shape
-    wide = r < c
-    M, N = (c, r) if wide else (r, c)
-    inv = (1.0 / d.reshape(-1).float()).contiguous()
-    if inv.numel() != K:
-        raise ValueError("one denominator per matrix")
-    _chk(inv, torch.float32)
+    M, N = max(stacks[0][0].shape[1:]), min(stacks[0][0].shape[1:])
+    args, out, types = [], [], {d.dtype for _, d in stacks}
+    d_type = _NS_D_TYPES.get(types.pop() if len(types) == 1 else None, 0)
+    for g, d in stacks:
+        _chk(g, torch.float32)
+        K, r, c = g.shape
+        if (max(r, c), min(r, c)) != (M, N):
+            raise ValueError("stacks of the same long and short side")
+        d = d.reshape(-1).contiguous()
+        if d.numel() != K:
+            raise ValueError("one denominator per matrix")
+        if not d.is_cuda:
+            raise RuntimeError("tfb ops need device tensors (the HIP kernels are the only implementation)")
+        d = d if d_type else d.float()
+        out.append((torch.empty(K, r, c, dtype=bf16, device=g.device), torch.empty(K, M, dtype=torch.float32, device=g.device)))
+        args.append((g, d, *out[-1], K, int(r < c)))
+    K = sum(a[4] for a in args)
     need = _lib.lib().tfb_ns5_workspace_bytes(K, M, N)
-    # one workspace per (device, stream), grown to the largest stack seen (never one per shape)
-    key = (g.device, torch.cuda.current_stream(g.device).cuda_stream)
+    # one workspace per (device, stream), grown to the largest call seen (never one per shape)
+    dev = stacks[0][0].device
+    key = (dev, torch.cuda.current_stream(dev).cuda_stream)
     ws = _NS_WS.get(key)
     if ws is None or ws.numel() < need:
-        ws = _NS_WS[key] = torch.empty(max(need, 256), dtype=torch.uint8, device=g.device)
-    y = torch.empty(K, r, c, dtype=bf16, device=g.device)
-    v = torch.empty(K, M, dtype=torch.float32, device=g.device)
+        ws = _NS_WS[key] = torch.empty(max(need, 256), dtype=torch.uint8, device=dev)
     co = (ctypes.c_float * 15)(*[float(x) for t in coeffs for x in t])
-    _lib.call("tfb_ns5", _p(g), _p(inv), co, _p(y), _p(v), K, M, N, int(wide), _p(ws), ws.numel(), _stream())
-    return y, v
+    a, b = ([*map(_p, s[:4]), *s[4:]] for s in (args + [(None,) * 4 + (0, 0)])[:2])
+    _lib.call("tfb_ns5_stacks", *a, *b, d_type or 1, co, M, N, _p(ws), ws.numel(), _stream())
+    return out
+
+
+def ns5(g, d, coeffs=NS_COEFFS):
+    """ns5_stacks of one stack: (y, v)."""
+    return ns5_stacks([(g, d)], coeffs)[0]
 
 
 # ------------------------------------------------------------------------------------------ dense bf16 fused MLP
