@@ -292,6 +292,10 @@ def test_nsk_both_stacks(api, dev):
     assert rel_l2(ya, yao) < 2e-2 and rel_l2(yb, ybo) < 2e-2 and rel_l2(va, vao) < 2e-2 and rel_l2(vb, vbo) < 2e-2
     e = api.nsk(ga.to(dev)[:0], gb.to(dev), da.to(dev)[:0], db.to(dev))
     assert e[0].shape == (0, 512, 256) and torch.equal(e[1], yb)
+    co = O.NS_COEFFS[::-1]      # coefficients of the caller's own, with both stacks and with one
+    yc, ybc, _, _ = api.nsk(ga.to(dev), gb.to(dev), da.to(dev), db.to(dev), co)
+    assert rel_l2(yc, O.ns5(ga, da, co)[0]) < 2e-2 and not torch.equal(yc, ya)
+    assert torch.equal(api.nsk(ga.to(dev)[:0], gb.to(dev), da.to(dev)[:0], db.to(dev), co)[1], ybc)
 
 
 @pytest.mark.parametrize("Ka,sa,Kb,sb", [(2, (512, 256), 3, (256, 512)), (1, (384, 384), 4, (384, 384)), (3, (128, 256), 1, (128, 256)),

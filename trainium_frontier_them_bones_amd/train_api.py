@@ -384,14 +384,14 @@ def nsk(ga, gb, d_a, d_b, coeffs=ops.NS_COEFFS):
         if g.shape[0] == 0:
             return (torch.empty(g.shape, dtype=bf16, device=g.device),
                     torch.empty(0, max(g.shape[1], g.shape[2]), dtype=torch.float32, device=g.device))
-        return ops.ns5(g.contiguous(), d)
+        return ops.ns5(g.contiguous(), d, coeffs)
     # Matrices of the same long and short side run as one stack: the launches of a few matrices leave most of the chip idle, and half as many
     # are launched (us, two calls -> one: 1 + 1 matrices of 3072 x 768 326 -> 193, 6 + 6 706 -> 552, 12 + 12 1126 -> 1035; 9 + 9 of 2304 x 768
     # 903 -> 675). Beyond 384 MB of workspace a stack fills it alone (12 + 12 of 4096 x 1024, 503 MB: 2348 -> 2364).
     if (ga.shape[0] and gb.shape[0] and sorted(ga.shape[1:]) == sorted(gb.shape[1:]) and ga.device == gb.device and "ns5" not in _lib.REPLACED
             and ga.shape[0] + gb.shape[0] <= 65535 and _lib.lib().tfb_ns5_workspace_bytes(
                 ga.shape[0] + gb.shape[0], max(ga.shape[1:]), min(ga.shape[1:])) <= 384 << 20):
-        (ya, va), (yb, vb) = ops.ns5_stacks([(ga.contiguous(), d_a), (gb.contiguous(), d_b)])
+        (ya, va), (yb, vb) = ops.ns5_stacks([(ga.contiguous(), d_a), (gb.contiguous(), d_b)], coeffs)
         return ya, yb, va, vb
     ya, va = one(ga, d_a)
     yb, vb = one(gb, d_b)
