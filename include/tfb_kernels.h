@@ -298,8 +298,9 @@ int tfb_attn_bwd(const void* q, const long* q_strides, const void* k, const long
                  const long* v_strides, const void* o, const long* o_strides, const void* d_o, const long* do_strides,
                  void* dq, const long* dq_strides, void* dk, const long* dk_strides, void* dv, const long* dv_strides,
                  const void* lse, void* delta, int B, int H, int T, int D, float scale, void* stream);
-/* Whether (0 = yes) a backward's dQ kernel (which 1) or its dK/dV kernel (which 2) is the one by pairs of wavefronts, under a band nw (0 =
- * none) and for token strides below 2^25 elements. The results do not depend on it. */
+/* Whether (0 = yes) a backward's dQ kernel (which 1) or its dK/dV kernel with 128 keys a workgroup (which 2) is the one by pairs of wavefronts,
+ * or dK/dV runs by pairs with 64 keys a workgroup instead (which 3), under a band nw (0 = none) and for token strides below 2^25 elements. The
+ * results do not depend on it. */
 int tfb_attn_bwd_pairs_applies(int which, int B, int H, int T, int D, int nw);
 /* tfb_attn_bwd for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): the same kernels and results, with the delta scratch taken from a static device

@@ -98,11 +98,12 @@ extern "C" int tfb_attn_bwd(const void* q, const long* qs, const void* k, const 
                            D, scale, stream);
 }
 
-// Whether a backward's dQ kernel (which 1) or its dK/dV kernel (2) is the one by pairs of wavefronts, for token strides that it takes.
+// Whether a backward's dQ kernel (which 1) or its dK/dV kernel with 128 keys a workgroup (2) is the one by pairs of wavefronts, or dK/dV runs by
+// pairs with 64 keys a workgroup instead of either (3), for token strides that they take.
 extern "C" int tfb_attn_bwd_pairs_applies(int which, int B, int H, int T, int D, int nw) {
-  if (which < 1 || which > 2 || B <= 0 || H <= 0 || T <= 0 || T % 128 || (D != 64 && D != 128) || nw < 0) return TFB_ERR_SHAPE;
+  if (which < 1 || which > 3 || B <= 0 || H <= 0 || T <= 0 || T % 128 || (D != 64 && D != 128) || nw < 0) return TFB_ERR_SHAPE;
   const long st[3] = {0, 0, D}, nbh = (long)B * H;
-  const bool yes = which == 1 ? tfb_attn_dq_pair_applies(D, T, nbh, nw, st, st) : D == 128 || tfb_attn_dkdv_pair_applies(T, nbh, nw, st, st);
+  const bool yes = which == 3 ? tfb_attn_dkdv_half_applies(D, T, nbh, nw, st, st) : which == 1 ? tfb_attn_dq_pair_applies(D, T, nbh, nw, st, st) : D == 128 || tfb_attn_dkdv_pair_applies(T, nbh, nw, st, st);
   return yes ? TFB_OK : TFB_ERR_SHAPE;
 }
 

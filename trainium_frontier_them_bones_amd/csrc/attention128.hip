@@ -28,7 +28,7 @@ namespace {
 // =========================================================================================== forward
 template <int D>
 __global__ __launch_bounds__(256, 2) void attnD_fwd_kernel(AttnT q, AttnT k, AttnT v, AttnT o, float* __restrict__ lse, int T,
-                                                           int H, float sl2, int nw) {
+                                                           int H, float sl2, int nw, int turn) {
   typedef Geo<D> G;
   constexpr int TILE = G::TILE, NKS = G::NKS, NDT = G::NDT, NA = 2 * NKS, NB = 4 * NDT;
   constexpr int AH = 4;  // fragments asked for ahead of their MFMA (6: no register left, 1 % slower)
@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256, 2) void attnD_fwd_kernel(AttnT q, AttnT k, Att
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int bx, bh;
-  xcd_block(T / 128, gridDim.y, bx, bh);
+  xcd_block(T / 128, gridDim.y, bx, bh, turn);
   const int b = bh / H, h = bh % H;
   const bf16_t* qp = q.p + b * q.sb + h * q.sh;
   const uint8_t* kp = (const uint8_t*)(k.p + b * k.sb + h * k.sh);
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(256, 2) void attnD_fwd_kernel(AttnT q, AttnT k, Att
 template <int D>
 __global__ __launch_bounds__(256, 2) void attnD_dq_kernel(AttnT q, AttnT k, AttnT v, AttnT go, AttnT dq,
                                                                         float* __restrict__ stats, long rows, int T, int H,
-                                                                        float scale, float sl2, int nw, AttnT o,
+                                                                        float scale, float sl2, int nw, int turn, AttnT o,
                                                                         const float* __restrict__ lse) {
   typedef Geo<D> G;
   constexpr int TILE = G::TILE, NKS = G::NKS, NDT = G::NDT;
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(256, 2) void attnD_dq_kernel(AttnT q, AttnT k, Attn
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int bx, bh;
-  xcd_block(T / 128, gridDim.y, bx, bh);
+  xcd_block(T / 128, gridDim.y, bx, bh, turn);
   const int b = bh / H, h = bh % H;
   const bf16_t* qp = q.p + b * q.sb + h * q.sh;
   const bf16_t* gp = go.p + b * go.sb + h * go.sh;
@@ -526,7 +526,7 @@ template <int D>
 int fwd_launch(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, void* o,
                const long* os, float* lse, int B, int H, int T, float scale, int nw, hipStream_t s) {
   hipLaunchKernelGGL(attnD_fwd_kernel<D>, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
-                     mk(o, os), lse, T, H, scale * LOG2E, nw);
+                     mk(o, os), lse, T, H, scale * LOG2E, nw, first_round(T / 128, B * H, true));
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
@@ -540,7 +540,7 @@ int bwd_launch(const void* q, const long* qs, const void* k, const long* ks, con
     if (st != TFB_OK) return st;
   } else {
     hipLaunchKernelGGL(attnD_dq_kernel<D>, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
-                       mk(go, gos), mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, nw, mk(o, os), lse);
+                       mk(go, gos), mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, nw, first_round(T / 128, B * H, true), mk(o, os), lse);
     TFB_LAUNCH_CHECK();
   }
   return tfb_attn_dkdv_impl(q, qs, k, ks, v, vs, go, gos, dk, dks, dv, dvs, stats, B, H, T, D, scale, nullptr, nullptr, nw, s);

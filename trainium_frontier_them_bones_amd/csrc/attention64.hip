@@ -126,14 +126,14 @@ __device__ __forceinline__ bf16x8 frag_cols(const uint8_t* tile, int dt, int tok
 
 // =========================================================================================== forward
 __global__ __launch_bounds__(256, TFB_FWD64_WPE) void attn64_fwd_kernel(AttnT q, AttnT k, AttnT v, AttnT o, float* __restrict__ lse,
-                                                            int T, int H, float sl2, int nw, int slots) {
+                                                            int T, int H, float sl2, int nw, int slots, int turn) {
   __shared__ __attribute__((aligned(1024))) uint8_t st0[2 * TILE];
   __shared__ __attribute__((aligned(1024))) uint8_t st1[2 * TILE];
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   stagger_start(slots);
   int bx, bh;
-  xcd_block(T / 128, gridDim.y, bx, bh);
+  xcd_block(T / 128, gridDim.y, bx, bh, turn);
   const int b = bh / H, h = bh % H;
   const bf16_t* qp = q.p + b * q.sb + h * q.sh;
   const uint8_t* kp = (const uint8_t*)(k.p + b * k.sb + h * k.sh);
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(256, TFB_FWD64_WPE) void attn64_fwd_kernel(AttnT q,
 __global__ __launch_bounds__(256, 2) void attn64_dkdv_kernel(AttnT q, AttnT k, AttnT v, AttnT go, AttnT dk, AttnT dv,
                                                              const float* __restrict__ stats, long rows, int T, int H,
                                                              float scale, float sl2, const bf16_t* __restrict__ cs,
-                                                             const bf16_t* __restrict__ sn, int nw, int slots) {
+                                                             const bf16_t* __restrict__ sn, int nw, int slots, int turn) {
   constexpr int QT = TFB_DKDV64_QT;       // 64-query tiles per LDS stage (one barrier per stage)
   constexpr int R = 64 * QT, RT = R * 128;  // rows and bytes of a staged Q (dO) tile
   constexpr int STAGE = 2 * RT + 8 * R;    // Q tile, dO tile, R x (-lse / scale), R x (-delta)
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(256, 2) void attn64_dkdv_kernel(AttnT q, AttnT k, A
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   stagger_start(slots);
   int bx, bh;
-  xcd_block(T / 128, gridDim.y, bx, bh);
+  xcd_block(T / 128, gridDim.y, bx, bh, turn);
   const int b = bh / H, h = bh % H;
   const uint8_t* qp = (const uint8_t*)(q.p + b * q.sb + h * q.sh);
   const uint8_t* gp = (const uint8_t*)(go.p + b * go.sb + h * go.sh);
@@ -601,7 +601,7 @@ __global__ __launch_bounds__(256, 2) void attn64_dkdv_kernel(AttnT q, AttnT k, A
 __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, AttnT k, AttnT v, AttnT go, AttnT dq,
                                                            float* __restrict__ stats, long rows, int T, int H,
                                                            float scale, float sl2, const bf16_t* __restrict__ cs,
-                                                           const bf16_t* __restrict__ sn, int nw, int slots, AttnT o,
+                                                           const bf16_t* __restrict__ sn, int nw, int slots, int turn, AttnT o,
                                                            const float* __restrict__ lse) {
   __shared__ __attribute__((aligned(1024))) uint8_t st0[2 * TILE];
   __shared__ __attribute__((aligned(1024))) uint8_t st1[2 * TILE];
@@ -609,7 +609,7 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   stagger_start(slots);
   int bx, bh;
-  xcd_block(T / 128, gridDim.y, bx, bh);
+  xcd_block(T / 128, gridDim.y, bx, bh, turn);
   const int b = bh / H, h = bh % H;
   const bf16_t* qp = q.p + b * q.sb + h * q.sh;
   const bf16_t* gp = go.p + b * go.sb + h * go.sh;
@@ -788,7 +788,7 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
 int tfb_attn64_fwd_impl(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, void* o,
                         const long* os, float* lse, int B, int H, int T, float scale, int nw, hipStream_t s) {
   hipLaunchKernelGGL(attn64_fwd_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(o, os), lse,
-                     T, H, scale * LOG2E, nw, tfb_resident_slots(2));
+                     T, H, scale * LOG2E, nw, tfb_resident_slots(2), first_round(T / 128, B * H, true));
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
@@ -808,13 +808,13 @@ int tfb_attn64_bwd_impl(const void* q, const long* qs, const void* k, const long
   } else {
     hipLaunchKernelGGL(attn64_dq_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
                        mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw,
-                       tfb_resident_slots(2), mk(o, os), lse);
+                       tfb_resident_slots(2), first_round(T / 128, B * H, true), mk(o, os), lse);
     TFB_LAUNCH_CHECK();
   }
-  if (tfb_attn_dkdv_pair_applies(T, (long)B * H, nw, qs, gos))
+  if (tfb_attn_dkdv_pair_applies(T, (long)B * H, nw, qs, gos) || tfb_attn_dkdv_half_applies(64, T, (long)B * H, nw, qs, gos))
     return tfb_attn_dkdv_impl(q, qs, k, ks, v, vs, go, gos, dk, dks, dv, dvs, stats, B, H, T, 64, scale, cos_t, sin_t, nw, s);
   hipLaunchKernelGGL(attn64_dkdv_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
-                     mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw, tfb_resident_slots(2));
+                     mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw, tfb_resident_slots(2), first_round(T / 128, B * H, true));
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }

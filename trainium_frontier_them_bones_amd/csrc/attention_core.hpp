@@ -52,6 +52,26 @@ static inline bool tfb_attn_dkdv_pair_applies(int T, long nbh, int nw, const lon
   const long cus = tfb_resident_slots(1);
   return l.longest > 1 && (l.blocks <= cus || 32 * l.work <= std::min(l.longest + 20, 36L) * cus * l.longest) && tfb_attn_dkdv_strides_ok(qs, gos);
 }
+// dK/dV by pairs with 64 keys a workgroup in place of 128: the longest block is half as long, what a block does besides its loop counts twice. One
+// workgroup for each CU always; beyond, by the work a CU has in units of the longest block of 128, as above: at D = 64 two workgroups share a CU,
+// at D = 128 (141 KB of LDS) one has it alone. dQ and dK/dV, us, 128 keys -> 64, blocks of 128 in brackets:
+//   D = 64   T128 [128] 13.7 -> 12.8, [192] 14.8 -> 15.1; T256 [128] 18.1 -> 15.2, [256] 20.2 -> 18.4, [320] 23.9 -> 24.7; T512 [192] 24.7 -> 21.4,
+//            [320] 29.1 -> 27.9, [384] 30.3 -> 30.5; T1024 [256] 36.4 -> 32.7, [384] 44.9 -> 41.3, [512] 48.0 -> 47.8; T2048 [192] 55.1 -> 48.3, [384] 67.7 ->
+//            66.4, [512] 80.1 -> 79.7, [576] 90.4 -> 91.0; T4096 [256] 100.3 -> 91.7, [384] 119 -> 117, [448] 136 -> 137; bands: 1 T2048 [128] 13.3 -> 12.4,
+//            [192] 15.0 -> 15.0; 2 [256] 20.9 -> 19.6, [384] 30.7 -> 29.7; 4 [256] 27.3 -> 26.1, [384] 42.7 -> 39.8; 8 [192] 36.9 -> 33.2, [256] 39.8 -> 40.0
+//   D = 128  T128 [128] 21.7 -> 18.6, [192] 25.6 -> 27.4; T256 [128] 27.9 -> 23.8, [192] 32.3 -> 32.4; T512 [192] 42.0 -> 40.9, [256] 43.0 -> 43.9;
+//            T1024 [192] 55.6 -> 50.0, [320] 68.2 -> 75.3; T1664 [208] 74.7 -> 66.0, [260] 89.3 -> 90.0; T2048 [256] 93.7 -> 88.4, [320] 114 -> 122; T4096 [256]
+//            162 -> 150, [320] 201 -> 210; bands of T2048: 1 [128] 21.8 -> 18.4, [192] 28.6 -> 30.1; 4 [128] 36.0 -> 31.5, [192] 44.4 -> 51.0
+static inline bool tfb_attn_dkdv_half_applies(int D, int T, long nbh, int nw, const long* qs, const long* gos) {
+  if (!tfb_attn_dkdv_strides_ok(qs, gos)) return false;
+  const AttnLoad l = attn_load(T, nbh, nw);
+  const long cus = tfb_resident_slots(1), nx = T / 128;
+  if (2 * l.blocks <= cus) return true;
+  if (D == 128) return 1000 * l.work <= 535 * cus * l.longest;
+  if (l.longest == 1) return false;
+  const long line = l.longest <= 4 && 4 * l.longest <= nx ? 14 : l.longest == nx && nx >= 8 && nx <= 16 ? 10 : 8;
+  return 10 * l.work <= line * cus * l.longest;
+}
 
 namespace {
 
@@ -120,8 +140,14 @@ __device__ __forceinline__ void store_grad_row(const f32x16 (&acc)[2], float sca
 // ran on alone; T2048 D64 12 heads B3 forward 57 -> 34 us, backward 165 -> 96; B7 103 -> 73, 297 -> 195; T3072 D128 6 heads B2
 // 64 -> 52, 230 -> 174). nx = blocks per (batch, head), nbh = batch*head count. One division and no branch: behind branches the kernels'
 // other arguments were loaded only after it (forward, us: D128 T2048 4 heads 32.6 -> 31.6, 12 heads 34.3 -> 33.3; D64 T256 12 heads 7.1 -> 6.9).
-__device__ __forceinline__ void xcd_block(int nx, int nbh, int& bx, int& bh) {
-  const int gx = gridDim.x, lin = blockIdx.y * gx + blockIdx.x, xcd = lin & 7;
+// turn: the workgroups that start first, one on a CU, where a second will share it with some of them (0: none does). These run in the opposite
+// order, so that the second ones, the shortest, come to the shorter of them and not to the longest (us: forward D128 T1664 24 heads 31.9 -> 29.6,
+// D64 T2048 24 heads 29.1 -> 27.0; dQ and dK/dV of 12 heads 62.1 -> 60.0, with 64 keys a workgroup 55.6 -> 52.8).
+__device__ __forceinline__ void xcd_block(int nx, int nbh, int& bx, int& bh, int turn = 0) {
+  const int gx = gridDim.x;
+  int lin = blockIdx.y * gx + blockIdx.x;
+  const int xcd = lin & 7;
+  if (lin < turn) lin = turn - 8 - lin + 2 * xcd;   // (a multiple of 8: the XCD stays)
   const bool dealt = nbh % 8 == 0, single = gx == nx;
   const unsigned id = dealt ? lin >> 3 : lin, by = single ? (dealt ? nbh >> 3 : nbh) : gx;
   const int quot = (int)(id / by), rem = (int)(id - quot * by);
@@ -150,6 +176,12 @@ __host__ inline unsigned paired_grid(int nx, int nbh, int per_cu) {
   if (nx % 2) return (unsigned)nx;
   const long wgs = (long)(nx / 2) * nbh, slots = tfb_resident_slots(per_cu), rounds = (wgs + slots - 1) / slots;
   return (unsigned)(wgs * 10 >= rounds * slots * 9 ? nx / 2 : nx);
+}
+
+// xcd_block's turn for nx x nbh workgroups of which two share a CU, blocks paired by paired_grid(nx, nbh, 2) or one by one
+__host__ inline int first_round(int nx, int nbh, bool may_pair) {
+  const int cus = (int)tfb_resident_slots(1) & ~7;
+  return (long)nx * nbh > cus && !(may_pair && (int)paired_grid(nx, nbh, 2) != nx) ? cus : 0;
 }
 
 }  // namespace

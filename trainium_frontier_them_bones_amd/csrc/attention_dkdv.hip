@@ -1,5 +1,5 @@
-// dK and dV of causal flash attention on gfx950, one 128-key block per workgroup, two wavefronts to every 32 keys: all launches of D = 128, and
-// those of D = 64 that do not fill the chip.
+// dK and dV of causal flash attention on gfx950, one block of 128 or 64 keys per workgroup, two wavefronts to every 32 keys: all launches of
+// D = 128, and those of D = 64 that do not fill the chip.
 //
 // The first of a pair ("dV") makes S and P of a 32-query half and dV += dO P, the second ("dK") makes dP and dS of it and dK += Q dS; P
 // passes from one to the other through 2 KB of LDS, packed as both hold it, and nothing else does. So a wavefront has one product's
@@ -13,6 +13,8 @@
 // D = 128 has no other kernel: with dQ's launch, over 1 to 512 heads (up to 1536 blocks), pairs take 0.85 - 0.94 of the time at T4096 and T2048,
 // 0.89 - 0.97 at T1024 to T512, 0.93 - 1.00 at T384 (96 heads 46.1 -> 46.1), 0.96 - 0.99 at T256 (512 heads 117.8 -> 116.3), and 0.1 - 0.4 us more where a sequence is one
 // block (8 heads 22.2 -> 22.4, 256 30.4 -> 30.8, 512 55.5 -> 55.8).
+// 64 keys a workgroup (two pairs) where the longest block sets the time: a wavefront alone on its SIMD issues as fast as two together, so half
+// the pairs on a CU take half as long (B1 H12 T2048 D64 35.6 -> 28; attention_core.hpp has the line, and both sides of it).
 #include "attention_slots.hpp"
 
 namespace {
@@ -38,25 +40,26 @@ struct PBlock {  // a 32 x 32 block of P on its way from one wavefront to anothe
   }
 };
 
-template <int D>
-__global__ __launch_bounds__(512, 2) void attn_dkdv_pair_kernel(AttnT q, AttnT k, AttnT v, AttnT go, AttnT dk, AttnT dv,
+template <int D, int PAIRS>
+__global__ __launch_bounds__(128 * PAIRS, 2) void attn_dkdv_pair_kernel(AttnT q, AttnT k, AttnT v, AttnT go, AttnT dk, AttnT dv,
                                                                 const float* __restrict__ stats, long rows, int T, int H, float scale,
                                                                 float sl2, const bf16_t* __restrict__ cs, const bf16_t* __restrict__ sn,
-                                                                int nw) {
+                                                                int nw, int turn) {
   typedef Geo<D> G;
   constexpr int TILE = G::TILE, NKS = G::NKS, NDT = G::NDT;
   constexpr int NI = 2 * NKS + 1;            // items of a half: the accumulator's start, NKS row fragments, NKS column fragments
   constexpr int AH = 4;                      // items asked for ahead of their use
-  constexpr int NL = 16 / G::TPI, SHARE = NL / 2 + 1;  // a wavefront's load instructions for a tile, and for a tile in a half (with statistics)
+  constexpr int KEYS = 32 * PAIRS;
+  constexpr int TL = 4 / PAIRS, NL = 16 / G::TPI * TL, SHARE = NL / 2 + 1;  // a wavefront's load instructions for a tile, and for a tile in a half (with statistics)
   constexpr int STAGE = 2 * TILE + 512;      // Q tile, dO tile, 64 x (-lse / scale), 64 x (-delta)
   static_assert(AH <= NKS && 2 * NDT == NKS, "the items ahead of the next half are its start and rows");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * STAGE + 2 * 4 * 2048];  // and P: two halves of four pairs
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * STAGE + 2 * PAIRS * 2048];  // and P: two halves of every pair
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave & 3;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), w = wave % PAIRS;
   int bx, bh;
-  xcd_block(T / 128, gridDim.y, bx, bh);
+  xcd_block(T / KEYS, gridDim.y, bx, bh, turn);
   const int b = bh / H, h = bh % H;
-  const int nx = T / 128, npass = paired_passes(nx);
+  const int nx = T / KEYS, npass = PAIRS == 4 ? paired_passes(nx) : 1;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t*)lds;
   const uint32_t pa = lds0 + 4 * STAGE + w * 2048 + lane * 16;
 
@@ -68,24 +71,26 @@ __global__ __launch_bounds__(512, 2) void attn_dkdv_pair_kernel(AttnT q, AttnT k
   auto run = [&](auto ROLE, int pass) __attribute__((always_inline)) {
     constexpr bool DK = decltype(ROLE)::value;
     constexpr int ROWT = DK ? TILE : 0, COLT = DK ? 0 : TILE, STAT = 2 * TILE + (DK ? 256 : 0);
-    const int kb = paired_block(nx, bx, pass, false);  // low key blocks see the most query tiles
-    const int mykey = kb * 128 + w * 32 + lr;
-    // with a band the keys of tile kb are seen by the queries of tiles kb .. kb + nw - 1 only
-    const int nall = nx - kb, nt = 2 * (nw > 0 && nw < nall ? nw : nall), nh = 2 * nt;  // 64-query tiles, 32-query halves (4 or more)
+    const int kb = PAIRS == 4 ? paired_block(nx, bx, pass, false) : bx;  // low key blocks see the most query tiles
+    const int mykey = kb * KEYS + w * 32 + lr;
+    // with a band the keys of a 128-token tile i are seen by the queries of tiles i .. i + nw - 1 only
+    const int t0 = kb * (KEYS / 64), nall = T / 64 - t0, nband = 2 * (t0 / 2 + nw) - t0;
+    const int nt = nw > 0 && nband < nall ? nband : nall, nh = 2 * nt;  // 64-query tiles, 32-query halves (PAIRS or more)
     const AttnT& rt = DK ? go : q;
     const AttnT& ft = DK ? v : k;
     const long rst = rt.st * 2;
-    const uint8_t* rp = (const uint8_t*)(rt.p + b * rt.sb + h * rt.sh + (long)kb * 128 * rt.st);
-    const float* sp = stats + (DK ? 0 : rows) + (long)bh * T + kb * 128;
-    TileLoad<D, NL> ld;
-    ld.init(rst, w, lane);
+    const uint8_t* rp = (const uint8_t*)(rt.p + b * rt.sb + h * rt.sh + (long)kb * KEYS * rt.st);
+    const float* sp = stats + (DK ? 0 : rows) + (long)bh * T + kb * KEYS;
+    TileLoad<D, NL / TL> ld[TL];  // (two pairs: each wavefront has two wavefronts' share)
+#pragma unroll
+    for (int i = 0; i < TL; ++i) ld[i].init(rst, w + 2 * i, lane);
     // (a load past the last tile brings that one again, into a stage nobody reads any more)
     auto load_one = [&](int tile, auto half, int i) __attribute__((always_inline)) {
       constexpr int hf = decltype(half)::value;
       const int from = tile < nt ? tile : nt - 1;
       uint8_t* to = lds + (tile & 3) * STAGE;
       if (i < NL / 2)
-        ld.issue_one(i + hf * (NL / 2), rp + (long)from * 64 * rst, rst, to + ROWT);
+        ld[TL == 1 ? 0 : hf].issue_one(TL == 1 ? i + hf * (NL / 2) : i, rp + (long)from * 64 * rst, rst, to + ROWT);
       else
         __builtin_amdgcn_global_load_lds((glb_void_t*)(sp + from * 64 + lane), (lds_void_t*)(to + STAT), 4, 0, 0);
     };
@@ -182,8 +187,8 @@ __global__ __launch_bounds__(512, 2) void attn_dkdv_pair_kernel(AttnT q, AttnT k
       pin(xw[x]);
     };
     // P's two places alternate
-    auto p_put = [&](auto par) __attribute__((always_inline)) { pb.template put<decltype(par)::value * 8192>(pa, xw); };
-    auto p_get = [&](auto par) __attribute__((always_inline)) { pb.template get<decltype(par)::value * 8192>(pa); };
+    auto p_put = [&](auto par) __attribute__((always_inline)) { pb.template put<decltype(par)::value * PAIRS * 2048>(pa, xw); };
+    auto p_get = [&](auto par) __attribute__((always_inline)) { pb.template get<decltype(par)::value * PAIRS * 2048>(pa); };
     auto begin = [&](auto par) __attribute__((always_inline)) {  // the barrier in front of step u, u > 0
       if constexpr (decltype(par)::value == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(SHARE) : "memory");
       asm volatile("s_barrier" ::: "memory");
@@ -303,9 +308,9 @@ __global__ __launch_bounds__(512, 2) void attn_dkdv_pair_kernel(AttnT q, AttnT k
         word_of(i, Xi{});
       });
     };
-    auto p_put_at = [&](int u) __attribute__((always_inline)) { pb.template put<0>(pa + (u & 1) * 8192, xw); };
+    auto p_put_at = [&](int u) __attribute__((always_inline)) { pb.template put<0>(pa + (u & 1) * (PAIRS * 2048), xw); };
     auto p_get_at = [&](int u) __attribute__((always_inline)) {
-      pb.template get<0>(pa + (u & 1) * 8192);
+      pb.template get<0>(pa + (u & 1) * (PAIRS * 2048));
       pb.template landed<0>();
     };
 
@@ -371,7 +376,7 @@ __global__ __launch_bounds__(512, 2) void attn_dkdv_pair_kernel(AttnT q, AttnT k
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   };
   for (int pass = 0; pass < npass; ++pass) {
-    if (wave < 4) run(std::false_type{}, pass);
+    if (wave < PAIRS) run(std::false_type{}, pass);
     else run(std::true_type{}, pass);
     if (pass + 1 < npass) __syncthreads();  // the stages are free for the partner block
   }
@@ -383,14 +388,16 @@ __global__ __launch_bounds__(512, 2) void attn_dkdv_pair_kernel(AttnT q, AttnT k
 int tfb_attn_dkdv_impl(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, const void* go,
                        const long* gos, void* dk, const long* dks, void* dv, const long* dvs, const float* stats, int B, int H, int T,
                        int D, float scale, const void* cos_t, const void* sin_t, int nw, hipStream_t s) {
-  const long rows = (long)B * H * T;
-  const dim3 grid(paired_grid(T / 128, B * H, 1), B * H);
-  if (D == 64)
-    hipLaunchKernelGGL(attn_dkdv_pair_kernel<64>, grid, dim3(512), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos), mk(dk, dks), mk(dv, dvs), stats,
-                       rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw);
-  else
-    hipLaunchKernelGGL(attn_dkdv_pair_kernel<128>, grid, dim3(512), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos), mk(dk, dks), mk(dv, dvs), stats,
-                       rows, T, H, scale, scale * LOG2E, nullptr, nullptr, nw);
+  const long rows = (long)B * H * T, nbh = (long)B * H;
+  const bool half = tfb_attn_dkdv_half_applies(D, T, nbh, nw, qs, gos);
+  const dim3 grid(half ? T / 64 : paired_grid(T / 128, B * H, 1), B * H), block(half ? 256 : 512);
+  const bf16_t *cs = D == 64 ? (const bf16_t*)cos_t : nullptr, *sn = D == 64 ? (const bf16_t*)sin_t : nullptr;
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos), mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale,
+                       scale * LOG2E, cs, sn, nw, half ? first_round(T / 64, B * H, false) : 0);
+  };
+  if (D == 64) half ? launch(attn_dkdv_pair_kernel<64, 2>) : launch(attn_dkdv_pair_kernel<64, 4>);
+  else half ? launch(attn_dkdv_pair_kernel<128, 2>) : launch(attn_dkdv_pair_kernel<128, 4>);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }

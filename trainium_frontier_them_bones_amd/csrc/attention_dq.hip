@@ -28,7 +28,7 @@ struct DsTile {  // dS of 32 queries and 64 keys, packed: fragment i is the oper
 template <int D>
 __global__ __launch_bounds__(256, 2) void attn_dq_pair_kernel(AttnT q, AttnT k, AttnT v, AttnT go, AttnT dq, float* __restrict__ stats, long rows,
                                                               int T, int H, float scale, float sl2, const bf16_t* __restrict__ cs,
-                                                              const bf16_t* __restrict__ sn, int nw, AttnT o, const float* __restrict__ lse) {
+                                                              const bf16_t* __restrict__ sn, int nw, AttnT o, const float* __restrict__ lse, int turn) {
   typedef Geo<D> G;
   constexpr int TILE = G::TILE, NKS = G::NKS, NDT = G::NDT, MDT = NDT / 2;  // MDT: 32-column tiles of dQ that are this wavefront's
   constexpr int AH = 4, NL = 16 / G::TPI;     // items asked for ahead of their use; load instructions of a wavefront for a K or V tile
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(256, 2) void attn_dq_pair_kernel(AttnT q, AttnT k, 
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), pair = wave >> 1, half = wave & 1;
   const int nx = T / 64;
   int bx, bh;
-  xcd_block(nx, gridDim.y, bx, bh);
+  xcd_block(nx, gridDim.y, bx, bh, turn);
   const int b = bh / H, h = bh % H, qb = nx - 1 - bx;   // the most tiles first
   const int myq = qb * 64 + pair * 32 + lr;
   const int n = qb + 1, t0 = band_first_tile(qb >> 1, nw);  // tile n - 1 is over the workgroup's own tokens
@@ -311,10 +311,10 @@ int tfb_attn_dq_pair_impl(const void* q, const long* qs, const void* k, const lo
   const dim3 grid(T / 64, B * H);
   if (D == 64)
     hipLaunchKernelGGL(attn_dq_pair_kernel<64>, grid, dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos), mk(dq, dqs), stats, rows, T, H,
-                       scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw, mk(o, os), lse);
+                       scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw, mk(o, os), lse, first_round(T / 64, B * H, false));
   else
     hipLaunchKernelGGL(attn_dq_pair_kernel<128>, grid, dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos), mk(dq, dqs), stats, rows, T, H,
-                       scale, scale * LOG2E, nullptr, nullptr, nw, mk(o, os), lse);
+                       scale, scale * LOG2E, nullptr, nullptr, nw, mk(o, os), lse, first_round(T / 64, B * H, false));
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
