@@ -98,6 +98,7 @@ struct EpiStoreRope {
   const bf16_t* cs;  // [T][32]
   const bf16_t* sn;
   int T, rot_cols;
+  FastDiv d_T;
   struct pre_t {  // the chunk's cos / sin values, requested before the k-loop
     u32x4 c, s;
   };
@@ -128,23 +129,25 @@ struct EpiStoreRope {
     }
     *(u32x4*)(out + (long)q * ld + p) = x;
   }
-  // the 256 x 256 kernel's protocol: the same from the rounded products
+  // the 256 x 256 kernel's protocol: the same from the rounded products, a chunk of a head's first half with its partner
+  static constexpr int kPartner = 32;
   __device__ __forceinline__ float pre(float x) const { return x; }
-  __device__ __forceinline__ void chunk(int p, int q, const u32x4& xin, const u32x4& y, const pre_t& tab) const {
-    u32x4 x = xin;
+  __device__ __forceinline__ long table(int p, int q) const { return (long)(q - fastdiv(q, d_T) * T) * 32 + (p & 31); }
+  __device__ __forceinline__ const void* at(int p, int q) const { return cs + table(p, q); }
+  __device__ __forceinline__ const void* at2(int p, int q) const { return sn + table(p, q); }
+  __device__ __forceinline__ void chunk2(int p, int q, u32x4 x, u32x4 y, const u32x4& c, const u32x4& s) const {
     if (p < rot_cols) {
-      const bool low = (p & 32) == 0;
-      const u32x4 c = tab.c, s = tab.s;
-      u32x4 o;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const float x0 = bflo(x[k]), x1 = bfhi(x[k]), y0 = bflo(y[k]), y1 = bfhi(y[k]);
         const float c0 = bflo(c[k]), c1 = bfhi(c[k]), s0 = bflo(s[k]), s1 = bfhi(s[k]);
-        o[k] = low ? pack2bf(x0 * c0 + y0 * s0, x1 * c1 + y1 * s1) : pack2bf(x0 * c0 - y0 * s0, x1 * c1 - y1 * s1);
+        x[k] = pack2bf(x0 * c0 + y0 * s0, x1 * c1 + y1 * s1);
+        y[k] = pack2bf(y0 * c0 - x0 * s0, y1 * c1 - x1 * s1);
       }
-      x = o;
     }
-    *(u32x4*)(out + (long)q * ld + p) = x;
+    bf16_t* o = out + (long)q * ld + p;
+    *(u32x4*)o = x;
+    *(u32x4*)(o + 32) = y;
   }
 };
 
@@ -230,7 +233,7 @@ extern "C" int tfb_qkv_rope_fwd(const void* x, const void* w, const void* cos_t,
     return TFB_ERR_SHAPE;
   using Cfg = GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>;
   GemmOperand P{(const uint8_t*)w, (long)K * 2}, Q{(const uint8_t*)x, (long)K * 2};
-  EpiStoreRope e{(bf16_t*)out, (long)N, (const bf16_t*)cos_t, (const bf16_t*)sin_t, T, rot_cols};
+  EpiStoreRope e{(bf16_t*)out, (long)N, (const bf16_t*)cos_t, (const bf16_t*)sin_t, T, rot_cols, fastdiv_make(T)};
   int st;
   if (gemm_ring_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream, st)) return st;
   if (gemm_pp_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, true, e, (hipStream_t)stream, st)) return st;

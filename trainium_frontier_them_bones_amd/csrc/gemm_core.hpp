@@ -695,6 +695,7 @@ struct EpiStoreRes {
   }
   // the same from the rounded product (the 256 x 256 kernel's epilogue protocol: pre() before the rounding, chunk() after)
   __device__ __forceinline__ float pre(float x) const { return x; }
+  __device__ __forceinline__ const void* at(int p, int q) const { return res + (long)q * ld + p; }
   __device__ __forceinline__ void chunk(int p, int q, const u32x4& v, const pre_t& r) const {
     float a[8], b[8];
     unpack8bf(v, a);

@@ -80,6 +80,11 @@ struct PpArgs {
   int ngroups;
   FastDiv d_ipx;
 };
+// The distance of the outputs that an epilogue takes together (0: none)
+template <class T, class = void>
+struct partner_of : std::integral_constant<int, 0> {};
+template <class T>
+struct partner_of<T, std::void_t<decltype(T::kPartner)>> : std::integral_constant<int, T::kPartner> {};
 template <class T, class = void>
 struct has_experts : std::false_type {};
 template <class T>
@@ -87,9 +92,10 @@ struct has_experts<T, std::void_t<decltype(T::kExperts)>> : std::true_type {};
 
 // Epilogue protocol of this kernel (every epilogue of the library rounds f(accumulator) to bf16 first):
 //   float pre(float acc)                      applied to every accumulator before its rounding to bf16;
-//   void chunk(p, q, v [, vp] [, pre_t])      8 consecutive rounded outputs D[p .. p + 7][q] as four packed bf16 pairs
-//                                             (p % 8 == 0); with kPartner32 also the 8 values 32 outputs away (p ^ 32); with a
-//                                             pre_t / prefetch(p, q) the operand requested before the block was staged.
+//   void chunk(p, q, v [, pre_t])             8 consecutive rounded outputs D[p .. p + 7][q] as four packed bf16 pairs (p % 8 == 0);
+//                                             with a pre_t (16 bytes) the operand from at(p, q) that the chunk needs;
+//   void chunk2(p, q, lo, hi, a, b)           with kPartner: the outputs from p and those kPartner (32 or 64) further on, a and b
+//                                             the 16 bytes from at(p, q) and at2(p, q).
 typedef short tfb_s16x8 __attribute__((ext_vector_type(8)));
 template <int OFF>
 __device__ __forceinline__ tfb_s16x4 tfb_lds_read_tr64(uint32_t addr) {
@@ -126,7 +132,12 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   constexpr bool NARROW = SHAPE != TFB_PP_256x256, QX = SHAPE == TFB_PP_256x192;
   constexpr int TP = SHAPE == TFB_PP_192x256 ? 192 : 256, TQ = QX ? 192 : 256;
   constexpr int LAYX = QX ? LAYQ : LAYP, LAYY = QX ? LAYP : LAYQ;
-  static_assert(!NARROW || (!kF32 && !has_experts<Epi>::value && !has_partner32<Epi>::value), "a narrow tile's half 1 has 32 rows of a wavefront");
+  constexpr int kPartner = partner_of<Epi>::value;
+  static_assert(!NARROW || (!kF32 && !has_experts<Epi>::value && !kPartner), "a narrow tile's half 1 has 32 rows of a wavefront");
+  // A partner 64 outputs away: a wavefront's two MFMA tiles of a P half are rows 32 wr .. and 64 + 32 wr ..
+  constexpr int XROWS = kPartner == 64 ? 32 : 64, XTILE = kPartner == 64 ? 64 : 32;  // rows of X from one group to the other; from tile i = 0 to 1
+  static_assert(kPartner != 64 || LAYX == TFB_K_CONTIG, "the fragments' rows");
+  constexpr bool kPipe = has_prefetch<Epi>::value;  // the epilogue reads an operand of its own
   static_assert(!NARROW || LAYX == TFB_K_CONTIG || ES == 2, "half a quarter of fp8 rows");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * 65536];
   __shared__ __attribute__((aligned(1024))) uint8_t stg_all[8 * 4096];  // epilogue staging, 4 KB per wavefront
@@ -266,7 +277,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   [[maybe_unused]] uint32_t ax1[4];  // of X half 1 of a narrow tile, where a wavefront's rows are wr * 32 ..
   {
     const uint32_t lbase = (uint32_t)(size_t)(tfb_lds_u8*)lds;
-    const int rx = wr * 64 + lr, rx1 = wr * 32 + lr, ry = wc * 32 + lr;
+    const int rx = wr * XROWS + lr, rx1 = wr * 32 + lr, ry = wc * 32 + lr;
     // k-contiguous, one address per k-step. bf16: k-step s (16 k) of a row is chunk 2 s + lh; fp8: k-step s (64 k) is
     // chunks 4 s + 2 lh, + 1: entry 2 s + u
 #pragma unroll
@@ -334,7 +345,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         fa[0][s] = tfb_lds_read128<h * 16384, r128_t>(ax[s]);
-        fa[1][s] = tfb_lds_read128<h * 16384 + 4096, r128_t>(ax[s]);
+        fa[1][s] = tfb_lds_read128<h * 16384 + XTILE * 128, r128_t>(ax[s]);
       }
     } else {
       fa[0][0] = tr_frag(std::integral_constant<int, h * 16384>{}, ax[0]);
@@ -451,22 +462,46 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   //   64 p (X = P, two tiles): row q = 128 bytes, 16-byte chunk c at slot c ^ ((q >> 1) & 7) (the 8-byte writes and the 16-byte
   //   reads then use the banks evenly), a row's 64 outputs on 8 consecutive lanes;
   //   32 p: row q = 64 bytes, chunk c at slot c ^ ((q >> 2) & 3), a row's outputs on 4 lanes; X = Q: tile i is rows 32 i .. of q.
-  constexpr bool kPrefetch = has_prefetch<Epi>::value;
-  auto store_block = [&](auto HX, auto HY, long tp0, long tq0) __attribute__((always_inline)) {
-    constexpr int hx = decltype(HX)::value, hy = decltype(HY)::value, NI = NARROW && hx ? 1 : 2;
-    constexpr bool wide = !QX && NI == 2;
-    const int x = hx * 128 + wr * (32 * NI), y = hy * 128 + wc * 32;
-    const int pb = (int)tp0 + (QX ? y : x), qb = (int)tq0 + (QX ? x : y);
-    constexpr int NCH = wide ? 4 : QX ? 2 * NI : 2, RSTEP = wide ? 8 : 16;  // chunks of a lane, rows apart
-    const int ch = wide ? lane & 7 : lane & 3, row0 = wide ? lane >> 3 : lane >> 2;
-    // the epilogue's own operand: all chunks requested up front when that is 16 registers, else one ahead
-    typedef typename prefetch_type<Epi>::type pre_t;
-    constexpr int kAhead = sizeof(pre_t) <= 16 ? NCH : 1;
-    [[maybe_unused]] pre_t pre[NCH];
-    if constexpr (kPrefetch) {
+  // The epilogue's own operand (a residual, rotation tables) is four 16-byte loads a lane and block, requested one store ahead by request_pre().
+  u32x4 pre[4] = {};
+  auto here = [](int x) __attribute__((always_inline)) {  // (what is made of it is not kept in registers across the loop)
+    if constexpr (kPipe) asm volatile("" : "+v"(x));
+    return x;
+  };
+  auto load_pre = [&](int k, const void* g) __attribute__((always_inline)) {
+    if constexpr (kPartner) asm volatile("global_load_dwordx4 %0, %1, off" : "+v"(pre[k]) : "v"(g) : "memory");
+    else asm volatile("global_load_dwordx4 %0, %1, off nt" : "+v"(pre[k]) : "v"(g) : "memory");  // (read once)
+  };
+  auto wait_pre = [&](auto AFTER) __attribute__((always_inline)) {  // AFTER: vector memory instructions issued since
+    auto& r = pre;
+    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(decltype(AFTER)::value) : "memory");
+  };
+  // a block's place: its first p and q, a lane's chunk and first row, rows from one of its chunks to the next, chunks
+  auto block_p = [&](auto HX, auto HY, long tp0) { return (int)tp0 + (QX ? decltype(HY)::value * 128 + wc * 32
+                                                                         : decltype(HX)::value * 128 + wr * (NARROW && decltype(HX)::value ? 32 : XROWS)); };
+  auto block_q = [&](auto HX, auto HY, long tq0) { return (int)tq0 + (QX ? decltype(HX)::value * 128 + wr * (NARROW && decltype(HX)::value ? 32 : 64)
+                                                                         : decltype(HY)::value * 128 + wc * 32); };
+  auto request_pre = [&](auto HX, auto HY, long tp0, long tq0, auto FROM) __attribute__((always_inline)) {
+    constexpr int hx = decltype(HX)::value, NI = NARROW && hx ? 1 : 2, from = decltype(FROM)::value;
+    constexpr bool wide = !QX && NI == 2 && !kPartner;
+    constexpr int NCH = wide ? 4 : kPartner ? 2 : QX ? 2 * NI : 2, RSTEP = wide ? 8 : 16;
+    const int ln = here(lane), p = block_p(HX, HY, tp0) + 8 * (wide ? ln & 7 : ln & 3), q = block_q(HX, HY, tq0) + (wide ? ln >> 3 : ln >> 2);
+    if constexpr (kPipe) {
 #pragma unroll
-      for (int k = 0; k < kAhead; ++k) pre[k] = epi.prefetch(pb + 8 * ch, qb + row0 + RSTEP * k);
+      for (int k = 0; k < NCH; ++k) {
+        if constexpr (kPartner != 0) {
+          load_pre(2 * k, epi.at(p, q + RSTEP * k));
+          load_pre(2 * k + 1, epi.at2(p, q + RSTEP * k));
+        } else {
+          load_pre(from + k, epi.at(p, q + RSTEP * k));
+        }
+      }
     }
+  };
+  auto store_block = [&](auto HX, auto HY, long tp0, long tq0, auto FROM) __attribute__((always_inline)) {
+    constexpr int hx = decltype(HX)::value, hy = decltype(HY)::value, NI = NARROW && hx ? 1 : 2, from = decltype(FROM)::value;
+    constexpr bool wide = !QX && NI == 2;
+    const int pb = block_p(HX, HY, tp0), qb = block_q(HX, HY, tq0), ln = here(lane);
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
@@ -480,23 +515,24 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
         }
       }
     __builtin_amdgcn_wave_barrier();
+    if constexpr (kPartner != 0) {  // a lane takes a chunk of the block's first 32 outputs and its partner together
 #pragma unroll
-    for (int k = 0; k < NCH; ++k) {
-      const int row = row0 + RSTEP * k;
-      const u32x4 v = wide ? *(const u32x4*)(stg + row * 128 + ((ch ^ ((row >> 1) & 7)) << 4))
-                           : *(const u32x4*)(stg + row * 64 + ((ch ^ ((row >> 2) & 3)) << 4));
-      const int p = pb + 8 * ch, q = qb + row;
-      if constexpr (kPrefetch) {
-        if (k + kAhead < NCH) pre[k + kAhead] = epi.prefetch(p, qb + row0 + RSTEP * (k + kAhead));
+      for (int k = 0; k < 2; ++k) {
+        const int row = (ln >> 2) + 16 * k, ch = ln & 3;
+        const u32x4 lo = *(const u32x4*)(stg + row * 128 + ((ch ^ ((row >> 1) & 7)) << 4));
+        const u32x4 hi = *(const u32x4*)(stg + row * 128 + (((ch + 4) ^ ((row >> 1) & 7)) << 4));
+        if constexpr (!kF32) epi.chunk2(pb + 8 * ch, qb + row, lo, hi, pre[2 * k], pre[2 * k + 1]);
       }
-      if constexpr (has_partner32<Epi>::value) {
-        const u32x4 vp = *(const u32x4*)(stg + row * 128 + (((ch ^ 4) ^ ((row >> 1) & 7)) << 4));  // 32 outputs away
-        if constexpr (kPrefetch) epi.chunk(p, q, v, vp, pre[k]);
-        else epi.chunk(p, q, v, vp);
-      } else if constexpr (kPrefetch) {
-        epi.chunk(p, q, v, pre[k]);
-      } else if constexpr (!kF32) {
-        epi.chunk(p, q, v);
+    } else {
+      constexpr int NCH = wide ? 4 : QX ? 2 * NI : 2, RSTEP = wide ? 8 : 16;  // chunks of a lane, rows apart
+      const int ch = wide ? ln & 7 : ln & 3, row0 = wide ? ln >> 3 : ln >> 2;
+#pragma unroll
+      for (int k = 0; k < NCH; ++k) {
+        const int row = row0 + RSTEP * k;
+        const u32x4 v = wide ? *(const u32x4*)(stg + row * 128 + ((ch ^ ((row >> 1) & 7)) << 4))
+                             : *(const u32x4*)(stg + row * 64 + ((ch ^ ((row >> 2) & 3)) << 4));
+        if constexpr (kPipe) epi.chunk(pb + 8 * ch, qb + row, v, pre[from + k]);
+        else if constexpr (!kF32) epi.chunk(pb + 8 * ch, qb + row, v);
       }
     }
     __builtin_amdgcn_wave_barrier();
@@ -538,131 +574,187 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   readB(H0{}, fb0);
   bool have_prev = false;  // the previous tile's accumulators are still to be stored
   long pp0 = 0, pq0 = 0;   // its origin
-  for (;;) {
-    // the workgroup's next work item (its first k-tiles are requested by this one's last iterations); past the end: this
-    // one again (loads nobody reads, from valid memory)
-    const int wn = w + w_step;
-    long pn = p0, qn = q0;
-    int splitn = split, k0n = k0, nktn = nkt;
+  // the workgroup's next work item (its first k-tiles are requested by this one's last iterations); past the end: this
+  // one again (loads nobody reads, from valid memory)
+  int wn, splitn, k0n, nktn;
+  long pn, qn;
+  const uint8_t *gxn, *gyn;
+  auto look_ahead = [&]() __attribute__((always_inline)) {
+    wn = w + w_step;
+    pn = p0;
+    qn = q0;
+    splitn = split;
+    k0n = k0;
+    nktn = nkt;
     if (wn < w_end) {
       tile_of(wn, pn, qn, splitn);
       krange(splitn, k0n, nktn);
     }
-    const uint8_t* gxn = origin(sx, QX ? qn : pn, k0n);
-    const uint8_t* gyn = origin(sy, QX ? pn : qn, k0n);
-
-    // One k-tile. In a tile's first iteration the MFMAs start from zero, and each accumulator block of the PREVIOUS tile is
-    // stored in the memory cluster in front of the MFMA cluster that overwrites it: the stores of one group (4 KB per
-    // wavefront and cluster) run under the other group's MFMAs.
-    auto iter = [&](auto FIRST, int kt) __attribute__((always_inline)) {
-      constexpr bool first = decltype(FIRST)::value;
-      // k positions one and two ahead in the workgroup's stream of k-tiles
-      const bool in1 = kt + 1 < nkt, in2 = kt + 2 < nkt;
-      const long k1 = in1 ? kt + 1 : 0, k2 = in2 ? kt + 2 : has_experts<Epi>::value && nkt < 2 ? 0 : kt + 2 - nkt;
-      const uint8_t* gx1 = (in1 ? gx : gxn) + k1 * sx.kstep;
-      const uint8_t* gx2 = (in2 ? gx : gxn) + k2 * sx.kstep;
-      const uint8_t* gy2 = (in2 ? gy : gyn) + k2 * sy.kstep;
-      auto store = [&](auto HX, auto HY) __attribute__((always_inline)) {
-        if constexpr (!kF32) {
-          if (first && have_prev) store_block(HX, HY, pp0, pq0);
-        }
-      };
-      if constexpr (!NARROW) {
-        // c0 (the Y fragments of half 0 were requested in the previous k-tile's c7)
-        readA(H0{});
-        dma(S ^ 1, 0, 1, gx1);
-        store(H0{}, H0{});
-        TFB_SBAR();
-        // c1
-        waitB(fb0);
-        waitA();
-        mma(FIRST, H0{}, H0{}, fb0);
-        TFB_SBAR();
-        // c2
-        readB(H1{}, fb1);
-        dma(S, 0, 0, gx2);
-        store(H0{}, H1{});
-        TFB_SBAR();
-        // c3
-        waitB(fb1);
-        mma(FIRST, H0{}, H1{}, fb1);
-        TFB_SBAR();
-        // c4
-        readA(H1{});
-        dma(S, 1, 0, gy2);
-        store(H1{}, H0{});
-        TFB_SBAR();
-        // c5
-        waitA();
-        mma(FIRST, H1{}, H0{}, fb0);
-        // Completion is reported in issue order, stores included. Everything up to the quarter requested in c0 has to be
-        // there one cluster before the other group's matching wait: all but the two quarters requested since (4
-        // instructions), and in a first iteration with stores all but those and the 12 stores (c0's four were issued
-        // behind its loads). After the barrier that ends c6 both groups have waited, so the next k-tile is complete.
-        if (!kF32 && first && have_prev) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        TFB_SBAR();
-        // c6
-        dma(S, 1, 1, gy2);
-        store(H1{}, H1{});
-        TFB_SBAR();
-        // c7: the next k-tile's first Y fragments are requested under this cluster's MFMAs (fb0 was last read in c5)
-        readB(H0{}, fb0, 0x10000u);
-        mma(FIRST, H1{}, H1{}, fb1);
-        TFB_SBAR();
-      } else {
-        // X half 1 is one MFMA tile a wavefront: three MFMA clusters of 8 instead of four. Quarters 0 are requested two k-tiles
-        // ahead, quarters 1 one ahead. A cluster's reads are waited for in front of its barrier (the requests behind them take longer),
-        // so a quarter is requested again only when a barrier has passed since either group had the old one in registers.
-        const uint8_t* gy1 = (in1 ? gy : gyn) + k1 * sy.kstep;
-        // c0 (Y half 0: see c5)
-        readA(H0{});
-        dma(S ^ 1, 1, 1, gy1);
-        dma(S ^ 1, 0, 1, gx1);
-        store(H0{}, H0{});
-        waitB(fb0);
-        waitA();
-        TFB_SBAR();
-        // c1
-        mma(FIRST, H0{}, H0{}, fb0);
-        TFB_SBAR();
-        // c2
-        readB(H1{}, fb1);
-        store(H0{}, H1{});
-        waitB(fb1);
-        TFB_SBAR();
-        // c3
-        mma(FIRST, H0{}, H1{}, fb1);
-        // The next k-tile's quarters 0 (requested in the previous iteration's c4) have to be there: all but what was requested
-        // since, c0's loads and in a first iteration with stores the 8 stores of c0 and c2. c5 reads them behind two more barriers.
-        if (first && have_prev) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + NX1 + 8) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + NX1) : "memory");
-        TFB_SBAR();
-        // c4
-        readA(H1{});
-        dma(S, 0, 0, gx2);
-        dma(S, 1, 0, gy2);
-        store(H1{}, H0{});
-        store(H1{}, H1{});
-        waitA1();
-        TFB_SBAR();
-        // c5
-        mma(FIRST, H1{}, H0{}, fb0);
-        readB(H0{}, fb0, 0x10000u);
-        mma(FIRST, H1{}, H1{}, fb1);
-        // The next k-tile's quarters 1 (c0) likewise: all but c4's four loads, and with stores the 8 of c0 and c2 and c4's 4.
-        if (first && have_prev) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-        TFB_SBAR();
+    gxn = origin(sx, QX ? qn : pn, k0n);
+    gyn = origin(sy, QX ? pn : qn, k0n);
+  };
+  auto go_on = [&]() __attribute__((always_inline)) {
+    p0 = pn;
+    q0 = qn;
+    split = splitn;
+    k0 = k0n;
+    nkt = nktn;
+    gx = gxn;
+    gy = gyn;
+  };
+  // One k-tile. In a tile's first iteration the MFMAs start from zero, and each accumulator block of the PREVIOUS tile is
+  // stored in the memory cluster in front of the MFMA cluster that overwrites it: the stores of one group (4 KB per
+  // wavefront and cluster) run under the other group's MFMAs. An epilogue with an operand of its own (kPipe) has it requested behind the
+  // stores of the cluster before (the first block's in the tile's last iteration) and in front of that cluster's operand loads: reported in issue
+  // order, it does not wait for them. Requested in its own cluster behind those loads, every one of a tile's four blocks waited for a trip to
+  // HBM (the QKV projection with its rotation, 32768 x 2304 x 768: 148 us, of 113 without; now 120). The requests take the registers as
+  // operands that go in and come out, so that no copy of them is made while a load is on its way.
+  auto iter = [&](auto FIRST, int kt) __attribute__((always_inline)) {
+    constexpr bool first = decltype(FIRST)::value, stores = first && !kF32;
+    // k positions one and two ahead in the workgroup's stream of k-tiles
+    const bool in1 = kt + 1 < nkt, in2 = kt + 2 < nkt;
+    const long k1 = in1 ? kt + 1 : 0, k2 = in2 ? kt + 2 : has_experts<Epi>::value && nkt < 2 ? 0 : kt + 2 - nkt;
+    const uint8_t* gx1 = (in1 ? gx : gxn) + k1 * sx.kstep;
+    const uint8_t* gx2 = (in2 ? gx : gxn) + k2 * sx.kstep;
+    const uint8_t* gy2 = (in2 ? gy : gyn) + k2 * sy.kstep;
+    auto store = [&](auto HX, auto HY, auto FROM) __attribute__((always_inline)) {
+      if constexpr (stores) {
+        if (have_prev) store_block(HX, HY, pp0, pq0, FROM);
       }
-      S ^= 1;
-#pragma unroll
-      for (int s = 0; s < NAX; ++s) ax[s] ^= 0x10000u;
-#pragma unroll
-      for (int s = 0; s < NAX1; ++s) ax1[s] ^= 0x10000u;
-#pragma unroll
-      for (int s = 0; s < NAY; ++s) ay[s] ^= 0x10000u;
     };
+    // kPipe: the block whose operand was requested before AFTER vector memory instructions; then next() asks for the next one's
+    auto store_pipe = [&](auto HX, auto HY, auto AFTER, auto next) __attribute__((always_inline)) {
+      if constexpr (stores && kPipe) {
+        if (have_prev) {
+          wait_pre(AFTER);
+          store_block(HX, HY, pp0, pq0, H0{});
+          next();
+        }
+      }
+    };
+    auto store_plain = [&](auto HX, auto HY) __attribute__((always_inline)) {
+      if constexpr (!kPipe) store(HX, HY, H0{});
+    };
+    auto request_first = [&]() __attribute__((always_inline)) {
+      if constexpr (kPipe && !first) {
+        if (!in1) request_pre(H0{}, H0{}, p0, q0, H0{});
+      }
+    };
+    auto nothing = []() {};
+    typedef std::integral_constant<int, 2> N2;
+    if constexpr (!NARROW) {
+      // c0 (the Y fragments of half 0 were requested in the previous k-tile's c7)
+      readA(H0{});
+      store_pipe(H0{}, H0{}, N2{}, [&]() { request_pre(H0{}, H1{}, pp0, pq0, H0{}); });
+      dma(S ^ 1, 0, 1, gx1);
+      store_plain(H0{}, H0{});
+      TFB_SBAR();
+      // c1
+      waitB(fb0);
+      waitA();
+      mma(FIRST, H0{}, H0{}, fb0);
+      TFB_SBAR();
+      // c2
+      readB(H1{}, fb1);
+      store_pipe(H0{}, H1{}, N2{}, [&]() { request_pre(H1{}, H0{}, pp0, pq0, H0{}); });
+      dma(S, 0, 0, gx2);
+      store_plain(H0{}, H1{});
+      TFB_SBAR();
+      // c3
+      waitB(fb1);
+      mma(FIRST, H0{}, H1{}, fb1);
+      TFB_SBAR();
+      // c4
+      readA(H1{});
+      store_pipe(H1{}, H0{}, N2{}, [&]() { request_pre(H1{}, H1{}, pp0, pq0, H0{}); });
+      dma(S, 1, 0, gy2);
+      store_plain(H1{}, H0{});
+      TFB_SBAR();
+      // c5
+      waitA();
+      mma(FIRST, H1{}, H0{}, fb0);
+      // Completion is reported in issue order, stores included. Everything up to the quarter requested in c0 has to be
+      // there one cluster before the other group's matching wait: all but the two quarters requested since (4
+      // instructions), and in a first iteration with stores all but those and the 12 stores (c0's four were issued
+      // behind its loads); kPipe: c2's and c4's stores and four requests each, in front of their loads. After the barrier that ends c6 both
+      // groups have waited, so the next k-tile is complete.
+      if (stores && have_prev) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPipe ? 20 : 16) : "memory");
+      else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      TFB_SBAR();
+      // c6
+      store_pipe(H1{}, H1{}, N2{}, nothing);
+      request_first();
+      dma(S, 1, 1, gy2);
+      store_plain(H1{}, H1{});
+      TFB_SBAR();
+      // c7: the next k-tile's first Y fragments are requested under this cluster's MFMAs (fb0 was last read in c5)
+      readB(H0{}, fb0, 0x10000u);
+      mma(FIRST, H1{}, H1{}, fb1);
+      TFB_SBAR();
+    } else {
+      // X half 1 is one MFMA tile a wavefront: three MFMA clusters of 8 instead of four. Quarters 0 are requested two k-tiles
+      // ahead, quarters 1 one ahead. A cluster's reads are waited for in front of its barrier (the requests behind them take longer),
+      // so a quarter is requested again only when a barrier has passed since either group had the old one in registers.
+      const uint8_t* gy1 = (in1 ? gy : gyn) + k1 * sy.kstep;
+      // c0 (Y half 0: see c5)
+      readA(H0{});
+      store_pipe(H0{}, H0{}, std::integral_constant<int, 4>{}, [&]() { request_pre(H0{}, H1{}, pp0, pq0, H0{}); });
+      dma(S ^ 1, 1, 1, gy1);
+      dma(S ^ 1, 0, 1, gx1);
+      store_plain(H0{}, H0{});
+      waitB(fb0);
+      waitA();
+      TFB_SBAR();
+      // c1
+      mma(FIRST, H0{}, H0{}, fb0);
+      TFB_SBAR();
+      // c2
+      readB(H1{}, fb1);
+      store_pipe(H0{}, H1{}, std::integral_constant<int, 2 + NX1>{}, [&]() {
+        request_pre(H1{}, H0{}, pp0, pq0, H0{});
+        request_pre(H1{}, H1{}, pp0, pq0, N2{});
+      });
+      store_plain(H0{}, H1{});
+      waitB(fb1);
+      TFB_SBAR();
+      // c3
+      mma(FIRST, H0{}, H1{}, fb1);
+      // The next k-tile's quarters 0 (requested in the previous iteration's c4) have to be there: all but what was requested
+      // since, c0's loads and in a first iteration with stores the 8 stores of c0 and c2, kPipe: and their eight requests. c5 reads them
+      // behind two more barriers.
+      if (stores && have_prev) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + NX1 + (kPipe ? 16 : 8)) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + NX1) : "memory");
+      TFB_SBAR();
+      // c4
+      readA(H1{});
+      store_pipe(H1{}, H0{}, H0{}, [&]() { store_block(H1{}, H1{}, pp0, pq0, N2{}); });
+      request_first();
+      dma(S, 0, 0, gx2);
+      dma(S, 1, 0, gy2);
+      store_plain(H1{}, H0{});
+      store_plain(H1{}, H1{});
+      waitA1();
+      TFB_SBAR();
+      // c5
+      mma(FIRST, H1{}, H0{}, fb0);
+      readB(H0{}, fb0, 0x10000u);
+      mma(FIRST, H1{}, H1{}, fb1);
+      // The next k-tile's quarters 1 (c0) likewise: all but c4's four loads, and with stores the 8 of c0 and c2 and c4's 4. (kPipe: c4 has
+      // waited for them.)
+      if (stores && have_prev) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      TFB_SBAR();
+    }
+    S ^= 1;
+#pragma unroll
+    for (int s = 0; s < NAX; ++s) ax[s] ^= 0x10000u;
+#pragma unroll
+    for (int s = 0; s < NAX1; ++s) ax1[s] ^= 0x10000u;
+#pragma unroll
+    for (int s = 0; s < NAY; ++s) ay[s] ^= 0x10000u;
+  };
+  for (;;) {
+    look_ahead();
     iter(std::true_type{}, 0);
     if constexpr (has_experts<Epi>::value) {
       for (int kt = 1; kt < nkt; ++kt) iter(std::false_type{}, kt);
@@ -685,23 +777,24 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     }
     w = wn;
     if (w >= w_end) break;
-    p0 = pn;
-    q0 = qn;
-    split = splitn;
-    k0 = k0n;
-    nkt = nktn;
-    gx = gxn;
-    gy = gyn;
+    go_on();
     if constexpr (kF32) {
       if (wr == 1) TFB_SBAR();  // group 1 falls one cluster behind again
     }
   }
   if constexpr (!kF32) {
     // the last tile's accumulators
-    store_block(H0{}, H0{}, pp0, pq0);
-    store_block(H0{}, H1{}, pp0, pq0);
-    store_block(H1{}, H0{}, pp0, pq0);
-    store_block(H1{}, H1{}, pp0, pq0);
+    auto flush = [&](auto HX, auto HY, auto request_it) __attribute__((always_inline)) {
+      if constexpr (kPipe) {
+        if constexpr (decltype(request_it)::value) request_pre(HX, HY, pp0, pq0, H0{});
+        wait_pre(H0{});
+      }
+      store_block(HX, HY, pp0, pq0, H0{});
+    };
+    flush(H0{}, H0{}, std::false_type{});
+    flush(H0{}, H1{}, std::true_type{});
+    flush(H1{}, H0{}, std::true_type{});
+    flush(H1{}, H1{}, std::true_type{});
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stream's last (unused) loads must have landed before LDS is released
 }
@@ -712,9 +805,12 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
 // contraction length (standalone, us, that kernel -> this one): bf16 2048 x 32768 x 768 (4.0 rounds) 140 -> 105, 8192 x 4096 x 768
 // (2.0) 69 -> 51, 10240 x 1024 x 768 (0.62) 27.8 -> 23.8, 16384 x 768 x 2304 (0.75) 78 -> 58; fp8 16384 x 3072 x 1024 (3.0) 69 -> 50;
 // at the line 8192 x 3072 x 768 (1.5) 46.4 -> 47.2, and below it 8192 x 2304 x 768 (1.12) 37.6 -> 41.8, 8192 x 1024 x 768 (0.5)
-// 18.5 -> 23.7. A heavy epilogue per tile (rotary embedding, residual add, the MLP's activation) is serial with the k-loop here and runs
+// 18.5 -> 23.7. A heavy epilogue per tile (residual add, the MLP's activation) is serial with the k-loop here and runs
 // under another workgroup's MFMAs there: those need 16 k-tiles or 4096 tiles as well (in the training step, 6 to 12 k-tiles:
-// 141 -> 148, 55 -> 60, 112 -> 111 us); 24 on a narrow tile (bf16 9600 x 1024 x 1024 with a residual 32.8 -> 34.2).
+// 55 -> 60, 112 -> 111 us); 24 on a narrow tile (bf16 32768 x 768 x 768 with a residual 49.9 -> 51.4, 16384 rows 27.2 -> 28.3).
+// The rotary embedding's tables are the same few for all heads, asked for ahead and out of the L2: it goes by the plain rule with lines 1.04 as
+// high (K 768, N 2304: 6144 rows 31.7 -> 28.3, 12288 56.1 -> 49.7, 16384 70.4 -> 68.2, 20480 90 -> 76, 32768 149 -> 120; N 1536, K 512: 10240
+// 24.6 -> 22.6, 32768 70.8 -> 58.7; N 768, K 256: 16384 17.6 -> 16.7, 65536 51.7 -> 38.3; at the plain lines 10240 x 2304 46.1 -> 47.5).
 // A narrow tile takes 0.75 / 0.92 (192 x 256) or 0.75 / 0.84 (256 x 192) of a 256 x 256 tile's time, so it is taken where its rounds save
 // that much (us, the kernel of before -> this one): fp8 16384 x 768 x 3072 40.9 -> 36.8, 32768 rows 73.0 -> 65.5, 9600 x 1024 x 4096 51.7 ->
 // 40.3, 11904 x 768 x 3072 50.6 -> 30.3; bf16 32768 x 768 x 2304 118 -> 104, 30336 x 768 x 768 55 -> 43, 12672 x 768 x 3072 95 -> 62; not in
@@ -729,7 +825,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
 #endif
 // The tile for an output of np x nq, or -1: the one that keeps the CUs busiest (256 x 256 also for all but the last 128 rows of q, where
 // it has a full round without them: a launch of the ring more, 0.15 of a round).
-static inline int gemm_pp_shape(long np, long nq, long kbytes, bool heavy_epilogue, bool narrow_ok) {
+// line: of the shares of their rounds that the tiles have to fill, for an epilogue between a plain and a heavy one.
+static inline int gemm_pp_shape(long np, long nq, long kbytes, bool heavy_epilogue, bool narrow_ok, double line = 1.0) {
   if (!TFB_PP || np <= 0 || nq <= 0 || kbytes < 256 || kbytes % 128) return -1;
   const long cus = tfb_resident_slots(1);
   const double core_rounds = (double)((np + 127) / 128) * (double)((nq + 127) / 128) / (double)(2 * cus), whole = (double)(long)core_rounds;
@@ -743,7 +840,7 @@ static inline int gemm_pp_shape(long np, long nq, long kbytes, bool heavy_epilog
     if (np % tp || tiles < 8 || (rest && (shape || rest != 128 || tiles < cus))) continue;
     const double cost = (double)rounds * (shape == 0 ? 1.0 : shape == TFB_PP_192x256 ? 0.75 / 0.92 : 0.75 / 0.84) + (rest ? 0.15 : 0.0);
     if (TFB_PP != 2 && TFB_PP_SHAPE < 0) {
-      if ((double)tiles < (rounds == 1 ? 0.6 : 0.7) * (double)(rounds * cus)) continue;
+      if ((double)tiles < (rounds == 1 ? 0.6 : 0.7) * line * (double)(rounds * cus)) continue;
       if (heavy_epilogue && kbytes / 128 < (shape ? 24 : 16) && tiles < 4096) continue;
       if (shape && (cost > (heavy_epilogue ? 0.9 : 0.95) * core || cost > 0.88 * whole_tiles)) continue;
     }

@@ -576,8 +576,8 @@ static bool gemm_ring_try(GemmOperand P, GemmOperand Q, int np, int nq, long kby
 // through the ring: 9600 x 3072 x 1024 in bf16 79 -> 62 us): true, with its status in st. heavy: the epilogue is heavy there.
 template <int ES, int LAYP, int LAYQ, int FMTP, int FMTQ, class Epi>
 static bool gemm_pp_try(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, bool heavy, Epi e, hipStream_t s, int& st) {
-  constexpr bool narrow_ok = LAYQ == TFB_K_CONTIG && !has_partner32<Epi>::value;
-  const int shape = gemm_pp_shape(np, nq, kbytes, heavy, narrow_ok);
+  constexpr bool rotation = partner_of<Epi>::value != 0, narrow_ok = LAYQ == TFB_K_CONTIG && !rotation;
+  const int shape = gemm_pp_shape(np, nq, kbytes, heavy && !rotation, narrow_ok, rotation ? 1.04 : 1.0);
   if (shape < 0) return false;
   if constexpr (narrow_ok) {
     if (shape == TFB_PP_192x256) st = gemm_pp_launch_lay<ES, FMTP, FMTQ, LAYP, LAYQ, TFB_PP_192x256>(P, Q, np, nq, kbytes, 1, e, s);

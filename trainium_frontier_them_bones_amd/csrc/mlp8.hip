@@ -551,6 +551,7 @@ struct EpiDescaleRes {
     *(u32x4*)(out + (long)q * ld + p) = pack8bf(a);
   }
   __device__ __forceinline__ float pre(float x) const { return x * dq; }
+  __device__ __forceinline__ const void* at(int p, int q) const { return res + (long)min(q, last) * ld + p; }
   __device__ __forceinline__ void chunk(int p, int q, const u32x4& v, const pre_t& rv) const {
     float a[8], b[8];
     unpack8bf(v, a);
