@@ -278,6 +278,8 @@ int tfb_mlp_dw_proj(const void* dy, const void* r, void* dw, long M, int d, int 
  * heads of 64) of its first rot_cols columns applied in the GEMM epilogue; row m is token m % T; cos_t, sin_t bf16
  * [T][32]. Equals tfb_gemm_bf16 followed by tfb_rope bit for bit. Replaces the c_attn projection + the rotation inside
  * nki_rope_attention (round1/source/train.py:8197, 4188-4193) as one launch. */
+int tfb_qkv_rope_heads_fwd(const void* x, const void* w, const void* cos_t, const void* sin_t, void* out, int M, int N, int K, int T,
+                           int rot_cols, int D, void* stream);   /* heads of D = 64 or 128, tables [T][D / 2] */
 int tfb_qkv_rope_fwd(const void* x, const void* w, const void* cos_t, const void* sin_t, void* out, int M, int N, int K, int T,
                      int rot_cols, void* stream);
 

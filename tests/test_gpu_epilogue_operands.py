@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from trainium_frontier_them_bones_amd import ops
+from trainium_frontier_them_bones_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -12,13 +12,20 @@ def _normal(g, *shape):
 
 
 # rows, tokens of a sequence, width of the rotated and of all columns, contraction: two, three and many k-tiles; part of a round, two rounds of
-# which the last is ragged, the last 128 rows by themselves; nothing rotated, all of it; sequences that end inside a tile
-@pytest.mark.parametrize("M,T,rot,N,K", [(16384, 2048, 512, 768, 128), (16384, 512, 768, 768, 192), (20480, 640, 1536, 2304, 128), (28672, 7168, 1024, 1536, 512),
+# which the last is ragged, the last 128 rows by themselves; nothing rotated, all of it; sequences that end inside a tile; and launches of the
+# kernels for fewer tiles
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("M,T,rot,N,K", [(128, 128, 256, 384, 64), (1152, 384, 1024, 1536, 512), (6144, 96, 2048, 3072, 128), (16384, 2048, 512, 768, 128), (16384, 512, 768, 768, 192), (20480, 640, 1536, 2304, 128), (28672, 7168, 1024, 1536, 512),
                                          (30336, 1264, 1024, 1536, 128), (12288, 384, 0, 2304, 768), (32768, 2048, 1536, 2304, 768)])
-def test_rotated_projection(M, T, rot, N, K):
-    D, g = 64, torch.Generator(device="cuda:0").manual_seed(M + N + K)
+def test_rotated_projection(M, T, rot, N, K, D):
+    g = torch.Generator(device="cuda:0").manual_seed(M + N + K)
     x, w, cos, sin = _normal(g, M, K), _normal(g, N, K), _normal(g, T, D // 2), _normal(g, T, D // 2)
-    got = ops.qkv_rope(x, w, cos, sin, T, rot)
+    if D == 64:
+        got = ops.qkv_rope(x, w, cos, sin, T, rot)
+    else:
+        got = torch.full((M, N), float("nan"), device=x.device, dtype=torch.bfloat16)
+        args = [t.data_ptr() for t in (x, w, cos, sin, got)] + [M, N, K, T, rot, D, torch.cuda.current_stream().cuda_stream]
+        assert _lib.lib().tfb_qkv_rope_heads_fwd(*args) == 0
     want = ops.matmul(x, w, trans_b=True)
     if rot:
         ops.rope_(want, cos, sin, T, rot // D, D)

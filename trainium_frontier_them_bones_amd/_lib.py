@@ -64,6 +64,7 @@ SIGNATURES = {
     "tfb_attn_bwd_rope": [_vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _vp, _vp, _vp,
                           _i, _i, _i, _i, _f, _vp],
     "tfb_qkv_rope_fwd": [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp],
+    "tfb_qkv_rope_heads_fwd": [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp],
     "tfb_precast8": [_vp, _vp, _vp, _vp, _i, _i, _vp],
     "tfb_gemm_fp8": [_vp, _i, _vp, _vp, _vp, _f, _vp, _l, _i, _i, _vp],
     "tfb_gemm_fp8_res": [_vp, _vp, _vp, _vp, _f, _vp, _vp, _l, _i, _i, _vp],

@@ -89,25 +89,28 @@ inline int ring_ranges(int N, int M, int K, bool strided, long ws_bytes) {
   return splits == 1 || 4 * (long)(N / 64) * (M / 64) > tfb_resident_slots(1) ? splits : 0;
 }
 
-// out [q][ld] = bf16(D) with the rotary embedding applied to the first rot_cols columns (heads of 64: y1 = x1 c + x2 s,
+// out [q][ld] = bf16(D) with the rotary embedding applied to the first rot_cols columns (heads of 2 HALF: y1 = x1 c + x2 s,
 // y2 = x2 c - x1 s on the bf16-rounded products, rounded again - what tfb_rope computes from the stored projection).
+template <int HALF>
 struct EpiStoreRope {
-  static constexpr bool kPartner32 = true;
+  static constexpr int kPartner = HALF;
   bf16_t* out;
   long ld;
-  const bf16_t* cs;  // [T][32]
+  const bf16_t* cs;  // [T][HALF]
   const bf16_t* sn;
   int T, rot_cols;
   FastDiv d_T;
   struct pre_t {  // the chunk's cos / sin values, requested before the k-loop
     u32x4 c, s;
   };
+  __device__ __forceinline__ long table(int p, int q) const { return (long)(q - fastdiv(q, d_T) * T) * HALF + (p & (HALF - 1)); }
+  __device__ __forceinline__ const void* at(int p, int q) const { return cs + table(p, q); }
+  __device__ __forceinline__ const void* at2(int p, int q) const { return sn + table(p, q); }
   __device__ __forceinline__ pre_t prefetch(int p, int q) const {
     pre_t r = {};
     if (p < rot_cols) {
-      const int t = q % T, idx = p & 31;
-      r.c = *(const u32x4*)(cs + (long)t * 32 + idx);
-      r.s = *(const u32x4*)(sn + (long)t * 32 + idx);
+      r.c = *(const u32x4*)at(p, q);
+      r.s = *(const u32x4*)at2(p, q);
     }
     return r;
   }
@@ -116,7 +119,7 @@ struct EpiStoreRope {
     u32x4 x = pack8bf(v);
     if (p < rot_cols) {
       const u32x4 y = pack8bf(vp);
-      const bool low = (p & 32) == 0;
+      const bool low = (p & HALF) == 0;
       const u32x4 c = tab.c, s = tab.s;
       u32x4 o;
 #pragma unroll
@@ -130,11 +133,7 @@ struct EpiStoreRope {
     *(u32x4*)(out + (long)q * ld + p) = x;
   }
   // the 256 x 256 kernel's protocol: the same from the rounded products, a chunk of a head's first half with its partner
-  static constexpr int kPartner = 32;
   __device__ __forceinline__ float pre(float x) const { return x; }
-  __device__ __forceinline__ long table(int p, int q) const { return (long)(q - fastdiv(q, d_T) * T) * 32 + (p & 31); }
-  __device__ __forceinline__ const void* at(int p, int q) const { return cs + table(p, q); }
-  __device__ __forceinline__ const void* at2(int p, int q) const { return sn + table(p, q); }
   __device__ __forceinline__ void chunk2(int p, int q, u32x4 x, u32x4 y, const u32x4& c, const u32x4& s) const {
     if (p < rot_cols) {
 #pragma unroll
@@ -147,9 +146,20 @@ struct EpiStoreRope {
     }
     bf16_t* o = out + (long)q * ld + p;
     *(u32x4*)o = x;
-    *(u32x4*)(o + 32) = y;
+    *(u32x4*)(o + HALF) = y;
   }
 };
+
+template <int HALF>
+int qkv_rope(const void* x, const void* w, const void* cos_t, const void* sin_t, void* out, int M, int N, int K, int T, int rot_cols, hipStream_t s) {
+  using Cfg = GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>;
+  GemmOperand P{(const uint8_t*)w, (long)K * 2}, Q{(const uint8_t*)x, (long)K * 2};
+  EpiStoreRope<HALF> e{(bf16_t*)out, (long)N, (const bf16_t*)cos_t, (const bf16_t*)sin_t, T, rot_cols, fastdiv_make(T)};
+  int st;
+  if (gemm_ring_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, e, s, st)) return st;
+  if (gemm_pp_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, true, e, s, st)) return st;
+  return gemm_launch<Cfg>(P, Q, N, M, (long)K * 2, 1, LoadIdentity{}, LoadIdentity{}, e, s);
+}
 
 }  // namespace
 
@@ -224,18 +234,20 @@ extern "C" int tfb_gemm_bf16_res(const void* A, const void* B, const void* res, 
 }
 
 // qkv [M][N] = rope(x [M][K] @ w [N][K]^T): the fused attention projection with the rotary embedding of the q and k
-// thirds (the first rot_cols columns, heads of 64 elements) applied in the GEMM epilogue; row m is token m % T.
-// cos_t, sin_t: bf16 [T][32]. The output equals tfb_gemm_bf16 followed by tfb_rope bit for bit.
+// thirds (the first rot_cols columns, heads of D = 64 or 128 elements) applied in the GEMM epilogue; row m is token m % T.
+// cos_t, sin_t: bf16 [T][D / 2]. The output equals tfb_gemm_bf16 followed by tfb_rope bit for bit. us, two launches -> one, D = 128:
+// 512 -> 1536 columns: 1152 rows 9.4 -> 6.8, 4096 18.6 -> 13.8, 12288 36.8 -> 30.9; 1024 -> 3072: 256 8.8 -> 8.2, 1152 17.1 -> 13.5, 6144 55.4 -> 48.5,
+// 9600 76.9 -> 72.9, 16384 113 -> 100 (and 12288 89.4 -> 93.6: the projection alone takes 256 x 192 tiles there, which have no rotation).
+extern "C" int tfb_qkv_rope_heads_fwd(const void* x, const void* w, const void* cos_t, const void* sin_t, void* out, int M, int N,
+                                      int K, int T, int rot_cols, int D, void* stream) {
+  if (!x || !w || !cos_t || !sin_t || !out) return TFB_ERR_ARG;
+  if ((D != 64 && D != 128) || M <= 0 || N <= 0 || K <= 0 || M % 128 || N % 128 || K % 64 || T <= 0 || rot_cols < 0 || rot_cols > N ||
+      rot_cols % D)
+    return TFB_ERR_SHAPE;
+  return D == 64 ? qkv_rope<32>(x, w, cos_t, sin_t, out, M, N, K, T, rot_cols, (hipStream_t)stream)
+                 : qkv_rope<64>(x, w, cos_t, sin_t, out, M, N, K, T, rot_cols, (hipStream_t)stream);
+}
 extern "C" int tfb_qkv_rope_fwd(const void* x, const void* w, const void* cos_t, const void* sin_t, void* out, int M, int N,
                                 int K, int T, int rot_cols, void* stream) {
-  if (!x || !w || !cos_t || !sin_t || !out) return TFB_ERR_ARG;
-  if (M <= 0 || N <= 0 || K <= 0 || M % 128 || N % 128 || K % 64 || T <= 0 || rot_cols < 0 || rot_cols > N || rot_cols % 64)
-    return TFB_ERR_SHAPE;
-  using Cfg = GemmCfg<128, 128, 2, 2, 2, TFB_K_CONTIG, TFB_K_CONTIG>;
-  GemmOperand P{(const uint8_t*)w, (long)K * 2}, Q{(const uint8_t*)x, (long)K * 2};
-  EpiStoreRope e{(bf16_t*)out, (long)N, (const bf16_t*)cos_t, (const bf16_t*)sin_t, T, rot_cols, fastdiv_make(T)};
-  int st;
-  if (gemm_ring_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, e, (hipStream_t)stream, st)) return st;
-  if (gemm_pp_try<2, TFB_K_CONTIG, TFB_K_CONTIG, 0, 0>(P, Q, N, M, (long)K * 2, true, e, (hipStream_t)stream, st)) return st;
-  return gemm_launch<Cfg>(P, Q, N, M, (long)K * 2, 1, LoadIdentity{}, LoadIdentity{}, e, (hipStream_t)stream);
+  return tfb_qkv_rope_heads_fwd(x, w, cos_t, sin_t, out, M, N, K, T, rot_cols, 64, stream);
 }

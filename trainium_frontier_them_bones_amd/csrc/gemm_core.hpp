@@ -197,22 +197,23 @@ struct TileDma<ROWS, NW, TFB_K_STRIDED, ES> {
 
 // ---- LDS -> MFMA fragments ---------------------------------------------------------------------------------------
 // Per-lane addressing of one operand: off(i, s) = byte offset of the lane's fragment of MFMA tile i, k-step s.
-template <int ROWS, int ES, int LAY>
+// TILE: rows from one MFMA tile of the wavefront to the next (k-contiguous operands; 32 otherwise).
+template <int ROWS, int ES, int LAY, int TILE = 32>
 struct FragReader;
 
-template <int ROWS>
-struct FragReader<ROWS, 2, TFB_K_CONTIG> {
+template <int ROWS, int TILE>
+struct FragReader<ROWS, 2, TFB_K_CONTIG, TILE> {
   static constexpr int KSTEPS = 4;
   typedef bf16x8 frag_t;
   int row, lh;
   __device__ __forceinline__ void init(int wave_row0, int lane) { row = wave_row0 + (lane & 31); lh = lane >> 5; }
   __device__ __forceinline__ frag_t read(const uint8_t* lds, int i, int s) const {
-    const int r = row + 32 * i;
+    const int r = row + TILE * i;
     return *(const bf16x8*)(lds + r * 128 + ((((2 * s + lh) ^ tfb_kc_swz(r)) & 7) << 4));
   }
 };
 template <int ROWS>
-struct FragReader<ROWS, 1, TFB_K_CONTIG> {
+struct FragReader<ROWS, 1, TFB_K_CONTIG, 32> {
   static constexpr int KSTEPS = 2;
   typedef i32x8 frag_t;
   int row, lh;
@@ -225,7 +226,7 @@ struct FragReader<ROWS, 1, TFB_K_CONTIG> {
   }
 };
 template <int ROWS>
-struct FragReader<ROWS, 2, TFB_K_STRIDED> {
+struct FragReader<ROWS, 2, TFB_K_STRIDED, 32> {
   static constexpr int KSTEPS = 4;
   typedef bf16x8 frag_t;
   static constexpr int PITCH = ROWS * 2;
@@ -252,7 +253,7 @@ struct FragReader<ROWS, 2, TFB_K_STRIDED> {
 // (k0 + j / 2, row0 + 8 (j % 2)) lane i receives 8 consecutive k of row row0 + i. 16-byte chunk c of k-row k sits at
 // slot c ^ (2 ((k >> 1) & 3)): the 8 k-rows x 2 chunks that 32 lanes read together then cover all 64 banks once.
 template <int ROWS>
-struct FragReader<ROWS, 1, TFB_K_STRIDED> {
+struct FragReader<ROWS, 1, TFB_K_STRIDED, 32> {
   static constexpr int KSTEPS = 2;
   typedef i32x8 frag_t;
   static constexpr int PITCH = ROWS;
@@ -312,13 +313,17 @@ __device__ __forceinline__ Epi epi_prepare(const Epi& e) {
   else return e;
 }
 
-// A staged epilogue with the static member kPartner32 also receives the 8 values 32 output columns away (p ^ 32: the
-// other half of a 64-wide head, for rotary embeddings): operator()(p, q, v, v_partner, split). Needs a wavefront slice
-// of exactly 64 staged columns.
+// A staged epilogue with the static member kPartner (32 or 64) also receives the 8 values that many output columns away (p ^ kPartner:
+// the other half of a head, for rotary embeddings): operator()(p, q, v, v_partner, split). Needs a wavefront slice of exactly 64
+// staged columns; with 64 that is columns 32 wp .. and 64 + 32 wp .. of a 128-column tile (tfb_slice_col).
 template <class T, class = void>
-struct has_partner32 : std::false_type {};
+struct partner_of : std::integral_constant<int, 0> {};
 template <class T>
-struct has_partner32<T, std::void_t<decltype(T::kPartner32)>> : std::true_type {};
+struct partner_of<T, std::void_t<decltype(T::kPartner)>> : std::integral_constant<int, T::kPartner> {};
+template <class Epi>
+__device__ __forceinline__ int tfb_slice_col(int wp, int cols, int c) {  // the tile's column of a wavefront's staged column c, of `cols`
+  return partner_of<Epi>::value == 64 ? 32 * wp + (c & 31) + 2 * (c & 32) : cols * wp + c;
+}
 
 template <class T, class = void>
 struct has_tile_epilogue : std::false_type {};
@@ -461,11 +466,13 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::OCC) void gemm_kernel(GemmArgs a, Pre
   if (nkt > 0) issue(buf0, 0);
 
   const Epi epi = epi_prepare(epi_for_group(epi_in, group));
-  typedef FragReader<BP, ES, Cfg::LAYP> RP;
+  constexpr bool kFar = partner_of<Epi>::value == 64;
+  static_assert(!kFar || (BP == 128 && Cfg::WP == 2 && TP == 2 && ES == 2 && Cfg::LAYP == TFB_K_CONTIG), "whole heads of 128");
+  typedef FragReader<BP, ES, Cfg::LAYP, kFar ? 64 : 32> RP;
   typedef FragReader<BQ, ES, Cfg::LAYQ> RQ;
   RP rp;
   RQ rq;
-  rp.init(wp * (TP * 32), lane);
+  rp.init(wp * (kFar ? 32 : TP * 32), lane);
   rq.init(wq * (TQ * 32), lane);
 
   f32x16 acc[TP][TQ];
@@ -488,7 +495,7 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::OCC) void gemm_kernel(GemmArgs a, Pre
       for (int j = 0; j < TQ; ++j)
 #pragma unroll
         for (int k = 0; k < EPI_NK; ++k)
-          pre[j][k] = epi.prefetch((int)p0 + wp * (TP * 32) + chunk_col(k), (int)q0 + wq * (TQ * 32) + j * 32 + chunk_row(k));
+          pre[j][k] = epi.prefetch((int)p0 + tfb_slice_col<Epi>(wp, TP * 32, chunk_col(k)), (int)q0 + wq * (TQ * 32) + j * 32 + chunk_row(k));
     }
   };
 #ifndef TFB_PREFETCH_AFTER_FIRST
@@ -580,13 +587,14 @@ __global__ __launch_bounds__(Cfg::NT, Cfg::OCC) void gemm_kernel(GemmArgs a, Pre
           f32x4 lo = *(const f32x4*)(stage + row * SLD + pc);
           f32x4 hi = *(const f32x4*)(stage + row * SLD + pc + 4);
           const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-          if constexpr (has_partner32<Epi>::value) {
+          if constexpr (partner_of<Epi>::value != 0) {
             static_assert(ETP == 2 && TP == 2, "partner epilogue: 64 staged columns per wavefront");
             f32x4 plo = *(const f32x4*)(stage + row * SLD + (pc ^ 32));
             f32x4 phi = *(const f32x4*)(stage + row * SLD + (pc ^ 32) + 4);
             const float vp[8] = {plo[0], plo[1], plo[2], plo[3], phi[0], phi[1], phi[2], phi[3]};
-            if constexpr (kPrefetch) epi((int)p0 + pw + pc, (int)q0 + qw + j * 32 + row, v, vp, pre[j][k], split);
-            else epi((int)p0 + pw + pc, (int)q0 + qw + j * 32 + row, v, vp, split);
+            const int p = (int)p0 + tfb_slice_col<Epi>(wp, TP * 32, pc);
+            if constexpr (kPrefetch) epi(p, (int)q0 + qw + j * 32 + row, v, vp, pre[j][k], split);
+            else epi(p, (int)q0 + qw + j * 32 + row, v, vp, split);
           } else if constexpr (kPrefetch) {
             epi((int)p0 + pw + pc, (int)q0 + qw + j * 32 + row, v, pre[j][k], split);
           } else {

@@ -80,11 +80,6 @@ struct PpArgs {
   int ngroups;
   FastDiv d_ipx;
 };
-// The distance of the outputs that an epilogue takes together (0: none)
-template <class T, class = void>
-struct partner_of : std::integral_constant<int, 0> {};
-template <class T>
-struct partner_of<T, std::void_t<decltype(T::kPartner)>> : std::integral_constant<int, T::kPartner> {};
 template <class T, class = void>
 struct has_experts : std::false_type {};
 template <class T>

@@ -91,7 +91,7 @@ __device__ __forceinline__ u32x2 ring_read_tr64(uint32_t addr) {
 
 // One operand's fragments of a k-tile: request() reads all of them into this object's registers, landed() ties those registers
 // to the wait that precedes it, get<i, s>() is the fragment of MFMA tile i, k-step s. The layouts are FragReader's.
-template <int ROWS, int NTILE, int ES, int LAY>
+template <int ROWS, int NTILE, int ES, int LAY, int TILE = 32>   // TILE: as FragReader's
 struct RingFrags;
 
 template <int ROWS, int NTILE>
@@ -99,8 +99,8 @@ struct RingAddr {   // per-lane byte offsets inside a stage's operand tile
   uint32_t off[4];
 };
 
-template <int ROWS, int NTILE, int ES>
-struct RingFrags<ROWS, NTILE, ES, TFB_K_CONTIG> {
+template <int ROWS, int NTILE, int ES, int TILE>
+struct RingFrags<ROWS, NTILE, ES, TFB_K_CONTIG, TILE> {
   static constexpr int KS = ES == 2 ? 4 : 2, PER = ES == 2 ? 1 : 2;   // 128-bit reads per fragment
   i32x4 v[NTILE][KS][PER];
   static __device__ __forceinline__ RingAddr<ROWS, NTILE> addr(int wave_row0, int lane) {
@@ -117,7 +117,7 @@ struct RingFrags<ROWS, NTILE, ES, TFB_K_CONTIG> {
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
       v[0][n / PER][n % PER] = ring_read128<0>(base + a.off[n]);
-      if constexpr (NTILE == 2) v[1][n / PER][n % PER] = ring_read128<4096>(base + a.off[n]);
+      if constexpr (NTILE == 2) v[1][n / PER][n % PER] = ring_read128<TILE * 128>(base + a.off[n]);
     }
   }
   __device__ __forceinline__ void landed() {
@@ -138,7 +138,7 @@ struct RingFrags<ROWS, NTILE, ES, TFB_K_CONTIG> {
 };
 
 template <int ROWS, int NTILE, int ES>
-struct RingFrags<ROWS, NTILE, ES, TFB_K_STRIDED> {
+struct RingFrags<ROWS, NTILE, ES, TFB_K_STRIDED, 32> {
   static constexpr int KS = ES == 2 ? 4 : 2, PER = ES == 2 ? 2 : 4;   // 64-bit transposing reads per fragment
   static constexpr int PITCH = ROWS * ES, KSTEP = (ES == 2 ? 16 : 64) * PITCH, KQ = (ES == 2 ? 4 : 8) * PITCH;
   u32x2 v[NTILE][KS][PER];
@@ -269,9 +269,11 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
     if (t < nkt) issue(t, t);
 
   const Epi epi = epi_prepare(epi_for_group(epi_in, group));
-  typedef RingFrags<BP, TP, ES, Cfg::LAYP> FP;
+  constexpr bool kFar = partner_of<Epi>::value == 64;
+  static_assert(!kFar || (BP == 128 && Cfg::WP == 2 && Cfg::LAYP == TFB_K_CONTIG), "whole heads of 128");
+  typedef RingFrags<BP, TP, ES, Cfg::LAYP, kFar ? 64 : 32> FP;
   typedef RingFrags<BQ, TQ, ES, Cfg::LAYQ> FQ;
-  const auto ap = FP::addr(wp * (TP * 32), lane);
+  const auto ap = FP::addr(wp * (kFar ? 32 : TP * 32), lane);
   const auto aq = FQ::addr(wq * (TQ * 32), lane);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(tfb_lds_void_t*)lds;
   FP fp[2];
@@ -390,7 +392,7 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
 #pragma unroll
     for (int j = 0; j < TQ; ++j)
 #pragma unroll
-      for (int k = 0; k < NK; ++k) pre[j][k] = epi.prefetch((int)p0 + pw + chunk_col(k), a.q_off + (int)q0 + qw + j * 32 + chunk_row(k));
+      for (int k = 0; k < NK; ++k) pre[j][k] = epi.prefetch((int)p0 + tfb_slice_col<Epi>(wp, TP * 32, chunk_col(k)), a.q_off + (int)q0 + qw + j * 32 + chunk_row(k));
   }
   int t = 0;
   for (; t + 1 + NS < nkt; t += 2) {
@@ -439,7 +441,7 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
 #pragma unroll
       for (int k = 0; k < NK; ++k) {
         const int row = chunk_row(k), pc = chunk_col(k);
-        const int p = (int)p0 + pw + pc, q = a.q_off + (int)q0 + qw + j * 32 + row;
+        const int p = (int)p0 + tfb_slice_col<Epi>(wp, TP * 32, pc), q = a.q_off + (int)q0 + qw + j * 32 + row;
         const f32x4 lo = *(const f32x4*)(stg + row * SLD + pc), hi = *(const f32x4*)(stg + row * SLD + pc + 4);
         const float v[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         if constexpr (is_symmetric<Epi>::value) {
@@ -448,7 +450,7 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
           else w = epi.value(v);
           *(u32x4*)(epi.out + (long)q * epi.ld + p) = w;
           if (tile_p != tile_q) Mirror::put(mirror, row, pc, w);
-        } else if constexpr (has_partner32<Epi>::value) {
+        } else if constexpr (partner_of<Epi>::value != 0) {
           static_assert(TP == 2, "partner epilogue: 64 staged columns per wavefront");
           const f32x4 plo = *(const f32x4*)(stg + row * SLD + (pc ^ 32)), phi = *(const f32x4*)(stg + row * SLD + (pc ^ 32) + 4);
           const float vp[8] = {plo[0], plo[1], plo[2], plo[3], phi[0], phi[1], phi[2], phi[3]};
@@ -547,7 +549,7 @@ static int gemm_ring_symmetric(GemmOperand X, long g_stride, int N, int nkt, int
 template <class Epi, int ES, int LAYP, int LAYQ, int FMTP, int FMTQ>
 static int gemm_ring_launch(int pick, GemmArgs a, int groups_y, int splits, Epi e, hipStream_t s, int ranges = 1, int q_off = 0) {
   a.q_off = q_off;
-  if constexpr (!has_partner32<Epi>::value && !has_tile_epilogue<Epi>::value) {   // (those take 64 columns of p per wavefront)
+  if constexpr (partner_of<Epi>::value == 0 && !has_tile_epilogue<Epi>::value) {   // (those take 64 columns of p per wavefront)
     if (pick == 1) {
       a.ntp = a.np / 64;
       return gemm_ring_launch_args<RingCfg<64, 64, 2, 2, ES, LAYP, LAYQ, FMTP, FMTQ, 4>>(a, groups_y, splits, ranges, e, s);

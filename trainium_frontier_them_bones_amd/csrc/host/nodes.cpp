@@ -557,7 +557,16 @@ struct QkvRopeAttention : Function<QkvRopeAttention> {
     chk(x), chk(w);
     TORCH_CHECK_VALUE(x.dim() == 3 && w.dim() == 2 && x.size(2) == w.size(1), "x is [B, T, in], w [3C, in]");
     const int64_t B = x.size(0), T = x.size(1), C = w.size(0) / 3;
-    const Tensor qkv = op::qkv_rope(x, w, cos, sin, T, 2 * C);
+    TORCH_CHECK_VALUE(n_head > 0 && w.size(0) % (3 * n_head) == 0, "qkv is [B, T, 3 heads D]");
+    const int64_t D = C / n_head;
+    Tensor qkv;
+    if (D == 64 || !any_replaced) {
+      qkv = D == 64 ? op::qkv_rope(x, w, cos, sin, T, 2 * C) : qkv_rope(x, w, cos, sin, T, 2 * C, D);
+    } else {   // (where an op of the package is replaced: of other heads, the ops one by one)
+      qkv = make({B, T, 3 * C}, BF16, x);
+      op::gemm(x, w, qkv, B * T, 3 * C, x.size(2), false, true, false);
+      op::rope(qkv, cos, sin, qkv, B * T, T, 2 * n_head, D, 3 * C, 3 * C, false);
+    }
     const QkvDims m = qkv_dims(qkv, n_head, scale);
     Tensor o = make({B, T, C}, BF16, x), lse = make({B, m.H, T}, F32, x);
     const int64_t R = 3 * C;
@@ -573,8 +582,10 @@ struct QkvRopeAttention : Function<QkvRopeAttention> {
     check_grad(go, s[3].numel());
     const int64_t R = 3 * m.C, K = w.size(1), M = m.B * m.T;
     const Tensor dqkv = make_like(qkv);
+    const bool fused = m.D == 64;   // the inverse rotation of dq, dk rides the backward kernels' stores
     op::attn_bwd(m.third(qkv, 0, R), m.third(qkv, 1, R), m.third(qkv, 2, R), s[3], go, m.third(dqkv, 0, R), m.third(dqkv, 1, R),
-             m.third(dqkv, 2, R), s[4], s[5], s[6], m.scale, 0);
+             m.third(dqkv, 2, R), s[4], fused ? s[5] : Tensor(), fused ? s[6] : Tensor(), m.scale, 0);
+    if (!fused) op::rope(dqkv, s[5], s[6], dqkv, M, m.T, 2 * m.H, m.D, R, R, true);
     auto [dx, dw] = linear_backward(dqkv, x, w, M, R, K);
     return {dx, dw, Tensor(), Tensor(), Tensor(), Tensor()};
   }

@@ -79,11 +79,11 @@ Tensor matmul_res(const Tensor& a, const Tensor& b, const Tensor& res, bool tb) 
   return out;
 }
 
-Tensor qkv_rope(const Tensor& x, const Tensor& w, const Tensor& cos, const Tensor& sin, int64_t T, int64_t rot_cols) {
+Tensor qkv_rope(const Tensor& x, const Tensor& w, const Tensor& cos, const Tensor& sin, int64_t T, int64_t rot_cols, int64_t D) {
   chk(x), chk(w), chk(cos), chk(sin);
   const int64_t K = last_dim(x), M = x.numel() / K, N = w.size(0);
   Tensor out = make(with_last(x, N), BF16, x);
-  TFB_CALL(tfb_qkv_rope_fwd, ptr(x), ptr(w), ptr(cos), ptr(sin), ptr(out), M, N, K, T, rot_cols, stream());
+  TFB_CALL(tfb_qkv_rope_heads_fwd, ptr(x), ptr(w), ptr(cos), ptr(sin), ptr(out), M, N, K, T, rot_cols, D, stream());
   return out;
 }
 

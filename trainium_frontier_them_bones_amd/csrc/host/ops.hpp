@@ -17,7 +17,7 @@ void linear_bwd(const Tensor& gy, const Tensor& x, const Tensor& w, const Tensor
 Tensor matmul(const Tensor& a, const Tensor& b, bool ta, bool tb, Tensor out, bool accumulate, at::ScalarType out_dtype,
               const Tensor& alpha);
 Tensor matmul_res(const Tensor& a, const Tensor& b, const Tensor& res, bool tb);
-Tensor qkv_rope(const Tensor& x2, const Tensor& w, const Tensor& cos, const Tensor& sin, int64_t T, int64_t rot_cols);
+Tensor qkv_rope(const Tensor& x2, const Tensor& w, const Tensor& cos, const Tensor& sin, int64_t T, int64_t rot_cols, int64_t D = 64);
 Tensor workspace(const Tensor& like);   // fp32 split-K scratch of the current stream
 
 // norms

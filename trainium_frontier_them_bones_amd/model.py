@@ -195,7 +195,7 @@ class GPT:
                 att = A.RopeAttentionFn.apply(qkv, self.cos[:T], self.sin[:T], cfg.n_head, scale)
                 att = A.Linear8Fn.apply(att, p["w_o.%d" % i], self.wo_state[i], None)
             else:
-                if cfg.head_dim == 64:   # rotation fused into the projection's epilogue and the backward kernels' stores
+                if cfg.head_dim in (64, 128):   # rotation fused into the projection's epilogue
                     att = A.QkvRopeAttentionFn.apply(h, p["w_qkv.%d" % i], self.cos[:T], self.sin[:T], cfg.n_head, scale)
                 else:
                     qkv = A.LinearFn.apply(h, p["w_qkv.%d" % i])
@@ -227,7 +227,7 @@ class GPT:
                 att = A.RopeAttentionFn.apply(qkv, self.cos[:T], self.sin[:T], cfg.n_head, scale)
                 x = A.Linear8Fn.apply(att, p["w_o.%d" % i], self.wo_state[i], None, None, x)
             else:
-                if cfg.head_dim == 64:
+                if cfg.head_dim in (64, 128):
                     att = A.QkvRopeAttentionFn.apply(h, p["w_qkv.%d" % i], self.cos[:T], self.sin[:T], cfg.n_head, scale)
                 else:
                     qkv = A.LinearFn.apply(h, p["w_qkv.%d" % i])
