@@ -414,59 +414,79 @@ __global__ __launch_bounds__(256) void emb_scatter_kernel(const IDX* __restrict_
   if (i < n) order[cursor[emb_bucket(idx[i], V)] + rank[i]] = (int)i;
 }
 
-// A workgroup sums EMB_SEG consecutive rows of the token-grouped order, thread t owning columns 8t .. 8t+7. A run of
+// A workgroup sums SEG consecutive rows of the token-grouped order, thread t owning columns 8t .. 8t+7. A run of
 // equal tokens that lies inside the segment has a single owner and is added with plain loads/stores; the first and the
 // last run may continue in the neighbouring segments and use atomics.
-#ifndef TFB_EMB_SEG
-#define TFB_EMB_SEG 32
-#endif
-constexpr int EMB_SEG = TFB_EMB_SEG;
-template <typename IDX>
+// What bounds it: with few rows latency, a trip to memory for every row and every sum it is added to (those of eight positions are asked for
+// together), so short segments; with many the atomics of the frequent tokens' runs on one row, one for each segment, so long ones. The whole call,
+// Zipf tokens, V 32768, C 768, us, segments of 8 / 16 / 32 / 64: 512 rows 22.5 / 25.3 / 32 / 44, 1152 26.3 / 25.7 / 32.3 / 44, 2048 30.0 / 27.1 / 32.4 / 44.5,
+// 4096 42 / 32.9 / 32.5 / 44, 16384 111 / 68 / 52 / 54, 32768 204 / 117 / 78.5 / 69 (C 512 at 32768: 181 / 103 / 67.5 / 58.5).
+constexpr int EMB_AHEAD = 8;
+template <typename IDX, int SEG>
 __global__ __launch_bounds__(128) void emb_reduce_kernel(const IDX* __restrict__ idx, const int* __restrict__ order,
                                                         const bf16_t* __restrict__ dy, float* __restrict__ dw, long n, int C,
                                                         int V) {
-  __shared__ int rows[EMB_SEG];
-  __shared__ int toks[EMB_SEG];
+  __shared__ int rows[SEG];
+  __shared__ int toks[SEG + 1];
   __shared__ int edge[2];  // the tokens of the rows just before and just after this segment (-1: none)
-  const long pos0 = (long)blockIdx.x * EMB_SEG;
-  const int cnt = (int)min((long)EMB_SEG, n - pos0);
+  const long pos0 = (long)blockIdx.x * SEG;
+  const int cnt = (int)min((long)SEG, n - pos0);
   if (threadIdx.x < cnt) {
     const int r = order[pos0 + threadIdx.x];
     rows[threadIdx.x] = r;
     toks[threadIdx.x] = emb_bucket(idx[r], V);
-  } else if (threadIdx.x == EMB_SEG) {
+  } else if (threadIdx.x == SEG) {
     edge[0] = pos0 > 0 ? emb_bucket(idx[order[pos0 - 1]], V) : -1;
-  } else if (threadIdx.x == EMB_SEG + 1) {
+  } else if (threadIdx.x == SEG + 1) {
     edge[1] = pos0 + cnt < n ? emb_bucket(idx[order[pos0 + cnt]], V) : -1;
   }
   __syncthreads();
   const int c = (blockIdx.y * 128 + threadIdx.x) * 8;
   if (c >= C) return;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  int run_start = 0;
-  for (int i = 0; i < cnt; ++i) {
-    u32x4 u = *(const u32x4*)(dy + (long)rows[i] * C + c);
+  const int first_tok = toks[0];
+  // how a run that ends at position i is added: 0 none ends there (or the bucket of out-of-range ids, dropped), 1 alone, 2 with the neighbours'
+  auto ends = [&](int i) {
+    if (i >= cnt || (i + 1 < cnt && toks[i + 1] == toks[i]) || toks[i] == V) return 0;
+    return (toks[i] == first_tok && edge[0] == toks[i]) || (i + 1 == cnt && edge[1] == toks[i]) ? 2 : 1;
+  };
+  for (int i0 = 0; i0 < cnt; i0 += EMB_AHEAD) {
+    u32x4 u[EMB_AHEAD];
+    f32x4 a0[EMB_AHEAD], a1[EMB_AHEAD];
+    int how[EMB_AHEAD];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      acc[2 * k] += bflo(u[k]);
-      acc[2 * k + 1] += bfhi(u[k]);
-    }
-    if (i + 1 == cnt || toks[i + 1] != toks[i]) {
-      float* d = dw + (long)toks[i] * C + c;
-      if (toks[i] == V) {
-        // the bucket of out-of-range ids: dropped
-      } else if ((run_start == 0 && edge[0] == toks[i]) || (i + 1 == cnt && edge[1] == toks[i])) {
-        // the token's run goes on in a neighbouring segment: another workgroup adds to the same row
-#pragma unroll
-        for (int k = 0; k < 8; ++k) atomicAdd(d + k, acc[k]);
-      } else {
-        f32x4 a0 = *(const f32x4*)d, a1 = *(const f32x4*)(d + 4);
-        *(f32x4*)d = f32x4{a0[0] + acc[0], a0[1] + acc[1], a0[2] + acc[2], a0[3] + acc[3]};
-        *(f32x4*)(d + 4) = f32x4{a1[0] + acc[4], a1[1] + acc[5], a1[2] + acc[6], a1[3] + acc[7]};
+    for (int x = 0; x < EMB_AHEAD; ++x) {
+      const int i = i0 + x;
+      how[x] = ends(i);
+      if (i < cnt) u[x] = *(const u32x4*)(dy + (long)rows[i] * C + c);
+      if (how[x] == 1) {
+        const float* d = dw + (long)toks[i] * C + c;
+        a0[x] = *(const f32x4*)d;
+        a1[x] = *(const f32x4*)(d + 4);
       }
+    }
 #pragma unroll
-      for (int k = 0; k < 8; ++k) acc[k] = 0.f;
-      run_start = i + 1;
+    for (int x = 0; x < EMB_AHEAD; ++x) {
+      const int i = i0 + x;
+      if (i >= cnt) break;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        acc[2 * k] += bflo(u[x][k]);
+        acc[2 * k + 1] += bfhi(u[x][k]);
+      }
+      if (i + 1 == cnt || toks[i + 1] != toks[i]) {
+        float* d = dw + (long)toks[i] * C + c;
+        if (how[x] == 2) {
+          // the token's run goes on in a neighbouring segment: another workgroup adds to the same row
+#pragma unroll
+          for (int k = 0; k < 8; ++k) atomicAdd(d + k, acc[k]);
+        } else if (how[x] == 1) {
+          *(f32x4*)d = f32x4{a0[x][0] + acc[0], a0[x][1] + acc[1], a0[x][2] + acc[2], a0[x][3] + acc[3]};
+          *(f32x4*)(d + 4) = f32x4{a1[x][0] + acc[4], a1[x][1] + acc[5], a1[x][2] + acc[6], a1[x][3] + acc[7]};
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[k] = 0.f;
+      }
     }
   }
 }
@@ -682,9 +702,16 @@ extern "C" int tfb_embedding_bwd_grouped(const void* idx, int idx64, const void*
     if (idx64) hipLaunchKernelGGL(emb_place_kernel<long>, dim3(nb), dim3(256), 0, s, (const long*)idx, cursor, order, n, V);
     else hipLaunchKernelGGL(emb_place_kernel<int>, dim3(nb), dim3(256), 0, s, (const int*)idx, cursor, order, n, V);
   }
-  dim3 grid((unsigned)((n + EMB_SEG - 1) / EMB_SEG), (unsigned)((C / 8 + 127) / 128));
-  if (idx64) hipLaunchKernelGGL(emb_reduce_kernel<long>, grid, dim3(128), 0, s, (const long*)idx, order, (const bf16_t*)dy, (float*)dw_f32, n, C, V);
-  else hipLaunchKernelGGL(emb_reduce_kernel<int>, grid, dim3(128), 0, s, (const int*)idx, order, (const bf16_t*)dy, (float*)dw_f32, n, C, V);
+  const auto reduce = [&](auto seg) {
+    constexpr int SEG = decltype(seg)::value;
+    const dim3 grid((unsigned)((n + SEG - 1) / SEG), (unsigned)((C / 8 + 127) / 128));
+    if (idx64) hipLaunchKernelGGL((emb_reduce_kernel<long, SEG>), grid, dim3(128), 0, s, (const long*)idx, order, (const bf16_t*)dy, (float*)dw_f32, n, C, V);
+    else hipLaunchKernelGGL((emb_reduce_kernel<int, SEG>), grid, dim3(128), 0, s, (const int*)idx, order, (const bf16_t*)dy, (float*)dw_f32, n, C, V);
+  };
+  if (n <= 512) reduce(std::integral_constant<int, 8>{});
+  else if (n <= 2048) reduce(std::integral_constant<int, 16>{});
+  else if (n < 24576) reduce(std::integral_constant<int, 32>{});
+  else reduce(std::integral_constant<int, 64>{});
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
