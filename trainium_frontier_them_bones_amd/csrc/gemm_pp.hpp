@@ -79,11 +79,79 @@ struct PpArgs {
   const int* seg;
   int ngroups;
   FastDiv d_ipx;
+  // over row tiles of groups (an epilogue with kRows): row_group[t] names the group of rows 128 t .. (-1: nobody's), its P lies
+  // p_group_stride bytes further
+  const int* row_group;
+  int row_tiles;
+  long p_group_stride;
 };
 template <class T, class = void>
 struct has_experts : std::false_type {};
 template <class T>
 struct has_experts<T, std::void_t<decltype(T::kExperts)>> : std::true_type {};
+
+template <class T, class = void>
+struct has_rows : std::false_type {};
+template <class T>
+struct has_rows<T, std::void_t<decltype(T::kRows)>> : std::true_type {};
+
+// A value that no store of this launch changes, by a scalar load (a vector load would be waited for behind the operand loads in flight)
+template <class T>
+__device__ __forceinline__ T tfb_scalar_load(const T* p) {
+  return *(const __attribute__((address_space(4))) T*)(uintptr_t)p;
+}
+
+// The grouped rows of a launch with kRows, cut into items of 256 rows from every group's first (128 where its last tile is alone), and what
+// the persistent kernel takes of the output tiles (256 columns of an item; item by item): whole rounds of the `nwg` workgroups, and a last part
+// of one too when it is 0.3 of a round or more (or the only one); what it leaves is finished by the ring (gemm_ring_rest_kernel). Only
+// the device knows the groups' loads; every wavefront reads the table for itself (64 tiles a lane-chunk, up to 4096 tiles).
+struct RowItems {
+  unsigned long long starts;  // lane c: the tiles among 64 c .. 64 c + 63 at which an item starts
+  int before;                 // lane c: the items that start in front of those
+  int items, total, taken;    // items; output tiles; those of the persistent kernel
+  bool ragged;                // it leaves some
+  __device__ __forceinline__ void init(const int* group, int tiles, int ncol, int nwg, int lane) {
+    starts = 0;
+    before = items = 0;
+    int seg0 = 0;  // the first tile of the group that a chunk begins in
+    for (int c0 = 0; 64 * c0 < tiles; c0 += 4) {
+      int g[4], gp[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int i = 64 * (c0 + x) + lane;
+        g[x] = i < tiles ? group[i] : -1;
+        gp[x] = i > 0 && i < tiles ? group[i - 1] : -1;
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        const int c = c0 + x, i = 64 * c + lane;
+        const unsigned long long b = __ballot(i == 0 || g[x] != gp[x]), le = b & (~0ull >> (63 - lane));
+        const int s0 = le ? 64 * c + 63 - __builtin_clzll(le) : seg0;
+        const unsigned long long m = __ballot(g[x] >= 0 && ((i - s0) & 1) == 0);
+        if (lane == c) {
+          starts = m;
+          before = items;
+        }
+        items += __builtin_popcountll(m);
+        if (b) seg0 = 64 * c + 63 - __builtin_clzll(b);
+      }
+    }
+    total = items * ncol;
+    const int full = total / nwg, rest = total - full * nwg;
+    ragged = full > 0 && rest > 0 && 10 * rest < 3 * nwg;
+    taken = ragged ? full * nwg : total;
+    chunks = (tiles + 63) >> 6;
+  }
+  int chunks;
+  // the first tile of item k
+  __device__ __forceinline__ int tile(int k, int lane) const {
+    const int c = 63 - __builtin_clzll(__ballot(lane < chunks && before <= k));
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)starts, c), hi = __builtin_amdgcn_readlane((unsigned)(starts >> 32), c);
+    const int r = k - __builtin_amdgcn_readlane(before, c), below = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0));
+    const unsigned bit = lane < 32 ? lo >> lane : hi >> (lane - 32);
+    return 64 * c + __builtin_ctzll(__ballot((bit & 1) && below == r));
+  }
+};
 
 // Epilogue protocol of this kernel (every epilogue of the library rounds f(accumulator) to bf16 first):
 //   float pre(float acc)                      applied to every accumulator before its rounding to bf16;
@@ -132,6 +200,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   // A partner 64 outputs away: a wavefront's two MFMA tiles of a P half are rows 32 wr .. and 64 + 32 wr ..
   constexpr int XROWS = kPartner == 64 ? 32 : 64, XTILE = kPartner == 64 ? 64 : 32;  // rows of X from one group to the other; from tile i = 0 to 1
   static_assert(kPartner != 64 || LAYX == TFB_K_CONTIG, "the fragments' rows");
+  constexpr bool kRows = has_rows<Epi>::value;
+  static_assert(!kRows || (!NARROW && !kF32 && LAYP == TFB_K_CONTIG && LAYQ == TFB_K_CONTIG && !has_prefetch<Epi>::value), "rows of groups");
   constexpr bool kPipe = has_prefetch<Epi>::value;  // the epilogue reads an operand of its own
   static_assert(!NARROW || LAYX == TFB_K_CONTIG || ES == 2, "half a quarter of fp8 rows");
   __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * 65536];
@@ -212,6 +282,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     }
   }
   const Side sx = make_side(QX ? a.Q : a.P, LAYX), sy = make_side(QX ? a.P : a.Q, LAYY);
+  [[maybe_unused]] RowItems ri;
+  if constexpr (kRows) ri.init(a.row_group, a.row_tiles, a.nfast, a.nwg, lane);
+  [[maybe_unused]] int row_group = 0;      // kRows, of the item that tile_of was last asked for: its group,
+  [[maybe_unused]] bool row_alone = false; // and whether its second 128 rows are not its group's
 
   // work item -> output tile origin and split
   auto tile_of = [&](int w, long& p0, long& q0, int& split) {
@@ -221,6 +295,14 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       w -= split * a.nout;
     }
     if constexpr (has_experts<Epi>::value) w -= first;
+    if constexpr (kRows) {
+      const int k = fastdiv(w, a.d_nfast), t = __builtin_amdgcn_readfirstlane(ri.tile(k, lane));
+      row_group = tfb_scalar_load(a.row_group + t);
+      row_alone = t + 1 >= a.row_tiles || tfb_scalar_load(a.row_group + t + 1) != row_group;
+      p0 = (long)(w - k * a.nfast) * TP;
+      q0 = (long)t * 128;
+      return;
+    }
     int fast, slow;
     if (a.rect) {
       const int x = w & 7, j = w >> 3;
@@ -255,14 +337,15 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   // quarter (X / Y, half h) of stage S <- the k-tile at g (the side's address of that k-tile of the output tile). The 64 rows of a
   // narrow tile's X half 1: k-contiguous, the first instruction alone; k-strided, both with the lanes of the chunks beyond them off.
   [[maybe_unused]] const bool in_half = ((lane & 15) ^ (4 * (lane >> 4))) < 8;
-  auto dma = [&](int S, int Y, int h, const uint8_t* g) __attribute__((always_inline)) {
+  // (alone, kRows: rows 128 .. 255 of the Y tile are another group's or no one's; the first 128 come twice, and are not stored again)
+  auto dma = [&](int S, int Y, int h, const uint8_t* g, bool alone = false) __attribute__((always_inline)) {
     const Side& sd = Y ? sy : sx;
     uint8_t* d = lds + S * 65536 + Y * 32768 + h * 16384 + wave * 1024;
     const bool half = NARROW && !Y && h;
     if (half && LAYX == TFB_K_STRIDED && !in_half) return;
 #pragma unroll
     for (int i = 0; i < (half && LAYX == TFB_K_CONTIG ? 1 : 2); ++i)
-      __builtin_amdgcn_global_load_lds((tfb_glb_void_t*)(g + h * sd.hstep + i * sd.istep + (size_t)sd.v),
+      __builtin_amdgcn_global_load_lds((tfb_glb_void_t*)(g + (kRows && alone ? 0 : h * sd.hstep) + i * sd.istep + (size_t)sd.v),
                                        (tfb_lds_void_t*)(d + i * 8192), 16, 0, 0);
   };
   constexpr int NX1 = NARROW && LAYX == TFB_K_CONTIG ? 1 : 2;  // a wavefront's load instructions for X half 1
@@ -410,11 +493,17 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   typedef std::integral_constant<int, 0> H0;
   typedef std::integral_constant<int, 1> H1;
 
-  const Epi epi = epi_prepare(epi_in);
+  Epi epi = epi_prepare(epi_in);
   int w = blockIdx.x, w_step = a.nwg, w_end = a.ntiles;  // this workgroup's items: w, w + w_step, .. below w_end
   if constexpr (has_experts<Epi>::value) {
     w = group_tile;
     w_end = 0;
+  } else if constexpr (kRows) {  // consecutive tiles for an XCD
+    const int per = (ri.taken + 7) >> 3, x0 = (w & 7) * per;
+    w = x0 + (w >> 3);
+    w_step = a.nwg >> 3;
+    w_end = x0 + per < ri.taken ? x0 + per : ri.taken;
+    if (w >= w_end) return;  // (whole workgroup)
   } else if (a.ipx > 0) {
     const int x0 = (w & 7) * a.ipx;
     w = x0 + (w >> 3);
@@ -428,6 +517,12 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   krange(split, k0, nkt);
   const uint8_t* gx = origin(sx, QX ? q0 : p0, k0);  // current work item: the sides' addresses of its first k-tile
   const uint8_t* gy = origin(sy, QX ? p0 : q0, k0);
+  [[maybe_unused]] bool alone = row_alone, alone_next = false, alone_prev = false;
+  [[maybe_unused]] Epi epi_now = epi, epi_next = epi;  // kRows: of this item and the next (epi: of the one that is stored)
+  if constexpr (kRows) {
+    gx += row_group * a.p_group_stride;
+    epi_now = epi_prepare(epi_in.for_group(row_group));
+  }
 
   // A segment without rows: nothing is loaded, its product is zero.
   if constexpr (has_experts<Epi>::value) {
@@ -441,12 +536,12 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   // ---- prologue: all of k-tile 0 into stage 0, three quarters of k-tile 1 into stage 1 (narrow tiles: the two quarters 0)
   dma(0, 1, 0, gy);
   dma(0, 0, 0, gx);
-  dma(0, 1, 1, gy);
+  dma(0, 1, 1, gy, alone);
   dma(0, 0, 1, gx);
   const long k_one = has_experts<Epi>::value && nkt < 2 ? 0 : 1;  // (a segment of one k-tile: that one again)
   dma(1, 0, 0, gx + k_one * sx.kstep);
   dma(1, 1, 0, gy + k_one * sy.kstep);
-  if constexpr (!NARROW) dma(1, 1, 1, gy + k_one * sy.kstep);
+  if constexpr (!NARROW) dma(1, 1, 1, gy + k_one * sy.kstep, alone);
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NARROW ? 4 : 6) : "memory");
   TFB_SBAR();               // k-tile 0 is there for everybody
   if (wr == 1) TFB_SBAR();  // group 1 runs one cluster behind from here on
@@ -587,6 +682,11 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     }
     gxn = origin(sx, QX ? qn : pn, k0n);
     gyn = origin(sy, QX ? pn : qn, k0n);
+    if constexpr (kRows) {
+      alone_next = row_alone;
+      gxn += row_group * a.p_group_stride;
+      epi_next = epi_prepare(epi_in.for_group(row_group));
+    }
   };
   auto go_on = [&]() __attribute__((always_inline)) {
     p0 = pn;
@@ -596,6 +696,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     nkt = nktn;
     gx = gxn;
     gy = gyn;
+    if constexpr (kRows) {
+      alone = alone_next;
+      epi_now = epi_next;
+    }
   };
   // One k-tile. In a tile's first iteration the MFMAs start from zero, and each accumulator block of the PREVIOUS tile is
   // stored in the memory cluster in front of the MFMA cluster that overwrites it: the stores of one group (4 KB per
@@ -614,7 +718,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     const uint8_t* gy2 = (in2 ? gy : gyn) + k2 * sy.kstep;
     auto store = [&](auto HX, auto HY, auto FROM) __attribute__((always_inline)) {
       if constexpr (stores) {
-        if (have_prev) store_block(HX, HY, pp0, pq0, FROM);
+        if (have_prev && !(kRows && decltype(HY)::value == 1 && alone_prev)) store_block(HX, HY, pp0, pq0, FROM);
       }
     };
     // kPipe: the block whose operand was requested before AFTER vector memory instructions; then next() asks for the next one's
@@ -673,13 +777,14 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       // instructions), and in a first iteration with stores all but those and the 12 stores (c0's four were issued
       // behind its loads); kPipe: c2's and c4's stores and four requests each, in front of their loads. After the barrier that ends c6 both
       // groups have waited, so the next k-tile is complete.
-      if (stores && have_prev) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPipe ? 20 : 16) : "memory");
+      if (kRows && stores && have_prev && alone_prev) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");  // (c2 has stored nothing)
+      else if (stores && have_prev) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kPipe ? 20 : 16) : "memory");
       else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
       TFB_SBAR();
       // c6
       store_pipe(H1{}, H1{}, N2{}, nothing);
       request_first();
-      dma(S, 1, 1, gy2);
+      dma(S, 1, 1, gy2, in2 ? alone : alone_next);
       store_plain(H1{}, H1{});
       TFB_SBAR();
       // c7: the next k-tile's first Y fragments are requested under this cluster's MFMAs (fb0 was last read in c5)
@@ -769,6 +874,10 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       have_prev = true;
       pp0 = p0;
       pq0 = q0;
+      if constexpr (kRows) {
+        alone_prev = alone;
+        epi = epi_now;
+      }
     }
     w = wn;
     if (w >= w_end) break;
@@ -787,9 +896,9 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
       store_block(HX, HY, pp0, pq0, H0{});
     };
     flush(H0{}, H0{}, std::false_type{});
-    flush(H0{}, H1{}, std::true_type{});
+    if (!(kRows && alone_prev)) flush(H0{}, H1{}, std::true_type{});
     flush(H1{}, H0{}, std::true_type{});
-    flush(H1{}, H1{}, std::true_type{});
+    if (!(kRows && alone_prev)) flush(H1{}, H1{}, std::true_type{});
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stream's last (unused) loads must have landed before LDS is released
 }
@@ -952,6 +1061,41 @@ static int gemm_pp_launch_experts(GemmOperand P0, GemmOperand Q0, int np0, int n
   a.seg = seg;
   a.ngroups = groups;
   hipLaunchKernelGGL((gemm_pp_kernel<1, TFB_FMT_E4M3, TFB_FMT_E5M2, TFB_K_STRIDED, TFB_K_STRIDED, Epi>), dim3(a.nwg), dim3(512), 0, stream, a, epi);
+  TFB_LAUNCH_CHECK();
+  return TFB_OK;
+}
+
+// A grouped fp8 product over the rows of all groups (row_group: PpArgs), both operands k-contiguous: D[p][q] = sum_k P_g[p][k] Q[q][k]. What it
+// leaves is the ring's (gemm_ring_rest).
+static inline int gemm_pp_rows_wgs() { return (int)tfb_resident_slots(1) & ~7; }
+// Used where half the CUs or more have an output tile (counted by the rows the tables hold). What bounds it is the k-loop, as in dense launches;
+// the 128 x 128 kernel moves twice the operand bytes (16384 tokens, two of eight experts, d 1024, F 2816: 120 and 131 -> 88 us, and 16.5 for the rest).
+// Forward and backward of the layer, us, 128 x 128 -> this (tiles over CUs): d 1024, F 2816: 6144 tokens x 2 (0.8) 418 -> 405, 16384 x 2 (2.1) 849
+// -> 803, 4096 x 2 (0.55) 338 -> 330, 6144 x 1 (0.43) 281 -> 301; d 768, F 1536: 16384 x 2 532 -> 495, 6144 x 2 (0.6) 265 -> 249, 8192 x 1 (0.42) 215 ->
+// 217; d 512, F 1024: 16384 x 2 (1.05) 306 -> 299, 8192 x 2 (0.53) 203 -> 200, 12288 x 1 (0.4) 175 -> 189.
+static inline bool gemm_pp_rows_applies(long np, long rows, long kbytes) {
+  const long cus = gemm_pp_rows_wgs();
+  return TFB_PP && cus > 0 && np % 256 == 0 && rows % 128 == 0 && rows <= 128L * 4096 && kbytes % 128 == 0 && kbytes >= 256 && (rows / 128) * (np / 256) >= cus;
+}
+template <int FMTP, int FMTQ, class Epi>
+static int gemm_pp_launch_rows(GemmOperand P, long p_group_stride, GemmOperand Q, int np, long rows, long kbytes, const int* row_group, Epi epi,
+                               hipStream_t stream) {
+  const int nwg = gemm_pp_rows_wgs();
+  if (nwg <= 0 || np <= 0 || np % 256 || rows <= 0 || rows % 128 || rows > 128L * 4096 || kbytes % 128 || kbytes < 256 || !row_group) return TFB_ERR_SHAPE;
+  if (P.ld <= 0 || Q.ld <= 0 || P.ld > (1L << 28) || Q.ld > (1L << 28)) return TFB_ERR_SHAPE;
+  if (((uintptr_t)P.base | (uintptr_t)Q.base | (uintptr_t)P.ld | (uintptr_t)Q.ld | (uintptr_t)p_group_stride) & 15) return TFB_ERR_ARG;
+  PpArgs a = {};
+  a.P = P;
+  a.Q = Q;
+  a.splits = 1;
+  a.nk_total = (int)(kbytes / 128);
+  a.nfast = np / 256;
+  a.d_nfast = fastdiv_make(a.nfast);
+  a.nwg = nwg;
+  a.row_group = row_group;
+  a.row_tiles = (int)(rows / 128);
+  a.p_group_stride = p_group_stride;
+  hipLaunchKernelGGL((gemm_pp_kernel<1, FMTP, FMTQ, TFB_K_CONTIG, TFB_K_CONTIG, Epi>), dim3(nwg), dim3(512), 0, stream, a, epi);
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }

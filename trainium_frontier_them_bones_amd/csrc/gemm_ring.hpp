@@ -203,9 +203,9 @@ __device__ __forceinline__ void ring_wait(int tiles) {
 #undef TFB_RING_WAIT
 }
 
-// Workgroup `block` of the launch: one output tile.
+// Workgroup `block` of the launch: one output tile (given_p >= 0: that one).
 template <class Cfg, bool RANGES, class Epi>
-__device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, int block, uint8_t* lds) {
+__device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, int block, uint8_t* lds, int given_p = -1, int given_q = 0) {
   constexpr int BP = Cfg::BP, BQ = Cfg::BQ, NW = Cfg::NW, TP = Cfg::TP, TQ = Cfg::TQ, ES = Cfg::ES, NS = Cfg::NS;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -224,6 +224,10 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
     tile_q = 0;
     for (; tile_p >= a.ntp - tile_q; ++tile_q) tile_p -= a.ntp - tile_q;   // row tile_q has ntp - tile_q tiles
     tile_p += tile_q;
+  } else if (given_p >= 0) {
+    lid = split = 0;
+    tile_p = given_p;
+    tile_q = given_q;
   } else {
     gemm_tile_of(a, block, lid, split, tile_p, tile_q);
   }
@@ -597,6 +601,34 @@ static bool gemm_pp_try(GemmOperand P, GemmOperand Q, int np, int nq, long kbyte
   a.nkt = (int)(kbytes / 128);
   st = gemm_ring_launch<Epi, ES, LAYP, LAYQ, FMTP, FMTQ>(128L * np <= 4096L * tfb_resident_slots(1) ? 1 : 2, a, 1, 1, e, s, 1, main);
   return true;
+}
+
+// What the persistent kernel leaves of a grouped product over rows (RowItems): its last output tiles as 128 x 64 ones, eight workgroups each.
+template <class Cfg, class Epi>
+__global__ __launch_bounds__(Cfg::NT, 2) void gemm_ring_rest_kernel(GemmArgs a, Epi epi_in, int row_tiles, int ncol, FastDiv d_ncol, int nwg) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[Cfg::LDS_BYTES];
+  static_assert(Cfg::BP == 128 && Cfg::BQ == 64, "eight tiles of 256 x 256");
+  const int lane = threadIdx.x & 63, sub = blockIdx.x & 7;
+  RowItems ri;
+  ri.init(a.q_group, row_tiles, ncol, nwg, lane);
+  const int w = ri.taken + (int)(blockIdx.x >> 3);
+  if (w >= ri.total) return;  // (the whole workgroup, as below)
+  const int k = fastdiv(w, d_ncol), t = __builtin_amdgcn_readfirstlane(ri.tile(k, lane));
+  if (sub >= 4 && (t + 1 >= row_tiles || a.q_group[t + 1] != a.q_group[t])) return;
+  gemm_ring_tile<Cfg, false>(a, epi_in, 0, lds, 2 * (w - k * ncol) + (sub & 1), 2 * t + (sub >> 1));
+}
+template <int FMTP, int FMTQ, class Epi>
+static int gemm_ring_rest(GemmArgs a, Epi e, hipStream_t s) {
+  using Cfg = RingCfg<128, 64, 2, 2, 1, TFB_K_CONTIG, TFB_K_CONTIG, FMTP, FMTQ, 3>;
+  a.ntp = a.np / 128;
+  a.q_off = 0;
+  const int row_tiles = a.nq / 128, ncol = a.np / 256, nwg = gemm_pp_rows_wgs();
+  const int st = gemm_ring_args<Cfg>(a, 1, 1);
+  if (st != TFB_OK) return st;
+  const long most = std::min((long)row_tiles * ncol, 3L * nwg / 10 + 1);
+  hipLaunchKernelGGL((gemm_ring_rest_kernel<Cfg, Epi>), dim3((unsigned)(8 * most)), dim3(Cfg::NT), 0, s, a, e, row_tiles, ncol, fastdiv_make(ncol), nwg);
+  TFB_LAUNCH_CHECK();
+  return TFB_OK;
 }
 
 // ---- several independent contractions in one launch ------------------------------------------------------------------

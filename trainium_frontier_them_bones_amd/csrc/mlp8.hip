@@ -516,6 +516,16 @@ struct EpiScaleStore {  // out = bf16(acc * sc[col])
 // out = bf16(res + bf16(acc * dq)): EpiScaleStore / EpiDescale with the residual add that follows the projection made in
 // the same store (the reference's projection-with-residual forward, K/nki_attn_nr8.py:1003, and the residual half of
 // K/nki_mlp_nr8.py:1032); dq = sc[col] when sc is given, else dq_imm * *dq_a * *dq_b. Two roundings, as the separate add.
+struct EpiScaleRows : EpiScaleStore {  // for the persistent kernel over the rows of groups
+  static constexpr bool kRows = true;
+  __device__ __forceinline__ EpiScaleRows for_group(int g) const { return EpiScaleRows{EpiScaleStore::for_group(g)}; }
+  __device__ __forceinline__ EpiScaleRows prepare() const {
+    EpiScaleRows e = *this;
+    e.dq = tfb_scalar_load(sc + col);
+    return e;
+  }
+};
+
 struct EpiDescaleRes {
   const float* sc;
   int col;
@@ -1193,7 +1203,7 @@ namespace {
 template <class Cfg, class Epi>
 int grouped_launch(const uint8_t* wbase, long wld, long wgroup_stride, const uint8_t* act, long ald, int np, long rmax, long kbytes,
                    const int* tile_expert, Epi e, hipStream_t s) {
-  GemmArgs a;
+  GemmArgs a = {};
   a.P = GemmOperand{wbase, wld};
   a.Q = GemmOperand{act, ald};
   a.np = np;
@@ -1203,6 +1213,12 @@ int grouped_launch(const uint8_t* wbase, long wld, long wgroup_stride, const uin
   a.q_group = tile_expert;
   a.p_group_stride = wgroup_stride;
   a.k_seg = nullptr;
+  if constexpr (std::is_same<Epi, EpiScaleStore>::value) {
+    if (gemm_pp_rows_applies(np, rmax, kbytes)) {
+      const int st = gemm_pp_launch_rows<Cfg::FMTP, Cfg::FMTQ>(a.P, wgroup_stride, a.Q, np, rmax, kbytes, tile_expert, EpiScaleRows{e}, s);
+      return st != TFB_OK ? st : gemm_ring_rest<Cfg::FMTP, Cfg::FMTQ>(a, e, s);
+    }
+  }
   if (const int pick = gemm_ring_pick(np, rmax, a.nkt, false))
     return gemm_ring_launch<Epi, Cfg::ES, Cfg::LAYP, Cfg::LAYQ, Cfg::FMTP, Cfg::FMTQ>(pick, a, 1, 1, e, s);
   return gemm_launch_args<Cfg>(a, 1, 1, LoadIdentity{}, LoadIdentity{}, e, s);
