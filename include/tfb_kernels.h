@@ -304,6 +304,8 @@ int tfb_attn_bwd(const void* q, const long* q_strides, const void* k, const long
  * or dK/dV runs by pairs with 64 keys a workgroup instead (which 3), under a band nw (0 = none) and for token strides below 2^25 elements. The
  * results do not depend on it. */
 int tfb_attn_bwd_pairs_applies(int which, int B, int H, int T, int D, int nw);
+/* The same of a forward, which has one such kernel. */
+int tfb_attn_fwd_pairs_applies(int B, int H, int T, int D, int nw);
 /* tfb_attn_bwd for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): the same kernels and results, with the delta scratch taken from a static device
  * array inside the library (8 MiB per GPU, held until the process ends) instead of from the caller. It allocates and

@@ -58,6 +58,7 @@ SIGNATURES = {
     "tfb_attn_bwd": [_vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _vp, _i, _i, _i, _i,
                      _f, _vp],
     "tfb_attn_bwd_pairs_applies": [_i, _i, _i, _i, _i, _i],
+    "tfb_attn_fwd_pairs_applies": [_i, _i, _i, _i, _i],
     "tfb_attn_bwd_static": [_vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _lp, _vp, _i, _i, _i, _i,
                             _f, _vp],
     "tfb_attn_bwd_static_max_rows": [],

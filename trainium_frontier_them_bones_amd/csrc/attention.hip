@@ -107,6 +107,13 @@ extern "C" int tfb_attn_bwd_pairs_applies(int which, int B, int H, int T, int D,
   return yes ? TFB_OK : TFB_ERR_SHAPE;
 }
 
+// Whether a forward runs by pairs of wavefronts, for token strides that it takes.
+extern "C" int tfb_attn_fwd_pairs_applies(int B, int H, int T, int D, int nw) {
+  if (B <= 0 || H <= 0 || T <= 0 || T % 128 || (D != 64 && D != 128) || nw < 0) return TFB_ERR_SHAPE;
+  const long st[3] = {0, 0, D};
+  return tfb_attn_fwd_pair_applies(D, T, (long)B * H, nw, st, st) ? TFB_OK : TFB_ERR_SHAPE;
+}
+
 // ---- attention backward for callers that cannot allocate --------------------------------------------------------------
 // tfb_attn_bwd needs fp32 [2][B*H][T] of device scratch (the row statistics its first kernel, dQ, leaves for
 // the second) and takes it from the caller. Code under HIP graph capture, tight serving loops and harnesses that forbid

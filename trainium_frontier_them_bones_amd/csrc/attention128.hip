@@ -525,6 +525,7 @@ __global__ __launch_bounds__(256, 2) void attnD_dq_kernel(AttnT q, AttnT k, Attn
 template <int D>
 int fwd_launch(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, void* o,
                const long* os, float* lse, int B, int H, int T, float scale, int nw, hipStream_t s) {
+  if (tfb_attn_fwd_pair_applies(D, T, (long)B * H, nw, ks, vs)) return tfb_attn_fwd_pair_impl(q, qs, k, ks, v, vs, o, os, lse, B, H, T, D, scale, nw, s);
   hipLaunchKernelGGL(attnD_fwd_kernel<D>, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs),
                      mk(o, os), lse, T, H, scale * LOG2E, nw, first_round(T / 128, B * H, true));
   TFB_LAUNCH_CHECK();

@@ -787,6 +787,7 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
 // Called by tfb_attn_fwd / tfb_attn_bwd for D = 64 (arguments already validated there: T % 128 == 0, strides % 8 == 0).
 int tfb_attn64_fwd_impl(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, void* o,
                         const long* os, float* lse, int B, int H, int T, float scale, int nw, hipStream_t s) {
+  if (tfb_attn_fwd_pair_applies(64, T, (long)B * H, nw, ks, vs)) return tfb_attn_fwd_pair_impl(q, qs, k, ks, v, vs, o, os, lse, B, H, T, 64, scale, nw, s);
   hipLaunchKernelGGL(attn64_fwd_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(o, os), lse,
                      T, H, scale * LOG2E, nw, tfb_resident_slots(2), first_round(T / 128, B * H, true));
   TFB_LAUNCH_CHECK();

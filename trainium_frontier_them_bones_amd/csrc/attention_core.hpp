@@ -16,6 +16,9 @@ static inline bool tfb_attn_dkdv_strides_ok(const long* qs, const long* gos) {
 int tfb_attn_dq_pair_impl(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, const void* o,
                           const long* os, const void* go, const long* gos, void* dq, const long* dqs, const float* lse, float* stats, int B, int H,
                           int T, int D, float scale, const void* cos_t, const void* sin_t, int nw, hipStream_t s);
+// The forward by pairs of wavefronts, 64 queries a workgroup (attention_fwd.hip). The same holds of its loads.
+int tfb_attn_fwd_pair_impl(const void* q, const long* qs, const void* k, const long* ks, const void* v, const long* vs, void* o, const long* os,
+                           float* lse, int B, int H, int T, int D, float scale, int nw, hipStream_t s);
 // Pairs divide a block's work between twice the wavefronts and do a little more of it. That shortens a launch whose longest block sets the
 // time and not one whose blocks keep the SIMDs busy, so what counts is the work a CU has in units of the longest block. A causal
 // block i of nx has i + 1 tiles, a band leaves it nw at most: the blocks of a short sequence or a narrow band are nearly alike and fill the
@@ -71,6 +74,22 @@ static inline bool tfb_attn_dkdv_half_applies(int D, int T, long nbh, int nw, co
   if (l.longest == 1) return false;
   const long line = l.longest <= 4 && 4 * l.longest <= nx ? 14 : l.longest == nx && nx >= 8 && nx <= 16 ? 10 : 8;
   return 10 * l.work <= line * cus * l.longest;
+}
+
+// The forward: one workgroup of 64 queries for each CU (but for blocks of one tile of D = 128), or as much work as this line, in the same units.
+// us, one wavefront to 32 queries -> pairs, blocks in brackets:
+//   D = 64   T128 [128] 5.9 -> 5.4, [192] 6.1 -> 6.2; T256 [192] 7.5 -> 6.7, [320] 9.9 -> 9.9; T512 [192] 9.8 -> 8.8, [256] 10.0 -> 9.2, [320] 11.1 -> 12.0; T1024
+//            [256] 14.8 -> 13.4, [320] 15.3 -> 15.7; T1664 [312] 21.2 -> 19.5, [364] 21.5 -> 22.8; T2048 [192] 24.2 -> 21.2, [320] 24.8 -> 22.8, [384] 25.2 ->
+//            27.1; T4096 [320] 44.7 -> 40.1, [384] 45.3 -> 47.1; bands of T2048: 2 [128] 7.0 -> 6.2, [192] 7.3 -> 7.4; 4 [128] 9.4 -> 8.3, [192] 9.8 -> 10.6;
+//            8 [192] 14.8 -> 13.6, [256] 15.2 -> 17.2
+//   D = 128  T128 [128] 7.6 -> 7.7; T256 [128] 9.7 -> 9.3, [192] 10.5 -> 14.2; T512 [128] 12.9 -> 12.2, [192] 13.6 -> 16.2; T1024 [128] 19.6 -> 18.4, [192]
+//            20.3 -> 20.1, [224] 20.6 -> 22.6; T1664 [208] 28.0 -> 26.1, [260] 28.9 -> 35.4; T2048 [192] 32.8 -> 30.7, [224] 32.9 -> 32.8, [256] 33.2 -> 34.8;
+//            T4096 [192] 58.1 -> 55.2, [256] 59.2 -> 59.1; bands of T2048: 4 [128] 13.0 -> 12.4, [192] 14.2 -> 22.0
+static inline bool tfb_attn_fwd_pair_applies(int D, int T, long nbh, int nw, const long* ks, const long* vs) {
+  const AttnLoad l = attn_load(T, nbh, nw);
+  const long cus = tfb_resident_slots(1);
+  if (!tfb_attn_dkdv_strides_ok(ks, vs) || (D == 128 && l.longest == 1)) return false;
+  return 2 * l.blocks <= cus || 1000 * l.work <= (D == 64 ? 665 : 440) * cus * l.longest;
 }
 
 namespace {
