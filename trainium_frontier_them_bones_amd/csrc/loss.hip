@@ -162,18 +162,31 @@ __device__ __forceinline__ MS ms_wave_row(const u32x4 (&u)[4], int t0, int V, fl
   }
   return a;
 }
-// d x_v = g (softmax_v - [v == t]) (1 - tanh^2) of eight values from v = i on
-__device__ __forceinline__ u32x4 loss_grad8(const u32x4& u, int i, long tt, float g, float l, float icap, float cap) {
-  float d[8];
+// d x_v = g (softmax_v - [v == t]) (1 - tanh^2) of eight values from v = i on; t: the row's target, -1 where it has none.
+// The target's one is taken off behind a branch that a wavefront takes for one of its chunks at most: a comparison, a select and a
+// subtraction for each value were a quarter of the vector instructions that these passes spend their time on beside memory.
+__device__ __forceinline__ u32x4 loss_grad8(const u32x4& u, int i, int t, float g, float l, float icap, float cap) {
+  float v[8], d[8];
+  unpack8bf(u, v);
+  if (cap > 0.f) {
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const float v = k & 1 ? bfhi(u[k >> 1]) : bflo(u[k >> 1]), hot = (i + k == tt) ? 1.0f : 0.0f;
-    if (cap > 0.f) {
-      const float t = tanh_fast(v * icap);
-      d[k] = g * (fexp(cap * t - l) - hot) * (1.0f - t * t);
-    } else {
-      d[k] = g * (fexp(v - l) - hot);
+    for (int k = 0; k < 8; ++k) {
+      v[k] = tanh_fast(v[k] * icap);
+      d[k] = fexp(cap * v[k] - l);
     }
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) d[k] = fexp(v[k] - l);
+  }
+  if ((unsigned)(t - i) < 8u) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) d[k] = t - i == k ? d[k] - 1.0f : d[k];
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) d[k] *= g;
+  if (cap > 0.f) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) d[k] *= 1.0f - v[k] * v[k];
   }
   return u32x4{pack2bf(d[0], d[1]), pack2bf(d[2], d[3]), pack2bf(d[4], d[5]), pack2bf(d[6], d[7])};
 }
@@ -231,7 +244,9 @@ __global__ __launch_bounds__(256) void loss_bwd_kernel(const bf16_t* __restrict_
   bf16_t* dr = dx + row * V;
   const int t0 = threadIdx.x % TPR;
   const long tt = (long)tg[row];
-  const float g = (unsigned long)tt < (unsigned long)V ? grow[row] : 0.f;  // out of range = ignored
+  const bool valid = (unsigned long)tt < (unsigned long)V;  // out of range = ignored
+  const float g = valid ? grow[row] : 0.f;
+  const int t = valid ? (int)tt : -1;   // (t - i of a chunk at i >= 0 is then no column of it)
   const float l = lse[row];
   const float icap = cap > 0.f ? 1.0f / cap : 0.f;
   // (the next chunk is requested before this chunk's store: a wait for loaded data also waits for every older store)
@@ -239,7 +254,7 @@ __global__ __launch_bounds__(256) void loss_bwd_kernel(const bf16_t* __restrict_
   for (int i = t0 * 8; i < V; i += TPR * 8) {
     const u32x4 u = unext;
     unext = logits8(xr, i + TPR * 8, V);
-    *(u32x4*)(dr + i) = loss_grad8(u, i, tt, g, l, icap, cap);
+    *(u32x4*)(dr + i) = loss_grad8(u, i, t, g, l, icap, cap);
   }
 }
 
@@ -248,6 +263,11 @@ __global__ __launch_bounds__(256) void loss_bwd_kernel(const bf16_t* __restrict_
 // the weighted row loss, and overwrite the row with d x_v = w (softmax_v - [v = t]) (1 - tanh^2): the gradient for an
 // upstream gradient of one, which the caller's two gradient GEMMs scale by the real one. The logits are read once and
 // written once where the two kernels read them twice; values equal theirs bit for bit.
+// Bound by memory and by the vector instructions beside it. The target's one behind a branch (loss_grad8) and a store that does not pass
+// through the caches: rows of 32768, 32768 of them 935 -> 790 us, 8192 249 -> 211, 2048 76 -> 66. A row of 32 chunks is unpacked twice, behind an
+// empty asm statement: kept unpacked, its 256 values spilled (4096 rows of 50304 431 us; with the branch alone 257, so 183). With 16 chunks the
+// registers suffice, and two wavefronts a SIMD that unpack once stream better than four that unpack twice (32768 rows 790 us to 860,
+// 2048 66 to 64).
 template <typename IDX, int NCH, int TPR>
 __global__ __launch_bounds__(256) void loss_fwd_bwd_kernel(bf16_t* x, const IDX* __restrict__ tg, const float* __restrict__ row_w,
                                                           float* __restrict__ loss, float* __restrict__ lse, long rows, int V, float cap) {
@@ -262,6 +282,7 @@ __global__ __launch_bounds__(256) void loss_fwd_bwd_kernel(bf16_t* x, const IDX*
   for (int j = 0; j < NCH; ++j) u[j] = logits8(xr, (t0 + j * TPR) * 8, V);
   const long tt = (long)tg[row];
   const bool valid = (unsigned long)tt < (unsigned long)V;  // a target outside [0, V) is an ignored row, never an address
+  const int t = valid ? (int)tt : -1;
   const float w = valid ? (row_w ? row_w[row] : 1.0f) : 0.f;
   const float xt = valid ? bf2f(xr[tt]) : 0.f;              // (read before any thread overwrites the row)
   MS a{cap > 0.f ? cap : -1e30f, 0.f};
@@ -286,7 +307,8 @@ __global__ __launch_bounds__(256) void loss_fwd_bwd_kernel(bf16_t* x, const IDX*
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
     const int i = (t0 + j * TPR) * 8;
-    if (i < V) *(u32x4*)(xr + i) = loss_grad8(u[j], i, tt, w, l, icap, cap);
+    if (NCH == 32) asm("" : "+v"(u[j]));
+    if (i < V) tfb_store_nt((u32x4*)(xr + i), loss_grad8(u[j], i, t, w, l, icap, cap));
   }
 }
 
