@@ -66,9 +66,7 @@ struct Row {
   }
 };
 
-// A row as loaded (bf16 pairs in 32-bit words), to be widened later: the kernels below request the NEXT row of a
-// wavefront before they store the current one. A wait for loaded data also waits for every older memory operation, stores
-// included (one counter orders both), so a loop that loads after its stores pays a full store round trip per row.
+// A row as loaded (bf16 pairs in 32-bit words), widened where it is used: half of a widened row's registers.
 template <int NCH, int G = 64>
 struct RawRow {
   u32x4 u[NCH];
@@ -79,6 +77,7 @@ struct RawRow {
       u[i] = c < C ? *(const u32x4*)(p + c) : u32x4{0u, 0u, 0u, 0u};
     }
   }
+  __device__ __forceinline__ float at(int i, int k) const { return k & 1 ? bfhi(u[i][k >> 1]) : bflo(u[i][k >> 1]); }
   __device__ __forceinline__ void widen(Row<NCH, G>& r) const {
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
@@ -107,7 +106,13 @@ __device__ __forceinline__ float row_dot(const Row<NCH, G>& a, const Row<NCH, G>
   return group_sum<G>(s);
 }
 
+// The pair's grids: a turn for each row up to here (a loop beyond).
+constexpr long ROW_GRID = 1L << 20;
+
 // ------------------------------------------------------------------------------------------
+// Bound by memory, in small launches by its latency. A row for each group of lanes and none asked for ahead: rows in flight come from
+// more wavefronts on a SIMD (the next row's registers, and the gain's in fp32, kept them at three), and a store has no load behind it to
+// hold up. bf16 and e4m3 out, gain: 32768 x 768 20.2 -> 17.0 us, 8192 x 768 9.8 -> 7.2, 2048 x 768 5.3 -> 4.7.
 template <int NCH, int G>
 __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ res,
                                                          const bf16_t* __restrict__ w, bf16_t* __restrict__ s_out,
@@ -115,29 +120,21 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restri
                                                          int C, float eps, uint8_t* __restrict__ y8, float y8_scale, long nrows_out) {
   constexpr int RPW = 64 / G;  // rows per wavefront
   const int lane = threadIdx.x & (G - 1), sub = (threadIdx.x & 63) / G, wave = threadIdx.x >> 6;
-  Row<NCH, G> wr;
+  RawRow<NCH, G> wr;
   if (w) wr.load(w, C, lane);
   const long step = (long)gridDim.x * ROWS_PER_BLOCK * RPW;
   long row = ((long)blockIdx.x * ROWS_PER_BLOCK + wave) * RPW + sub;
-  RawRow<NCH, G> xa, xr;
-  if (row < nrows) {
+  for (; row < nrows; row += step) {
+    RawRow<NCH, G> xa, xr;
     xa.load(x + row * C, C, lane);
     if (res) xr.load(res + row * C, C, lane);
-  }
-  for (; row < nrows; row += step) {
     Row<NCH, G> a;
     xa.widen(a);
-    Row<NCH, G> r;
-    if (res) xr.widen(r);
-    if (row + step < nrows) {  // the next row's loads go out before this row's stores
-      xa.load(x + (row + step) * C, C, lane);
-      if (res) xr.load(res + (row + step) * C, C, lane);
-    }
     if (res) {
 #pragma unroll
       for (int i = 0; i < NCH; ++i)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) a.v[i][k] = round_bf(a.v[i][k] + r.v[i][k]);
+        for (int k = 0; k < 8; ++k) a.v[i][k] = round_bf(a.v[i][k] + xr.at(i, k));
       if (s_out) a.store(s_out + row * C, C, lane);
     }
     float ss = row_dot(a, a);
@@ -145,7 +142,7 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restri
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
 #pragma unroll
-      for (int k = 0; k < 8; ++k) a.v[i][k] = w ? a.v[i][k] * rs * wr.v[i][k] : a.v[i][k] * rs;
+      for (int k = 0; k < 8; ++k) a.v[i][k] = w ? a.v[i][k] * rs * wr.at(i, k) : a.v[i][k] * rs;
     if (y) a.store(y + row * C, C, lane);
     if (y8) {  // e4m3(bf16(y) * scale): the cast the fp8 GEMM that consumes y would otherwise make in a pass of its own
       a.round();
@@ -176,54 +173,50 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restri
 }
 
 // dx = gs + J^T(gy): J^T(gy) = inv * (gh - s * (gh . s) * inv^2 / C), gh = gy * w.
-// dw partial [gridDim.x][C] = sum over the workgroup's rows of gy * s * inv.
-template <int NCH, int G>
+// dw partial [gridDim.x][C] = sum over the workgroup's rows of gy * s * inv (W: there is a gain).
+// Bound as the forward, and as that one without a row asked for ahead. With a gain, 8192 x 768: 16.1 -> 12.8 us in a training step, alone
+// 16384 x 768 21.0 -> 17.8, 2048 x 1024 6.5 -> 5.8, 4096 x 4096 48 -> 40, 32768 x 768 32.5 -> 31.4; without one, by a kernel of its own (half the
+// registers) with a turn for each row: 256 x 768 3.2 -> 3.1, 8192 x 768 9.7 -> 8.3, 4096 x 4096 28 -> 21, 32768 x 1024 40.0 -> 38.7. Widening the row twice
+// (119 registers for 166 at 768 columns) gave as much on many rows with a gain and cost 1500 x 1024 without one 0.6 us of 4.1.
+template <int NCH, int G, bool W>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ gs,
                                                          const bf16_t* __restrict__ s, const bf16_t* __restrict__ w,
                                                          const float* __restrict__ inv, bf16_t* __restrict__ dx,
                                                          float* __restrict__ dw_part, float* __restrict__ amax_part, long nrows,
                                                          int C) {
   constexpr int RPW = 64 / G, RPB = ROWS_PER_BLOCK * RPW;  // rows per wavefront, per workgroup
-  __shared__ float red[RPB][NCH * G * 8];
+  __shared__ float red[W ? RPB : 1][W ? NCH * G * 8 : 1];
   __shared__ float amred[ROWS_PER_BLOCK];
   const int lane = threadIdx.x & (G - 1), sub = (threadIdx.x & 63) / G, wave = threadIdx.x >> 6;
   float am = 0.f;   // amax of the rounded dx this wavefront wrote (amax_part: one value per workgroup)
-  Row<NCH, G> wr, dwacc;
-  if (w) wr.load(w, C, lane);
-  dwacc.zero();
+  Row<NCH, G> dwacc;
+  RawRow<NCH, G> wr;
+  if (W) {
+    wr.load(w, C, lane);
+    dwacc.zero();
+  }
   const long step = (long)gridDim.x * RPB;
   long row = ((long)blockIdx.x * ROWS_PER_BLOCK + wave) * RPW + sub;
   RawRow<NCH, G> xg, xa, xr;
-  float rs_next = 0.f;
-  if (row < nrows) {
+  for (; row < nrows; row += step) {
+    const float rs = inv[row];
     xg.load(gy + row * C, C, lane);
     xa.load(s + row * C, C, lane);
     if (gs) xr.load(gs + row * C, C, lane);
-    rs_next = inv[row];
-  }
-  for (; row < nrows; row += step) {
-    Row<NCH, G> g, a, r;
+    Row<NCH, G> g, a;
     xg.widen(g);
     xa.widen(a);
-    if (gs) xr.widen(r);
-    const float rs = rs_next;
-    if (row + step < nrows) {  // the next row's loads go out before this row's store
-      xg.load(gy + (row + step) * C, C, lane);
-      xa.load(s + (row + step) * C, C, lane);
-      if (gs) xr.load(gs + (row + step) * C, C, lane);
-      rs_next = inv[row + step];
-    }
-    if (w) {
+    if (W) {
 #pragma unroll
       for (int i = 0; i < NCH; ++i)
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
           dwacc.v[i][k] += g.v[i][k] * a.v[i][k] * rs;
-          g.v[i][k] *= wr.v[i][k];
+          g.v[i][k] *= wr.at(i, k);
         }
     }
-    float dot = row_dot(g, a);
-    float coef = dot * rs * rs * (1.0f / C);
+    const float dot = row_dot(g, a);
+    const float coef = dot * rs * rs * (1.0f / C);
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
 #pragma unroll
@@ -232,7 +225,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const bf16_t* __restri
 #pragma unroll
       for (int i = 0; i < NCH; ++i)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) g.v[i][k] += r.v[i][k];
+        for (int k = 0; k < 8; ++k) g.v[i][k] += xr.at(i, k);
     }
     if (amax_part) {
       g.round();
@@ -256,7 +249,7 @@ __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const bf16_t* __restri
       amax_part[blockIdx.x] = t;
     }
   }
-  if (w && dw_part) {
+  if (W) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
 #pragma unroll
@@ -588,7 +581,7 @@ static int rmsnorm_fwd_impl(const void* x, const void* res, const void* w, void*
   if (res && !s_out) return TFB_ERR_ARG;
   if (!norm_shape_ok(nrows, C) || nrows_out < nrows) return TFB_ERR_SHAPE;
   const long rpb = norm_rows_per_block(C), nb = (nrows_out + rpb - 1) / rpb;
-  int grid = (int)(nb < 8192 ? nb : 8192);
+  const int grid = (int)std::min(nb, ROW_GRID);
 #define CALL(N, G)                                                                                                    \
   hipLaunchKernelGGL((rmsnorm_fwd_kernel<N, G>), dim3(grid), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)x,     \
                      (const bf16_t*)res, (const bf16_t*)w, (bf16_t*)s_out, (bf16_t*)y, (float*)inv, nrows, C, eps,    \
@@ -618,19 +611,23 @@ static int rmsnorm_bwd_impl(const void* gy, const void* gs, const void* s, const
   if (!gy || !s || !inv || !dx) return TFB_ERR_ARG;
   if (w && !dw_part) return TFB_ERR_ARG;
   if (!norm_shape_ok(nrows, C)) return TFB_ERR_SHAPE;
-  // (the grid is tfb_norm_bwd_blocks(nrows) whatever the rows per workgroup: every partial row of dw_part / amax_part is
-  // written, by a workgroup without rows as zeros)
-  int grid = grid_for(nrows, 1024);
-#define CALL(N, G)                                                                                                     \
-  hipLaunchKernelGGL((rmsnorm_bwd_kernel<N, G>), dim3(grid), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)gy,     \
-                     (const bf16_t*)gs, (const bf16_t*)s, (const bf16_t*)w, (const float*)inv, (bf16_t*)dx,            \
+  // (with partials the grid is tfb_norm_bwd_blocks(nrows) whatever the rows per workgroup: every partial row of dw_part /
+  // amax_part is written, by a workgroup without rows as zeros; without any, a turn for each row)
+  const int parts = grid_for(nrows, 1024);
+  const long rpb = norm_rows_per_block(C);
+  const int grid = w || amax_part ? parts : (int)std::min((nrows + rpb - 1) / rpb, ROW_GRID);
+#define LAUNCH(N, G, W)                                                                                                 \
+  hipLaunchKernelGGL((rmsnorm_bwd_kernel<N, G, W>), dim3(grid), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)gy,   \
+                     (const bf16_t*)gs, (const bf16_t*)s, (const bf16_t*)w, (const float*)inv, (bf16_t*)dx,             \
                      (float*)dw_part, (float*)amax_part, nrows, C)
+#define CALL(N, G) do { if (w) LAUNCH(N, G, true); else LAUNCH(N, G, false); } while (0)
   DISPATCH_ROWS(C, CALL);
 #undef CALL
+#undef LAUNCH
   TFB_LAUNCH_CHECK();
   if (w && dw) {
     hipLaunchKernelGGL(colsum_kernel, dim3((C + 63) / 64), dim3(64, 16), 0, (hipStream_t)stream, (const float*)dw_part,
-                       (float*)dw, grid, C, dw_accumulate, 0L, 0L);
+                       (float*)dw, parts, C, dw_accumulate, 0L, 0L);
     TFB_LAUNCH_CHECK();
   }
   return TFB_OK;
