@@ -33,6 +33,44 @@ struct Ws8Args {
   int tq, more;   // token tiles per XCD; the first `more` XCDs have one more
   int per_wg;     // steps per workgroup (a step = one token tile under one panel; an XCD's steps in panel-major order)
   FastDiv d_tq, d_tq1;       // by tq, by tq + 1
+  const int* row_group;      // kRows: the group of each 128 rows of Q (-1: nobody's), whose weights lie p_group_stride bytes apart
+  long p_group_stride;
+  int row_tiles;             // entries of row_group
+};
+// kRows. An XCD's tiles are a range of row_group's entries; the ranges have about the same cost, a tile of 128 rows counting WS8_TILE and a
+// group's first one WS8_START more (the weights of another group are other registers to load: with eight experts of which six have three tiles
+// each, all of them in the last XCD's eighth, 32768 x 2816 x 1024 182 / 188 us up / dH with equal numbers of tiles, 151 / 161 so; 6 and 9 for
+// WS8_START 158 / 170 and 161 / 171). Only the device knows the groups' loads: every wavefront reads the table for itself.
+constexpr int WS8_TILE = 2, WS8_START = 4, WS8_CHUNKS = 13;   // WS8_CHUNKS: of 64 entries
+constexpr long WS8_ROWS_MAX = 128L * 800;   // of 800 entries an XCD's range has 244 at most; a wavefront keeps 256
+struct Ws8Range {
+  int first, count;
+  __device__ __forceinline__ void init(const int* group, int tiles, int x, int lane) {
+    int g[WS8_CHUNKS];
+#pragma unroll
+    for (int c = 0; c < WS8_CHUNKS; ++c) g[c] = 64 * c + lane < tiles ? group[64 * c + lane] : -1;
+    int cost[WS8_CHUNKS], total = 0, end = 0, before = -1;   // cost: of the entries in front of this lane's
+    const unsigned long long lower = lane ? ~0ull >> (64 - lane) : 0;
+#pragma unroll
+    for (int c = 0; c < WS8_CHUNKS; ++c) {
+      const int up = __shfl_up(g[c], 1, 64), gp = lane ? up : before;
+      const unsigned long long live = __ballot(g[c] >= 0), start = __ballot(g[c] >= 0 && (g[c] != gp || 64 * c + lane == 0));
+      cost[c] = total + WS8_TILE * __builtin_popcountll(live & lower) + WS8_START * __builtin_popcountll(start & lower);
+      total += WS8_TILE * __builtin_popcountll(live) + WS8_START * __builtin_popcountll(start);
+      if (live) end = 64 * c + 64 - __builtin_clzll(live);
+      before = __builtin_amdgcn_readlane(g[c], 63);
+    }
+    int b[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int share = (total * (x + e) + 7) >> 3;
+      b[e] = 0;
+#pragma unroll
+      for (int c = 0; c < WS8_CHUNKS; ++c) b[e] += __builtin_popcountll(__ballot(64 * c + lane < end && cost[c] < share));
+    }
+    first = b[0];
+    count = b[1] - b[0];
+  }
 };
 
 #ifndef TFB_WS8
@@ -75,16 +113,39 @@ __global__ __launch_bounds__(512, 2) void gemm_ws8_kernel(Ws8Args a, Epi epi_in)
   const int lr = lane & 31, lh = lane >> 5;
 
   const int x = blockIdx.x & 7, wi = blockIdx.x >> 3;
-  const int s0 = wi * a.per_wg, tq = a.tq + (x < a.more ? 1 : 0), tile0 = x * a.tq + (x < a.more ? x : a.more);
+  constexpr bool kRows = has_rows<Epi>::value;
+  [[maybe_unused]] Ws8Range range = {};
+  if constexpr (kRows) range.init(a.row_group, a.row_tiles, x, lane);
+  constexpr int PER = 128 / TT;
+  const int tq = kRows ? PER * range.count : a.tq + (x < a.more ? 1 : 0);
+  const int tile0 = kRows ? PER * range.first : x * a.tq + (x < a.more ? x : a.more);
+  const int per_wg = kRows ? (a.panels * tq + (gridDim.x >> 3) - 1) / (int)(gridDim.x >> 3) : a.per_wg;
+  const int s0 = wi * per_wg;
   int T = a.panels * tq - s0;
-  if (T > a.per_wg) T = a.per_wg;
+  if (T > per_wg) T = per_wg;
   if (T <= 0) return;  // (whole workgroup, before any barrier)
-  const Epi epi = epi_prepare(epi_in);
+  [[maybe_unused]] int rg[4];   // the groups of this XCD's tiles: entry i in lane i & 63 of rg[i >> 6]
+  [[maybe_unused]] float inv_tq = 0.f;
+  if constexpr (kRows) {
+    inv_tq = 1.0f / (float)tq;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rg[i] = 64 * i + lane < range.count ? a.row_group[range.first + 64 * i + lane] : -1;
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(rg[0]), "+v"(rg[1]), "+v"(rg[2]), "+v"(rg[3]));
+  }
+  auto group_at = [&](long q0) {
+    const int i = (int)(q0 >> 7) - range.first, l = i & 63;
+    const int v[4] = {__builtin_amdgcn_readlane(rg[0], l), __builtin_amdgcn_readlane(rg[1], l), __builtin_amdgcn_readlane(rg[2], l),
+                      __builtin_amdgcn_readlane(rg[3], l)};
+    return i < 128 ? (i < 64 ? v[0] : v[1]) : (i < 192 ? v[2] : v[3]);
+  };
+  int epi_group = -1;
+  Epi epi = kRows ? epi_in : epi_prepare(epi_in);
 
   // step -> panel, first token
   auto where = [&](int t, int& panel, long& q0) {
     const int s = s0 + t;
-    panel = x < a.more ? fastdiv(s, a.d_tq1) : fastdiv(s, a.d_tq);
+    if constexpr (kRows) panel = __builtin_amdgcn_readfirstlane((int)(((float)s + 0.5f) * inv_tq));   // (exact: s < 2^21, which the host sees to)
+    else panel = x < a.more ? fastdiv(s, a.d_tq1) : fastdiv(s, a.d_tq);
     q0 = (long)TT * (tile0 + (s - panel * tq));
   };
 
@@ -109,9 +170,9 @@ __global__ __launch_bounds__(512, 2) void gemm_ws8_kernel(Ws8Args a, Epi epi_in)
   // (loaded and waited for in inline assembly: behind compiler-visible loads the first MFMA of EVERY tile would wait for
   // all vector-memory operations in flight, the next tile's among them, because a run may have crossed a panel border)
   i32x4 Alo[KS], Ahi[KS];
-  int cur_panel = -1;
-  auto load_panel = [&](int panel) __attribute__((always_inline)) {
-    const uint8_t* g = a.P.base + ((long)panel * 256 + 32 * wave + lr) * a.P.ld + 32 * lh;
+  int cur_panel = -1, cur_group = 0;
+  auto load_panel = [&](int panel, int group) __attribute__((always_inline)) {
+    const uint8_t* g = a.P.base + (kRows ? group * a.p_group_stride : 0) + ((long)panel * 256 + 32 * wave + lr) * a.P.ld + 32 * lh;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(Alo[ks]) : "v"(g + 64 * ks));
@@ -123,6 +184,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ws8_kernel(Ws8Args a, Epi epi_in)
                    : "+v"(Alo[ks]), "+v"(Ahi[ks]), "+v"(Alo[ks + 1]), "+v"(Ahi[ks + 1]), "+v"(Alo[ks + 2]), "+v"(Ahi[ks + 2]),
                      "+v"(Alo[ks + 3]), "+v"(Ahi[ks + 3]));
     cur_panel = panel;
+    cur_group = group;
   };
 
   // ---- B fragment addresses in stage 0: token row lr (+ 32 j as an immediate), k-step 2 kt + u: chunks 4 u + 2 lh + e
@@ -157,7 +219,9 @@ __global__ __launch_bounds__(512, 2) void gemm_ws8_kernel(Ws8Args a, Epi epi_in)
       for (int k = 0; k < NP; ++k) pre[k] = epi.prefetch(p, (int)q0 + ql + 8 * k);
     }
     if constexpr (NS > 2) dma(t + NS - 1);
-    if (panel != cur_panel) load_panel(panel);
+    // (a tile that nobody has is multiplied with the weights at hand, and not finished)
+    const int group = kRows ? group_at(q0) : 0;
+    if ((panel != cur_panel || group != cur_group) && group >= 0) load_panel(panel, group);
     const uint32_t so = (t & (NS - 1)) * STAGE;
     f32x16 acc[NA];
 #pragma unroll
@@ -210,6 +274,14 @@ __global__ __launch_bounds__(512, 2) void gemm_ws8_kernel(Ws8Args a, Epi epi_in)
     int panel;
     long q0;
     where(t, panel, q0);
+    if constexpr (kRows) {
+      const int group = group_at(q0);
+      if (group < 0) return;
+      if (group != epi_group) {
+        epi = epi_prepare(epi_in.for_group(group));
+        epi_group = group;
+      }
+    }
     const int p = panel * 256 + 64 * (wave >> 1) + 8 * (lane & 7);
     const int ql = (TT / 2) * (wave & 1) + (lane >> 3);
     [[maybe_unused]] long off = 0, down = 0;
@@ -242,7 +314,7 @@ __global__ __launch_bounds__(512, 2) void gemm_ws8_kernel(Ws8Args a, Epi epi_in)
     int panel;
     long q0;
     where(0, panel, q0);
-    load_panel(panel);
+    load_panel(panel, kRows ? max(group_at(q0), 0) : 0);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   TFB_SBAR();
@@ -296,15 +368,30 @@ static inline bool gemm_ws8_applies(long np, long nq, long kbytes) {
          (np / 256) * (nq / 64) >= 8L * tfb_resident_slots(1);
 }
 
+// ... over the rows of groups: twice as many steps, for a run also loads the weights of each of its groups (us, this kernel against the tiled one,
+// up-projection / dH of eight experts with the same load, then with two that have nearly all: 1024 x 2816, 12288 rows 60 / 66 against 69 / 69 and
+// 72 / 77 against 65 / 75; 24576 rows 111 / 119 against 132 / 134 and 122 / 126 against 122 / 128; 768 x 3072, 11264 rows 47 / 55 against
+// 46 / 59 and 52 / 61 against 46 / 59; 32768 rows 103 / 119 against 155 / 152 and 120 / 121 against 156 / 155; 1024 x 4096, 32768 rows 173 / 180
+// against 274 / 273; sixteen experts, 1024 x 2816, 32768 rows 138 / 149 against 167 / 172).
+static inline bool gemm_ws8_rows_applies(long np, long nq, long kbytes) {
+  return gemm_ws8_applies(np, nq, kbytes) && nq <= WS8_ROWS_MAX && (np / 256) * (nq / 64) >= 16L * tfb_resident_slots(1) &&
+         (np / 256) * (nq / 32) < (1L << 21);
+}
+
 // K1024: also contractions of 1024 bytes.
 template <int FMTP, int FMTQ, bool K1024, class Epi>
-static int gemm_ws8_launch(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Epi epi, hipStream_t stream) {
+static int gemm_ws8_launch(GemmOperand P, GemmOperand Q, int np, int nq, long kbytes, Epi epi, hipStream_t stream,
+                           const int* row_group = nullptr, long p_group_stride = 0) {
+  if (has_rows<Epi>::value && (!row_group || !gemm_ws8_rows_applies(np, nq, kbytes) || (p_group_stride & 15))) return TFB_ERR_SHAPE;
   if ((kbytes != 768 && (!K1024 || kbytes != 1024)) || np <= 0 || nq <= 0 || np % 256 || nq % 128) return TFB_ERR_SHAPE;
   if (P.ld <= 0 || Q.ld <= 0 || P.ld > (1L << 24) || Q.ld > (1L << 24)) return TFB_ERR_SHAPE;
   if (((uintptr_t)P.base | (uintptr_t)Q.base | (uintptr_t)P.ld | (uintptr_t)Q.ld) & 15) return TFB_ERR_ARG;
   Ws8Args a = {};
   a.P = P;
   a.Q = Q;
+  a.row_group = row_group;
+  a.p_group_stride = p_group_stride;
+  a.row_tiles = nq / 128;
   const int tiles = nq / (kbytes == 768 ? 64 : 32);
   a.panels = np / 256;
   a.tq = tiles / 8;
@@ -314,7 +401,7 @@ static int gemm_ws8_launch(GemmOperand P, GemmOperand Q, int np, int nq, long kb
   int per_x = tfb_resident_slots(1) / 8;  // workgroups per XCD: one per CU
   if (per_x < 1) per_x = 1;
   a.per_wg = (steps_x + per_x - 1) / per_x;
-  const int wgs_x = (steps_x + a.per_wg - 1) / a.per_wg;
+  const int wgs_x = has_rows<Epi>::value ? per_x : (steps_x + a.per_wg - 1) / a.per_wg;
   a.d_tq = fastdiv_make(a.tq > 0 ? a.tq : 1);
   a.d_tq1 = fastdiv_make(a.tq + 1);
   auto go = [&](auto nk) {

@@ -436,10 +436,11 @@ struct EpiUp {  // pre = x8 @ wf8^T: r, h8
     e.sc = sc + g * NSC;
     return e;
   }
-  __device__ __forceinline__ EpiUp prepare() const {
+  __device__ __forceinline__ EpiUp prepare() const { return with(sc[SC_DQ_FC], sc[SC_C_H]); }
+  __device__ __forceinline__ EpiUp with(float dq_fc, float c_h) const {
     EpiUp e = *this;
-    e.dq = sc[SC_DQ_FC];
-    e.c = sc[SC_C_H];
+    e.dq = dq_fc;
+    e.c = c_h;
     e.fast = is_pow2(e.c);
     e.inv_c2 = 1.0f / (e.c * e.c);
     e.lim = H_CLAMP * H_CLAMP * e.inv_c2;
@@ -516,7 +517,13 @@ struct EpiScaleStore {  // out = bf16(acc * sc[col])
 // out = bf16(res + bf16(acc * dq)): EpiScaleStore / EpiDescale with the residual add that follows the projection made in
 // the same store (the reference's projection-with-residual forward, K/nki_attn_nr8.py:1003, and the residual half of
 // K/nki_mlp_nr8.py:1032); dq = sc[col] when sc is given, else dq_imm * *dq_a * *dq_b. Two roundings, as the separate add.
-struct EpiScaleRows : EpiScaleStore {  // for the persistent kernel over the rows of groups
+// for the persistent kernels over the rows of groups
+struct EpiUpRows : EpiUp {
+  static constexpr bool kRows = true;
+  __device__ __forceinline__ EpiUpRows for_group(int g) const { return EpiUpRows{EpiUp::for_group(g)}; }
+  __device__ __forceinline__ EpiUpRows prepare() const { return EpiUpRows{with(tfb_scalar_load(sc + SC_DQ_FC), tfb_scalar_load(sc + SC_C_H))}; }
+};
+struct EpiScaleRows : EpiScaleStore {
   static constexpr bool kRows = true;
   __device__ __forceinline__ EpiScaleRows for_group(int g) const { return EpiScaleRows{EpiScaleStore::for_group(g)}; }
   __device__ __forceinline__ EpiScaleRows prepare() const {
@@ -623,11 +630,12 @@ struct EpiDh {  // dh = dy8 @ wp8: dpre = bf16((acc*dq_dh2)*r), dp8 = e5m2(dpre*
     e.sc = sc + g * NSC;
     return e;
   }
-  __device__ __forceinline__ EpiDh prepare() const {
+  __device__ __forceinline__ EpiDh prepare() const { return with(sc[SC_DQ_DH2], sc[SC_S_DP], sc[SC_S_H]); }
+  __device__ __forceinline__ EpiDh with(float dq_dh2, float s_dp, float s_h) const {
     EpiDh e = *this;
-    e.dq = sc[SC_DQ_DH2];
-    e.sdp = sc[SC_S_DP];
-    e.sh = sc[SC_S_H];
+    e.dq = dq_dh2;
+    e.sdp = s_dp;
+    e.sh = s_h;
 #ifndef TFB_DH_FASTCAST
 #define TFB_DH_FASTCAST 1
 #endif
@@ -713,6 +721,14 @@ struct EpiDh {  // dh = dy8 @ wp8: dpre = bf16((acc*dq_dh2)*r), dp8 = e5m2(dpre*
         *(u32x2*)(hq8 + off) = q;
       }
     }
+  }
+};
+
+struct EpiDhRows : EpiDh {
+  static constexpr bool kRows = true;
+  __device__ __forceinline__ EpiDhRows for_group(int g) const { return EpiDhRows{EpiDh::for_group(g)}; }
+  __device__ __forceinline__ EpiDhRows prepare() const {
+    return EpiDhRows{with(tfb_scalar_load(sc + SC_DQ_DH2), tfb_scalar_load(sc + SC_S_DP), tfb_scalar_load(sc + SC_S_H))};
   }
 };
 
@@ -1218,6 +1234,11 @@ int grouped_launch(const uint8_t* wbase, long wld, long wgroup_stride, const uin
       const int st = gemm_pp_launch_rows<Cfg::FMTP, Cfg::FMTQ>(a.P, wgroup_stride, a.Q, np, rmax, kbytes, tile_expert, EpiScaleRows{e}, s);
       return st != TFB_OK ? st : gemm_ring_rest<Cfg::FMTP, Cfg::FMTQ>(a, e, s);
     }
+  }
+  if constexpr (std::is_same<Epi, EpiUp>::value || std::is_same<Epi, EpiDh>::value) {
+    using Rows = std::conditional_t<std::is_same<Epi, EpiUp>::value, EpiUpRows, EpiDhRows>;
+    if (gemm_ws8_rows_applies(np, rmax, kbytes))
+      return gemm_ws8_launch<Cfg::FMTP, Cfg::FMTQ, true>(a.P, a.Q, np, (int)rmax, kbytes, Rows{e}, s, tile_expert, wgroup_stride);
   }
   if (const int pick = gemm_ring_pick(np, rmax, a.nkt, false))
     return gemm_ring_launch<Epi, Cfg::ES, Cfg::LAYP, Cfg::LAYQ, Cfg::FMTP, Cfg::FMTQ>(pick, a, 1, 1, e, s);
