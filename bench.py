@@ -90,7 +90,7 @@ def _work(name, a):
     if name == "tfb_attn_fwd":
         B, H, T, D = a[-6:-2]
         return "attention forward", "mfma", 2.0 * B * H * T * T * D
-    if name == "tfb_qkv_rope_fwd":           # x, w, cos, sin, out, M, N, K, T, rot, stream
+    if name in ("tfb_qkv_rope_fwd", "tfb_qkv_rope_heads_fwd"):   # x, w, cos, sin, out, M, N, K, T, rot, [D,] stream
         M, N, K = a[5:8]
         return "QKV projection + RoPE %dx%dx%d" % (M, N, K), "mfma", 2.0 * M * N * K
     if name in ("tfb_gemm_bf16", "tfb_gemm_bf16_scaled"):   # A, B, C, M, N, K, ta, tb, ...
