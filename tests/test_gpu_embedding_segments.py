@@ -25,3 +25,8 @@ def test_segments(n, C, V):
     most = int(torch.bincount(idx[ok]).max()) if bool(ok.any()) else 1
     bound = dw.double().abs().index_add_(0, idx[ok], dy[ok].double().abs()) * (most + 1) * 2.0 ** -24
     assert bool(((got.cpu().double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("n", [32767, 32768])   # (rows of 512 columns: segments of 32, then of 64)
+def test_segments_of_narrower_rows(n):
+    test_segments(n, 512, 500)

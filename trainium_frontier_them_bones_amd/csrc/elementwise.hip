@@ -418,64 +418,70 @@ __global__ __launch_bounds__(256) void emb_scatter_kernel(const IDX* __restrict_
 // equal tokens that lies inside the segment has a single owner and is added with plain loads/stores; the first and the
 // last run may continue in the neighbouring segments and use atomics.
 // What bounds it: with few rows latency, a trip to memory for every row and every sum it is added to (those of eight positions are asked for
-// together), so short segments; with many the atomics of the frequent tokens' runs on one row, one for each segment, so long ones. The whole call,
-// Zipf tokens, V 32768, C 768, us, segments of 8 / 16 / 32 / 64: 512 rows 22.5 / 25.3 / 32 / 44, 1152 26.3 / 25.7 / 32.3 / 44, 2048 30.0 / 27.1 / 32.4 / 44.5,
-// 4096 42 / 32.9 / 32.5 / 44, 16384 111 / 68 / 52 / 54, 32768 204 / 117 / 78.5 / 69 (C 512 at 32768: 181 / 103 / 67.5 / 58.5).
+// together), so short segments; with many the atomics of the frequent tokens' runs on one row, one for each segment, so long ones; where tokens
+// seldom repeat, and rows are narrow, the workgroups in flight, so not the longest. The whole call, us, segments of 8 / 16 / 32 / 64, Zipf tokens and
+// uniform ones, V 32768:
+//   C 768  512 rows 21.9 / 23.3 / 27.0 / 35.7, 21.3 / 23.5 / 27.8 / 36.4; 2048 29.7 / 26.6 / 28.7 / 36.4, 23.0 / 25.3 / 30.6 / 39.4; 4096 41 / 31.4 / 30.3 / 39.3,
+//          26.8 / 28.7 / 35.4 / 48.7; 16384 109 / 69 / 53.2 / 56.8, 52 / 42.5 / 40.6 / 49.8; 24576 154 / 93 / 65.8 / 63.1, 75 / 55.5 / 48.1 / 53.0; 32768 203 /
+//          117 / 80.4 / 70.0, 100 / 67 / 57.7 / 56.4
+//   C 256  16384 87 / 57.6 / 44.6 / 45.6, 34.8 / 31.0 / 35.6 / 49.0; 32768 158 / 95 / 67.8 / 65.5, 50.9 / 40.4 / 39.9 / 48.9; 49152 223 / 130 / 86.8 / 74.3, 73.5 / 51.1 /
+//          46.5 / 50.4
 constexpr int EMB_AHEAD = 8;
 template <typename IDX, int SEG>
 __global__ __launch_bounds__(128) void emb_reduce_kernel(const IDX* __restrict__ idx, const int* __restrict__ order,
                                                         const bf16_t* __restrict__ dy, float* __restrict__ dw, long n, int C,
                                                         int V) {
-  __shared__ int rows[SEG];
-  __shared__ int toks[SEG + 1];
-  __shared__ int edge[2];  // the tokens of the rows just before and just after this segment (-1: none)
+  // of every position: its row, its token, and how a run that ends there is added: 0 none ends, 1 alone, 2 with the neighbours', 3 not at all (the
+  // bucket of out-of-range ids). The first wavefront finds them for all, so that a position costs one LDS read and no waits in turn.
+  static_assert(SEG <= 64 && SEG % EMB_AHEAD == 0, "a lane for each position");
+  __shared__ int4 at[SEG];
   const long pos0 = (long)blockIdx.x * SEG;
   const int cnt = (int)min((long)SEG, n - pos0);
-  if (threadIdx.x < cnt) {
-    const int r = order[pos0 + threadIdx.x];
-    rows[threadIdx.x] = r;
-    toks[threadIdx.x] = emb_bucket(idx[r], V);
-  } else if (threadIdx.x == SEG) {
-    edge[0] = pos0 > 0 ? emb_bucket(idx[order[pos0 - 1]], V) : -1;
-  } else if (threadIdx.x == SEG + 1) {
-    edge[1] = pos0 + cnt < n ? emb_bucket(idx[order[pos0 + cnt]], V) : -1;
+  if (threadIdx.x < 64) {
+    const int i = threadIdx.x;
+    const int row = i < cnt ? order[pos0 + i] : -1, before = pos0 > 0 ? order[pos0 - 1] : -1, after = pos0 + cnt < n ? order[pos0 + cnt] : -1;
+    const int tok = row >= 0 ? emb_bucket(idx[row], V) : -1, tok_before = before >= 0 ? emb_bucket(idx[before], V) : -1,
+              tok_after = after >= 0 ? emb_bucket(idx[after], V) : -1;
+    const int next = __shfl_down(tok, 1, 64), first = __builtin_amdgcn_readfirstlane(tok);
+    int how = 0;
+    if (i < cnt && (i + 1 == cnt || next != tok))
+      how = tok == V ? 3 : (tok == first && tok_before == tok) || (i + 1 == cnt && tok_after == tok) ? 2 : 1;
+    if (i < SEG) at[i] = int4{row, tok, how, 0};
   }
   __syncthreads();
   const int c = (blockIdx.y * 128 + threadIdx.x) * 8;
   if (c >= C) return;
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  const int first_tok = toks[0];
-  // how a run that ends at position i is added: 0 none ends there (or the bucket of out-of-range ids, dropped), 1 alone, 2 with the neighbours'
-  auto ends = [&](int i) {
-    if (i >= cnt || (i + 1 < cnt && toks[i + 1] == toks[i]) || toks[i] == V) return 0;
-    return (toks[i] == first_tok && edge[0] == toks[i]) || (i + 1 == cnt && edge[1] == toks[i]) ? 2 : 1;
-  };
   for (int i0 = 0; i0 < cnt; i0 += EMB_AHEAD) {
     u32x4 u[EMB_AHEAD];
     f32x4 a0[EMB_AHEAD], a1[EMB_AHEAD];
-    int how[EMB_AHEAD];
+    int tok[EMB_AHEAD], how[EMB_AHEAD], row[EMB_AHEAD];
 #pragma unroll
     for (int x = 0; x < EMB_AHEAD; ++x) {
-      const int i = i0 + x;
-      how[x] = ends(i);
-      if (i < cnt) u[x] = *(const u32x4*)(dy + (long)rows[i] * C + c);
+      const int4 e = at[i0 + x];
+      row[x] = __builtin_amdgcn_readfirstlane(e.x);
+      tok[x] = __builtin_amdgcn_readfirstlane(e.y);
+      how[x] = __builtin_amdgcn_readfirstlane(e.z);
+    }
+#pragma unroll
+    for (int x = 0; x < EMB_AHEAD; ++x) {
+      if (row[x] >= 0) u[x] = *(const u32x4*)(dy + (long)row[x] * C + c);
       if (how[x] == 1) {
-        const float* d = dw + (long)toks[i] * C + c;
+        const float* d = dw + (long)tok[x] * C + c;
         a0[x] = *(const f32x4*)d;
         a1[x] = *(const f32x4*)(d + 4);
       }
     }
 #pragma unroll
     for (int x = 0; x < EMB_AHEAD; ++x) {
-      const int i = i0 + x;
-      if (i >= cnt) break;
+      if (row[x] < 0) break;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         acc[2 * k] += bflo(u[x][k]);
         acc[2 * k + 1] += bfhi(u[x][k]);
       }
-      if (i + 1 == cnt || toks[i + 1] != toks[i]) {
-        float* d = dw + (long)toks[i] * C + c;
+      if (how[x]) {
+        float* d = dw + (long)tok[x] * C + c;
         if (how[x] == 2) {
           // the token's run goes on in a neighbouring segment: another workgroup adds to the same row
 #pragma unroll
@@ -715,7 +721,7 @@ extern "C" int tfb_embedding_bwd_grouped(const void* idx, int idx64, const void*
   };
   if (n <= 512) reduce(std::integral_constant<int, 8>{});
   else if (n <= 2048) reduce(std::integral_constant<int, 16>{});
-  else if (n < 24576) reduce(std::integral_constant<int, 32>{});
+  else if (n < 24576 || n * C < (16L << 20)) reduce(std::integral_constant<int, 32>{});
   else reduce(std::integral_constant<int, 64>{});
   TFB_LAUNCH_CHECK();
   return TFB_OK;
