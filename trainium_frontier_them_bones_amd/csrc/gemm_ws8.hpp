@@ -40,7 +40,8 @@ struct Ws8Args {
 // kRows. An XCD's tiles are a range of row_group's entries; the ranges have about the same cost, a tile of 128 rows counting WS8_TILE and a
 // group's first one WS8_START more (the weights of another group are other registers to load: with eight experts of which six have three tiles
 // each, all of them in the last XCD's eighth, 32768 x 2816 x 1024 182 / 188 us up / dH with equal numbers of tiles, 151 / 161 so; 6 and 9 for
-// WS8_START 158 / 170 and 161 / 171). Only the device knows the groups' loads: every wavefront reads the table for itself.
+// WS8_START 158 / 170 and 161 / 171). A tile that nobody has, in front of the last one that somebody has, counts like another: it takes as many
+// steps, and no range is then longer than a wavefront keeps. Only the device knows the groups' loads: every wavefront reads the table for itself.
 constexpr int WS8_TILE = 2, WS8_START = 4, WS8_CHUNKS = 13;   // WS8_CHUNKS: of 64 entries
 constexpr long WS8_ROWS_MAX = 128L * 800;   // of 800 entries an XCD's range has 244 at most; a wavefront keeps 256
 struct Ws8Range {
@@ -49,17 +50,23 @@ struct Ws8Range {
     int g[WS8_CHUNKS];
 #pragma unroll
     for (int c = 0; c < WS8_CHUNKS; ++c) g[c] = 64 * c + lane < tiles ? group[64 * c + lane] : -1;
-    int cost[WS8_CHUNKS], total = 0, end = 0, before = -1;   // cost: of the entries in front of this lane's
+    int end = 0;   // behind the last tile that somebody has
+#pragma unroll
+    for (int c = 0; c < WS8_CHUNKS; ++c) {
+      const unsigned long long live = __ballot(g[c] >= 0);
+      if (live) end = 64 * c + 64 - __builtin_clzll(live);
+    }
+    int cost[WS8_CHUNKS], starts = 0, before = -1;   // cost: of the entries in front of this lane's
     const unsigned long long lower = lane ? ~0ull >> (64 - lane) : 0;
 #pragma unroll
     for (int c = 0; c < WS8_CHUNKS; ++c) {
       const int up = __shfl_up(g[c], 1, 64), gp = lane ? up : before;
-      const unsigned long long live = __ballot(g[c] >= 0), start = __ballot(g[c] >= 0 && (g[c] != gp || 64 * c + lane == 0));
-      cost[c] = total + WS8_TILE * __builtin_popcountll(live & lower) + WS8_START * __builtin_popcountll(start & lower);
-      total += WS8_TILE * __builtin_popcountll(live) + WS8_START * __builtin_popcountll(start);
-      if (live) end = 64 * c + 64 - __builtin_clzll(live);
+      const unsigned long long start = __ballot(g[c] >= 0 && (g[c] != gp || 64 * c + lane == 0));
+      cost[c] = WS8_TILE * (64 * c + lane) + WS8_START * (starts + __builtin_popcountll(start & lower));
+      starts += __builtin_popcountll(start);
       before = __builtin_amdgcn_readlane(g[c], 63);
     }
+    const int total = WS8_TILE * end + WS8_START * starts;
     int b[2];
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
