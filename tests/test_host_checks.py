@@ -206,3 +206,18 @@ def test_wrappers_for_sequences_take_three_dimensions(A):
         _passes(lambda: fn(_t(2, 128, 256)))
         _refused(lambda: fn(_t(256, 256)))
         _refused(lambda: fn(_t(2, 2, 64, 256)))
+
+
+def test_newton_schulz_stacks(A):
+    from trainium_frontier_them_bones_amd import ops
+    g, w = _t(2, 256, 128, dtype=f32), _t(3, 128, 256, dtype=f32)
+    d, dw = _t(2, dtype=f32), _t(3, dtype=bf16)
+    _passes(lambda: ops.ns5_stacks([(g, d)]))
+    _passes(lambda: ops.ns5_stacks([(g, d), (w, dw)]))
+    _refused(lambda: ops.ns5_stacks([]))
+    _refused(lambda: ops.ns5_stacks([(g, d), (w, dw), (g, d)]))          # (the kernels take two)
+    _refused(lambda: ops.ns5_stacks([(g, d), (_t(3, 128, 128, dtype=f32), dw)]))
+    _refused(lambda: ops.ns5_stacks([(g, dw)]))
+    far = torch.empty(3, 128, 256, dtype=f32, device="cuda:1")
+    _refused(lambda: ops.ns5_stacks([(g, d), (far, dw)]))
+    _refused(lambda: ops.ns5_stacks([(g, torch.empty(2, dtype=f32, device="cuda:1"))]))

@@ -592,7 +592,10 @@ def ns5_stacks(stacks, coeffs=NS_COEFFS):
     (tall r >= c, or wide: handled as the transposes) from X0 = bf16(bf16(g) / d), d [K] (any float dtype; the reciprocal is taken in
     fp32 as the reference's sc_tile does). Returns [(y bf16 [K, r, c], v fp32 [K, max(r, c)] = the sums of y^2 along the short side), ..]."""
     import ctypes
+    if not 1 <= len(stacks) <= 2:
+        raise ValueError("one or two stacks")
     M, N = max(stacks[0][0].shape[1:]), min(stacks[0][0].shape[1:])
+    dev = stacks[0][0].device
     args, out, types = [], [], {d.dtype for _, d in stacks}
     d_type = _NS_D_TYPES.get(types.pop() if len(types) == 1 else None, 0)
     for g, d in stacks:
@@ -605,13 +608,15 @@ def ns5_stacks(stacks, coeffs=NS_COEFFS):
             raise ValueError("one denominator per matrix")
         if not d.is_cuda:
             raise RuntimeError("tfb ops need device tensors (the HIP kernels are the only implementation)")
+        if g.device != dev or d.device != dev:
+            raise ValueError("stacks and denominators on one device")
         d = d if d_type else d.float()
         out.append((torch.empty(K, r, c, dtype=bf16, device=g.device), torch.empty(K, M, dtype=torch.float32, device=g.device)))
         args.append((g, d, *out[-1], K, int(r < c)))
     K = sum(a[4] for a in args)
     need = _lib.lib().tfb_ns5_workspace_bytes(K, M, N)
-    # one workspace per (device, stream), grown to the largest call seen (never one per shape)
-    dev = stacks[0][0].device
+    # one workspace per (device, stream), grown to the largest call seen (never one per shape) and kept: two stacks hold both stacks' at once,
+    # twice what each alone needs
     key = (dev, torch.cuda.current_stream(dev).cuda_stream)
     ws = _NS_WS.get(key)
     if ws is None or ws.numel() < need:
