@@ -221,3 +221,15 @@ def test_newton_schulz_stacks(A):
     far = torch.empty(3, 128, 256, dtype=f32, device="cuda:1")
     _refused(lambda: ops.ns5_stacks([(g, d), (far, dw)]))
     _refused(lambda: ops.ns5_stacks([(g, torch.empty(2, dtype=f32, device="cuda:1"))]))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_rotation_tables_of_the_projection(A, D):
+    T, x, w = 256, _t(2, 256, 256), _t(3 * 256, 256)
+    tab = lambda *s: (_t(*s), _t(*s))  # noqa: E731
+    call = lambda c, s: (lambda: A.QkvRopeAttentionFn.apply(x, w, c, s, 256 // D, 0.1))  # noqa: E731
+    _passes(call(*tab(T, D // 2)))
+    _passes(call(*tab(2 * T, D // 2)))                    # (of a longer sequence)
+    _refused(call(*tab(T, D // 4)))                       # of heads half as wide: the kernels would read past them
+    _refused(call(*tab(T - 1, D // 2)))
+    _refused(call(_t(T, D // 2), _t(T // 2, D // 2)))

@@ -559,6 +559,7 @@ struct QkvRopeAttention : Function<QkvRopeAttention> {
     const int64_t B = x.size(0), T = x.size(1), C = w.size(0) / 3;
     TORCH_CHECK_VALUE(n_head > 0 && w.size(0) % (3 * n_head) == 0, "qkv is [B, T, 3 heads D]");
     const int64_t D = C / n_head;
+    TORCH_CHECK_VALUE(cos.numel() >= T * (D / 2) && sin.numel() >= T * (D / 2), "cos, sin are [T, D / 2]");
     Tensor qkv;
     if (D == 64 || !any_replaced) {
       qkv = D == 64 ? op::qkv_rope(x, w, cos, sin, T, 2 * C) : qkv_rope(x, w, cos, sin, T, 2 * C, D);
