@@ -116,8 +116,9 @@ class RopeNormAttentionHeadsFn:
 
 class QkvRopeAttentionFn:
     """(x, w_qkv, cos, sin, n_head, scale): the attention block's core in one node: qkv = rope(x @ w_qkv^T) (rotation in the
-    projection's epilogue), causal attention on the thirds, and in backward the inverse rotation inside the attention kernels'
-    stores followed by the projection's dX and dW (accumulated into w_qkv.grad_buf when present). Head dimension 64."""
+    projection's epilogue), causal attention on the thirds, and in backward the inverse rotation (head dimension 64: inside the
+    attention kernels' stores; 128: a launch of its own) followed by the projection's dX and dW (accumulated into w_qkv.grad_buf
+    when present). cos, sin [T, D / 2]."""
     apply = _Node("qkv_rope_attention")
 
 
