@@ -195,11 +195,8 @@ class GPT:
                 att = A.RopeAttentionFn.apply(qkv, self.cos[:T], self.sin[:T], cfg.n_head, scale)
                 att = A.Linear8Fn.apply(att, p["w_o.%d" % i], self.wo_state[i], None)
             else:
-                if cfg.head_dim in (64, 128):   # rotation fused into the projection's epilogue
-                    att = A.QkvRopeAttentionFn.apply(h, p["w_qkv.%d" % i], self.cos[:T], self.sin[:T], cfg.n_head, scale)
-                else:
-                    qkv = A.LinearFn.apply(h, p["w_qkv.%d" % i])
-                    att = A.RopeAttentionFn.apply(qkv, self.cos[:T], self.sin[:T], cfg.n_head, scale)
+                # (rotation fused into the projection's epilogue)
+                att = A.QkvRopeAttentionFn.apply(h, p["w_qkv.%d" % i], self.cos[:T], self.sin[:T], cfg.n_head, scale)
                 att = A.LinearFn.apply(att, p["w_o.%d" % i])
             x, h = A.AddRMSNormFn.apply(x, att, p["norm2.%d" % i], cfg.norm_eps)
             m = A.Mlp8Fn.apply(h, p["w_fc.%d" % i], p["w_proj.%d" % i], self.mlp_state[i])
@@ -227,11 +224,7 @@ class GPT:
                 att = A.RopeAttentionFn.apply(qkv, self.cos[:T], self.sin[:T], cfg.n_head, scale)
                 x = A.Linear8Fn.apply(att, p["w_o.%d" % i], self.wo_state[i], None, None, x)
             else:
-                if cfg.head_dim in (64, 128):
-                    att = A.QkvRopeAttentionFn.apply(h, p["w_qkv.%d" % i], self.cos[:T], self.sin[:T], cfg.n_head, scale)
-                else:
-                    qkv = A.LinearFn.apply(h, p["w_qkv.%d" % i])
-                    att = A.RopeAttentionFn.apply(qkv, self.cos[:T], self.sin[:T], cfg.n_head, scale)
+                att = A.QkvRopeAttentionFn.apply(h, p["w_qkv.%d" % i], self.cos[:T], self.sin[:T], cfg.n_head, scale)
                 x = A.LinearFn.apply(att, p["w_o.%d" % i], x)
             keep(x)
             # (with the weight gradients in fp8 too the MLP reads only the norm's bytes: its bf16 rows are not written)
