@@ -528,23 +528,15 @@ __global__ __launch_bounds__(ADAM_T) void adamw_kernel(float* __restrict__ p, co
   const long n4 = n & ~3L;
   const long step = (long)gridDim.x * ADAM_T * 4;
   long i = ((long)blockIdx.x * ADAM_T + threadIdx.x) * 4;
-  // (beyond ADAM_MAX_BLOCKS groups of a workgroup) the next group's four loads go out before this group's stores: a wait for loaded data also waits for every older
-  // store (one counter orders both), so loading after the stores would cost a store round trip per group
-  f32x4 pp, mm, vv, gg;
-  u32x2 gb;
-  auto fetch = [&](long j) {
-    pp = tfb_load_nt((const f32x4*)(p + j), TFB_NT_D);
-    mm = tfb_load_nt((const f32x4*)(m + j), TFB_NT_D);
-    vv = tfb_load_nt((const f32x4*)(v + j), TFB_NT_D);
-    if (GF32) gg = tfb_load_nt((const f32x4*)((const float*)g + j), TFB_NT_D);
-    else gb = tfb_load_nt((const u32x2*)((const bf16_t*)g + j), TFB_NT_D);
-  };
-  if (i < n4) fetch(i);
-  for (; i < n4; i += step) {
-    f32x4 cp = pp, cm = mm, cv = vv, cg;
-    if (GF32) cg = gg;
-    else cg = f32x4{bflo(gb.x), bfhi(gb.x), bflo(gb.y), bfhi(gb.y)};
-    if (i + step < n4) fetch(i + step);
+  for (; i < n4; i += step) {  // (a second turn beyond 2^32 elements)
+    f32x4 cp = tfb_load_nt((const f32x4*)(p + i), TFB_NT_D), cm = tfb_load_nt((const f32x4*)(m + i), TFB_NT_D),
+          cv = tfb_load_nt((const f32x4*)(v + i), TFB_NT_D), cg;
+    if (GF32) {
+      cg = tfb_load_nt((const f32x4*)((const float*)g + i), TFB_NT_D);
+    } else {
+      const u32x2 gb = tfb_load_nt((const u32x2*)((const bf16_t*)g + i), TFB_NT_D);
+      cg = f32x4{bflo(gb.x), bfhi(gb.x), bflo(gb.y), bfhi(gb.y)};
+    }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       float pk = cp[k], mk = cm[k], vk = cv[k];
