@@ -274,6 +274,7 @@ __global__ __launch_bounds__(256, 2) void attnD_fwd_kernel(AttnT q, AttnT k, Att
       last_tile(even, scA, pA);
       tile_barrier();
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load into LDS is on its way when it is given back (both ways have waited)
 
     const int myq = qw0 + lr;
     const float lt = l + __shfl_xor(l, 32, 64);

@@ -707,7 +707,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   // stores of the cluster before (the first block's in the tile's last iteration) and in front of that cluster's operand loads: reported in issue
   // order, it does not wait for them. Requested in its own cluster behind those loads, every one of a tile's four blocks waited for a trip to
   // HBM (the QKV projection with its rotation, 32768 x 2304 x 768: 148 us, of 113 without; now 120). The requests take the registers as
-  // operands that go in and come out, so that no copy of them is made while a load is on its way.
+  // operands that go in and come out, which leaves no reason for a copy of them while a load is on its way; that none is made, and none of the
+  // registers used, is checked in the built code (tests/test_built_code_waits.py).
   auto iter = [&](auto FIRST, int kt) __attribute__((always_inline)) {
     constexpr bool first = decltype(FIRST)::value, stores = first && !kF32;
     // k positions one and two ahead in the workgroup's stream of k-tiles
@@ -887,6 +888,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     }
   }
   if constexpr (!kF32) {
+    waitB(fb0);  // the stream's last fragments, which nobody multiplies, land before their registers are used again
     // the last tile's accumulators
     auto flush = [&](auto HX, auto HY, auto request_it) __attribute__((always_inline)) {
       if constexpr (kPipe) {

@@ -407,6 +407,13 @@ __device__ __forceinline__ void gemm_ring_tile(GemmArgs a, const Epi& epi_in, in
     step(0, t, std::false_type{});
     if (t + 1 < nkt) step(1, t + 1, std::false_type{});
   }
+  // (nothing is on its way into the fragments' registers here, on no path: the check of the built code follows them all)
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int set = 0; set < 2; ++set) {
+    fp[set].landed();
+    fq[set].landed();
+  }
   if constexpr (RANGES) {
     if (range > 1) {
 #pragma unroll
