@@ -237,7 +237,8 @@ extern "C" int tfb_gemm_bf16_res(const void* A, const void* B, const void* res, 
 // thirds (the first rot_cols columns, heads of D = 64 or 128 elements) applied in the GEMM epilogue; row m is token m % T.
 // cos_t, sin_t: bf16 [T][D / 2]. The output equals tfb_gemm_bf16 followed by tfb_rope bit for bit. us, two launches -> one, D = 128:
 // 512 -> 1536 columns: 1152 rows 9.4 -> 6.8, 4096 18.6 -> 13.8, 12288 36.8 -> 30.9; 1024 -> 3072: 256 8.8 -> 8.2, 1152 17.1 -> 13.5, 6144 55.4 -> 48.5,
-// 9600 76.9 -> 72.9, 16384 113 -> 100 (and 12288 89.4 -> 93.6: the projection alone takes 256 x 192 tiles there, which have no rotation).
+// 9600 76.9 -> 72.9, 16384 113 -> 100. Where the projection alone takes tiles that fill its rounds better, which have no rotation, two launches gain
+// or lose a little (12288 93.3 -> 95.8; 768 -> 2304: 9600 49.2 -> 50.4, 4096 27.2 -> 27.5).
 extern "C" int tfb_qkv_rope_heads_fwd(const void* x, const void* w, const void* cos_t, const void* sin_t, void* out, int M, int N,
                                       int K, int T, int rot_cols, int D, void* stream) {
   if (!x || !w || !cos_t || !sin_t || !out) return TFB_ERR_ARG;

@@ -548,7 +548,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
 
   // ---- epilogue of one accumulator block, acc[hx][i][hy][4 jj + e] = D[pb + 8 jj + 4 lh + e][qb + lr] of MFMA tile i: every
   // accumulator goes through epi.pre() and is rounded to bf16, the block passes through the wavefront's own 4 KB of LDS, and every
-  // lane finishes 8 consecutive outputs of a row: epi.chunk(p, q, v [, partner] [, prefetched]). Two forms:
+  // lane finishes 8 consecutive outputs of a row (with kPartner those and their partners): epi.chunk() or epi.chunk2(). Two forms:
   //   64 p (X = P, two tiles): row q = 128 bytes, 16-byte chunk c at slot c ^ ((q >> 1) & 7) (the 8-byte writes and the 16-byte
   //   reads then use the banks evenly), a row's 64 outputs on 8 consecutive lanes;
   //   32 p: row q = 64 bytes, chunk c at slot c ^ ((q >> 2) & 3), a row's outputs on 4 lanes; X = Q: tile i is rows 32 i .. of q.

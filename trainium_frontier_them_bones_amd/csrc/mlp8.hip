@@ -514,9 +514,6 @@ struct EpiScaleStore {  // out = bf16(acc * sc[col])
   __device__ __forceinline__ void chunk(int p, int q, const u32x4& v) const { *(u32x4*)(out + (long)q * ld + p) = v; }
 };
 
-// out = bf16(res + bf16(acc * dq)): EpiScaleStore / EpiDescale with the residual add that follows the projection made in
-// the same store (the reference's projection-with-residual forward, K/nki_attn_nr8.py:1003, and the residual half of
-// K/nki_mlp_nr8.py:1032); dq = sc[col] when sc is given, else dq_imm * *dq_a * *dq_b. Two roundings, as the separate add.
 // for the persistent kernels over the rows of groups
 struct EpiUpRows : EpiUp {
   static constexpr bool kRows = true;
@@ -533,6 +530,9 @@ struct EpiScaleRows : EpiScaleStore {
   }
 };
 
+// out = bf16(res + bf16(acc * dq)): EpiScaleStore / EpiDescale with the residual add that follows the projection made in
+// the same store (the reference's projection-with-residual forward, K/nki_attn_nr8.py:1003, and the residual half of
+// K/nki_mlp_nr8.py:1032); dq = sc[col] when sc is given, else dq_imm * *dq_a * *dq_b. Two roundings, as the separate add.
 struct EpiDescaleRes {
   const float* sc;
   int col;
