@@ -111,3 +111,21 @@ def test_head_dimensions_that_attention_refuses(dev, fuse):
         m = GPT(GPTConfig(n_layer=1, d_model=256, n_head=heads, d_ff=1024, vocab=1024, seq_len=128, fuse_residual=fuse), dev)
         with pytest.raises(TfbError):
             m.forward(idx, tg)
+
+
+def test_the_timed_entry_point_of_either_head_dimension(dev):
+    """A program that times an entry point by its name gets its calls with the arguments that the header gives it."""
+    from trainium_frontier_them_bones_amd import _lib, autograd as A, ops
+    narrow, wide = [], []
+    x, w, _, tabs = _inputs(dev, 1, 128, 4, 256, D=64)
+    tabs128 = _inputs(dev, 1, 128, 2, 256)[3]
+    _lib.TIMED.update(tfb_qkv_rope_fwd=narrow, tfb_qkv_rope_heads_fwd=wide)
+    try:
+        ops.qkv_rope(x[0], w, *tabs, 128, 512)
+        A.QkvRopeAttentionFn.apply(x, w, *tabs, 4, 0.125)
+        A.QkvRopeAttentionFn.apply(x, w, *tabs128, 2, 0.125)
+    finally:
+        del _lib.TIMED["tfb_qkv_rope_fwd"], _lib.TIMED["tfb_qkv_rope_heads_fwd"]
+    torch.cuda.synchronize()
+    assert [r[-1][5:10] for r in narrow] == [(128, 768, 256, 128, 512)] * 2 and [len(r[-1]) for r in narrow] == [11, 11]
+    assert [r[-1][5:11] for r in wide] == [(128, 768, 256, 128, 512, 128)]

@@ -83,7 +83,10 @@ Tensor qkv_rope(const Tensor& x, const Tensor& w, const Tensor& cos, const Tenso
   chk(x), chk(w), chk(cos), chk(sin);
   const int64_t K = last_dim(x), M = x.numel() / K, N = w.size(0);
   Tensor out = make(with_last(x, N), BF16, x);
-  TFB_CALL(tfb_qkv_rope_heads_fwd, ptr(x), ptr(w), ptr(cos), ptr(sin), ptr(out), M, N, K, T, rot_cols, D, stream());
+  if (D == 64)
+    TFB_CALL(tfb_qkv_rope_fwd, ptr(x), ptr(w), ptr(cos), ptr(sin), ptr(out), M, N, K, T, rot_cols, stream());
+  else
+    TFB_CALL(tfb_qkv_rope_heads_fwd, ptr(x), ptr(w), ptr(cos), ptr(sin), ptr(out), M, N, K, T, rot_cols, D, stream());
   return out;
 }
 
