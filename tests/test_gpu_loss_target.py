@@ -35,3 +35,25 @@ def test_target_column(V, cap):
         z = x.to(dev)
         ops.loss_fwd_bwd(z, tg.clamp(-1, V).int().to(dev), w.to(dev), cap)
         assert torch.equal(y, z)
+
+
+@pytest.mark.parametrize("cap", [0.0, 15.0])
+@pytest.mark.parametrize("V,n", [(24, 8188), (24, 8189), (2048, 8195), (2056, 2047), (2056, 2048), (8200, 2049), (16392, 2050), (32776, 2048)])
+def test_long_launches_take_the_same_bits(V, n, cap):
+    # a launch of 2048 blocks and more may go through its values in another order than one of a few rows: no bit depends on it
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(V + n)
+    x = (3 * torch.randn(n, V, generator=g, device=dev)).bfloat16()
+    tg = torch.randint(-2, V + 2, (n,), generator=g, device=dev)
+    w = 0.5 + torch.rand(n, generator=g, device=dev)
+    for t in (tg, tg.int()):
+        y = x.clone()
+        rows, lse = ops.loss_fwd_bwd(y, t, w, cap)
+        two = ops.loss_bwd(x, t, lse, w, cap)
+        assert torch.equal(y, two)
+        for a in range(0, n, 1000):
+            b = min(a + 1000, n)
+            z = x[a:b].clone()
+            r, l = ops.loss_fwd_bwd(z, t[a:b].contiguous(), w[a:b].contiguous(), cap)
+            assert torch.equal(z, y[a:b]) and torch.equal(r, rows[a:b]) and torch.equal(l, lse[a:b])
+            assert torch.equal(ops.loss_bwd(x[a:b].contiguous(), t[a:b].contiguous(), l, w[a:b].contiguous(), cap), z)

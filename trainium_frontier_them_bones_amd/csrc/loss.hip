@@ -193,6 +193,26 @@ __device__ __forceinline__ u32x4 loss_grad8(const u32x4& u, int i, int t, float 
   return u32x4{pack2bf(d[0], d[1]), pack2bf(d[2], d[3]), pack2bf(d[4], d[5]), pack2bf(d[6], d[7])};
 }
 
+// The same bits with a softcap, one value after the other. Where a launch keeps the SIMDs full, eight values' exponentials and reciprocals side by
+// side only wait for one another, and the target's one is then a twelfth of the instructions; a short launch has the row's end to wait for. us,
+// cap = 15, side by side -> each (from 2048 blocks on, eight for each CU): rows of 8192, 128 of them 5.8 -> 6.8, 1024 14.5 -> 15.1, 2048 24.3 -> 24.1, 8192 77.7 -> 74.8, 16384 146 -> 139; of 1024, 2048
+// of them 6.4 -> 6.5, 16384 28.4 -> 27.5; the backward alone, of 8192, 128 of them 4.5 -> 5.5, 1024 9.6 -> 9.9, 8192 46.0 -> 44.5.
+__device__ __forceinline__ u32x4 loss_grad8_each(const u32x4& u, int i, int t, float g, float l, float icap, float cap) {
+  float d[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const float x = k & 1 ? bfhi(u[k >> 1]) : bflo(u[k >> 1]), hot = i + k == t ? 1.0f : 0.0f;
+    if (cap > 0.f) {  // (always; the branch is what keeps the values apart)
+      const float th = tanh_fast(x * icap);
+      d[k] = g * (fexp(cap * th - l) - hot) * (1.0f - th * th);
+    } else {
+      d[k] = g * (fexp(x - l) - hot);
+    }
+  }
+  return u32x4{pack2bf(d[0], d[1]), pack2bf(d[2], d[3]), pack2bf(d[4], d[5]), pack2bf(d[6], d[7])};
+}
+static inline bool loss_each(long blocks, float softcap) { return softcap > 0.f && blocks >= 2048; }
+
 // loss_row = w * (lse - s_t) with w = row_w[row] (or 1), 0 for a target outside [0, V). Bound by memory: four 16-byte loads a
 // lane in flight. EVAL: the pass over the LM head's logits where the GEMM leaves it to one.
 template <typename IDX, int TPR, bool EVAL>
@@ -236,7 +256,7 @@ __global__ __launch_bounds__(256) void loss_fwd_kernel(const bf16_t* __restrict_
 }
 
 // g_row = grow[row] (upstream grad x row weight); a target outside [0, V) -> 0.
-template <typename IDX, int TPR>
+template <typename IDX, int TPR, bool EACH>
 __global__ __launch_bounds__(256) void loss_bwd_kernel(const bf16_t* __restrict__ x, const IDX* __restrict__ tg,
                                                       const float* __restrict__ lse, const float* __restrict__ grow,
                                                       bf16_t* __restrict__ dx, long rows, int V, float cap) {
@@ -256,7 +276,7 @@ __global__ __launch_bounds__(256) void loss_bwd_kernel(const bf16_t* __restrict_
   for (int i = t0 * 8; i < V; i += TPR * 8) {
     const u32x4 u = unext;
     unext = logits8(xr, i + TPR * 8, V);
-    *(u32x4*)(dr + i) = loss_grad8(u, i, t, g, l, icap, cap);
+    *(u32x4*)(dr + i) = EACH ? loss_grad8_each(u, i, t, g, l, icap, cap) : loss_grad8(u, i, t, g, l, icap, cap);
   }
 }
 
@@ -268,9 +288,11 @@ __global__ __launch_bounds__(256) void loss_bwd_kernel(const bf16_t* __restrict_
 // Bound by memory and by the vector instructions beside it. The target's one behind a branch (loss_grad8) and a store that does not pass
 // through the caches: rows of 32768, 32768 of them 935 -> 790 us, 8192 249 -> 211, 2048 76 -> 66. A row of 32 chunks is unpacked twice, behind an
 // empty asm statement: kept unpacked, its 256 values spilled (4096 rows of 50304 431 us; with the branch alone 257, so 183). With 16 chunks the
-// registers suffice, and two wavefronts a SIMD that unpack once stream better than four that unpack twice (32768 rows 790 us to 860,
-// 2048 66 to 64).
-template <typename IDX, int NCH, int TPR>
+// registers suffice: without a softcap two wavefronts a SIMD that unpack once stream better than four that unpack twice (32768 rows 790 us to 860,
+// 2048 66 to 64); with one, the four hide more of the exponentials (rows of 32768, cap = 15: 2048 84.0 -> 78.8, 16384 588 -> 532; up to 1024 alike).
+// The kernel of 32 chunks is 70 KB of code, more than the instruction cache holds, and moves by up to 8 % with its place in the library.
+// EACH: loss_grad8_each. TWICE: unpacked twice.
+template <typename IDX, int NCH, int TPR, bool EACH, bool TWICE>
 __global__ __launch_bounds__(256) void loss_fwd_bwd_kernel(bf16_t* x, const IDX* __restrict__ tg, const float* __restrict__ row_w,
                                                           float* __restrict__ loss, float* __restrict__ lse, long rows, int V, float cap) {
   __shared__ float rm[4], rs[4], lsh;
@@ -309,8 +331,8 @@ __global__ __launch_bounds__(256) void loss_fwd_bwd_kernel(bf16_t* x, const IDX*
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
     const int i = (t0 + j * TPR) * 8;
-    if (NCH == 32) asm("" : "+v"(u[j]));
-    if (i < V) tfb_store_nt((u32x4*)(xr + i), loss_grad8(u[j], i, t, w, l, icap, cap));
+    if (TWICE) asm("" : "+v"(u[j]));
+    if (i < V) tfb_store_nt((u32x4*)(xr + i), EACH ? loss_grad8_each(u[j], i, t, w, l, icap, cap) : loss_grad8(u[j], i, t, w, l, icap, cap));
   }
 }
 
@@ -592,19 +614,25 @@ extern "C" int tfb_loss_fwd_bwd(void* logits, const void* targets, int idx64, co
   if (!logits || !targets || !loss || !lse) return TFB_ERR_ARG;
   if (rows <= 0 || V <= 0 || V % 8 || V > 65536) return TFB_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-#define TFB_LFB(IDX, NCH, TPR)                                                                                              \
-  hipLaunchKernelGGL((loss_fwd_bwd_kernel<IDX, NCH, TPR>), dim3((unsigned)((rows + 256 / TPR - 1) / (256 / TPR))), dim3(256), 0, s, \
-                     (bf16_t*)logits, (const IDX*)targets, (const float*)row_w, (float*)loss, (float*)lse, rows, V, softcap)
-  if (V <= WAVE_ROW_V) {
-    if (idx64) TFB_LFB(long, 4, 64); else TFB_LFB(int, 4, 64);
-  } else if (V <= 8192) {
-    if (idx64) TFB_LFB(long, 4, 256); else TFB_LFB(int, 4, 256);
-  } else if (V <= 16384) {
-    if (idx64) TFB_LFB(long, 8, 256); else TFB_LFB(int, 8, 256);
-  } else if (V <= 32768) {
-    if (idx64) TFB_LFB(long, 16, 256); else TFB_LFB(int, 16, 256);
+  const long blocks = V <= WAVE_ROW_V ? (rows + 3) / 4 : rows;
+  const bool each = loss_each(blocks, softcap);
+#define TFB_LFB(NCH, TPR, EACH, TWICE)                                                                                         \
+  do {                                                                                                                         \
+    if (idx64) hipLaunchKernelGGL((loss_fwd_bwd_kernel<long, NCH, TPR, EACH, TWICE>), dim3((unsigned)blocks), dim3(256), 0, s, (bf16_t*)logits,  \
+                                  (const long*)targets, (const float*)row_w, (float*)loss, (float*)lse, rows, V, softcap);     \
+    else hipLaunchKernelGGL((loss_fwd_bwd_kernel<int, NCH, TPR, EACH, TWICE>), dim3((unsigned)blocks), dim3(256), 0, s, (bf16_t*)logits,         \
+                            (const int*)targets, (const float*)row_w, (float*)loss, (float*)lse, rows, V, softcap);            \
+  } while (0)
+  if (V > 32768) {
+    TFB_LFB(32, 256, false, true);
+  } else if (V > 16384) {
+    if (softcap > 0.f) TFB_LFB(16, 256, false, true); else TFB_LFB(16, 256, false, false);
+  } else if (V > 8192) {
+    if (each) TFB_LFB(8, 256, true, false); else TFB_LFB(8, 256, false, false);
+  } else if (V > WAVE_ROW_V) {
+    if (each) TFB_LFB(4, 256, true, false); else TFB_LFB(4, 256, false, false);
   } else {
-    if (idx64) TFB_LFB(long, 32, 256); else TFB_LFB(int, 32, 256);
+    if (each) TFB_LFB(4, 64, true, false); else TFB_LFB(4, 64, false, false);
   }
 #undef TFB_LFB
   TFB_LAUNCH_CHECK();
@@ -617,13 +645,19 @@ extern "C" int tfb_loss_bwd(const void* logits, const void* targets, int idx64, 
   if (!logits || !targets || !lse || !grow || !dlogits) return TFB_ERR_ARG;
   if (rows <= 0 || V <= 0 || V % 8) return TFB_ERR_SHAPE;
   hipStream_t s = (hipStream_t)stream;
-#define TFB_LB(IDX, TPR)                                                                                                     \
-  hipLaunchKernelGGL((loss_bwd_kernel<IDX, TPR>), dim3((unsigned)((rows + 256 / TPR - 1) / (256 / TPR))), dim3(256), 0, s,    \
-                     (const bf16_t*)logits, (const IDX*)targets, (const float*)lse, (const float*)grow, (bf16_t*)dlogits, rows, V, softcap)
+  const long blocks = V <= WAVE_ROW_V ? (rows + 3) / 4 : rows;
+  const bool each = loss_each(blocks, softcap);
+#define TFB_LB(TPR, EACH)                                                                                                      \
+  do {                                                                                                                         \
+    if (idx64) hipLaunchKernelGGL((loss_bwd_kernel<long, TPR, EACH>), dim3((unsigned)blocks), dim3(256), 0, s, (const bf16_t*)logits,  \
+                                  (const long*)targets, (const float*)lse, (const float*)grow, (bf16_t*)dlogits, rows, V, softcap);    \
+    else hipLaunchKernelGGL((loss_bwd_kernel<int, TPR, EACH>), dim3((unsigned)blocks), dim3(256), 0, s, (const bf16_t*)logits,         \
+                            (const int*)targets, (const float*)lse, (const float*)grow, (bf16_t*)dlogits, rows, V, softcap);           \
+  } while (0)
   if (V <= WAVE_ROW_V) {
-    if (idx64) TFB_LB(long, 64); else TFB_LB(int, 64);
+    if (each) TFB_LB(64, true); else TFB_LB(64, false);
   } else {
-    if (idx64) TFB_LB(long, 256); else TFB_LB(int, 256);
+    if (each) TFB_LB(256, true); else TFB_LB(256, false);
   }
 #undef TFB_LB
   TFB_LAUNCH_CHECK();
