@@ -77,19 +77,24 @@ static inline bool tfb_attn_dkdv_half_applies(int D, int T, long nbh, int nw, co
 }
 
 // The forward: one workgroup of 64 queries for each CU (but for blocks of one tile of D = 128), or as much work as this line, in the same units.
-// us, one wavefront to 32 queries -> pairs, blocks in brackets:
+// At D = 128 a second workgroup finds no room on a CU, so beyond one for each only a sequence pays whose light blocks end early enough for the
+// rest: six tiles and more without a band. us, one wavefront to 32 queries -> pairs, blocks in brackets:
 //   D = 64   T128 [128] 5.9 -> 5.4, [192] 6.1 -> 6.2; T256 [192] 7.5 -> 6.7, [320] 9.9 -> 9.9; T512 [192] 9.8 -> 8.8, [256] 10.0 -> 9.2, [320] 11.1 -> 12.0; T1024
 //            [256] 14.8 -> 13.4, [320] 15.3 -> 15.7; T1664 [312] 21.2 -> 19.5, [364] 21.5 -> 22.8; T2048 [192] 24.2 -> 21.2, [320] 24.8 -> 22.8, [384] 25.2 ->
 //            27.1; T4096 [320] 44.7 -> 40.1, [384] 45.3 -> 47.1; bands of T2048: 2 [128] 7.0 -> 6.2, [192] 7.3 -> 7.4; 4 [128] 9.4 -> 8.3, [192] 9.8 -> 10.6;
 //            8 [192] 14.8 -> 13.6, [256] 15.2 -> 17.2
-//   D = 128  T128 [128] 7.6 -> 7.7; T256 [128] 9.7 -> 9.3, [192] 10.5 -> 14.2; T512 [128] 12.9 -> 12.2, [192] 13.6 -> 16.2; T1024 [128] 19.6 -> 18.4, [192]
-//            20.3 -> 20.1, [224] 20.6 -> 22.6; T1664 [208] 28.0 -> 26.1, [260] 28.9 -> 35.4; T2048 [192] 32.8 -> 30.7, [224] 32.9 -> 32.8, [256] 33.2 -> 34.8;
-//            T4096 [192] 58.1 -> 55.2, [256] 59.2 -> 59.1; bands of T2048: 4 [128] 13.0 -> 12.4, [192] 14.2 -> 22.0
+//   D = 128  T128 [96] 7.8 -> 7.7, [144] 8.0 -> 11.3; T256 [128] 9.5 -> 9.2, [144] 9.8 -> 11.5; T384 [108] 11.1 -> 10.4, [144] 11.5 -> 12.6; T512 [96] 12.7 ->
+//            11.8, [144] 13.4 -> 13.3, [192] 13.4 -> 15.8; T640 [120] 14.6 -> 13.4, [180] 15.1 -> 16.1; T768 [144] 16.4 -> 15.4, [216] 16.8 -> 19.2; T1024 [128]
+//            19.3 -> 18.2, [192] 19.7 -> 19.6, [224] 20.6 -> 22.6; T1664 [208] 27.5 -> 25.8, [260] 28.9 -> 35.4; T2048 [192] 32.4 -> 31.2, [256] 32.8 -> 34.3;
+//            T4096 [192] 58.1 -> 54.5, [256] 58.2 -> 57.7; bands: 2 T2048 [128] 9.6 -> 9.2, [192] 10.4 -> 16.3; 4 T2048 [128] 12.7 -> 12.1, [192] 13.5 -> 21.5;
+//            8 T2048 [128] 19.3 -> 18.2, [192] 19.9 -> 27.3
 static inline bool tfb_attn_fwd_pair_applies(int D, int T, long nbh, int nw, const long* ks, const long* vs) {
   const AttnLoad l = attn_load(T, nbh, nw);
-  const long cus = tfb_resident_slots(1);
+  const long cus = tfb_resident_slots(1), nx = T / 128;
   if (!tfb_attn_dkdv_strides_ok(ks, vs) || (D == 128 && l.longest == 1)) return false;
-  return 2 * l.blocks <= cus || 1000 * l.work <= (D == 64 ? 665 : 440) * cus * l.longest;
+  if (2 * l.blocks <= cus) return true;
+  if (D == 64) return 1000 * l.work <= 665 * cus * l.longest;
+  return l.longest == nx && nx >= 6 && 1000 * l.work <= (nx >= 8 ? 440 : 350) * cus * l.longest;
 }
 
 namespace {
