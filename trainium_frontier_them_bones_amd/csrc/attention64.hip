@@ -782,6 +782,11 @@ __global__ __launch_bounds__(256, TFB_DQ64_WPE) void attn64_dq_kernel(AttnT q, A
   }
 }
 
+// The turn where the workgroups are at most two for each CU, or the sequence has eight blocks and more: a third workgroup on a CU evens out the short
+// sequences' blocks by itself. us, no turn -> the turn, blocks in brackets: forward T512 [576] 14.8 -> 15.4, T640 [720] 18.2 -> 18.6, T1024 [576] 20.5 -> 19.6,
+// T2048 [768] 38.5 -> 37.4; backward T384 [576] 37.8 -> 39.6, T512 [576] 43.4 -> 42.3, T640 [640] 47.3 -> 49.1, T768 [576] 48.7 -> 49.9, T1664 [832] 103 -> 99.6
+int first_round64(int nx, int nbh) { return nx < 8 && (long)nx * nbh > tfb_resident_slots(2) ? 0 : first_round(nx, nbh, true); }
+
 }  // namespace
 
 // Called by tfb_attn_fwd / tfb_attn_bwd for D = 64 (arguments already validated there: T % 128 == 0, strides % 8 == 0).
@@ -789,7 +794,7 @@ int tfb_attn64_fwd_impl(const void* q, const long* qs, const void* k, const long
                         const long* os, float* lse, int B, int H, int T, float scale, int nw, hipStream_t s) {
   if (tfb_attn_fwd_pair_applies(64, T, (long)B * H, nw, ks, vs)) return tfb_attn_fwd_pair_impl(q, qs, k, ks, v, vs, o, os, lse, B, H, T, 64, scale, nw, s);
   hipLaunchKernelGGL(attn64_fwd_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(o, os), lse,
-                     T, H, scale * LOG2E, nw, tfb_resident_slots(2), first_round(T / 128, B * H, true));
+                     T, H, scale * LOG2E, nw, tfb_resident_slots(2), first_round64(T / 128, B * H));
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
@@ -809,13 +814,13 @@ int tfb_attn64_bwd_impl(const void* q, const long* qs, const void* k, const long
   } else {
     hipLaunchKernelGGL(attn64_dq_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
                        mk(dq, dqs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw,
-                       tfb_resident_slots(2), first_round(T / 128, B * H, true), mk(o, os), lse);
+                       tfb_resident_slots(2), first_round64(T / 128, B * H), mk(o, os), lse);
     TFB_LAUNCH_CHECK();
   }
   if (tfb_attn_dkdv_pair_applies(T, (long)B * H, nw, qs, gos) || tfb_attn_dkdv_half_applies(64, T, (long)B * H, nw, qs, gos))
     return tfb_attn_dkdv_impl(q, qs, k, ks, v, vs, go, gos, dk, dks, dv, dvs, stats, B, H, T, 64, scale, cos_t, sin_t, nw, s);
   hipLaunchKernelGGL(attn64_dkdv_kernel, dim3(paired_grid(T / 128, B * H, 2), B * H), dim3(256), 0, s, mk(q, qs), mk(k, ks), mk(v, vs), mk(go, gos),
-                     mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw, tfb_resident_slots(2), first_round(T / 128, B * H, true));
+                     mk(dk, dks), mk(dv, dvs), stats, rows, T, H, scale, scale * LOG2E, (const bf16_t*)cos_t, (const bf16_t*)sin_t, nw, tfb_resident_slots(2), first_round64(T / 128, B * H));
   TFB_LAUNCH_CHECK();
   return TFB_OK;
 }
