@@ -553,7 +553,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   //   reads then use the banks evenly), a row's 64 outputs on 8 consecutive lanes;
   //   32 p: row q = 64 bytes, chunk c at slot c ^ ((q >> 2) & 3), a row's outputs on 4 lanes; X = Q: tile i is rows 32 i .. of q.
   // The epilogue's own operand (a residual, rotation tables) is four 16-byte loads a lane and block, requested one store ahead by request_pre().
-  u32x4 pre[4] = {};
+  u32x4 pre[8] = {};  // (the second four only behind the loop)
   auto here = [](int x) __attribute__((always_inline)) {  // (what is made of it is not kept in registers across the loop)
     if constexpr (kPipe) asm volatile("" : "+v"(x));
     return x;
@@ -562,8 +562,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     if constexpr (kPartner) asm volatile("global_load_dwordx4 %0, %1, off" : "+v"(pre[k]) : "v"(g) : "memory");
     else asm volatile("global_load_dwordx4 %0, %1, off nt" : "+v"(pre[k]) : "v"(g) : "memory");  // (read once)
   };
-  auto wait_pre = [&](auto AFTER) __attribute__((always_inline)) {  // AFTER: vector memory instructions issued since
-    auto& r = pre;
+  auto wait_pre = [&](auto AFTER, auto FROM) __attribute__((always_inline)) {  // AFTER: vector memory instructions issued since
+    auto* r = pre + decltype(FROM)::value;
     asm volatile("s_waitcnt vmcnt(%4)" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : "n"(decltype(AFTER)::value) : "memory");
   };
   // a block's place: its first p and q, a lane's chunk and first row, rows from one of its chunks to the next, chunks
@@ -580,8 +580,8 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
 #pragma unroll
       for (int k = 0; k < NCH; ++k) {
         if constexpr (kPartner != 0) {
-          load_pre(2 * k, epi.at(p, q + RSTEP * k));
-          load_pre(2 * k + 1, epi.at2(p, q + RSTEP * k));
+          load_pre(from + 2 * k, epi.at(p, q + RSTEP * k));
+          load_pre(from + 2 * k + 1, epi.at2(p, q + RSTEP * k));
         } else {
           load_pre(from + k, epi.at(p, q + RSTEP * k));
         }
@@ -611,7 +611,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
         const int row = (ln >> 2) + 16 * k, ch = ln & 3;
         const u32x4 lo = *(const u32x4*)(stg + row * 128 + ((ch ^ ((row >> 1) & 7)) << 4));
         const u32x4 hi = *(const u32x4*)(stg + row * 128 + (((ch + 4) ^ ((row >> 1) & 7)) << 4));
-        if constexpr (!kF32) epi.chunk2(pb + 8 * ch, qb + row, lo, hi, pre[2 * k], pre[2 * k + 1]);
+        if constexpr (!kF32) epi.chunk2(pb + 8 * ch, qb + row, lo, hi, pre[from + 2 * k], pre[from + 2 * k + 1]);
       }
     } else {
       constexpr int NCH = wide ? 4 : QX ? 2 * NI : 2, RSTEP = wide ? 8 : 16;  // chunks of a lane, rows apart
@@ -726,7 +726,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
     auto store_pipe = [&](auto HX, auto HY, auto AFTER, auto next) __attribute__((always_inline)) {
       if constexpr (stores && kPipe) {
         if (have_prev) {
-          wait_pre(AFTER);
+          wait_pre(AFTER, H0{});
           store_block(HX, HY, pp0, pq0, H0{});
           next();
         }
@@ -890,17 +890,29 @@ __global__ __launch_bounds__(512, 2) void gemm_pp_kernel(PpArgs a, Epi epi_in) {
   if constexpr (!kF32) {
     waitB(fb0);  // the stream's last fragments, which nobody multiplies, land before their registers are used again
     // the last tile's accumulators
-    auto flush = [&](auto HX, auto HY, auto request_it) __attribute__((always_inline)) {
-      if constexpr (kPipe) {
-        if constexpr (decltype(request_it)::value) request_pre(HX, HY, pp0, pq0, H0{});
-        wait_pre(H0{});
-      }
-      store_block(HX, HY, pp0, pq0, H0{});
-    };
-    flush(H0{}, H0{}, std::false_type{});
-    if (!(kRows && alone_prev)) flush(H0{}, H1{}, std::true_type{});
-    flush(H1{}, H0{}, std::true_type{});
-    if (!(kRows && alone_prev)) flush(H1{}, H1{}, std::true_type{});
+    if constexpr (kPipe) {
+      // Each block's operand is requested in front of the stores of the block before it, into the other four registers. Behind them its wait
+      // covered those stores as well, three times a launch (us, bf16 with a residual: 12288 x 1024 x 1024 37.6 -> 35.3, 10240 x 1024 x 1024 36.2 -> 33.8,
+      // 4096 x 3072 x 1024 37.0 -> 34.6; fp8 20480 x 512 x 2048 32.9 -> 30.2, 12288 x 768 x 3072 35.5 -> 33.1; 10240 x 1536 with its rotation 24.8 -> 23.7).
+      constexpr int HALF = NARROW ? 2 : 4;  // requests and stores of a block of half 1; half 0: four
+      typedef std::integral_constant<int, 4> N4;
+      request_pre(H0{}, H1{}, pp0, pq0, N4{});
+      wait_pre(N4{}, H0{});
+      store_block(H0{}, H0{}, pp0, pq0, H0{});
+      request_pre(H1{}, H0{}, pp0, pq0, H0{});
+      wait_pre(std::integral_constant<int, 4 + HALF>{}, N4{});
+      store_block(H0{}, H1{}, pp0, pq0, N4{});
+      request_pre(H1{}, H1{}, pp0, pq0, N4{});
+      wait_pre(std::integral_constant<int, 4 + HALF>{}, H0{});
+      store_block(H1{}, H0{}, pp0, pq0, H0{});
+      wait_pre(std::integral_constant<int, HALF>{}, N4{});
+      store_block(H1{}, H1{}, pp0, pq0, N4{});
+    } else {
+      store_block(H0{}, H0{}, pp0, pq0, H0{});
+      if (!(kRows && alone_prev)) store_block(H0{}, H1{}, pp0, pq0, H0{});
+      store_block(H1{}, H0{}, pp0, pq0, H0{});
+      if (!(kRows && alone_prev)) store_block(H1{}, H1{}, pp0, pq0, H0{});
+    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stream's last (unused) loads must have landed before LDS is released
 }
