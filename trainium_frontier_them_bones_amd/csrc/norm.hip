@@ -177,7 +177,8 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_kernel(const bf16_t* __restri
 // Bound as the forward, and as that one without a row asked for ahead. With a gain, 8192 x 768: 16.1 -> 12.8 us in a training step, alone
 // 16384 x 768 21.0 -> 17.8, 2048 x 1024 6.5 -> 5.8, 4096 x 4096 48 -> 40, 32768 x 768 32.5 -> 31.4; without one, by a kernel of its own (half the
 // registers) with a turn for each row: 256 x 768 3.2 -> 3.1, 8192 x 768 9.7 -> 8.3, 4096 x 4096 28 -> 21, 32768 x 1024 40.0 -> 38.7; slower only at 4096 columns from
-// 32768 rows on with partials to write (a gain 319 -> 339, maxima 288 -> 299; half the registers there were slower still). Widening the row twice
+// 32768 rows on with partials to write (65536 with a gain 308 -> 317, gs too 318 -> 339, maxima 288 -> 298; half the registers there were slower
+// still, and a row asked for ahead from raw registers spills). Widening the row twice
 // (119 registers for 166 at 768 columns) gave as much on many rows with a gain and cost 1500 x 1024 without one 0.6 us of 4.1.
 template <int NCH, int G, bool W>
 __global__ __launch_bounds__(256) void rmsnorm_bwd_kernel(const bf16_t* __restrict__ gy, const bf16_t* __restrict__ gs,
